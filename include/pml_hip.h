@@ -546,6 +546,41 @@ int pml_hip_argsort(const pml_hip_argsort_desc* desc, const void* tensor, void* 
  * of its run of values by applying precomputed powers of the step matrix instead of stepping from the beginning. */
 int pml_hip_prng(const void* state, int64_t count, void* values, void* new_state, pml_hip_stream s);
 
+/* ---- products over free strides, and the gradients of a convolution -------------
+ * C[b][m][n] = tail( init + sum_k A[b][m][k] * B[b][k][n] ) with an element stride for every index of every operand (C's
+ * columns are contiguous), up to three batch indices, and no demand on alignment or on sizes: what a contraction of
+ * the multiply-add kind is when pml_hip_gemm's row layout does not fit it (the reference tiles such nests around the
+ * same strided micro-kernel, pmlc/dialect/pxa/transforms/stencil_gemm.cc:297-321).  One of a_ms / a_ks and one of
+ * b_ks / b_ns should be 1: other strides are read element by element.
+ *   in_dtype F32 -> fp32 MFMA, out_dtype F32;  in_dtype BF16 -> bf16 MFMA, fp32 accumulate, out_dtype BF16 or F32.
+ * The tail may hold up to four plain arithmetic steps in out_dtype on immediates and tensors of that type
+ * (pml_hip_product_takes_tail); its rows are C's element offsets divided by row_len. */
+typedef struct {
+  int32_t in_dtype, out_dtype;
+  int32_t n_batch;
+  int32_t init_kind; /* 0: none, 1: a tensor of out_dtype addressed with init_row_stride / init_col_stride */
+  int64_t batch[3], a_batch[3], b_batch[3], c_batch[3];
+  int64_t m, n, k;
+  int64_t a_ms, a_ks, b_ks, b_ns, c_ms;
+  int64_t row_len;
+  int64_t init_row_stride, init_col_stride;
+  pml_hip_epilogue tail;
+} pml_hip_product_desc;
+
+int64_t pml_hip_product_dispatch(const pml_hip_product_desc* desc);
+int pml_hip_product_takes_tail(const pml_hip_epilogue* tail, int out_dtype); /* host arithmetic only */
+int pml_hip_product_invoke(int64_t plan, const void* a, const void* b, void* c, const void* init, const void* const* operands,
+                           pml_hip_stream s);
+
+/* The two gradients of a convolution (plaidml/op/lib/ops.cc:1342-1450 with its deriv_mode): `desc` describes the forward
+ * convolution (F32 or BF16, no tail, no initial value); G is the gradient of its output [n][oh][ow][co].
+ *   which 0, data:   dI[n, sy*y + dy*ky - py, sx*x + dx*kx - px, ci] += G[n,y,x,co] * F[ky,kx,ci,co]   (other = F, result dI)
+ *   which 1, filter: dF[ky,kx,ci,co] += I[n, sy*y + dy*ky - py, sx*x + dx*kx - px, ci] * G[n,y,x,co]   (other = I, result dF)
+ * The filter gradient needs dil_w = 1 or kw = 1 (pml_hip_conv2d_grad_takes). */
+int pml_hip_conv2d_grad_takes(const pml_hip_conv2d_desc* desc, int which); /* host arithmetic only */
+int64_t pml_hip_conv2d_grad_dispatch(const pml_hip_conv2d_desc* desc, int which);
+int pml_hip_conv2d_grad_invoke(int64_t plan, const void* g, const void* other, void* result, pml_hip_stream s);
+
 /* ---- any contraction ---------------------------------------------------------
  * The loop-nest form a contraction takes after bounds computation: the
  * `affine.parallel` + `pxa.load` + `pxa.reduce` nest of
@@ -595,7 +630,8 @@ int pml_hip_contract_invoke(int64_t plan, const void* const* srcs, void* out, pm
 
 /* sizeof() of a descriptor struct as this library was compiled, so that a foreign-language
  * binding can verify its own layout: 0 epilogue, 1 gemm, 2 conv2d, 3 dwconv2d, 4 pool2d,
- * 5 eltwise, 6 select, 7 contract, 8 form, 9 gather, 10 scatter, 11 argsort, 12 softmax.  Returns 0 for an unknown id. */
+ * 5 eltwise, 6 select, 7 contract, 8 form, 9 gather, 10 scatter, 11 argsort, 12 softmax,
+ * 13 product.  Returns 0 for an unknown id. */
 size_t pml_hip_struct_size(int which);
 
 /* Releases a plan returned by any *_dispatch. */

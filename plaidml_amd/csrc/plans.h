@@ -273,6 +273,46 @@ hipError_t scatter_launch(const pml_hip_scatter_desc& d, const void* data, const
 hipError_t argsort_launch(const pml_hip_argsort_desc& d, const void* tensor, void* out, hipStream_t s);
 hipError_t prng_launch(const void* state, int64_t count, void* values, void* new_state, hipStream_t s);
 
+// Products over free strides (strided.hip).  C[batch][m][n] = tail(init + sum_k A[batch][m][k] * B[batch][k][n]).
+struct StridedOp {
+  int32_t opcode, pad;
+  float imm;        // already rounded to the result type
+  const void* ptr;  // operand tensor of the result type (null: imm), addressed by result row and column
+  int64_t rs, cs;
+};
+struct StridedArgs {
+  const void *A, *B;
+  void* C;
+  int64_t M, N, K;
+  int64_t a_ms, a_ks, b_ks, b_ns, c_ms;  // element strides; C's columns are contiguous
+  int64_t row_len;                       // the tail's row number of a result row = its element offset in C / row_len
+  int32_t n_batch, out_bf16;
+  int64_t batch[3], a_batch[3], b_batch[3], c_batch[3];
+  const void* init;  // of the result type, or null
+  int64_t init_rs, init_cs;
+  int32_t n_ops, splits;
+  StridedOp ops[4];
+  // filled in by strided_plan: tile grid, K values per split, workspace [splits][ws_rows][ws_pitch]
+  int tiles_m, tiles_n, tiles_per_tap, pad;
+  int64_t k_per_split, ws_rows, ws_pitch;
+  float* ws;
+  // filter gradient: A is the NHWC image, K runs over the gradient's pixels, M over [ky][row_cols = kw * ci]
+  int64_t row_cols;
+  int H, W, CI, OH, OW, SH, SW, PH, PW, DH;
+  unsigned div_per_magic, div_ow_magic;
+  int div_per_shift, div_ow_shift;
+};
+void strided_plan(StridedArgs* a, bool bf, bool conv, int n_cus, int* mi);
+hipError_t strided_launch(const StridedArgs& a, bool bf, bool conv, int mi, hipStream_t s);
+struct Col2imArgs {
+  const float* cols;  // [N][OH][OW][KH][KW][CI]
+  void* out;          // [N][H][W][CI]
+  int N, H, W, CI, OH, OW, KH, KW, SH, SW, PH, PW, DH, DW;
+};
+hipError_t col2im_launch(const Col2imArgs& a, bool bf, hipStream_t s);
+hipError_t pad_rows_launch(int es, const void* in, void* out, int64_t rows, int64_t cols, int64_t pitch, hipStream_t s);
+hipError_t flip_filter_launch(int es, const void* f, void* bt, int64_t taps, int64_t ci, int64_t co, int64_t pitch, hipStream_t s);
+
 // window kernels (window.hip)
 struct DwconvArgs {
   pml_hip_dwconv2d_desc d;

@@ -3,6 +3,7 @@
 // it many times.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
 #include <cstdio>
 #include <cstdlib>
@@ -29,7 +30,7 @@ int check(hipError_t e, const char* what) {
   return 1;
 }
 
-enum PlanKind { PLAN_GEMM = 1, PLAN_CONV, PLAN_DWCONV, PLAN_POOL, PLAN_ELTWISE, PLAN_CONTRACT };
+enum PlanKind { PLAN_GEMM = 1, PLAN_CONV, PLAN_DWCONV, PLAN_POOL, PLAN_ELTWISE, PLAN_CONTRACT, PLAN_PRODUCT, PLAN_CONV_GRAD };
 
 struct Plan {
   int kind = 0;
@@ -70,6 +71,15 @@ struct Plan {
   int sk_splits = 0, sk_per = 0, sk_pitch = 0;
   // register-filter convolution: a filter packed once, in the order the kernel holds it in registers
   void* reg_image = nullptr;
+  // product over free strides, and a convolution's gradients built on it: the prepared arguments (workspace in `ws`),
+  // element kind, tile; a data gradient of unit stride is a convolution of the gradient (`sub`, its channels padded to
+  // whole 16-byte vectors in `padded`), one of a larger stride a product into `cols`, images `grad_chunk` at a time
+  StridedArgs strided;
+  bool strided_bf = false, strided_conv = false;
+  int strided_mi = 1, grad_which = 0;
+  Plan* sub = nullptr;
+  void *padded = nullptr, *cols = nullptr;
+  int64_t co_pad = 0, grad_chunk = 0;
   // resident-filter convolution: LDS bytes (0 = not used), window rows, tile count, CUs of the device
   size_t halo_lds = 0;
   int halo_rows = 0, halo_tiles = 0, halo_variant = 0, n_cus = 0;
@@ -83,6 +93,9 @@ struct Plan {
     if (ws) (void)hipFree(ws);
     if (dw_filter) (void)hipFree(dw_filter);
     if (dw_paired) (void)hipFree(dw_paired);
+    if (padded) (void)hipFree(padded);
+    if (cols) (void)hipFree(cols);
+    delete sub;
   }
 };
 
@@ -333,6 +346,15 @@ bool valid_tail(const pml_hip_epilogue& t, bool allow64 = false) {
     if (!allow64 && dt_size(op.dtype) == 8 && op.opcode != PML_HIP_EPI_STORE) return false;  // 64-bit steps: general path only
   }
   return true;
+}
+
+// fp32 rounded to bf16 (nearest even), as fp32; NaNs stay NaNs
+float host_round_bf16(float f) {
+  uint32_t u;
+  std::memcpy(&u, &f, 4);
+  u = (u & 0x7fffffffu) > 0x7f800000u ? ((u & 0xffff0000u) | 0x00400000u) : ((u + 0x7fffu + ((u >> 16) & 1u)) & 0xffff0000u);
+  std::memcpy(&f, &u, 4);
+  return f;
 }
 
 // Compute units of the current device (persistent kernels size their grids by it).
@@ -1240,6 +1262,287 @@ int pml_hip_conv2d_pack_filter(int64_t plan, const void* filter, pml_hip_stream 
 }
 
 // ---------------------------------------------------------------------------
+// products over free strides, gradients of a convolution
+// ---------------------------------------------------------------------------
+
+int pml_hip_product_takes_tail(const pml_hip_epilogue* t, int out_dtype) {
+  if (!t || !valid_tail(*t) || t->n_ops > 4 || (out_dtype != PML_HIP_F32 && out_dtype != PML_HIP_BF16)) return 0;
+  for (int i = 0; i < t->n_ops; ++i) {
+    const pml_hip_epi_op& op = t->ops[i];
+    switch (op.opcode) {
+      case PML_HIP_EPI_ADD: case PML_HIP_EPI_SUB: case PML_HIP_EPI_RSUB: case PML_HIP_EPI_MUL: case PML_HIP_EPI_DIV:
+      case PML_HIP_EPI_RDIV: case PML_HIP_EPI_MAX: case PML_HIP_EPI_MIN: case PML_HIP_EPI_MAX_GT: case PML_HIP_EPI_RELU: case PML_HIP_EPI_NEG:
+        break;
+      default: return 0;
+    }
+    if (op.dtype != out_dtype || (op.operand_kind == PML_HIP_OPND_TENSOR && t->operand_dtype[op.operand] != out_dtype)) return 0;
+  }
+  return 1;
+}
+
+// Grid, split and workspace of a plan whose `strided` arguments name the problem; false with the error text set.
+static bool prepare_strided(Plan* p) {
+  StridedArgs& a = p->strided;
+  strided_plan(&a, p->strided_bf, p->strided_conv, device_cus(), &p->strided_mi);
+  a.ws = nullptr;
+  if (a.splits > 1 && hipMalloc(&p->ws, (size_t)a.splits * a.ws_rows * a.ws_pitch * 4) != hipSuccess) {
+    (void)hipGetLastError();
+    p->ws = nullptr;  // (no memory for the partial results: the K loop is not split)
+    a.splits = 1;
+    a.k_per_split = (a.K + 63) / 64 * 64;
+  }
+  a.ws = (float*)p->ws;
+  int64_t nb = (int64_t)a.tiles_m * a.tiles_n;
+  for (int d = 0; d < a.n_batch; ++d) nb *= a.batch[d];
+  if (nb >= ((int64_t)1 << 31)) {
+    fail("product: too many result tiles");
+    return false;
+  }
+  return true;
+}
+
+int64_t pml_hip_product_dispatch(const pml_hip_product_desc* d) {
+  if (!d) {
+    fail("null descriptor");
+    return 0;
+  }
+  const bool bf = d->in_dtype == PML_HIP_BF16;
+  if ((d->in_dtype != PML_HIP_F32 && !bf) || (d->out_dtype != PML_HIP_F32 && (!bf || d->out_dtype != PML_HIP_BF16))) {
+    fail("product: in_dtype must be F32 or BF16 and out_dtype F32 or in_dtype");
+    return 0;
+  }
+  bool ok = d->m > 0 && d->n > 0 && d->k > 0 && d->n_batch >= 0 && d->n_batch <= 3 && d->a_ms >= 0 && d->a_ks >= 0 && d->b_ks >= 0 &&
+            d->b_ns >= 0 && d->c_ms >= 0 && d->row_len > 0 && (d->init_kind == 0 || d->init_kind == 1);
+  int64_t batches = 1;
+  for (int i = 0; ok && i < d->n_batch; ++i) {
+    ok = d->batch[i] > 0 && d->a_batch[i] >= 0 && d->b_batch[i] >= 0 && d->c_batch[i] >= 0 && d->batch[i] < ((int64_t)1 << 31);
+    if (ok) batches *= d->batch[i];
+    ok = ok && batches < ((int64_t)1 << 31);
+  }
+  if (!ok) {
+    fail("product: bad sizes or strides");
+    return 0;
+  }
+  if (!pml_hip_product_takes_tail(&d->tail, d->out_dtype)) {
+    fail("product: the tail holds steps this kernel does not run");
+    return 0;
+  }
+  Plan* p = new Plan();
+  p->kind = PLAN_PRODUCT;
+  p->strided_bf = bf;
+  StridedArgs& a = p->strided;
+  std::memset(&a, 0, sizeof a);
+  a.M = d->m, a.N = d->n, a.K = d->k;
+  a.a_ms = d->a_ms, a.a_ks = d->a_ks, a.b_ks = d->b_ks, a.b_ns = d->b_ns, a.c_ms = d->c_ms;
+  a.row_len = d->row_len;
+  a.n_batch = d->n_batch;
+  a.out_bf16 = d->out_dtype == PML_HIP_BF16;
+  for (int i = 0; i < d->n_batch; ++i) {
+    a.batch[i] = d->batch[i];
+    a.a_batch[i] = d->a_batch[i];
+    a.b_batch[i] = d->b_batch[i];
+    a.c_batch[i] = d->c_batch[i];
+  }
+  a.init_rs = d->init_row_stride;
+  a.init_cs = d->init_col_stride;
+  p->gemm.init_kind = d->init_kind;
+  p->gemm.tail = d->tail;
+  a.n_ops = d->tail.n_ops;
+  for (int i = 0; i < d->tail.n_ops; ++i) {
+    const pml_hip_epi_op& op = d->tail.ops[i];
+    StridedOp& o = a.ops[i];
+    o.opcode = op.opcode;
+    o.imm = op.operand_kind != PML_HIP_OPND_IMM ? 0.f : a.out_bf16 ? host_round_bf16((float)op.imm) : (float)op.imm;
+    if (op.operand_kind == PML_HIP_OPND_TENSOR) {
+      o.rs = d->tail.operand_row_stride[op.operand];
+      o.cs = d->tail.operand_col_stride[op.operand];
+    }
+  }
+  if (!prepare_strided(p)) {
+    delete p;
+    return 0;
+  }
+  char buf[256];
+  std::snprintf(buf, sizeof buf, "product %s batch=%lld m=%lld n=%lld k=%lld tile=%dx%d splits=%d", bf ? "bf16" : "f32", (long long)batches,
+                (long long)d->m, (long long)d->n, (long long)d->k, 64 * p->strided_mi, 64 * p->strided_mi, a.splits);
+  p->text = buf;
+  return (int64_t)(intptr_t)p;
+}
+
+int pml_hip_product_invoke(int64_t plan, const void* a, const void* b, void* c, const void* init, const void* const* operands,
+                           pml_hip_stream s) {
+  Plan* p = (Plan*)(intptr_t)plan;
+  if (!p || p->kind != PLAN_PRODUCT) return fail("product_invoke: not a product plan");
+  if (!a || !b || !c) return fail("product_invoke: null operand");
+  if (p->gemm.init_kind && !init) return fail("product_invoke: the plan expects an initial value");
+  StridedArgs g = p->strided;
+  g.A = a;
+  g.B = b;
+  g.C = c;
+  g.init = p->gemm.init_kind ? init : nullptr;
+  for (int i = 0; i < g.n_ops; ++i) {
+    const pml_hip_epi_op& op = p->gemm.tail.ops[i];
+    if (op.operand_kind != PML_HIP_OPND_TENSOR) continue;
+    if (!operands || !operands[op.operand]) return fail("product_invoke: missing tail operand");
+    g.ops[i].ptr = operands[op.operand];
+  }
+  return check(strided_launch(g, p->strided_bf, false, p->strided_mi, (hipStream_t)s), "strided_launch");
+}
+
+int pml_hip_conv2d_grad_takes(const pml_hip_conv2d_desc* d, int which) {
+  if (!d || (which != 0 && which != 1) || (d->in_dtype != PML_HIP_F32 && d->in_dtype != PML_HIP_BF16) || d->out_dtype != d->in_dtype || d->flags != 0 ||
+      d->tail.n_ops != 0 || d->init_kind != 0)
+    return 0;
+  if (d->n <= 0 || d->h <= 0 || d->w <= 0 || d->ci <= 0 || d->kh <= 0 || d->kw <= 0 || d->co <= 0 || d->oh <= 0 || d->ow <= 0 ||
+      d->stride_h <= 0 || d->stride_w <= 0 || d->dil_h <= 0 || d->dil_w <= 0)
+    return 0;
+  const int64_t lim = (int64_t)1 << 31;  // (pixel numbers and offsets inside an image are 32-bit)
+  if (d->n * d->oh * d->ow >= lim || d->h * d->w * d->ci >= lim || d->kh * d->kw * d->ci >= lim || d->kh * d->kw * d->co >= lim ||
+      d->n * d->h * d->w >= lim || std::llabs(d->pad_h) >= (1 << 20) || std::llabs(d->pad_w) >= (1 << 20) ||
+      (d->ow * d->stride_w + std::llabs(d->pad_w) + d->kw) * d->ci >= lim)
+    return 0;
+  return which == 0 || d->dil_w == 1 || d->kw == 1;
+}
+
+int64_t pml_hip_conv2d_grad_dispatch(const pml_hip_conv2d_desc* d, int which) {
+  if (!pml_hip_conv2d_grad_takes(d, which)) {
+    fail("conv2d_grad: bad geometry, types or options");
+    return 0;
+  }
+  const bool bf = d->in_dtype == PML_HIP_BF16;
+  const int es = bf ? 2 : 4;
+  Plan* p = new Plan();
+  p->kind = PLAN_CONV_GRAD;
+  p->conv = *d;
+  p->grad_which = which;
+  p->strided_bf = bf;
+  StridedArgs& a = p->strided;
+  std::memset(&a, 0, sizeof a);
+  a.row_len = 1;
+  char buf[256];
+  if (which == 1) {
+    p->strided_conv = true;
+    a.row_cols = d->kw * d->ci;
+    a.M = d->kh * a.row_cols;
+    a.N = d->co;
+    a.K = d->n * d->oh * d->ow;
+    a.b_ks = d->co;
+    a.b_ns = 1;
+    a.c_ms = d->co;
+    a.out_bf16 = bf;
+    a.H = (int)d->h, a.W = (int)d->w, a.CI = (int)d->ci, a.OH = (int)d->oh, a.OW = (int)d->ow;
+    a.SH = (int)d->stride_h, a.SW = (int)d->stride_w, a.PH = (int)d->pad_h, a.PW = (int)d->pad_w, a.DH = (int)d->dil_h;
+    fast_div_magic((unsigned)(d->oh * d->ow), &a.div_per_magic, &a.div_per_shift);
+    fast_div_magic((unsigned)d->ow, &a.div_ow_magic, &a.div_ow_shift);
+    if (!prepare_strided(p)) {
+      delete p;
+      return 0;
+    }
+    std::snprintf(buf, sizeof buf, "conv2d filter gradient %s: %lld pixels x (%lld window values, %lld channels) tile=%dx%d splits=%d", bf ? "bf16" : "f32",
+                  (long long)a.K, (long long)a.M, (long long)a.N, 64 * p->strided_mi, 64 * p->strided_mi, a.splits);
+    p->text = buf;
+    return (int64_t)(intptr_t)p;
+  }
+  // Data gradient.  Unit stride: the convolution of the gradient with the filter's taps in reverse and its channels'
+  // roles exchanged, on the convolution kernels; channel counts that do not fill 16-byte vectors are padded with zeros
+  // in a copy of the gradient (one pass over it, against a patch matrix of kh * kw times its size).
+  const int64_t v = 16 / es;
+  p->co_pad = (d->co + v - 1) / v * v;
+  const int64_t back_h = d->dil_h * (d->kh - 1) - d->pad_h, back_w = d->dil_w * (d->kw - 1) - d->pad_w;
+  if (d->stride_h == 1 && d->stride_w == 1 && back_h >= 0 && back_w >= 0 && d->n * d->oh * d->ow * p->co_pad * es < ((int64_t)1 << 31)) {
+    pml_hip_conv2d_desc c = *d;
+    c.h = d->oh, c.w = d->ow, c.ci = p->co_pad, c.co = d->ci, c.oh = d->h, c.ow = d->w;
+    c.pad_h = back_h, c.pad_w = back_w;
+    c.c_dtype = d->in_dtype;
+    p->sub = (Plan*)(intptr_t)pml_hip_conv2d_dispatch(&c);
+    if (!p->sub) {
+      delete p;
+      return 0;
+    }
+    p->sub->packed = true;  // (every invoke lays the filter out itself)
+    if (p->co_pad != d->co && hipMalloc(&p->padded, (size_t)(d->n * d->oh * d->ow * p->co_pad * es)) != hipSuccess) {
+      delete p;
+      fail("conv2d_grad: cannot allocate the padded gradient");
+      return 0;
+    }
+    p->text = "conv2d data gradient as a convolution of the gradient: " + p->sub->text;
+    return (int64_t)(intptr_t)p;
+  }
+  // Larger strides: every gradient pixel's product with the whole filter, cols[pixel][ky][kx][ci] in fp32, then a pass
+  // that adds the columns up into the image.  (A convolution over the gradient spread out with zeros would multiply
+  // stride^2 times as much.)  Columns are made for as many images at a time as fit 256 MiB.
+  const int64_t taps_ci = d->kh * d->kw * d->ci, per_image = d->oh * d->ow * taps_ci * 4;
+  p->grad_chunk = std::max<int64_t>(1, std::min<int64_t>(d->n, ((int64_t)256 << 20) / per_image));
+  a.M = p->grad_chunk * d->oh * d->ow;
+  a.N = taps_ci;
+  a.K = d->co;
+  a.a_ms = d->co;
+  a.a_ks = 1;
+  a.b_ks = 1;
+  a.b_ns = d->co;
+  a.c_ms = taps_ci;
+  if (hipMalloc(&p->cols, (size_t)(p->grad_chunk * per_image)) != hipSuccess) {
+    delete p;
+    fail("conv2d_grad: cannot allocate the columns");
+    return 0;
+  }
+  if (!prepare_strided(p)) {
+    delete p;
+    return 0;
+  }
+  std::snprintf(buf, sizeof buf, "conv2d data gradient %s by columns: product m=%lld n=%lld k=%lld tile=%dx%d splits=%d, %lld images at a time", bf ? "bf16" : "f32",
+                (long long)a.M, (long long)a.N, (long long)a.K, 64 * p->strided_mi, 64 * p->strided_mi, a.splits, (long long)p->grad_chunk);
+  p->text = buf;
+  return (int64_t)(intptr_t)p;
+}
+
+int pml_hip_conv2d_grad_invoke(int64_t plan, const void* g, const void* other, void* result, pml_hip_stream s) {
+  Plan* p = (Plan*)(intptr_t)plan;
+  if (!p || p->kind != PLAN_CONV_GRAD) return fail("conv2d_grad_invoke: not a gradient plan");
+  if (!g || !other || !result) return fail("conv2d_grad_invoke: null operand");
+  const pml_hip_conv2d_desc& d = p->conv;
+  const int es = p->strided_bf ? 2 : 4;
+  hipStream_t st = (hipStream_t)s;
+  if (p->grad_which == 1) {
+    StridedArgs a = p->strided;
+    a.A = other;
+    a.B = g;
+    a.C = result;
+    return check(strided_launch(a, p->strided_bf, true, p->strided_mi, st), "strided_launch");
+  }
+  if (p->sub) {
+    const void* in = g;
+    if (p->padded) {
+      if (check(pad_rows_launch(es, g, p->padded, d.n * d.oh * d.ow, d.co, p->co_pad, st), "pad_rows_launch")) return 1;
+      in = p->padded;
+    }
+    if (check(flip_filter_launch(es, other, p->sub->bt, d.kh * d.kw, d.ci, d.co, p->co_pad, st), "flip_filter_launch")) return 1;
+    return pml_hip_conv2d_invoke((int64_t)(intptr_t)p->sub, in, nullptr, result, nullptr, nullptr, nullptr, s);
+  }
+  const int64_t g_step = d.oh * d.ow * d.co * es, r_step = d.h * d.w * d.ci * es;
+  for (int64_t i = 0; i < d.n; i += p->grad_chunk) {
+    const int64_t cnt = std::min<int64_t>(p->grad_chunk, d.n - i);
+    StridedArgs a = p->strided;
+    a.A = (const char*)g + i * g_step;
+    a.B = other;
+    a.C = p->cols;
+    if (cnt != p->grad_chunk) {  // (a last, shorter run: its rows past the end would be another image's)
+      a.M = cnt * d.oh * d.ow;
+      a.tiles_m = (int)((a.M + 64 * p->strided_mi - 1) / (64 * p->strided_mi));
+      a.ws_rows = a.M;
+    }
+    if (check(strided_launch(a, p->strided_bf, false, p->strided_mi, st), "strided_launch")) return 1;
+    Col2imArgs c;
+    c.cols = (const float*)p->cols;
+    c.out = (char*)result + i * r_step;
+    c.N = (int)cnt, c.H = (int)d.h, c.W = (int)d.w, c.CI = (int)d.ci, c.OH = (int)d.oh, c.OW = (int)d.ow, c.KH = (int)d.kh, c.KW = (int)d.kw;
+    c.SH = (int)d.stride_h, c.SW = (int)d.stride_w, c.PH = (int)d.pad_h, c.PW = (int)d.pad_w, c.DH = (int)d.dil_h, c.DW = (int)d.dil_w;
+    if (check(col2im_launch(c, p->strided_bf, st), "col2im_launch")) return 1;
+  }
+  return 0;
+}
+
+// ---------------------------------------------------------------------------
 // depthwise conv, pooling
 // ---------------------------------------------------------------------------
 
@@ -1648,6 +1951,7 @@ size_t pml_hip_struct_size(int which) {
     case 10: return sizeof(pml_hip_scatter_desc);
     case 11: return sizeof(pml_hip_argsort_desc);
     case 12: return sizeof(pml_hip_softmax_desc);
+    case 13: return sizeof(pml_hip_product_desc);
   }
   return 0;
 }

@@ -1,0 +1,640 @@
+// Matrix products over free strides: batched products, products whose rows are no whole 16-byte vectors, products of
+// transposed operands, and the filter gradient of a convolution, all on the matrix cores.
+//
+// igemm.hip streams K-contiguous, 16-byte aligned rows straight into LDS; what it cannot address comes here.  Operands
+// pass through registers on their way to LDS, which costs a few vector instructions per 16 bytes but takes any
+// alignment (global loads of 8 and 16 bytes need none on this target) and any of three layouts per operand:
+//   ROWS_K     row m (column n) of the operand is contiguous along K
+//   ROWS_M     row k is contiguous along m (n), or has a free element stride there
+//   ROWS_CONV  (left-hand side of a filter gradient) row k is an output pixel; its elements are the kw * ci
+//              neighbouring values of one filter row's window, which lie contiguously in an NHWC image (dilation 1)
+// A workgroup of four wavefronts owns a tile of 64 MI x 64 NI results, each wavefront a quarter as MI x NI blocks of
+// 32 x 32.  K goes by in slabs of 32 (fp32) or 64 (bf16) values, double-buffered in LDS: the next slab's global loads
+// are in flight while the current one is multiplied, one barrier per slab.
+//   fp32: LDS holds [k][m]; a lane reads one word per operand and MFMA (v_mfma_f32_32x32x2_f32), 32 neighbouring
+//         words per half wavefront.
+//   bf16: LDS holds [m][k], 128 bytes a row, the 16-byte chunk c of row m at slot c ^ key(m): both the transposed
+//         8-byte stores of a ROWS_M operand (lanes step m by 4) and the 16-byte fragment reads (lanes step m by 1)
+//         then meet all banks (v_mfma_f32_32x32x16_bf16).
+// Few tiles and a long K (a filter gradient: 9 tiles of 50176 pixels at 16 x 56 x 56 x 64): the K loop is split over
+// workgroups, partial tiles go to a workspace and a second launch adds them in a fixed order and runs the tail.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+
+#include "device_common.h"
+#include "plans.h"
+
+namespace pml {
+namespace {
+
+enum { ROWS_K = 0, ROWS_M = 1, ROWS_CONV = 2 };
+constexpr int kThreads = 256;
+
+template <int N>
+struct Words {
+  uint32_t w[N];
+};
+
+// N 32-bit words from an address of any alignment
+template <int N>
+__device__ __forceinline__ Words<N> load_words(const void* p) {
+  Words<N> v;
+  __builtin_memcpy(&v, p, sizeof v);
+  return v;
+}
+
+// The tail on four neighbouring results of one row: the contraction's value rounded to the result type, then each step
+// in that type.  `row_at`: the row's element offset in the result.
+__device__ __forceinline__ void strided_tail(const StridedArgs& p, float (&v)[4], int64_t row_at, int64_t col, int live) {
+  const bool bf = p.out_bf16;
+  auto rnd = [&](float x) { return bf ? round_to_bf16(x) : x; };
+  auto fetch = [&](const void* base, int64_t at) { return bf ? bf16_bits_to_f32(((const uint16_t*)base)[at]) : ((const float*)base)[at]; };
+  const int64_t row = (p.init != nullptr || p.n_ops > 0) ? row_at / p.row_len : 0;
+  if (p.init) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      if (q < live) v[q] += fetch(p.init, row * p.init_rs + (col + q) * p.init_cs);
+  }
+#pragma unroll
+  for (int q = 0; q < 4; ++q) v[q] = rnd(v[q]);
+  for (int s = 0; s < p.n_ops; ++s) {
+    const StridedOp& op = p.ops[s];
+    float x[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) x[q] = op.ptr ? (q < live ? fetch(op.ptr, row * op.rs + (col + q) * op.cs) : 0.f) : op.imm;
+#define PML_EACH(EXPR)                                                            \
+  _Pragma("unroll") for (int q = 0; q < 4; ++q) {                                 \
+    const float a = v[q], b = x[q];                                               \
+    v[q] = rnd(EXPR);                                                             \
+  }                                                                               \
+  break;
+    switch (op.opcode) {
+      case PML_HIP_EPI_ADD: PML_EACH(a + b)
+      case PML_HIP_EPI_SUB: PML_EACH(a - b)
+      case PML_HIP_EPI_RSUB: PML_EACH(b - a)
+      case PML_HIP_EPI_MUL: PML_EACH(a * b)
+      case PML_HIP_EPI_DIV: PML_EACH(a / b)
+      case PML_HIP_EPI_RDIV: PML_EACH(b / a)
+      case PML_HIP_EPI_MAX: PML_EACH((a < b) ? b : a)
+      case PML_HIP_EPI_MIN: PML_EACH((a < b) ? a : b)
+      case PML_HIP_EPI_RELU: PML_EACH((a < 0.f) ? 0.f : a)
+      case PML_HIP_EPI_NEG: PML_EACH(-a)
+      case PML_HIP_EPI_MAX_GT: PML_EACH((a > b) ? a : b)
+      default: break;
+    }
+#undef PML_EACH
+  }
+}
+
+__device__ __forceinline__ void store_results(const StridedArgs& p, void* c, int64_t at, const float (&v)[4], int live) {
+  if (p.out_bf16) {
+    uint16_t h[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) h[q] = f32_to_bf16_bits(v[q]);
+    uint16_t* const to = (uint16_t*)c + at;
+    if (live == 4) {
+      __builtin_memcpy(to, h, 8);
+    } else {
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        if (q < live) to[q] = h[q];
+    }
+  } else {
+    float* const to = (float*)c + at;
+    if (live == 4) {
+      __builtin_memcpy(to, v, 16);
+    } else {
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        if (q < live) to[q] = v[q];
+    }
+  }
+}
+
+// One operand's share of a workgroup: T rows (of m or n) by one slab of K.
+//   fetch(k0): the slab's values of this thread, into registers;   put(lds): from there into the slab's LDS buffer
+template <bool BF, int MODE, int T>
+struct Side {
+  static constexpr int BK = BF ? 64 : 32;
+  static constexpr int kPitch = BF ? 0 : (MODE == ROWS_K ? T + 1 : T + 4);  // fp32: words per K-row
+  static constexpr int kBytes = BF ? T * 128 : (BK * kPitch * 4 + 15) / 16 * 16;
+  static constexpr int kPasses = T / 32;  // fp32, and bf16 ROWS_K: 16-byte chunks per thread
+  static constexpr int kBlocks = T / 64;  // bf16 ROWS_M: blocks of 4 x 4 values per thread
+  const char* base;     // the tile's first row, K-index 0 (ROWS_CONV: the image)
+  int64_t ms, ks;       // element strides
+  int64_t live;         // rows of the tile that exist
+  bool whole;           // every row exists and is contiguous where the layout says so
+  uint32_t regs[BF ? (MODE == ROWS_K ? kPasses * 4 : kBlocks * 8) : kPasses * 4];
+
+  __device__ __forceinline__ static int key(int m) { return (m ^ (m >> 2)) & 7; }
+
+  // `n` values from element `at` on, those at or past `live_n` as zeros; st: their element stride
+  template <int N>
+  __device__ __forceinline__ void gather(uint32_t* to, int64_t at, int64_t live_n, int64_t st) {
+    if constexpr (BF) {
+      uint16_t h[N];
+#pragma unroll
+      for (int e = 0; e < N; ++e) h[e] = e < live_n ? ((const uint16_t*)base)[at + e * st] : (uint16_t)0;
+      __builtin_memcpy(to, h, 2 * N);
+    } else {
+#pragma unroll
+      for (int e = 0; e < N; ++e) to[e] = e < live_n ? ((const uint32_t*)base)[at + e * st] : 0u;
+    }
+  }
+  template <int N>
+  __device__ __forceinline__ void straight(uint32_t* to, int64_t at) {
+    constexpr int W = N * (BF ? 2 : 4) / 4;
+    const Words<W> v = load_words<W>(base + at * (BF ? 2 : 4));
+#pragma unroll
+    for (int e = 0; e < W; ++e) to[e] = v.w[e];
+  }
+  template <int N>
+  __device__ __forceinline__ void checked(uint32_t* to, int64_t at, int64_t live_n, int64_t st) {
+    if (live_n >= N && st == 1)
+      straight<N>(to, at);
+    else
+      gather<N>(to, at, live_n, st);
+  }
+
+  // N neighbouring values of pixel k's window row, the first at column j0 of the tile
+  template <int N>
+  __device__ __forceinline__ void conv_row(const StridedArgs& p, uint32_t* to, int64_t k, int64_t k_end, int j0) {
+    constexpr int W = N * (BF ? 2 : 4) / 4;
+#pragma unroll
+    for (int e = 0; e < W; ++e) to[e] = 0;
+    if (k >= k_end) return;
+    const unsigned pix = (unsigned)k;
+    const unsigned img = fast_div(pix, p.div_per_magic, p.div_per_shift);
+    const unsigned rem = pix - img * (unsigned)(p.OH * p.OW);
+    const unsigned oy = fast_div(rem, p.div_ow_magic, p.div_ow_shift);
+    const int ox = (int)(rem - oy * (unsigned)p.OW);
+    const int iy = (int)oy * p.SH + (int)ms * p.DH - p.PH;
+    if (iy < 0 || iy >= p.H) return;
+    const int first = (ox * p.SW - p.PW) * p.CI + (int)ks + j0;  // (ks: the tile's first column inside the window row)
+    const int row_elems = p.W * p.CI;
+    const int64_t at = ((int64_t)img * p.H + iy) * row_elems + first;
+    if (j0 + N <= live && first >= 0 && first + N <= row_elems) {
+      straight<N>(to, at);
+    } else {
+      if constexpr (BF) {
+        uint16_t h[N];
+#pragma unroll
+        for (int e = 0; e < N; ++e)
+          h[e] = (j0 + e < live && first + e >= 0 && first + e < row_elems) ? ((const uint16_t*)base)[at + e] : (uint16_t)0;
+        __builtin_memcpy(to, h, 2 * N);
+      } else {
+#pragma unroll
+        for (int e = 0; e < N; ++e)
+          to[e] = (j0 + e < live && first + e >= 0 && first + e < row_elems) ? ((const uint32_t*)base)[at + e] : 0u;
+      }
+    }
+  }
+
+  __device__ __forceinline__ void fetch(const StridedArgs& p, int64_t k0, int64_t k_end, int tid) {
+    const bool full = whole && k0 + BK <= k_end;  // uniform: no lane checks anything
+    if constexpr (MODE == ROWS_K) {
+      constexpr int N = BF ? 8 : 4;
+#pragma unroll
+      for (int i = 0; i < kPasses; ++i) {
+        const int row = tid / 8 + 32 * i, kq = (tid % 8) * N;
+        const int64_t at = row * ms + (k0 + kq) * ks;
+        if (full)
+          straight<N>(&regs[4 * i], at);
+        else
+          checked<N>(&regs[4 * i], at, row < live ? k_end - k0 - kq : 0, ks);
+      }
+    } else if constexpr (!BF) {
+      constexpr int PER = T / 4;
+#pragma unroll
+      for (int i = 0; i < kPasses; ++i) {
+        const int c = tid + kThreads * i, k = c / PER, m4 = (c % PER) * 4;
+        if constexpr (MODE == ROWS_CONV) {
+          conv_row<4>(p, &regs[4 * i], k0 + k, k_end, m4);
+        } else {
+          const int64_t at = (k0 + k) * ks + m4 * ms;
+          if (full)
+            straight<4>(&regs[4 * i], at);
+          else
+            checked<4>(&regs[4 * i], at, k0 + k < k_end ? live - m4 : 0, ms);
+        }
+      }
+    } else {
+      constexpr int PER = T / 4;  // blocks of four columns
+#pragma unroll
+      for (int i = 0; i < kBlocks; ++i) {
+        const int c = tid + kThreads * i, k4 = (c / PER) * 4, m4 = (c % PER) * 4;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          if constexpr (MODE == ROWS_CONV) {
+            conv_row<4>(p, &regs[8 * i + 2 * e], k0 + k4 + e, k_end, m4);
+          } else {
+            const int64_t at = (k0 + k4 + e) * ks + m4 * ms;
+            if (full)
+              straight<4>(&regs[8 * i + 2 * e], at);
+            else
+              checked<4>(&regs[8 * i + 2 * e], at, k0 + k4 + e < k_end ? live - m4 : 0, ms);
+          }
+        }
+      }
+    }
+  }
+
+  __device__ __forceinline__ void put(char* lds, int tid) const {
+    if constexpr (BF && MODE == ROWS_K) {
+#pragma unroll
+      for (int i = 0; i < kPasses; ++i) {
+        const int row = tid / 8 + 32 * i, c = tid % 8;
+        *(i32x4_t*)(lds + row * 128 + ((c ^ key(row)) * 16)) =
+            i32x4_t{(int)regs[4 * i], (int)regs[4 * i + 1], (int)regs[4 * i + 2], (int)regs[4 * i + 3]};
+      }
+    } else if constexpr (BF) {
+      constexpr int PER = T / 4;
+#pragma unroll
+      for (int i = 0; i < kBlocks; ++i) {
+        const int c = tid + kThreads * i, k4 = c / PER, m4 = (c % PER) * 4;
+        const uint32_t* r = &regs[8 * i];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          // value e of the four K-rows
+          const unsigned sel = (e & 1) ? 0x07060302u : 0x05040100u;
+          const int h = e >> 1;
+          const uint2 w = make_uint2(__builtin_amdgcn_perm(r[2 + h], r[h], sel), __builtin_amdgcn_perm(r[6 + h], r[4 + h], sel));
+          const int m = m4 + e;
+          *(uint2*)(lds + m * 128 + (((k4 >> 1) ^ key(m)) * 16) + (k4 & 1) * 8) = w;
+        }
+      }
+    } else if constexpr (MODE == ROWS_K) {
+#pragma unroll
+      for (int i = 0; i < kPasses; ++i) {
+        const int row = tid / 8 + 32 * i, kq = (tid % 8) * 4;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) *(uint32_t*)(lds + ((kq + e) * kPitch + row) * 4) = regs[4 * i + e];
+      }
+    } else {
+      constexpr int PER = T / 4;
+#pragma unroll
+      for (int i = 0; i < kPasses; ++i) {
+        const int c = tid + kThreads * i, k = c / PER, m4 = (c % PER) * 4;
+        *(i32x4_t*)(lds + (k * kPitch + m4) * 4) = i32x4_t{(int)regs[4 * i], (int)regs[4 * i + 1], (int)regs[4 * i + 2], (int)regs[4 * i + 3]};
+      }
+    }
+  }
+};
+
+template <bool BF, int AMODE, int BMODE, int MI, int NI>
+__global__ __launch_bounds__(kThreads) void strided_kernel(StridedArgs p_by_value) {
+  // (read where the dispatcher put it: indexing a by-value copy would move the copy to scratch memory)
+  const StridedArgs& p = *(const StridedArgs*)(const __attribute__((address_space(4))) void*)__builtin_amdgcn_kernarg_segment_ptr();
+  constexpr int TM = 64 * MI, TN = 64 * NI, ES = BF ? 2 : 4;
+  typedef Side<BF, AMODE, TM> side_a;
+  typedef Side<BF, BMODE, TN> side_b;
+  constexpr int BK = side_a::BK, kStage = side_a::kBytes + side_b::kBytes;
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave >> 1, wn = wave & 1;
+
+  unsigned t = blockIdx.x;
+  const int tn = (int)(t % (unsigned)p.tiles_n);
+  t /= (unsigned)p.tiles_n;
+  const int tm = (int)(t % (unsigned)p.tiles_m);
+  t /= (unsigned)p.tiles_m;
+  int64_t a_at = 0, b_at = 0, c_at = 0;
+  const unsigned batch = t;
+  for (int d = p.n_batch - 1; d >= 0; --d) {
+    const unsigned sz = (unsigned)p.batch[d], i = t % sz;
+    t /= sz;
+    a_at += i * p.a_batch[d];
+    b_at += i * p.b_batch[d];
+    c_at += i * p.c_batch[d];
+  }
+  int64_t m0, m_rows;  // first result row of the tile, rows it has
+  side_a sa;
+  side_b sb;
+  if constexpr (AMODE == ROWS_CONV) {
+    // tiles of one filter row's window columns after those of the row before it
+    const int tap = tm / p.tiles_per_tap, j0 = (tm - tap * p.tiles_per_tap) * TM;
+    m0 = (int64_t)tap * p.row_cols + j0;
+    m_rows = p.row_cols - j0 < TM ? p.row_cols - j0 : TM;
+    sa.base = (const char*)p.A;
+    sa.ks = j0;
+    sa.ms = tap;  // (the filter row)
+    sa.live = m_rows;
+    sa.whole = false;
+  } else {
+    m0 = (int64_t)tm * TM;
+    m_rows = p.M - m0 < TM ? p.M - m0 : TM;
+    sa.base = (const char*)p.A + (a_at + m0 * p.a_ms) * ES;
+    sa.ms = p.a_ms;
+    sa.ks = p.a_ks;
+    sa.live = m_rows;
+    sa.whole = m_rows == TM && (AMODE == ROWS_K ? p.a_ks : p.a_ms) == 1;
+  }
+  const int64_t n0 = (int64_t)tn * TN;
+  const int64_t n_cols = p.N - n0 < TN ? p.N - n0 : TN;
+  sb.base = (const char*)p.B + (b_at + n0 * p.b_ns) * ES;
+  sb.ms = p.b_ns;
+  sb.ks = p.b_ks;
+  sb.live = n_cols;
+  sb.whole = n_cols == TN && (BMODE == ROWS_K ? p.b_ks : p.b_ns) == 1;
+
+  const int64_t k_begin = (int64_t)blockIdx.y * p.k_per_split;
+  const int64_t k_end = k_begin + p.k_per_split < p.K ? k_begin + p.k_per_split : p.K;
+
+  f32x16_t acc[MI][NI];
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int j = 0; j < NI; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+
+  sa.fetch(p, k_begin, k_end, tid);
+  sb.fetch(p, k_begin, k_end, tid);
+  sa.put(smem, tid);
+  sb.put(smem + side_a::kBytes, tid);
+  __syncthreads();
+  int stage = 0;
+  const int row = lane & 31, half = lane >> 5;
+  for (int64_t k = k_begin; k < k_end; k += BK) {
+    const bool more = k + BK < k_end;
+    if (more) {
+      sa.fetch(p, k + BK, k_end, tid);
+      sb.fetch(p, k + BK, k_end, tid);
+    }
+    const char* la = smem + stage * kStage;
+    const char* lb = la + side_a::kBytes;
+    if constexpr (BF) {
+#pragma unroll
+      for (int kk = 0; kk < 4; ++kk) {
+        bf16x8_t fa[MI], fb[NI];
+#pragma unroll
+        for (int i = 0; i < MI; ++i) {
+          const int m = (wm * MI + i) * 32 + row;
+          fa[i] = *(const bf16x8_t*)(la + m * 128 + (((kk * 2 + half) ^ side_a::key(m)) * 16));
+        }
+#pragma unroll
+        for (int j = 0; j < NI; ++j) {
+          const int n = (wn * NI + j) * 32 + row;
+          fb[j] = *(const bf16x8_t*)(lb + n * 128 + (((kk * 2 + half) ^ side_b::key(n)) * 16));
+        }
+        // (the right-hand fragment is the row operand: a lane then holds one result row m = lane % 32 and in it the
+        // columns 8 (r / 4) + 4 (lane / 32) + r % 4 -- runs of four)
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+          for (int j = 0; j < NI; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[j], fa[i], acc[i][j], 0, 0, 0);
+      }
+    } else {
+#pragma unroll
+      for (int kk = 0; kk < BK / 2; ++kk) {
+        float fa[MI], fb[NI];
+#pragma unroll
+        for (int i = 0; i < MI; ++i) fa[i] = *(const float*)(la + ((kk * 2 + half) * side_a::kPitch + (wm * MI + i) * 32 + row) * 4);
+#pragma unroll
+        for (int j = 0; j < NI; ++j) fb[j] = *(const float*)(lb + ((kk * 2 + half) * side_b::kPitch + (wn * NI + j) * 32 + row) * 4);
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+          for (int j = 0; j < NI; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fb[j], fa[i], acc[i][j], 0, 0, 0);
+      }
+    }
+    stage ^= 1;
+    if (more) {
+      sa.put(smem + stage * kStage, tid);
+      sb.put(smem + stage * kStage + side_a::kBytes, tid);
+    }
+    __syncthreads();
+  }
+
+  // The tile goes through LDS once, so that a row's results leave in runs of 16 (8) bytes per lane and the tail is one
+  // small loop over them.
+  float* const ctile = (float*)smem;
+  constexpr int CS = TN + 4;
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int j = 0; j < NI; ++j)
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        *(f32x4_t*)&ctile[((wm * MI + i) * 32 + row) * CS + (wn * NI + j) * 32 + 8 * g + 4 * half] =
+            f32x4_t{acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
+  __syncthreads();
+  const int lc = (tid % (TN / 4)) * 4;
+  if (lc >= n_cols) return;
+  const int live = n_cols - lc < 4 ? (int)(n_cols - lc) : 4;
+  const int64_t n = n0 + lc;
+  for (int lr = tid / (TN / 4); lr < m_rows; lr += kThreads / (TN / 4)) {
+    const int64_t m = m0 + lr;
+    const f32x4_t w = *(const f32x4_t*)&ctile[lr * CS + lc];
+    if (p.ws != nullptr) {
+      // (rows of the workspace are whole 16-byte vectors)
+      *(f32x4_t*)(p.ws + (((int64_t)blockIdx.y * p.ws_rows + (int64_t)batch * p.M + m) * p.ws_pitch + n)) = w;
+    } else {
+      float v[4] = {w[0], w[1], w[2], w[3]};
+      const int64_t at = c_at + m * p.c_ms;
+      strided_tail(p, v, at, n, live);
+      store_results(p, p.C, at + n, v, live);
+    }
+  }
+}
+
+// Adds the partial results up in split order and runs the tail: a thread per four columns of a row.
+__global__ __launch_bounds__(256) void strided_reduce_kernel(StridedArgs p_by_value) {
+  const StridedArgs& p = *(const StridedArgs*)(const __attribute__((address_space(4))) void*)__builtin_amdgcn_kernarg_segment_ptr();
+  const int64_t per_row = p.ws_pitch / 4;
+  const int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (g >= p.ws_rows * per_row) return;
+  const int64_t row = g / per_row, n = (g - row * per_row) * 4;
+  const f32x4_t* at = (const f32x4_t*)(p.ws + row * p.ws_pitch + n);
+  const int64_t step = p.ws_rows * p.ws_pitch / 4;
+  f32x4_t sum = {0.f, 0.f, 0.f, 0.f};
+  for (int s = 0; s < p.splits; s += 8) {
+    f32x4_t got[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) got[u] = s + u < p.splits ? at[(s + u) * step] : f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int u = 0; u < 8; ++u) sum += got[u];
+  }
+  float v[4] = {sum[0], sum[1], sum[2], sum[3]};
+  int64_t b = row / p.M, c_at = (row - b * p.M) * p.c_ms;
+  for (int d = p.n_batch - 1; d >= 0; --d) {
+    c_at += (b % p.batch[d]) * p.c_batch[d];
+    b /= p.batch[d];
+  }
+  const int live = p.N - n < 4 ? (int)(p.N - n) : 4;
+  strided_tail(p, v, c_at, n, live);
+  store_results(p, p.C, c_at + n, v, live);
+}
+
+template <bool BF, int AMODE, int BMODE, int MI, int NI>
+hipError_t launch_tile(const StridedArgs& a, hipStream_t s) {
+  const size_t lds = std::max<size_t>(2 * (Side<BF, AMODE, 64 * MI>::kBytes + Side<BF, BMODE, 64 * NI>::kBytes), 64 * MI * (64 * NI + 4) * 4);
+  auto kern = strided_kernel<BF, AMODE, BMODE, MI, NI>;
+  static DynamicLdsLimit limit;
+  if (hipError_t e = limit.ensure((const void*)kern, lds); e != hipSuccess) return e;
+  int64_t nb = (int64_t)a.tiles_m * a.tiles_n;
+  for (int d = 0; d < a.n_batch; ++d) nb *= a.batch[d];
+  hipLaunchKernelGGL(kern, dim3((unsigned)nb, (unsigned)a.splits), dim3(kThreads), lds, s, a);
+  return hipGetLastError();
+}
+
+template <bool BF, int MI>
+hipError_t launch_modes(const StridedArgs& a, int amode, int bmode, hipStream_t s) {
+  if (amode == ROWS_CONV) return launch_tile<BF, ROWS_CONV, ROWS_M, MI, MI>(a, s);
+  if (amode == ROWS_K) return bmode == ROWS_K ? launch_tile<BF, ROWS_K, ROWS_K, MI, MI>(a, s) : launch_tile<BF, ROWS_K, ROWS_M, MI, MI>(a, s);
+  return bmode == ROWS_K ? launch_tile<BF, ROWS_M, ROWS_K, MI, MI>(a, s) : launch_tile<BF, ROWS_M, ROWS_M, MI, MI>(a, s);
+}
+
+}  // namespace
+// The tile and, for few tiles and a long K, the split: 128 x 128 where that still gives every CU a workgroup (half the
+// operand traffic per result), 64 x 64 otherwise; K is split when the tiles alone leave CUs idle, into runs of at least
+// four slabs, for about three workgroups per CU (their LDS fits four times into one).
+void strided_plan(StridedArgs* a, bool bf, bool conv, int n_cus, int* mi) {
+  int64_t batches = 1;
+  for (int d = 0; d < a->n_batch; ++d) batches *= a->batch[d];
+  const int64_t bk = bf ? 64 : 32, slabs = (a->K + bk - 1) / bk;
+  auto tiles = [&](int64_t t) {
+    const int64_t rows = conv ? (a->M / a->row_cols) * ((a->row_cols + t - 1) / t) : (a->M + t - 1) / t;
+    return rows * ((a->N + t - 1) / t) * batches;
+  };
+  *mi = tiles(128) >= n_cus ? 2 : 1;
+  const int64_t t = 64 * *mi;
+  a->tiles_per_tap = conv ? (int)((a->row_cols + t - 1) / t) : 1;
+  a->tiles_m = conv ? (int)(a->M / a->row_cols) * a->tiles_per_tap : (int)((a->M + t - 1) / t);
+  a->tiles_n = (int)((a->N + t - 1) / t);
+  a->splits = 1;
+  a->k_per_split = slabs * bk;
+  a->ws_rows = batches * a->M;
+  a->ws_pitch = (a->N + 3) / 4 * 4;
+  const int64_t have = tiles(t);
+  if (have < n_cus && slabs >= 8) {
+    int64_t want = std::min<int64_t>((3 * n_cus + have - 1) / have, slabs / 4);
+    // the partial results: at most 256 MiB of them
+    want = std::min<int64_t>(want, ((int64_t)256 << 20) / std::max<int64_t>(1, a->ws_rows * a->ws_pitch * 4));
+    if (want >= 2) {
+      const int64_t per = (slabs + want - 1) / want;
+      a->k_per_split = per * bk;
+      a->splits = (int)((slabs + per - 1) / per);
+    }
+  }
+}
+
+hipError_t strided_launch(const StridedArgs& a, bool bf, bool conv, int mi, hipStream_t s) {
+  int64_t nb = (int64_t)a.tiles_m * a.tiles_n;
+  for (int d = 0; d < a.n_batch; ++d) nb *= a.batch[d];
+  if (nb <= 0 || nb >= ((int64_t)1 << 31) || a.splits < 1 || a.splits > 65535 || (a.splits > 1) != (a.ws != nullptr)) return hipErrorInvalidValue;
+  const int amode = conv ? ROWS_CONV : (a.a_ks == 1 ? ROWS_K : ROWS_M), bmode = a.b_ks == 1 && !conv ? ROWS_K : ROWS_M;
+  hipError_t e;
+  if (bf)
+    e = mi == 2 ? launch_modes<true, 2>(a, amode, bmode, s) : launch_modes<true, 1>(a, amode, bmode, s);
+  else
+    e = mi == 2 ? launch_modes<false, 2>(a, amode, bmode, s) : launch_modes<false, 1>(a, amode, bmode, s);
+  if (e != hipSuccess || a.splits == 1) return e;
+  const int64_t groups = a.ws_rows * (a.ws_pitch / 4), blocks = (groups + 255) / 256;
+  if (blocks >= ((int64_t)1 << 31)) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(strided_reduce_kernel, dim3((unsigned)blocks), dim3(256), 0, s, a);
+  return hipGetLastError();
+}
+
+namespace {
+
+// The columns of a strided convolution's data gradient, cols[pixel of the gradient][ky][kx][ci] in fp32, added up into
+// the image: an image value takes the columns of every tap and gradient pixel whose window covers it, taps in order.
+// A thread per V channels of an image pixel; columns are read once, V * 4 bytes at a time.
+template <bool BF, int V>
+__global__ __launch_bounds__(256) void col2im_kernel(Col2imArgs a) {
+  const int64_t per_img = (int64_t)a.H * a.W * a.CI / V;
+  const int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (g >= per_img * a.N) return;
+  const int64_t img = g / per_img;
+  const unsigned rem = (unsigned)(g - img * per_img), cv = (unsigned)(a.CI / V);
+  const int c = (int)(rem % cv) * V, pix = (int)(rem / cv), y = pix / a.W, x = pix % a.W;
+  float sum[V];
+#pragma unroll
+  for (int e = 0; e < V; ++e) sum[e] = 0.f;
+  for (int ky = 0; ky < a.KH; ++ky) {
+    const int ty = y + a.PH - ky * a.DH;
+    if (ty < 0 || ty % a.SH != 0 || ty / a.SH >= a.OH) continue;
+    for (int kx = 0; kx < a.KW; ++kx) {
+      const int tx = x + a.PW - kx * a.DW;
+      if (tx < 0 || tx % a.SW != 0 || tx / a.SW >= a.OW) continue;
+      const float* at = a.cols + (((img * a.OH + ty / a.SH) * a.OW + tx / a.SW) * (a.KH * a.KW) + ky * a.KW + kx) * a.CI + c;
+      const Words<V> w = load_words<V>(at);
+#pragma unroll
+      for (int e = 0; e < V; ++e) sum[e] += __uint_as_float(w.w[e]);
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < V; ++e) {
+    const int64_t o = g * V + e;
+    if constexpr (BF)
+      ((uint16_t*)a.out)[o] = f32_to_bf16_bits(sum[e]);
+    else
+      ((float*)a.out)[o] = sum[e];
+  }
+}
+
+// Rows of `cols` elements copied to rows of `pitch` elements, the rest of a row zeros.
+template <typename T>
+__global__ __launch_bounds__(256) void pad_rows_kernel(const T* in, T* out, int64_t rows, int cols, int pitch) {
+  const int64_t stride = (int64_t)gridDim.x * 256, total = rows * pitch;
+  for (int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x; g < total; g += stride) {
+    const int64_t row = g / pitch;
+    const int c = (int)(g - row * pitch);
+    out[g] = c < cols ? in[row * cols + c] : (T)0;
+  }
+}
+
+// Bt[ci][tap][pitch] = F[taps - 1 - tap][ci][co]: the filter of a data gradient seen as a convolution of the gradient,
+// taps in reverse and the channels' roles exchanged; already contiguous along what that convolution sums over.
+template <typename T>
+__global__ __launch_bounds__(256) void flip_filter_kernel(const T* f, T* bt, int taps, int ci, int co, int pitch) {
+  const int64_t total = (int64_t)ci * taps * co;
+  const int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (g >= total) return;
+  const int c = (int)(g % co);
+  const int64_t r = g / co;
+  const int tap = (int)(r % taps), n = (int)(r / taps);
+  bt[((int64_t)n * taps + tap) * pitch + c] = f[((int64_t)(taps - 1 - tap) * ci + n) * co + c];
+}
+
+}  // namespace
+
+hipError_t col2im_launch(const Col2imArgs& a, bool bf, hipStream_t s) {
+  const int v = a.CI % 4 == 0 ? 4 : 1;
+  const int64_t blocks = ((int64_t)a.N * a.H * a.W * a.CI / v + 255) / 256;
+  if (blocks <= 0 || blocks >= ((int64_t)1 << 31)) return hipErrorInvalidValue;
+  const dim3 grid((unsigned)blocks), block(256);
+  if (bf) {
+    if (v == 4) hipLaunchKernelGGL((col2im_kernel<true, 4>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((col2im_kernel<true, 1>), grid, block, 0, s, a);
+  } else {
+    if (v == 4) hipLaunchKernelGGL((col2im_kernel<false, 4>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((col2im_kernel<false, 1>), grid, block, 0, s, a);
+  }
+  return hipGetLastError();
+}
+
+hipError_t pad_rows_launch(int es, const void* in, void* out, int64_t rows, int64_t cols, int64_t pitch, hipStream_t s) {
+  if (rows * pitch == 0) return hipSuccess;
+  const unsigned blocks = (unsigned)std::min<int64_t>((rows * pitch + 255) / 256, 256 * 32);
+  if (es == 2)
+    hipLaunchKernelGGL(pad_rows_kernel<uint16_t>, dim3(blocks), dim3(256), 0, s, (const uint16_t*)in, (uint16_t*)out, rows, (int)cols, (int)pitch);
+  else
+    hipLaunchKernelGGL(pad_rows_kernel<uint32_t>, dim3(blocks), dim3(256), 0, s, (const uint32_t*)in, (uint32_t*)out, rows, (int)cols, (int)pitch);
+  return hipGetLastError();
+}
+
+hipError_t flip_filter_launch(int es, const void* f, void* bt, int64_t taps, int64_t ci, int64_t co, int64_t pitch, hipStream_t s) {
+  const int64_t blocks = (taps * ci * co + 255) / 256;
+  if (blocks <= 0 || blocks >= ((int64_t)1 << 31)) return hipErrorInvalidValue;
+  if (es == 2)
+    hipLaunchKernelGGL(flip_filter_kernel<uint16_t>, dim3((unsigned)blocks), dim3(256), 0, s, (const uint16_t*)f, (uint16_t*)bt, (int)taps, (int)ci, (int)co, (int)pitch);
+  else
+    hipLaunchKernelGGL(flip_filter_kernel<uint32_t>, dim3((unsigned)blocks), dim3(256), 0, s, (const uint32_t*)f, (uint32_t*)bt, (int)taps, (int)ci, (int)co, (int)pitch);
+  return hipGetLastError();
+}
+
+}  // namespace pml

@@ -54,6 +54,8 @@ EXPORTS = [
     'pml_hip_conv2d_dispatch', 'pml_hip_conv2d_invoke', 'pml_hip_dwconv2d_dispatch', 'pml_hip_dwconv2d_invoke',
     'pml_hip_pool2d_dispatch', 'pml_hip_pool2d_invoke', 'pml_hip_eltwise_dispatch', 'pml_hip_eltwise_invoke',
     'pml_hip_select', 'pml_hip_softmax', 'pml_hip_index', 'pml_hip_contract_dispatch', 'pml_hip_contract_invoke', 'pml_hip_plan_free',
+    'pml_hip_product_dispatch', 'pml_hip_product_takes_tail', 'pml_hip_product_invoke', 'pml_hip_conv2d_grad_takes',
+    'pml_hip_conv2d_grad_dispatch', 'pml_hip_conv2d_grad_invoke',
     'pml_hip_plan_describe', 'pml_hip_struct_size', 'pml_hip_gemm_pack_b', 'pml_hip_conv2d_pack_filter', 'pml_hip_conv2d_takes_maxpool',
     'pml_hip_gather', 'pml_hip_scatter', 'pml_hip_argsort', 'pml_hip_prng',
 ]
@@ -77,6 +79,14 @@ class GemmDesc(ctypes.Structure):
                 ('init_col_stride', i64), ('c_dtype', i32), ('b_layout', i32), ('tail', Epilogue),
                 ('k2', i64), ('lda2', i64), ('ldb2', i64), ('a2_stride', i32), ('init2_kind', i32),
                 ('a2_h', i64), ('a2_w', i64), ('a2_oh', i64), ('a2_ow', i64), ('flags', i32), ('reserved', i32)]
+
+
+class ProductDesc(ctypes.Structure):
+    _fields_ = [('in_dtype', i32), ('out_dtype', i32), ('n_batch', i32), ('init_kind', i32),
+                ('batch', i64 * 3), ('a_batch', i64 * 3), ('b_batch', i64 * 3), ('c_batch', i64 * 3),
+                ('m', i64), ('n', i64), ('k', i64),
+                ('a_ms', i64), ('a_ks', i64), ('b_ks', i64), ('b_ns', i64), ('c_ms', i64), ('row_len', i64),
+                ('init_row_stride', i64), ('init_col_stride', i64), ('tail', Epilogue)]
 
 
 class Conv2dDesc(ctypes.Structure):
@@ -195,6 +205,14 @@ def lib():
         L.pml_hip_softmax.argtypes = [ctypes.POINTER(SoftmaxDesc), vp, vp, vp]
         L.pml_hip_index.argtypes = [vp, i32, ctypes.POINTER(i64), i32, vp]
         L.pml_hip_contract_invoke.argtypes = [ctypes.c_int64, pp, vp, vp]
+        L.pml_hip_product_dispatch.restype = ctypes.c_int64
+        L.pml_hip_product_dispatch.argtypes = [ctypes.POINTER(ProductDesc)]
+        L.pml_hip_product_takes_tail.argtypes = [ctypes.POINTER(Epilogue), ctypes.c_int]
+        L.pml_hip_product_invoke.argtypes = [ctypes.c_int64, vp, vp, vp, vp, pp, vp]
+        L.pml_hip_conv2d_grad_takes.argtypes = [ctypes.POINTER(Conv2dDesc), ctypes.c_int]
+        L.pml_hip_conv2d_grad_dispatch.restype = ctypes.c_int64
+        L.pml_hip_conv2d_grad_dispatch.argtypes = [ctypes.POINTER(Conv2dDesc), ctypes.c_int]
+        L.pml_hip_conv2d_grad_invoke.argtypes = [ctypes.c_int64, vp, vp, vp, vp]
         L.pml_hip_plan_free.argtypes = [ctypes.c_int64]
         L.pml_hip_plan_describe.argtypes = [ctypes.c_int64, ctypes.c_char_p, sz]
         L.pml_hip_struct_size.restype = sz

@@ -265,6 +265,8 @@ void Planner::emitContraction(size_t i) {
   if (opt_.specialise && !emptyBox(op)) {
     if (tryGemm(i)) return;
     if (tryConv(i)) return;
+    if (tryConvGrad(i)) return;
+    if (tryProduct(i)) return;
     if (tryDepthwise(i)) return;
     if (tryPool(i)) return;
     if (tryGlobalPool(i)) return;

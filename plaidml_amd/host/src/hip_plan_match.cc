@@ -334,6 +334,239 @@ bool Planner::tryConv(size_t i) {
   return true;
 }
 
+// The gradients of a convolution (plaidml/op/lib/ops.cc:1342-1450, deriv_mode):
+//   data     O[n, s*y + d*ky - p, s*x + d*kx - p, ci] += G[n,y,x,co] * F[ky,kx,ci,co]
+//   filter   O[ky,kx,ci,co] += I[n, s*y + d*ky - p, s*x + d*kx - p, ci] * G[n,y,x,co]
+// over the whole of G and F (taps that leave the image are left out).  Both are the forward convolution's index set with
+// another tensor as the result; indices of range 1 have been folded to the constant 0.
+bool Planner::tryConvGrad(size_t i) {
+  const Op& op = prog_->ops[i];
+  if (op.agg != AggKind::add || op.combo != ComboKind::mul || op.operands.size() != 2 || op.init || !op.constraints.empty()) return false;
+  const DataType dt = op.result->shape.elementType;
+  if ((dt != DataType::f32 && dt != DataType::bf16) || op.operands[0]->shape.elementType != dt || op.operands[1]->shape.elementType != dt) return false;
+  const TensorShape* sh[3] = {&op.result->shape, &op.operands[0]->shape, &op.operands[1]->shape};
+  for (const TensorShape* s : sh)
+    if (s->getRank() != 4) return false;
+  const Normalised n = normalise(op);
+  // the access of dimension k of tensor t as a plain index over its whole extent; -1: folded; -2: neither
+  auto plain = [&](size_t t, size_t k) {
+    const Affine& a = n.acc[t][k];
+    if (a.den != 1) return -2;
+    if (sh[t]->sizes[k] == 1 && a.isConstant() && a.c0 == 0) return -1;
+    const int v = a.plainIndex();
+    return v >= 0 && op.lower[v] == 0 && op.upper[v] == sh[t]->sizes[k] - 1 ? v : -2;
+  };
+  for (int which = 0; which < 2; ++which) {
+    // the tensors in the roles of image, gradient and filter
+    const size_t I = which ? 1 : 0, G = which ? 2 : 1, F = which ? 0 : 2;
+    int g[4], f[4], seen = 0;
+    bool ok = true;
+    std::set<int> roles;
+    for (size_t k = 0; k < 4 && ok; ++k) {
+      g[k] = plain(G, k);
+      f[k] = plain(F, k);
+      ok = g[k] != -2 && f[k] != -2;
+    }
+    if (!ok || g[3] != f[3] || sh[G]->sizes[3] != sh[F]->sizes[3]) continue;
+    const int in_n = plain(I, 0), in_c = plain(I, 3);
+    if (in_n == -2 || in_c == -2 || in_n != g[0] || in_c != f[2] || sh[I]->sizes[0] != sh[G]->sizes[0] || sh[I]->sizes[3] != sh[F]->sizes[2]) continue;
+    for (int v : {g[0], g[1], g[2], g[3], f[0], f[1], f[2]})
+      if (v >= 0) {
+        roles.insert(v);
+        ++seen;
+      }
+    if (static_cast<int>(roles.size()) != seen) continue;  // seven different indices, less the folded ones
+    for (size_t v = 0; v < n.nIdx; ++v) ok = ok && (!n.active[v] || roles.count(static_cast<int>(v)));
+    int64_t stride[2] = {1, 1}, dil[2] = {1, 1}, pad[2] = {0, 0};
+    for (int d = 0; d < 2 && ok; ++d) {
+      const Affine& a = n.acc[I][1 + d];
+      ok = a.den == 1;
+      pad[d] = -a.c0;
+      for (size_t v = 0; v < a.coef.size() && ok; ++v) {
+        if (!a.coef[v]) continue;
+        if (static_cast<int>(v) == g[1 + d]) stride[d] = a.coef[v];
+        else if (static_cast<int>(v) == f[d]) dil[d] = a.coef[v];
+        else ok = false;
+      }
+      ok = ok && (g[1 + d] < 0 || a.coef[g[1 + d]] > 0) && (f[d] < 0 || a.coef[f[d]] > 0);
+    }
+    if (!ok) continue;
+    Step s;
+    s.kind = Step::ConvGrad;
+    s.grad_which = which;
+    pml_hip_conv2d_desc& d = s.conv;
+    d.in_dtype = d.out_dtype = d.c_dtype = hipType(dt);
+    d.n = sh[I]->sizes[0];
+    d.h = sh[I]->sizes[1];
+    d.w = sh[I]->sizes[2];
+    d.ci = sh[I]->sizes[3];
+    d.kh = sh[F]->sizes[0];
+    d.kw = sh[F]->sizes[1];
+    d.co = sh[F]->sizes[3];
+    d.oh = sh[G]->sizes[1];
+    d.ow = sh[G]->sizes[2];
+    d.stride_h = stride[0];
+    d.stride_w = stride[1];
+    d.dil_h = dil[0];
+    d.dil_w = dil[1];
+    d.pad_h = pad[0];
+    d.pad_w = pad[1];
+    if (!pml_hip_conv2d_grad_takes(&d, which)) return false;
+    s.a = bufferFor(op.operands[G - 1]);
+    s.b = bufferFor(op.operands[(which ? I : F) - 1]);
+    s.c = bufferFor(op.result);
+    s.flops = 2.0 * d.n * d.oh * d.ow * d.kh * d.kw * d.ci * d.co;
+    s.bytes = static_cast<double>(sh[0]->elements() + sh[1]->elements() + sh[2]->elements()) * util::byteSize(dt);
+    std::stringstream ss;
+    ss << "conv2d " << (which ? "filter" : "data") << " gradient " << util::mnemonic(dt) << " " << sh[1]->str() << ", " << sh[2]->str() << " stride=" << d.stride_h
+       << "x" << d.stride_w << " pad=" << d.pad_h << "," << d.pad_w << " -> " << sh[0]->str();
+    s.text = ss.str();
+    plan_->steps.push_back(s);
+    return true;
+  }
+  return false;
+}
+
+// A multiply-add contraction whose indices fall into batch (in all three tensors), row, column and summed groups, each
+// group one flat index with an element stride per tensor: what tryGemm leaves -- batches, transposed operands, rows that
+// are no whole 16-byte vectors.
+bool Planner::tryProduct(size_t i) {
+  const Op& op = prog_->ops[i];
+  if (op.agg != AggKind::add || op.combo != ComboKind::mul || op.operands.size() != 2 || !op.constraints.empty()) return false;
+  const DataType dt = op.result->shape.elementType;
+  if ((dt != DataType::f32 && dt != DataType::bf16) || op.operands[0]->shape.elementType != dt || op.operands[1]->shape.elementType != dt) return false;
+  // (operands of 2 GiB and more stay with the general kernel, as they do for the other matrix-core kernels)
+  for (const ValuePtr& v : op.operands)
+    if (v->shape.getByteSize() >= size_t(1) << 31) return false;
+  const Normalised n = normalise(op);
+  const TensorShape* sh[3] = {&op.result->shape, &op.operands[0]->shape, &op.operands[1]->shape};
+  std::vector<int64_t> st[3];
+  int64_t base[3];
+  for (size_t t = 0; t < 3; ++t) {
+    if (!indexStrides(n.acc[t], *sh[t], &st[t], &base[t])) return false;
+    for (size_t d = 0; d < n.acc[t].size(); ++d)
+      if (!impliedByBox(op, n.acc[t][d], sh[t]->sizes[d])) return false;
+  }
+  // an index that walks two dimensions of a tensor (a diagonal) still has one stride; negative strides stay general
+  struct Group {
+    int64_t range, s[3];  // strides in result, left, right
+  };
+  std::vector<Group> M, N, K, B;
+  for (size_t v = 0; v < n.nIdx; ++v) {
+    if (!n.active[v]) continue;
+    if (op.lower[v] != 0) return false;
+    Group g{op.upper[v] + 1, {st[0][v], st[1][v], st[2][v]}};
+    if (g.s[0] < 0 || g.s[1] < 0 || g.s[2] < 0) return false;
+    const bool o = g.s[0] != 0, a = g.s[1] != 0, b = g.s[2] != 0;
+    if (o && a && b) B.push_back(g);
+    else if (o && a) M.push_back(g);
+    else if (o && b) N.push_back(g);
+    else if (!o && a && b) K.push_back(g);
+    else return false;
+  }
+  if (K.empty()) return false;
+  // neighbours (in the order of one tensor's strides) become one index where every stride allows it
+  auto merge = [](std::vector<Group>& g, int by) {
+    std::sort(g.begin(), g.end(), [&](const Group& x, const Group& y) { return x.s[by] > y.s[by]; });
+    for (size_t k = 0; k + 1 < g.size();) {
+      bool join = true;
+      for (int t = 0; t < 3; ++t) join = join && g[k].s[t] == g[k + 1].s[t] * g[k + 1].range;
+      if (!join) {
+        ++k;
+        continue;
+      }
+      g[k + 1].range *= g[k].range;
+      g.erase(g.begin() + static_cast<long>(k));
+    }
+  };
+  merge(M, 0);
+  merge(N, 0);
+  merge(B, 0);
+  merge(K, 1);
+  if (M.size() > 1 || N.size() > 1 || K.size() != 1 || B.size() > 3) return false;
+  Group m{1, {0, 0, 0}}, nn{1, {1, 0, 1}};
+  if (!M.empty()) m = M[0];
+  if (!N.empty()) nn = N[0];
+  // the result's columns have to be contiguous; where the rows are, the operands change places
+  bool swapped = false;
+  if (nn.s[0] != 1) {
+    if (M.empty() || m.s[0] != 1) return false;
+    std::swap(m, nn);
+    std::swap(m.s[1], m.s[2]);
+    std::swap(nn.s[1], nn.s[2]);
+    swapped = true;
+  } else if (N.empty() && m.s[0] == 1 && m.range > 1) {
+    // matrix times vector: the vector as the one row, so that the results are columns of it
+    std::swap(m, nn);
+    std::swap(m.s[1], m.s[2]);
+    std::swap(nn.s[1], nn.s[2]);
+    m.s[0] = nn.range;
+    swapped = true;
+  }
+  int64_t all = m.range * nn.range;
+  for (const Group& g : B) all *= g.range;
+  if (base[0] != 0 || all != op.result->shape.elements()) return false;
+  Step s;
+  s.kind = Step::Product;
+  pml_hip_product_desc& d = s.prod;
+  const int L = swapped ? 2 : 1, R = swapped ? 1 : 2;
+  d.in_dtype = d.out_dtype = hipType(dt);
+  d.m = m.range;
+  d.n = nn.range;
+  d.k = K[0].range;
+  d.a_ms = m.s[1];
+  d.a_ks = K[0].s[L];
+  d.b_ns = nn.s[2];
+  d.b_ks = K[0].s[R];
+  d.c_ms = M.empty() && !swapped ? nn.range : m.s[0];
+  if (m.range == 1) d.c_ms = nn.range;
+  d.n_batch = static_cast<int32_t>(B.size());
+  for (size_t k = 0; k < B.size(); ++k) {
+    d.batch[k] = B[k].range;
+    d.a_batch[k] = B[k].s[L];
+    d.b_batch[k] = B[k].s[R];
+    d.c_batch[k] = B[k].s[0];
+  }
+  // rows and columns as the tail sees them: the result's last dimension is the columns
+  bool rows_ok = op.result->shape.getRank() >= 1 && op.result->shape.sizes.back() == nn.range && (m.range == 1 || d.c_ms % nn.range == 0);
+  for (const Group& g : B) rows_ok = rows_ok && g.s[0] % nn.range == 0;
+  d.row_len = nn.range;
+  if (op.init) {
+    int32_t idt = 0;
+    if (!rows_ok || op.init->kind == Value::Literal || op.init->shape.elementType != dt) return false;
+    if (!denseInit(op, &d.init_kind, &idt, &d.init_row_stride, &d.init_col_stride, &s.init)) return false;
+  }
+  TailBuild tb;
+  tb.final_value = op.result;
+  tb.final_dtype = dt;
+  if (rows_ok) {
+    extendTail(&tb, op.result, i, /*two_d=*/true, /*allow64=*/false);
+    if (!tb.outs.empty() || tb.final_dtype != dt || !pml_hip_product_takes_tail(&tb.tail, hipType(dt))) {
+      unconsume(tb);
+      tb = TailBuild();
+      tb.final_value = op.result;
+      tb.final_dtype = dt;
+    }
+  }
+  d.tail = tb.tail;
+  s.a = bufferFor(op.operands[static_cast<size_t>(L - 1)]);
+  s.b = bufferFor(op.operands[static_cast<size_t>(R - 1)]);
+  s.a_off = base[L];
+  s.b_off = base[R];
+  s.c = bufferFor(tb.final_value);
+  attachTail(&s, tb);
+  s.flops = 2.0 * static_cast<double>(all) * d.k;
+  s.bytes = static_cast<double>(sh[0]->elements() + sh[1]->elements() + sh[2]->elements()) * util::byteSize(dt);
+  std::stringstream ss;
+  ss << "product " << util::mnemonic(dt);
+  for (const Group& g : B) ss << " batch=" << g.range;
+  ss << " m=" << d.m << " n=" << d.n << " k=" << d.k << " A strides " << d.a_ms << "," << d.a_ks << " B strides " << d.b_ks << "," << d.b_ns
+     << (d.init_kind ? " +init" : "") << tailText(tb) << " -> " << tb.final_value->shape.str();
+  s.text = ss.str();
+  plan_->steps.push_back(s);
+  return true;
+}
+
 // out[n,y,x,c] += I[n, sy*y + dy*ky - py, sx*x + dx*kx - px, c] * F[ky,kx,c,0]
 bool Planner::tryDepthwise(size_t i) {
   const Op& op = prog_->ops[i];

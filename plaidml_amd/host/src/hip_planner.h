@@ -214,6 +214,8 @@ class Planner {
   static bool sameIndex(const Affine& a, int idx) { return idx >= 0 ? a.plainIndex() == idx : (a.isConstant() && a.c0 == 0); }
 
   bool tryConv(size_t i);
+  bool tryConvGrad(size_t i);
+  bool tryProduct(size_t i);
   bool tryDepthwise(size_t i);
   bool poolGeometry(const Op& op, const Normalised& n, pml_hip_pool2d_desc* d, Spatial* sy, Spatial* sx);
   bool tryGlobalPool(size_t i);

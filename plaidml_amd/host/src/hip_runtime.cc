@@ -76,7 +76,7 @@ class HipExecutable final : public Executable {
       for (const Step& s : plan_->steps)
         if (s.kind != Step::Gemm && s.kind != Step::Conv2d && s.kind != Step::Dwconv2d && s.kind != Step::Pool2d &&
             s.kind != Step::Eltwise && s.kind != Step::Contract && s.kind != Step::Select && s.kind != Step::Copy &&
-            s.kind != Step::Softmax)
+            s.kind != Step::Softmax && s.kind != Step::Product && s.kind != Step::ConvGrad)
           graphable_ = false;
     } catch (...) {
       release();
@@ -313,6 +313,8 @@ class HipExecutable final : public Executable {
       case Step::Pool2d: h = pml_hip_pool2d_dispatch(&s.pool); break;
       case Step::Eltwise: h = pml_hip_eltwise_dispatch(&s.elt); break;
       case Step::Contract: h = pml_hip_contract_dispatch(&s.con); break;
+      case Step::Product: h = pml_hip_product_dispatch(&s.prod); break;
+      case Step::ConvGrad: h = pml_hip_conv2d_grad_dispatch(&s.conv, s.grad_which); break;
       case Step::Select:
       case Step::Index:
       case Step::Gather:
@@ -384,6 +386,14 @@ class HipExecutable final : public Executable {
         break;
       case Step::Contract:
         hipCheck(pml_hip_contract_invoke(handles_[i], operands, ptr(s.c), stream_), s.text.c_str());
+        break;
+      case Step::Product:
+        hipCheck(pml_hip_product_invoke(handles_[i], ptr(s.a, s.a_off, elemSize(s.prod.in_dtype)), ptr(s.b, s.b_off, elemSize(s.prod.in_dtype)),
+                                        ptr(s.c), ptr(s.init), operands, stream_),
+                 s.text.c_str());
+        break;
+      case Step::ConvGrad:
+        hipCheck(pml_hip_conv2d_grad_invoke(handles_[i], ptr(s.a), ptr(s.b), ptr(s.c), stream_), s.text.c_str());
         break;
       case Step::Copy:
         hipCheck(pml_hip_memcpy_d2d(ptr(s.c), ptr(s.a), s.copy_bytes, stream_), s.text.c_str());

@@ -1,0 +1,68 @@
+"""Products over free strides and the gradients of a convolution (csrc/strided.hip) against float64 on the CPU, at the sizes where
+tiles, slabs, splits and 16-byte vectors end raggedly."""
+import numpy as np
+import pytest
+import torch
+
+from plaidml_amd import edsl as P
+from plaidml_amd import op as Pop
+
+pytestmark = pytest.mark.gpu
+DT = {'f32': P.DType.FLOAT32, 'bf16': P.DType.BFLOAT16}
+
+
+def values(rng, shape, dtype, scale=1.0):
+    a = rng.standard_normal(shape).astype(np.float32) * np.float32(scale)
+    return P.round_bf16(a) if dtype == 'bf16' else a
+
+
+def check(got, want, dtype):
+    err = np.linalg.norm(got - want) / max(np.linalg.norm(want), 1e-30)
+    assert np.isfinite(got).all() and err < (6e-3 if dtype == 'bf16' else 2e-6), err
+
+
+def plan_of(program):
+    return [v for k, v in program.passes if k == 'hip-plan'][0]
+
+
+@pytest.mark.parametrize('dtype', ['f32', 'bf16'])
+@pytest.mark.parametrize('b,m,n,k,ta,tb', [
+    (1, 1, 1, 2, 0, 0), (1, 300, 777, 1001, 0, 0), (3, 64, 64, 64, 0, 1), (5, 65, 31, 33, 0, 0), (2, 127, 129, 100, 1, 0),
+    (7, 19, 276, 32, 0, 1), (1, 130, 70, 5003, 1, 0), (2, 3, 5, 7, 1, 1), (1, 1100, 2051, 67, 0, 0), (4, 1, 33, 130, 0, 1)])
+def test_product(dtype, b, m, n, k, ta, tb):
+    rng = np.random.default_rng(m * 7 + n)
+    A, B = values(rng, (b, k, m) if ta else (b, m, k), dtype), values(rng, (b, n, k) if tb else (b, k, n), dtype, k ** -0.5)
+    bias = values(rng, (n,), dtype)
+    X, Y, Z = (P.Placeholder(DT[dtype], x.shape) for x in (A, B, bias))
+    bi, i, j, q = P.TensorIndexes(4)
+    C = P.Contraction().outShape(b, m, n).outAccess(bi, i, j).sum((X[bi, q, i] if ta else X[bi, i, q]) * (Y[bi, j, q] if tb else Y[bi, q, j])).build()
+    program = P.Program('product', [X, Y, Z], [Pop.relu(C * 0.5 + Z)])
+    got, = P.Runner(program, target='hip').run([A, B, bias])
+    want = np.matmul((A.transpose(0, 2, 1) if ta else A).astype(np.float64), (B.transpose(0, 2, 1) if tb else B).astype(np.float64))
+    check(got, np.maximum(want * 0.5 + bias, 0), dtype)
+    assert 'general' not in plan_of(program)
+
+
+@pytest.mark.parametrize('dtype', ['f32', 'bf16'])
+@pytest.mark.parametrize('n,hw,ci,co,k,stride', [
+    (2, 14, 64, 64, 3, 1), (1, 7, 3, 16, 3, 2), (3, 9, 19, 33, 5, 1), (2, 15, 70, 20, 3, 2), (1, 10, 5, 17, 1, 2), (2, 8, 24, 40, 1, 1),
+    (1, 112, 3, 37, 5, 1), (5, 11, 130, 65, 3, 1), (1, 2, 8, 16, 3, 1), (4, 40, 16, 24, 5, 2)])
+def test_conv_gradients(dtype, n, hw, ci, co, k, stride):
+    rng = np.random.default_rng(hw * 3 + co)
+    o = (hw + stride - 1) // stride
+    Iv, Fv, Gv = values(rng, (n, hw, hw, ci), dtype), values(rng, (k, k, ci, co), dtype, (k * k * co) ** -0.5), values(rng, (n, o, o, co), dtype)
+    X, F, G = (P.Placeholder(DT[dtype], x.shape) for x in (Iv, Fv, Gv))
+    dX = Pop.convolution(G, F, strides=[stride, stride], deriv_mode=Pop.DERIV_DATA, result_shape=[hw, hw])
+    dF = Pop.convolution(X, G, strides=[stride, stride], deriv_mode=Pop.DERIV_FILTER, result_shape=[k, k])
+    program = P.Program('gradients', [X, F, G], [dX, dF])
+    runner = P.Runner(program, target='hip')
+    for _ in range(4):  # one by one, then as a recorded graph
+        gx, gf = runner.run([Iv, Fv, Gv])
+    before = max(0, (o - 1) * stride + k - hw) // 2
+    x = torch.nn.functional.pad(torch.from_numpy(Iv).double().permute(0, 3, 1, 2), (before, k + stride, before, k + stride)).requires_grad_(True)
+    f = torch.from_numpy(Fv).double().permute(3, 2, 0, 1).requires_grad_(True)
+    y = torch.nn.functional.conv2d(x, f, stride=stride)[:, :, :o, :o]
+    y.backward(torch.from_numpy(Gv).double().permute(0, 3, 1, 2))
+    check(gx, x.grad[:, :, before:before + hw, before:before + hw].permute(0, 2, 3, 1).numpy(), dtype)
+    check(gf, f.grad.permute(2, 3, 1, 0).numpy(), dtype)
+    assert 'general' not in plan_of(program)
