@@ -71,6 +71,12 @@ int pml_hip_host_free(void* hptr);
 int pml_hip_memcpy_h2d(void* dst, const void* src, size_t nbytes, pml_hip_stream s);
 int pml_hip_memcpy_d2h(void* dst, const void* src, size_t nbytes, pml_hip_stream s);
 int pml_hip_memcpy_d2d(void* dst, const void* src, size_t nbytes, pml_hip_stream s);
+/* The same without waiting: host memory must be page-locked and stay untouched until the stream has passed the copy. */
+int pml_hip_memcpy_h2d_async(void* dst, const void* src, size_t nbytes, pml_hip_stream s);
+int pml_hip_memcpy_d2h_async(void* dst, const void* src, size_t nbytes, pml_hip_stream s);
+/* n copies between device and page-locked host memory (any direction) by one kernel: for a few hundred kilobytes the
+ * copy engines' set-up and hand-over to the compute queue cost more than the transfer. */
+int pml_hip_copy_spans(int n, void* const* dst, const void* const* src, const size_t* nbytes, pml_hip_stream s);
 /* Fills with a 32-bit pattern using a kernel (safe to capture into a graph). */
 int pml_hip_fill_u32(void* dptr, uint32_t pattern, size_t n_words, pml_hip_stream s);
 

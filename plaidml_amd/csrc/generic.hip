@@ -702,6 +702,26 @@ __global__ __launch_bounds__(256) void fill_kernel(uint32_t* p, uint32_t pattern
   for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) p[i] = pattern;
 }
 
+// Up to kMaxSpans copies, blockIdx.y the span: 16 bytes a thread, four in flight (a read over the link takes about 2 us),
+// any alignment.  Memory on either side may be page-locked memory of the host.
+__global__ __launch_bounds__(256) void copy_spans_kernel(SpanArgs a) {
+  const unsigned char* src = (const unsigned char*)a.src[blockIdx.y];
+  unsigned char* dst = (unsigned char*)a.dst[blockIdx.y];
+  const size_t n_vec = a.bytes[blockIdx.y] / 16, stride = (size_t)gridDim.x * 256;
+  const size_t first = (size_t)blockIdx.x * 256 + threadIdx.x;
+  constexpr int U = 4;
+  for (size_t g0 = first; g0 < n_vec; g0 += U * stride) {
+    i32x4_t v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (g0 + u * stride < n_vec) __builtin_memcpy(&v[u], src + (g0 + u * stride) * 16, 16);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (g0 + u * stride < n_vec) __builtin_memcpy(dst + (g0 + u * stride) * 16, &v[u], 16);
+  }
+  for (size_t i = n_vec * 16 + first; i < a.bytes[blockIdx.y]; i += stride) dst[i] = src[i];
+}
+
 inline unsigned grid_for(int64_t work_items) {
   int64_t blocks = (work_items + 255) / 256;
   if (blocks < 1) blocks = 1;
@@ -961,6 +981,16 @@ hipError_t softmax_launch(const pml_hip_softmax_desc& d, const void* x, void* y,
     hipLaunchKernelGGL(softmax_rows_kernel<true>, dim3((unsigned)d.rows), dim3(256), 0, s, x, y, d.cols);
   else
     hipLaunchKernelGGL(softmax_rows_kernel<false>, dim3((unsigned)d.rows), dim3(256), 0, s, x, y, d.cols);
+  return hipGetLastError();
+}
+
+hipError_t copy_spans_launch(const SpanArgs& a, hipStream_t s) {
+  if (a.n <= 0) return hipSuccess;
+  size_t most = 0;
+  for (int i = 0; i < a.n; ++i) most = most < a.bytes[i] ? a.bytes[i] : most;
+  size_t blocks = (most / 16 + 4 * 256 - 1) / (4 * 256);
+  blocks = blocks < 1 ? 1 : blocks > 64 ? 64 : blocks;
+  hipLaunchKernelGGL(copy_spans_kernel, dim3((unsigned)blocks, (unsigned)a.n), dim3(256), 0, s, a);
   return hipGetLastError();
 }
 

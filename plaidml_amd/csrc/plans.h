@@ -263,6 +263,14 @@ hipError_t eltwise_launch(const EltwiseArgs& a, hipStream_t s);
 hipError_t select_launch(const pml_hip_select_desc& d, const void* c, const void* t, const void* f, void* out,
                          hipStream_t s);
 hipError_t index_launch(void* out, int rank, const int64_t* sizes, int axis, hipStream_t s);
+constexpr int kMaxSpans = 16;
+struct SpanArgs {
+  void* dst[kMaxSpans];
+  const void* src[kMaxSpans];
+  size_t bytes[kMaxSpans];
+  int n;
+};
+hipError_t copy_spans_launch(const SpanArgs& a, hipStream_t s);
 hipError_t fill_u32_launch(void* p, uint32_t pattern, size_t n_words, hipStream_t s);
 hipError_t softmax_launch(const pml_hip_softmax_desc& d, const void* x, void* y, hipStream_t s);
 

@@ -571,6 +571,28 @@ int pml_hip_memcpy_d2d(void* dst, const void* src, size_t nbytes, pml_hip_stream
   if (nbytes == 0) return 0;
   return check(hipMemcpyAsync(dst, src, nbytes, hipMemcpyDeviceToDevice, (hipStream_t)s), "hipMemcpyAsync(d2d)");
 }
+int pml_hip_memcpy_h2d_async(void* dst, const void* src, size_t nbytes, pml_hip_stream s) {
+  return nbytes ? check(hipMemcpyAsync(dst, src, nbytes, hipMemcpyHostToDevice, (hipStream_t)s), "hipMemcpyAsync(h2d)") : 0;
+}
+int pml_hip_memcpy_d2h_async(void* dst, const void* src, size_t nbytes, pml_hip_stream s) {
+  return nbytes ? check(hipMemcpyAsync(dst, src, nbytes, hipMemcpyDeviceToHost, (hipStream_t)s), "hipMemcpyAsync(d2h)") : 0;
+}
+int pml_hip_copy_spans(int n, void* const* dst, const void* const* src, const size_t* nbytes, pml_hip_stream s) {
+  if (n < 0 || (n > 0 && (!dst || !src || !nbytes))) return fail("copy_spans: bad argument");
+  for (int i = 0; i < n; i += kMaxSpans) {
+    SpanArgs a;
+    std::memset(&a, 0, sizeof a);
+    for (int j = i; j < n && j < i + kMaxSpans; ++j) {
+      if (nbytes[j] == 0) continue;
+      if (!dst[j] || !src[j]) return fail("copy_spans: null pointer");
+      a.dst[a.n] = dst[j];
+      a.src[a.n] = src[j];
+      a.bytes[a.n++] = nbytes[j];
+    }
+    if (check(copy_spans_launch(a, (hipStream_t)s), "copy_spans_launch")) return 1;
+  }
+  return 0;
+}
 int pml_hip_fill_u32(void* dptr, uint32_t pattern, size_t n_words, pml_hip_stream s) {
   return check(fill_u32_launch(dptr, pattern, n_words, (hipStream_t)s), "fill");
 }

@@ -17,7 +17,7 @@ import numpy as np
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, 'lib', 'libplaidml.so')
 
-vp, sz, i64, f64 = ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int64, ctypes.c_double
+vp, sz, i32, i64, f64 = ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int32, ctypes.c_int64, ctypes.c_double
 
 
 class Error(ctypes.Structure):
@@ -98,7 +98,8 @@ _SIGS = {
 # the two functions that take no plaidml_error, and the statistics helper
 EXPORTS = sorted(list(_SIGS) + ['plaidml_string_ptr', 'plaidml_string_free', 'plaidml_hip_last_run_stats',
                                'plaidml_hip_last_run_memory', 'plaidml_hip_last_run_step_ms', 'plaidml_hip_last_run_replayed',
-                               'plaidml_hip_last_run_graph_note'])
+                               'plaidml_hip_last_run_graph_note', 'plaidml_hip_executable_run_arrays', 'plaidml_hip_host_alloc',
+                               'plaidml_hip_host_free', 'plaidml_hip_executable_download'])
 
 _lib = None
 
@@ -128,6 +129,14 @@ def lib():
         L.plaidml_hip_last_run_graph_note.restype = ctypes.c_char_p
         L.plaidml_hip_last_run_graph_note.argtypes = []
         L.plaidml_hip_last_run_step_ms.argtypes = [sz, ctypes.POINTER(f64)]
+        L.plaidml_hip_executable_run_arrays.restype = f64
+        L.plaidml_hip_executable_run_arrays.argtypes = [ctypes.POINTER(Error), vp, sz, vp, vp, vp, sz, vp, vp, vp]
+        L.plaidml_hip_executable_download.restype = None
+        L.plaidml_hip_executable_download.argtypes = [ctypes.POINTER(Error), vp, sz, vp]
+        L.plaidml_hip_host_alloc.restype = vp
+        L.plaidml_hip_host_alloc.argtypes = [sz]
+        L.plaidml_hip_host_free.restype = None
+        L.plaidml_hip_host_free.argtypes = [vp]
         _lib = L
         call('plaidml_init')
         call('plaidml_edsl_init')
@@ -983,6 +992,30 @@ def round_bf16(a):
     return from_bf16_bits(to_bf16_bits(a))
 
 
+class _ResultMemory:
+    """Memory of one result array, given back to the library's pool when the last array over it goes."""
+    __slots__ = ('__array_interface__', '_ptr')
+
+    def __init__(self, ptr, dtype, sizes):
+        self._ptr = ptr
+        self.__array_interface__ = {'data': (ptr, False), 'shape': sizes, 'typestr': dtype.str, 'version': 3}
+
+    def __del__(self):
+        try:
+            _lib.plaidml_hip_host_free(self._ptr)
+        except Exception:
+            pass
+
+
+def _result_array(dtype, sizes, nbytes):
+    # small results come through the executable's own staging; large ones land in page-locked memory directly
+    if nbytes >= 32768:
+        ptr = _lib.plaidml_hip_host_alloc(nbytes)
+        if ptr:
+            return np.asarray(_ResultMemory(ptr, dtype, sizes))
+    return np.empty(sizes, dtype)
+
+
 class Runner:
     """Compiles once, then runs with numpy arrays (reference: plaidml/exec/__init__.py:49-63).
     bfloat16 inputs are given as float32 arrays (rounded on the way in) and returned as float32."""
@@ -993,7 +1026,32 @@ class Runner:
         self.exe = Executable(program, device)
         self.in_shapes = program.inputs
         self.out_shapes = program.outputs
-        self.outputs = [Buffer(s) for s in self.out_shapes]
+        self._outputs = None
+        self._behind = False  # the last run's results are on the device and not in self._outputs
+        self._in = [self._layout(s) for s in self.in_shapes]
+        self._out = [self._layout(s) for s in self.out_shapes]
+        n, m = builtins.max(1, len(self._in)), builtins.max(1, len(self._out))
+        self._args = ((vp * n)(), (sz * n)(), (i32 * n)(), (vp * m)(), (sz * m)(), (i32 * m)())
+        for i, (dt, sizes, nbytes, bf16) in enumerate(self._out):
+            self._args[4][i], self._args[5][i] = nbytes, bf16
+
+    @staticmethod
+    def _layout(shape):
+        """(numpy type, sizes, bytes) of a value's array on the caller's side, and whether it stands for bfloat16"""
+        bf16 = shape.dtype == DType.BFLOAT16
+        dt = np.dtype(np.float32 if bf16 else shape.dtype.into_numpy())
+        sizes = tuple(shape.sizes)
+        return dt, sizes, dt.itemsize * int(np.prod(sizes, dtype=np.int64)), bf16
+
+    @property
+    def outputs(self):
+        """The buffers run_staged() writes, holding the results of the last run of either kind."""
+        if self._outputs is None:
+            self._outputs = [Buffer(s) for s in self.out_shapes]
+        if self._behind:
+            self._behind = False
+            call('plaidml_hip_executable_download', self.exe.as_ptr(), len(self._outputs), _ptr_array([b.as_ptr() for b in self._outputs]))
+        return self._outputs
 
     def _converted(self, inputs):
         for shape, a in zip(self.in_shapes, inputs):
@@ -1015,12 +1073,31 @@ class Runner:
 
     def run_staged(self, bufs):
         """One run over staged inputs; results stay in self.outputs until fetch().  Returns the wall ms."""
+        self._behind = False
         self.ms = self.exe.run(bufs, self.outputs)
         return self.ms
 
     def run(self, inputs):
-        self.ms = self.exe.run([Buffer(shape, data=a) for shape, a in self._converted(inputs)], self.outputs)
-        return self.fetch()
+        # One call into the library, which rounds to and from bfloat16 and moves the arrays itself.  Inputs are passed
+        # where they lie if they lie contiguously in the value's type; the results are arrays of their own.
+        in_ptr, in_bytes, in_f32, out_ptr, out_bytes, out_f32 = self._args
+        keep = []
+        for i, (a, (dt, sizes, nbytes, bf16)) in enumerate(zip(inputs, self._in)):
+            a = np.asarray(a)
+            bits = bf16 and a.dtype == np.uint16
+            a = np.ascontiguousarray(a, dtype=None if bits else dt)
+            if a.shape != sizes:
+                a = a.reshape(sizes)
+            keep.append(a)
+            in_ptr[i], in_bytes[i] = a.ctypes.data, a.nbytes
+            in_f32[i] = bf16 and not bits
+        outs = [_result_array(dt, sizes, nbytes) for dt, sizes, nbytes, _ in self._out]
+        for i, a in enumerate(outs):
+            out_ptr[i] = a.ctypes.data
+        self.ms = call('plaidml_hip_executable_run_arrays', self.exe.as_ptr(), len(keep), in_ptr, in_bytes, in_f32, len(outs), out_ptr, out_bytes,
+                       out_f32)
+        self._behind = True
+        return outs
 
     def fetch(self):
         outs = []

@@ -834,6 +834,52 @@ double plaidml_executable_run(plaidml_error* err, plaidml_executable* exec, size
   });
 }
 
+// Not part of the reference ABI: a run on arrays in plain memory.  Input / output i takes in_bytes[i] / out_bytes[i] bytes
+// at in[i] / out[i]; in_f32[i] / out_f32[i] non-zero: a bfloat16 tensor given / wanted as fp32 values.
+double plaidml_hip_executable_run_arrays(plaidml_error* err, plaidml_executable* exec, size_t ninputs, void** in, const size_t* in_bytes,
+                                         const int32_t* in_f32, size_t noutputs, void** out, const size_t* out_bytes, const int32_t* out_f32) {
+  return ffi_wrap<double>(err, 0.0, [&] {
+    const auto& prog = *exec->program;
+    if (prog.inputs.size() != ninputs) {
+      throw std::runtime_error("Program expects " + std::to_string(prog.inputs.size()) + " inputs, but " +
+                               std::to_string(ninputs) + " were specified");
+    }
+    if (prog.outputs.size() != noutputs) {
+      throw std::runtime_error("Program expects " + std::to_string(prog.outputs.size()) + " outputs, but " +
+                               std::to_string(noutputs) + " were specified");
+    }
+    std::vector<rt::HostSpan> src(ninputs), dst(noutputs);
+    for (size_t i = 0; i < ninputs; ++i) {
+      if (in_f32[i] && prog.inputs[i]->shape.elementType != util::DataType::bf16) throw std::runtime_error("input #" + std::to_string(i) + " is no bfloat16 tensor");
+      src[i] = {in[i], in_bytes[i], in_f32[i] != 0};
+    }
+    for (size_t i = 0; i < noutputs; ++i) {
+      if (out_f32[i] && prog.outputs[i]->shape.elementType != util::DataType::bf16) throw std::runtime_error("output #" + std::to_string(i) + " is no bfloat16 tensor");
+      dst[i] = {out[i], out_bytes[i], out_f32[i] != 0};
+    }
+    return exec->exec->invokeHost(src, dst);
+  });
+}
+
+// The results of the executable's last run of either kind, copied from the device into `outputs`.
+void plaidml_hip_executable_download(plaidml_error* err, plaidml_executable* exec, size_t noutputs, plaidml_buffer** outputs) {
+  ffi_wrap_void(err, [&] {
+    std::vector<rt::HostSpan> out;
+    for (size_t i = 0; i < noutputs; ++i) out.push_back({outputs[i]->buffer->data(), outputs[i]->buffer->size(), false});
+    exec->exec->download(out);
+  });
+}
+
+// Memory for the results of such runs: page-locked and recycled where possible, else (nullptr) the caller takes its own.
+void* plaidml_hip_host_alloc(size_t bytes) {
+  try {
+    return rt::pinnedAllocRaw(bytes);
+  } catch (const std::exception&) {
+    return nullptr;
+  }
+}
+void plaidml_hip_host_free(void* p) { rt::pinnedFree(p); }
+
 // Not part of the reference ABI: timing breakdown of the calling thread's most recent run, for benchmarks.
 void plaidml_hip_last_run_stats(double* kernel_ms, double* h2d_ms, double* d2h_ms, size_t* launches) {
   rt::InvokeStats s = rt::lastInvokeStats();

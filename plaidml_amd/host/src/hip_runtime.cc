@@ -10,6 +10,7 @@
 #include <regex>
 #include <sstream>
 
+#include "host_copy.h"
 #include "pml_hip.h"
 
 namespace pmlc::rt {
@@ -87,6 +88,19 @@ class HipExecutable final : public Executable {
   ~HipExecutable() override { release(); }
 
   double invoke(const std::vector<util::BufferPtr>& inputs, const std::vector<util::BufferPtr>& outputs) override {
+    std::vector<HostSpan> in, out;
+    for (const auto& b : inputs) in.push_back({b->data(), b->size(), false});
+    for (const auto& b : outputs) out.push_back({b->data(), b->size(), false});
+    return invokeHost(in, out);
+  }
+
+  // One run.  Everything is queued on the executable's stream -- uploads, launches, downloads -- and waited for once.
+  //   inputs   in page-locked memory already: straight from there.  Elsewhere (or fp32 values of a bf16 tensor): through
+  //            the executable's page-locked staging, a few megabytes at a time, so that the link carries one piece
+  //            while the host passes over the next.
+  //   outputs  the mirror image; staged ones are passed on after the wait.
+  // Short transfers are made by one kernel each way (pml_hip_copy_spans), long ones by the copy engines.
+  double invokeHost(const std::vector<HostSpan>& inputs, const std::vector<HostSpan>& outputs) override {
     hipCheck(pml_hip_init(ordinal_), "pml_hip_init");
     if (inputs.size() != plan_->input_buffers.size() || outputs.size() != plan_->output_buffers.size())
       throw std::runtime_error("executable invoked with the wrong number of buffers");
@@ -94,71 +108,97 @@ class HipExecutable final : public Executable {
     const double start = nowMs();
     double t0 = start;
     const bool profile = profileRequested();
-    for (size_t i = 0; i < inputs.size(); ++i) {
-      const BufferInfo& b = plan_->buffers[plan_->input_buffers[i]];
-      if (inputs[i]->size() < b.bytes) throw std::runtime_error("input buffer #" + std::to_string(i) + " is too small");
-      hipCheck(pml_hip_memcpy_h2d(device_[plan_->input_buffers[i]], inputs[i]->data(), b.bytes, stream_), "h2d");
-    }
-    st.h2d_ms = nowMs() - t0;
-    if (profile && step_events_.size() != plan_->steps.size() + 1) {
-      step_events_.assign(plan_->steps.size() + 1, nullptr);
-      for (auto& e : step_events_) hipCheck(pml_hip_event_create(&e), "event");
-    }
-    // The launches of a run never change (same plans, same device buffers), so from the third run on they are
-    // replayed as one graph recorded during that run; the first two run one by one (first runs of a kernel plan may
-    // allocate, which cannot be recorded).  A recording that fails leaves the executable with one-by-one launches.
-    if (graphable_ && !profile && !graph_ && runs_ >= 2) record();
-    ++runs_;
-    hipCheck(pml_hip_event_record(ev0_, stream_), "event record");
-    if (graph_ && !profile) {
-      hipCheck(pml_hip_graph_launch(graph_, stream_), "graph launch");
-      st.replayed = true;
-    } else {
-      for (size_t i = 0; i < plan_->steps.size(); ++i) {
-        if (profile) hipCheck(pml_hip_event_record(step_events_[i], stream_), "event record");
-        launch(i);
+    for (size_t i = 0; i < outputs.size(); ++i)
+      if (outputs[i].bytes < spanBytes(plan_->output_buffers[i], outputs[i])) throw std::runtime_error("output buffer #" + std::to_string(i) + " is too small");
+    for (size_t i = 0; i < inputs.size(); ++i)
+      if (inputs[i].bytes < spanBytes(plan_->input_buffers[i], inputs[i])) throw std::runtime_error("input buffer #" + std::to_string(i) + " is too small");
+    Spans up, down;
+    std::vector<char*> staged(outputs.size(), nullptr);  // where an output waits to be passed on
+    try {
+      size_t at = 0;
+      for (size_t i = 0; i < inputs.size(); ++i)
+        if (!direct(plan_->input_buffers[i], inputs[i])) at += padded(plan_->buffers[plan_->input_buffers[i]].bytes);
+      for (size_t i = 0; i < outputs.size(); ++i)
+        if (!direct(plan_->output_buffers[i], outputs[i])) at += padded(plan_->buffers[plan_->output_buffers[i]].bytes);
+      char* stage = staging(at);
+      for (size_t i = 0; i < inputs.size(); ++i) {
+        const int buf = plan_->input_buffers[i];
+        const size_t bytes = plan_->buffers[buf].bytes;
+        if (direct(buf, inputs[i])) {
+          upload(device_[buf], inputs[i].data, bytes, &up);
+        } else if (stage) {
+          stageIn(stage, inputs[i], bytes, static_cast<char*>(device_[buf]), &up);
+          stage += padded(bytes);
+        } else {
+          // (no page-locked memory to be had)
+          std::vector<uint16_t> tmp;
+          const void* from = inputs[i].data;
+          if (inputs[i].f32) {
+            tmp.resize(bytes / 2);
+            hostToBf16(tmp.data(), static_cast<const float*>(from), tmp.size());
+            from = tmp.data();
+          }
+          hipCheck(pml_hip_memcpy_h2d(device_[buf], from, bytes, stream_), "h2d");
+        }
       }
-    }
-    if (profile) hipCheck(pml_hip_event_record(step_events_.back(), stream_), "event record");
-    hipCheck(pml_hip_event_record(ev1_, stream_), "event record");
-    hipCheck(pml_hip_event_sync(ev1_), "event sync");
-    float ms = 0;
-    hipCheck(pml_hip_event_elapsed_ms(ev0_, ev1_, &ms), "event elapsed");
-    st.kernel_ms = ms;
-    st.launches = plan_->steps.size();
-    st.graph_note = graph_note_;
-    st.arena_bytes = arena_bytes_;
-    st.unshared_temp_bytes = unshared_temp_bytes_;
-    st.device_bytes = arena_bytes_ + fixed_bytes_;
-    if (profile) {
-      // One row per launch, in the reference's format (pmlc/rt/instrument.cc:22-43: id, loc, tag, seconds since
-      // the previous point, seconds since the start); loc is the plan's line for the step, tag its kind.
-      std::printf("\"id\",\"loc\",\"tag\",\"elapsed\",\"accumulated\"\n");
-      double total = 0;
-      st.step_ms.resize(plan_->steps.size());
-      for (size_t i = 0; i < plan_->steps.size(); ++i) {
-        float step = 0;
-        hipCheck(pml_hip_event_elapsed_ms(step_events_[i], step_events_[i + 1], &step), "event elapsed");
-        st.step_ms[i] = step;
-        total += step;
-        std::printf("%03d,\"%s\",%d,%7.6f,%7.6f\n", static_cast<int>(i), plan_->steps[i].text.c_str(),
-                    static_cast<int>(plan_->steps[i].kind), step * 1e-3, total * 1e-3);
+      up.issue(stream_);
+      st.h2d_ms = nowMs() - t0;
+      launchAll(profile, &st);
+      t0 = nowMs();
+      for (size_t i = 0; i < outputs.size(); ++i) {
+        const int buf = plan_->output_buffers[i];
+        const size_t bytes = plan_->buffers[buf].bytes;
+        if (direct(buf, outputs[i])) {
+          download(outputs[i].data, device_[buf], bytes, &down);
+        } else if (stage) {
+          staged[i] = stage;
+          stage += padded(bytes);
+          download(staged[i], device_[buf], bytes, &down);
+        }
       }
-      std::printf("%03d,%s,%d,%7.6f,%7.6f\n", 9999, "endTime", 9999, 0.0, total * 1e-3);
-      std::fflush(stdout);
+      down.issue(stream_);
+    } catch (...) {
+      (void)pml_hip_stream_sync(stream_);  // queued copies may still use the caller's memory
+      throw;
     }
-    t0 = nowMs();
+    hipCheck(pml_hip_stream_sync(stream_), "stream sync");
     for (size_t i = 0; i < outputs.size(); ++i) {
-      const BufferInfo& b = plan_->buffers[plan_->output_buffers[i]];
-      if (outputs[i]->size() < b.bytes) throw std::runtime_error("output buffer #" + std::to_string(i) + " is too small");
-      hipCheck(pml_hip_memcpy_d2h(outputs[i]->data(), device_[plan_->output_buffers[i]], b.bytes, stream_), "d2h");
+      const int buf = plan_->output_buffers[i];
+      const size_t bytes = plan_->buffers[buf].bytes;
+      if (direct(buf, outputs[i])) continue;
+      std::vector<char> tmp;
+      const char* from = staged[i];
+      if (!from) {
+        if (!outputs[i].f32) {
+          hipCheck(pml_hip_memcpy_d2h(outputs[i].data, device_[buf], bytes, stream_), "d2h");
+          continue;
+        }
+        tmp.resize(bytes);
+        hipCheck(pml_hip_memcpy_d2h(tmp.data(), device_[buf], bytes, stream_), "d2h");
+        from = tmp.data();
+      }
+      if (outputs[i].f32)
+        hostFromBf16(static_cast<float*>(outputs[i].data), reinterpret_cast<const uint16_t*>(from), bytes / 2);
+      else
+        hostCopy(outputs[i].data, from, bytes);
     }
     st.d2h_ms = nowMs() - t0;
+    finish(profile, &st);
     st.wall_ms = nowMs() - start;
     g_stats = st;
     // wall time of the whole run, transfers included, as the reference returns the time around its jitted main
     // (pmlc/rt/jit_executable.cc:484-490); the device time alone is in the statistics
     return st.wall_ms;
+  }
+
+  void download(const std::vector<HostSpan>& outputs) override {
+    hipCheck(pml_hip_init(ordinal_), "pml_hip_init");
+    if (outputs.size() != plan_->output_buffers.size()) throw std::runtime_error("executable asked for the wrong number of results");
+    for (size_t i = 0; i < outputs.size(); ++i) {
+      const int buf = plan_->output_buffers[i];
+      if (outputs[i].f32 || outputs[i].bytes < plan_->buffers[buf].bytes) throw std::runtime_error("output buffer #" + std::to_string(i) + " is too small");
+      hipCheck(pml_hip_memcpy_d2h(outputs[i].data, device_[buf], plan_->buffers[buf].bytes, stream_), "d2h");
+    }
   }
 
  private:
@@ -177,6 +217,123 @@ class HipExecutable final : public Executable {
   bool graphable_ = false;
   int runs_ = 0;
   std::string graph_note_;
+  void* staging_ = nullptr;          // page-locked: what a run passes between the caller's memory and the device
+  size_t staging_bytes_ = 0;
+  bool staging_failed_ = false;
+
+  // transfers up to this many bytes go by kernel, longer ones by copy engine
+  static constexpr size_t kKernelCopy = 512 << 10;
+  // bytes the host stages before it hands them to the copy engine
+  static constexpr size_t kStageRun = 4 << 20;
+
+  struct Spans {
+    std::vector<void*> dst;
+    std::vector<const void*> src;
+    std::vector<size_t> bytes;
+    void add(void* d, const void* s, size_t n) {
+      dst.push_back(d);
+      src.push_back(s);
+      bytes.push_back(n);
+    }
+    void issue(pml_hip_stream stream) {
+      if (!dst.empty()) hipCheck(pml_hip_copy_spans(static_cast<int>(dst.size()), dst.data(), src.data(), bytes.data(), stream), "copy");
+    }
+  };
+
+  // bytes the caller's side of a value takes
+  size_t spanBytes(int buf, const HostSpan& h) const { return plan_->buffers[buf].bytes * (h.f32 ? 2 : 1); }
+  bool direct(int buf, const HostSpan& h) const { return !h.f32 && isPinned(h.data, plan_->buffers[buf].bytes); }
+
+  char* staging(size_t bytes) {
+    if (bytes > staging_bytes_ && !staging_failed_) {
+      if (staging_) pinnedFree(staging_);
+      staging_bytes_ = 0;
+      staging_ = pinnedAllocRaw(bytes);
+      if (staging_)
+        staging_bytes_ = bytes;
+      else
+        staging_failed_ = true;
+    }
+    return bytes <= staging_bytes_ ? static_cast<char*>(staging_) : nullptr;
+  }
+
+  void upload(void* dst, const void* src, size_t bytes, Spans* spans) {
+    if (bytes <= kKernelCopy)
+      spans->add(dst, src, bytes);
+    else
+      hipCheck(pml_hip_memcpy_h2d_async(dst, src, bytes, stream_), "h2d");
+  }
+  void download(void* dst, const void* src, size_t bytes, Spans* spans) {
+    if (bytes <= kKernelCopy)
+      spans->add(dst, src, bytes);
+    else
+      hipCheck(pml_hip_memcpy_d2h_async(dst, src, bytes, stream_), "d2h");
+  }
+  void stageIn(char* stage, const HostSpan& in, size_t bytes, char* dev, Spans* spans) {
+    for (size_t at = 0; at < bytes; at += kStageRun) {
+      const size_t n = std::min(kStageRun, bytes - at);
+      if (in.f32)
+        hostToBf16(reinterpret_cast<uint16_t*>(stage + at), static_cast<const float*>(in.data) + at / 2, n / 2);
+      else
+        hostCopy(stage + at, static_cast<const char*>(in.data) + at, n);
+      if (bytes <= kKernelCopy)
+        spans->add(dev + at, stage + at, n);
+      else
+        hipCheck(pml_hip_memcpy_h2d_async(dev + at, stage + at, n, stream_), "h2d");
+    }
+  }
+
+  void launchAll(bool profile, InvokeStats* st) {
+    if (profile && step_events_.size() != plan_->steps.size() + 1) {
+      step_events_.assign(plan_->steps.size() + 1, nullptr);
+      for (auto& e : step_events_) hipCheck(pml_hip_event_create(&e), "event");
+    }
+    // The launches of a run never change (same plans, same device buffers), so from the third run on they are
+    // replayed as one graph recorded during that run; the first two run one by one (first runs of a kernel plan may
+    // allocate, which cannot be recorded).  A recording that fails leaves the executable with one-by-one launches.
+    if (graphable_ && !profile && !graph_ && runs_ >= 2) record();
+    ++runs_;
+    hipCheck(pml_hip_event_record(ev0_, stream_), "event record");
+    if (graph_ && !profile) {
+      hipCheck(pml_hip_graph_launch(graph_, stream_), "graph launch");
+      st->replayed = true;
+    } else {
+      for (size_t i = 0; i < plan_->steps.size(); ++i) {
+        if (profile) hipCheck(pml_hip_event_record(step_events_[i], stream_), "event record");
+        launch(i);
+      }
+    }
+    if (profile) hipCheck(pml_hip_event_record(step_events_.back(), stream_), "event record");
+    hipCheck(pml_hip_event_record(ev1_, stream_), "event record");
+  }
+
+  // statistics of a run that has been waited for
+  void finish(bool profile, InvokeStats* st) {
+    float ms = 0;
+    hipCheck(pml_hip_event_elapsed_ms(ev0_, ev1_, &ms), "event elapsed");
+    st->kernel_ms = ms;
+    st->launches = plan_->steps.size();
+    st->graph_note = graph_note_;
+    st->arena_bytes = arena_bytes_;
+    st->unshared_temp_bytes = unshared_temp_bytes_;
+    st->device_bytes = arena_bytes_ + fixed_bytes_;
+    if (!profile) return;
+    // One row per launch, in the reference's format (pmlc/rt/instrument.cc:22-43: id, loc, tag, seconds since
+    // the previous point, seconds since the start); loc is the plan's line for the step, tag its kind.
+    std::printf("\"id\",\"loc\",\"tag\",\"elapsed\",\"accumulated\"\n");
+    double total = 0;
+    st->step_ms.resize(plan_->steps.size());
+    for (size_t i = 0; i < plan_->steps.size(); ++i) {
+      float step = 0;
+      hipCheck(pml_hip_event_elapsed_ms(step_events_[i], step_events_[i + 1], &step), "event elapsed");
+      st->step_ms[i] = step;
+      total += step;
+      std::printf("%03d,\"%s\",%d,%7.6f,%7.6f\n", static_cast<int>(i), plan_->steps[i].text.c_str(), static_cast<int>(plan_->steps[i].kind),
+                  step * 1e-3, total * 1e-3);
+    }
+    std::printf("%03d,%s,%d,%7.6f,%7.6f\n", 9999, "endTime", 9999, 0.0, total * 1e-3);
+    std::fflush(stdout);
+  }
 
   void record() {
     if (pml_hip_capture_begin(stream_) != 0) {
@@ -291,6 +448,8 @@ class HipExecutable final : public Executable {
     graph_ = nullptr;
     if (stream_) pml_hip_stream_destroy(stream_);
     stream_ = nullptr;
+    if (staging_) pinnedFree(staging_);
+    staging_ = nullptr;
   }
 
   char* ptr(int buf, int64_t elem_off = 0, size_t elem_size = 1) const {
@@ -464,43 +623,102 @@ void registerRuntime(const std::string& id, std::shared_ptr<Runtime> runtime) {
 // program) sets PLAIDML_PINNED=0; the total is capped (PLAIDML_PINNED_MAX_MB, default 4096) because page-locked
 // memory is taken from what the host can page.  Beyond the cap, and on any failure, the caller falls back to
 // ordinary memory (nullptr here).
+//
+// Blocks come in sizes of 1/8 steps between powers of two and, when freed, are kept for the next allocation of their
+// size as long as all kept ones together stay under kPinnedKeep; the one kept longest goes back to the system first.
 namespace {
-std::mutex g_pinned_mutex;
-std::map<void*, size_t> g_pinned_sizes;
-size_t g_pinned_total = 0;
+constexpr size_t kPinnedKeep = size_t{256} << 20;
+struct PinnedPool {
+  std::mutex mutex;
+  std::map<const char*, size_t> live;                   // block -> its size
+  std::vector<std::pair<char*, size_t>> kept;           // free blocks, the one freed first in front
+  size_t live_total = 0, kept_total = 0;
+};
+PinnedPool& pinnedPool() {  // (never destroyed: buffers may be freed while the process ends)
+  static PinnedPool* pool = new PinnedPool();
+  return *pool;
+}
+size_t pinnedSize(size_t bytes) {
+  size_t step = 4096;
+  while (step * 16 <= bytes) step *= 2;
+  return (std::max<size_t>(bytes, 1) + step - 1) / step * step;
+}
 }  // namespace
 
 void* pinnedAlloc(size_t bytes) {
+  void* p = pinnedAllocRaw(bytes);
+  if (p) std::memset(p, 0, bytes);
+  return p;
+}
+
+void* pinnedAllocRaw(size_t bytes) {
   const std::string enabled = util::Settings::Instance()->get("PLAIDML_PINNED");
   if (enabled == "0" || enabled == "false" || enabled == "off") return nullptr;
   const std::string cap_text = util::Settings::Instance()->get("PLAIDML_PINNED_MAX_MB");
   const size_t cap = (cap_text.empty() ? size_t{4096} : static_cast<size_t>(std::strtoull(cap_text.c_str(), nullptr, 10))) << 20;
+  PinnedPool& pool = pinnedPool();
+  if (bytes > cap) return nullptr;
+  const size_t size = pinnedSize(bytes);
+  char* p = nullptr;
   {
-    std::lock_guard<std::mutex> lock(g_pinned_mutex);
-    if (bytes > cap || g_pinned_total > cap - bytes) return nullptr;
+    std::lock_guard<std::mutex> lock(pool.mutex);
+    if (pool.live_total > cap - bytes) return nullptr;
+    for (size_t i = pool.kept.size(); i-- > 0;) {
+      if (pool.kept[i].second != size) continue;
+      p = pool.kept[i].first;
+      pool.kept.erase(pool.kept.begin() + static_cast<long>(i));
+      pool.kept_total -= size;
+      pool.live[p] = size;
+      pool.live_total += size;
+      break;
+    }
   }
-  initRuntimes();
-  if (listDevices().empty()) return nullptr;
-  void* p = nullptr;
-  if (pml_hip_host_alloc(&p, bytes) != 0 || !p) return nullptr;
-  std::memset(p, 0, bytes);
-  std::lock_guard<std::mutex> lock(g_pinned_mutex);
-  g_pinned_sizes[p] = bytes;
-  g_pinned_total += bytes;
+  if (!p) {
+    initRuntimes();
+    if (listDevices().empty()) return nullptr;
+    void* fresh = nullptr;
+    if (pml_hip_host_alloc(&fresh, size) != 0 || !fresh) return nullptr;
+    p = static_cast<char*>(fresh);
+    std::lock_guard<std::mutex> lock(pool.mutex);
+    pool.live[p] = size;
+    pool.live_total += size;
+  }
   return p;
 }
 
 void pinnedFree(void* p) {
   if (!p) return;
+  PinnedPool& pool = pinnedPool();
+  std::vector<char*> back;
   {
-    std::lock_guard<std::mutex> lock(g_pinned_mutex);
-    const auto it = g_pinned_sizes.find(p);
-    if (it != g_pinned_sizes.end()) {
-      g_pinned_total -= it->second;
-      g_pinned_sizes.erase(it);
+    std::lock_guard<std::mutex> lock(pool.mutex);
+    const auto it = pool.live.find(static_cast<const char*>(p));
+    if (it == pool.live.end()) return;
+    const size_t size = it->second;
+    pool.live.erase(it);
+    pool.live_total -= size;
+    if (size > kPinnedKeep) {
+      back.push_back(static_cast<char*>(p));
+    } else {
+      pool.kept.emplace_back(static_cast<char*>(p), size);
+      pool.kept_total += size;
+      while (pool.kept_total > kPinnedKeep) {
+        back.push_back(pool.kept.front().first);
+        pool.kept_total -= pool.kept.front().second;
+        pool.kept.erase(pool.kept.begin());
+      }
     }
   }
-  pml_hip_host_free(p);
+  for (char* b : back) pml_hip_host_free(b);
+}
+
+bool isPinned(const void* p, size_t bytes) {
+  PinnedPool& pool = pinnedPool();
+  std::lock_guard<std::mutex> lock(pool.mutex);
+  auto it = pool.live.upper_bound(static_cast<const char*>(p));
+  if (it == pool.live.begin()) return false;
+  --it;
+  return static_cast<const char*>(p) + bytes <= it->first + it->second;
 }
 
 void initRuntimes() {

@@ -19,9 +19,20 @@
 
 namespace pmlc::rt {
 
+// A program input or output in host memory; f32: a bf16 tensor held as fp32 values there
+struct HostSpan {
+  void* data;
+  size_t bytes;
+  bool f32;
+};
+
 class Executable {
  public:
   virtual ~Executable() = default;
+  // the same on plain memory (inputs are only read)
+  virtual double invokeHost(const std::vector<HostSpan>& inputs, const std::vector<HostSpan>& outputs) = 0;
+  // the results of the last run, from the device
+  virtual void download(const std::vector<HostSpan>& outputs) = 0;
   // returns the wall time of the run in milliseconds, host-device transfers included
   virtual double invoke(const std::vector<util::BufferPtr>& inputs, const std::vector<util::BufferPtr>& outputs) = 0;
 };
@@ -47,9 +58,13 @@ std::shared_ptr<Device> getDevice(const std::string& deviceID);
 
 // Host memory the GPU can read and write directly (page-locked), for buffers the library allocates itself: a
 // copy to or from it runs at the link's rate instead of being staged through the driver's own bounce buffers.
-// Zero-initialised.  nullptr when no GPU is visible (the caller falls back to ordinary memory).
+// Zero-initialised (pinnedAllocRaw: not).  nullptr when no GPU is visible (the caller falls back to ordinary memory).
+// Freed blocks up to a bound are kept for the next allocation: page-locking costs about as much as copying the block.
 void* pinnedAlloc(size_t bytes);
+void* pinnedAllocRaw(size_t bytes);  // not zeroed
 void pinnedFree(void* p);
+// whether [p, p + bytes) lies in one live block of it
+bool isPinned(const void* p, size_t bytes);
 
 // statistics of the most recent invoke of any hip executable in this thread (for benchmarks)
 struct InvokeStats {
