@@ -467,6 +467,54 @@ typedef struct {
 } pml_hip_softmax_desc;
 int pml_hip_softmax(const pml_hip_softmax_desc* desc, const void* x, void* y, pml_hip_stream s);
 
+/* ---- operations along the rows of a matrix ---------------------------------------
+ * A short program over every row of a dense [rows][cols] matrix in one launch: element-wise steps and reductions of the
+ * row, in the order given -- what the op library composes a normalisation from (plaidml/op/lib/ops.cc:1970-2033), or any
+ * chain of such operations.  Every step's result is rounded to `dtype` as the separate operation would round it; sums
+ * accumulate in fp32 and are rounded once. */
+#define PML_HIP_ROWS_STEPS 24
+#define PML_HIP_ROWS_IO 6
+#define PML_HIP_ROWS_SCALARS 16
+#define PML_HIP_ROWS_VECTORS 8
+enum {
+  PML_HIP_ROWS_MAP = 0,      /* vector[dst] = opcode(a, b): an arithmetic PML_HIP_EPI_* (a is v, b is x), or 0: a itself */
+  PML_HIP_ROWS_MAP_SCALAR,   /* scalar[dst] = the same on scalar operands */
+  PML_HIP_ROWS_REDUCE,       /* scalar[dst] = aggregation `opcode` (PML_HIP_AGG_*) over the row a, from the identity imm on */
+  PML_HIP_ROWS_STORE,        /* out[dst][row][:] = a */
+  PML_HIP_ROWS_STORE_SCALAR  /* out[dst][row] = scalar[a] */
+};
+enum { /* where an operand comes from */
+  PML_HIP_ROWS_NONE = 0,
+  PML_HIP_ROWS_VECTOR,  /* vector[index] */
+  PML_HIP_ROWS_SCALAR,  /* scalar[index] */
+  PML_HIP_ROWS_FULL,    /* in[index], a [rows][cols] tensor */
+  PML_HIP_ROWS_COLUMNS, /* in[index], one value per column */
+  PML_HIP_ROWS_ROW,     /* in[index], one value per row */
+  PML_HIP_ROWS_ONE,     /* in[index], a single value */
+  PML_HIP_ROWS_IMM      /* the step's imm */
+};
+typedef struct {
+  int32_t kind, opcode, dst;
+  int32_t a_kind, a, b_kind, b;
+  float imm;
+} pml_hip_rows_step;
+typedef struct {
+  int32_t dtype; /* F32 or BF16 */
+  int32_t n_steps, n_vectors, n_in, n_out, reserved;
+  int64_t rows, cols;
+  pml_hip_rows_step steps[PML_HIP_ROWS_STEPS];
+} pml_hip_rows_desc;
+int pml_hip_rows_takes(const pml_hip_rows_desc* desc); /* host arithmetic only: well-formed, and the rows fit a CU's LDS */
+int pml_hip_rows(const pml_hip_rows_desc* desc, const void* const* in, void* const* out, pml_hip_stream s);
+/* out[row] = the last position of the row's largest element (plaidml/op/lib/ops.cc:505-521: max over positions whose value
+ * equals the maximum; no NaN is ever the maximum).  F32 or BF16 rows, dense; int32 results. */
+int pml_hip_argmax_rows(int dtype, int64_t rows, int64_t cols, const void* x, int32_t* out, pml_hip_stream s);
+/* The first k elements of every row in ascending (0) or descending (1) order and their positions, as argsort followed by
+ * gathers gives them (ties in position order, NaNs last); values or positions may be null.  Types up to 32 bits;
+ * k <= cols <= PML_HIP_MAX_SORT_LINE. */
+int pml_hip_topk_rows(int dtype, int descending, int64_t rows, int64_t cols, int k, const void* x, void* values, int32_t* positions,
+                      pml_hip_stream s);
+
 /* three-input select(cond, t, f) with broadcasting (tile.select, SelectOp of
  * pmlc/conversion/tile_to_linalg/tile_to_linalg.cc:262-273) */
 typedef struct {
@@ -637,7 +685,7 @@ int pml_hip_contract_invoke(int64_t plan, const void* const* srcs, void* out, pm
 /* sizeof() of a descriptor struct as this library was compiled, so that a foreign-language
  * binding can verify its own layout: 0 epilogue, 1 gemm, 2 conv2d, 3 dwconv2d, 4 pool2d,
  * 5 eltwise, 6 select, 7 contract, 8 form, 9 gather, 10 scatter, 11 argsort, 12 softmax,
- * 13 product.  Returns 0 for an unknown id. */
+ * 13 product, 14 rows.  Returns 0 for an unknown id. */
 size_t pml_hip_struct_size(int which);
 
 /* Releases a plan returned by any *_dispatch. */

@@ -974,9 +974,114 @@ __global__ __launch_bounds__(256) void softmax_rows_kernel(const void* x_, void*
   }
 }
 
+// The same for rows of up to 4 U LANES elements: a lane keeps its U runs of four neighbouring elements in registers from
+// the one read to the one write (the walks above read the row three times and take every exponential twice), and short
+// rows have a wavefront each, which meets no barrier.  500 x 8000 fp32: 37 -> 15 us, 4096 x 1000: 20 -> 13 us.
+template <bool BF, int LANES, int U>
+__global__ __launch_bounds__(256) void softmax_regs_kernel(const void* x_, void* y_, int64_t rows, int cols) {
+  __shared__ float part[4];
+  const int lane = LANES == 64 ? (int)(threadIdx.x & 63) : (int)threadIdx.x;
+  const int64_t row = (int64_t)blockIdx.x * (256 / LANES) + (LANES == 64 ? (int)(threadIdx.x >> 6) : 0);
+  if (row >= rows) return;  // (a whole wavefront of a kernel without barriers, or nobody)
+  auto rounded = [](float v) { return BF ? round_to_bf16(v) : v; };
+  auto across = [&](float v, auto fold) {
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) v = fold(v, __shfl_xor(v, d, 64));
+    if constexpr (LANES == 256) {
+      __syncthreads();
+      if ((lane & 63) == 0) part[lane >> 6] = v;
+      __syncthreads();
+      v = fold(fold(part[0], part[1]), fold(part[2], part[3]));
+    }
+    return v;
+  };
+  const int64_t base = row * cols;
+  float v[4 * U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int c = (lane + u * LANES) * 4;
+    if (c + 4 <= cols) {
+      if constexpr (BF) {
+        uint16_t h[4];
+        __builtin_memcpy(h, (const uint16_t*)x_ + base + c, 8);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[4 * u + e] = bf16_bits_to_f32(h[e]);
+      } else {
+        __builtin_memcpy(&v[4 * u], (const float*)x_ + base + c, 16);
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        v[4 * u + e] = c + e >= cols ? -INFINITY : BF ? bf16_bits_to_f32(((const uint16_t*)x_)[base + c + e]) : ((const float*)x_)[base + c + e];
+    }
+  }
+  float m = -INFINITY;
+#pragma unroll
+  for (int e = 0; e < 4 * U; ++e) m = v[e] > m ? v[e] : m;
+  m = across(m, [](float a, float b) { return b > a ? b : a; });
+  float sum = 0.f;
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      v[4 * u + e] = rounded(expf(rounded(v[4 * u + e] - m)));
+      sum += (lane + u * LANES) * 4 + e < cols ? v[4 * u + e] : 0.f;
+    }
+  sum = rounded(across(sum, [](float a, float b) { return a + b; }));
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int c = (lane + u * LANES) * 4;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[4 * u + e] = rounded(v[4 * u + e] / sum);
+    if constexpr (BF) {
+      uint16_t h[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) h[e] = f32_to_bf16_bits(v[4 * u + e]);
+      if (c + 4 <= cols) {
+        __builtin_memcpy((uint16_t*)y_ + base + c, h, 8);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (c + e < cols) ((uint16_t*)y_)[base + c + e] = h[e];
+      }
+    } else {
+      if (c + 4 <= cols) {
+        __builtin_memcpy((float*)y_ + base + c, &v[4 * u], 16);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (c + e < cols) ((float*)y_)[base + c + e] = v[4 * u + e];
+      }
+    }
+  }
+}
+
+template <bool BF>
+bool softmax_in_regs(const pml_hip_softmax_desc& d, const void* x, void* y, hipStream_t s) {
+  if (d.cols > 256 * 32) return false;
+  // a wavefront per row up to 512 columns, and up to 1024 where the rows fill the chip that way
+  const bool narrow = d.cols <= 512 || (d.cols <= 1024 && d.rows >= 1024);
+  const int64_t chunks = (d.cols + (narrow ? 255 : 1023)) / (narrow ? 256 : 1024);
+  const dim3 grid((unsigned)(narrow ? (d.rows + 3) / 4 : d.rows)), block(256);
+#define PML_GO(LANES, U) hipLaunchKernelGGL((softmax_regs_kernel<BF, LANES, U>), grid, block, 0, s, x, y, d.rows, (int)d.cols)
+  if (narrow) {
+    if (chunks <= 1) PML_GO(64, 1);
+    else if (chunks <= 2) PML_GO(64, 2);
+    else PML_GO(64, 4);
+  } else {
+    if (chunks <= 1) PML_GO(256, 1);
+    else if (chunks <= 2) PML_GO(256, 2);
+    else if (chunks <= 4) PML_GO(256, 4);
+    else PML_GO(256, 8);
+  }
+#undef PML_GO
+  return true;
+}
+
 hipError_t softmax_launch(const pml_hip_softmax_desc& d, const void* x, void* y, hipStream_t s) {
   if (d.rows == 0 || d.cols == 0) return hipSuccess;
   if (d.rows > 0x7fffffff) return hipErrorInvalidValue;
+  if (d.dtype == PML_HIP_BF16 ? softmax_in_regs<true>(d, x, y, s) : softmax_in_regs<false>(d, x, y, s)) return hipGetLastError();
   if (d.dtype == PML_HIP_BF16)
     hipLaunchKernelGGL(softmax_rows_kernel<true>, dim3((unsigned)d.rows), dim3(256), 0, s, x, y, d.cols);
   else

@@ -274,6 +274,18 @@ hipError_t copy_spans_launch(const SpanArgs& a, hipStream_t s);
 hipError_t fill_u32_launch(void* p, uint32_t pattern, size_t n_words, hipStream_t s);
 hipError_t softmax_launch(const pml_hip_softmax_desc& d, const void* x, void* y, hipStream_t s);
 
+// operations along rows (rows.hip)
+struct RowsProgramArgs {
+  pml_hip_rows_desc d;
+  const void* in[PML_HIP_ROWS_IO];
+  void* out[PML_HIP_ROWS_IO];
+};
+size_t rows_program_lds(const pml_hip_rows_desc& d, int* lanes);
+hipError_t rows_program_launch(const RowsProgramArgs& a, hipStream_t s);
+hipError_t argmax_rows_launch(int dtype, int64_t rows, int64_t cols, const void* x, int32_t* out, hipStream_t s);
+hipError_t topk_rows_launch(int dtype, int descending, int64_t rows, int64_t cols, int k, const void* x, void* values, int32_t* positions,
+                            hipStream_t s);
+
 // special operations (special.hip)
 hipError_t gather_launch(const pml_hip_gather_desc& d, const void* tensor, const void* indices, void* out, hipStream_t s);
 hipError_t scatter_launch(const pml_hip_scatter_desc& d, const void* data, const void* indices, const void* updates, void* out,

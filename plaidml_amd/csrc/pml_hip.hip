@@ -1284,6 +1284,71 @@ int pml_hip_conv2d_pack_filter(int64_t plan, const void* filter, pml_hip_stream 
 }
 
 // ---------------------------------------------------------------------------
+// operations along rows
+// ---------------------------------------------------------------------------
+
+int pml_hip_rows_takes(const pml_hip_rows_desc* d) {
+  if (!d || (d->dtype != PML_HIP_F32 && d->dtype != PML_HIP_BF16) || d->rows < 0 || d->cols < 0 || d->cols > (1 << 20) || d->n_steps < 0 ||
+      d->n_steps > PML_HIP_ROWS_STEPS || d->n_vectors < 0 || d->n_vectors > PML_HIP_ROWS_VECTORS || d->n_in < 0 || d->n_in > PML_HIP_ROWS_IO ||
+      d->n_out < 0 || d->n_out > PML_HIP_ROWS_IO)
+    return 0;
+  auto operand = [&](int kind, int index, bool scalar) {
+    switch (kind) {
+      case PML_HIP_ROWS_NONE: case PML_HIP_ROWS_IMM: return true;
+      case PML_HIP_ROWS_VECTOR: return !scalar && index >= 0 && index < d->n_vectors;
+      case PML_HIP_ROWS_SCALAR: return index >= 0 && index < PML_HIP_ROWS_SCALARS;
+      case PML_HIP_ROWS_FULL: case PML_HIP_ROWS_COLUMNS: return !scalar && index >= 0 && index < d->n_in;
+      case PML_HIP_ROWS_ROW: case PML_HIP_ROWS_ONE: return index >= 0 && index < d->n_in;
+    }
+    return false;
+  };
+  for (int i = 0; i < d->n_steps; ++i) {
+    const pml_hip_rows_step& s = d->steps[i];
+    bool ok = s.dst >= 0;
+    switch (s.kind) {
+      case PML_HIP_ROWS_MAP: ok = ok && s.dst < d->n_vectors && operand(s.a_kind, s.a, false) && operand(s.b_kind, s.b, false); break;
+      case PML_HIP_ROWS_MAP_SCALAR: ok = ok && s.dst < PML_HIP_ROWS_SCALARS && operand(s.a_kind, s.a, true) && operand(s.b_kind, s.b, true); break;
+      case PML_HIP_ROWS_REDUCE: ok = ok && s.dst < PML_HIP_ROWS_SCALARS && operand(s.a_kind, s.a, false) && s.opcode >= PML_HIP_AGG_ADD && s.opcode <= PML_HIP_AGG_MUL; break;
+      case PML_HIP_ROWS_STORE: ok = ok && s.dst < d->n_out && operand(s.a_kind, s.a, false); break;
+      case PML_HIP_ROWS_STORE_SCALAR: ok = ok && s.dst < d->n_out && s.a >= 0 && s.a < PML_HIP_ROWS_SCALARS; break;
+      default: ok = false;
+    }
+    if (!ok) return 0;
+  }
+  int lanes = 0;
+  return rows_program_lds(*d, &lanes) <= 158 * 1024 ? 1 : 0;
+}
+
+int pml_hip_rows(const pml_hip_rows_desc* d, const void* const* in, void* const* out, pml_hip_stream s) {
+  if (!pml_hip_rows_takes(d)) return fail("rows: malformed program, or rows too long for it");
+  RowsProgramArgs a;
+  std::memset(&a, 0, sizeof a);
+  a.d = *d;
+  for (int i = 0; i < d->n_in; ++i) {
+    if (!in || !in[i]) return fail("rows: missing input");
+    a.in[i] = in[i];
+  }
+  for (int i = 0; i < d->n_out; ++i) {
+    if (!out || !out[i]) return fail("rows: missing output");
+    a.out[i] = out[i];
+  }
+  return check(rows_program_launch(a, (hipStream_t)s), "rows_program_launch");
+}
+
+int pml_hip_argmax_rows(int dtype, int64_t rows, int64_t cols, const void* x, int32_t* out, pml_hip_stream s) {
+  if ((dtype != PML_HIP_F32 && dtype != PML_HIP_BF16) || rows < 0 || cols <= 0 || cols > 0x7fffffff) return fail("argmax_rows: bad type or sizes");
+  if (rows && (!x || !out)) return fail("argmax_rows: null operand");
+  return check(argmax_rows_launch(dtype, rows, cols, x, out, (hipStream_t)s), "argmax_rows_launch");
+}
+
+int pml_hip_topk_rows(int dtype, int descending, int64_t rows, int64_t cols, int k, const void* x, void* values, int32_t* positions,
+                      pml_hip_stream s) {
+  if (dt_size(dtype) == 0 || dt_size(dtype) == 8 || rows < 0 || k < 0 || k > cols || cols > PML_HIP_MAX_SORT_LINE) return fail("topk_rows: bad type or sizes");
+  if (rows && k && (!x || (!values && !positions))) return fail("topk_rows: null operand");
+  return check(topk_rows_launch(dtype, descending != 0, rows, cols, k, x, values, positions, (hipStream_t)s), "topk_rows_launch");
+}
+
+// ---------------------------------------------------------------------------
 // products over free strides, gradients of a convolution
 // ---------------------------------------------------------------------------
 
@@ -1974,6 +2039,7 @@ size_t pml_hip_struct_size(int which) {
     case 11: return sizeof(pml_hip_argsort_desc);
     case 12: return sizeof(pml_hip_softmax_desc);
     case 13: return sizeof(pml_hip_product_desc);
+    case 14: return sizeof(pml_hip_rows_desc);
   }
   return 0;
 }

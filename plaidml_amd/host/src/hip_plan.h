@@ -26,7 +26,7 @@ struct BufferInfo {
 };
 
 struct Step {
-  enum Kind { Gemm, Conv2d, Dwconv2d, Pool2d, Eltwise, Select, Index, Contract, Copy, Gather, Scatter, ArgSort, Prng, Softmax, Product, ConvGrad } kind = Copy;
+  enum Kind { Gemm, Conv2d, Dwconv2d, Pool2d, Eltwise, Select, Index, Contract, Copy, Gather, Scatter, ArgSort, Prng, Softmax, Product, ConvGrad, Rows, Argmax, TopK } kind = Copy;
   std::string text;  // one line for the plan dump
   std::string schedule;  // "{tile=...,conv=...}" when the target options or a schedule file named this step's tiling
   // descriptors (only the one matching `kind` is meaningful)
@@ -42,6 +42,9 @@ struct Step {
   pml_hip_argsort_desc srt{};
   pml_hip_softmax_desc sm{};
   pml_hip_product_desc prod{};
+  pml_hip_rows_desc rows{};
+  int topk = 0;             // TopK (and Argmax: rows and columns in `sm`): entries taken, order; values in c, positions in out2
+  bool topk_descending = false;
   int grad_which = 0;       // ConvGrad: `conv` describes the forward convolution; 0 = gradient of its data, 1 = of its filter
   int64_t prng_count = 0;   // Prng: values drawn
   bool prng_state = false;  //       the step yields the advanced state instead of the values

@@ -42,6 +42,7 @@ void Planner::emitSpecial(size_t i) {
     for (size_t d = 0; d < sh.getRank(); ++d) sizes[d] = sh.sizes[d];
   };
   auto param = [&](size_t k) { return static_cast<int64_t>(op.params.at(k)); };
+  if (op.fn == "argsort" && opt_.fuse && opt_.specialise && tryTopk(i)) return;
   Step s;
   s.c = bufferFor(op.result);
   for (const ValuePtr& v : op.operands) s.operands.push_back(bufferFor(v));
@@ -271,6 +272,8 @@ void Planner::emitContraction(size_t i) {
     if (tryPool(i)) return;
     if (tryGlobalPool(i)) return;
     if (opt_.fuse && trySoftmax(i)) return;
+    if (opt_.fuse && tryArgmax(i)) return;
+    if (opt_.fuse && tryRowProgram(i)) return;
   }
   emitGeneral(i);
 }

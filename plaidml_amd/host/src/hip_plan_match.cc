@@ -861,9 +861,9 @@ bool Planner::reducesLastAxis(const Op& op, AggKind agg) {
   if (!op.constraints.empty() || op.accesses.size() != 2) return false;
   const TensorShape &is = op.operands[0]->shape, &os = op.result->shape;
   const size_t r = is.getRank();
-  if (r < 1 || os.getRank() != r || op.idxNames.size() != r || op.accesses[0].size() != r || op.accesses[1].size() != r) return false;
+  if (r < 1 || os.getRank() != r || op.idxNames.size() < r || op.accesses[0].size() != r || op.accesses[1].size() != r) return false;
   if (os.elementType != is.elementType || os.sizes[r - 1] != 1) return false;
-  std::vector<bool> seen(r, false);
+  std::vector<bool> seen(op.idxNames.size(), false);
   for (size_t d = 0; d < r; ++d) {
     const int v = op.accesses[1][d].plainIndex();
     if (v < 0 || seen[v]) return false;
@@ -872,9 +872,14 @@ bool Planner::reducesLastAxis(const Op& op, AggKind agg) {
     if (d + 1 < r) {
       if (os.sizes[d] != is.sizes[d] || op.accesses[0][d].plainIndex() != v) return false;
     } else if (!(op.accesses[0][d].isConstant() && op.accesses[0][d].c0 == 0)) {
-      return false;
+      // (or an index of its own that can only be 0)
+      const int w = op.accesses[0][d].plainIndex();
+      if (w < 0 || seen[w] || op.lower[w] != 0 || op.upper[w] != 0) return false;
+      seen[w] = true;
     }
   }
+  for (bool used : seen)
+    if (!used) return false;
   return true;
 }
 

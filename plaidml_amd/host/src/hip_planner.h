@@ -2,6 +2,7 @@
 //   hip_plan.cc        the driver: buffers, the walk over the program, schedule overrides, the plan dump
 //   hip_plan_match.cc  recognising matrix products, convolutions, depthwise convolutions and pooling in a contraction
 //   hip_plan_fuse.cc   elementwise tails folded into kernels, second products, row pitches, dead steps
+//   hip_plan_rows.cc   row programs, argmax, the first k of a sort: operations along the last axis in one launch
 //   hip_plan_emit.cc   elementwise and special operations, and the general loop nest for every other contraction
 // Not part of the library's interface.
 #pragma once
@@ -224,6 +225,11 @@ class Planner {
   bool matchWindowArgmax(size_t ui, const Op& pool, const pml_hip_pool2d_desc& pd);
   static bool reducesLastAxis(const Op& op, AggKind agg);
   bool trySoftmax(size_t i);
+  bool usedOnlyBy(const ValuePtr& v, const std::set<size_t>& users);
+  bool tryArgmax(size_t i);
+  bool isTakenInOrder(const ValuePtr& taken, const ValuePtr& X, const ValuePtr& order, std::set<size_t>* between);
+  bool tryTopk(size_t i);
+  bool tryRowProgram(size_t i);
 
   // ----- the general contraction kernel ---------------------------------------------------
 

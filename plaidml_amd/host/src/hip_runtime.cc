@@ -77,7 +77,8 @@ class HipExecutable final : public Executable {
       for (const Step& s : plan_->steps)
         if (s.kind != Step::Gemm && s.kind != Step::Conv2d && s.kind != Step::Dwconv2d && s.kind != Step::Pool2d &&
             s.kind != Step::Eltwise && s.kind != Step::Contract && s.kind != Step::Select && s.kind != Step::Copy &&
-            s.kind != Step::Softmax && s.kind != Step::Product && s.kind != Step::ConvGrad)
+            s.kind != Step::Softmax && s.kind != Step::Product && s.kind != Step::ConvGrad && s.kind != Step::Rows &&
+            s.kind != Step::Argmax && s.kind != Step::TopK)
           graphable_ = false;
     } catch (...) {
       release();
@@ -481,6 +482,9 @@ class HipExecutable final : public Executable {
       case Step::ArgSort:
       case Step::Prng:
       case Step::Softmax:
+      case Step::Rows:
+      case Step::Argmax:
+      case Step::TopK:
       case Step::Copy: return;
     }
     if (!h) throw std::runtime_error("hip dispatch failed for '" + s.text + "': " + pml_hip_last_error());
@@ -538,6 +542,17 @@ class HipExecutable final : public Executable {
         break;
       case Step::Softmax:
         hipCheck(pml_hip_softmax(&s.sm, ptr(s.a), ptr(s.c), stream_), s.text.c_str());
+        break;
+      case Step::Rows:
+        hipCheck(pml_hip_rows(&s.rows, operands, outs, stream_), s.text.c_str());
+        break;
+      case Step::Argmax:
+        hipCheck(pml_hip_argmax_rows(s.sm.dtype, s.sm.rows, s.sm.cols, ptr(s.a), reinterpret_cast<int32_t*>(ptr(s.c)), stream_), s.text.c_str());
+        break;
+      case Step::TopK:
+        hipCheck(pml_hip_topk_rows(s.sm.dtype, s.topk_descending, s.sm.rows, s.sm.cols, s.topk, ptr(s.a), ptr(s.c),
+                                   reinterpret_cast<int32_t*>(ptr(s.out2)), stream_),
+                 s.text.c_str());
         break;
       case Step::Index:
         hipCheck(pml_hip_index(ptr(s.c), static_cast<int32_t>(s.index_sizes.size()), s.index_sizes.data(), s.index_axis, stream_),
