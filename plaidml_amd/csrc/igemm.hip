@@ -672,6 +672,31 @@ __global__ __launch_bounds__(256) void transpose_bytes_kernel(const uint8_t* __r
   for (int j = 0; j < 4; ++j) *(i32x4_t*)(Bt + (n + j) * ldbt + k) = out[j];
 }
 
+// The same for 2-byte elements: a thread takes 8 K-rows x 4 N-columns as eight 8-byte loads, turns them with v_perm_b32
+// and writes 16 bytes of K to each of its four Bt rows; a wavefront covers 32 x 64 elements (128-byte runs read), the
+// four of a workgroup lie one after the other in K (256-byte runs written).  Memory-bound; the plain kernel's 2-byte
+// accesses through LDS took 22 us for 4096 x 4096 (3.0 TB/s), a product of that size with it 149 us; now 134.
+// K % 8 == 0, N % 4 == 0, ldb % 4 == 0, ldbt % 8 == 0, B 8-byte and Bt 16-byte aligned.
+__global__ __launch_bounds__(256) void transpose_halves_kernel(const uint16_t* __restrict__ B, uint16_t* __restrict__ Bt,
+                                                               int64_t K, int64_t N, int64_t ldb, int64_t ldbt) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t n = (int64_t)blockIdx.x * 64 + 4 * (lane & 15);
+  const int64_t k = (int64_t)blockIdx.y * 128 + 32 * wave + 8 * (lane >> 4);
+  if (n >= N || k >= K) return;
+  uint2 r[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) r[i] = *(const uint2*)(B + (k + i) * ldb + n);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const unsigned sel = (j & 1) ? 0x07060302u : 0x05040100u;
+    i32x4_t out;
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      out[q] = (int)(j < 2 ? __builtin_amdgcn_perm(r[2 * q + 1].x, r[2 * q].x, sel) : __builtin_amdgcn_perm(r[2 * q + 1].y, r[2 * q].y, sel));
+    *(i32x4_t*)(Bt + (n + j) * ldbt + k) = out;
+  }
+}
+
 // The same for 4-byte elements with 16-byte global accesses on both sides: a workgroup turns a 64 x 64
 // tile through LDS (row stride 65 words: the transposed reads touch every bank once).
 // K % 4 == 0, N % 4 == 0, ldb % 4 == 0, ldbt % 4 == 0, both pointers 16-byte aligned.
@@ -982,6 +1007,11 @@ hipError_t transpose_pack(int elem_size, const void* B, void* Bt, int64_t K, int
       hipLaunchKernelGGL(transpose_kernel<uint8_t>, grid, dim3(256), 0, s, (const uint8_t*)B, (uint8_t*)Bt, K, N, ldb, ldbt);
       break;
     case 2:
+      if (K % 8 == 0 && N % 4 == 0 && ldb % 4 == 0 && ldbt % 8 == 0 && ((uintptr_t)B & 7) == 0 && ((uintptr_t)Bt & 15) == 0) {
+        dim3 grid_h((unsigned)((N + 63) / 64), (unsigned)((K + 127) / 128));
+        hipLaunchKernelGGL(transpose_halves_kernel, grid_h, dim3(256), 0, s, (const uint16_t*)B, (uint16_t*)Bt, K, N, ldb, ldbt);
+        break;
+      }
       hipLaunchKernelGGL(transpose_kernel<uint16_t>, grid, dim3(256), 0, s, (const uint16_t*)B, (uint16_t*)Bt, K, N, ldb, ldbt);
       break;
     case 4:
