@@ -214,6 +214,8 @@ enum {
   PML_HIP_TILE_128x64_N2,      /* 4 wavefronts of 32x64 (split fp32 kind only) */
   PML_HIP_TILE_192x384_W8,     /* 8 wavefronts of 96x96 (bf16 and int8) */
   PML_HIP_TILE_64x64_KSPLIT,   /* 64x64 tiles whose K loop is shared out among several workgroups, partial tiles added up by a second launch */
+  PML_HIP_TILE_16x16_W8,       /* 8 wavefronts that share the K of one 16x16 tile, fragments straight from memory (16x64 with B as [K][N]) */
+  PML_HIP_TILE_32x32_W8,       /* the same with 32x32 (32x64) results */
   PML_HIP_TILE_COUNT_
 };
 enum {

@@ -1,0 +1,331 @@
+// Matrix products and implicit-GEMM convolutions with few result tiles: small tiles, fragments straight from memory.
+//
+// What bounds such a problem (one image through the last stages of a network, one row through a dense layer) is
+// latency: 49 x 512 results of K = 4608 are eight 64 x 64 tiles, each a chain of 72 slabs through LDS with a barrier
+// apiece, and splitting that chain over workgroups costs a second launch that adds the parts up.  Here a workgroup of
+// eight wavefronts owns 16 x 16 or 32 x 32 results -- four to sixteen times the workgroups -- and the wavefronts share
+// its K out among themselves: every one loads the fragments of its own run of K from memory into registers (a lane's
+// 16 bytes of a row are what the MFMA takes, no LDS and no barrier on the way; sixteen requests in flight per lane),
+// and the eight partial tiles meet in LDS once, are added in wavefront order and go through the common tail.
+// What is paid for it is traffic: a 16 x 16 tile fetches every operand byte for 16 results.  It comes out of L2, and
+// `direct_tile_of` (pml_hip.hip) says up to where that is the better deal.
+//
+// KN: the right-hand side is the caller's B[K][N] as it lies.  A lane takes four neighbouring columns of every K-row of
+// its chunk and turns them in registers (v_perm) into fragments of four column blocks, block j holding the columns
+// 4 r + j: tiles are 64 columns wide, and no transposed copy is written and read back.
+#include <hip/hip_runtime.h>
+
+#include "device_common.h"
+#include "igemm_tail.h"
+#include "plans.h"
+
+namespace pml {
+namespace {
+
+constexpr int kWaves = 8;
+constexpr unsigned kRsrcFlags = 0x00020000u;  // raw buffer, 32-bit data format
+constexpr unsigned kBufRange = 0x80000000u;   // every real offset is below 2 GiB (checked at launch) ...
+constexpr unsigned kOutside = 0x80000000u;    // ... and this one reads as zeros, with any offset below 2 GiB added
+
+// 16 x 16 results += a 64-byte step of K: a lane holds 16 bytes of row lane % 16, chunk lane / 16 of the step.  (The
+// chunks need not be the MFMA's own K order: both operands use the same one.)
+// NA partial sums in turn (`u`: the step's number): shorter chains of dependent MFMAs, and of roundings.
+template <int KIND, int NA, class V>
+__device__ __forceinline__ void mma16(V (&sums)[NA], int u, const i32x4_t& b, const i32x4_t& a) {
+  V& acc = sums[u % NA];
+  if constexpr (KIND == KIND_BF16) {
+    bf16x8_t av, bv;
+    __builtin_memcpy(&av, &a, 16);
+    __builtin_memcpy(&bv, &b, 16);
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bv, av, acc, 0, 0, 0);
+  } else if constexpr (KIND == KIND_I8) {
+    acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(b, a, acc, 0, 0, 0);
+  } else {
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      sums[q % NA] = __builtin_amdgcn_mfma_f32_16x16x4f32(__int_as_float(b[q]), __int_as_float(a[q]), sums[q % NA], 0, 0, 0);
+  }
+}
+
+// Four fragments (16 bytes of K each) of four neighbouring columns from the 16 words of their K-rows as they lie.
+template <int KIND>
+__device__ __forceinline__ void turn(const int (&raw)[16], i32x4_t (&frag)[4]) {
+  if constexpr (KIND == KIND_F32) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) frag[j] = i32x4_t{raw[j], raw[4 + j], raw[8 + j], raw[12 + j]};
+  } else if constexpr (KIND == KIND_BF16) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const unsigned sel = (j & 1) ? 0x07060302u : 0x05040100u;
+      const int h = j >> 1;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) frag[j][q] = (int)__builtin_amdgcn_perm((unsigned)raw[4 * q + 2 + h], (unsigned)raw[4 * q + h], sel);
+    }
+  } else {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const unsigned r0 = (unsigned)raw[4 * q], r1 = (unsigned)raw[4 * q + 1], r2 = (unsigned)raw[4 * q + 2], r3 = (unsigned)raw[4 * q + 3];
+      const unsigned t0 = __builtin_amdgcn_perm(r1, r0, 0x05010400u), t1 = __builtin_amdgcn_perm(r1, r0, 0x07030602u);
+      const unsigned t2 = __builtin_amdgcn_perm(r3, r2, 0x05010400u), t3 = __builtin_amdgcn_perm(r3, r2, 0x07030602u);
+      frag[0][q] = (int)__builtin_amdgcn_perm(t2, t0, 0x05040100u);
+      frag[1][q] = (int)__builtin_amdgcn_perm(t2, t0, 0x07060302u);
+      frag[2][q] = (int)__builtin_amdgcn_perm(t3, t1, 0x05040100u);
+      frag[3][q] = (int)__builtin_amdgcn_perm(t3, t1, 0x07060302u);
+    }
+  }
+}
+
+// MB x NB blocks of 16 x 16 results per workgroup.
+template <int KIND, bool CONV, int MB, int NB, bool KN>
+__global__ __launch_bounds__(64 * kWaves, 4) void direct_kernel(IgemmArgs p_by_value) {
+  // (read where the dispatcher put it: indexing a by-value copy would move the copy to scratch memory)
+  const IgemmArgs& p = *(const IgemmArgs*)(const __attribute__((address_space(4))) void*)__builtin_amdgcn_kernarg_segment_ptr();
+  static_assert(!KN || (NB == 4 && !CONV), "a [K][N] right-hand side is taken four columns per lane");
+  typedef typename Acc<KIND>::scalar accs_t;
+  typedef accs_t acc4_t __attribute__((ext_vector_type(4)));
+  constexpr int ES = KIND == KIND_BF16 ? 2 : (KIND == KIND_I8 ? 1 : 4);
+  constexpr int TM = 16 * MB, TN = 16 * NB;
+  // steps in flight: 64 registers of requests, fewer where the accumulators leave less room
+  constexpr int U = KN ? (MB == 1 ? 3 : 2) : 16 / (MB + NB);
+  constexpr int CS = TN + 4;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  accs_t* const parts = (accs_t*)smem;  // [wavefront][TM][CS]
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r = lane & 15, g = lane >> 4;
+  int tile_m, tile_n;
+  tile_of(p.order, blockIdx.x, &tile_m, &tile_n);
+  const int64_t m0 = (int64_t)tile_m * TM, n0 = (int64_t)tile_n * TN;
+
+  const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void*)p.A, 0, (int)kBufRange, kRsrcFlags);
+  const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void*)p.Bt, 0, (int)kBufRange, kRsrcFlags);
+  const bool two = !CONV && !KN && p.K2 > 0;
+  const __amdgpu_buffer_rsrc_t ra2 = __builtin_amdgcn_make_buffer_rsrc((void*)(two ? p.A2 : p.A), 0, (int)kBufRange, kRsrcFlags);
+  const __amdgpu_buffer_rsrc_t rb2 = __builtin_amdgcn_make_buffer_rsrc((void*)(two ? p.Bt2 : p.Bt), 0, (int)kBufRange, kRsrcFlags);
+
+  const int kbytes = (int)(CONV ? p.CI * ES : p.K * ES);  // valid bytes per (tap) row
+  const int steps_per_tap = (kbytes + 63) >> 6;
+  const int k2_bytes = two ? (int)(p.K2 * ES) : 0;
+  const int n_steps = CONV ? p.KH * p.KW * steps_per_tap : steps_per_tap + ((k2_bytes + 63) >> 6);
+  const int per = (n_steps + kWaves - 1) / kWaves;
+  const int first = wave * per;
+  const int last = first + per < n_steps ? first + per : n_steps;
+
+  // byte offsets of this lane's rows (CONV: of the input pixel tap (0, 0) reads, which may lie outside the image)
+  unsigned a_off[MB], a2_off[CONV ? 1 : MB], b_off[KN ? 1 : NB], b2_off[CONV || KN ? 1 : NB];
+  int a_ih[MB], a_iw[MB];
+#pragma unroll
+  for (int i = 0; i < MB; ++i) {
+    const int64_t m = m0 + 16 * i + r;
+    const bool ok = m < p.M;
+    const unsigned mu = (unsigned)(ok ? m : 0);
+    if constexpr (CONV) {
+      const unsigned nb = fast_div(mu, p.div_per_magic, p.div_per_shift);
+      const unsigned rem = mu - nb * (unsigned)(p.OH * p.OW);
+      const unsigned oh = fast_div(rem, p.div_ow_magic, p.div_ow_shift);
+      const int ow = (int)(rem - oh * (unsigned)p.OW);
+      a_ih[i] = ok ? (int)oh * p.SH - p.PH : -(1 << 28);
+      a_iw[i] = ow * p.SW - p.PW;
+      a_off[i] = (unsigned)((int64_t)nb * ((int64_t)p.H * p.W * kbytes)) + (unsigned)(a_ih[i] * p.W + a_iw[i]) * (unsigned)kbytes;
+    } else {
+      a_off[i] = ok ? (unsigned)(m * p.lda * ES) : kOutside;
+      int64_t row = mu;
+      if (two && p.g2_stride > 0) {
+        const unsigned nb = fast_div(mu, p.g2_ohw_magic, p.g2_ohw_shift);
+        const unsigned rem = mu - nb * (unsigned)p.g2_ohw;
+        const unsigned oy = fast_div(rem, p.g2_ow_magic, p.g2_ow_shift);
+        const unsigned ox = rem - oy * (unsigned)p.g2_ow;
+        row = ((int64_t)nb * p.g2_h + (int64_t)oy * p.g2_stride) * p.g2_w + (int64_t)ox * p.g2_stride;
+      }
+      a2_off[i] = (two && ok) ? (unsigned)(row * p.lda2 * ES) : kOutside;
+    }
+  }
+  if constexpr (KN) {
+    const int64_t n = n0 + 4 * r;  // (N is a multiple of four: a lane's columns exist together)
+    b_off[0] = n < p.N ? (unsigned)(n * ES) : kOutside;
+  } else {
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+      const int64_t n = n0 + 16 * j + r;
+      b_off[j] = n < p.N ? (unsigned)(n * p.ldbt * ES) : kOutside;
+      if constexpr (!CONV) b2_off[j] = (two && n < p.N) ? (unsigned)(n * p.ldbt2 * ES) : kOutside;
+    }
+  }
+
+  // CONV: the tap of the next step to be requested and the step inside it, as counters
+  int cs = 0, kh = 0, kw = 0;
+  if constexpr (CONV) {
+    const int tap = first / steps_per_tap;
+    cs = first - tap * steps_per_tap;
+    kh = tap / p.KW;
+    kw = tap - kh * p.KW;
+  }
+
+  // (fp32: the same number for every tile, so that a result has the same bits whatever tile or layout it comes from)
+  constexpr int NA = KIND == KIND_F32 || MB * NB == 1 ? 2 : 1;
+  acc4_t sums[MB][NB][NA];
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+      for (int c = 0; c < NA; ++c) sums[i][j][c] = acc4_t{0, 0, 0, 0};
+
+  for (int s0 = first; s0 < last; s0 += U) {
+    i32x4_t fa[U][MB];
+    i32x4_t fb[KN ? 1 : U][KN ? 1 : NB];
+    int raw[KN ? U : 1][16];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const bool live = s0 + u < last;
+      if constexpr (CONV) {
+        const int cb = cs * 64 + g * 16;
+        const bool ok = live & (cb < kbytes);
+        const int dh = kh * p.DH, dw = kw * p.DW;
+        const unsigned at = (unsigned)((dh * p.W + dw) * kbytes + cb);
+#pragma unroll
+        for (int i = 0; i < MB; ++i) {
+          const bool in = ok & ((unsigned)(a_ih[i] + dh) < (unsigned)p.H) & ((unsigned)(a_iw[i] + dw) < (unsigned)p.W);
+          fa[u][i] = __builtin_bit_cast(i32x4_t, __builtin_amdgcn_raw_buffer_load_b128(ra, in ? (int)(a_off[i] + at) : (int)kOutside, 0, 0));
+        }
+        const unsigned bk = (unsigned)((kh * p.KW + kw) * kbytes + cb);
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+          fb[u][j] = __builtin_bit_cast(i32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rb, ok ? (int)(b_off[j] + bk) : (int)kOutside, 0, 0));
+        if (++cs == steps_per_tap) {
+          cs = 0;
+          if (++kw == p.KW) {
+            kw = 0;
+            ++kh;
+          }
+        }
+      } else {
+        const bool second = !KN && s0 + u >= steps_per_tap;
+        const int cb = (second ? s0 + u - steps_per_tap : s0 + u) * 64 + g * 16;
+        const bool ok = live & (cb < (second ? k2_bytes : kbytes));
+#pragma unroll
+        for (int i = 0; i < MB; ++i)
+          fa[u][i] = __builtin_bit_cast(i32x4_t, __builtin_amdgcn_raw_buffer_load_b128(
+                                                     second ? ra2 : ra, ok ? (int)((second ? a2_off[i] : a_off[i]) + (unsigned)cb) : (int)kOutside, 0, 0));
+        if constexpr (KN) {
+          constexpr int E = 16 / ES;  // K-rows of the lane's chunk: all of them exist or none (K is whole 16-byte vectors)
+          const unsigned pitch = (unsigned)(p.ldbt * ES);
+          const unsigned at = b_off[0] + (unsigned)(cb / ES) * pitch;
+          const bool in = ok & (b_off[0] != kOutside);
+#pragma unroll
+          for (int e = 0; e < E; ++e) {
+            const int off = in ? (int)(at + (unsigned)e * pitch) : (int)kOutside;
+            if constexpr (KIND == KIND_F32) {
+              const i32x4_t v = __builtin_bit_cast(i32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rb, off, 0, 0));
+#pragma unroll
+              for (int q = 0; q < 4; ++q) raw[u][4 * e + q] = v[q];
+            } else if constexpr (KIND == KIND_BF16) {
+              typedef int i32x2_t __attribute__((ext_vector_type(2)));
+              const i32x2_t v = __builtin_bit_cast(i32x2_t, __builtin_amdgcn_raw_buffer_load_b64(rb, off, 0, 0));
+              raw[u][2 * e] = v[0];
+              raw[u][2 * e + 1] = v[1];
+            } else {
+              raw[u][e] = (int)__builtin_amdgcn_raw_buffer_load_b32(rb, off, 0, 0);
+            }
+          }
+        } else {
+#pragma unroll
+          for (int j = 0; j < NB; ++j)
+            fb[u][j] = __builtin_bit_cast(i32x4_t, __builtin_amdgcn_raw_buffer_load_b128(
+                                                       second ? rb2 : rb, ok ? (int)((second ? b2_off[j] : b_off[j]) + (unsigned)cb) : (int)kOutside, 0, 0));
+        }
+      }
+    }
+    // (the right-hand fragment is the row operand: a lane then holds result row m = lane % 16 and four block rows)
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if constexpr (KN) {
+        i32x4_t frag[4];
+        turn<KIND>(raw[u], frag);
+#pragma unroll
+        for (int i = 0; i < MB; ++i)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) mma16<KIND, NA>(sums[i][j], u, frag[j], fa[u][i]);
+      } else {
+#pragma unroll
+        for (int i = 0; i < MB; ++i)
+#pragma unroll
+          for (int j = 0; j < NB; ++j) mma16<KIND, NA>(sums[i][j], u, fb[u][j], fa[u][i]);
+      }
+    }
+  }
+
+  acc4_t acc[MB][NB];
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+      acc[i][j] = sums[i][j][0];
+#pragma unroll
+      for (int c = 1; c < NA; ++c) acc[i][j] += sums[i][j][c];
+    }
+#pragma unroll
+  for (int i = 0; i < MB; ++i) {
+    accs_t* const row = &parts[(wave * TM + 16 * i + r) * CS];
+    if constexpr (KN) {
+      // block j's rows are the columns 4 (row) + j: the lane's four blocks hold neighbouring columns
+#pragma unroll
+      for (int e = 0; e < 4; ++e) *(acc4_t*)&row[16 * g + 4 * e] = acc4_t{acc[i][0][e], acc[i][1][e], acc[i][2][e], acc[i][3][e]};
+    } else {
+#pragma unroll
+      for (int j = 0; j < NB; ++j) *(acc4_t*)&row[16 * j + 4 * g] = acc[i][j];
+    }
+  }
+  __syncthreads();
+  constexpr int kQuads = TM * TN / 4;  // one thread each
+  static_assert(kQuads <= 64 * kWaves, "a thread per four results");
+  if (tid >= kQuads) return;
+  accs_t* const mine = &parts[(tid / (TN / 4)) * CS + (tid % (TN / 4)) * 4];
+  acc4_t sum = *(const acc4_t*)mine;
+#pragma unroll
+  for (int w = 1; w < kWaves; ++w) sum += *(const acc4_t*)(mine + w * (TM * CS));
+  *(acc4_t*)mine = sum;
+  // (each thread's tail reads the four results it has just written)
+  tile_tail<KIND, TM, TN, kQuads>(p, parts, m0, n0, tid);
+}
+
+template <int KIND, bool CONV, int MB, int NB, bool KN>
+hipError_t launch(const IgemmArgs& a, hipStream_t s) {
+  const int64_t tiles_m = (a.M + 16 * MB - 1) / (16 * MB), tiles_n = (a.N + 16 * NB - 1) / (16 * NB);
+  const int64_t tiles = tiles_m * tiles_n;
+  if (tiles <= 0 || tiles >= ((int64_t)1 << 31)) return hipErrorInvalidValue;
+  const size_t lds = (size_t)kWaves * 16 * MB * (16 * NB + 4) * 4;
+  auto kern = direct_kernel<KIND, CONV, MB, NB, KN>;
+  static DynamicLdsLimit limit;
+  if (hipError_t e = limit.ensure((const void*)kern, lds); e != hipSuccess) return e;
+  IgemmArgs b = a;
+  b.order = make_tile_order((int)tiles_m, (int)tiles_n);
+  hipLaunchKernelGGL(kern, dim3((unsigned)tiles), dim3(64 * kWaves), lds, s, b);
+  return hipGetLastError();
+}
+
+}  // namespace
+
+#ifndef PML_KIND
+#error "compile with -DPML_KIND=0|1|2 (fp32 | bf16 | int8)"
+#endif
+#define PML_CAT_(a, b) a##b
+#define PML_CAT(a, b) PML_CAT_(a, b)
+
+// cfg: TILE_16x16_W8 or TILE_32x32_W8 (with a [K][N] right-hand side: 16 x 64 and 32 x 64 results)
+hipError_t PML_CAT(direct_launch_kind_, PML_KIND)(int cfg, bool conv, const IgemmArgs& a, hipStream_t s) {
+  const bool small = cfg == TILE_16x16_W8;
+  if (conv) {
+    // (K-runs that span several pixels are the re-blocked convolution's: igemm.hip)
+    if (a.b_kn || a.pix_pitch) return hipErrorInvalidValue;
+    return small ? launch<PML_KIND, true, 1, 1, false>(a, s) : launch<PML_KIND, true, 2, 2, false>(a, s);
+  }
+  if (a.b_kn) {
+    if (a.K2 > 0 || a.N % 4 != 0 || a.ldbt % 4 != 0) return hipErrorInvalidValue;
+    return small ? launch<PML_KIND, false, 1, 4, true>(a, s) : launch<PML_KIND, false, 2, 4, true>(a, s);
+  }
+  return small ? launch<PML_KIND, false, 1, 1, false>(a, s) : launch<PML_KIND, false, 2, 2, false>(a, s);
+}
+
+}  // namespace pml

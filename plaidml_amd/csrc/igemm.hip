@@ -39,6 +39,9 @@ hipError_t igemm_launch_kind_1(int cfg, bool conv, const IgemmArgs& a, hipStream
 hipError_t igemm_launch_kind_2(int cfg, bool conv, const IgemmArgs& a, hipStream_t s);
 hipError_t igemm_launch_kind_3(int cfg, bool conv, const IgemmArgs& a, hipStream_t s);
 hipError_t igemm_launch_kind_4(int cfg, bool conv, const IgemmArgs& a, hipStream_t s);
+hipError_t direct_launch_kind_0(int cfg, bool conv, const IgemmArgs& a, hipStream_t s);  // direct.hip
+hipError_t direct_launch_kind_1(int cfg, bool conv, const IgemmArgs& a, hipStream_t s);
+hipError_t direct_launch_kind_2(int cfg, bool conv, const IgemmArgs& a, hipStream_t s);
 
 namespace {
 
@@ -957,8 +960,18 @@ hipError_t igemm_launch(int kind, int cfg, bool conv, const IgemmArgs& a, hipStr
   // the kernel addresses both operands with 32-bit byte offsets below 2 GiB
   const int64_t es = kind == KIND_BF16 ? 2 : (kind == KIND_I8 ? 1 : 4);
   const int64_t a_bytes = conv ? (int64_t)a.NB * a.H * a.W * (a.pix_pitch ? a.pix_pitch : a.CI * es) + 256 : a.M * a.lda * es;
-  const int64_t b_bytes = a.N * a.ldbt * es;
+  const int64_t b_bytes = (a.b_kn ? a.K : a.N) * a.ldbt * es;
   if (a_bytes >= ((int64_t)1 << 31) || b_bytes >= ((int64_t)1 << 31) || (conv && a.M >= ((int64_t)1 << 31))) return hipErrorInvalidValue;
+  if (cfg == TILE_16x16_W8 || cfg == TILE_32x32_W8) {
+    if (!conv || !a.pix_pitch) {
+      switch (kind) {
+        case KIND_F32: return direct_launch_kind_0(cfg, conv, a, s);
+        case KIND_BF16: return direct_launch_kind_1(cfg, conv, a, s);
+        case KIND_I8: return direct_launch_kind_2(cfg, conv, a, s);
+      }
+    }
+    cfg = TILE_64x64;  // (not built for the split fp32 kinds, nor for K-runs over several pixels)
+  }
   switch (kind) {
     case KIND_F32: return igemm_launch_kind_0(cfg, conv, a, s);
     case KIND_BF16: return igemm_launch_kind_1(cfg, conv, a, s);

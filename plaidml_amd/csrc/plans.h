@@ -40,7 +40,8 @@ enum { KIND_F32 = 0, KIND_BF16 = 1, KIND_I8 = 2, KIND_F32X3 = 3, KIND_F32X3P = 4
 enum { TILE_64x64 = PML_HIP_TILE_64x64, TILE_128x64 = PML_HIP_TILE_128x64, TILE_128x128 = PML_HIP_TILE_128x128, TILE_128x64_W8 = PML_HIP_TILE_128x64_W8,
        TILE_128x128_W8 = PML_HIP_TILE_128x128_W8, TILE_256x128_W16 = PML_HIP_TILE_256x128_W16, TILE_128x128_W8_S2 = PML_HIP_TILE_128x128_W8_S2,
        TILE_64x64_W8_K2 = PML_HIP_TILE_64x64_W8_K2, TILE_256x256_W8 = PML_HIP_TILE_256x256_W8, TILE_128x64_N2 = PML_HIP_TILE_128x64_N2,
-       TILE_192x384_W8 = PML_HIP_TILE_192x384_W8, TILE_64x64_KSPLIT = PML_HIP_TILE_64x64_KSPLIT };
+       TILE_192x384_W8 = PML_HIP_TILE_192x384_W8, TILE_64x64_KSPLIT = PML_HIP_TILE_64x64_KSPLIT,
+       TILE_16x16_W8 = PML_HIP_TILE_16x16_W8, TILE_32x32_W8 = PML_HIP_TILE_32x32_W8 };
 
 struct TailPtrs {
   const void* operands[PML_HIP_MAX_EPI_OPERANDS];

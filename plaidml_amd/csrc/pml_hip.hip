@@ -32,6 +32,10 @@ int check(hipError_t e, const char* what) {
 
 enum PlanKind { PLAN_GEMM = 1, PLAN_CONV, PLAN_DWCONV, PLAN_POOL, PLAN_ELTWISE, PLAN_CONTRACT, PLAN_PRODUCT, PLAN_CONV_GRAD };
 
+struct DirectTiles {
+  int rows = -1, given = -1;
+};
+
 struct Plan {
   int kind = 0;
   int mfma_kind = 0;
@@ -69,6 +73,9 @@ struct Plan {
   // K split over workgroups: workspace of partial tiles and how the slabs are shared out (splits < 2: no split)
   void* ws = nullptr;
   int sk_splits = 0, sk_per = 0, sk_pitch = 0;
+  // the direct tiles a product takes instead of `tile`, and the one a convolution takes with a packed filter (-1: none)
+  DirectTiles direct;
+  int tile_direct = -1;
   // register-filter convolution: a filter packed once, in the order the kernel holds it in registers
   void* reg_image = nullptr;
   // product over free strides, and a convolution's gradients built on it: the prepared arguments (workspace in `ws`),
@@ -122,6 +129,8 @@ const char* tile_name(int t) {
     case TILE_128x128_W8_S2: return "128x128 (8 wavefronts, 2 stages)";
     case TILE_192x384_W8: return "192x384 (8 wavefronts of 96x96)";
     case TILE_64x64_KSPLIT: return "64x64, K split over workgroups";
+    case TILE_16x16_W8: return "16x16 (8 wavefronts sharing K)";
+    case TILE_32x32_W8: return "32x32 (8 wavefronts sharing K)";
   }
   return "?";
 }
@@ -131,7 +140,52 @@ constexpr int kMaxpoolBits = 0x1f << 20;
 bool schedule_bits_ok(int flags) {
   return PML_HIP_FLAG_TILE_OF(flags) < PML_HIP_TILE_COUNT_ && PML_HIP_FLAG_CONV_OF(flags) <= PML_HIP_CONV_BLOCKS;
 }
-const char* const kTileShort[PML_HIP_TILE_COUNT_] = {"64x64", "128x64", "128x128", "128x64w8", "128x128w8", "256x128w16", "128x128w8s2", "64x64w8k2", "256x256w8", "128x64n2", "192x384w8", "64x64ks"};
+const char* const kTileShort[PML_HIP_TILE_COUNT_] = {"64x64", "128x64", "128x128", "128x64w8", "128x128w8", "256x128w16", "128x128w8s2", "64x64w8k2", "256x256w8", "128x64n2", "192x384w8", "64x64ks", "16x16w8", "32x32w8"};
+
+// One of the direct tiles (direct.hip) where it beats the LDS kernels, or -1.  Both sides are priced in microseconds, from
+// measurements of 27 matrix products and 18 convolutions per element kind (one row to 3136, K of 64 to 4608; back to back
+// in a recorded graph): a direct kernel takes 2.6 plus, per round of one tile on each of 256 CUs, 0.8 (fp32 32 x 32: 1.9)
+// and its operand bytes at 40 KB a microsecond and CU.  An LDS kernel takes 4.2 plus its chain of 128-byte slabs (0.23 each,
+// int8 0.28, fp32 0.58), or -- K split over workgroups -- 5.2 (fp32 6.5) plus 0.4 per KB of K plus writing and reading the
+// partial tiles at 3 TB/s.  The prices meet the measurements to about 15 %; a direct tile has to be 5 % ahead.
+//   us, before -> direct                       bf16              fp32              int8
+//   1 x 1000, K = 2048                     7.4 ->  5.0       9.3 ->  7.3       6.7 ->  4.3
+//   196 x 256, K = 1024                    7.5 ->  5.2       9.7 ->  6.5       6.4 ->  4.4
+//   28 x 28 x 128 (*) 3 x 3 x 128          9.1 ->  7.7      11.1 (12.8)        7.4 ->  5.2
+//   49 x 512, K = 4608: stays split        8.6 (11.2)       12.9 (18.7)        7.6 ( 7.4)
+// A right-hand side that arrives with the call as [K][N]: tiles are then 16 or 32 x 64 (60 KB a microsecond; fp32 45,
+// int8 36 unless rows are whole 64-byte runs), and an LDS kernel that needs Bt pays for the transposed copy besides, 3 and
+// its bytes both ways at 2.2 TB/s:
+// bf16 512 x 512 x 512 9.4 -> 5.0, 1024^3 14.6 -> 10.6, 64 x 2048 x 2048 16.5 -> 8.8; fp32 128 x 4096 x 1024 23.4 -> 12.3.
+// kn_ldb: that right-hand side's row pitch in bytes (0: Bt); always: the better of the two whatever the LDS kernel takes
+int direct_tile_of(int64_t m, int64_t n, int64_t k_bytes, int kind, int64_t kn_ldb = 0, bool always = false) {
+  if (kind != KIND_F32 && kind != KIND_BF16 && kind != KIND_I8) return -1;
+  auto tiles = [&](int64_t bm, int64_t bn) { return ((m + bm - 1) / bm) * ((n + bn - 1) / bn); };
+  const double kb = (double)k_bytes;
+  const int es = kind == KIND_BF16 ? 2 : (kind == KIND_I8 ? 1 : 4);
+  const bool kn = kn_ldb > 0, f32 = kind == KIND_F32;
+  const double rate = !kn ? 40e3 : f32 ? 45e3 : (kind == KIND_I8 && kn_ldb % 64 != 0) ? 36e3 : 60e3;
+  auto direct_us = [&](int64_t side) {
+    const int64_t wide = kn ? 64 : side;
+    const double rounds = std::max(1.0, (double)tiles(side, wide) / 256);
+    return 2.6 + rounds * ((f32 && !kn && side == 32 ? 1.9 : 0.8) + (double)(std::min(m, side) + std::min(n, wide)) * kb / rate);
+  };
+  const int64_t slabs = (k_bytes + 127) / 128;
+  double lds_us = 4.2 + (f32 ? 0.58 : kind == KIND_I8 ? 0.28 : 0.23) * (double)slabs;
+  bool needs_bt = kind == KIND_BF16 || n % (16 / es) != 0 || kn_ldb % 16 != 0;
+  if (tiles(64, 64) <= 64 && k_bytes >= 2048) {
+    int splits = 1, per = 0;
+    igemm_split_plan(m, n, slabs, 256, &splits, &per);
+    if (splits >= 2) {
+      lds_us = (f32 ? 6.5 : 5.2) + kb / 2500 + 8.0 * splits * (double)m * (double)n / 3e6;
+      needs_bt = true;
+    }
+  }
+  if (kn && needs_bt) lds_us += 3.0 + 2.0 * kb * (double)n / 2.2e6;
+  const double small = direct_us(16), large = direct_us(32);
+  if (!always && std::min(small, large) > 0.95 * lds_us) return -1;
+  return small <= large ? TILE_16x16_W8 : TILE_32x32_W8;
+}
 
 // Stated tiling choice per shape class.  Measured on MI355X, bf16 unless said otherwise (us; w8 / w16 =
 // 8 / 16 wavefronts per workgroup; s2 = two ring stages and LDS cut to what the result tile needs, so that two
@@ -723,6 +777,19 @@ int pml_hip_gemm_tail_cheaper_apart(const pml_hip_gemm_desc* d) {
   return choose_tile(d->m, d->n, k_bytes, kind, true) == TILE_256x256_W8 && choose_tile(d->m, d->n, k_bytes, kind, false) != TILE_256x256_W8;
 }
 
+// The direct tiles of a product (-1: none): over Bt rows that are at hand (packed earlier, or [N][K] as given), and over a
+// [K][N] right-hand side as it lies.  One that has to be transposed first, and a tile the descriptor names, stay with the
+// plan's tile -- except that fp32 sums are the same bits in either layout: there the layout decides which direct tile, not whether.
+static DirectTiles direct_tiles(const pml_hip_gemm_desc& d, int kind) {
+  DirectTiles t;
+  if (PML_HIP_FLAG_TILE_OF(d.flags) >= 0) return t;
+  const int es = dt_size(d.in_dtype);
+  t.rows = direct_tile_of(d.m, d.n, (d.k + d.k2) * es, kind);
+  if (d.b_layout || d.k2 > 0 || (kind == KIND_F32 && t.rows < 0)) return t;
+  t.given = direct_tile_of(d.m, d.n, d.k * es, kind, d.ldb * es, /*always=*/kind == KIND_F32);
+  return t;
+}
+
 int64_t pml_hip_gemm_dispatch(const pml_hip_gemm_desc* d) {
   const int kind = gemm_desc_kind(d);
   if (kind < 0) return 0;
@@ -758,6 +825,8 @@ int64_t pml_hip_gemm_dispatch(const pml_hip_gemm_desc* d) {
                 (long long)d->m, (long long)d->n, (long long)d->k, tile_name(p->tile),
                 kind == KIND_F32 ? "f32_32x32x2" : kind == KIND_BF16 ? "f32_32x32x16_bf16" : kind == KIND_I8 ? "i32_32x32x32_i8" : "3 x f32_32x32x16_bf16 (fp32 split into bf16 head + remainder)");
   p->text = buf;
+  p->direct = direct_tiles(*d, kind);
+  if (p->direct.rows >= 0) p->text += std::string(", with rows of K at hand tile=") + tile_name(p->direct.rows);
   if (d->k2 > 0) p->text += " + second product k2=" + std::to_string(d->k2) + (d->a2_stride > 0 ? " over pixel rows of stride " + std::to_string(d->a2_stride) : "");
   return (int64_t)(intptr_t)p;
 }
@@ -777,6 +846,12 @@ struct SecondProduct {
 // fp32 kinds gather their K-values from [k][n] slabs, int8 reads them with transposing LDS reads); everything else
 // is transposed into Bt[N][K] first.  Rows must be whole 16-byte vectors.
 static bool reads_b_as_given(const pml_hip_gemm_desc& d, int mfma_kind, const void* b, int tile) {
+  if ((tile == TILE_16x16_W8 || tile == TILE_32x32_W8) && mfma_kind != KIND_F32X3) {
+    // (four neighbouring columns per lane and K-row, whatever the type: direct.hip)
+    const int64_t es = dt_size(d.in_dtype);
+    return b && !d.b_layout && d.k2 == 0 && d.n % 4 == 0 && d.ldb % 4 == 0 && ((uintptr_t)b & (4 * es - 1)) == 0 &&
+           d.k * d.ldb * es < ((int64_t)1 << 31);
+  }
   if (mfma_kind != KIND_F32 && mfma_kind != KIND_F32X3 && mfma_kind != KIND_I8) return false;
   if (tile == TILE_64x64_KSPLIT) return false;  // (the split kernel reads Bt)
   if (tile == TILE_192x384_W8) return false;  // (24 chunks per row: the position swizzle of the [k][n] form needs a power of two)
@@ -796,7 +871,7 @@ static bool reads_b_as_given(const pml_hip_gemm_desc& d, int mfma_kind, const vo
   return true;
 }
 
-static int gemm_run(const pml_hip_gemm_desc& d, int mfma_kind, int tile, void* bt, int64_t bt_ld, bool packed,
+static int gemm_run(const pml_hip_gemm_desc& d, int mfma_kind, int tile, const DirectTiles& direct, void* bt, int64_t bt_ld, bool packed,
                     const void* a, const void* b, void* c, const void* init, const void* const* operands,
                     void* const* outs, pml_hip_stream s, const SecondProduct* second = nullptr, bool bt_is_split = false,
                     const Plan* split_plan = nullptr) {
@@ -809,6 +884,13 @@ static int gemm_run(const pml_hip_gemm_desc& d, int mfma_kind, int tile, void* b
   if (((uintptr_t)a & 15) != 0) return fail("gemm_invoke: A must be 16-byte aligned");
   if (d.init_kind && !init) return fail("gemm_invoke: the plan expects an initial value");
   const int es = dt_size(d.in_dtype);
+  if (!b || d.b_layout) {
+    if (direct.rows >= 0) tile = direct.rows;
+  } else if (direct.given >= 0 && reads_b_as_given(d, mfma_kind, b, direct.given)) {
+    tile = direct.given;
+  } else if (direct.rows >= 0 && mfma_kind == KIND_F32) {
+    tile = direct.rows;
+  }
   const bool b_as_given = reads_b_as_given(d, mfma_kind, b, tile);
   if (b && !d.b_layout && !b_as_given && check(transpose_pack(es, b, bt, d.k, d.n, d.ldb, bt_ld, (hipStream_t)s), "transpose_pack"))
     return 1;
@@ -888,7 +970,7 @@ int pml_hip_gemm_invoke(int64_t plan, const void* a, const void* b, void* c, con
   const bool split = p->bt_is_split;
   // a right-hand side that this run transposes overwrites the packed copy
   if (b && !p->gemm.b_layout && !reads_b_as_given(p->gemm, p->mfma_kind, b, p->tile)) p->bt_is_split = false;
-  return gemm_run(p->gemm, p->mfma_kind, p->tile, p->bt, p->bt_ld, p->packed, a, b, c, init, operands, outs, s, nullptr, split, p);
+  return gemm_run(p->gemm, p->mfma_kind, p->tile, p->direct, p->bt, p->bt_ld, p->packed, a, b, c, init, operands, outs, s, nullptr, split, p);
 }
 
 int pml_hip_gemm_invoke2(int64_t plan, const void* a, const void* b, void* c, const void* init, const void* a2, const void* b2,
@@ -902,7 +984,7 @@ int pml_hip_gemm_invoke2(int64_t plan, const void* a, const void* b, void* c, co
   sp.init2 = init2;
   sp.bt2 = p->bt2;
   sp.packed2 = p->packed2;
-  return gemm_run(p->gemm, p->mfma_kind, p->tile, p->bt, p->bt_ld, p->packed, a, b, c, init, operands, outs, s, &sp);
+  return gemm_run(p->gemm, p->mfma_kind, p->tile, p->direct, p->bt, p->bt_ld, p->packed, a, b, c, init, operands, outs, s, &sp);
 }
 
 int pml_hip_gemm_run_static(const pml_hip_gemm_desc* d, const void* a, const void* b, void* c, const void* init,
@@ -925,7 +1007,7 @@ int pml_hip_gemm_run_static(const pml_hip_gemm_desc* d, const void* a, const voi
   const bool plain = mode == 1 || mode == 2 || tail_requant(d->tail, d->out_dtype, d->c_dtype, mode, nullptr);
   // (no workspace may be allocated here: the K loop is never split over workgroups)
   const int tile = choose_tile(d->m, d->n, d->k * dt_size(d->in_dtype), kind, plain, PML_HIP_FLAG_TILE_OF(d->flags), /*allow_split=*/false);
-  return gemm_run(*d, kind, tile, bt, d->k, false, a, b, c, init, operands, outs, s);
+  return gemm_run(*d, kind, tile, direct_tiles(*d, kind), bt, d->k, false, a, b, c, init, operands, outs, s);
 }
 
 // ---------------------------------------------------------------------------
@@ -1019,6 +1101,7 @@ int64_t pml_hip_conv2d_dispatch(const pml_hip_conv2d_desc* d) {
       return 0;
     }
   }
+  if (!via_s2d && !via_patches && PML_HIP_FLAG_TILE_OF(d->flags) < 0) p->tile_direct = direct_tile_of(M, d->co, K * es, kind);
   if (!via_s2d && !via_patches) prepare_split(p, M, d->co, d->kh * d->kw * ((d->ci * es + 127) / 128));
   if (p->tile == TILE_64x64_KSPLIT && !p->ws) p->tile = TILE_64x64;
   // (whole 128-byte chunks per filter tap, so that no chunk of heads + remainders straddles two taps)
@@ -1054,6 +1137,7 @@ int64_t pml_hip_conv2d_dispatch(const pml_hip_conv2d_desc* d) {
                 (long long)d->oh, (long long)d->ow, (long long)M, (long long)d->co, (long long)K, p->halo_lds ? (p->halo_variant == 3 ? "256x64 resident filter, in registers" : p->halo_variant ? "256x64 resident filter, pipelined 3x3" : "256x64 resident filter") : tile_name(p->tile));
   p->text = buf;
   if (kind == KIND_F32X3) p->text += " mfma=3 x f32_32x32x16_bf16 (fp32 split into bf16 head + remainder)";
+  if (p->tile_direct >= 0 && !p->halo_lds) p->text += std::string(", with a packed filter ") + tile_name(p->tile_direct);
   if (via_patches) p->text += " via patch matrix (k padded to " + std::to_string(p->kpad) + ")";
   if (via_s2d) {
     p->text += " over 2x2 pixel blocks (" + std::to_string(p->s2d_ka) + "x" + std::to_string(p->s2d_kaw) + " block taps of " +
@@ -1196,7 +1280,8 @@ int pml_hip_conv2d_invoke(int64_t plan, const void* input, const void* filter, v
   if (p->halo_lds)
     return check(conv_halo_launch(p->mfma_kind, g, p->halo_lds, p->n_cus, (hipStream_t)s), "conv_halo_launch");
   split_args(p, g);
-  return check(igemm_launch(p->b_split ? KIND_F32X3P : p->mfma_kind, p->tile, true, g, (hipStream_t)s), "igemm_launch");
+  const int tile = !filter && p->tile_direct >= 0 ? p->tile_direct : p->tile;
+  return check(igemm_launch(p->b_split ? KIND_F32X3P : p->mfma_kind, tile, true, g, (hipStream_t)s), "igemm_launch");
 }
 
 int pml_hip_gemm_pack_b(int64_t plan, const void* b, pml_hip_stream s) {

@@ -1,0 +1,141 @@
+"""The direct tiles (csrc/direct.hip): 16 x 16 and 32 x 32 results per workgroup, eight wavefronts sharing its K, fragments
+straight from memory.  Against float64 (int8: exact) where tiles, K steps and the
+wavefronts' shares end raggedly."""
+import ctypes
+
+import numpy as np
+import pytest
+
+import test_kernels_gpu as T
+from oracle import tile_oracle as E
+from plaidml_amd import hipkernels as hk
+
+pytestmark = pytest.mark.gpu
+TILES = ['16x16w8', '32x32w8']
+
+
+@pytest.fixture(scope='module', autouse=True)
+def _device():
+    hk.init(0)
+
+
+def operands(kind, M, N, K, seed):
+    rng = np.random.default_rng(seed)
+    if kind == 'i8':
+        return rng.integers(-127, 128, (M, K), dtype=np.int8), rng.integers(-127, 128, (K, N), dtype=np.int8)
+    A, B = rng.standard_normal((M, K)).astype(np.float32), rng.standard_normal((K, N)).astype(np.float32)
+    return (E.round_bf16(A), E.round_bf16(B)) if kind == 'bf16' else (A, B)
+
+
+def check(got, want, kind, K):
+    # sums of K terms of size one: fp32 rounds every partial sum (at most sqrt(K) in size) to 2^-24, K of them in a row
+    # at the very worst; a bf16 result is rounded once more, to 2^-9 of its value
+    if kind == 'i8':
+        np.testing.assert_array_equal(got, want)
+    else:
+        np.testing.assert_allclose(got, want, rtol=2.0 ** -8 if kind == 'bf16' else 1e-6, atol=2.0 ** -24 * K * np.sqrt(K) + 1e-6)
+
+
+# one row; N odd (the right-hand side cannot be read as it lies), N a multiple of 4 and of 64; K of one chunk, of a partial
+# step, of fewer steps than wavefronts, of one step more than whole shares; more tiles than CUs
+SIZES = [(1, 1, 16), (1, 20, 32), (15, 17, 80), (16, 64, 512), (17, 68, 528), (33, 130, 1040), (49, 96, 2048), (70, 36, 272), (1000, 260, 48)]
+
+
+@pytest.mark.parametrize('kind', ['f32', 'bf16', 'i8'])
+@pytest.mark.parametrize('tile', TILES + [None])
+@pytest.mark.parametrize('M,N,K', SIZES)
+def test_gemm(kind, tile, M, N, K, monkeypatch):
+    if tile:
+        monkeypatch.setitem(T.FORCED, 'flags', hk.flag_tile(tile))
+    A, B = operands(kind, M, N, K, M + N + K)
+    want = A.astype(np.float64) @ B.astype(np.float64)
+    if kind == 'i8':
+        check(T.run_gemm(A, B, hk.I8, hk.I32, invokes=2), want.astype(np.int64), kind, K)
+    elif kind == 'f32':
+        bias = np.linspace(-1, 1, N, dtype=np.float32)
+        tail = hk.make_tail(ops=[(hk.EPI_RELU, hk.F32, 0, 0, 0.0)])
+        got = T.run_gemm(A, B, hk.F32, hk.F32, init=bias, init_strides=(0, 1), init_dt=hk.F32, tail=tail)
+        check(got, np.maximum(want + bias, 0), kind, K)
+    else:
+        res = E.round_bf16(np.random.default_rng(3).standard_normal((M, N)).astype(np.float32))
+        tail = hk.make_tail(ops=[(hk.EPI_ADD, hk.BF16, hk.OPND_TENSOR, 0, 0.0)], operands=[(hk.BF16, N, 1)])
+        got = E.bf16_from_bits(T.run_gemm(T.bf16(A), T.bf16(B), hk.BF16, hk.BF16, tail=tail, operands=[T.bf16(res)]))
+        # (two roundings to bf16, the first of a sum of size sqrt(K))
+        np.testing.assert_allclose(got, want + res, rtol=2.0 ** -8, atol=2.0 ** -8 * 4 * np.sqrt(K))
+
+
+@pytest.mark.parametrize('tile', TILES)
+def test_int8_requantised(tile, monkeypatch):
+    monkeypatch.setitem(T.FORCED, 'flags', hk.flag_tile(tile))
+    M, N, K = 37, 76, 336
+    A, B = operands('i8', M, N, K, 5)
+    scale = np.full(N, 2.0 ** -12, np.float32)
+    tail = hk.make_tail(ops=[(hk.EPI_CAST, hk.F32, 0, 0, 0.0), (hk.EPI_MUL, hk.F32, hk.OPND_TENSOR, 0, 0.0),
+                             (hk.EPI_MAX_GT, hk.F32, hk.OPND_IMM, 0, -127.0), (hk.EPI_MIN, hk.F32, hk.OPND_IMM, 0, 127.0),
+                             (hk.EPI_ROUND, hk.F32, 0, 0, 0.0), (hk.EPI_CAST, hk.I8, 0, 0, 0.0)], operands=[(hk.F32, 0, 1)])
+    got = T.run_gemm(A, B, hk.I8, hk.I32, c_dt=hk.I8, tail=tail, operands=[scale])
+    v = np.clip((A.astype(np.int64) @ B.astype(np.int64)) / 4096.0, -127, 127)
+    np.testing.assert_array_equal(got, (np.sign(v) * np.floor(np.abs(v) + 0.5)).astype(np.int8))
+
+
+@pytest.mark.parametrize('kind', ['f32', 'bf16', 'i8'])
+@pytest.mark.parametrize('tile', TILES + [None])
+@pytest.mark.parametrize('shape,k,co,stride', [((1, 7, 7, 64), 3, 48, 1), ((2, 9, 5, 16), 3, 20, 2), ((1, 14, 14, 80), 5, 33, 1), ((3, 6, 6, 32), 1, 64, 2)])
+def test_conv(kind, tile, shape, k, co, stride, monkeypatch):
+    flags = hk.flag_conv(hk.CONV_IGEMM) | (hk.flag_tile(tile) if tile else 0)
+    monkeypatch.setitem(T.FORCED, 'flags', flags)
+    rng = np.random.default_rng(co)
+    I, F = (rng.integers(-9, 10, s).astype(np.float32) for s in (shape, (k, k, shape[3], co)))  # exact sums in every type
+    dt, out, cast = {'f32': (hk.F32, hk.F32, lambda a: a), 'bf16': (hk.BF16, hk.BF16, T.bf16), 'i8': (hk.I8, hk.I32, lambda a: a.astype(np.int8))}[kind]
+    got = T.run_conv(cast(I), cast(F), dt, out, stride=stride, packed=True)
+    n, h, w, _ = shape
+    oh, ow = -(-h // stride), -(-w // stride)
+    ph, pw = max(0, (oh - 1) * stride + k - h) // 2, max(0, (ow - 1) * stride + k - w) // 2
+    pad = np.zeros((n, h + 2 * k, w + 2 * k, shape[3]))
+    pad[:, ph:ph + h, pw:pw + w] = I
+    want = sum(pad[:, y:y + (oh - 1) * stride + 1:stride, x:x + (ow - 1) * stride + 1:stride] @ F[y, x].astype(np.float64) for y in range(k) for x in range(k))
+    if kind == 'bf16':
+        np.testing.assert_array_equal(E.bf16_from_bits(got), E.round_bf16(want.astype(np.float32)))
+    else:
+        np.testing.assert_array_equal(got, want)
+
+
+@pytest.mark.parametrize('stride', [0, 2])
+def test_two_products(stride):
+    """A.B + A2.B2 over rows packed once: a wavefront's share of K begins in the first product and ends in the second."""
+    rng = np.random.default_rng(21)
+    OH, K1, K2, N = 7, 520, 264, 136
+    M = OH * OH
+    A, A2, B, B2 = (E.round_bf16(rng.standard_normal(s).astype(np.float32)) for s in ((M, K1), (M, K2), (K1, N), (K2, N)))
+    side = (OH - 1) * 2 + 1
+    image = np.zeros((side, side, K2), np.float32)
+    image[::2, ::2] = A2.reshape(OH, OH, K2)
+    d = hk.GemmDesc()
+    d.in_dtype = d.out_dtype = d.c_dtype = hk.BF16
+    d.m, d.n, d.k, d.lda, d.ldb, d.ldc = M, N, K1, K1, N, N
+    d.k2, d.lda2, d.ldb2 = K2, K2, N
+    if stride:
+        d.a2_stride, d.a2_h, d.a2_w, d.a2_oh, d.a2_ow = stride, side, side, OH, OH
+    L = hk.lib()
+    plan = L.pml_hip_gemm_dispatch(ctypes.byref(d))
+    assert plan and 'wavefronts sharing K' in hk.describe(plan)
+    dA, dB, dA2, dB2 = (hk.DeviceBuffer.from_numpy(T.bf16(x)) for x in (A, B, image if stride else A2, B2))
+    dC, none = hk.DeviceBuffer(M * N * 2), hk.ptr_array([])
+    hk.check(L.pml_hip_gemm_pack_b(plan, dB.ptr, None))
+    hk.check(L.pml_hip_gemm_pack_b2(plan, dB2.ptr, None))
+    hk.check(L.pml_hip_gemm_invoke2(plan, dA.ptr, None, dC.ptr, None, dA2.ptr, None, None, none, none, None))
+    hk.check(L.pml_hip_stream_sync(None))
+    check(E.bf16_from_bits(dC.to_numpy(np.uint16, (M, N))), A.astype(np.float64) @ B + A2.astype(np.float64) @ B2, 'bf16', K1 + K2)
+    L.pml_hip_plan_free(plan)
+
+
+@pytest.mark.parametrize('kind', ['f32', 'bf16', 'i8'])
+@pytest.mark.parametrize('M,N,K', [(49, 512, 2048), (300, 72, 2064)])
+def test_split_over_workgroups_by_name(kind, M, N, K, monkeypatch):
+    """The two-launch split, which the direct tiles otherwise replace for most of these shapes."""
+    monkeypatch.setitem(T.FORCED, 'flags', hk.flag_tile('64x64ks'))
+    A, B = operands(kind, M, N, K, 9)
+    dt, cast = {'f32': (hk.F32, lambda a: a), 'bf16': (hk.BF16, T.bf16), 'i8': (hk.I8, lambda a: a)}[kind]
+    got = T.run_gemm(cast(A), cast(B), dt, hk.I32 if kind == 'i8' else dt, invokes=2)
+    want = A.astype(np.float64) @ B.astype(np.float64)
+    check(E.bf16_from_bits(got) if kind == 'bf16' else got, want, kind, K)
