@@ -325,6 +325,9 @@ struct StridedArgs {
 };
 void strided_plan(StridedArgs* a, bool bf, bool conv, int n_cus, int* mi);
 hipError_t strided_launch(const StridedArgs& a, bool bf, bool conv, int mi, hipStream_t s);
+// Products with few result tiles: rows of the direct tile a shape takes (0: none), and its launch (`splits` and `ws` unused).
+int product_direct_rows(const StridedArgs& a, bool bf, int n_cus);
+hipError_t product_direct_launch(const StridedArgs& a, bool bf, int rows, hipStream_t s);
 struct Col2imArgs {
   const float* cols;  // [N][OH][OW][KH][KW][CI]
   void* out;          // [N][H][W][CI]

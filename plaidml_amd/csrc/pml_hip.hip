@@ -83,7 +83,7 @@ struct Plan {
   // whole 16-byte vectors in `padded`), one of a larger stride a product into `cols`, images `grad_chunk` at a time
   StridedArgs strided;
   bool strided_bf = false, strided_conv = false;
-  int strided_mi = 1, grad_which = 0;
+  int strided_mi = 1, grad_which = 0, product_rows = 0;
   Plan* sub = nullptr;
   void *padded = nullptr, *cols = nullptr;
   int64_t co_pad = 0, grad_chunk = 0;
@@ -1530,13 +1530,16 @@ int64_t pml_hip_product_dispatch(const pml_hip_product_desc* d) {
       o.cs = d->tail.operand_col_stride[op.operand];
     }
   }
-  if (!prepare_strided(p)) {
+  strided_plan(&a, bf, false, device_cus(), &p->strided_mi);
+  p->product_rows = product_direct_rows(a, bf, device_cus());
+  if (!p->product_rows && !prepare_strided(p)) {
     delete p;
     return 0;
   }
   char buf[256];
   std::snprintf(buf, sizeof buf, "product %s batch=%lld m=%lld n=%lld k=%lld tile=%dx%d splits=%d", bf ? "bf16" : "f32", (long long)batches,
-                (long long)d->m, (long long)d->n, (long long)d->k, 64 * p->strided_mi, 64 * p->strided_mi, a.splits);
+                (long long)d->m, (long long)d->n, (long long)d->k, p->product_rows ? p->product_rows : 64 * p->strided_mi,
+                p->product_rows ? 64 : 64 * p->strided_mi, p->product_rows ? 1 : a.splits);
   p->text = buf;
   return (int64_t)(intptr_t)p;
 }
@@ -1558,6 +1561,7 @@ int pml_hip_product_invoke(int64_t plan, const void* a, const void* b, void* c, 
     if (!operands || !operands[op.operand]) return fail("product_invoke: missing tail operand");
     g.ops[i].ptr = operands[op.operand];
   }
+  if (p->product_rows) return check(product_direct_launch(g, p->strided_bf, p->product_rows, (hipStream_t)s), "product_direct_launch");
   return check(strided_launch(g, p->strided_bf, false, p->strided_mi, (hipStream_t)s), "strided_launch");
 }
 

@@ -21,6 +21,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 
 #include "device_common.h"
 #include "plans.h"
@@ -487,7 +488,251 @@ hipError_t launch_modes(const StridedArgs& a, int amode, int bmode, hipStream_t 
   return bmode == ROWS_K ? launch_tile<BF, ROWS_M, ROWS_K, MI, MI>(a, s) : launch_tile<BF, ROWS_M, ROWS_M, MI, MI>(a, s);
 }
 
+// Few result tiles: the direct form (direct.hip has the reasons), over rows of any alignment.  16 MB x 64 results per
+// workgroup; its eight wavefronts share K and load fragments from memory into registers, the whole steps of K without a
+// check per lane (rows past the last one are read as the last one and never stored), U steps in flight; what is left of K
+// after the last whole step is the last wavefront's.  A lane holds the columns 4 r .. 4 r + 3 of a 16-row block: from a
+// [K][N] right-hand side four neighbours of every K-row, turned with v_perm (bf16) or by naming (fp32), near the right edge
+// the last four columns instead; from an [N][K] one four rows.  The partial tiles meet in LDS and are added in wavefront order.
+template <bool BF, int BMODE, int MB>
+__global__ __launch_bounds__(512, 4) void product_direct_kernel(StridedArgs p_by_value) {
+  const StridedArgs& p = *(const StridedArgs*)(const __attribute__((address_space(4))) void*)__builtin_amdgcn_kernarg_segment_ptr();
+  constexpr int kWaves = 8, TM = 16 * MB, TN = 64, CS = TN + 4, ES = BF ? 2 : 4;
+  constexpr int E = 16 / ES, KS = 4 * E;  // K-values per lane and step, per step
+  constexpr int U = MB == 1 ? 4 : 2, NA = BF ? 1 : 2;
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  float* const parts = (float*)smem;  // [wavefront][TM][CS]
+  const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+
+  // XCD x (workgroup ids x, x + 8, ...) takes a run of tiles, the rows of a column block one after the other
+  const unsigned nb = gridDim.x, x = blockIdx.x & 7u, rem = nb & 7u;
+  unsigned t = x * (nb >> 3) + (x < rem ? x : rem) + (blockIdx.x >> 3);
+  const int64_t m0 = (int64_t)(t % (unsigned)p.tiles_m) * TM;
+  t /= (unsigned)p.tiles_m;
+  const int64_t n0 = (int64_t)(t % (unsigned)p.tiles_n) * TN;
+  t /= (unsigned)p.tiles_n;
+  int64_t a_at = 0, b_at = 0, c_at = 0;
+  for (int d = p.n_batch - 1; d >= 0; --d) {
+    const unsigned sz = (unsigned)p.batch[d], i = t % sz;
+    t /= sz;
+    a_at += i * p.a_batch[d];
+    b_at += i * p.b_batch[d];
+    c_at += i * p.c_batch[d];
+  }
+
+  const int64_t steps = p.K / KS;  // whole ones
+  const int64_t per = (steps + kWaves - 1) / kWaves, first = wave * per;
+  const int64_t last = first + per < steps ? first + per : steps;
+
+  const char* a_ptr[MB];
+#pragma unroll
+  for (int i = 0; i < MB; ++i) {
+    const int64_t m = m0 + 16 * i + r;
+    a_ptr[i] = (const char*)p.A + (a_at + (m < p.M ? m : p.M - 1) * p.a_ms + g * E) * ES;
+  }
+  const char* b_ptr[BMODE == ROWS_K ? 4 : 1];
+  const int64_t n = n0 + 4 * r;
+  if constexpr (BMODE == ROWS_K) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) b_ptr[j] = (const char*)p.B + (b_at + (n + j < p.N ? n + j : p.N - 1) * p.b_ns + g * E) * ES;
+  } else {
+    b_ptr[0] = (const char*)p.B + (b_at + (n + 4 <= p.N ? n : p.N - 4) + g * E * p.b_ks) * ES;  // (N is at least four)
+  }
+  const int64_t b_pitch = p.b_ks * ES;
+
+  f32x4_t sums[MB][4][NA];
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int c = 0; c < NA; ++c) sums[i][j][c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+  auto multiply = [&](const Words<4> (&fa)[MB], const uint32_t (&raw)[16]) {
+    Words<4> frag[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        if constexpr (BMODE == ROWS_K)
+          frag[j].w[q] = raw[4 * j + q];
+        else if constexpr (BF)
+          frag[j].w[q] = __builtin_amdgcn_perm(raw[4 * q + 2 + (j >> 1)], raw[4 * q + (j >> 1)], (j & 1) ? 0x07060302u : 0x05040100u);
+        else
+          frag[j].w[q] = raw[4 * q + j];
+      }
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if constexpr (BF) {
+          bf16x8_t av, bv;
+          __builtin_memcpy(&av, &fa[i], 16);
+          __builtin_memcpy(&bv, &frag[j], 16);
+          sums[i][j][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bv, av, sums[i][j][0], 0, 0, 0);
+        } else {
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            sums[i][j][q % NA] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(frag[j].w[q]), __uint_as_float(fa[i].w[q]), sums[i][j][q % NA], 0, 0, 0);
+        }
+      }
+  };
+
+  for (int64_t s0 = first; s0 < last; s0 += U) {
+    Words<4> fa[U][MB];
+    uint32_t raw[U][16];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int64_t k = (s0 + u < last ? s0 + u : last - 1) * KS;  // (a step past the run is read again and not multiplied)
+#pragma unroll
+      for (int i = 0; i < MB; ++i) fa[u][i] = load_words<4>(a_ptr[i] + k * ES);
+      if constexpr (BMODE == ROWS_K) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const Words<4> v = load_words<4>(b_ptr[j] + k * ES);
+#pragma unroll
+          for (int q = 0; q < 4; ++q) raw[u][4 * j + q] = v.w[q];
+        }
+      } else {
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+          const Words<ES> v = load_words<ES>(b_ptr[0] + (k + e) * b_pitch);
+#pragma unroll
+          for (int q = 0; q < ES; ++q) raw[u][ES * e + q] = v.w[q];
+        }
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (s0 + u < last) multiply(fa[u], raw[u]);
+  }
+
+  const int left = (int)(p.K - steps * KS);
+  if (left > 0 && wave == kWaves - 1) {
+    // value by value, zeros past the end on both sides
+    const int64_t k = steps * KS;
+    Words<4> fa[MB];
+    uint32_t raw[16];
+    auto value = [&](const char* at, bool ok) -> uint32_t { return !ok ? 0u : BF ? *(const uint16_t*)at : *(const uint32_t*)at; };
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const char* const at = a_ptr[i] + k * ES + 4 * q;
+        const int kk = g * E + (BF ? 2 * q : q);
+        fa[i].w[q] = value(at, kk < left) | (BF ? value(at + 2, kk + 1 < left) << 16 : 0u);
+      }
+    if constexpr (BMODE == ROWS_K) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const char* const at = b_ptr[j] + k * ES + 4 * q;
+          const int kk = g * E + (BF ? 2 * q : q);
+          raw[4 * j + q] = value(at, kk < left) | (BF ? value(at + 2, kk + 1 < left) << 16 : 0u);
+        }
+    } else {
+#pragma unroll
+      for (int e = 0; e < E; ++e)
+#pragma unroll
+        for (int q = 0; q < ES; ++q) {
+          const char* const at = b_ptr[0] + (k + e) * b_pitch + 4 * q;
+          raw[ES * e + q] = value(at, g * E + e < left) | (BF ? value(at + 2, g * E + e < left) << 16 : 0u);
+        }
+    }
+    multiply(fa, raw);
+  }
+
+  // lane r, g holds row r and, of block j, the rows 4 g + e: column 4 (4 g + e) + j
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      f32x4_t q = {sums[i][0][0][e], sums[i][1][0][e], sums[i][2][0][e], sums[i][3][0][e]};
+      if constexpr (NA == 2) q += f32x4_t{sums[i][0][1][e], sums[i][1][1][e], sums[i][2][1][e], sums[i][3][1][e]};
+      *(f32x4_t*)&parts[(wave * TM + 16 * i + r) * CS + 16 * g + 4 * e] = q;
+    }
+  __syncthreads();
+  const int lr = tid / 16, lc = (tid & 15) * 4;
+  const int64_t m = m0 + lr, col = n0 + lc;
+  if (lr >= TM || m >= p.M || col >= p.N) return;
+  const float* const at = &parts[lr * CS + lc];
+  f32x4_t sum = *(const f32x4_t*)at;
+#pragma unroll
+  for (int w = 1; w < kWaves; ++w) sum += *(const f32x4_t*)(at + w * (TM * CS));
+  const int live = p.N - col < 4 ? (int)(p.N - col) : 4;
+  float v[4] = {sum[0], sum[1], sum[2], sum[3]};
+  if (BMODE != ROWS_K && live < 4) {  // the quad holds the last four columns: its own are the last `live` of them
+    v[0] = live == 3 ? sum[1] : live == 2 ? sum[2] : sum[3];
+    v[1] = live == 3 ? sum[2] : sum[3];
+    v[2] = sum[3];
+  }
+  const int64_t c_row = c_at + m * p.c_ms;
+  strided_tail(p, v, c_row, col, live);
+  store_results(p, p.C, c_row + col, v, live);
+}
+
+template <bool BF, int BMODE, int MB>
+hipError_t launch_direct(const StridedArgs& a, hipStream_t s) {
+  const size_t lds = (size_t)8 * 16 * MB * 68 * 4;
+  auto kern = product_direct_kernel<BF, BMODE, MB>;
+  static DynamicLdsLimit limit;
+  if (hipError_t e = limit.ensure((const void*)kern, lds); e != hipSuccess) return e;
+  StridedArgs b = a;
+  b.tiles_m = (int)((a.M + 16 * MB - 1) / (16 * MB));
+  b.tiles_n = (int)((a.N + 63) / 64);
+  int64_t nb = (int64_t)b.tiles_m * b.tiles_n;
+  for (int d = 0; d < a.n_batch; ++d) nb *= a.batch[d];
+  if (nb <= 0 || nb >= ((int64_t)1 << 31)) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(kern, dim3((unsigned)nb), dim3(512), lds, s, b);
+  return hipGetLastError();
+}
+
 }  // namespace
+
+// Rows of the direct tile (16 or 32), 0: the tiles through LDS that strided_plan has laid out.  Both sides are priced in
+// microseconds from 25 shapes per type and layout (1 to 2000 rows, K of 32 to 2047, batches up to 96).  Direct: 2.6 plus, per
+// round of one tile on each CU, 0.8 (1.8 where bf16 has a broken last step of K) and the tile's operand bytes at 38 KB a
+// microsecond for fp32 with 16 rows, 32 with 32 rows (the matrix cores), bf16 25 from [K][N] and 17.5 from [N][K] (16-byte
+// loads at 2-byte alignment).  Through LDS: 3 and 1.65 a slab (bf16 [K][N] 3.6 and 1.55, [N][K] 4 and 1.1); split, 1.8 more
+// and the partial results written and read at 3 TB/s.  A direct tile has to be 8 % ahead.
+//   us, through LDS -> direct              fp32 [K][N]       bf16 [K][N]       bf16 [N][K]
+//   3 x 1001, K = 333                    14.9 ->  5.0      13.2 ->  6.4      10.6 ->  7.7
+//   300 x 777, K = 1001                  20.5 -> 10.9      13.9 ->  9.9      12.6 (15.1)
+//   1000 x 1001, K = 1001                55.3 -> 32.1      28.0 -> 19.0      21.1 (25.3)
+//   20 of 100 x 77, K = 100              10.4 ->  4.6       8.5 ->  5.2       8.0 ->  4.9
+//   50 x 777, K = 1777: stays split      13.6 (22.1)       12.6 (17.8)       11.4 (23.4)
+int product_direct_rows(const StridedArgs& a, bool bf, int n_cus) {
+  const bool nk = a.b_ks == 1;
+  if (a.a_ks != 1 || (!nk && (a.b_ns != 1 || a.N < 4))) return 0;
+  double batches = 1;
+  for (int d = 0; d < a.n_batch; ++d) batches *= (double)a.batch[d];
+  const double kb = (double)a.K * (bf ? 2 : 4);
+  auto direct_us = [&](int64_t rows) {
+    const double tiles = batches * (double)((a.M + rows - 1) / rows) * (double)((a.N + 63) / 64);
+    const double rate = bf ? (nk ? 17.5e3 : 25e3) : (rows == 16 ? 38e3 : 32e3);
+    const double live = (double)(rows == 16 ? std::min<int64_t>(a.M, 16) : 32) + 64;
+    return 2.6 + std::ceil(tiles / n_cus) * ((bf && a.K % 32 != 0 ? 1.8 : 0.8) + live * kb / rate);
+  };
+  const double slabs = (double)((std::min(a.K, a.k_per_split) + (bf ? 63 : 31)) / (bf ? 64 : 32));
+  double lds_us = !bf ? 3 + 1.65 * slabs : nk ? 4 + 1.1 * slabs : 3.6 + 1.55 * slabs;
+  if (a.splits > 1) lds_us += 1.8 + 8.0 * a.splits * (double)a.ws_rows * (double)a.ws_pitch / 3e6;
+  const double small = direct_us(16), large = direct_us(32);
+  if (std::min(small, large) > 0.92 * lds_us) return 0;
+  return small <= large ? 16 : 32;
+}
+
+hipError_t product_direct_launch(const StridedArgs& a, bool bf, int rows, hipStream_t s) {
+  const bool nk = a.b_ks == 1;
+  if (bf) {
+    if (rows == 16) return nk ? launch_direct<true, ROWS_K, 1>(a, s) : launch_direct<true, ROWS_M, 1>(a, s);
+    return nk ? launch_direct<true, ROWS_K, 2>(a, s) : launch_direct<true, ROWS_M, 2>(a, s);
+  }
+  if (rows == 16) return nk ? launch_direct<false, ROWS_K, 1>(a, s) : launch_direct<false, ROWS_M, 1>(a, s);
+  return nk ? launch_direct<false, ROWS_K, 2>(a, s) : launch_direct<false, ROWS_M, 2>(a, s);
+}
+
 // The tile and, for few tiles and a long K, the split: 128 x 128 where that still gives every CU a workgroup (half the
 // operand traffic per result), 64 x 64 otherwise; K is split when the tiles alone leave CUs idle, into runs of at least
 // four slabs, for about three workgroups per CU (their LDS fits four times into one).

@@ -44,6 +44,27 @@ def test_product(dtype, b, m, n, k, ta, tb):
 
 
 @pytest.mark.parametrize('dtype', ['f32', 'bf16'])
+@pytest.mark.parametrize('tb', [0, 1])
+@pytest.mark.parametrize('b,m,n,k', [
+    (1, 1, 4, 1), (1, 3, 66, 31), (1, 16, 61, 33), (2, 17, 67, 96), (1, 33, 131, 255), (3, 32, 65, 257), (1, 31, 5, 300), (9, 100, 77, 100)])
+def test_product_of_few_tiles(dtype, tb, b, m, n, k):
+    """Direct tiles of 16 or 32 rows by 64 columns: one, two and three columns past a quad, K short of a step, of whole steps
+    only, and with one value left; an infinity in the last row and column of B stays in its own results."""
+    rng = np.random.default_rng(m + n + k)
+    A, B = values(rng, (b, m, k), dtype), values(rng, (b, n, k) if tb else (b, k, n), dtype, k ** -0.5)
+    A = np.abs(A) + 1
+    (B[:, n - 1:, k - 1] if tb else B[:, k - 1, n - 1:])[...] = np.inf
+    X, Y = P.Placeholder(DT[dtype], A.shape), P.Placeholder(DT[dtype], B.shape)
+    bi, i, j, q = P.TensorIndexes(4)
+    C = P.Contraction().outShape(b, m, n).outAccess(bi, i, j).sum(X[bi, i, q] * (Y[bi, j, q] if tb else Y[bi, q, j])).build()
+    got, = P.Runner(P.Program('product', [X, Y], [C]), target='hip').run([P.round_bf16(A) if dtype == 'bf16' else A, B])
+    A = (P.round_bf16(A) if dtype == 'bf16' else A).astype(np.float64)
+    want = np.matmul(A, (B.transpose(0, 2, 1) if tb else B).astype(np.float64))
+    assert np.isposinf(got[..., -1]).all()
+    check(got[..., :-1], want[..., :-1], dtype)
+
+
+@pytest.mark.parametrize('dtype', ['f32', 'bf16'])
 @pytest.mark.parametrize('n,hw,ci,co,k,stride', [
     (2, 14, 64, 64, 3, 1), (1, 7, 3, 16, 3, 2), (3, 9, 19, 33, 5, 1), (2, 15, 70, 20, 3, 2), (1, 10, 5, 17, 1, 2), (2, 8, 24, 40, 1, 1),
     (1, 112, 3, 37, 5, 1), (5, 11, 130, 65, 3, 1), (1, 2, 8, 16, 3, 1), (4, 40, 16, 24, 5, 2)])
