@@ -157,8 +157,9 @@ const char* const kTileShort[PML_HIP_TILE_COUNT_] = {"64x64", "128x64", "128x128
 // int8 36 unless rows are whole 64-byte runs), and an LDS kernel that needs Bt pays for the transposed copy besides, 3 and
 // its bytes both ways at 2.2 TB/s:
 // bf16 512 x 512 x 512 9.4 -> 5.0, 1024^3 14.6 -> 10.6, 64 x 2048 x 2048 16.5 -> 8.8; fp32 128 x 4096 x 1024 23.4 -> 12.3.
-// kn_ldb: that right-hand side's row pitch in bytes (0: Bt); always: the better of the two whatever the LDS kernel takes
-int direct_tile_of(int64_t m, int64_t n, int64_t k_bytes, int kind, int64_t kn_ldb = 0, bool always = false) {
+// kn_ldb: that right-hand side's row pitch in bytes (0: Bt); always: the better of the two whatever the LDS kernel takes;
+// can_split: the LDS kernel may split K
+int direct_tile_of(int64_t m, int64_t n, int64_t k_bytes, int kind, int64_t kn_ldb = 0, bool always = false, bool can_split = true) {
   if (kind != KIND_F32 && kind != KIND_BF16 && kind != KIND_I8) return -1;
   auto tiles = [&](int64_t bm, int64_t bn) { return ((m + bm - 1) / bm) * ((n + bn - 1) / bn); };
   const double kb = (double)k_bytes;
@@ -173,7 +174,7 @@ int direct_tile_of(int64_t m, int64_t n, int64_t k_bytes, int kind, int64_t kn_l
   const int64_t slabs = (k_bytes + 127) / 128;
   double lds_us = 4.2 + (f32 ? 0.58 : kind == KIND_I8 ? 0.28 : 0.23) * (double)slabs;
   bool needs_bt = kind == KIND_BF16 || n % (16 / es) != 0 || kn_ldb % 16 != 0;
-  if (tiles(64, 64) <= 64 && k_bytes >= 2048) {
+  if (can_split && tiles(64, 64) <= 64 && k_bytes >= 2048) {
     int splits = 1, per = 0;
     igemm_split_plan(m, n, slabs, 256, &splits, &per);
     if (splits >= 2) {
@@ -784,7 +785,8 @@ static DirectTiles direct_tiles(const pml_hip_gemm_desc& d, int kind) {
   DirectTiles t;
   if (PML_HIP_FLAG_TILE_OF(d.flags) >= 0) return t;
   const int es = dt_size(d.in_dtype);
-  t.rows = direct_tile_of(d.m, d.n, (d.k + d.k2) * es, kind);
+  // (the launch of two products does not split K: one chain of all slabs otherwise)
+  t.rows = direct_tile_of(d.m, d.n, (d.k + d.k2) * es, kind, 0, false, /*can_split=*/d.k2 == 0);
   if (d.b_layout || d.k2 > 0 || (kind == KIND_F32 && t.rows < 0)) return t;
   t.given = direct_tile_of(d.m, d.n, d.k * es, kind, d.ldb * es, /*always=*/kind == KIND_F32);
   return t;
