@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <atomic>
 #include <cstdio>
 #include <cstdlib>
@@ -144,13 +145,16 @@ const char* const kTileShort[PML_HIP_TILE_COUNT_] = {"64x64", "128x64", "128x128
 
 // One of the direct tiles (direct.hip) where it beats the LDS kernels, or -1.  Both sides are priced in microseconds, from
 // measurements of 27 matrix products and 18 convolutions per element kind (one row to 3136, K of 64 to 4608; back to back
-// in a recorded graph): a direct kernel takes 2.6 plus, per round of one tile on each of 256 CUs, 0.8 (fp32 32 x 32: 1.9)
-// and its operand bytes at 40 KB a microsecond and CU.  An LDS kernel takes 4.2 plus its chain of 128-byte slabs (0.23 each,
-// int8 0.28, fp32 0.58), or -- K split over workgroups -- 5.2 (fp32 6.5) plus 0.4 per KB of K plus writing and reading the
-// partial tiles at 3 TB/s.  The prices meet the measurements to about 15 %; a direct tile has to be 5 % ahead.
+// in a recorded graph): a direct kernel takes 2.6 plus, per round of one tile on each of 256 CUs (fp32 and 32 x 64: whole
+// rounds), 0.8 (fp32 32 x 32: 1.9; 32 x 64, which replaces 32 x 32 beyond one round: bf16 1.6, int8 1.0, fp32 2.3) and its
+// operand bytes at 40 KB a microsecond and CU (32 x 64: bf16 50, int8 60, fp32 32).  An LDS kernel takes 4.2 plus its chain
+// of 128-byte slabs (0.23 each, int8 0.28, fp32 0.58), or -- K split over workgroups -- 5.2 (fp32 5.6) plus 0.4 per KB of K
+// plus writing and reading the partial tiles at 3 TB/s.  The prices meet the measurements to about 15 %; a direct tile has
+// to be 5 % ahead.
 //   us, before -> direct                       bf16              fp32              int8
 //   1 x 1000, K = 2048                     7.4 ->  5.0       9.3 ->  7.3       6.7 ->  4.3
 //   196 x 256, K = 1024                    7.5 ->  5.2       9.7 ->  6.5       6.4 ->  4.4
+//   784 x 512, K = 256: 32 x 64            5.1 ( 5.4)       9.6 ->  8.5       4.8 ->  4.5
 //   28 x 28 x 128 (*) 3 x 3 x 128          9.1 ->  7.7      11.1 (12.8)        7.4 ->  5.2
 //   49 x 512, K = 4608: stays split        8.6 (11.2)       12.9 (18.7)        7.6 ( 7.4)
 // A right-hand side that arrives with the call as [K][N]: tiles are then 16 or 32 x 64 (60 KB a microsecond; fp32 45,
@@ -165,11 +169,16 @@ int direct_tile_of(int64_t m, int64_t n, int64_t k_bytes, int kind, int64_t kn_l
   const double kb = (double)k_bytes;
   const int es = kind == KIND_BF16 ? 2 : (kind == KIND_I8 ? 1 : 4);
   const bool kn = kn_ldb > 0, f32 = kind == KIND_F32;
+  const bool wide_tiles = !kn && tiles(32, 32) > 256;  // (32 x 64 in the place of 32 x 32)
   const double rate = !kn ? 40e3 : f32 ? 45e3 : (kind == KIND_I8 && kn_ldb % 64 != 0) ? 36e3 : 60e3;
   auto direct_us = [&](int64_t side) {
-    const int64_t wide = kn ? 64 : side;
-    const double rounds = std::max(1.0, (double)tiles(side, wide) / 256);
-    return 2.6 + rounds * ((f32 && !kn && side == 32 ? 1.9 : 0.8) + (double)(std::min(m, side) + std::min(n, wide)) * kb / rate);
+    const bool w = wide_tiles && side == 32;
+    const int64_t wide = kn || w ? 64 : side;
+    double rounds = std::max(1.0, (double)tiles(side, wide) / 256);
+    if ((f32 && !kn) || w) rounds = std::ceil(rounds);
+    const double start = w ? (f32 ? 2.3 : kind == KIND_I8 ? 1.0 : 1.6) : f32 && !kn && side == 32 ? 1.9 : 0.8;
+    const double r = w ? (f32 ? 32e3 : kind == KIND_I8 ? 60e3 : 50e3) : rate;
+    return 2.6 + rounds * (start + (double)(std::min(m, side) + std::min(n, wide)) * kb / r);
   };
   const int64_t slabs = (k_bytes + 127) / 128;
   double lds_us = 4.2 + (f32 ? 0.58 : kind == KIND_I8 ? 0.28 : 0.23) * (double)slabs;
@@ -178,7 +187,7 @@ int direct_tile_of(int64_t m, int64_t n, int64_t k_bytes, int kind, int64_t kn_l
     int splits = 1, per = 0;
     igemm_split_plan(m, n, slabs, 256, &splits, &per);
     if (splits >= 2) {
-      lds_us = (f32 ? 6.5 : 5.2) + kb / 2500 + 8.0 * splits * (double)m * (double)n / 3e6;
+      lds_us = (f32 ? 5.6 : 5.2) + kb / 2500 + 8.0 * splits * (double)m * (double)n / 3e6;
       needs_bt = true;
     }
   }

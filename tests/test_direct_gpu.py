@@ -38,7 +38,7 @@ def check(got, want, kind, K):
 
 # one row; N odd (the right-hand side cannot be read as it lies), N a multiple of 4 and of 64; K of one chunk, of a partial
 # step, of fewer steps than wavefronts, of one step more than whole shares; more tiles than CUs
-SIZES = [(1, 1, 16), (1, 20, 32), (15, 17, 80), (16, 64, 512), (17, 68, 528), (33, 130, 1040), (49, 96, 2048), (70, 36, 272), (1000, 260, 48)]
+SIZES = [(1, 1, 16), (1, 20, 32), (15, 17, 80), (16, 64, 512), (17, 68, 528), (33, 130, 1040), (49, 96, 2048), (70, 36, 272), (1000, 260, 48), (1000, 270, 80)]
 
 
 @pytest.mark.parametrize('kind', ['f32', 'bf16', 'i8'])
