@@ -74,7 +74,7 @@ struct Plan {
   // K split over workgroups: workspace of partial tiles and how the slabs are shared out (splits < 2: no split)
   void* ws = nullptr;
   int sk_splits = 0, sk_per = 0, sk_pitch = 0;
-  // the direct tiles a product takes instead of `tile`, and the one a convolution takes with a packed filter (-1: none)
+  // the direct tiles a product takes instead of `tile`, and the one a convolution takes (-1: none)
   DirectTiles direct;
   int tile_direct = -1;
   // register-filter convolution: a filter packed once, in the order the kernel holds it in registers
@@ -1148,7 +1148,7 @@ int64_t pml_hip_conv2d_dispatch(const pml_hip_conv2d_desc* d) {
                 (long long)d->oh, (long long)d->ow, (long long)M, (long long)d->co, (long long)K, p->halo_lds ? (p->halo_variant == 3 ? "256x64 resident filter, in registers" : p->halo_variant ? "256x64 resident filter, pipelined 3x3" : "256x64 resident filter") : tile_name(p->tile));
   p->text = buf;
   if (kind == KIND_F32X3) p->text += " mfma=3 x f32_32x32x16_bf16 (fp32 split into bf16 head + remainder)";
-  if (p->tile_direct >= 0 && !p->halo_lds) p->text += std::string(", with a packed filter ") + tile_name(p->tile_direct);
+  if (p->tile_direct >= 0 && !p->halo_lds) p->text += std::string(", direct tile=") + tile_name(p->tile_direct);
   if (via_patches) p->text += " via patch matrix (k padded to " + std::to_string(p->kpad) + ")";
   if (via_s2d) {
     p->text += " over 2x2 pixel blocks (" + std::to_string(p->s2d_ka) + "x" + std::to_string(p->s2d_kaw) + " block taps of " +
@@ -1291,7 +1291,7 @@ int pml_hip_conv2d_invoke(int64_t plan, const void* input, const void* filter, v
   if (p->halo_lds)
     return check(conv_halo_launch(p->mfma_kind, g, p->halo_lds, p->n_cus, (hipStream_t)s), "conv_halo_launch");
   split_args(p, g);
-  const int tile = !filter && p->tile_direct >= 0 ? p->tile_direct : p->tile;
+  const int tile = p->tile_direct >= 0 ? p->tile_direct : p->tile;
   return check(igemm_launch(p->b_split ? KIND_F32X3P : p->mfma_kind, tile, true, g, (hipStream_t)s), "igemm_launch");
 }
 

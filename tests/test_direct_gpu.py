@@ -79,15 +79,16 @@ def test_int8_requantised(tile, monkeypatch):
 
 
 @pytest.mark.parametrize('kind', ['f32', 'bf16', 'i8'])
-@pytest.mark.parametrize('tile', TILES + [None])
-@pytest.mark.parametrize('shape,k,co,stride', [((1, 7, 7, 64), 3, 48, 1), ((2, 9, 5, 16), 3, 20, 2), ((1, 14, 14, 80), 5, 33, 1), ((3, 6, 6, 32), 1, 64, 2)])
-def test_conv(kind, tile, shape, k, co, stride, monkeypatch):
+@pytest.mark.parametrize('packed', [True, False])
+@pytest.mark.parametrize('tile', TILES + [None, '64x64ks'])
+@pytest.mark.parametrize('shape,k,co,stride', [((1, 7, 7, 64), 3, 48, 1), ((1, 7, 7, 512), 3, 96, 1), ((2, 9, 11, 96), 5, 40, 1), ((2, 9, 5, 16), 3, 20, 2), ((1, 14, 14, 80), 5, 33, 1), ((3, 6, 6, 32), 1, 64, 2)])
+def test_conv(kind, tile, packed, shape, k, co, stride, monkeypatch):
     flags = hk.flag_conv(hk.CONV_IGEMM) | (hk.flag_tile(tile) if tile else 0)
     monkeypatch.setitem(T.FORCED, 'flags', flags)
     rng = np.random.default_rng(co)
-    I, F = (rng.integers(-9, 10, s).astype(np.float32) for s in (shape, (k, k, shape[3], co)))  # exact sums in every type
+    I, F = (rng.integers(-9, 10, s).astype(np.float32) for s in (shape, (k, k, shape[3], co)))  # exact sums in every type (fp32: below 2^24)
     dt, out, cast = {'f32': (hk.F32, hk.F32, lambda a: a), 'bf16': (hk.BF16, hk.BF16, T.bf16), 'i8': (hk.I8, hk.I32, lambda a: a.astype(np.int8))}[kind]
-    got = T.run_conv(cast(I), cast(F), dt, out, stride=stride, packed=True)
+    got = T.run_conv(cast(I), cast(F), dt, out, stride=stride, packed=packed)
     n, h, w, _ = shape
     oh, ow = -(-h // stride), -(-w // stride)
     ph, pw = max(0, (oh - 1) * stride + k - h) // 2, max(0, (ow - 1) * stride + k - w) // 2
