@@ -503,8 +503,19 @@ bool Planner::tryProduct(size_t i) {
     m.s[0] = nn.range;
     swapped = true;
   }
-  int64_t all = m.range * nn.range;
-  for (const Group& g : B) all *= g.range;
+  // The kernel writes every result once, as if its indices were the only ones to reach it, so they have to cover the result
+  // once: in order of size each index's step in the result is the product of the ranges below it.  (An output access that is
+  // a sum of indices, O[i + j], can have as many index tuples as elements and still meet in some and leave others out.)
+  std::vector<Group> cover(B);
+  cover.push_back(m);
+  cover.push_back(nn);
+  std::sort(cover.begin(), cover.end(), [](const Group& x, const Group& y) { return x.s[0] < y.s[0]; });
+  int64_t all = 1;
+  for (const Group& g : cover) {
+    if (g.range == 1) continue;
+    if (g.s[0] != all) return false;
+    all *= g.range;
+  }
   if (base[0] != 0 || all != op.result->shape.elements()) return false;
   Step s;
   s.kind = Step::Product;

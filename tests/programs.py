@@ -99,6 +99,32 @@ def flatten_by_contraction(E, op):
     return E.Program('no_reduce', [I], [O]), [_rng(3).standard_normal((10, 10)).astype(np.float32)], EXACT
 
 
+def shared_results(E, op, out, step_i, batch=0, step_b=0, m=8, n=8, K=5, dtype_name='FLOAT32'):
+    """O[step_b b + step_i i + j] += A[(b,) i, k] * B[(b,) k, j]: a matrix product's index set whose results meet -- as many index
+    tuples as elements of O, some elements reached by several of them and others by none (they hold the sum's 0)."""
+    dt = getattr(E.DType, dtype_name)
+    rng = _rng(11)
+    lead = (batch,) if batch else ()
+    av, bv = rng.integers(-4, 5, lead + (m, K)).astype(np.float32), rng.integers(-4, 5, lead + (K, n)).astype(np.float32)
+    A, B = E.Placeholder(dt, av.shape), E.Placeholder(dt, bv.shape)
+    b, i, j, k = E.TensorIndexes(4)
+    if batch:
+        O = E.Contraction().outShape(out).outAccess(step_b * b + step_i * i + j).sum(A[b, i, k] * B[b, k, j]).build()
+    else:
+        O = E.Contraction().outShape(out).outAccess(step_i * i + j).sum(A[i, k] * B[k, j]).build()
+    return E.Program('shared_results', [A, B], [O]), [av, bv], EXACT
+
+
+SHARED_RESULTS = {  # (the last one covers its results once)
+    'shared_results_diagonals': lambda E, op: shared_results(E, op, 64, 1),
+    'shared_results_overlap': lambda E, op: shared_results(E, op, 4, 1, m=2, n=2),
+    'shared_results_gap': lambda E, op: shared_results(E, op, 8, 2, m=2, n=4),
+    'shared_results_batched': lambda E, op: shared_results(E, op, 256, 8, batch=4, step_b=8),
+    'shared_results_batched_bf16': lambda E, op: shared_results(E, op, 256, 8, batch=4, step_b=1, dtype_name='BFLOAT16'),
+    'shared_results_none': lambda E, op: shared_results(E, op, 64, 8),
+}
+
+
 def scatter_form_transposed_conv(E, op, N=2, H=6, CI=3, CO=4, dtype_name='FLOAT32'):
     """A stride-2 transposed convolution written from the input's point of view: every input pixel (x, y) adds its
     3x3 footprint to O[n, 2x + i - 1, 2y + j - 1, co].  Two output coordinates are sums of indices, many index
@@ -768,6 +794,7 @@ ALL = {
     'flatten_by_contraction': flatten_by_contraction,
     'scatter_form_transposed_conv': scatter_form_transposed_conv,
     'mirrored_sum_of_indices': mirrored_sum_of_indices,
+    **SHARED_RESULTS,
     'max_rows': max_rows,
     'use_default': use_default,
     'eltwise_mix': eltwise_mix,

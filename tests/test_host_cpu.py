@@ -62,6 +62,17 @@ def test_depthwise_temporary_gets_a_pitch_of_whole_lines():
     assert 'row pitch' not in t
 
 
+@pytest.mark.parametrize('name', sorted(programs.SHARED_RESULTS))
+def test_products_whose_results_meet_take_the_general_kernel(name):
+    """The product kernels write every result once: a result that several index tuples share, or that none reaches, is the
+    general kernel's, however many tuples there are."""
+    t = plan_of(programs.SHARED_RESULTS[name](E, op)[0])
+    if name.endswith('_none'):
+        assert 'product f32 m=8 n=8 k=5' in t and 'general' not in t, t
+    else:
+        assert 'contract (general)' in t and 'product' not in t, t
+
+
 def test_output_coordinates_that_are_sums_are_solved_for_one_index():
     """O[n, 2x + i - 1, 2y + j - 1, co]: the planner solves each such coordinate for its widest index (x, y), so the
     kernel's threads walk the taps and input channels only -- 7 indices (4 output coordinates + i, j, ci), not 11;
