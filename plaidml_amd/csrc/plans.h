@@ -334,6 +334,13 @@ struct Col2imArgs {
   int N, H, W, CI, OH, OW, KH, KW, SH, SW, PH, PW, DH, DW;
 };
 hipError_t col2im_launch(const Col2imArgs& a, bool bf, hipStream_t s);
+struct ConvBorderArgs {
+  const void *g, *f;  // [N][OH][OW][CO], [KH][KW][CI][CO]
+  void* out;          // [N][H][W][CI], the data gradient
+  int N, H, W, CI, OH, OW, CO, KH, KW, PH, PW, DH, DW;
+  int y0, y1, x0, x1;  // pixels all of whose taps lie inside the gradient: y0 <= y < y1, x0 <= x < x1
+};
+hipError_t conv_border_launch(const ConvBorderArgs& a, bool bf, hipStream_t s);
 hipError_t pad_rows_launch(int es, const void* in, void* out, int64_t rows, int64_t cols, int64_t pitch, hipStream_t s);
 hipError_t flip_filter_launch(int es, const void* f, void* bt, int64_t taps, int64_t ci, int64_t co, int64_t pitch, hipStream_t s);
 

@@ -1704,7 +1704,19 @@ int pml_hip_conv2d_grad_invoke(int64_t plan, const void* g, const void* other, v
       in = p->padded;
     }
     if (check(flip_filter_launch(es, other, p->sub->bt, d.kh * d.kw, d.ci, d.co, p->co_pad, st), "flip_filter_launch")) return 1;
-    return pml_hip_conv2d_invoke((int64_t)(intptr_t)p->sub, in, nullptr, result, nullptr, nullptr, nullptr, s);
+    if (pml_hip_conv2d_invoke((int64_t)(intptr_t)p->sub, in, nullptr, result, nullptr, nullptr, nullptr, s)) return 1;
+    ConvBorderArgs b;
+    b.g = g, b.f = other, b.out = result;
+    b.N = (int)d.n, b.H = (int)d.h, b.W = (int)d.w, b.CI = (int)d.ci, b.OH = (int)d.oh, b.OW = (int)d.ow, b.CO = (int)d.co;
+    b.KH = (int)d.kh, b.KW = (int)d.kw, b.PH = (int)d.pad_h, b.PW = (int)d.pad_w, b.DH = (int)d.dil_h, b.DW = (int)d.dil_w;
+    // an image row y meets the gradient's rows y + pad - ky * dil
+    auto inside = [](int64_t size, int64_t grad, int64_t k, int64_t dil, int64_t pad, int* from, int* to) {
+      *from = (int)std::min(size, std::max<int64_t>(0, dil * (k - 1) - pad));
+      *to = (int)std::max<int64_t>(*from, std::min(size, grad - pad));
+    };
+    inside(d.h, d.oh, d.kh, d.dil_h, d.pad_h, &b.y0, &b.y1);
+    inside(d.w, d.ow, d.kw, d.dil_w, d.pad_w, &b.x0, &b.x1);
+    return check(conv_border_launch(b, p->strided_bf, st), "conv_border_launch");
   }
   const int64_t g_step = d.oh * d.ow * d.co * es, r_step = d.h * d.w * d.ci * es;
   for (int64_t i = 0; i < d.n; i += p->grad_chunk) {

@@ -87,3 +87,47 @@ def test_conv_gradients(dtype, n, hw, ci, co, k, stride):
     check(gx, x.grad[:, :, before:before + hw, before:before + hw].permute(0, 2, 3, 1).numpy(), dtype)
     check(gf, f.grad.permute(2, 3, 1, 0).numpy(), dtype)
     assert 'general' not in plan_of(program)
+
+
+@pytest.mark.parametrize('dtype', ['f32', 'bf16'])
+@pytest.mark.parametrize('n,h,w,ci,co,k,stride', [
+    (2, 14, 14, 64, 64, 3, 1), (16, 56, 56, 64, 64, 3, 1), (1, 7, 9, 3, 16, 3, 2), (3, 9, 8, 19, 33, 5, 1), (2, 12, 15, 70, 20, 3, 2),
+    (1, 5, 6, 64, 96, 1, 1), (2, 3, 2, 8, 24, 5, 1)])
+def test_conv_gradients_leave_taps_outside_out(dtype, n, h, w, ci, co, k, stride):
+    """Taps that leave the image are no terms of either gradient: an infinity or a NaN in the gradient's border (filter
+    gradient) or in the filter (data gradient) is in the results that it reaches and in no other.  Sums of up to a tile, of
+    split K, of every convolution kernel the data gradient runs on, image rows of their own length."""
+    rng = np.random.default_rng(h * 3 + co)
+    oh, ow = (h + stride - 1) // stride, (w + stride - 1) // stride
+    py, px = (max(0, (o - 1) * stride + k - s) // 2 for o, s in ((oh, h), (ow, w)))
+    Iv, Fv, Gv = values(rng, (n, h, w, ci), dtype), values(rng, (k, k, ci, co), dtype, (k * k * co) ** -0.5), values(rng, (n, oh, ow, co), dtype)
+    # (one of a kind per channel: a sum holds one infinity, whose sign is known, or a NaN of its own)
+    Gv[0, 0, 0, 0], Gv[n - 1, oh - 1, ow // 2, 1], Gv[0, oh // 2, ow - 1, 2] = np.inf, np.nan, -np.inf
+    Gv[n - 1, 0, :, co - 1] = np.inf
+    Fv[0, 0, 0, 3], Fv[k - 1, 0, ci - 1, 4], Fv[k // 2, k - 1, 1, 5] = np.inf, np.nan, -np.inf
+    finite_f, finite_g = np.where(np.isfinite(Fv), Fv, 0.5).astype(np.float32), np.where(np.isfinite(Gv), Gv, 0.5).astype(np.float32)
+    X, F, G = (P.Placeholder(DT[dtype], x.shape) for x in (Iv, Fv, Gv))
+    dX = Pop.convolution(G, F, strides=[stride, stride], deriv_mode=Pop.DERIV_DATA, result_shape=[h, w])
+    dF = Pop.convolution(X, G, strides=[stride, stride], deriv_mode=Pop.DERIV_FILTER, result_shape=[k, k])
+    runner = P.Runner(P.Program('gradients', [X, F, G], [dX, dF]), target='hip')
+    gf = runner.run([Iv, finite_f, Gv])[1]
+    gx = runner.run([Iv, Fv, finite_g])[0]
+    want_x, want_f = np.zeros((n, h, w, ci)), np.zeros((k, k, ci, co))
+    with np.errstate(invalid='ignore'):
+        for ky in range(k):
+            for kx in range(k):
+                ys = [y for y in range(oh) if 0 <= y * stride + ky - py < h]
+                xs = [x for x in range(ow) if 0 <= x * stride + kx - px < w]
+                if not ys or not xs:
+                    continue
+                at = np.ix_(range(n), [y * stride + ky - py for y in ys], [x * stride + kx - px for x in xs])
+                of = np.ix_(range(n), ys, xs)
+                for c in range(ci):  # (term by term: a zero weight of a matrix product would itself make NaNs)
+                    want_x[at + (c,)] += (finite_g[of].astype(np.float64) * Fv[ky, kx, c]).sum(-1)
+                    want_f[ky, kx, c] = (Iv[at + (c,)].astype(np.float64)[..., None] * Gv[of]).sum((0, 1, 2))
+    assert not np.isfinite(want_f).all() and (k > w or not np.isfinite(want_x).all())  # (5 taps over 2 pixels: those three are never inside)
+    for got, want in ((gx, want_x), (gf, want_f)):
+        np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+        np.testing.assert_array_equal(np.isposinf(got), np.isposinf(want))
+        np.testing.assert_array_equal(np.isneginf(got), np.isneginf(want))
+        check(got[np.isfinite(want)], want[np.isfinite(want)], dtype)
