@@ -802,7 +802,9 @@ hipError_t product_direct_launch(const StridedArgs& a, bool bf, int rows, hipStr
 }
 
 // The tile and, for few tiles and a long K, the split: 128 x 128 where that still gives every CU a workgroup (half the
-// operand traffic per result), 64 x 64 otherwise; K is split when the tiles alone leave CUs idle, into runs of at least
+// operand traffic per result) and covers at most a third more results than 64 x 64, which otherwise is the tile (1000 of
+// 64 x 64 with K = 64, fp32: 43.7 us with tiles of 128, three quarters of them empty, 18.7 with tiles of 64; 1000 of 48 x 48,
+// K = 33, bf16: 44.1 and 18.4); K is split when the tiles alone leave CUs idle, into runs of at least
 // four slabs, for about three workgroups per CU (their LDS fits four times into one).
 void strided_plan(StridedArgs* a, bool bf, bool conv, int n_cus, int* mi) {
   int64_t batches = 1;
@@ -812,7 +814,7 @@ void strided_plan(StridedArgs* a, bool bf, bool conv, int n_cus, int* mi) {
     const int64_t rows = conv ? (a->M / a->row_cols) * ((a->row_cols + t - 1) / t) : (a->M + t - 1) / t;
     return rows * ((a->N + t - 1) / t) * batches;
   };
-  *mi = tiles(128) >= n_cus ? 2 : 1;
+  *mi = tiles(128) >= n_cus && 3 * tiles(128) <= tiles(64) ? 2 : 1;
   const int64_t t = 64 * *mi;
   a->tiles_per_tap = conv ? (int)((a->row_cols + t - 1) / t) : 1;
   a->tiles_m = conv ? (int)(a->M / a->row_cols) * a->tiles_per_tap : (int)((a->M + t - 1) / t);
