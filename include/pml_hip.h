@@ -625,6 +625,9 @@ typedef struct {
 
 int64_t pml_hip_product_dispatch(const pml_hip_product_desc* desc);
 int pml_hip_product_takes_tail(const pml_hip_epilogue* tail, int out_dtype); /* host arithmetic only */
+/* Whether this product is expected to be faster than the same sums through pml_hip_contract (many products of a few values
+ * each leave nearly all of a tile empty), and no larger than one launch can be.  Host arithmetic only, priced for a whole device. */
+int pml_hip_product_pays(const pml_hip_product_desc* desc);
 int pml_hip_product_invoke(int64_t plan, const void* a, const void* b, void* c, const void* init, const void* const* operands,
                            pml_hip_stream s);
 

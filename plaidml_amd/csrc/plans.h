@@ -13,6 +13,9 @@
 
 namespace pml {
 
+// HIP takes fewer than 2^32 threads in a dimension of a launch.
+constexpr int64_t kMaxLaunchThreads = ((int64_t)1 << 32) - 1;
+
 // The dynamic-LDS ceiling of a kernel (hipFuncAttributeMaxDynamicSharedMemorySize) belongs to the kernel on one
 // device.  One of these per kernel instantiation remembers, per device, the largest size already set.
 struct DynamicLdsLimit {
@@ -250,6 +253,8 @@ struct ContractArgs {
   void* out;
 };
 hipError_t contract_launch(const ContractArgs& a, hipStream_t s);
+// what contract_launch is expected to take for an fp32 or bf16 multiply-add of `k` terms for each of `results`, in microseconds
+double contract_product_us(double results, double k);
 
 struct EltwiseArgs {
   pml_hip_eltwise_desc d;
@@ -325,8 +330,10 @@ struct StridedArgs {
 };
 void strided_plan(StridedArgs* a, bool bf, bool conv, int n_cus, int* mi);
 hipError_t strided_launch(const StridedArgs& a, bool bf, bool conv, int mi, hipStream_t s);
-// Products with few result tiles: rows of the direct tile a shape takes (0: none), and its launch (`splits` and `ws` unused).
-int product_direct_rows(const StridedArgs& a, bool bf, int n_cus);
+// After strided_plan: rows of the direct tile a product takes (0: the LDS tiles of `mi`), and the microseconds it is expected
+// to take that way (an infinity where no kernel can be launched over so many tiles); the direct tiles' launch (`splits`
+// and `ws` unused).
+int product_direct_rows(const StridedArgs& a, bool bf, int mi, int n_cus, double* us);
 hipError_t product_direct_launch(const StridedArgs& a, bool bf, int rows, hipStream_t s);
 struct Col2imArgs {
   const float* cols;  // [N][OH][OW][KH][KW][CI]

@@ -1477,43 +1477,33 @@ static bool prepare_strided(Plan* p) {
   a.ws = (float*)p->ws;
   int64_t nb = (int64_t)a.tiles_m * a.tiles_n;
   for (int d = 0; d < a.n_batch; ++d) nb *= a.batch[d];
-  if (nb >= ((int64_t)1 << 31)) {
-    fail("product: too many result tiles");
+  if (nb > kMaxLaunchThreads / 256) {
+    fail("product: too many result tiles for one launch");
     return false;
   }
   return true;
 }
 
-int64_t pml_hip_product_dispatch(const pml_hip_product_desc* d) {
-  if (!d) {
-    fail("null descriptor");
-    return 0;
-  }
+// nullptr, or what is wrong with a product's types, sizes and strides; *batches: their number
+static const char* product_fault(const pml_hip_product_desc* d, int64_t* batches) {
+  if (!d) return "null descriptor";
   const bool bf = d->in_dtype == PML_HIP_BF16;
-  if ((d->in_dtype != PML_HIP_F32 && !bf) || (d->out_dtype != PML_HIP_F32 && (!bf || d->out_dtype != PML_HIP_BF16))) {
-    fail("product: in_dtype must be F32 or BF16 and out_dtype F32 or in_dtype");
-    return 0;
-  }
+  if ((d->in_dtype != PML_HIP_F32 && !bf) || (d->out_dtype != PML_HIP_F32 && (!bf || d->out_dtype != PML_HIP_BF16)))
+    return "product: in_dtype must be F32 or BF16 and out_dtype F32 or in_dtype";
   bool ok = d->m > 0 && d->n > 0 && d->k > 0 && d->n_batch >= 0 && d->n_batch <= 3 && d->a_ms >= 0 && d->a_ks >= 0 && d->b_ks >= 0 &&
             d->b_ns >= 0 && d->c_ms >= 0 && d->row_len > 0 && (d->init_kind == 0 || d->init_kind == 1);
-  int64_t batches = 1;
+  *batches = 1;
   for (int i = 0; ok && i < d->n_batch; ++i) {
     ok = d->batch[i] > 0 && d->a_batch[i] >= 0 && d->b_batch[i] >= 0 && d->c_batch[i] >= 0 && d->batch[i] < ((int64_t)1 << 31);
-    if (ok) batches *= d->batch[i];
-    ok = ok && batches < ((int64_t)1 << 31);
+    if (ok) *batches *= d->batch[i];
+    ok = ok && *batches < ((int64_t)1 << 31);
   }
-  if (!ok) {
-    fail("product: bad sizes or strides");
-    return 0;
-  }
-  if (!pml_hip_product_takes_tail(&d->tail, d->out_dtype)) {
-    fail("product: the tail holds steps this kernel does not run");
-    return 0;
-  }
-  Plan* p = new Plan();
-  p->kind = PLAN_PRODUCT;
-  p->strided_bf = bf;
-  StridedArgs& a = p->strided;
+  return ok ? nullptr : "product: bad sizes or strides";
+}
+
+// The kernel arguments that sizes and strides fix.
+static StridedArgs product_args(const pml_hip_product_desc* d) {
+  StridedArgs a;
   std::memset(&a, 0, sizeof a);
   a.M = d->m, a.N = d->n, a.K = d->k;
   a.a_ms = d->a_ms, a.a_ks = d->a_ks, a.b_ks = d->b_ks, a.b_ns = d->b_ns, a.c_ms = d->c_ms;
@@ -1526,6 +1516,38 @@ int64_t pml_hip_product_dispatch(const pml_hip_product_desc* d) {
     a.b_batch[i] = d->b_batch[i];
     a.c_batch[i] = d->c_batch[i];
   }
+  return a;
+}
+
+int pml_hip_product_pays(const pml_hip_product_desc* d) {
+  int64_t batches = 1;
+  if (product_fault(d, &batches)) return 0;
+  const bool bf = d->in_dtype == PML_HIP_BF16;
+  StridedArgs a = product_args(d);
+  int mi = 1;
+  double us = 0;
+  const int n_cus = 256;  // (of the whole device; asking for it would start the GPU runtime in a process that only plans)
+  strided_plan(&a, bf, false, n_cus, &mi);
+  (void)product_direct_rows(a, bf, mi, n_cus, &us);
+  return us <= contract_product_us((double)batches * (double)d->m * (double)d->n, (double)d->k) ? 1 : 0;
+}
+
+int64_t pml_hip_product_dispatch(const pml_hip_product_desc* d) {
+  int64_t batches = 1;
+  if (const char* fault = product_fault(d, &batches)) {
+    fail(fault);
+    return 0;
+  }
+  const bool bf = d->in_dtype == PML_HIP_BF16;
+  if (!pml_hip_product_takes_tail(&d->tail, d->out_dtype)) {
+    fail("product: the tail holds steps this kernel does not run");
+    return 0;
+  }
+  Plan* p = new Plan();
+  p->kind = PLAN_PRODUCT;
+  p->strided_bf = bf;
+  p->strided = product_args(d);
+  StridedArgs& a = p->strided;
   a.init_rs = d->init_row_stride;
   a.init_cs = d->init_col_stride;
   p->gemm.init_kind = d->init_kind;
@@ -1542,7 +1564,8 @@ int64_t pml_hip_product_dispatch(const pml_hip_product_desc* d) {
     }
   }
   strided_plan(&a, bf, false, device_cus(), &p->strided_mi);
-  p->product_rows = product_direct_rows(a, bf, device_cus());
+  double us = 0;
+  p->product_rows = product_direct_rows(a, bf, p->strided_mi, device_cus(), &us);
   if (!p->product_rows && !prepare_strided(p)) {
     delete p;
     return 0;
@@ -1660,6 +1683,7 @@ int64_t pml_hip_conv2d_grad_dispatch(const pml_hip_conv2d_desc* d, int which) {
   // stride^2 times as much.)  Columns are made for as many images at a time as fit 256 MiB.
   const int64_t taps_ci = d->kh * d->kw * d->ci, per_image = d->oh * d->ow * taps_ci * 4;
   p->grad_chunk = std::max<int64_t>(1, std::min<int64_t>(d->n, ((int64_t)256 << 20) / per_image));
+  p->grad_chunk = std::max<int64_t>(1, std::min(p->grad_chunk, kMaxLaunchThreads / (d->h * d->w * d->ci)));  // (a thread per value at most)
   a.M = p->grad_chunk * d->oh * d->ow;
   a.N = taps_ci;
   a.K = d->co;

@@ -22,6 +22,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <limits>
 
 #include "device_common.h"
 #include "plans.h"
@@ -752,42 +753,70 @@ hipError_t launch_direct(const StridedArgs& a, hipStream_t s) {
   b.tiles_n = (int)((a.N + 63) / 64);
   int64_t nb = (int64_t)b.tiles_m * b.tiles_n;
   for (int d = 0; d < a.n_batch; ++d) nb *= a.batch[d];
-  if (nb <= 0 || nb >= ((int64_t)1 << 31)) return hipErrorInvalidValue;
+  if (nb <= 0 || nb > kMaxLaunchThreads / 512) return hipErrorInvalidValue;
   hipLaunchKernelGGL(kern, dim3((unsigned)nb), dim3(512), lds, s, b);
   return hipGetLastError();
 }
 
 }  // namespace
 
-// Rows of the direct tile (16 or 32), 0: the tiles through LDS that strided_plan has laid out.  Both sides are priced in
-// microseconds from 25 shapes per type and layout (1 to 2000 rows, K of 32 to 2047, batches up to 96).  Direct: 2.6 plus, per
-// round of one tile on each CU, 0.8 (1.8 where bf16 has a broken last step of K) and the tile's operand bytes at 38 KB a
-// microsecond for fp32 with 16 rows, 32 with 32 rows (the matrix cores), bf16 25 from [K][N] and 17.5 from [N][K] (16-byte
-// loads at 2-byte alignment).  Through LDS: 3 and 1.65 a slab (bf16 [K][N] 3.6 and 1.55, [N][K] 4 and 1.1); split, 1.8 more
-// and the partial results written and read at 3 TB/s.  A direct tile has to be 8 % ahead.
+// Which of its two kernels a product takes -- the direct tile's rows (16 or 32), or 0: the tiles through LDS that strided_plan
+// has laid out -- and what it is expected to take in microseconds (an infinity: neither can be launched).  Both sides are
+// priced from 25 shapes per type and layout (1 to 2000 rows, K of 32 to 2047, batches up to 96) and from 45 with many small
+// tiles (batches of 100 to 100000, 1 to 128 rows and columns, K of 3 to 4096).  Direct: 2.6 plus, per round of one tile on
+// each CU, 0.8 (1.8 where bf16 has a broken last step of K; fp32 1.4 from the second round on) and the tile's operand bytes
+// at 38 KB a microsecond for fp32 with 16 rows, 32 with 32 rows (the matrix cores), bf16 25 from [K][N] and 17.5 from [N][K]
+// (16-byte loads at 2-byte alignment).  Through LDS: 3 and 1.65 a slab (bf16 [K][N] 3.6 and 1.55, [N][K] 4 and 1.1); every
+// further round -- workgroups share a CU by then -- 0.6 and 0.95 a slab (bf16 [K][N] 0.3 and 1.5, [N][K] 0.75 and 0.5, 0.55
+// more where the rows are read element by element); tiles of 128 in the first round 4 and 6 (bf16 10 and 6 or 2.5), in the others
+// 1.5 and 3.1 (bf16 1 and 6, 1.7 and 1.75); split, 1.8 more and the partial results written and read at 3 TB/s.  A direct
+// tile has to be 8 % ahead.
 //   us, through LDS -> direct              fp32 [K][N]       bf16 [K][N]       bf16 [N][K]
 //   3 x 1001, K = 333                    14.9 ->  5.0      13.2 ->  6.4      10.6 ->  7.7
 //   300 x 777, K = 1001                  20.5 -> 10.9      13.9 ->  9.9      12.6 (15.1)
 //   1000 x 1001, K = 1001                55.3 -> 32.1      28.0 -> 19.0      21.1 (25.3)
 //   20 of 100 x 77, K = 100              10.4 ->  4.6       8.5 ->  5.2       8.0 ->  4.9
 //   50 x 777, K = 1777: stays split      13.6 (22.1)       12.6 (17.8)       11.4 (23.4)
-int product_direct_rows(const StridedArgs& a, bool bf, int n_cus) {
+//   10000 of 1 x 16, K = 64              99.4 -> 66.2      71.2 -> 56.0      53.0 (52.2)
+//   10000 of 16 x 16, K = 16             63.5 (60.4)       73.6 (110)        56.4 (91.1)
+//   1000 of 1 x 1, K = 4096               463 -> 113                          135 -> 34
+int product_direct_rows(const StridedArgs& a, bool bf, int mi, int n_cus, double* us) {
   const bool nk = a.b_ks == 1;
-  if (a.a_ks != 1 || (!nk && (a.b_ns != 1 || a.N < 4))) return 0;
   double batches = 1;
   for (int d = 0; d < a.n_batch; ++d) batches *= (double)a.batch[d];
+  const double never = std::numeric_limits<double>::infinity();
+  const double lds_tiles = batches * (double)a.tiles_m * (double)a.tiles_n;
+  double lds_us = never;
+  if (lds_tiles * kThreads <= (double)kMaxLaunchThreads) {
+    const double slabs = (double)((std::min(a.K, a.k_per_split) + (bf ? 63 : 31)) / (bf ? 64 : 32));
+    const double more = std::max(0.0, lds_tiles / n_cus - 1);
+    const bool gathered = bf && a.a_ks != 1 && a.a_ms != 1;
+    double first, each;
+    if (mi == 2) {
+      first = !bf ? 4 + 6 * slabs : 10 + (nk ? 2.5 : 6) * slabs;
+      each = !bf ? 1.5 + 3.1 * slabs : nk ? 1.7 + 1.75 * slabs : 1 + 6 * slabs;
+    } else {
+      first = !bf ? 3 + 1.65 * slabs : nk ? 4 + 1.1 * slabs : 3.6 + 1.55 * slabs;
+      each = !bf ? 0.6 + 0.95 * slabs : nk ? 0.75 + 0.5 * slabs : 0.3 + 1.5 * slabs;
+      if (gathered) each += 0.55 * slabs * (double)std::min<int64_t>(a.M, 64) / 64;
+    }
+    lds_us = first + more * each;
+    if (a.splits > 1) lds_us += 1.8 + 8.0 * a.splits * (double)a.ws_rows * (double)a.ws_pitch / 3e6;
+  }
   const double kb = (double)a.K * (bf ? 2 : 4);
   auto direct_us = [&](int64_t rows) {
     const double tiles = batches * (double)((a.M + rows - 1) / rows) * (double)((a.N + 63) / 64);
+    if (tiles * 512 > (double)kMaxLaunchThreads) return never;
     const double rate = bf ? (nk ? 17.5e3 : 25e3) : (rows == 16 ? 38e3 : 32e3);
     const double live = (double)(rows == 16 ? std::min<int64_t>(a.M, 16) : 32) + 64;
-    return 2.6 + std::ceil(tiles / n_cus) * ((bf && a.K % 32 != 0 ? 1.8 : 0.8) + live * kb / rate);
+    const double rounds = std::ceil(tiles / n_cus);
+    return 2.6 + rounds * ((bf && a.K % 32 != 0 ? 1.8 : 0.8) + live * kb / rate) + (!bf && a.K % 16 != 0 ? 0.6 * (rounds - 1) : 0);
   };
-  const double slabs = (double)((std::min(a.K, a.k_per_split) + (bf ? 63 : 31)) / (bf ? 64 : 32));
-  double lds_us = !bf ? 3 + 1.65 * slabs : nk ? 4 + 1.1 * slabs : 3.6 + 1.55 * slabs;
-  if (a.splits > 1) lds_us += 1.8 + 8.0 * a.splits * (double)a.ws_rows * (double)a.ws_pitch / 3e6;
-  const double small = direct_us(16), large = direct_us(32);
-  if (std::min(small, large) > 0.92 * lds_us) return 0;
+  *us = lds_us;
+  if (a.a_ks != 1 || (!nk && (a.b_ns != 1 || a.N < 4))) return 0;
+  const double small = direct_us(16), large = direct_us(32), direct = std::min(small, large);
+  if (direct > 0.92 * lds_us || direct == never) return 0;
+  *us = direct;
   return small <= large ? 16 : 32;
 }
 
@@ -839,7 +868,7 @@ void strided_plan(StridedArgs* a, bool bf, bool conv, int n_cus, int* mi) {
 hipError_t strided_launch(const StridedArgs& a, bool bf, bool conv, int mi, hipStream_t s) {
   int64_t nb = (int64_t)a.tiles_m * a.tiles_n;
   for (int d = 0; d < a.n_batch; ++d) nb *= a.batch[d];
-  if (nb <= 0 || nb >= ((int64_t)1 << 31) || a.splits < 1 || a.splits > 65535 || (a.splits > 1) != (a.ws != nullptr)) return hipErrorInvalidValue;
+  if (nb <= 0 || nb > kMaxLaunchThreads / kThreads || a.splits < 1 || a.splits > 65535 || (a.splits > 1) != (a.ws != nullptr)) return hipErrorInvalidValue;
   const int amode = conv ? ROWS_CONV : (a.a_ks == 1 ? ROWS_K : ROWS_M), bmode = a.b_ks == 1 && !conv ? ROWS_K : ROWS_M;
   hipError_t e;
   if (bf)
@@ -848,7 +877,7 @@ hipError_t strided_launch(const StridedArgs& a, bool bf, bool conv, int mi, hipS
     e = mi == 2 ? launch_modes<false, 2>(a, amode, bmode, s) : launch_modes<false, 1>(a, amode, bmode, s);
   if (e != hipSuccess || a.splits == 1) return e;
   const int64_t groups = a.ws_rows * (a.ws_pitch / 4), blocks = (groups + 255) / 256;
-  if (blocks >= ((int64_t)1 << 31)) return hipErrorInvalidValue;
+  if (blocks > kMaxLaunchThreads / 256) return hipErrorInvalidValue;
   hipLaunchKernelGGL(strided_reduce_kernel, dim3((unsigned)blocks), dim3(256), 0, s, a);
   return hipGetLastError();
 }
@@ -986,7 +1015,7 @@ hipError_t conv_border_launch(const ConvBorderArgs& a, bool bf, hipStream_t s) {
 hipError_t col2im_launch(const Col2imArgs& a, bool bf, hipStream_t s) {
   const int v = a.CI % 4 == 0 ? 4 : 1;
   const int64_t blocks = ((int64_t)a.N * a.H * a.W * a.CI / v + 255) / 256;
-  if (blocks <= 0 || blocks >= ((int64_t)1 << 31)) return hipErrorInvalidValue;
+  if (blocks <= 0 || blocks > kMaxLaunchThreads / 256) return hipErrorInvalidValue;
   const dim3 grid((unsigned)blocks), block(256);
   if (bf) {
     if (v == 4) hipLaunchKernelGGL((col2im_kernel<true, 4>), grid, block, 0, s, a);
@@ -1010,7 +1039,7 @@ hipError_t pad_rows_launch(int es, const void* in, void* out, int64_t rows, int6
 
 hipError_t flip_filter_launch(int es, const void* f, void* bt, int64_t taps, int64_t ci, int64_t co, int64_t pitch, hipStream_t s) {
   const int64_t blocks = (taps * ci * co + 255) / 256;
-  if (blocks <= 0 || blocks >= ((int64_t)1 << 31)) return hipErrorInvalidValue;
+  if (blocks <= 0 || blocks > kMaxLaunchThreads / 256) return hipErrorInvalidValue;
   if (es == 2)
     hipLaunchKernelGGL(flip_filter_kernel<uint16_t>, dim3((unsigned)blocks), dim3(256), 0, s, (const uint16_t*)f, (uint16_t*)bt, (int)taps, (int)ci, (int)co, (int)pitch);
   else

@@ -267,8 +267,8 @@ void Planner::emitContraction(size_t i) {
     if (tryGemm(i)) return;
     if (tryConv(i)) return;
     if (tryConvGrad(i)) return;
+    if (tryDepthwise(i)) return;  // (before tryProduct: a window of one row without padding has a product's index set, too)
     if (tryProduct(i)) return;
-    if (tryDepthwise(i)) return;
     if (tryPool(i)) return;
     if (tryGlobalPool(i)) return;
     if (opt_.fuse && trySoftmax(i)) return;

@@ -529,6 +529,7 @@ bool Planner::tryProduct(size_t i) {
   d.a_ks = K[0].s[L];
   d.b_ns = nn.s[2];
   d.b_ks = K[0].s[R];
+  d.row_len = nn.range;
   d.c_ms = M.empty() && !swapped ? nn.range : m.s[0];
   if (m.range == 1) d.c_ms = nn.range;
   d.n_batch = static_cast<int32_t>(B.size());
@@ -538,10 +539,10 @@ bool Planner::tryProduct(size_t i) {
     d.b_batch[k] = B[k].s[R];
     d.c_batch[k] = B[k].s[0];
   }
+  if (!pml_hip_product_pays(&d)) return false;
   // rows and columns as the tail sees them: the result's last dimension is the columns
   bool rows_ok = op.result->shape.getRank() >= 1 && op.result->shape.sizes.back() == nn.range && (m.range == 1 || d.c_ms % nn.range == 0);
   for (const Group& g : B) rows_ok = rows_ok && g.s[0] % nn.range == 0;
-  d.row_len = nn.range;
   if (op.init) {
     int32_t idt = 0;
     if (!rows_ok || op.init->kind == Value::Literal || op.init->shape.elementType != dt) return false;

@@ -73,6 +73,46 @@ def test_products_whose_results_meet_take_the_general_kernel(name):
         assert 'contract (general)' in t and 'product' not in t, t
 
 
+def _products(b, m, n, k, batch_inside=False):
+    A, B = E.Placeholder(D.FLOAT32, [m, k, b] if batch_inside else [b, m, k]), E.Placeholder(D.FLOAT32, [k, n, b] if batch_inside else [b, k, n])
+    x, i, j, q = E.TensorIndexes(4)
+    C = E.Contraction().outShape(b, m, n).outAccess(x, i, j)
+    return E.Program('products', [A, B], [C.sum(A[i, q, x] * B[q, j, x] if batch_inside else A[x, i, q] * B[x, q, j]).build()])
+
+
+@pytest.mark.parametrize('b,m,n,k,inside,product', [
+    (100000, 1, 1, 64, False, False), (100000, 4, 4, 4, False, False), (10000, 3, 3, 3, True, False), (20000000, 1, 1, 16, False, False),
+    (1, 1, 1, 2, False, True), (1000, 1, 1, 64, False, True), (96, 128, 128, 100, False, True), (10000, 16, 16, 16, True, True), (1000, 1, 256, 64, False, True)])
+def test_many_small_products_are_planned_by_price(b, m, n, k, inside, product):
+    """Products of a few values each leave nearly all of a tile empty: the plan takes the product kernels where they are
+    expected to be the faster ones."""
+    t = plan_of(_products(b, m, n, k, inside))
+    assert ('product f32' in t) == product and ('contract (general)' in t) != product, t
+
+
+def test_a_window_of_one_row_stays_with_the_depthwise_kernel():
+    """O[n, y, x, c] += I[n, y + i, x + j, c] * F[i, j, c, 0] over one row and without padding has a product's index set, too."""
+    I, F = E.Placeholder(D.FLOAT32, [1, 1, 300, 64]), E.Placeholder(D.FLOAT32, [1, 3, 64, 1])
+    n, y, x, c, i, j = E.TensorIndexes(6)
+    O = E.Contraction().outShape(1, 1, 298, 64).outAccess(n, y, x, c).sum(I[n, y + i, x + j, c] * F[i, j, c, 0]).build()
+    t = plan_of(E.Program('dw', [I, F], [O]))
+    assert 'dwconv2d f32' in t, t
+
+
+@pytest.mark.parametrize('batch,pays', [(8, 1), (1 << 20, 1), ((1 << 24) - 1, 1), (1 << 24, 0), (1 << 30, 0)])
+def test_products_of_more_tiles_than_a_launch_holds_do_not_pay(batch, pays):
+    """2^24 tiles are 2^32 threads, one more than a launch can have."""
+    import ctypes
+
+    from plaidml_amd import hipkernels as hk
+    d = hk.ProductDesc()
+    d.in_dtype = d.out_dtype = hk.F32
+    d.m = d.n = d.k = d.row_len = d.c_ms = d.b_ks = 64
+    d.a_ms, d.a_ks, d.b_ns, d.n_batch = 64, 1, 1, 1
+    d.batch[0], d.a_batch[0], d.b_batch[0], d.c_batch[0] = batch, 4096, 4096, 4096
+    assert hk.lib().pml_hip_product_pays(ctypes.byref(d)) == pays
+
+
 def test_output_coordinates_that_are_sums_are_solved_for_one_index():
     """O[n, 2x + i - 1, 2y + j - 1, co]: the planner solves each such coordinate for its widest index (x, y), so the
     kernel's threads walk the taps and input channels only -- 7 indices (4 output coordinates + i, j, ci), not 11;

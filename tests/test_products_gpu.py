@@ -28,7 +28,8 @@ def plan_of(program):
 @pytest.mark.parametrize('dtype', ['f32', 'bf16'])
 @pytest.mark.parametrize('b,m,n,k,ta,tb', [
     (1, 1, 1, 2, 0, 0), (1, 300, 777, 1001, 0, 0), (3, 64, 64, 64, 0, 1), (5, 65, 31, 33, 0, 0), (2, 127, 129, 100, 1, 0),
-    (7, 19, 276, 32, 0, 1), (1, 130, 70, 5003, 1, 0), (2, 3, 5, 7, 1, 1), (1, 1100, 2051, 67, 0, 0), (4, 1, 33, 130, 0, 1)])
+    (7, 19, 276, 32, 0, 1), (1, 130, 70, 5003, 1, 0), (2, 3, 5, 7, 1, 1), (1, 1100, 2051, 67, 0, 0), (4, 1, 33, 130, 0, 1),
+    (300, 100, 100, 40, 1, 0), (300, 128, 65, 70, 0, 1), (300, 64, 70, 33, 1, 1)])  # (many tiles: of 128, and of 64 where those would be empty)
 def test_product(dtype, b, m, n, k, ta, tb):
     rng = np.random.default_rng(m * 7 + n)
     A, B = values(rng, (b, k, m) if ta else (b, m, k), dtype), values(rng, (b, n, k) if tb else (b, k, n), dtype, k ** -0.5)
