@@ -366,11 +366,12 @@ struct SortKey {  // DT: the element type where it is one of the common ones, 0:
 
 size_t rows_program_lds(const pml_hip_rows_desc& d, int* lanes) {
   // A wavefront per row needs no barrier between steps, which is what a row costs most of (4096 x 1000: 35 us with a
-  // workgroup per row): for short rows, and for rows of up to 2048 when there are enough of them to fill the chip that way.
+  // workgroup per row): for short rows, and for rows of up to 2048 when there are enough of them to fill the chip that way
+  // and four of them fit the LDS (from five vectors of 2048 columns on they do not).
   const size_t pitch = (size_t)(d.cols + 3) / 4 * 4;
-  *lanes = d.cols <= 512 || (d.cols <= 2048 && d.rows >= 1024) ? 64 : 256;
-  const size_t groups = 256 / *lanes;
-  return (groups * PML_HIP_ROWS_SCALARS + 4 + groups * (size_t)d.n_vectors * pitch) * 4;
+  auto bytes = [&](size_t groups) { return (groups * PML_HIP_ROWS_SCALARS + 4 + groups * (size_t)d.n_vectors * pitch) * 4; };
+  *lanes = d.cols <= 512 || (d.cols <= 2048 && d.rows >= 1024 && bytes(4) <= kRowsLds) ? 64 : 256;
+  return bytes(256 / *lanes);
 }
 
 namespace {

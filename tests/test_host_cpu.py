@@ -113,6 +113,19 @@ def test_products_of_more_tiles_than_a_launch_holds_do_not_pay(batch, pays):
     assert hk.lib().pml_hip_product_pays(ctypes.byref(d)) == pays
 
 
+@pytest.mark.parametrize('rows', [1023, 1024])
+@pytest.mark.parametrize('cols', [2016, 2020, 2048])
+def test_rows_that_fit_a_workgroup_one_by_one_are_taken(rows, cols):
+    """Five vectors of 2020 columns fit the LDS once and not four times: many such rows are taken as well as few."""
+    X = E.Placeholder(D.FLOAT32, [rows, cols])
+    t = X - op.max(X, 1, True)
+    a, b = E.exp(t), E.tanh(t)
+    c, d = a * b, b * b
+    s = [op.sum(v, 1, True) for v in (a, b, c, d)]
+    text = plan_of(E.Program('rows', [X], [a / s[0] + b / s[1] + c / s[2] + d / s[3] + t]))
+    assert 'row program' in text and '1 launches' in text, text
+
+
 def test_output_coordinates_that_are_sums_are_solved_for_one_index():
     """O[n, 2x + i - 1, 2y + j - 1, co]: the planner solves each such coordinate for its widest index (x, y), so the
     kernel's threads walk the taps and input channels only -- 7 indices (4 output coordinates + i, j, ci), not 11;

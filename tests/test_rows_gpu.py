@@ -61,6 +61,24 @@ def test_row_program_with_several_results():
     np.testing.assert_array_equal(m, -x.max(1, keepdims=True))
 
 
+@pytest.mark.parametrize('rows,cols', [(1024, 1500), (1024, 2016), (1025, 2020), (1030, 2048)])
+def test_row_program_with_many_live_vectors(rows, cols):
+    """Five values per column are live at once: four rows of up to 2016 columns share a workgroup's LDS, longer ones have it alone."""
+    x = values(np.random.default_rng(cols), (rows, cols), 'f32')
+
+    def make(X):
+        t = X - Pop.max(X, 1, True)
+        a, b = P.exp(t), P.tanh(t)
+        c, d = a * b, b * b
+        sums = [Pop.sum(v, 1, True) for v in (a, b, c, d)]
+        return [a / sums[0] + b / sums[1] + c / sums[2] + d / sums[3] + t]
+    got, = run(make, [x], 'f32', 'row program')
+    t = x.astype(np.float64) - x.max(1, keepdims=True)
+    a, b = np.exp(t), np.tanh(t)
+    want = sum(v / v.sum(1, keepdims=True) for v in (a, b, a * b, b * b)) + t
+    assert np.linalg.norm(got - want) < 2e-6 * np.linalg.norm(want)
+
+
 @pytest.mark.parametrize('dtype', ['f32', 'bf16'])
 @pytest.mark.parametrize('shape', SHAPES)
 def test_argmax_rows(dtype, shape):
