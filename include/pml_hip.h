@@ -506,7 +506,7 @@ typedef struct {
   int64_t rows, cols;
   pml_hip_rows_step steps[PML_HIP_ROWS_STEPS];
 } pml_hip_rows_desc;
-int pml_hip_rows_takes(const pml_hip_rows_desc* desc); /* host arithmetic only: well-formed, and the rows fit a CU's LDS */
+int pml_hip_rows_takes(const pml_hip_rows_desc* desc); /* host arithmetic only: well-formed, a row fits a CU's LDS and all of them one launch */
 int pml_hip_rows(const pml_hip_rows_desc* desc, const void* const* in, void* const* out, pml_hip_stream s);
 /* out[row] = the last position of the row's largest element (plaidml/op/lib/ops.cc:505-521: max over positions whose value
  * equals the maximum; no NaN is ever the maximum).  F32 or BF16 rows, dense; int32 results. */

@@ -760,7 +760,7 @@ hipError_t contract_launch(const ContractArgs& a, hipStream_t s) {
     ra.lanes = (ra.cols >= 2048 && d.out_elems * 64 < (int64_t)256 * 1024) ? 256 : 64;
     const int per_block = 256 / ra.lanes;
     const int64_t nb = (d.out_elems + per_block - 1) / per_block;
-    if (nb <= 0x7fffffff) {
+    if (nb <= kMaxLaunchThreads / 256) {
       const dim3 grid((unsigned)nb), block(256);
       const bool same = d.src_dtype[0] == d.dtype;
 #define PML_ROWS(DT, AGG)                                                                                   \
@@ -1092,7 +1092,7 @@ bool softmax_in_regs(const pml_hip_softmax_desc& d, const void* x, void* y, hipS
 
 hipError_t softmax_launch(const pml_hip_softmax_desc& d, const void* x, void* y, hipStream_t s) {
   if (d.rows == 0 || d.cols == 0) return hipSuccess;
-  if (d.rows > 0x7fffffff) return hipErrorInvalidValue;
+  if (d.rows > kMaxLaunchThreads / 256) return hipErrorInvalidValue;
   if (d.dtype == PML_HIP_BF16 ? softmax_in_regs<true>(d, x, y, s) : softmax_in_regs<false>(d, x, y, s)) return hipGetLastError();
   if (d.dtype == PML_HIP_BF16)
     hipLaunchKernelGGL(softmax_rows_kernel<true>, dim3((unsigned)d.rows), dim3(256), 0, s, x, y, d.cols);

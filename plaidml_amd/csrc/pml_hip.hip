@@ -421,6 +421,16 @@ float host_round_bf16(float f) {
   return f;
 }
 
+// Row kernels have up to 256 threads for a row: a launch takes 2^23 of them, the next one the rows that follow.
+template <typename F>
+int in_row_runs(int64_t rows, F&& launch) {
+  constexpr int64_t kRun = (int64_t)1 << 23;
+  static_assert(kRun * 256 <= kMaxLaunchThreads, "a run of rows is one launch");
+  for (int64_t first = 0; first < rows; first += kRun)
+    if (int rc = launch(first, std::min(kRun, rows - first))) return rc;
+  return 0;
+}
+
 // Compute units of the current device (persistent kernels size their grids by it).
 int device_cus() {
   static int cached[64] = {0};
@@ -1412,7 +1422,8 @@ int pml_hip_rows_takes(const pml_hip_rows_desc* d) {
     if (!ok) return 0;
   }
   int lanes = 0;
-  return rows_program_lds(*d, &lanes) <= 158 * 1024 ? 1 : 0;
+  if (rows_program_lds(*d, &lanes) > 158 * 1024) return 0;
+  return (d->rows + 256 / lanes - 1) / (256 / lanes) <= kMaxLaunchThreads / 256 ? 1 : 0;
 }
 
 int pml_hip_rows(const pml_hip_rows_desc* d, const void* const* in, void* const* out, pml_hip_stream s) {
@@ -1434,14 +1445,20 @@ int pml_hip_rows(const pml_hip_rows_desc* d, const void* const* in, void* const*
 int pml_hip_argmax_rows(int dtype, int64_t rows, int64_t cols, const void* x, int32_t* out, pml_hip_stream s) {
   if ((dtype != PML_HIP_F32 && dtype != PML_HIP_BF16) || rows < 0 || cols <= 0 || cols > 0x7fffffff) return fail("argmax_rows: bad type or sizes");
   if (rows && (!x || !out)) return fail("argmax_rows: null operand");
-  return check(argmax_rows_launch(dtype, rows, cols, x, out, (hipStream_t)s), "argmax_rows_launch");
+  return in_row_runs(rows, [&](int64_t first, int64_t n) {
+    return check(argmax_rows_launch(dtype, n, cols, (const char*)x + first * cols * dt_size(dtype), out + first, (hipStream_t)s), "argmax_rows_launch");
+  });
 }
 
 int pml_hip_topk_rows(int dtype, int descending, int64_t rows, int64_t cols, int k, const void* x, void* values, int32_t* positions,
                       pml_hip_stream s) {
   if (dt_size(dtype) == 0 || dt_size(dtype) == 8 || rows < 0 || k < 0 || k > cols || cols > PML_HIP_MAX_SORT_LINE) return fail("topk_rows: bad type or sizes");
   if (rows && k && (!x || (!values && !positions))) return fail("topk_rows: null operand");
-  return check(topk_rows_launch(dtype, descending != 0, rows, cols, k, x, values, positions, (hipStream_t)s), "topk_rows_launch");
+  return in_row_runs(rows, [&](int64_t first, int64_t n) {
+    return check(topk_rows_launch(dtype, descending != 0, n, cols, k, (const char*)x + first * cols * dt_size(dtype),
+                                  values ? (char*)values + first * k * dt_size(dtype) : nullptr, positions ? positions + first * k : nullptr, (hipStream_t)s),
+                 "topk_rows_launch");
+  });
 }
 
 // ---------------------------------------------------------------------------
@@ -1982,7 +1999,12 @@ int pml_hip_softmax(const pml_hip_softmax_desc* d, const void* x, void* y, pml_h
   if (!d || !x || !y) return fail("softmax: null argument");
   if (d->dtype != PML_HIP_F32 && d->dtype != PML_HIP_BF16) return fail("softmax: dtype must be F32 or BF16");
   if (d->rows < 0 || d->cols < 0 || d->rows > 0x7fffffff) return fail("softmax: rows or cols out of range");
-  return check(softmax_launch(*d, x, y, (hipStream_t)s), "softmax_launch");
+  return in_row_runs(d->rows, [&](int64_t first, int64_t rows) {
+    pml_hip_softmax_desc run = *d;
+    run.rows = rows;
+    const int64_t at = first * d->cols * dt_size(d->dtype);
+    return check(softmax_launch(run, (const char*)x + at, (char*)y + at, (hipStream_t)s), "softmax_launch");
+  });
 }
 
 int pml_hip_index(void* out, int32_t rank, const int64_t* sizes, int32_t axis, pml_hip_stream s) {

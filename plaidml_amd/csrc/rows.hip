@@ -400,7 +400,7 @@ hipError_t rows_program_launch(const RowsProgramArgs& a, hipStream_t s) {
   int lanes = 0;
   const size_t lds = rows_program_lds(a.d, &lanes);
   const int64_t blocks = (a.d.rows + 256 / lanes - 1) / (256 / lanes);
-  if (blocks > 0x7fffffff || lds > kRowsLds) return hipErrorInvalidValue;
+  if (blocks > kMaxLaunchThreads / 256 || lds > kRowsLds) return hipErrorInvalidValue;
   if (a.d.dtype == PML_HIP_BF16) return lanes == 64 ? launch_program<true, 64>(a, lds, blocks, s) : launch_program<true, 256>(a, lds, blocks, s);
   return lanes == 64 ? launch_program<false, 64>(a, lds, blocks, s) : launch_program<false, 256>(a, lds, blocks, s);
 }
@@ -410,7 +410,7 @@ hipError_t argmax_rows_launch(int dtype, int64_t rows, int64_t cols, const void*
   // a wavefront per row; the whole workgroup for long rows too few to fill the chip
   const bool wide = cols >= 2048 && rows * 64 < (int64_t)256 * 1024;
   const int64_t blocks = wide ? rows : (rows + 3) / 4;
-  if (blocks > 0x7fffffff || cols > 0x7fffffff) return hipErrorInvalidValue;
+  if (blocks > kMaxLaunchThreads / 256 || cols > 0x7fffffff) return hipErrorInvalidValue;
   const dim3 grid((unsigned)blocks), block(256);
   const bool bf = dtype == PML_HIP_BF16;
   if (bf && wide) hipLaunchKernelGGL((argmax_rows_kernel<true, 256>), grid, block, 0, s, x, out, rows, (int)cols);
@@ -427,7 +427,7 @@ hipError_t topk_rows_launch(int dtype, int descending, int64_t rows, int64_t col
   const int waves = in_regs ? 4 : 1;  // longer rows: up to 64 KB of keys in LDS, one row per workgroup
   const size_t lds = in_regs ? 0 : (size_t)cols * 4;
   const int64_t blocks = (rows + waves - 1) / waves;
-  if (blocks > 0x7fffffff || lds > kRowsLds) return hipErrorInvalidValue;
+  if (blocks > kMaxLaunchThreads / 256 || lds > kRowsLds) return hipErrorInvalidValue;
   const dim3 grid((unsigned)blocks), block(64 * waves);
 #define PML_GO(DT, E)                                                                                                          \
   {                                                                                                                            \

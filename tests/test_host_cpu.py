@@ -126,6 +126,18 @@ def test_rows_that_fit_a_workgroup_one_by_one_are_taken(rows, cols):
     assert 'row program' in text and '1 launches' in text, text
 
 
+@pytest.mark.parametrize('rows,cols,takes', [((1 << 26) - 4, 16, 1), (1 << 26, 16, 0), ((1 << 24) - 1, 3000, 1), (1 << 24, 3000, 0)])
+def test_row_programs_of_more_rows_than_a_launch_holds_are_refused(rows, cols, takes):
+    """Four short rows or one long one to a workgroup of 256 threads, and fewer than 2^32 threads to a launch."""
+    import ctypes
+    import struct
+
+    from plaidml_amd import hipkernels as hk
+    # pml_hip_rows_desc: dtype, n_steps, n_vectors, n_in, n_out, reserved, rows, cols, 24 steps of 32 bytes
+    d = struct.pack('6i2q', hk.F32, 0, 2, 0, 0, 0, rows, cols) + bytes(24 * 32)
+    assert hk.lib().pml_hip_rows_takes(ctypes.create_string_buffer(d, len(d))) == takes
+
+
 def test_output_coordinates_that_are_sums_are_solved_for_one_index():
     """O[n, 2x + i - 1, 2y + j - 1, co]: the planner solves each such coordinate for its widest index (x, y), so the
     kernel's threads walk the taps and input channels only -- 7 indices (4 output coordinates + i, j, ci), not 11;

@@ -116,3 +116,22 @@ def test_softmax_rows(dtype, shape):
     e = np.exp(x.astype(np.float64) - x.max(-1, keepdims=True))
     want = e / e.sum(-1, keepdims=True)
     assert np.linalg.norm(got - want) < (1e-2 if dtype == 'bf16' else 2e-6) * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize('which', ['argmax', 'topk', 'softmax'])
+def test_more_rows_than_one_launch_takes(which):
+    """2^23 rows and some: they go in two launches, the second with the rows that are left."""
+    rows, cols = (1 << 23) + 5, 3
+    x = np.random.default_rng(9).random((rows, cols), dtype=np.float32)
+    X = P.Placeholder(DT['f32'], x.shape)
+    outs = {'argmax': lambda: [Pop.argmax(X, 1)], 'topk': lambda: list(Pop.topk(X, 2)), 'softmax': lambda: [Pop.softmax(X, 1)]}[which]()
+    got = P.Runner(P.Program(which, [X], outs), target='hip').run([x])
+    if which == 'argmax':
+        np.testing.assert_array_equal(got[0], np.argmax(x, 1))  # (no ties among these)
+    elif which == 'topk':
+        order = np.argsort(-x, 1, kind='stable')[:, :2]
+        np.testing.assert_array_equal(got[1], order)
+        np.testing.assert_array_equal(got[0], np.take_along_axis(x, order, 1))
+    else:
+        e = np.exp(x - x.max(1, keepdims=True))
+        np.testing.assert_allclose(got[0], e / e.sum(1, keepdims=True), rtol=2e-6)
