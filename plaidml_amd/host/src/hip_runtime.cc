@@ -11,6 +11,7 @@
 #include <sstream>
 
 #include "host_copy.h"
+#include "pinned_pool.h"
 #include "pml_hip.h"
 
 namespace pmlc::rt {
@@ -635,28 +636,20 @@ void registerRuntime(const std::string& id, std::shared_ptr<Runtime> runtime) {
 
 // Page-locked host memory for buffers the library allocates itself.  Asking for it initialises the GPU runtime as a
 // side effect, so a process that must not touch the GPU (one that only builds programs, or that will exec another
-// program) sets PLAIDML_PINNED=0; the total is capped (PLAIDML_PINNED_MAX_MB, default 4096) because page-locked
-// memory is taken from what the host can page.  Beyond the cap, and on any failure, the caller falls back to
-// ordinary memory (nullptr here).
-//
-// Blocks come in sizes of 1/8 steps between powers of two and, when freed, are kept for the next allocation of their
-// size as long as all kept ones together stay under kPinnedKeep; the one kept longest goes back to the system first.
+// program) sets PLAIDML_PINNED=0; the total of all blocks, those kept for the next allocation among them, is capped
+// (PLAIDML_PINNED_MAX_MB, default 4096) because page-locked memory is taken from what the host can page.  Beyond the
+// cap, and on any failure, the caller falls back to ordinary memory (nullptr here).
 namespace {
-constexpr size_t kPinnedKeep = size_t{256} << 20;
-struct PinnedPool {
-  std::mutex mutex;
-  std::map<const char*, size_t> live;                   // block -> its size
-  std::vector<std::pair<char*, size_t>> kept;           // free blocks, the one freed first in front
-  size_t live_total = 0, kept_total = 0;
-};
 PinnedPool& pinnedPool() {  // (never destroyed: buffers may be freed while the process ends)
-  static PinnedPool* pool = new PinnedPool();
+  static PinnedPool* pool = new PinnedPool(
+      [](size_t bytes) -> void* {
+        initRuntimes();
+        if (listDevices().empty()) return nullptr;
+        void* p = nullptr;
+        return pml_hip_host_alloc(&p, bytes) == 0 ? p : nullptr;
+      },
+      [](void* p) { (void)pml_hip_host_free(p); }, size_t{256} << 20);
   return *pool;
-}
-size_t pinnedSize(size_t bytes) {
-  size_t step = 4096;
-  while (step * 16 <= bytes) step *= 2;
-  return (std::max<size_t>(bytes, 1) + step - 1) / step * step;
 }
 }  // namespace
 
@@ -671,70 +664,14 @@ void* pinnedAllocRaw(size_t bytes) {
   if (enabled == "0" || enabled == "false" || enabled == "off") return nullptr;
   const std::string cap_text = util::Settings::Instance()->get("PLAIDML_PINNED_MAX_MB");
   const size_t cap = (cap_text.empty() ? size_t{4096} : static_cast<size_t>(std::strtoull(cap_text.c_str(), nullptr, 10))) << 20;
-  PinnedPool& pool = pinnedPool();
-  if (bytes > cap) return nullptr;
-  const size_t size = pinnedSize(bytes);
-  char* p = nullptr;
-  {
-    std::lock_guard<std::mutex> lock(pool.mutex);
-    if (pool.live_total > cap - bytes) return nullptr;
-    for (size_t i = pool.kept.size(); i-- > 0;) {
-      if (pool.kept[i].second != size) continue;
-      p = pool.kept[i].first;
-      pool.kept.erase(pool.kept.begin() + static_cast<long>(i));
-      pool.kept_total -= size;
-      pool.live[p] = size;
-      pool.live_total += size;
-      break;
-    }
-  }
-  if (!p) {
-    initRuntimes();
-    if (listDevices().empty()) return nullptr;
-    void* fresh = nullptr;
-    if (pml_hip_host_alloc(&fresh, size) != 0 || !fresh) return nullptr;
-    p = static_cast<char*>(fresh);
-    std::lock_guard<std::mutex> lock(pool.mutex);
-    pool.live[p] = size;
-    pool.live_total += size;
-  }
-  return p;
+  return pinnedPool().take(bytes, cap);
 }
 
 void pinnedFree(void* p) {
-  if (!p) return;
-  PinnedPool& pool = pinnedPool();
-  std::vector<char*> back;
-  {
-    std::lock_guard<std::mutex> lock(pool.mutex);
-    const auto it = pool.live.find(static_cast<const char*>(p));
-    if (it == pool.live.end()) return;
-    const size_t size = it->second;
-    pool.live.erase(it);
-    pool.live_total -= size;
-    if (size > kPinnedKeep) {
-      back.push_back(static_cast<char*>(p));
-    } else {
-      pool.kept.emplace_back(static_cast<char*>(p), size);
-      pool.kept_total += size;
-      while (pool.kept_total > kPinnedKeep) {
-        back.push_back(pool.kept.front().first);
-        pool.kept_total -= pool.kept.front().second;
-        pool.kept.erase(pool.kept.begin());
-      }
-    }
-  }
-  for (char* b : back) pml_hip_host_free(b);
+  if (p) pinnedPool().put(p);
 }
 
-bool isPinned(const void* p, size_t bytes) {
-  PinnedPool& pool = pinnedPool();
-  std::lock_guard<std::mutex> lock(pool.mutex);
-  auto it = pool.live.upper_bound(static_cast<const char*>(p));
-  if (it == pool.live.begin()) return false;
-  --it;
-  return static_cast<const char*>(p) + bytes <= it->first + it->second;
-}
+bool isPinned(const void* p, size_t bytes) { return pinnedPool().holds(p, bytes); }
 
 void initRuntimes() {
   static bool done = false;
