@@ -28,7 +28,16 @@ int fail(const std::string& msg) {
 int check(hipError_t e, const char* what) {
   if (e == hipSuccess) return 0;
   g_err = std::string(what) + ": " + hipGetErrorString(e);
+  (void)hipGetLastError();  // (reported here, and not again by the launch that comes next)
   return 1;
+}
+
+// Device memory that a caller can do without: nullptr when there is none.
+void* alloc_or_null(size_t bytes) {
+  void* p = nullptr;
+  if (hipMalloc(&p, bytes) == hipSuccess) return p;
+  (void)hipGetLastError();
+  return nullptr;
 }
 
 enum PlanKind { PLAN_GEMM = 1, PLAN_CONV, PLAN_DWCONV, PLAN_POOL, PLAN_ELTWISE, PLAN_CONTRACT, PLAN_PRODUCT, PLAN_CONV_GRAD };
@@ -477,10 +486,9 @@ void prepare_split(Plan* p, int64_t m, int64_t n, int64_t slabs) {
   igemm_split_plan(m, n, slabs, device_cus(), &splits, &per);
   if (splits < 2) return;
   const int64_t pitch = (n + 3) / 4 * 4;
-  if (pitch >= ((int64_t)1 << 31) || hipMalloc(&p->ws, (size_t)splits * m * pitch * 4) != hipSuccess) {
-    p->ws = nullptr;
-    return;
-  }
+  if (pitch >= ((int64_t)1 << 31)) return;
+  p->ws = alloc_or_null((size_t)splits * m * pitch * 4);
+  if (!p->ws) return;
   p->sk_splits = splits;
   p->sk_per = per;
   p->sk_pitch = (int)pitch;
@@ -831,12 +839,12 @@ int64_t pml_hip_gemm_dispatch(const pml_hip_gemm_desc* d) {
   p->bt_bytes = (size_t)d->n * d->k * es;
   if (p->tile == TILE_64x64_KSPLIT && !p->ws) p->tile = TILE_64x64;  // (not worth splitting, or no memory for the workspace)
   p->b_split = kind == KIND_F32X3 && !d->b_layout && d->k % 32 == 0 && !p->ws;
-  if (!d->b_layout && hipMalloc(&p->bt, p->bt_bytes) != hipSuccess) {
+  if (!d->b_layout && !(p->bt = alloc_or_null(p->bt_bytes))) {
     delete p;
     fail("gemm: cannot allocate the packed right-hand side");
     return 0;
   }
-  if (d->k2 > 0 && !d->b_layout && hipMalloc(&p->bt2, (size_t)d->n * d->k2 * es) != hipSuccess) {
+  if (d->k2 > 0 && !d->b_layout && !(p->bt2 = alloc_or_null((size_t)d->n * d->k2 * es))) {
     delete p;
     fail("gemm: cannot allocate the second packed right-hand side");
     return 0;
@@ -1116,7 +1124,7 @@ int64_t pml_hip_conv2d_dispatch(const pml_hip_conv2d_desc* d) {
     const int64_t v = 16 / es;
     p->kpad = (K + v - 1) / v * v;
     p->bt_ld = p->kpad;
-    if (hipMalloc(&p->patches, (size_t)M * p->kpad * es) != hipSuccess) {
+    if (!(p->patches = alloc_or_null((size_t)M * p->kpad * es))) {
       delete p;
       fail("conv2d: cannot allocate the patch matrix");
       return 0;
@@ -1128,7 +1136,7 @@ int64_t pml_hip_conv2d_dispatch(const pml_hip_conv2d_desc* d) {
   // (whole 128-byte chunks per filter tap, so that no chunk of heads + remainders straddles two taps)
   p->b_split = kind == KIND_F32X3 && !via_s2d && !via_patches && d->ci % 32 == 0 && !p->ws;
   p->bt_bytes = (size_t)d->co * p->bt_ld * es;
-  if (hipMalloc(&p->bt, p->bt_bytes) != hipSuccess || hipMemset(p->bt, 0, p->bt_bytes) != hipSuccess) {
+  if (!(p->bt = alloc_or_null(p->bt_bytes)) || hipMemset(p->bt, 0, p->bt_bytes) != hipSuccess) {
     delete p;
     fail("conv2d: cannot allocate the packed filter");
     return 0;
@@ -1279,10 +1287,8 @@ int pml_hip_conv2d_invoke(int64_t plan, const void* input, const void* filter, v
       {
         std::lock_guard<std::mutex> lock(p->s2d_mutex);
         // 256 spare bytes: a K-run that starts left of the image is addressed (never read) below the buffer's end only
-        if (!p->s2d && hipMalloc(&p->s2d, (size_t)d.n * p->s2d_h * p->s2d_w * p->s2d_ch * es + 256) != hipSuccess) {
-          p->s2d = nullptr;
-          return fail("conv2d_invoke: cannot allocate the re-blocked input");
-        }
+        if (!p->s2d) p->s2d = alloc_or_null((size_t)d.n * p->s2d_h * p->s2d_w * p->s2d_ch * es + 256);
+        if (!p->s2d) return fail("conv2d_invoke: cannot allocate the re-blocked input");
       }
       g.A = p->s2d;
       S2dArgs sa;
@@ -1485,9 +1491,8 @@ static bool prepare_strided(Plan* p) {
   StridedArgs& a = p->strided;
   strided_plan(&a, p->strided_bf, p->strided_conv, device_cus(), &p->strided_mi);
   a.ws = nullptr;
-  if (a.splits > 1 && hipMalloc(&p->ws, (size_t)a.splits * a.ws_rows * a.ws_pitch * 4) != hipSuccess) {
-    (void)hipGetLastError();
-    p->ws = nullptr;  // (no memory for the partial results: the K loop is not split)
+  if (a.splits > 1) p->ws = alloc_or_null((size_t)a.splits * a.ws_rows * a.ws_pitch * 4);
+  if (a.splits > 1 && !p->ws) {  // (no memory for the partial results: the K loop is not split)
     a.splits = 1;
     a.k_per_split = (a.K + 63) / 64 * 64;
   }
@@ -1687,7 +1692,7 @@ int64_t pml_hip_conv2d_grad_dispatch(const pml_hip_conv2d_desc* d, int which) {
       return 0;
     }
     p->sub->packed = true;  // (every invoke lays the filter out itself)
-    if (p->co_pad != d->co && hipMalloc(&p->padded, (size_t)(d->n * d->oh * d->ow * p->co_pad * es)) != hipSuccess) {
+    if (p->co_pad != d->co && !(p->padded = alloc_or_null((size_t)(d->n * d->oh * d->ow * p->co_pad * es)))) {
       delete p;
       fail("conv2d_grad: cannot allocate the padded gradient");
       return 0;
@@ -1709,7 +1714,7 @@ int64_t pml_hip_conv2d_grad_dispatch(const pml_hip_conv2d_desc* d, int which) {
   a.b_ks = 1;
   a.b_ns = d->co;
   a.c_ms = taps_ci;
-  if (hipMalloc(&p->cols, (size_t)(p->grad_chunk * per_image)) != hipSuccess) {
+  if (!(p->cols = alloc_or_null((size_t)(p->grad_chunk * per_image)))) {
     delete p;
     fail("conv2d_grad: cannot allocate the columns");
     return 0;
