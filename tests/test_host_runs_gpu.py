@@ -19,3 +19,58 @@ def test_an_allocation_that_fails_does_not_fail_the_next_launch():
     buf = hk.DeviceBuffer(4096)
     hk.check(L.pml_hip_fill_u32(buf.ptr, 0x01020304, 1024, None))
     np.testing.assert_array_equal(buf.to_numpy(np.uint32, (1024,)), 0x01020304)
+
+
+def _program(dtype, n, m=300):
+    X, Y = P.Placeholder(DT[dtype], [n]), P.Placeholder(DT[dtype], [m])
+    return P.Program('host', [X, Y], [X * 2.0 + 1.0, Y - 1.0, X * -1.0])
+
+
+def _round(a, dtype):
+    return P.round_bf16(a) if dtype == 'bf16' else a
+
+
+def _arrays(seed, dtype, n, m=300):
+    rng = np.random.default_rng(seed)
+    return [rng.standard_normal(n).astype(np.float32), rng.standard_normal(m).astype(np.float32)]
+
+
+def _check(got, arrays, dtype):
+    x, y = (_round(a, dtype) for a in arrays)
+    # (rounded after each operation, as the separate operations round)
+    want = [_round(_round(x * np.float32(2), dtype) + np.float32(1), dtype), _round(y - np.float32(1), dtype), -x]
+    for g, w in zip(got, want):
+        np.testing.assert_array_equal(g, w)
+
+
+# elements of a 4 MB piece, and of the 512 KB that still go by kernel
+PIECE, KERNEL = {'f32': 1 << 20, 'bf16': 1 << 21}, {'f32': 1 << 17, 'bf16': 1 << 18}
+
+
+@pytest.mark.parametrize('dtype', ['f32', 'bf16'])
+@pytest.mark.parametrize('pinned_results', [True, False])
+@pytest.mark.parametrize('size', ['one', 'kernel', 'past kernel', 'piece', 'past piece', 'slots', 'past slots', 'two rounds'])
+def test_arrays_around_the_sizes_of_the_staging(monkeypatch, dtype, pinned_results, size):
+    """A value and its two results, with a small one beside them: copied by kernel, in a place of their own (32 MB in all),
+    through the eight slots in turn; every run with other values."""
+    k, p = KERNEL[dtype], PIECE[dtype]
+    n = {'one': 1, 'kernel': k, 'past kernel': k + 1, 'piece': p, 'past piece': p + 1, 'slots': 8 * p // 3, 'past slots': 8 * p // 3 + 4096,
+         'two rounds': 13 * p + 3}[size]
+    if not pinned_results:
+        monkeypatch.setattr(P, '_result_array', lambda dt, sizes, nbytes: np.empty(sizes, dt))
+    runner = P.Runner(_program(dtype, n), target='hip')
+    for run in range(4):
+        arrays = _arrays(run, dtype, n)
+        _check(runner.run(arrays), arrays, dtype)
+
+
+@pytest.mark.parametrize('dtype', ['f32', 'bf16'])
+def test_runs_without_page_locked_memory(monkeypatch, dtype):
+    """PLAIDML_PINNED=0 and a cap that is reached: ordinary copies; the staging is back as soon as there is memory for it."""
+    n = PIECE[dtype] + 5
+    runner = P.Runner(_program(dtype, n), target='hip')
+    for run, (key, value) in enumerate([('PLAIDML_PINNED', '0'), ('PLAIDML_PINNED_MAX_MB', '1'), ('PLAIDML_PINNED', '1'), ('PLAIDML_PINNED_MAX_MB', '2')]):
+        with monkeypatch.context() as patch:
+            patch.setenv(key, value)
+            arrays = _arrays(run, dtype, n)
+            _check(runner.run(arrays), arrays, dtype)
