@@ -963,6 +963,8 @@ class Executable(_Handle):
 
 
 def last_run_stats():
+    """Of this thread's last run: its wall time as kernel_ms (device, first to last launch), h2d_ms (host, up to the last upload it
+    queues) and d2h_ms (the rest); its launches and whether they ran as a recorded graph; the executable's device memory."""
     k, h, d, n = f64(), f64(), f64(), sz()
     lib().plaidml_hip_last_run_stats(ctypes.byref(k), ctypes.byref(h), ctypes.byref(d), ctypes.byref(n))
     a, u, t = sz(), sz(), sz()

@@ -880,7 +880,8 @@ void* plaidml_hip_host_alloc(size_t bytes) {
 }
 void plaidml_hip_host_free(void* p) { rt::pinnedFree(p); }
 
-// Not part of the reference ABI: timing breakdown of the calling thread's most recent run, for benchmarks.
+// Not part of the reference ABI: the wall time of the calling thread's most recent run in three parts, for benchmarks -- the
+// device's from first to last launch, the host's up to the last upload it queues, and the rest (rt::InvokeStats).
 void plaidml_hip_last_run_stats(double* kernel_ms, double* h2d_ms, double* d2h_ms, size_t* launches) {
   rt::InvokeStats s = rt::lastInvokeStats();
   if (kernel_ms) *kernel_ms = s.kernel_ms;

@@ -108,7 +108,6 @@ class HipExecutable final : public Executable {
       throw std::runtime_error("executable invoked with the wrong number of buffers");
     InvokeStats st;
     const double start = nowMs();
-    double t0 = start;
     const bool profile = profileRequested();
     for (size_t i = 0; i < outputs.size(); ++i)
       if (outputs[i].bytes < spanBytes(plan_->output_buffers[i], outputs[i])) throw std::runtime_error("output buffer #" + std::to_string(i) + " is too small");
@@ -147,9 +146,8 @@ class HipExecutable final : public Executable {
         }
       }
       up.issue(stream_);
-      st.h2d_ms = nowMs() - t0;
+      st.h2d_ms = nowMs() - start;
       launchAll(profile, &st);
-      t0 = nowMs();
       for (size_t i = 0; i < outputs.size(); ++i) {
         const int buf = plan_->output_buffers[i];
         const size_t bytes = plan_->buffers[buf].bytes;
@@ -177,9 +175,9 @@ class HipExecutable final : public Executable {
       hipCheck(pml_hip_memcpy_d2h(tmp.data(), device_[buf], bytes, stream_), "d2h");
       hostFromBf16(static_cast<float*>(outputs[i].data), tmp.data(), tmp.size());
     }
-    st.d2h_ms = nowMs() - t0;
-    finish(profile, &st);
     st.wall_ms = nowMs() - start;
+    finish(profile, &st);
+    st.d2h_ms = std::max(0.0, st.wall_ms - st.h2d_ms - st.kernel_ms);
     g_stats = st;
     // wall time of the whole run, transfers included, as the reference returns the time around its jitted main
     // (pmlc/rt/jit_executable.cc:484-490); the device time alone is in the statistics

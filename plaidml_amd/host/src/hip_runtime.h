@@ -68,7 +68,11 @@ bool isPinned(const void* p, size_t bytes);
 
 // statistics of the most recent invoke of any hip executable in this thread (for benchmarks)
 struct InvokeStats {
-  double kernel_ms = 0;  // first launch -> last launch, HIP events
+  // The wall time in three parts.  Uploads, launches and downloads are queued on one stream and waited for once, so where
+  // the link's share ends is not seen from here (two more events a run would cost 2 to 15 us): h2d_ms is the host's time up
+  // to the last upload it queues, rounding and staging included; kernel_ms the device's, first launch -> last launch, by HIP
+  // events; d2h_ms the rest -- what of the uploads is still under way then, the downloads, the passes over the results.
+  double kernel_ms = 0;
   double h2d_ms = 0;
   double d2h_ms = 0;
   size_t launches = 0;

@@ -74,3 +74,14 @@ def test_runs_without_page_locked_memory(monkeypatch, dtype):
             patch.setenv(key, value)
             arrays = _arrays(run, dtype, n)
             _check(runner.run(arrays), arrays, dtype)
+
+
+@pytest.mark.parametrize('dtype,n', [('f32', 1000), ('bf16', 3 * PIECE['bf16'] + 1)])
+def test_statistics_are_the_wall_time_in_three_parts(dtype, n):
+    runner = P.Runner(_program(dtype, n), target='hip')
+    for run in range(4):
+        runner.run(_arrays(run, dtype, n))
+        s = P.last_run_stats()
+        assert s['kernel_ms'] > 0 and s['h2d_ms'] > 0 and s['d2h_ms'] >= 0
+        # (the reading of the events themselves comes after the clock)
+        assert s['h2d_ms'] + s['kernel_ms'] + s['d2h_ms'] == pytest.approx(runner.ms, rel=1e-6, abs=1e-9)
