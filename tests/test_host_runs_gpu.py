@@ -1,5 +1,6 @@
 """Runs on arrays in host memory (host/src/hip_runtime.cc, Runner) around the edges of their staging."""
 import ctypes
+import threading
 
 import numpy as np
 import pytest
@@ -85,3 +86,87 @@ def test_statistics_are_the_wall_time_in_three_parts(dtype, n):
         assert s['kernel_ms'] > 0 and s['h2d_ms'] > 0 and s['d2h_ms'] >= 0
         # (the reading of the events themselves comes after the clock)
         assert s['h2d_ms'] + s['kernel_ms'] + s['d2h_ms'] == pytest.approx(runner.ms, rel=1e-6, abs=1e-9)
+
+
+@pytest.mark.parametrize('n', [5, 70000, 600001])
+def test_inputs_of_other_types_and_layouts(n):
+    """bfloat16 as stored bits, arrays that are not contiguous, of another type, lists: what arrives is their value."""
+    runner = P.Runner(_program('bf16', n), target='hip')
+    x, y = _arrays(n, 'bf16', n)
+    x[:3] = [np.nan, np.inf, -0.0]
+    want = runner.run([x, y])
+    _check([w[3:] if len(w) == n else w for w in want], [x[3:], y], 'bf16')
+    wide = np.repeat(x, 2)
+    for a in (P.to_bf16_bits(x), np.repeat(P.to_bf16_bits(x), 2)[::2], wide[::2], x.astype(np.float64), x[::-1].copy()[::-1], list(map(float, x)) if n < 10 else x):
+        for g, w in zip(runner.run([a, y]), want):
+            np.testing.assert_array_equal(g.view(np.uint32), w.view(np.uint32))
+
+
+@pytest.mark.parametrize('dtype', ['f32', 'bf16'])
+@pytest.mark.parametrize('n', [1000, 40000, 300000, 1200007])
+def test_results_fed_back(dtype, n):
+    """A result lies in page-locked memory and goes back from where it lies; so does a part of it that begins at any element."""
+    X = P.Placeholder(DT[dtype], [n])
+    runner = P.Runner(P.Program('step', [X], [X + 1.0]), target='hip')
+    x = np.arange(n, dtype=np.float32) % 100
+    first, = runner.run([x])
+    second, = runner.run([first])
+    np.testing.assert_array_equal(first, x + 1)  # (the second run left the first one's results alone)
+    np.testing.assert_array_equal(second, x + 2)
+    Y = P.Placeholder(DT[dtype], [n - 3])
+    part = P.Runner(P.Program('step', [Y], [Y + 1.0]), target='hip')
+    for _ in range(4):
+        got, = part.run([second[1:n - 2]])
+        np.testing.assert_array_equal(got, x[1:n - 2] + 3)
+        got, = part.run([second[::-1][:n - 3]])
+        np.testing.assert_array_equal(got, x[::-1][:n - 3] + 3)
+
+
+@pytest.mark.parametrize('dtype', ['f32', 'bf16'])
+def test_runs_from_several_threads(dtype):
+    """An executable of its own per thread; their passes over arrays share the helper threads, which only one of them gets."""
+    n, wrong = 3 * PIECE[dtype] + 11, []
+
+    def work(seed):
+        try:
+            runner = P.Runner(_program(dtype, n), target='hip')
+            for run in range(4):
+                arrays = _arrays(10 * seed + run, dtype, n)
+                _check(runner.run(arrays), arrays, dtype)
+                assert runner.ms > 0
+        except BaseException as e:  # noqa: B902
+            wrong.append(e)
+    threads = [threading.Thread(target=work, args=(s,)) for s in range(3)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong, wrong[0]
+
+
+@pytest.mark.parametrize('dtype', ['f32', 'bf16'])
+def test_outputs_hold_the_last_run_of_either_kind(dtype):
+    n = 50000
+    runner = P.Runner(_program(dtype, n), target='hip')
+    sets = [_arrays(s, dtype, n) for s in range(4)]
+    staged = runner.stage(sets[1])
+    _check(runner.run(sets[0]), sets[0], dtype)
+    _check(runner.fetch(), sets[0], dtype)
+    runner.run_staged(staged)
+    _check(runner.fetch(), sets[1], dtype)
+    kept = runner.run(sets[2])
+    _check(runner.fetch(), sets[2], dtype)
+    _check(runner.run(sets[3]), sets[3], dtype)
+    _check(kept, sets[2], dtype)
+    runner.run_staged(staged)
+    _check(runner.fetch(), sets[1], dtype)
+
+
+def test_arrays_that_do_not_fit_are_refused():
+    runner = P.Runner(_program('f32', 100), target='hip')
+    x, y = _arrays(0, 'f32', 100)
+    with pytest.raises(Exception):
+        runner.run([x[:99], y])
+    with pytest.raises(Exception):
+        runner.run([x])
+    _check(runner.run([x, y]), [x, y], 'f32')
