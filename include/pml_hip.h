@@ -695,6 +695,8 @@ size_t pml_hip_struct_size(int which);
 
 /* Releases a plan returned by any *_dispatch. */
 int pml_hip_plan_free(int64_t plan);
+/* Device memory that the plan holds: re-laid operands, workspaces (some are first asked for by an invoke or a pack). */
+size_t pml_hip_plan_bytes(int64_t plan);
 /* Writes a one-line description of the plan (kernel family, tile, grid) for plan dumps. */
 int pml_hip_plan_describe(int64_t plan, char* buf, size_t buf_len);
 

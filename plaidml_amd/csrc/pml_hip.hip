@@ -101,6 +101,19 @@ struct Plan {
   size_t halo_lds = 0;
   int halo_rows = 0, halo_tiles = 0, halo_variant = 0, n_cus = 0;
   std::string text;
+  std::atomic<size_t> held{0};  // bytes of device memory in all of the above
+  void* hold(size_t bytes) {
+    void* mem = alloc_or_null(bytes);
+    if (mem) held += bytes;
+    return mem;
+  }
+  void drop(void** mem, size_t bytes) {
+    if (*mem) {
+      (void)hipFree(*mem);
+      held -= bytes;
+    }
+    *mem = nullptr;
+  }
   ~Plan() {
     if (bt) (void)hipFree(bt);
     if (bt2) (void)hipFree(bt2);
@@ -478,7 +491,7 @@ void* scratch_of_current_device() {
   return g_scratch_ptr[dev];
 }
 
-// A plan whose tile is TILE_64x64_KSPLIT: decides the split for m x n results over `slabs` slabs of K and allocates the
+// A plan whose tile is TILE_64x64_KSPLIT and is what its invokes may run: decides the split for m x n results over `slabs` slabs of K and allocates the
 // workspace.  Leaves the plan unsplit (the plain 64 x 64 tile runs) when a split is not worth it or memory is short.
 void prepare_split(Plan* p, int64_t m, int64_t n, int64_t slabs) {
   if (p->tile != TILE_64x64_KSPLIT) return;
@@ -487,7 +500,7 @@ void prepare_split(Plan* p, int64_t m, int64_t n, int64_t slabs) {
   if (splits < 2) return;
   const int64_t pitch = (n + 3) / 4 * 4;
   if (pitch >= ((int64_t)1 << 31)) return;
-  p->ws = alloc_or_null((size_t)splits * m * pitch * 4);
+  p->ws = p->hold((size_t)splits * m * pitch * 4);
   if (!p->ws) return;
   p->sk_splits = splits;
   p->sk_per = per;
@@ -832,29 +845,34 @@ int64_t pml_hip_gemm_dispatch(const pml_hip_gemm_desc* d) {
     classify_tail(d->tail, d->out_dtype, d->c_dtype, &mode, &relu);
     const bool plain = mode == 1 || mode == 2 || tail_requant(d->tail, d->out_dtype, d->c_dtype, mode, nullptr);
     p->tile = choose_tile(d->m, d->n, (d->k + d->k2) * dt_size(d->in_dtype), kind, plain, PML_HIP_FLAG_TILE_OF(d->flags));
-    // (a second product's slabs follow the first one's on the slab axis the splits share out)
-    prepare_split(p, d->m, d->n, (d->k * dt_size(d->in_dtype) + 127) / 128 + (d->k2 * dt_size(d->in_dtype) + 127) / 128);
+    // (a second product's slabs follow the first one's on the slab axis the splits share out.)  With a direct tile over rows
+    // that are at hand the LDS tile is only left for a [K][N] right-hand side that arrives with the call and cannot be read
+    // as it lies; pml_hip_gemm_pack_b ends that.
+    p->direct = direct_tiles(*d, kind);
+    if (!(p->direct.rows >= 0 && (d->b_layout || kind == KIND_F32)))
+      prepare_split(p, d->m, d->n, (d->k * dt_size(d->in_dtype) + 127) / 128 + (d->k2 * dt_size(d->in_dtype) + 127) / 128);
   }
   p->bt_ld = d->k;
   p->bt_bytes = (size_t)d->n * d->k * es;
-  if (p->tile == TILE_64x64_KSPLIT && !p->ws) p->tile = TILE_64x64;  // (not worth splitting, or no memory for the workspace)
+  // (the text names the LDS tile of the problem's shape beside the direct tile that takes its place)
+  const int lds_tile = p->tile;
+  if (p->tile == TILE_64x64_KSPLIT && !p->ws) p->tile = TILE_64x64;  // (not worth splitting, no memory for the workspace, or not run)
   p->b_split = kind == KIND_F32X3 && !d->b_layout && d->k % 32 == 0 && !p->ws;
-  if (!d->b_layout && !(p->bt = alloc_or_null(p->bt_bytes))) {
+  if (!d->b_layout && !(p->bt = p->hold(p->bt_bytes))) {
     delete p;
     fail("gemm: cannot allocate the packed right-hand side");
     return 0;
   }
-  if (d->k2 > 0 && !d->b_layout && !(p->bt2 = alloc_or_null((size_t)d->n * d->k2 * es))) {
+  if (d->k2 > 0 && !d->b_layout && !(p->bt2 = p->hold((size_t)d->n * d->k2 * es))) {
     delete p;
     fail("gemm: cannot allocate the second packed right-hand side");
     return 0;
   }
   char buf[256];
   std::snprintf(buf, sizeof buf, "gemm %s m=%lld n=%lld k=%lld tile=%s mfma=%s", d->in_dtype == PML_HIP_F32 ? "f32" : d->in_dtype == PML_HIP_BF16 ? "bf16" : "i8",
-                (long long)d->m, (long long)d->n, (long long)d->k, tile_name(p->tile),
+                (long long)d->m, (long long)d->n, (long long)d->k, tile_name(p->direct.rows >= 0 ? lds_tile : p->tile),
                 kind == KIND_F32 ? "f32_32x32x2" : kind == KIND_BF16 ? "f32_32x32x16_bf16" : kind == KIND_I8 ? "i32_32x32x32_i8" : "3 x f32_32x32x16_bf16 (fp32 split into bf16 head + remainder)");
   p->text = buf;
-  p->direct = direct_tiles(*d, kind);
   if (p->direct.rows >= 0) p->text += std::string(", with rows of K at hand tile=") + tile_name(p->direct.rows);
   if (d->k2 > 0) p->text += " + second product k2=" + std::to_string(d->k2) + (d->a2_stride > 0 ? " over pixel rows of stride " + std::to_string(d->a2_stride) : "");
   return (int64_t)(intptr_t)p;
@@ -1124,19 +1142,15 @@ int64_t pml_hip_conv2d_dispatch(const pml_hip_conv2d_desc* d) {
     const int64_t v = 16 / es;
     p->kpad = (K + v - 1) / v * v;
     p->bt_ld = p->kpad;
-    if (!(p->patches = alloc_or_null((size_t)M * p->kpad * es))) {
+    if (!(p->patches = p->hold((size_t)M * p->kpad * es))) {
       delete p;
       fail("conv2d: cannot allocate the patch matrix");
       return 0;
     }
   }
   if (!via_s2d && !via_patches && PML_HIP_FLAG_TILE_OF(d->flags) < 0) p->tile_direct = direct_tile_of(M, d->co, K * es, kind);
-  if (!via_s2d && !via_patches) prepare_split(p, M, d->co, d->kh * d->kw * ((d->ci * es + 127) / 128));
-  if (p->tile == TILE_64x64_KSPLIT && !p->ws) p->tile = TILE_64x64;
-  // (whole 128-byte chunks per filter tap, so that no chunk of heads + remainders straddles two taps)
-  p->b_split = kind == KIND_F32X3 && !via_s2d && !via_patches && d->ci % 32 == 0 && !p->ws;
   p->bt_bytes = (size_t)d->co * p->bt_ld * es;
-  if (!(p->bt = alloc_or_null(p->bt_bytes)) || hipMemset(p->bt, 0, p->bt_bytes) != hipSuccess) {
+  if (!(p->bt = p->hold(p->bt_bytes)) || hipMemset(p->bt, 0, p->bt_bytes) != hipSuccess) {
     delete p;
     fail("conv2d: cannot allocate the packed filter");
     return 0;
@@ -1159,11 +1173,16 @@ int64_t pml_hip_conv2d_dispatch(const pml_hip_conv2d_desc* d) {
       }
     }
   }
+  if (!via_s2d && !via_patches && !p->halo_lds && p->tile_direct < 0) prepare_split(p, M, d->co, d->kh * d->kw * ((d->ci * es + 127) / 128));
+  const int lds_tile = p->tile;  // (named in the text beside the direct tile that takes its place)
+  if (p->tile == TILE_64x64_KSPLIT && !p->ws) p->tile = TILE_64x64;
+  // (whole 128-byte chunks per filter tap, so that no chunk of heads + remainders straddles two taps)
+  p->b_split = kind == KIND_F32X3 && !via_s2d && !via_patches && d->ci % 32 == 0 && !p->ws;
   char buf[256];
   std::snprintf(buf, sizeof buf, "conv2d %s n=%lld %lldx%lldx%lld k=%lldx%lld co=%lld -> %lldx%lld (implicit gemm m=%lld n=%lld k=%lld) tile=%s",
                 d->in_dtype == PML_HIP_F32 ? "f32" : d->in_dtype == PML_HIP_BF16 ? "bf16" : "i8", (long long)d->n,
                 (long long)d->h, (long long)d->w, (long long)d->ci, (long long)d->kh, (long long)d->kw, (long long)d->co,
-                (long long)d->oh, (long long)d->ow, (long long)M, (long long)d->co, (long long)K, p->halo_lds ? (p->halo_variant == 3 ? "256x64 resident filter, in registers" : p->halo_variant ? "256x64 resident filter, pipelined 3x3" : "256x64 resident filter") : tile_name(p->tile));
+                (long long)d->oh, (long long)d->ow, (long long)M, (long long)d->co, (long long)K, p->halo_lds ? (p->halo_variant == 3 ? "256x64 resident filter, in registers" : p->halo_variant ? "256x64 resident filter, pipelined 3x3" : "256x64 resident filter") : tile_name(p->tile_direct >= 0 ? lds_tile : p->tile));
   p->text = buf;
   if (kind == KIND_F32X3) p->text += " mfma=3 x f32_32x32x16_bf16 (fp32 split into bf16 head + remainder)";
   if (p->tile_direct >= 0 && !p->halo_lds) p->text += std::string(", direct tile=") + tile_name(p->tile_direct);
@@ -1287,7 +1306,7 @@ int pml_hip_conv2d_invoke(int64_t plan, const void* input, const void* filter, v
       {
         std::lock_guard<std::mutex> lock(p->s2d_mutex);
         // 256 spare bytes: a K-run that starts left of the image is addressed (never read) below the buffer's end only
-        if (!p->s2d) p->s2d = alloc_or_null((size_t)d.n * p->s2d_h * p->s2d_w * p->s2d_ch * es + 256);
+        if (!p->s2d) p->s2d = p->hold((size_t)d.n * p->s2d_h * p->s2d_w * p->s2d_ch * es + 256);
         if (!p->s2d) return fail("conv2d_invoke: cannot allocate the re-blocked input");
       }
       g.A = p->s2d;
@@ -1321,6 +1340,12 @@ int pml_hip_gemm_pack_b(int64_t plan, const void* b, pml_hip_stream s) {
   if (p->b_split && check(split_rows_launch(p->bt, d.n, p->bt_ld, d.k, (hipStream_t)s), "split_rows_launch")) return 1;
   p->bt_is_split = p->b_split;
   p->packed = true;
+  if ((p->direct.rows >= 0 || d.k2 > 0) && p->ws) {
+    // (its invokes take the direct tile from now on; one that brings a right-hand side all the same does not split K, nor do
+    // those of two products)
+    p->drop(&p->ws, (size_t)p->sk_splits * d.m * p->sk_pitch * 4);
+    p->tile = TILE_64x64;
+  }
   return 0;
 }
 
@@ -1388,7 +1413,7 @@ int pml_hip_conv2d_pack_filter(int64_t plan, const void* filter, pml_hip_stream 
   if (check(pack_conv_filter(p, filter, (hipStream_t)s), "pack_conv_filter")) return 1;
   if (p->halo_lds && p->halo_variant == 3 && regfilter_takes_image((int)d.ow)) {
     // the register-filter kernel takes a constant filter in its own register order: no trip through LDS per launch
-    if (!p->reg_image && check(hipMalloc(&p->reg_image, kRegfilterImageBytes), "hipMalloc")) return 1;
+    if (!p->reg_image && !(p->reg_image = p->hold(kRegfilterImageBytes))) return fail("conv2d_pack_filter: cannot allocate the filter in register order");
     if (check(regfilter_image_launch(p->bt, p->bt_ld * dt_size(d.in_dtype), p->reg_image, (hipStream_t)s), "regfilter_image_launch")) return 1;
   }
   p->packed = true;
@@ -1491,7 +1516,7 @@ static bool prepare_strided(Plan* p) {
   StridedArgs& a = p->strided;
   strided_plan(&a, p->strided_bf, p->strided_conv, device_cus(), &p->strided_mi);
   a.ws = nullptr;
-  if (a.splits > 1) p->ws = alloc_or_null((size_t)a.splits * a.ws_rows * a.ws_pitch * 4);
+  if (a.splits > 1) p->ws = p->hold((size_t)a.splits * a.ws_rows * a.ws_pitch * 4);
   if (a.splits > 1 && !p->ws) {  // (no memory for the partial results: the K loop is not split)
     a.splits = 1;
     a.k_per_split = (a.K + 63) / 64 * 64;
@@ -1692,7 +1717,7 @@ int64_t pml_hip_conv2d_grad_dispatch(const pml_hip_conv2d_desc* d, int which) {
       return 0;
     }
     p->sub->packed = true;  // (every invoke lays the filter out itself)
-    if (p->co_pad != d->co && !(p->padded = alloc_or_null((size_t)(d->n * d->oh * d->ow * p->co_pad * es)))) {
+    if (p->co_pad != d->co && !(p->padded = p->hold((size_t)(d->n * d->oh * d->ow * p->co_pad * es)))) {
       delete p;
       fail("conv2d_grad: cannot allocate the padded gradient");
       return 0;
@@ -1714,7 +1739,7 @@ int64_t pml_hip_conv2d_grad_dispatch(const pml_hip_conv2d_desc* d, int which) {
   a.b_ks = 1;
   a.b_ns = d->co;
   a.c_ms = taps_ci;
-  if (!(p->cols = alloc_or_null((size_t)(p->grad_chunk * per_image)))) {
+  if (!(p->cols = p->hold((size_t)(p->grad_chunk * per_image)))) {
     delete p;
     fail("conv2d_grad: cannot allocate the columns");
     return 0;
@@ -1861,12 +1886,9 @@ int pml_hip_dwconv2d_pack_filter(int64_t plan, const void* filter, pml_hip_strea
   if (!p || p->kind != PLAN_DWCONV || !filter) return fail("dwconv2d_pack_filter: bad argument");
   const pml_hip_dwconv2d_desc& d = p->dw;
   const size_t bytes = (size_t)d.kh * d.kw * d.c * dt_size(d.dtype);
-  if (!p->dw_filter && check(hipMalloc(&p->dw_filter, bytes), "hipMalloc")) return 1;
+  if (!p->dw_filter && !(p->dw_filter = p->hold(bytes))) return fail("dwconv2d_pack_filter: cannot allocate the filter");
   if (check(hipMemcpyAsync(p->dw_filter, filter, bytes, hipMemcpyDeviceToDevice, (hipStream_t)s), "hipMemcpyAsync")) return 1;
-  if (p->dw_paired) {
-    (void)hipFree(p->dw_paired);
-    p->dw_paired = nullptr;
-  }
+  p->drop(&p->dw_paired, (size_t)12 * (d.c / 8) * 4 * 4);
   if (!dwconv2d_takes_paired_filter(d)) return 0;
   // once per filter: its weights are looked at on the host (the paired kernel is for finite weights only) and re-laid there
   std::vector<uint16_t> host(bytes / 2);
@@ -1875,10 +1897,9 @@ int pml_hip_dwconv2d_pack_filter(int64_t plan, const void* filter, pml_hip_strea
     return 1;
   std::vector<uint32_t> packed((size_t)12 * (d.c / 8) * 4);
   if (!dwconv2d_pair_filter(host.data(), d.c, packed.data())) return 0;  // an infinite or NaN weight: the general kernel
-  if (check(hipMalloc(&p->dw_paired, packed.size() * 4), "hipMalloc")) return 1;
+  if (!(p->dw_paired = p->hold(packed.size() * 4))) return fail("dwconv2d_pack_filter: cannot allocate the paired filter");
   if (check(hipMemcpy(p->dw_paired, packed.data(), packed.size() * 4, hipMemcpyHostToDevice), "hipMemcpy")) {
-    (void)hipFree(p->dw_paired);
-    p->dw_paired = nullptr;
+    p->drop(&p->dw_paired, packed.size() * 4);
     return 1;
   }
   return 0;
@@ -2210,6 +2231,11 @@ size_t pml_hip_struct_size(int which) {
 int pml_hip_plan_free(int64_t plan) {
   delete (Plan*)(intptr_t)plan;
   return 0;
+}
+
+size_t pml_hip_plan_bytes(int64_t plan) {
+  const Plan* p = (const Plan*)(intptr_t)plan;
+  return p ? p->held + (p->sub ? p->sub->held.load() : 0) : 0;
 }
 
 int pml_hip_plan_describe(int64_t plan, char* buf, size_t buf_len) {

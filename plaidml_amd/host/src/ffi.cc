@@ -891,7 +891,7 @@ void plaidml_hip_last_run_stats(double* kernel_ms, double* h2d_ms, double* d2h_m
 }
 
 // Device memory of the executable behind the calling thread's most recent run: the arena its temporaries share,
-// what they would take unshared, and everything it holds on the device (arena + inputs + outputs + constants).
+// what they would take unshared, and everything it holds on the device (arena + inputs + outputs + constants + its kernel plans' memory).
 void plaidml_hip_last_run_memory(size_t* arena_bytes, size_t* unshared_temp_bytes, size_t* device_bytes) {
   rt::InvokeStats s = rt::lastInvokeStats();
   if (arena_bytes) *arena_bytes = s.arena_bytes;

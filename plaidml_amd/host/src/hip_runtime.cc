@@ -401,6 +401,8 @@ class HipExecutable final : public Executable {
     st->arena_bytes = arena_bytes_;
     st->unshared_temp_bytes = unshared_temp_bytes_;
     st->device_bytes = arena_bytes_ + fixed_bytes_;
+    for (int64_t h : handles_)
+      if (h) st->device_bytes += pml_hip_plan_bytes(h);
     if (!profile) return;
     // One row per launch, in the reference's format (pmlc/rt/instrument.cc:22-43: id, loc, tag, seconds since
     // the previous point, seconds since the start); loc is the plan's line for the step, tag its kind.

@@ -79,7 +79,7 @@ struct InvokeStats {
   double wall_ms = 0;              // the whole run, transfers included (what invoke returns)
   size_t arena_bytes = 0;          // device memory shared by the temporaries
   size_t unshared_temp_bytes = 0;  // what the temporaries would take with memory of their own
-  size_t device_bytes = 0;         // arena + inputs + outputs + constants
+  size_t device_bytes = 0;         // arena + inputs + outputs + constants + what the kernel plans hold
   std::vector<double> step_ms;     // per launch, only with PLAIDML_PROFILE=1
   bool replayed = false;           // the launches ran as one recorded graph
   std::string graph_note;          // why they did not, when recording was tried and failed

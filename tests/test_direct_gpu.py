@@ -140,3 +140,74 @@ def test_split_over_workgroups_by_name(kind, M, N, K, monkeypatch):
     got = T.run_gemm(cast(A), cast(B), dt, hk.I32 if kind == 'i8' else dt, invokes=2)
     want = A.astype(np.float64) @ B.astype(np.float64)
     check(E.bf16_from_bits(got) if kind == 'bf16' else got, want, kind, K)
+
+
+@pytest.mark.parametrize('M,N,K', [(49, 512, 2048), (196, 256, 2048), (100, 130, 4096), (1, 1000, 2048), (300, 72, 2064)])
+def test_gemm_k_split_where_direct_tiles_would_be_taken(M, N, K, monkeypatch, capsys):
+    """The K split over workgroups by name: most of these shapes take a direct tile otherwise."""
+    monkeypatch.setitem(T.FORCED, 'flags', hk.flag_tile('64x64ks'))
+    T.test_gemm_k_split_over_workgroups(M, N, K, capsys)
+
+
+@pytest.mark.parametrize('kind', ['bf16', 'f32'])
+@pytest.mark.parametrize('shape,k,co,stride', [((1, 7, 7, 512), 3, 512, 1), ((1, 14, 14, 256), 3, 256, 2), ((2, 9, 11, 96), 5, 40, 1)])
+def test_conv_k_split_where_direct_tiles_would_be_taken(kind, shape, k, co, stride, monkeypatch, capsys):
+    monkeypatch.setitem(T.FORCED, 'flags', hk.flag_tile('64x64ks'))
+    T.test_conv_k_split_over_workgroups(kind, shape, k, co, stride, capsys)
+
+
+def held(desc, family='gemm', which=None):
+    L = hk.lib()
+    plan = L.pml_hip_conv2d_grad_dispatch(ctypes.byref(desc), which) if which is not None else getattr(L, 'pml_hip_%s_dispatch' % family)(ctypes.byref(desc))
+    assert plan, L.pml_hip_last_error()
+    return plan, L.pml_hip_plan_bytes(plan)
+
+
+@pytest.mark.parametrize('kind,es', [('bf16', 2), ('i8', 1), ('f32', 4)])
+def test_plans_hold_what_their_invokes_read(kind, es):
+    """Workspaces of a split K only where no direct tile is taken: not for rows at hand, not for fp32, until the right-hand
+    side is packed for the rest; right-hand sides of [K][N] for the transposed copy."""
+    L, dt, N = hk.lib(), {'bf16': hk.BF16, 'i8': hk.I8, 'f32': hk.F32}[kind], 256
+    d = hk.GemmDesc()
+    d.in_dtype, d.out_dtype, d.c_dtype = dt, hk.I32 if kind == 'i8' else dt, hk.I32 if kind == 'i8' else dt
+    d.m, d.n, d.k = 196, N, 2048 if kind == 'i8' else 1024
+    d.lda = d.ldb = d.k
+    d.ldc, d.b_layout = N, 1
+    plan, bytes_ = held(d)
+    assert 'at hand tile=' in hk.describe(plan) and bytes_ == 0
+    L.pml_hip_plan_free(plan)
+    d.b_layout, d.ldb = 0, N
+    plan, bytes_ = held(d)
+    copy = N * d.k * es
+    assert bytes_ == copy if kind == 'f32' else bytes_ > copy
+    B = hk.DeviceBuffer(copy)
+    hk.check(L.pml_hip_fill_u32(B.ptr, 0, copy // 4, None))
+    hk.check(L.pml_hip_gemm_pack_b(plan, B.ptr, None))
+    assert L.pml_hip_plan_bytes(plan) == copy
+    L.pml_hip_plan_free(plan)
+
+
+def conv(dt, n, hw, ci, co, k, stride):
+    d = hk.Conv2dDesc()
+    d.in_dtype = d.out_dtype = d.c_dtype = dt
+    o = (hw + stride - 1) // stride
+    d.n, d.h, d.w, d.ci, d.kh, d.kw, d.co, d.oh, d.ow = n, hw, hw, ci, k, k, co, o, o
+    d.stride_h = d.stride_w = stride
+    d.dil_h = d.dil_w = 1
+    d.pad_h = d.pad_w = max(0, (o - 1) * stride + k - hw) // 2
+    return d
+
+
+def test_convolution_plans_hold_what_their_invokes_read():
+    for (hw, ci, co, k), split in (((28, 128, 128, 3), False), ((7, 512, 512, 3), True), ((56, 64, 64, 3), False)):
+        plan, bytes_ = held(conv(hk.BF16, 1, hw, ci, co, k, 1), 'conv2d')
+        filter_ = k * k * ci * co * 2
+        assert bytes_ > filter_ if split else bytes_ == filter_, hk.describe(plan)
+        hk.lib().pml_hip_plan_free(plan)
+    # a data gradient: the flipped filter and the padded gradient of 70 channels; the columns of a stride of 2
+    plan, bytes_ = held(conv(hk.BF16, 2, 14, 64, 70, 3, 1), which=0)
+    assert bytes_ >= 9 * 64 * 72 * 2 + 2 * 14 * 14 * 72 * 2
+    hk.lib().pml_hip_plan_free(plan)
+    plan, bytes_ = held(conv(hk.F32, 2, 14, 64, 70, 3, 2), which=0)
+    assert bytes_ >= 2 * 7 * 7 * 9 * 64 * 4
+    hk.lib().pml_hip_plan_free(plan)
