@@ -313,11 +313,11 @@ hipError_t launch(const IgemmArgs& a, hipStream_t s) {
 #define PML_CAT_(a, b) a##b
 #define PML_CAT(a, b) PML_CAT_(a, b)
 
-// 32 x 32 tiles that are more than one round of the chip give way to 32 x 64: three quarters of the operand bytes per
+// 32 x 32 tiles that are more than one on each CU give way to 32 x 64: three quarters of the operand bytes per
 // result (784 x 512, K = 256: fp32 9.3 -> 8.5 us, bf16 6.2 -> 5.4, int8 4.8 -> 4.5; 1000 x 300, K = 2000 int8 7.6 -> 6.5).
 template <bool CONV>
 static hipError_t launch_large(const IgemmArgs& a, hipStream_t s) {
-  return ((a.M + 31) / 32) * ((a.N + 31) / 32) > 256 ? launch<PML_KIND, CONV, 2, 4, false>(a, s) : launch<PML_KIND, CONV, 2, 2, false>(a, s);
+  return ((a.M + 31) / 32) * ((a.N + 31) / 32) > a.n_cus ? launch<PML_KIND, CONV, 2, 4, false>(a, s) : launch<PML_KIND, CONV, 2, 2, false>(a, s);
 }
 
 // cfg: TILE_16x16_W8 or TILE_32x32_W8 (with a [K][N] right-hand side: 16 x 64 and 32 x 64 results)

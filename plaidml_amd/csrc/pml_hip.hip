@@ -32,6 +32,8 @@ int check(hipError_t e, const char* what) {
   return 1;
 }
 
+int device_cus();
+
 // Device memory that a caller can do without: nullptr when there is none.
 void* alloc_or_null(size_t bytes) {
   void* p = nullptr;
@@ -167,7 +169,7 @@ const char* const kTileShort[PML_HIP_TILE_COUNT_] = {"64x64", "128x64", "128x128
 
 // One of the direct tiles (direct.hip) where it beats the LDS kernels, or -1.  Both sides are priced in microseconds, from
 // measurements of 27 matrix products and 18 convolutions per element kind (one row to 3136, K of 64 to 4608; back to back
-// in a recorded graph): a direct kernel takes 2.6 plus, per round of one tile on each of 256 CUs (fp32 and 32 x 64: whole
+// in a recorded graph): a direct kernel takes 2.6 plus, per round of one tile on each CU (fp32 and 32 x 64: whole
 // rounds), 0.8 (fp32 32 x 32: 1.9; 32 x 64, which replaces 32 x 32 beyond one round: bf16 1.6, int8 1.0, fp32 2.3) and its
 // operand bytes at 40 KB a microsecond and CU (32 x 64: bf16 50, int8 60, fp32 32).  An LDS kernel takes 4.2 plus its chain
 // of 128-byte slabs (0.23 each, int8 0.28, fp32 0.58), or -- K split over workgroups -- 5.2 (fp32 5.6) plus 0.4 per KB of K
@@ -191,12 +193,13 @@ int direct_tile_of(int64_t m, int64_t n, int64_t k_bytes, int kind, int64_t kn_l
   const double kb = (double)k_bytes;
   const int es = kind == KIND_BF16 ? 2 : (kind == KIND_I8 ? 1 : 4);
   const bool kn = kn_ldb > 0, f32 = kind == KIND_F32;
-  const bool wide_tiles = !kn && tiles(32, 32) > 256;  // (32 x 64 in the place of 32 x 32)
+  const int n_cus = device_cus();
+  const bool wide_tiles = !kn && tiles(32, 32) > n_cus;  // (32 x 64 in the place of 32 x 32)
   const double rate = !kn ? 40e3 : f32 ? 45e3 : (kind == KIND_I8 && kn_ldb % 64 != 0) ? 36e3 : 60e3;
   auto direct_us = [&](int64_t side) {
     const bool w = wide_tiles && side == 32;
     const int64_t wide = kn || w ? 64 : side;
-    double rounds = std::max(1.0, (double)tiles(side, wide) / 256);
+    double rounds = std::max(1.0, (double)tiles(side, wide) / n_cus);
     if ((f32 && !kn) || w) rounds = std::ceil(rounds);
     const double start = w ? (f32 ? 2.3 : kind == KIND_I8 ? 1.0 : 1.6) : f32 && !kn && side == 32 ? 1.9 : 0.8;
     const double r = w ? (f32 ? 32e3 : kind == KIND_I8 ? 60e3 : 50e3) : rate;
@@ -207,7 +210,7 @@ int direct_tile_of(int64_t m, int64_t n, int64_t k_bytes, int kind, int64_t kn_l
   bool needs_bt = kind == KIND_BF16 || n % (16 / es) != 0 || kn_ldb % 16 != 0;
   if (can_split && tiles(64, 64) <= 64 && k_bytes >= 2048) {
     int splits = 1, per = 0;
-    igemm_split_plan(m, n, slabs, 256, &splits, &per);
+    igemm_split_plan(m, n, slabs, n_cus, &splits, &per);
     if (splits >= 2) {
       lds_us = (f32 ? 5.6 : 5.2) + kb / 2500 + 8.0 * splits * (double)m * (double)n / 3e6;
       needs_bt = true;
@@ -874,6 +877,8 @@ int64_t pml_hip_gemm_dispatch(const pml_hip_gemm_desc* d) {
                 kind == KIND_F32 ? "f32_32x32x2" : kind == KIND_BF16 ? "f32_32x32x16_bf16" : kind == KIND_I8 ? "i32_32x32x32_i8" : "3 x f32_32x32x16_bf16 (fp32 split into bf16 head + remainder)");
   p->text = buf;
   if (p->direct.rows >= 0) p->text += std::string(", with rows of K at hand tile=") + tile_name(p->direct.rows);
+  if (p->direct.given >= 0)
+    p->text += std::string(", with B as it lies tile=") + (p->direct.given == TILE_16x16_W8 ? "16x64" : "32x64") + " (8 wavefronts sharing K)";
   if (d->k2 > 0) p->text += " + second product k2=" + std::to_string(d->k2) + (d->a2_stride > 0 ? " over pixel rows of stride " + std::to_string(d->a2_stride) : "");
   return (int64_t)(intptr_t)p;
 }

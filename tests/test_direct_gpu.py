@@ -180,6 +180,7 @@ def test_plans_hold_what_their_invokes_read(kind, es):
     plan, bytes_ = held(d)
     copy = N * d.k * es
     assert bytes_ == copy if kind == 'f32' else bytes_ > copy
+    assert 'with B as it lies tile=' in hk.describe(plan)
     B = hk.DeviceBuffer(copy)
     hk.check(L.pml_hip_fill_u32(B.ptr, 0, copy // 4, None))
     hk.check(L.pml_hip_gemm_pack_b(plan, B.ptr, None))
