@@ -142,20 +142,6 @@ def test_split_over_workgroups_by_name(kind, M, N, K, monkeypatch):
     check(E.bf16_from_bits(got) if kind == 'bf16' else got, want, kind, K)
 
 
-@pytest.mark.parametrize('M,N,K', [(49, 512, 2048), (196, 256, 2048), (100, 130, 4096), (1, 1000, 2048), (300, 72, 2064)])
-def test_gemm_k_split_where_direct_tiles_would_be_taken(M, N, K, monkeypatch, capsys):
-    """The K split over workgroups by name: most of these shapes take a direct tile otherwise."""
-    monkeypatch.setitem(T.FORCED, 'flags', hk.flag_tile('64x64ks'))
-    T.test_gemm_k_split_over_workgroups(M, N, K, capsys)
-
-
-@pytest.mark.parametrize('kind', ['bf16', 'f32'])
-@pytest.mark.parametrize('shape,k,co,stride', [((1, 7, 7, 512), 3, 512, 1), ((1, 14, 14, 256), 3, 256, 2), ((2, 9, 11, 96), 5, 40, 1)])
-def test_conv_k_split_where_direct_tiles_would_be_taken(kind, shape, k, co, stride, monkeypatch, capsys):
-    monkeypatch.setitem(T.FORCED, 'flags', hk.flag_tile('64x64ks'))
-    T.test_conv_k_split_over_workgroups(kind, shape, k, co, stride, capsys)
-
-
 def held(desc, family='gemm', which=None):
     L = hk.lib()
     plan = L.pml_hip_conv2d_grad_dispatch(ctypes.byref(desc), which) if which is not None else getattr(L, 'pml_hip_%s_dispatch' % family)(ctypes.byref(desc))
