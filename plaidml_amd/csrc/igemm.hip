@@ -792,7 +792,8 @@ hipError_t launch_splitk(const IgemmArgs& a, hipStream_t s) {
 
 template <int KIND, int BM, int BN, int WAVES_M, bool CONV, int NT = kThreads, int STAGES = 0, int WAVES_K = 1, int SLAB = 128>
 hipError_t launch_cfg(const IgemmArgs& a, hipStream_t s) {
-  if constexpr ((KIND == KIND_F32 || KIND == KIND_F32X3 || KIND == KIND_I8) && !CONV && SLAB == 128 && (BN & (BN - 1)) == 0) {
+  if constexpr ((KIND == KIND_F32 || KIND == KIND_F32X3 || KIND == KIND_I8) && !CONV && SLAB == 128 && (BN & (BN - 1)) == 0 &&
+                !(KIND == KIND_I8 && BM == 256 && BN == 256)) {  // (given.hip)
     if (a.b_kn) {
       const int64_t tiles_m = (a.M + BM - 1) / BM, tiles_n = (a.N + BN - 1) / BN;
       const int64_t tiles = tiles_m * tiles_n;
@@ -962,6 +963,7 @@ hipError_t igemm_launch(int kind, int cfg, bool conv, const IgemmArgs& a, hipStr
   const int64_t a_bytes = conv ? (int64_t)a.NB * a.H * a.W * (a.pix_pitch ? a.pix_pitch : a.CI * es) + 256 : a.M * a.lda * es;
   const int64_t b_bytes = (a.b_kn ? a.K : a.N) * a.ldbt * es;
   if (a_bytes >= ((int64_t)1 << 31) || b_bytes >= ((int64_t)1 << 31) || (conv && a.M >= ((int64_t)1 << 31))) return hipErrorInvalidValue;
+  if (cfg == TILE_256x256_W8 && a.b_kn && (kind == KIND_BF16 || kind == KIND_I8)) return given_launch(kind, a, s);
   if (cfg == TILE_16x16_W8 || cfg == TILE_32x32_W8) {
     if (!conv || !a.pix_pitch) {
       switch (kind) {

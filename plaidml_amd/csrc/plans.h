@@ -208,6 +208,8 @@ struct IgemmArgs {
 };
 
 hipError_t igemm_launch(int kind, int cfg, bool conv, const IgemmArgs& a, hipStream_t s);
+// TILE_256x256_W8 of a bf16 or int8 GEMM whose right-hand side is read as it lies (a.b_kn): given.hip
+hipError_t given_launch(int kind, const IgemmArgs& a, hipStream_t s);
 // How TILE_64x64_KSPLIT shares the K loop out: slabs of 128 bytes of K in all, and for a device of n_cus compute units
 // the number of splits (1: not worth splitting) with the slabs each takes -- about one workgroup per CU, at least two
 // slabs per split, at most 16 splits.

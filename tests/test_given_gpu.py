@@ -1,0 +1,108 @@
+"""The 256 x 256 tile that reads a [K][N] right-hand side as it lies, through registers (csrc/given.hip).  Small whole numbers
+make every sum exact, so every tail is compared value for value with numpy, where tiles, slabs and chunks of K end raggedly."""
+import ctypes
+
+import numpy as np
+import pytest
+
+import test_kernels_gpu as T
+from oracle import tile_oracle as E
+from plaidml_amd import hipkernels as hk
+
+pytestmark = pytest.mark.gpu
+
+# one row, one chunk of K; four columns; rows, columns and K just below, at and above a tile / a slab / the ring's depth;
+# N that ends inside a lane's sixteen columns; more tiles than CUs
+SIZES = [(1, 4, 16), (255, 260, 48), (256, 256, 128), (257, 252, 144), (300, 64, 512), (129, 516, 640), (600, 1040, 1168), (4200, 4112, 80)]
+
+
+@pytest.fixture(autouse=True)
+def _tile(monkeypatch):
+    hk.init(0)
+    monkeypatch.setitem(T.FORCED, 'flags', hk.flag_tile('256x256w8'))
+
+
+def whole(rng, shape):
+    return rng.integers(-4, 5, shape).astype(np.float32)
+
+
+@pytest.mark.parametrize('M,N,K', SIZES)
+def test_bf16(M, N, K):
+    rng = np.random.default_rng(M + N + K)
+    A, B = whole(rng, (M, K)), whole(rng, (K, N))
+    S = A @ B  # at most 16 K: exact
+    bias, scale, shift, res = whole(rng, N), whole(rng, N), whole(rng, N), whole(rng, (M, N))
+    r = E.round_bf16
+    relu = (hk.EPI_RELU, hk.BF16, 0, 0, 0.0)
+    kw = dict(init=T.bf16(bias), init_strides=(0, 1), init_dt=hk.BF16, invokes=2)
+
+    def run(tail, operands=()):
+        return E.bf16_from_bits(T.run_gemm(T.bf16(A), T.bf16(B), hk.BF16, hk.BF16, tail=tail, operands=[T.bf16(o) for o in operands], **kw))
+
+    np.testing.assert_array_equal(run(hk.make_tail(ops=[relu])), r(np.maximum(S + bias, 0)))
+    add = hk.make_tail(ops=[(hk.EPI_ADD, hk.BF16, hk.OPND_TENSOR, 0, 0.0), relu], operands=[(hk.BF16, N, 1)])
+    np.testing.assert_array_equal(run(add, [res]), r(np.maximum(r(S + bias) + res, 0)))
+    fold = hk.make_tail(ops=[(hk.EPI_MUL, hk.BF16, hk.OPND_TENSOR, 0, 0.0), (hk.EPI_ADD, hk.BF16, hk.OPND_TENSOR, 1, 0.0), relu],
+                        operands=[(hk.BF16, 0, 1), (hk.BF16, 0, 1)])
+    np.testing.assert_array_equal(run(fold, [scale, shift]), r(np.maximum(r(r(S + bias) * scale) + shift, 0)))
+    steps = hk.make_tail(ops=[(hk.EPI_NEG, hk.BF16, 0, 0, 0.0), relu])  # (through LDS and the common tail)
+    np.testing.assert_array_equal(run(steps), r(np.maximum(-r(S + bias), 0)))
+
+
+def requant(n, with_sums):
+    store = [(hk.EPI_STORE, hk.I32, 0, 0, 0.0)] if with_sums else []
+    return hk.make_tail(ops=store + [(hk.EPI_CAST, hk.F32, 0, 0, 0.0), (hk.EPI_MUL, hk.F32, hk.OPND_TENSOR, 0, 0.0),
+                                     (hk.EPI_MAX_GT, hk.F32, hk.OPND_IMM, 0, -127.0), (hk.EPI_MIN, hk.F32, hk.OPND_IMM, 0, 127.0),
+                                     (hk.EPI_ROUND, hk.F32, 0, 0, 0.0), (hk.EPI_CAST, hk.I8, 0, 0, 0.0)], operands=[(hk.F32, 0, 1)])
+
+
+@pytest.mark.parametrize('M,N,K', SIZES)
+def test_int8(M, N, K):
+    rng = np.random.default_rng(M + N + K)
+    A, B = rng.integers(-127, 128, (M, K), dtype=np.int8), rng.integers(-127, 128, (K, N), dtype=np.int8)
+    S = (A.astype(np.float64) @ B.astype(np.float64)).astype(np.int32)  # exact in float64
+    np.testing.assert_array_equal(T.run_gemm(A, B, hk.I8, hk.I32, invokes=2), S)
+    start = rng.integers(-1000, 1000, N, dtype=np.int32)
+    scale = rng.uniform(0.5, 2, N).astype(np.float32) / np.float32(60 * np.sqrt(K))
+    v = np.clip((S + start).astype(np.float32) * scale, -127, 127)
+    want = np.trunc(v + np.copysign(np.float32(0.5), v)).astype(np.int8)
+    kw = dict(init=start, init_strides=(0, 1), init_dt=hk.I32, operands=[scale], c_dt=hk.I8)
+    np.testing.assert_array_equal(T.run_gemm(A, B, hk.I8, hk.I32, tail=requant(N, False), **kw), want)
+    got, sums = T.run_gemm(A, B, hk.I8, hk.I32, tail=requant(N, True), extra_out=np.int32, **kw)
+    np.testing.assert_array_equal(got, want)
+    np.testing.assert_array_equal(sums, S + start)
+
+
+@pytest.mark.parametrize('kind', ['bf16', 'i8'])
+@pytest.mark.parametrize('n,ldb', [(260, 264), (260, 262), (258, 258)])
+def test_packed_and_given_in_turn(kind, n, ldb):
+    """A right-hand side packed once, ones that arrive with the call and are read as they lie, and ones that have to be turned
+    (rows that are no multiple of four elements), which take the packed copy's place: each call multiplies what it was given."""
+    M, K = 270, 272
+    rng = np.random.default_rng(ldb)
+    dt, out = (hk.BF16, hk.F32) if kind == 'bf16' else (hk.I8, hk.I32)
+    A = whole(rng, (M, K))
+    Bs = [whole(rng, (K, ldb)) for _ in range(2)]
+    code = T.bf16 if kind == 'bf16' else lambda x: x.astype(np.int8)
+    d = hk.GemmDesc()
+    d.in_dtype, d.out_dtype, d.c_dtype, d.flags = dt, out, out, T.FORCED['flags']
+    d.m, d.n, d.k, d.lda, d.ldb, d.ldc = M, n, K, K, ldb, n
+    plan = hk.lib().pml_hip_gemm_dispatch(ctypes.byref(d))
+    assert plan, hk.lib().pml_hip_last_error()
+    dA, dC = hk.DeviceBuffer.from_numpy(code(A)), hk.DeviceBuffer(M * n * 4)
+    dB = [hk.DeviceBuffer.from_numpy(code(B)) for B in Bs]
+    none = hk.ptr_array([])
+
+    def call(b):
+        hk.check(hk.lib().pml_hip_gemm_invoke(plan, dA.ptr, b, dC.ptr, None, none, none, None))
+        hk.check(hk.lib().pml_hip_stream_sync(None))
+        return dC.to_numpy(np.float32 if kind == 'bf16' else np.int32, (M, n)).astype(np.float32)
+
+    want = [A @ B[:, :n] for B in Bs]
+    np.testing.assert_array_equal(call(dB[0].ptr), want[0])
+    hk.check(hk.lib().pml_hip_gemm_pack_b(plan, dB[1].ptr, None))
+    np.testing.assert_array_equal(call(None), want[1])
+    np.testing.assert_array_equal(call(dB[0].ptr), want[0])
+    hk.check(hk.lib().pml_hip_gemm_pack_b(plan, dB[1].ptr, None))
+    np.testing.assert_array_equal(call(None), want[1])
+    hk.lib().pml_hip_plan_free(plan)
