@@ -78,6 +78,7 @@ __device__ __forceinline__ void turn(const int (&raw)[16], i32x4_t (&frag)[4]) {
 // MB x NB blocks of 16 x 16 results per workgroup.
 template <int KIND, bool CONV, int MB, int NB, bool KN>
 __global__ __launch_bounds__(64 * kWaves, 4) void direct_kernel(IgemmArgs p_by_value) {
+  warm_arguments<sizeof(IgemmArgs)>();
   // (read where the dispatcher put it: indexing a by-value copy would move the copy to scratch memory)
   const IgemmArgs& p = *(const IgemmArgs*)(const __attribute__((address_space(4))) void*)__builtin_amdgcn_kernarg_segment_ptr();
   static_assert(!KN || (NB == 4 && !CONV), "a [K][N] right-hand side is taken four columns per lane");

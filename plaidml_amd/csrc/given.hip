@@ -238,6 +238,7 @@ __device__ __forceinline__ void given_tail_requant(const IgemmArgs& p, const i32
 
 template <int KIND>
 __global__ __launch_bounds__(kThreads, 2) void given_kernel(IgemmArgs p_by_value) {
+  warm_arguments<sizeof(IgemmArgs)>();
   // (read where the dispatcher put it: indexing a by-value copy would move the copy to scratch memory)
   const IgemmArgs& p = *(const IgemmArgs*)(const __attribute__((address_space(4))) void*)__builtin_amdgcn_kernarg_segment_ptr();
   typedef Given<KIND> G;

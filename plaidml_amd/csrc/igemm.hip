@@ -102,6 +102,7 @@ constexpr int igemm_waves_per_simd() {
 template <int KIND, int BM, int BN, int WAVES_M, bool CONV, int NT = kThreads, int STAGES = 0, int WAVES_K = 1, int SLAB = 128,
           bool BKN = false, bool SPLITK = false>
 __global__ __launch_bounds__(NT, (igemm_waves_per_simd<BM, BN, STAGES, SLAB, NT>())) void igemm_kernel(IgemmArgs p_by_value) {
+  warm_arguments<sizeof(IgemmArgs)>();
   // The argument block is read where the dispatcher put it (the kernel-argument segment, scalar loads),
   // through a reference: taking the by-value parameter's address instead makes the compiler copy all of
   // it to scratch memory as soon as one field is indexed with a run-time value.
@@ -739,6 +740,7 @@ __global__ __launch_bounds__(256) void transpose_words_kernel(const uint32_t* __
 // accesses of 8 bytes, about 20 us; against 12-13 us for the two launches.)
 template <int KIND>
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(IgemmArgs p_by_value, int strips_n) {
+  warm_arguments<sizeof(IgemmArgs)>();
   const IgemmArgs& p = *(const IgemmArgs*)(const __attribute__((address_space(4))) void*)__builtin_amdgcn_kernarg_segment_ptr();
   typedef typename Acc<KIND>::scalar accs_t;
   typedef accs_t acc4_t __attribute__((ext_vector_type(4)));

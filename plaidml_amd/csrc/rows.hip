@@ -24,6 +24,7 @@ constexpr size_t kRowsLds = 158 * 1024;  // dynamic LDS of a workgroup at most (
 // launches, 23 us in one (events around both included; the traffic takes 6.5 us at the rate of a large copy).
 template <bool BF, int LANES, int U>
 __global__ __launch_bounds__(256) void rows_program_kernel(RowsProgramArgs p_by_value) {
+  warm_arguments<sizeof(RowsProgramArgs)>();
   const RowsProgramArgs& p = *(const RowsProgramArgs*)(const __attribute__((address_space(4))) void*)__builtin_amdgcn_kernarg_segment_ptr();
   const pml_hip_rows_desc& d = p.d;
   constexpr int GROUPS = 256 / LANES;  // rows per workgroup
