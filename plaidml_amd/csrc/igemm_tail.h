@@ -353,6 +353,61 @@ __device__ __forceinline__ void direct_tail_bf16(const IgemmArgs& p, f32x16_t (&
   }
 }
 
+// Four neighbouring results of tail_mode 1 or 2 -- the sums with their start value, res the residual tensor's bits -- finished
+// and stored at element `at` of C.
+template <int KIND>
+__device__ __forceinline__ void store_quad(void* C, int64_t at, int out_dtype, const typename Acc<KIND>::scalar (&v4)[4], const i32x4_t& res,
+                                           bool residual, bool relu) {
+  if (KIND == KIND_I8) {
+    i32x4_t w;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int v = (int)((unsigned)(int)v4[q] + (unsigned)res[q]);
+      w[q] = (relu && v < 0) ? 0 : v;
+    }
+    *(i32x4_t*)((int*)C + at) = w;
+  } else if (out_dtype == PML_HIP_BF16) {
+    // v_cvt_pk_bf16_f32 rounds to nearest even.  relu is applied to the fp32 value just before
+    // the last rounding (a result in (-2^-134, 0) stores +0 where the definition gives -0).
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    float v[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) v[q] = (float)v4[q];
+    if (residual) {
+      // the contraction result is rounded first, then the bf16 addition rounds again
+      const bf16x2 r01 = __builtin_convertvector(f32x2{v[0], v[1]}, bf16x2);
+      const bf16x2 r23 = __builtin_convertvector(f32x2{v[2], v[3]}, bf16x2);
+      uint32_t w01, w23;
+      __builtin_memcpy(&w01, &r01, 4);
+      __builtin_memcpy(&w23, &r23, 4);
+      const uint32_t x01 = (uint32_t)res[0], x23 = (uint32_t)res[1];
+      v[0] = __uint_as_float(w01 << 16) + __uint_as_float(x01 << 16);
+      v[1] = __uint_as_float(w01 & 0xffff0000u) + __uint_as_float(x01 & 0xffff0000u);
+      v[2] = __uint_as_float(w23 << 16) + __uint_as_float(x23 << 16);
+      v[3] = __uint_as_float(w23 & 0xffff0000u) + __uint_as_float(x23 & 0xffff0000u);
+    }
+    if (relu) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) v[q] = v[q] < 0.f ? 0.f : v[q];
+    }
+    const bf16x2 h01 = __builtin_convertvector(f32x2{v[0], v[1]}, bf16x2);
+    const bf16x2 h23 = __builtin_convertvector(f32x2{v[2], v[3]}, bf16x2);
+    uint32_t o01, o23;
+    __builtin_memcpy(&o01, &h01, 4);
+    __builtin_memcpy(&o23, &h23, 4);
+    *(uint2*)((uint16_t*)C + at) = make_uint2(o01, o23);
+  } else {
+    f32x4_t w;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const float v = residual ? (float)v4[q] + __int_as_float(res[q]) : (float)v4[q];
+      w[q] = (relu && v < 0.f) ? 0.f : v;
+    }
+    *(f32x4_t*)((float*)C + at) = w;
+  }
+}
+
 // Tail over an accumulator tile held in LDS as ctile[BM][BN + 4] (row-major):
 // adds the initial value, runs the fused elementwise chain once per element and
 // stores contiguous 8/16-byte pieces.  A thread owns 4 consecutive columns; rows
@@ -458,54 +513,7 @@ __device__ __forceinline__ void tile_tail(const IgemmArgs& p, const typename Acc
             v4[q] += KIND == KIND_I8 ? (accs_t)b.i : (accs_t)b.f;
           }
         }
-        if (KIND == KIND_I8) {
-          i32x4_t w;
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const int v = (int)((unsigned)(int)v4[q] + (unsigned)res[c][q]);
-            w[q] = (p.tail_relu && v < 0) ? 0 : v;
-          }
-          *(i32x4_t*)((int*)p.C + m * p.ldc + n) = w;
-        } else if (p.out_dtype == PML_HIP_BF16) {
-          // v_cvt_pk_bf16_f32 rounds to nearest even.  relu is applied to the fp32 value just before
-          // the last rounding (a result in (-2^-134, 0) stores +0 where the definition gives -0).
-          typedef float f32x2 __attribute__((ext_vector_type(2)));
-          typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-          float v[4];
-#pragma unroll
-          for (int q = 0; q < 4; ++q) v[q] = (float)v4[q];
-          if (residual) {
-            // the contraction result is rounded first, then the bf16 addition rounds again
-            const bf16x2 r01 = __builtin_convertvector(f32x2{v[0], v[1]}, bf16x2);
-            const bf16x2 r23 = __builtin_convertvector(f32x2{v[2], v[3]}, bf16x2);
-            uint32_t w01, w23;
-            __builtin_memcpy(&w01, &r01, 4);
-            __builtin_memcpy(&w23, &r23, 4);
-            const uint32_t x01 = (uint32_t)res[c][0], x23 = (uint32_t)res[c][1];
-            v[0] = __uint_as_float(w01 << 16) + __uint_as_float(x01 << 16);
-            v[1] = __uint_as_float(w01 & 0xffff0000u) + __uint_as_float(x01 & 0xffff0000u);
-            v[2] = __uint_as_float(w23 << 16) + __uint_as_float(x23 << 16);
-            v[3] = __uint_as_float(w23 & 0xffff0000u) + __uint_as_float(x23 & 0xffff0000u);
-          }
-          if (p.tail_relu) {
-#pragma unroll
-            for (int q = 0; q < 4; ++q) v[q] = v[q] < 0.f ? 0.f : v[q];
-          }
-          const bf16x2 h01 = __builtin_convertvector(f32x2{v[0], v[1]}, bf16x2);
-          const bf16x2 h23 = __builtin_convertvector(f32x2{v[2], v[3]}, bf16x2);
-          uint32_t o01, o23;
-          __builtin_memcpy(&o01, &h01, 4);
-          __builtin_memcpy(&o23, &h23, 4);
-          *(uint2*)((uint16_t*)p.C + m * p.ldc + n) = make_uint2(o01, o23);
-        } else {
-          f32x4_t w;
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const float v = residual ? (float)v4[q] + __int_as_float(res[c][q]) : (float)v4[q];
-            w[q] = (p.tail_relu && v < 0.f) ? 0.f : v;
-          }
-          *(f32x4_t*)((float*)p.C + m * p.ldc + n) = w;
-        }
+        store_quad<KIND>(p.C, m * p.ldc + n, p.out_dtype, v4, res[c], residual, p.tail_relu != 0);
       }
     }
     return;

@@ -198,3 +198,37 @@ def test_convolution_plans_hold_what_their_invokes_read():
     plan, bytes_ = held(conv(hk.F32, 2, 14, 64, 70, 3, 2), which=0)
     assert bytes_ >= 2 * 7 * 7 * 9 * 64 * 4
     hk.lib().pml_hip_plan_free(plan)
+
+
+@pytest.mark.parametrize('kind,out', [('f32', 'f32'), ('bf16', 'bf16'), ('bf16', 'f32'), ('i8', 'i32')])
+@pytest.mark.parametrize('tile', TILES)
+@pytest.mark.parametrize('M,N,ldr,shift', [(33, 72, 72, 0), (17, 20, 28, 0), (1, 4, 4, 0), (33, 72, 72, 1), (17, 18, 18, 0), (40, 64, 70, 0)])
+def test_tail_operands_read_ahead(kind, out, tile, M, N, ldr, shift):
+    """A bias and a residual tensor, read before the sums exist where they are whole quads -- last rows and columns, rows of
+    the residual longer than N -- and after them otherwise (a bias off its alignment, N or the residual's rows no multiple
+    of four).  Whole numbers: every result is exact."""
+    K = 80
+    rng = np.random.default_rng(M + N + shift)
+    A, B = rng.integers(-4, 5, (M, K)).astype(np.float32), rng.integers(-4, 5, (K, N)).astype(np.float32)
+    bias, res = rng.integers(-9, 10, N + shift).astype(np.float32), rng.integers(-9, 10, (M, ldr)).astype(np.float32)
+    dts = {'f32': (hk.F32, lambda a: a, np.float32), 'bf16': (hk.BF16, T.bf16, np.uint16), 'i8': (hk.I8, lambda a: a.astype(np.int8), np.int8),
+           'i32': (hk.I32, lambda a: a.astype(np.int32), np.int32)}
+    (dt, cast, _), (odt, ocast, onp) = dts[kind], dts[out]
+    d = hk.GemmDesc()
+    d.in_dtype, d.out_dtype, d.c_dtype, d.flags = dt, odt, odt, hk.flag_tile(tile)
+    d.m, d.n, d.k, d.lda, d.ldb, d.ldc = M, N, K, K, N, N
+    d.init_kind, d.init_dtype, d.init_col_stride = 1, odt, 1
+    d.tail = hk.make_tail(ops=[(hk.EPI_ADD, odt, hk.OPND_TENSOR, 0, 0.0), (hk.EPI_RELU, odt, 0, 0, 0.0)], operands=[(odt, ldr, 1)])
+    plan = hk.lib().pml_hip_gemm_dispatch(ctypes.byref(d))
+    assert plan, hk.lib().pml_hip_last_error()
+    dA, dB, dI, dR = (hk.DeviceBuffer.from_numpy(x) for x in (cast(A), cast(B), ocast(bias), ocast(res)))
+    es = np.dtype(onp).itemsize
+    dC = hk.DeviceBuffer(M * N * es)
+    hk.check(hk.lib().pml_hip_gemm_invoke(plan, dA.ptr, dB.ptr, dC.ptr, (dI.ptr.value if hasattr(dI.ptr, 'value') else dI.ptr) + shift * es,
+                                          hk.ptr_array([dR.ptr]), hk.ptr_array([]), None))
+    hk.check(hk.lib().pml_hip_stream_sync(None))
+    got = dC.to_numpy(onp, (M, N))
+    hk.lib().pml_hip_plan_free(plan)
+    r = E.round_bf16 if out == 'bf16' else lambda a: a
+    want = np.maximum(r(r(A @ B + bias[shift:]) + res[:, :N]), 0)
+    np.testing.assert_array_equal(E.bf16_from_bits(got) if out == 'bf16' else got, want)
