@@ -77,6 +77,11 @@ int pml_hip_memcpy_d2h_async(void* dst, const void* src, size_t nbytes, pml_hip_
 /* n copies between device and page-locked host memory (any direction) by one kernel: for a few hundred kilobytes the
  * copy engines' set-up and hand-over to the compute queue cost more than the transfer. */
 int pml_hip_copy_spans(int n, void* const* dst, const void* const* src, const size_t* nbytes, pml_hip_stream s);
+/* The same, and the device's clock (pml_hip_clock_khz ticks a millisecond) to *stamp, in page-locked or device memory: as
+ * the copies begin, or, with `after`, when they are made (to the microsecond).  n = 0: the clock alone. */
+int pml_hip_copy_spans_stamped(int n, void* const* dst, const void* const* src, const size_t* nbytes, uint64_t* stamp, int after,
+                               pml_hip_stream s);
+int pml_hip_clock_khz(void); /* 0 on failure */
 /* Fills with a 32-bit pattern using a kernel (safe to capture into a graph). */
 int pml_hip_fill_u32(void* dptr, uint32_t pattern, size_t n_words, pml_hip_stream s);
 

@@ -711,6 +711,8 @@ __global__ __launch_bounds__(256) void copy_spans_kernel(SpanArgs a) {
   unsigned char* dst = (unsigned char*)a.dst[blockIdx.y];
   const size_t n_vec = a.bytes[blockIdx.y] / 16, stride = (size_t)gridDim.x * 256;
   const size_t first = (size_t)blockIdx.x * 256 + threadIdx.x;
+  const bool stamps = a.stamp != nullptr && first == 0 && blockIdx.y == 0;
+  if (stamps && !a.stamp_after) *a.stamp = wall_clock64();
   constexpr int U = 4;
   for (size_t g0 = first; g0 < n_vec; g0 += U * stride) {
     i32x4_t v[U];
@@ -722,6 +724,7 @@ __global__ __launch_bounds__(256) void copy_spans_kernel(SpanArgs a) {
       if (g0 + u * stride < n_vec) __builtin_memcpy(dst + (g0 + u * stride) * 16, &v[u], 16);
   }
   for (size_t i = n_vec * 16 + first; i < a.bytes[blockIdx.y]; i += stride) dst[i] = src[i];
+  if (stamps && a.stamp_after) *a.stamp = wall_clock64();
 }
 
 inline unsigned grid_for(int64_t work_items) {
@@ -1102,12 +1105,12 @@ hipError_t softmax_launch(const pml_hip_softmax_desc& d, const void* x, void* y,
 }
 
 hipError_t copy_spans_launch(const SpanArgs& a, hipStream_t s) {
-  if (a.n <= 0) return hipSuccess;
+  if (a.n <= 0 && !a.stamp) return hipSuccess;
   size_t most = 0;
   for (int i = 0; i < a.n; ++i) most = most < a.bytes[i] ? a.bytes[i] : most;
   size_t blocks = (most / 16 + 4 * 256 - 1) / (4 * 256);
   blocks = blocks < 1 ? 1 : blocks > 64 ? 64 : blocks;
-  hipLaunchKernelGGL(copy_spans_kernel, dim3((unsigned)blocks, (unsigned)a.n), dim3(256), 0, s, a);
+  hipLaunchKernelGGL(copy_spans_kernel, dim3((unsigned)blocks, (unsigned)(a.n > 0 ? a.n : 1)), dim3(256), 0, s, a);
   return hipGetLastError();
 }
 

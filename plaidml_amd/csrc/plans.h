@@ -276,7 +276,8 @@ struct SpanArgs {
   void* dst[kMaxSpans];
   const void* src[kMaxSpans];
   size_t bytes[kMaxSpans];
-  int n;
+  int n, stamp_after;
+  uint64_t* stamp;  // the device's clock goes here, before or after the copies; or null
 };
 hipError_t copy_spans_launch(const SpanArgs& a, hipStream_t s);
 hipError_t fill_u32_launch(void* p, uint32_t pattern, size_t n_words, hipStream_t s);

@@ -679,8 +679,12 @@ int pml_hip_memcpy_d2h_async(void* dst, const void* src, size_t nbytes, pml_hip_
   return nbytes ? check(hipMemcpyAsync(dst, src, nbytes, hipMemcpyDeviceToHost, (hipStream_t)s), "hipMemcpyAsync(d2h)") : 0;
 }
 int pml_hip_copy_spans(int n, void* const* dst, const void* const* src, const size_t* nbytes, pml_hip_stream s) {
+  return pml_hip_copy_spans_stamped(n, dst, src, nbytes, nullptr, 0, s);
+}
+int pml_hip_copy_spans_stamped(int n, void* const* dst, const void* const* src, const size_t* nbytes, uint64_t* stamp, int after,
+                               pml_hip_stream s) {
   if (n < 0 || (n > 0 && (!dst || !src || !nbytes))) return fail("copy_spans: bad argument");
-  for (int i = 0; i < n; i += kMaxSpans) {
+  for (int i = 0; i == 0 || i < n; i += kMaxSpans) {
     SpanArgs a;
     std::memset(&a, 0, sizeof a);
     for (int j = i; j < n && j < i + kMaxSpans; ++j) {
@@ -690,9 +694,16 @@ int pml_hip_copy_spans(int n, void* const* dst, const void* const* src, const si
       a.src[a.n] = src[j];
       a.bytes[a.n++] = nbytes[j];
     }
+    if (after ? i + kMaxSpans >= n : i == 0) a.stamp = stamp;
+    a.stamp_after = after;
     if (check(copy_spans_launch(a, (hipStream_t)s), "copy_spans_launch")) return 1;
   }
   return 0;
+}
+int pml_hip_clock_khz(void) {
+  int dev = 0, khz = 0;
+  if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev) != hipSuccess) return 0;
+  return khz;
 }
 int pml_hip_fill_u32(void* dptr, uint32_t pattern, size_t n_words, pml_hip_stream s) {
   return check(fill_u32_launch(dptr, pattern, n_words, (hipStream_t)s), "fill");

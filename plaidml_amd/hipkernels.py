@@ -54,7 +54,7 @@ EXPORTS = [
     'pml_hip_conv2d_dispatch', 'pml_hip_conv2d_invoke', 'pml_hip_dwconv2d_dispatch', 'pml_hip_dwconv2d_invoke',
     'pml_hip_pool2d_dispatch', 'pml_hip_pool2d_invoke', 'pml_hip_eltwise_dispatch', 'pml_hip_eltwise_invoke',
     'pml_hip_select', 'pml_hip_softmax', 'pml_hip_index', 'pml_hip_contract_dispatch', 'pml_hip_contract_invoke', 'pml_hip_plan_free',
-    'pml_hip_rows_takes', 'pml_hip_rows', 'pml_hip_argmax_rows', 'pml_hip_topk_rows', 'pml_hip_memcpy_h2d_async', 'pml_hip_memcpy_d2h_async', 'pml_hip_copy_spans', 'pml_hip_product_dispatch', 'pml_hip_product_takes_tail', 'pml_hip_plan_bytes', 'pml_hip_product_pays', 'pml_hip_product_invoke', 'pml_hip_conv2d_grad_takes',
+    'pml_hip_rows_takes', 'pml_hip_rows', 'pml_hip_argmax_rows', 'pml_hip_topk_rows', 'pml_hip_memcpy_h2d_async', 'pml_hip_memcpy_d2h_async', 'pml_hip_copy_spans', 'pml_hip_copy_spans_stamped', 'pml_hip_clock_khz', 'pml_hip_product_dispatch', 'pml_hip_product_takes_tail', 'pml_hip_plan_bytes', 'pml_hip_product_pays', 'pml_hip_product_invoke', 'pml_hip_conv2d_grad_takes',
     'pml_hip_conv2d_grad_dispatch', 'pml_hip_conv2d_grad_invoke',
     'pml_hip_plan_describe', 'pml_hip_struct_size', 'pml_hip_gemm_pack_b', 'pml_hip_conv2d_pack_filter', 'pml_hip_conv2d_takes_maxpool',
     'pml_hip_gather', 'pml_hip_scatter', 'pml_hip_argsort', 'pml_hip_prng',

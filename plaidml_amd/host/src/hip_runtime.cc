@@ -68,6 +68,11 @@ class HipExecutable final : public Executable {
       }
       handles_.assign(plan_->steps.size(), 0);
       for (size_t i = 0; i < plan_->steps.size(); ++i) dispatch(i);
+      // Where a run begins and ends on the device is read off its clock by the kernels that copy, or by one of their kind
+      // (two events around the launches cost a run 8 us); with events where that cannot be had, and under PLAIDML_PROFILE.
+      clock_khz_ = pml_hip_clock_khz();
+      void* stamps = nullptr;
+      if (clock_khz_ > 0 && pml_hip_host_alloc(&stamps, 2 * sizeof(uint64_t)) == 0) stamps_ = static_cast<uint64_t*>(stamps);
       hipCheck(pml_hip_event_create(&ev0_), "event");
       hipCheck(pml_hip_event_create(&ev1_), "event");
       hipCheck(pml_hip_stream_create(&stream_), "stream");
@@ -145,9 +150,17 @@ class HipExecutable final : public Executable {
           hipCheck(pml_hip_memcpy_h2d(device_[buf], from, bytes, stream_), "h2d");
         }
       }
-      up.issue(stream_);
+      const bool stamped = stamps_ && !profile;
+      up.issue(stream_, stamped ? &stamps_[0] : nullptr, true);
       st.h2d_ms = nowMs() - start;
       launchAll(profile, &st);
+      // (ahead of what the copy engines fetch; otherwise by the kernel that fetches the results)
+      uint64_t* end = stamped ? &stamps_[1] : nullptr;
+      for (int buf : plan_->output_buffers)
+        if (end && plan_->buffers[buf].bytes > kKernelCopy) {
+          Spans().issue(stream_, end, false);
+          end = nullptr;
+        }
       for (size_t i = 0; i < outputs.size(); ++i) {
         const int buf = plan_->output_buffers[i];
         const size_t bytes = plan_->buffers[buf].bytes;
@@ -158,7 +171,7 @@ class HipExecutable final : public Executable {
         else
           unstaged.push_back(i);
       }
-      down.issue(stream_);
+      down.issue(stream_, end, false);
       collect(&stage, arriving);
     } catch (...) {
       (void)pml_hip_stream_sync(stream_);  // queued copies may still use the caller's memory
@@ -204,6 +217,8 @@ class HipExecutable final : public Executable {
   size_t arena_bytes_ = 0, fixed_bytes_ = 0, unshared_temp_bytes_ = 0;
   std::vector<int64_t> handles_;
   pml_hip_event ev0_ = nullptr, ev1_ = nullptr;
+  uint64_t* stamps_ = nullptr;  // page-locked: the device's clock ahead of and behind a run's launches
+  int clock_khz_ = 0;
   std::vector<pml_hip_event> step_events_;
   pml_hip_stream stream_ = nullptr;  // every copy and launch of this executable
   pml_hip_graph graph_ = nullptr;    // the launches of one run, recorded
@@ -230,8 +245,9 @@ class HipExecutable final : public Executable {
       src.push_back(s);
       bytes.push_back(n);
     }
-    void issue(pml_hip_stream stream) {
-      if (!dst.empty()) hipCheck(pml_hip_copy_spans(static_cast<int>(dst.size()), dst.data(), src.data(), bytes.data(), stream), "copy");
+    void issue(pml_hip_stream stream, uint64_t* stamp, bool after) {
+      if (!dst.empty() || stamp)
+        hipCheck(pml_hip_copy_spans_stamped(static_cast<int>(dst.size()), dst.data(), src.data(), bytes.data(), stamp, after ? 1 : 0, stream), "copy");
     }
   };
 
@@ -377,7 +393,8 @@ class HipExecutable final : public Executable {
     // allocate, which cannot be recorded).  A recording that fails leaves the executable with one-by-one launches.
     if (graphable_ && !profile && !graph_ && runs_ >= 2) record();
     ++runs_;
-    hipCheck(pml_hip_event_record(ev0_, stream_), "event record");
+    const bool events = profile || !stamps_;
+    if (events) hipCheck(pml_hip_event_record(ev0_, stream_), "event record");
     if (graph_ && !profile) {
       hipCheck(pml_hip_graph_launch(graph_, stream_), "graph launch");
       st->replayed = true;
@@ -388,14 +405,18 @@ class HipExecutable final : public Executable {
       }
     }
     if (profile) hipCheck(pml_hip_event_record(step_events_.back(), stream_), "event record");
-    hipCheck(pml_hip_event_record(ev1_, stream_), "event record");
+    if (events) hipCheck(pml_hip_event_record(ev1_, stream_), "event record");
   }
 
   // statistics of a run that has been waited for
   void finish(bool profile, InvokeStats* st) {
-    float ms = 0;
-    hipCheck(pml_hip_event_elapsed_ms(ev0_, ev1_, &ms), "event elapsed");
-    st->kernel_ms = ms;
+    if (stamps_ && !profile) {
+      st->kernel_ms = static_cast<double>(stamps_[1] - stamps_[0]) / clock_khz_;
+    } else {
+      float ms = 0;
+      hipCheck(pml_hip_event_elapsed_ms(ev0_, ev1_, &ms), "event elapsed");
+      st->kernel_ms = ms;
+    }
     st->launches = plan_->steps.size();
     st->graph_note = graph_note_;
     st->arena_bytes = arena_bytes_;
@@ -533,6 +554,8 @@ class HipExecutable final : public Executable {
     if (ev0_) pml_hip_event_destroy(ev0_);
     if (ev1_) pml_hip_event_destroy(ev1_);
     ev0_ = ev1_ = nullptr;
+    if (stamps_) pml_hip_host_free(stamps_);
+    stamps_ = nullptr;
     if (graph_) pml_hip_graph_destroy(graph_);
     graph_ = nullptr;
     if (stream_) pml_hip_stream_destroy(stream_);
