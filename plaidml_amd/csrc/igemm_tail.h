@@ -353,11 +353,32 @@ __device__ __forceinline__ void direct_tail_bf16(const IgemmArgs& p, f32x16_t (&
   }
 }
 
+// `live` (1 to 4) neighbouring elements of ES bytes each from w to element `at` of C, which may lie on any element's
+// boundary: one store for four of them.
+template <int ES, class W>
+__device__ __forceinline__ void store_live(void* C, int64_t at, const W& w, int live) {
+  unsigned char* const to = (unsigned char*)C + at * ES;
+  if (live == 4) {
+    __builtin_memcpy(to, &w, 4 * ES);
+    return;
+  }
+  const unsigned char* const from = (const unsigned char*)&w;
+#pragma unroll
+  for (int q = 0; q < 3; ++q)
+    if (q < live) __builtin_memcpy(to + q * ES, from + q * ES, ES);
+}
+
 // Four neighbouring results of tail_mode 1 or 2 -- the sums with their start value, res the residual tensor's bits -- finished
-// and stored at element `at` of C.
-template <int KIND>
+// and stored at element `at` of C.  RAGGED: `live` of them, anywhere.
+template <int KIND, bool RAGGED = false>
 __device__ __forceinline__ void store_quad(void* C, int64_t at, int out_dtype, const typename Acc<KIND>::scalar (&v4)[4], const i32x4_t& res,
-                                           bool residual, bool relu) {
+                                           bool residual, bool relu, int live = 4) {
+  auto put = [&](auto* to, const auto& w) {
+    if constexpr (RAGGED)
+      store_live<sizeof(w) / 4>(C, at, w, live);
+    else
+      *to = w;
+  };
   if (KIND == KIND_I8) {
     i32x4_t w;
 #pragma unroll
@@ -365,7 +386,7 @@ __device__ __forceinline__ void store_quad(void* C, int64_t at, int out_dtype, c
       const int v = (int)((unsigned)(int)v4[q] + (unsigned)res[q]);
       w[q] = (relu && v < 0) ? 0 : v;
     }
-    *(i32x4_t*)((int*)C + at) = w;
+    put((i32x4_t*)((int*)C + at), w);
   } else if (out_dtype == PML_HIP_BF16) {
     // v_cvt_pk_bf16_f32 rounds to nearest even.  relu is applied to the fp32 value just before
     // the last rounding (a result in (-2^-134, 0) stores +0 where the definition gives -0).
@@ -396,7 +417,7 @@ __device__ __forceinline__ void store_quad(void* C, int64_t at, int out_dtype, c
     uint32_t o01, o23;
     __builtin_memcpy(&o01, &h01, 4);
     __builtin_memcpy(&o23, &h23, 4);
-    *(uint2*)((uint16_t*)C + at) = make_uint2(o01, o23);
+    put((uint2*)((uint16_t*)C + at), make_uint2(o01, o23));
   } else {
     f32x4_t w;
 #pragma unroll
@@ -404,7 +425,7 @@ __device__ __forceinline__ void store_quad(void* C, int64_t at, int out_dtype, c
       const float v = residual ? (float)v4[q] + __int_as_float(res[q]) : (float)v4[q];
       w[q] = (relu && v < 0.f) ? 0.f : v;
     }
-    *(f32x4_t*)((float*)C + at) = w;
+    put((f32x4_t*)((float*)C + at), w);
   }
 }
 
@@ -451,6 +472,18 @@ __device__ __forceinline__ void tile_tail(const IgemmArgs& p, const typename Acc
         const f32x4_t w = *(const f32x4_t*)((const float*)p.init + n);
 #pragma unroll
         for (int q = 0; q < 4; ++q) cinit[q] = (accs_t)w[q];
+      }
+    } else if (p.init_dtype == natural) {
+      // the same off its alignment, at the right edge or with a stride: an element at a time, requested together
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int64_t at = (n + q < p.N ? n + q : n) * p.init_cs;
+        if (natural == PML_HIP_BF16)
+          cinit[q] = (accs_t)__uint_as_float((uint32_t)((const uint16_t*)p.init)[at] << 16);
+        else if (natural == PML_HIP_I32)
+          cinit[q] = (accs_t)((const int*)p.init)[at];
+        else
+          cinit[q] = (accs_t)((const float*)p.init)[at];
       }
     } else {
 #pragma unroll
@@ -827,6 +860,65 @@ __device__ __forceinline__ void tile_tail(const IgemmArgs& p, const typename Acc
 #pragma unroll
       for (int c = 0; c < kRows; ++c)
         if (live[c]) store4(p.C, c);
+    }
+    return;
+  }
+
+  // The same tails where the last quad of columns is not whole, or rows of C begin anywhere: row by row, and not unrolled -- the
+  // unrolled code above, with the checks this takes in it, spilled 90 registers of the 128 some tiles may have.  (Before
+  // this the interpreter below ran every result of such a problem: bf16 1402 x 162, K = 2528 29.9 -> 27.7 us, int8 129 x 35,
+  // K = 912 with requantisation 53.9 -> 12.6, 1636 x 749, K = 400 58.1 -> 12.8, a float convolution to 7 x 47 x 47 x 19
+  // 11.0 -> 8.4.)
+  const bool requant = KIND == KIND_I8 && p.tail_mode == 4 && p.tail_rq;
+  if (p.tail_mode == 1 || p.tail_mode == 2 || requant) {
+    const int live = full4 ? 4 : (int)(p.N - n);
+    f32x4_t sc = {0, 0, 0, 0};
+    if (requant) {
+      const float* const scale = (const float*)p.operands[p.rq_scale];
+      const bool one = p.tail.operand_col_stride[p.rq_scale] == 0;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) sc[q] = scale[one ? 0 : q < live ? n + q : n];
+    }
+#pragma unroll 1
+    for (int row = row0; row < BM; row += RPP) {
+      const int64_t m = m0 + row;
+      if (m >= p.M) break;
+      accs_t v4[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) v4[q] = ctile[row * CS + c4 + q] + cinit[q];
+      if (p.init && !col_init) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          if (q >= live) break;
+          Scalar<float, int> b = load_scalar<float, int>(p.init, m * p.init_rs + (n + q) * p.init_cs, p.init_dtype);
+          v4[q] += KIND == KIND_I8 ? (accs_t)b.i : (accs_t)b.f;
+        }
+      }
+      const int64_t at = m * p.ldc + n;
+      if (requant) {
+        // (as above: clamps, then round half away from zero and the cast in one)
+        if (p.rq_store >= 0) store_live<4>(p.outs[p.rq_store], at, i32x4_t{(int)v4[0], (int)v4[1], (int)v4[2], (int)v4[3]}, live);
+        uint32_t w = 0;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const float v = __builtin_fminf(__builtin_fmaxf((float)v4[q] * sc[q], p.rq_lo), p.rq_hi);
+          w |= (uint32_t)((int)(v + __builtin_copysignf(0.5f, v)) & 255) << (8 * q);
+        }
+        store_live<1>(p.C, at, w, live);
+        continue;
+      }
+      i32x4_t res = {0, 0, 0, 0};
+      if (residual) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int64_t from = m * res_rs + (q < live ? n + q : n);
+          if (KIND != KIND_I8 && p.out_dtype == PML_HIP_BF16)
+            res[q >> 1] |= (int)((uint32_t)((const uint16_t*)p.operands[0])[from] << (16 * (q & 1)));
+          else
+            res[q] = ((const int*)p.operands[0])[from];
+        }
+      }
+      store_quad<KIND, true>(p.C, at, p.out_dtype, v4, res, residual, p.tail_relu != 0, live);
     }
     return;
   }
