@@ -174,6 +174,9 @@ __global__ __launch_bounds__(64 * kWaves, 4) void direct_kernel(IgemmArgs p_by_v
   const __amdgpu_buffer_rsrc_t rb2 = __builtin_amdgcn_make_buffer_rsrc((void*)(two ? p.Bt2 : Bt), 0, (int)kBufRange, kRsrcFlags);
 
   const int kbytes = (int)(CONV ? p.CI * ES : K * ES);  // valid bytes per (tap) row
+  // CONV: bytes between pixels; less than a row's when a tap is a run of pixels (a chunk's pixel by multiply-and-shift then)
+  const int pitch = CONV && p.pix_pitch ? p.pix_pitch : kbytes;
+  const unsigned pitch_magic = CONV && p.pix_pitch ? ((1u << 20) + (unsigned)pitch - 1) / (unsigned)pitch : 0u;
   const int steps_per_tap = (kbytes + 63) >> 6;
   const int k2_bytes = two ? (int)(K2 * ES) : 0;
   const int n_steps = CONV ? KH * KW * steps_per_tap : steps_per_tap + ((k2_bytes + 63) >> 6);
@@ -196,7 +199,7 @@ __global__ __launch_bounds__(64 * kWaves, 4) void direct_kernel(IgemmArgs p_by_v
       const int ow = (int)(rem - oh * (unsigned)p.OW);
       a_ih[i] = ok ? (int)oh * p.SH - p.PH : -(1 << 28);
       a_iw[i] = ow * p.SW - p.PW;
-      a_off[i] = (unsigned)((int64_t)nb * ((int64_t)H * W * kbytes)) + (unsigned)(a_ih[i] * W + a_iw[i]) * (unsigned)kbytes;
+      a_off[i] = (unsigned)((int64_t)nb * ((int64_t)H * W * pitch)) + (unsigned)(a_ih[i] * W + a_iw[i]) * (unsigned)pitch;
     } else {
       a_off[i] = ok ? (unsigned)(m * lda * ES) : kOutside;
       int64_t row = mu;
@@ -259,11 +262,11 @@ __global__ __launch_bounds__(64 * kWaves, 4) void direct_kernel(IgemmArgs p_by_v
       if constexpr (CONV) {
         const int cb = cs * 64 + g * 16;
         const bool ok = live & (cb < kbytes);
-        const int dh = kh * DH, dw = kw * DW;
-        const unsigned at = (unsigned)((dh * W + dw) * kbytes + cb);
+        const int dh = kh * DH, dw = kw * DW, px = dw + (int)(__umul24((unsigned)cb, pitch_magic) >> 20);
+        const unsigned at = (unsigned)((dh * W + dw) * pitch + cb);
 #pragma unroll
         for (int i = 0; i < MB; ++i) {
-          const bool in = ok & ((unsigned)(a_ih[i] + dh) < (unsigned)H) & ((unsigned)(a_iw[i] + dw) < (unsigned)W);
+          const bool in = ok & ((unsigned)(a_ih[i] + dh) < (unsigned)H) & ((unsigned)(a_iw[i] + px) < (unsigned)W);
           fa[u][i] = __builtin_bit_cast(i32x4_t, __builtin_amdgcn_raw_buffer_load_b128(ra, in ? (int)(a_off[i] + at) : (int)kOutside, 0, 0));
         }
         const unsigned bk = (unsigned)((kh * KW + kw) * kbytes + cb);
@@ -414,8 +417,7 @@ static hipError_t launch_large(const IgemmArgs& a, hipStream_t s) {
 hipError_t PML_CAT(direct_launch_kind_, PML_KIND)(int cfg, bool conv, const IgemmArgs& a, hipStream_t s) {
   const bool small = cfg == TILE_16x16_W8;
   if (conv) {
-    // (K-runs that span several pixels are the re-blocked convolution's: igemm.hip)
-    if (a.b_kn || a.pix_pitch) return hipErrorInvalidValue;
+    if (a.b_kn) return hipErrorInvalidValue;
     return small ? launch<PML_KIND, true, 1, 1, false>(a, s) : launch_large<true>(a, s);
   }
   if (a.b_kn) {

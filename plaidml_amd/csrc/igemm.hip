@@ -967,14 +967,12 @@ hipError_t igemm_launch(int kind, int cfg, bool conv, const IgemmArgs& a, hipStr
   if (a_bytes >= ((int64_t)1 << 31) || b_bytes >= ((int64_t)1 << 31) || (conv && a.M >= ((int64_t)1 << 31))) return hipErrorInvalidValue;
   if (cfg == TILE_256x256_W8 && a.b_kn && (kind == KIND_BF16 || kind == KIND_I8)) return given_launch(kind, a, s);
   if (cfg == TILE_16x16_W8 || cfg == TILE_32x32_W8) {
-    if (!conv || !a.pix_pitch) {
-      switch (kind) {
-        case KIND_F32: return direct_launch_kind_0(cfg, conv, a, s);
-        case KIND_BF16: return direct_launch_kind_1(cfg, conv, a, s);
-        case KIND_I8: return direct_launch_kind_2(cfg, conv, a, s);
-      }
+    switch (kind) {
+      case KIND_F32: return direct_launch_kind_0(cfg, conv, a, s);
+      case KIND_BF16: return direct_launch_kind_1(cfg, conv, a, s);
+      case KIND_I8: return direct_launch_kind_2(cfg, conv, a, s);
     }
-    cfg = TILE_64x64;  // (not built for the split fp32 kinds, nor for K-runs over several pixels)
+    cfg = TILE_64x64;  // (not built for the split fp32 kinds)
   }
   switch (kind) {
     case KIND_F32: return igemm_launch_kind_0(cfg, conv, a, s);

@@ -74,3 +74,23 @@ def test_int8_tails(tile, M, N, monkeypatch):
                 got, stored = got
                 np.testing.assert_array_equal(stored, S + start)
             np.testing.assert_array_equal(got, want)
+
+
+@pytest.mark.parametrize('kind', ['f32', 'bf16', 'i8'])
+@pytest.mark.parametrize('tile', ['64x64', '128x128w8s2', '64x64ks', '16x16w8', '32x32w8'])
+@pytest.mark.parametrize('shape,kh,kw,co,stride', [((2, 5, 3, 16), 7, 7, 20, 1), ((1, 12, 9, 48), 5, 5, 70, 2), ((1, 6, 17, 112), 3, 3, 33, 1), ((3, 9, 10, 32), 1, 5, 64, 1)])
+def test_filter_rows_as_one_tap(kind, tile, shape, kh, kw, co, stride, monkeypatch):
+    """Pixels of less than a slab (or of a broken number of them): the taps of a filter row are one run over neighbouring
+    pixels, whose chunks lie inside or outside the image one by one -- images narrower than the filter among them."""
+    monkeypatch.setitem(T.FORCED, 'flags', hk.flag_conv(hk.CONV_IGEMM) | hk.flag_tile(tile))
+    rng = np.random.default_rng(co)
+    n, h, w, ci = shape
+    I, F = whole(rng, shape), whole(rng, (kh, kw, ci, co))  # sums below 2^24
+    dt, out, cast = {'f32': (hk.F32, hk.F32, lambda a: a), 'bf16': (hk.BF16, hk.BF16, T.bf16), 'i8': (hk.I8, hk.I32, lambda a: a.astype(np.int8))}[kind]
+    got = T.run_conv(cast(I), cast(F), dt, out, stride=stride)
+    oh, ow = -(-h // stride), -(-w // stride)
+    ph, pw = max(0, (oh - 1) * stride + kh - h) // 2, max(0, (ow - 1) * stride + kw - w) // 2
+    pad = np.zeros((n, h + 2 * kh, w + 2 * kw, ci))
+    pad[:, ph:ph + h, pw:pw + w] = I
+    want = sum(pad[:, y:y + (oh - 1) * stride + 1:stride, x:x + (ow - 1) * stride + 1:stride] @ F[y, x].astype(np.float64) for y in range(kh) for x in range(kw))
+    np.testing.assert_array_equal(E.bf16_from_bits(got) if kind == 'bf16' else got, E.round_bf16(want.astype(np.float32)) if kind == 'bf16' else want)
