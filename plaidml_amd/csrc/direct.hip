@@ -13,6 +13,11 @@
 // KN: the right-hand side is the caller's B[K][N] as it lies.  A lane takes four neighbouring columns of every K-row of
 // its chunk and turns them in registers (v_perm) into fragments of four column blocks, block j holding the columns
 // 4 r + j: tiles are 64 columns wide, and no transposed copy is written and read back.
+// RAGGED: the same from rows that begin at any element (N or the pitch no multiple of four, bf16 and int8): a lane fetches
+// the aligned words around its four columns and shifts them together -- how far is the same for all lanes, since 16 bytes of
+// K further down the rows lie as before.  Columns past N are fetched as what follows in memory, or as zeros behind the last
+// row (the descriptor ends there), and never stored.  Before, such a right-hand side was transposed by a launch of its own: 7 x 327, K = 192 bf16 10.4 -> 4.5 us,
+// 51 x 861, K = 2272 int8 15.7 -> 9.1, 6 x 3382, K = 256 fp32 (which needs no shifting) 11.4 -> 5.4; 36 sizes drawn 1.43x.
 #include <hip/hip_runtime.h>
 
 #include "device_common.h"
@@ -134,18 +139,20 @@ __device__ __forceinline__ void add_start(const i32x4_t& bits, bool bf, typename
 }
 
 // MB x NB blocks of 16 x 16 results per workgroup.
-template <int KIND, bool CONV, int MB, int NB, bool KN>
+template <int KIND, bool CONV, int MB, int NB, bool KN, bool RAGGED>
 __global__ __launch_bounds__(64 * kWaves, 4) void direct_kernel(IgemmArgs p_by_value) {
   warm_arguments<sizeof(IgemmArgs)>();
   // (read where the dispatcher put it: indexing a by-value copy would move the copy to scratch memory)
   const IgemmArgs& p = *(const IgemmArgs*)(const __attribute__((address_space(4))) void*)__builtin_amdgcn_kernarg_segment_ptr();
   static_assert(!KN || (NB == 4 && !CONV), "a [K][N] right-hand side is taken four columns per lane");
+  static_assert(!RAGGED || (KN && KIND != KIND_F32), "four-byte elements are whole words wherever they lie");
   typedef typename Acc<KIND>::scalar accs_t;
   typedef accs_t acc4_t __attribute__((ext_vector_type(4)));
   constexpr int ES = KIND == KIND_BF16 ? 2 : (KIND == KIND_I8 ? 1 : 4);
   constexpr int TM = 16 * MB, TN = 16 * NB;
   // steps in flight: 64 registers of requests, fewer where the accumulators leave less room
-  constexpr int U = KN ? (MB == 1 ? 3 : 2) : MB + NB > 4 ? 2 : 16 / (MB + NB);
+  constexpr int U = KN ? (MB == 1 && !RAGGED ? 3 : 2) : MB + NB > 4 ? 2 : 16 / (MB + NB);
+  constexpr int RW = RAGGED ? (KIND == KIND_BF16 ? 24 : 32) : 16;  // KN: words fetched for a lane's chunk
   constexpr int CS = TN + 4;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   accs_t* const parts = (accs_t*)smem;  // [wavefront][TM][CS]
@@ -168,7 +175,10 @@ __global__ __launch_bounds__(64 * kWaves, 4) void direct_kernel(IgemmArgs p_by_v
   if constexpr (CONV) hold(H, W, KH, KW, DH, DW);
 
   const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void*)A, 0, (int)kBufRange, kRsrcFlags);
-  const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void*)Bt, 0, (int)kBufRange, kRsrcFlags);
+  // (KN: from the word its first element lies in to the end of the word its last one lies in -- the lanes at the right edge
+  // fetch past rows; words are inside or outside the range as a whole)
+  const int b_rem = KN ? (int)((uintptr_t)Bt & 3) : 0;
+  const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void*)((uintptr_t)Bt - b_rem), 0, KN ? (b_rem + (int)(((K - 1) * ldbt + N) * ES) + 3) & ~3 : (int)kBufRange, kRsrcFlags);
   const bool two = !CONV && !KN && K2 > 0;
   const __amdgpu_buffer_rsrc_t ra2 = __builtin_amdgcn_make_buffer_rsrc((void*)(two ? p.A2 : A), 0, (int)kBufRange, kRsrcFlags);
   const __amdgpu_buffer_rsrc_t rb2 = __builtin_amdgcn_make_buffer_rsrc((void*)(two ? p.Bt2 : Bt), 0, (int)kBufRange, kRsrcFlags);
@@ -214,7 +224,7 @@ __global__ __launch_bounds__(64 * kWaves, 4) void direct_kernel(IgemmArgs p_by_v
     }
   }
   if constexpr (KN) {
-    const int64_t n = n0 + 4 * r;  // (N is a multiple of four: a lane's columns exist together)
+    const int64_t n = n0 + 4 * r;
     b_off[0] = n < N ? (unsigned)(n * ES) : kOutside;
   } else {
 #pragma unroll
@@ -255,7 +265,7 @@ __global__ __launch_bounds__(64 * kWaves, 4) void direct_kernel(IgemmArgs p_by_v
   for (int s0 = first; s0 < last; s0 += U) {
     i32x4_t fa[U][MB];
     i32x4_t fb[KN ? 1 : U][KN ? 1 : NB];
-    int raw[KN ? U : 1][16];
+    int raw[KN ? U : 1][RW];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const bool live = s0 + u < last;
@@ -295,12 +305,19 @@ __global__ __launch_bounds__(64 * kWaves, 4) void direct_kernel(IgemmArgs p_by_v
           const bool in = ok & (b_off[0] != kOutside);
 #pragma unroll
           for (int e = 0; e < E; ++e) {
-            const int off = in ? (int)(at + (unsigned)e * pitch) : (int)kOutside;
+            // (RAGGED: the word a row's first byte lies in, counted from the aligned base; the same for all lanes but `at`)
+            const int row = RAGGED ? (b_rem + e * (int)pitch) & ~3 : e * (int)pitch;
+            const int off = in ? (int)(at + (unsigned)row) : (int)kOutside;
             if constexpr (KIND == KIND_F32) {
               const i32x4_t v = __builtin_bit_cast(i32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rb, off, 0, 0));
 #pragma unroll
               for (int q = 0; q < 4; ++q) raw[u][4 * e + q] = v[q];
-            } else if constexpr (KIND == KIND_BF16) {
+            } else if constexpr (RAGGED && KIND == KIND_BF16) {
+              typedef int i32x3_t __attribute__((ext_vector_type(3)));
+              const i32x3_t v = __builtin_bit_cast(i32x3_t, __builtin_amdgcn_raw_buffer_load_b96(rb, off, 0, 0));
+#pragma unroll
+              for (int q = 0; q < 3; ++q) raw[u][3 * e + q] = v[q];
+            } else if constexpr (RAGGED || KIND == KIND_BF16) {
               typedef int i32x2_t __attribute__((ext_vector_type(2)));
               const i32x2_t v = __builtin_bit_cast(i32x2_t, __builtin_amdgcn_raw_buffer_load_b64(rb, off, 0, 0));
               raw[u][2 * e] = v[0];
@@ -322,7 +339,21 @@ __global__ __launch_bounds__(64 * kWaves, 4) void direct_kernel(IgemmArgs p_by_v
     for (int u = 0; u < U; ++u) {
       if constexpr (KN) {
         i32x4_t frag[4];
-        turn<KIND>(raw[u], frag);
+        if constexpr (RAGGED) {
+          // the four columns of each row out of the words around them
+          int words[16];
+          constexpr int E = 16 / ES, W = RW / E, V = 16 / E;  // rows, words fetched of each, words of it wanted
+#pragma unroll
+          for (int e = 0; e < E; ++e) {
+            const unsigned shift = (unsigned)((b_rem + e * (int)(ldbt * ES)) & 3) * 8;
+#pragma unroll
+            for (int q = 0; q < V; ++q)
+              words[V * e + q] = (int)__builtin_amdgcn_alignbit((unsigned)raw[u][W * e + q + 1], (unsigned)raw[u][W * e + q], shift);
+          }
+          turn<KIND>(words, frag);
+        } else {
+          turn<KIND>(raw[u], frag);
+        }
 #pragma unroll
         for (int i = 0; i < MB; ++i)
 #pragma unroll
@@ -383,13 +414,13 @@ __global__ __launch_bounds__(64 * kWaves, 4) void direct_kernel(IgemmArgs p_by_v
   tile_tail<KIND, TM, TN, kQuads>(p, parts, m0, n0, tid);
 }
 
-template <int KIND, bool CONV, int MB, int NB, bool KN>
+template <int KIND, bool CONV, int MB, int NB, bool KN, bool RAGGED = false>
 hipError_t launch(const IgemmArgs& a, hipStream_t s) {
   const int64_t tiles_m = (a.M + 16 * MB - 1) / (16 * MB), tiles_n = (a.N + 16 * NB - 1) / (16 * NB);
   const int64_t tiles = tiles_m * tiles_n;
   if (tiles <= 0 || tiles >= ((int64_t)1 << 31)) return hipErrorInvalidValue;
   const size_t lds = (size_t)kWaves * 16 * MB * (16 * NB + 4) * 4;
-  auto kern = direct_kernel<KIND, CONV, MB, NB, KN>;
+  auto kern = direct_kernel<KIND, CONV, MB, NB, KN, RAGGED>;
   static DynamicLdsLimit limit;
   if (hipError_t e = limit.ensure((const void*)kern, lds); e != hipSuccess) return e;
   IgemmArgs b = a;
@@ -421,7 +452,10 @@ hipError_t PML_CAT(direct_launch_kind_, PML_KIND)(int cfg, bool conv, const Igem
     return small ? launch<PML_KIND, true, 1, 1, false>(a, s) : launch_large<true>(a, s);
   }
   if (a.b_kn) {
-    if (a.K2 > 0 || a.N % 4 != 0 || a.ldbt % 4 != 0) return hipErrorInvalidValue;
+    if (a.K2 > 0) return hipErrorInvalidValue;
+    if constexpr (PML_KIND != KIND_F32)
+      if (((a.N | a.ldbt) & 3) != 0 || ((uintptr_t)a.Bt & (PML_KIND == KIND_BF16 ? 7 : 3)) != 0)
+        return small ? launch<PML_KIND, false, 1, 4, true, true>(a, s) : launch<PML_KIND, false, 2, 4, true, true>(a, s);
     return small ? launch<PML_KIND, false, 1, 4, true>(a, s) : launch<PML_KIND, false, 2, 4, true>(a, s);
   }
   return small ? launch<PML_KIND, false, 1, 1, false>(a, s) : launch_large<false>(a, s);

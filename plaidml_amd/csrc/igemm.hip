@@ -635,10 +635,15 @@ __global__ __launch_bounds__(256) void transpose_kernel(const T* __restrict__ B,
   __shared__ T tile[64][65];
   const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
   const int64_t k0 = (int64_t)blockIdx.y * 64, n0 = (int64_t)blockIdx.x * 64;
-  for (int r = ty; r < 64; r += 4) {
-    const int64_t k = k0 + r, n = n0 + tx;
-    tile[r][tx] = (k < K && n < N) ? B[k * ldb + n] : (T)0;
+  // (all sixteen in flight: one after the other they were a chain of memory latencies)
+  T v[16];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const int64_t k = k0 + ty + 4 * i, n = n0 + tx;
+    v[i] = (k < K && n < N) ? B[k * ldb + n] : (T)0;
   }
+#pragma unroll
+  for (int i = 0; i < 16; ++i) tile[ty + 4 * i][tx] = v[i];
   __syncthreads();
   for (int r = ty; r < 64; r += 4) {
     const int64_t n = n0 + r, k = k0 + tx;

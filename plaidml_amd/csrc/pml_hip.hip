@@ -937,10 +937,9 @@ struct SecondProduct {
 // is transposed into Bt[N][K] first.  Rows must be whole 16-byte vectors.
 static bool reads_b_as_given(const pml_hip_gemm_desc& d, int mfma_kind, const void* b, int tile) {
   if ((tile == TILE_16x16_W8 || tile == TILE_32x32_W8) && mfma_kind != KIND_F32X3) {
-    // (four neighbouring columns per lane and K-row, whatever the type: direct.hip)
+    // (four neighbouring columns per lane and K-row, whatever the type and wherever the rows begin: direct.hip)
     const int64_t es = dt_size(d.in_dtype);
-    return b && !d.b_layout && d.k2 == 0 && d.n % 4 == 0 && d.ldb % 4 == 0 && ((uintptr_t)b & (4 * es - 1)) == 0 &&
-           d.k * d.ldb * es < ((int64_t)1 << 31);
+    return b && !d.b_layout && d.k2 == 0 && ((uintptr_t)b & (es - 1)) == 0 && d.k * d.ldb * es < ((int64_t)1 << 31);
   }
   if (tile == TILE_256x256_W8 && (mfma_kind == KIND_BF16 || mfma_kind == KIND_I8))
     return b && takes_b_as_given(d, mfma_kind, tile, d.ldb) && ((uintptr_t)b & (4 * dt_size(d.in_dtype) - 1)) == 0;

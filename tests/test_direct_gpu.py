@@ -232,3 +232,34 @@ def test_tail_operands_read_ahead(kind, out, tile, M, N, ldr, shift):
     r = E.round_bf16 if out == 'bf16' else lambda a: a
     want = np.maximum(r(r(A @ B + bias[shift:]) + res[:, :N]), 0)
     np.testing.assert_array_equal(E.bf16_from_bits(got) if out == 'bf16' else got, want)
+
+
+@pytest.mark.parametrize('kind', ['f32', 'bf16', 'i8'])
+@pytest.mark.parametrize('tile', TILES)
+@pytest.mark.parametrize('M,N,K,ldb,shift', [(1, 1, 16, 1, 0), (17, 67, 80, 67, 0), (33, 130, 272, 131, 1), (40, 65, 48, 66, 1), (5, 63, 1040, 67, 3), (20, 64, 80, 64, 1)])
+def test_right_hand_side_rows_that_begin_anywhere(kind, tile, M, N, K, ldb, shift):
+    """[K][N] read as it lies with N, the pitch and the pointer (`shift` elements off) no multiple of four: exact sums of whole
+    numbers; the gap of the pitch holds NaNs / values that must not be read into a result; the buffer ends with the last row."""
+    rng = np.random.default_rng(M + N + shift)
+    top = 100 if kind == 'i8' else 4
+    A, B = rng.integers(-top, top + 1, (M, K)).astype(np.float32), rng.integers(-top, top + 1, (K, N)).astype(np.float32)
+    dt, out, cast, onp = {'f32': (hk.F32, hk.F32, lambda a: a.astype(np.float32), np.float32), 'bf16': (hk.BF16, hk.F32, T.bf16, np.float32),
+                          'i8': (hk.I8, hk.I32, lambda a: a.astype(np.int8), np.int32)}[kind]
+    flat = np.full(shift + (K - 1) * ldb + N, 77 if kind == 'i8' else np.nan, np.float32)
+    for k in range(K):
+        flat[shift + k * ldb:shift + k * ldb + N] = B[k]
+    d = hk.GemmDesc()
+    d.in_dtype, d.out_dtype, d.c_dtype = dt, out, out
+    d.m, d.n, d.k, d.lda, d.ldb, d.ldc = M, N, K, K, ldb, N
+    plan = hk.lib().pml_hip_gemm_dispatch(ctypes.byref(d))
+    assert plan and 'with B as it lies' in hk.describe(plan), hk.describe(plan)
+    hk.lib().pml_hip_plan_free(plan)
+    d.flags = hk.flag_tile(tile)
+    plan = hk.lib().pml_hip_gemm_dispatch(ctypes.byref(d))
+    dA, dB, dC = hk.DeviceBuffer.from_numpy(cast(A)), hk.DeviceBuffer.from_numpy(cast(flat)), hk.DeviceBuffer(M * N * 4)
+    at = (dB.ptr.value if hasattr(dB.ptr, 'value') else dB.ptr) + shift * cast(flat).itemsize
+    none = hk.ptr_array([])
+    hk.check(hk.lib().pml_hip_gemm_invoke(plan, dA.ptr, at, dC.ptr, None, none, none, None))
+    hk.check(hk.lib().pml_hip_stream_sync(None))
+    np.testing.assert_array_equal(dC.to_numpy(onp, (M, N)), A @ B)
+    hk.lib().pml_hip_plan_free(plan)
