@@ -170,13 +170,25 @@ bool schedule_bits_ok(int flags) {
 }
 const char* const kTileShort[PML_HIP_TILE_COUNT_] = {"64x64", "128x64", "128x128", "128x64w8", "128x128w8", "256x128w16", "128x128w8s2", "64x64w8k2", "256x256w8", "128x64n2", "192x384w8", "64x64ks", "16x16w8", "32x32w8"};
 
+// Whether the K loop of 64 x 64 tiles is shared out among workgroups (TILE_64x64_KSPLIT).  Few tiles and a long K: always.
+// Up to five eighths of a round of tiles it is where the chain is long enough to pay for the second launch, for bf16 and the
+// split fp32 kind: bf16 40 x 20 x 20 x 96 (*) 7 x 7 x 96 stride 2, 126 tiles of 74 slabs, 29.8 -> 20.5 us; 593 x 606, K = 3808
+// 28.9 -> 17.5; 900 x 512, K = 2992 24.0 -> 17.4; but 700 x 600, K = 2048 11.2, 13.9 split (the operands of the longer ones
+// are past an L2's 4 MB).  fp32 as three products 1210 x 511, K = 2832 41.1 -> 35.6.  fp32 takes direct tiles there, or is
+// slower split (725 x 364, K = 880: 13.1, 17.3).
+bool splits_k(int64_t m, int64_t n, int64_t k_bytes, int kind) {
+  const int64_t t = ((m + 63) / 64) * ((n + 63) / 64);
+  if (k_bytes < 2048) return false;
+  return t <= 64 || (t <= 160 && ((kind == KIND_BF16 && k_bytes >= 5632) || (kind == KIND_F32X3 && k_bytes >= 8192)));
+}
+
 // One of the direct tiles (direct.hip) where it beats the LDS kernels, or -1.  Both sides are priced in microseconds, from
 // measurements of 27 matrix products and 18 convolutions per element kind (one row to 3136, K of 64 to 4608; back to back
 // in a recorded graph): a direct kernel takes 2.6 plus, per round of one tile on each CU (fp32 and 32 x 64: whole
 // rounds), 0.8 (fp32 32 x 32: 1.9; 32 x 64, which replaces 32 x 32 beyond one round: bf16 1.6, int8 1.0, fp32 2.3) and its
 // operand bytes at 40 KB a microsecond and CU (32 x 64: bf16 50, int8 60, fp32 32).  An LDS kernel takes 4.2 plus its chain
 // of 128-byte slabs (0.23 each, int8 0.28, fp32 0.58), or -- K split over workgroups -- 5.2 (fp32 5.6) plus 0.4 per KB of K
-// plus writing and reading the partial tiles at 3 TB/s.  The prices meet the measurements to about 15 %; a direct tile has
+// (more than 64 tiles: 0.5 per slab of a split) plus writing and reading the partial tiles at 3 TB/s.  The prices meet the measurements to about 15 %; a direct tile has
 // to be 5 % ahead.
 //   us, before -> direct                       bf16              fp32              int8
 //   1 x 1000, K = 2048                     7.4 ->  5.0       9.3 ->  7.3       6.7 ->  4.3
@@ -211,11 +223,11 @@ int direct_tile_of(int64_t m, int64_t n, int64_t k_bytes, int kind, int64_t kn_l
   const int64_t slabs = (k_bytes + 127) / 128;
   double lds_us = 4.2 + (f32 ? 0.58 : kind == KIND_I8 ? 0.28 : 0.23) * (double)slabs;
   bool needs_bt = kind == KIND_BF16 || n % (16 / es) != 0 || kn_ldb % 16 != 0;
-  if (can_split && tiles(64, 64) <= 64 && k_bytes >= 2048) {
+  if (can_split && splits_k(m, n, k_bytes, kind)) {
     int splits = 1, per = 0;
     igemm_split_plan(m, n, slabs, n_cus, &splits, &per);
     if (splits >= 2) {
-      lds_us = (f32 ? 5.6 : 5.2) + kb / 2500 + 8.0 * splits * (double)m * (double)n / 3e6;
+      lds_us = (f32 ? 5.6 : 5.2) + (tiles(64, 64) <= 64 ? kb / 2500 : 0.5 * (double)per) + 8.0 * splits * (double)m * (double)n / 3e6;
       needs_bt = true;
     }
   }
@@ -259,7 +271,7 @@ int choose_tile(int64_t m, int64_t n, int64_t k_bytes, int kind = KIND_BF16, boo
   auto tiles = [&](int64_t bm, int64_t bn) { return ((m + bm - 1) / bm) * ((n + bn - 1) / bn); };
   // Few tiles and a long K (a network's last stages at batch 1: 49 x 512 x 4608 is 8 tiles of 72 slabs): the K loop is
   // shared out among workgroups and a second launch adds the partial tiles up.  Measured inside ResNet-50 at batch 1.
-  if (allow_split && tiles(64, 64) <= 64 && k_bytes >= 2048) return TILE_64x64_KSPLIT;
+  if (allow_split && splits_k(m, n, k_bytes, kind)) return TILE_64x64_KSPLIT;
   if (kind == KIND_F32X3) {
     // A fragment that is split in registers costs 24 vector instructions whatever it is multiplied with, so the
     // tile a wavefront holds decides how many MFMAs share that cost -- but the problems this kind meets here are

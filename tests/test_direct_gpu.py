@@ -263,3 +263,26 @@ def test_right_hand_side_rows_that_begin_anywhere(kind, tile, M, N, K, ldb, shif
     hk.check(hk.lib().pml_hip_stream_sync(None))
     np.testing.assert_array_equal(dC.to_numpy(onp, (M, N)), A @ B)
     hk.lib().pml_hip_plan_free(plan)
+
+
+@pytest.mark.parametrize('kind,M,N,K,split', [('bf16', 593, 606, 3808, True), ('bf16', 593, 606, 2816, True), ('bf16', 593, 606, 2800, False), ('f32x3', 450, 390, 2048, True), ('f32x3', 450, 390, 2032, False)])
+def test_long_chains_of_some_tiles_are_split(kind, M, N, K, split):
+    """More than 64 tiles: the K loop is shared out from the length on at which that pays."""
+    if kind == 'f32x3':
+        rng = np.random.default_rng(K)
+        A, B = rng.uniform(-1, 1, (M, K)).astype(np.float32), rng.uniform(-1, 1, (K, N)).astype(np.float32)
+    else:
+        A, B = operands('bf16', M, N, K, K)
+    d = hk.GemmDesc()
+    dt = hk.F32 if kind == 'f32x3' else hk.BF16
+    d.in_dtype = d.out_dtype = d.c_dtype = dt
+    d.m, d.n, d.k, d.lda, d.ldb, d.ldc, d.flags = M, N, K, K, N, N, hk.FP32_AS_BF16X3 if kind == 'f32x3' else 0
+    plan, _ = held(d)
+    assert ('K split over workgroups' in hk.describe(plan)) == split, hk.describe(plan)
+    hk.lib().pml_hip_plan_free(plan)
+    want = A.astype(np.float64) @ B.astype(np.float64)
+    if kind == 'f32x3':
+        got = T.run_gemm(A, B, hk.F32, hk.F32, flags=hk.FP32_AS_BF16X3, invokes=2)
+        assert np.abs(got - want).max() < 4 * 2.0 ** -16 * np.sqrt(K) * 0.25 + 1e-5
+    else:
+        check(E.bf16_from_bits(T.run_gemm(T.bf16(A), T.bf16(B), hk.BF16, hk.BF16, invokes=2)), want, 'bf16', K)
