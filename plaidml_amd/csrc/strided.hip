@@ -563,12 +563,19 @@ hipError_t launch_modes(const StridedArgs& a, int amode, int bmode, hipStream_t 
 // after the last whole step is the last wavefront's.  A lane holds the columns 4 r .. 4 r + 3 of a 16-row block: from a
 // [K][N] right-hand side four neighbours of every K-row, turned with v_perm (bf16) or by naming (fp32), near the right edge
 // the last four columns instead; from an [N][K] one four rows.  The partial tiles meet in LDS and are added in wavefront order.
-template <bool BF, int BMODE, int MB>
+// WORDS (bf16, matrices below 2 GiB): rows that begin at any value are fetched as the aligned words around a lane's values,
+// through descriptors that end with the matrix, and shifted together (16-byte loads from 2-byte boundaries reach 17 KB a
+// microsecond and CU); a broken last step of K is a step like the others with the values past K cleared on both sides.
+// Columns past N are whatever follows, and never stored.  Two steps in flight: three and four are slower (registers).
+// 300 x 777, K = 1001 10.1 -> 7.1 us from [K][N], 15.1 -> 9.4 from [N][K]; 33 x 131, K = 255 8.7 -> 4.6; 1000 x 1001, K = 1001
+// 19.6 -> 13.2.
+template <bool BF, int BMODE, int MB, bool WORDS>
 __global__ __launch_bounds__(512, 4) void product_direct_kernel(StridedArgs p_by_value) {
   const StridedArgs& p = *(const StridedArgs*)(const __attribute__((address_space(4))) void*)__builtin_amdgcn_kernarg_segment_ptr();
   constexpr int kWaves = 8, TM = 16 * MB, TN = 64, CS = TN + 4, ES = BF ? 2 : 4;
   constexpr int E = 16 / ES, KS = 4 * E;  // K-values per lane and step, per step
-  constexpr int U = MB == 1 ? 4 : 2, NA = BF ? 1 : 2;
+  constexpr int U = !WORDS && MB == 1 ? 4 : 2, NA = BF ? 1 : 2;
+  static_assert(!WORDS || BF, "fp32 values are words wherever they lie");
   extern __shared__ __attribute__((aligned(16))) char smem[];
   float* const parts = (float*)smem;  // [wavefront][TM][CS]
   const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, g = lane >> 4;
@@ -590,25 +597,56 @@ __global__ __launch_bounds__(512, 4) void product_direct_kernel(StridedArgs p_by
     c_at += i * p.c_batch[d];
   }
 
-  const int64_t steps = p.K / KS;  // whole ones
+  const int64_t steps = WORDS ? (p.K + KS - 1) / KS : p.K / KS;  // (whole ones)
   const int64_t per = (steps + kWaves - 1) / kWaves, first = wave * per;
   const int64_t last = first + per < steps ? first + per : steps;
 
-  const char* a_ptr[MB];
-#pragma unroll
-  for (int i = 0; i < MB; ++i) {
-    const int64_t m = m0 + 16 * i + r;
-    a_ptr[i] = (const char*)p.A + (a_at + (m < p.M ? m : p.M - 1) * p.a_ms + g * E) * ES;
-  }
-  const char* b_ptr[BMODE == ROWS_K ? 4 : 1];
+  constexpr unsigned kFlags = 0x00020000u;     // raw buffer, 32-bit data format
+  constexpr unsigned kOutside = 0x80000000u;   // past every range, with any offset below 2 GiB added
   const int64_t n = n0 + 4 * r;
-  if constexpr (BMODE == ROWS_K) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) b_ptr[j] = (const char*)p.B + (b_at + (n + j < p.N ? n + j : p.N - 1) * p.b_ns + g * E) * ES;
-  } else {
-    b_ptr[0] = (const char*)p.B + (b_at + (n + 4 <= p.N ? n : p.N - 4) + g * E * p.b_ks) * ES;  // (N is at least four)
-  }
   const int64_t b_pitch = p.b_ks * ES;
+  constexpr int NB = BMODE == ROWS_K ? 4 : 1;
+  const char* a_ptr[WORDS ? 1 : MB];
+  const char* b_ptr[WORDS ? 1 : NB];
+  // WORDS: offsets of the words the lane's chunks begin in, and by how many bits the values begin behind that
+  unsigned a_off[MB], a_shift[MB], b_off[NB], b_shift[NB];
+  int b_rem = 0;
+  __amdgpu_buffer_rsrc_t ra, rb;
+  if constexpr (WORDS) {
+    auto matrix = [&](const void* base, int64_t at, int64_t values, int* rem) {
+      const uintptr_t first = (uintptr_t)base + (uintptr_t)(at * ES);
+      *rem = (int)(first & 3);
+      return __builtin_amdgcn_make_buffer_rsrc((void*)(first - *rem), 0, (*rem + (int)(values * ES) + 3) & ~3, kFlags);
+    };
+    int a_rem;
+    ra = matrix(p.A, a_at, (p.M - 1) * p.a_ms + p.K, &a_rem);
+    rb = matrix(p.B, b_at, (p.K - 1) * p.b_ks + (p.N - 1) * p.b_ns + 1, &b_rem);
+#pragma unroll
+    for (int i = 0; i < MB; ++i) {
+      const int64_t m = m0 + 16 * i + r;
+      const unsigned at = (unsigned)((m * p.a_ms + g * E) * ES) + (unsigned)a_rem;
+      a_off[i] = m < p.M ? at & ~3u : kOutside;
+      a_shift[i] = (at & 3) * 8;
+    }
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+      const unsigned at = BMODE == ROWS_K ? (unsigned)(((n + j) * p.b_ns + g * E) * ES) + (unsigned)b_rem : (unsigned)((n + g * E * p.b_ks) * ES);
+      b_off[j] = n + j < p.N ? (BMODE == ROWS_K ? at & ~3u : at) : kOutside;
+      b_shift[j] = (at & 3) * 8;
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < MB; ++i) {
+      const int64_t m = m0 + 16 * i + r;
+      a_ptr[i] = (const char*)p.A + (a_at + (m < p.M ? m : p.M - 1) * p.a_ms + g * E) * ES;
+    }
+    if constexpr (BMODE == ROWS_K) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) b_ptr[j] = (const char*)p.B + (b_at + (n + j < p.N ? n + j : p.N - 1) * p.b_ns + g * E) * ES;
+    } else {
+      b_ptr[0] = (const char*)p.B + (b_at + (n + 4 <= p.N ? n : p.N - 4) + g * E * p.b_ks) * ES;  // (N is at least four)
+    }
+  }
 
   f32x4_t sums[MB][4][NA];
 #pragma unroll
@@ -648,18 +686,89 @@ __global__ __launch_bounds__(512, 4) void product_direct_kernel(StridedArgs p_by
       }
   };
 
-  for (int64_t s0 = first; s0 < last; s0 += U) {
+  if constexpr (WORDS) {
+    constexpr int WB = BMODE == ROWS_K ? 20 : 24;  // words fetched of B's 16
+    typedef int i32x3_t __attribute__((ext_vector_type(3)));
+    auto fetch5 = [](__amdgpu_buffer_rsrc_t rs, unsigned off, uint32_t* to) {
+      const i32x4_t v = __builtin_bit_cast(i32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)off, 0, 0));
+#pragma unroll
+      for (int q = 0; q < 4; ++q) to[q] = (uint32_t)v[q];
+      to[4] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rs, (int)(off + 16), 0, 0);
+    };
+    for (int64_t s0 = first; s0 < last; s0 += U) {
+      uint32_t wa[U][MB][5], wb[U][WB];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const bool live = s0 + u < last;
+        const unsigned k = (unsigned)((s0 + u) * KS);
+#pragma unroll
+        for (int i = 0; i < MB; ++i) fetch5(ra, live ? a_off[i] + k * ES : kOutside, wa[u][i]);
+        if constexpr (BMODE == ROWS_K) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) fetch5(rb, live ? b_off[j] + k * ES : kOutside, &wb[u][5 * j]);
+        } else {
+          const unsigned at = b_off[0] + k * (unsigned)b_pitch;
+#pragma unroll
+          for (int e = 0; e < E; ++e) {
+            const bool in = live & (b_off[0] != kOutside) & (k + g * E + e < (unsigned)p.K);
+            const i32x3_t v = __builtin_bit_cast(i32x3_t, __builtin_amdgcn_raw_buffer_load_b96(rb, (int)(in ? at + (unsigned)((b_rem + e * (int)b_pitch) & ~3) : kOutside), 0, 0));
+#pragma unroll
+            for (int q = 0; q < 3; ++q) wb[u][3 * e + q] = (uint32_t)v[q];
+          }
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if (s0 + u >= last) continue;
+        Words<4> fa[MB];
+        uint32_t raw[16];
+#pragma unroll
+        for (int i = 0; i < MB; ++i)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) fa[i].w[q] = __builtin_amdgcn_alignbit(wa[u][i][q + 1], wa[u][i][q], a_shift[i]);
+        if constexpr (BMODE == ROWS_K) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) raw[4 * j + q] = __builtin_amdgcn_alignbit(wb[u][5 * j + q + 1], wb[u][5 * j + q], b_shift[j]);
+        } else {
+#pragma unroll
+          for (int e = 0; e < E; ++e) {
+            const unsigned shift = (unsigned)((b_rem + e * (int)b_pitch) & 3) * 8;
+#pragma unroll
+            for (int q = 0; q < 2; ++q) raw[2 * e + q] = __builtin_amdgcn_alignbit(wb[u][3 * e + q + 1], wb[u][3 * e + q], shift);
+          }
+        }
+        if ((s0 + u + 1) * KS > p.K) {
+          // the values past K: cleared in A, and in B where a lane holds values of K (its rows past K arrive as zeros)
+          const int have = (int)(p.K - (s0 + u) * KS) - g * E;
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const uint32_t keep = 2 * q + 1 < have ? 0xffffffffu : 2 * q < have ? 0xffffu : 0u;
+#pragma unroll
+            for (int i = 0; i < MB; ++i) fa[i].w[q] &= keep;
+            if constexpr (BMODE == ROWS_K) {
+#pragma unroll
+              for (int j = 0; j < 4; ++j) raw[4 * j + q] &= keep;
+            }
+          }
+        }
+        multiply(fa, raw);
+      }
+    }
+  }
+  for (int64_t s0 = first; !WORDS && s0 < last; s0 += U) {
     Words<4> fa[U][MB];
     uint32_t raw[U][16];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int64_t k = (s0 + u < last ? s0 + u : last - 1) * KS;  // (a step past the run is read again and not multiplied)
 #pragma unroll
-      for (int i = 0; i < MB; ++i) fa[u][i] = load_words<4>(a_ptr[i] + k * ES);
+      for (int i = 0; i < MB; ++i) fa[u][i] = load_words<4>(a_ptr[WORDS ? 0 : i] + k * ES);
       if constexpr (BMODE == ROWS_K) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          const Words<4> v = load_words<4>(b_ptr[j] + k * ES);
+          const Words<4> v = load_words<4>(b_ptr[WORDS ? 0 : j] + k * ES);
 #pragma unroll
           for (int q = 0; q < 4; ++q) raw[u][4 * j + q] = v.w[q];
         }
@@ -677,7 +786,7 @@ __global__ __launch_bounds__(512, 4) void product_direct_kernel(StridedArgs p_by
       if (s0 + u < last) multiply(fa[u], raw[u]);
   }
 
-  const int left = (int)(p.K - steps * KS);
+  const int left = WORDS ? 0 : (int)(p.K - steps * KS);
   if (left > 0 && wave == kWaves - 1) {
     // value by value, zeros past the end on both sides
     const int64_t k = steps * KS;
@@ -688,7 +797,7 @@ __global__ __launch_bounds__(512, 4) void product_direct_kernel(StridedArgs p_by
     for (int i = 0; i < MB; ++i)
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const char* const at = a_ptr[i] + k * ES + 4 * q;
+        const char* const at = a_ptr[WORDS ? 0 : i] + k * ES + 4 * q;
         const int kk = g * E + (BF ? 2 * q : q);
         fa[i].w[q] = value(at, kk < left) | (BF ? value(at + 2, kk + 1 < left) << 16 : 0u);
       }
@@ -697,7 +806,7 @@ __global__ __launch_bounds__(512, 4) void product_direct_kernel(StridedArgs p_by
       for (int j = 0; j < 4; ++j)
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          const char* const at = b_ptr[j] + k * ES + 4 * q;
+          const char* const at = b_ptr[WORDS ? 0 : j] + k * ES + 4 * q;
           const int kk = g * E + (BF ? 2 * q : q);
           raw[4 * j + q] = value(at, kk < left) | (BF ? value(at + 2, kk + 1 < left) << 16 : 0u);
         }
@@ -732,7 +841,7 @@ __global__ __launch_bounds__(512, 4) void product_direct_kernel(StridedArgs p_by
   for (int w = 1; w < kWaves; ++w) sum += *(const f32x4_t*)(at + w * (TM * CS));
   const int live = p.N - col < 4 ? (int)(p.N - col) : 4;
   float v[4] = {sum[0], sum[1], sum[2], sum[3]};
-  if (BMODE != ROWS_K && live < 4) {  // the quad holds the last four columns: its own are the last `live` of them
+  if (!WORDS && BMODE != ROWS_K && live < 4) {  // the quad holds the last four columns: its own are the last `live` of them
     v[0] = live == 3 ? sum[1] : live == 2 ? sum[2] : sum[3];
     v[1] = live == 3 ? sum[2] : sum[3];
     v[2] = sum[3];
@@ -742,10 +851,25 @@ __global__ __launch_bounds__(512, 4) void product_direct_kernel(StridedArgs p_by
   store_results(p, p.C, c_row + col, v, live);
 }
 
-template <bool BF, int BMODE, int MB>
+// Whether a direct bf16 tile takes its rows as shifted words (offsets fit 31 bits): where one begins off a word or K ends
+// within a step, and with 16 rows between 64 and 512 of K, where a wavefront has one or two steps and the other form fetches four
+// (33 x 136, K = 256: [K][N] 5.1 -> 4.7 us, [N][K] 6.0 -> 5.4).
+bool direct_by_words(const StridedArgs& a, int64_t rows) {
+  int64_t odd = a.a_ms | (a.b_ks == 1 ? a.b_ns : a.b_ks);
+  for (int d = 0; d < a.n_batch; ++d) odd |= a.a_batch[d] | a.b_batch[d];
+  const bool off_words = (odd & 1) != 0 || (((uintptr_t)a.A | (uintptr_t)a.B) & 3) != 0;
+  if (!off_words && a.K % 32 == 0 && (rows != 16 || a.K <= 64 || a.K > 512)) return false;
+  const int64_t limit = ((int64_t)1 << 30) - 64;
+  return (double)a.M * (double)a.a_ms + (double)a.K < (double)limit &&
+         (double)(a.K + 64) * (double)a.b_ks + (double)a.N * (double)a.b_ns < (double)limit;
+}
+
+template <bool BF, int BMODE, int MB, bool WORDS = false>
 hipError_t launch_direct(const StridedArgs& a, hipStream_t s) {
+  if constexpr (BF && !WORDS)
+    if (direct_by_words(a, 16 * MB)) return launch_direct<BF, BMODE, MB, true>(a, s);
   const size_t lds = (size_t)8 * 16 * MB * 68 * 4;
-  auto kern = product_direct_kernel<BF, BMODE, MB>;
+  auto kern = product_direct_kernel<BF, BMODE, MB, WORDS>;
   static DynamicLdsLimit limit;
   if (hipError_t e = limit.ensure((const void*)kern, lds); e != hipSuccess) return e;
   StridedArgs b = a;
@@ -763,23 +887,26 @@ hipError_t launch_direct(const StridedArgs& a, hipStream_t s) {
 // Which of its two kernels a product takes -- the direct tile's rows (16 or 32), or 0: the tiles through LDS that strided_plan
 // has laid out -- and what it is expected to take in microseconds (an infinity: neither can be launched).  Both sides are
 // priced from 25 shapes per type and layout (1 to 2000 rows, K of 32 to 2047, batches up to 96) and from 45 with many small
-// tiles (batches of 100 to 100000, 1 to 128 rows and columns, K of 3 to 4096).  Direct: 2.6 plus, per round of one tile on
-// each CU, 0.8 (1.8 where bf16 has a broken last step of K; fp32 1.4 from the second round on) and the tile's operand bytes
-// at 38 KB a microsecond for fp32 with 16 rows, 32 with 32 rows (the matrix cores), bf16 25 from [K][N] and 17.5 from [N][K]
-// (16-byte loads at 2-byte alignment).  Through LDS: 3 and 1.65 a slab (bf16 [K][N] 3.6 and 1.55, [N][K] 4 and 1.1); every
-// further round -- workgroups share a CU by then -- 0.6 and 0.95 a slab (bf16 [K][N] 0.3 and 1.5, [N][K] 0.75 and 0.5, 0.55
-// more where the rows are read element by element); tiles of 128 in the first round 4 and 6 (bf16 10 and 6 or 2.5), in the others
-// 1.5 and 3.1 (bf16 1 and 6, 1.7 and 1.75); split, 1.8 more and the partial results written and read at 3 TB/s.  A direct
-// tile has to be 8 % ahead.
+// tiles (batches of 100 to 100000, 1 to 128 rows and columns, K of 3 to 4096); bf16 again from 136 of both sorts, half of them
+// with odd rows, and the choice checked on 70 others: it takes 0.9 % longer than the best of the three would on average.
+// Direct, fp32: 2.6 plus, per round of one tile on each CU, 0.8 (1.4 from the second round on where K has a broken last step)
+// and the tile's operand bytes at 38 KB a microsecond with 16 rows, 32 with 32 rows (the matrix cores).  Direct, bf16, whose
+// workgroups share CUs: 3.6 plus the operand bytes at 60 KB a microsecond from [K][N] and 38 from [N][K], 48 and 28 as shifted
+// words, and for every further tile per CU as much and 0.95, with 32 rows 0.5 once.  Through LDS: 3 and 1.65 a slab (bf16 4.8 and
+// 1.5, [N][K] 1.1); every further round 0.6 and 0.95 a slab (bf16 0.8 and 0.5, 1.2 from odd [K][N] rows, [N][K] 0.9 and 0.35,
+// 0.55 more where the rows are read element by element); tiles of 128 in the first round 4 and 6 (bf16 10 and 6 or 2.5), in the
+// others 1.5 and 3.1 (bf16 1 and 6, 1.7 and 1.75); split, 1.8 more and the partial results written and read at 3 TB/s.  A direct
+// fp32 tile has to be 8 % ahead.
 //   us, through LDS -> direct              fp32 [K][N]       bf16 [K][N]       bf16 [N][K]
-//   3 x 1001, K = 333                    14.9 ->  5.0      13.2 ->  6.4      10.6 ->  7.7
-//   300 x 777, K = 1001                  20.5 -> 10.9      13.9 ->  9.9      12.6 (15.1)
-//   1000 x 1001, K = 1001                55.3 -> 32.1      28.0 -> 19.0      21.1 (25.3)
-//   20 of 100 x 77, K = 100              10.4 ->  4.6       8.5 ->  5.2       8.0 ->  4.9
-//   50 x 777, K = 1777: stays split      13.6 (22.1)       12.6 (17.8)       11.4 (23.4)
-//   10000 of 1 x 16, K = 64              99.4 -> 66.2      71.2 -> 56.0      53.0 (52.2)
-//   10000 of 16 x 16, K = 16             63.5 (60.4)       73.6 (110)        56.4 (91.1)
-//   1000 of 1 x 1, K = 4096               463 -> 113                          135 -> 34
+//   3 x 1001, K = 333                    14.9 ->  5.0      13.5 ->  4.2      11.0 ->  4.6
+//   300 x 777, K = 1001                  20.5 -> 10.9      14.4 ->  7.2      13.3 ->  9.4
+//   1000 x 1001, K = 1001                55.3 -> 32.1      28.7 -> 13.2      22.2 -> 18.7
+//   20 of 100 x 77, K = 100              10.4 ->  4.6       8.6 ->  4.5       7.8 ->  4.4
+//   50 x 777, K = 1777: fp32, [N][K] split  13.6 (22.1)    13.1 ->  9.1      12.0 (14.0)
+//   10000 of 1 x 16, K = 64              99.4 -> 66.2        60 ->   45        46 ->   40
+//   10000 of 17 x 17, K = 17                                 68 ->   54        54 ->   48
+//   96 of 128 x 64, K = 128                                 6.9 ->  4.5       6.4 ->  5.2
+//   1000 of 1 x 1, K = 4096               463 -> 113                          135 ->   23
 int product_direct_rows(const StridedArgs& a, bool bf, int mi, int n_cus, double* us) {
   const bool nk = a.b_ks == 1;
   double batches = 1;
@@ -796,8 +923,9 @@ int product_direct_rows(const StridedArgs& a, bool bf, int mi, int n_cus, double
       first = !bf ? 4 + 6 * slabs : 10 + (nk ? 2.5 : 6) * slabs;
       each = !bf ? 1.5 + 3.1 * slabs : nk ? 1.7 + 1.75 * slabs : 1 + 6 * slabs;
     } else {
-      first = !bf ? 3 + 1.65 * slabs : nk ? 4 + 1.1 * slabs : 3.6 + 1.55 * slabs;
-      each = !bf ? 0.6 + 0.95 * slabs : nk ? 0.75 + 0.5 * slabs : 0.3 + 1.5 * slabs;
+      first = !bf ? 3 + 1.65 * slabs : nk ? 4.8 + 1.1 * slabs : 4.8 + 1.5 * slabs;
+      each = !bf ? 0.6 + 0.95 * slabs : nk ? 0.9 + 0.35 * slabs : 0.8 + 0.5 * slabs;
+      if (bf && !nk && (a.b_ks & 1)) each += 0.7 * slabs;
       if (gathered) each += 0.55 * slabs * (double)std::min<int64_t>(a.M, 64) / 64;
     }
     lds_us = first + more * each;
@@ -807,15 +935,19 @@ int product_direct_rows(const StridedArgs& a, bool bf, int mi, int n_cus, double
   auto direct_us = [&](int64_t rows) {
     const double tiles = batches * (double)((a.M + rows - 1) / rows) * (double)((a.N + 63) / 64);
     if (tiles * 512 > (double)kMaxLaunchThreads) return never;
-    const double rate = bf ? (nk ? 17.5e3 : 25e3) : (rows == 16 ? 38e3 : 32e3);
     const double live = (double)(rows == 16 ? std::min<int64_t>(a.M, 16) : 32) + 64;
+    if (bf) {
+      const double each = live * kb / (direct_by_words(a, rows) ? (nk ? 28e3 : 48e3) : nk ? 38e3 : 60e3), more = std::max(0.0, tiles / n_cus - 1);
+      return 3.6 + each + more * (0.95 + each) + (rows == 32 ? 0.5 * std::min(1.0, more) : 0);
+    }
+    const double rate = rows == 16 ? 38e3 : 32e3;
     const double rounds = std::ceil(tiles / n_cus);
-    return 2.6 + rounds * ((bf && a.K % 32 != 0 ? 1.8 : 0.8) + live * kb / rate) + (!bf && a.K % 16 != 0 ? 0.6 * (rounds - 1) : 0);
+    return 2.6 + rounds * (0.8 + live * kb / rate) + (a.K % 16 != 0 ? 0.6 * (rounds - 1) : 0);
   };
   *us = lds_us;
   if (a.a_ks != 1 || (!nk && (a.b_ns != 1 || a.N < 4))) return 0;
   const double small = direct_us(16), large = direct_us(32), direct = std::min(small, large);
-  if (direct > 0.92 * lds_us || direct == never) return 0;
+  if (direct > (bf ? 1 : 0.92) * lds_us || direct == never) return 0;
   *us = direct;
   return small <= large ? 16 : 32;
 }

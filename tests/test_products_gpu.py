@@ -1,10 +1,13 @@
 """Products over free strides and the gradients of a convolution (csrc/strided.hip) against float64 on the CPU, at the sizes where
 tiles, slabs, splits and 16-byte vectors end raggedly."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
 from plaidml_amd import edsl as P
+from plaidml_amd import hipkernels as hk
 from plaidml_amd import op as Pop
 
 pytestmark = pytest.mark.gpu
@@ -132,3 +135,42 @@ def test_conv_gradients_leave_taps_outside_out(dtype, n, h, w, ci, co, k, stride
         np.testing.assert_array_equal(np.isposinf(got), np.isposinf(want))
         np.testing.assert_array_equal(np.isneginf(got), np.isneginf(want))
         check(got[np.isfinite(want)], want[np.isfinite(want)], dtype)
+
+
+@pytest.mark.parametrize('nk', [0, 1])
+@pytest.mark.parametrize('at', [0, 1])
+@pytest.mark.parametrize('b,m,n,k', [(1, 1, 4, 65), (1, 3, 2050, 95), (2, 17, 67, 33), (1, 33, 65, 257), (1, 16, 64, 512), (3, 15, 66, 66), (1, 40, 5, 1001), (260, 33, 7, 31), (9, 31, 70, 287)])
+def test_bf16_rows_that_begin_off_a_word(nk, at, b, m, n, k):
+    """Direct bf16 tiles over matrices that begin at an odd value or not, with rows a few values longer than K or N and NaN in
+    all that belongs to neither matrix: whole and broken steps of K, one and two rounds of steps, columns past a quad."""
+    rng = np.random.default_rng(m * n + k + at)
+    pa, pb, pc = k + 3 - at, (k if nk else n) + 2 + at, n + 1
+    rows_b = n if nk else k
+
+    def embed(rows, cols, pitch):
+        v = P.round_bf16(rng.standard_normal((b, rows, cols)).astype(np.float32))
+        flat = torch.full((at + b * rows * pitch + 4,), float('nan'), dtype=torch.bfloat16, device='cuda')
+        flat[at:at + b * rows * pitch].view(b, rows, pitch)[:, :, :cols] = torch.from_numpy(v).to('cuda', torch.bfloat16)
+        return v.astype(np.float64), flat
+    A, da = embed(m, k, pa)
+    B, db = embed(rows_b, k if nk else n, pb)
+    out = torch.full((at + b * m * pc + 4,), 7.0, dtype=torch.bfloat16, device='cuda')
+    d = hk.ProductDesc()
+    d.in_dtype = d.out_dtype = hk.BF16
+    d.n_batch, d.m, d.n, d.k, d.a_ms, d.a_ks, d.c_ms, d.row_len = 1, m, n, k, pa, 1, pc, n
+    d.batch[0], d.a_batch[0], d.b_batch[0], d.c_batch[0] = b, m * pa, rows_b * pb, m * pc
+    d.b_ks, d.b_ns = (1, pb) if nk else (pb, 1)
+    L = hk.lib()
+    plan = L.pml_hip_product_dispatch(ctypes.byref(d))
+    text = hk.describe(plan)
+    assert 'tile=16x64' in text or 'tile=32x64' in text, text
+    torch.cuda.synchronize()
+    hk.check(L.pml_hip_product_invoke(plan, da.data_ptr() + 2 * at, db.data_ptr() + 2 * at, out.data_ptr() + 2 * at, None, None, None))
+    torch.cuda.synchronize()
+    L.pml_hip_plan_free(plan)
+    got = out[at:at + b * m * pc].view(b, m, pc).float().cpu().numpy()
+    assert (got[:, :, n:] == 7).all() and (out[at + b * m * pc:] == 7).all() and (out[:at] == 7).all()
+    want = np.matmul(A, B.transpose(0, 2, 1) if nk else B)
+    # rounding to bf16 (2^-9), and fp32 sums of k products whichever way they are ordered
+    bound = np.abs(want) * 2.0 ** -8 + np.matmul(np.abs(A), np.abs(B.transpose(0, 2, 1) if nk else B)) * (k * 2.0 ** -23)
+    assert (np.abs(got[:, :, :n] - want) <= bound).all()
