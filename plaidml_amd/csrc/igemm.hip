@@ -971,6 +971,7 @@ hipError_t igemm_launch(int kind, int cfg, bool conv, const IgemmArgs& a, hipStr
   const int64_t b_bytes = (a.b_kn ? a.K : a.N) * a.ldbt * es;
   if (a_bytes >= ((int64_t)1 << 31) || b_bytes >= ((int64_t)1 << 31) || (conv && a.M >= ((int64_t)1 << 31))) return hipErrorInvalidValue;
   if (cfg == TILE_256x256_W8 && a.b_kn && (kind == KIND_BF16 || kind == KIND_I8)) return given_launch(kind, a, s);
+  if (kind == KIND_BF16 && stream_takes(cfg, conv, a)) return stream_launch(conv, a, s);
   if (cfg == TILE_16x16_W8 || cfg == TILE_32x32_W8) {
     switch (kind) {
       case KIND_F32: return direct_launch_kind_0(cfg, conv, a, s);

@@ -142,7 +142,8 @@ inline void tile_of(const TileOrder& o, unsigned bid, int* tm, int* tn) {
 
 struct IgemmArgs {
   TileOrder order;  // filled in by the launcher for the tile grid of the configuration it launches
-  int b_kn;         // 1: Bt / ldbt are the caller's row-major B[K][N] and its row length (fp32 and int8 GEMMs)
+  int b_kn;         // 1: Bt / ldbt are the caller's row-major B[K][N] and its row length (GEMMs)
+  int stream;       // 1: the tile was chosen for the problem's sizes, not named by the caller: rows may stream instead (stream.hip)
   // conv_blocks4x4_kernel only: the caller's NHWC image of 3 bf16 channels (raw_h x raw_w pixels, raw_w even), from
   // which the kernel builds the rows of 2x2 pixel blocks itself; null: A already holds the re-blocked image
   const void* raw_in;
@@ -210,6 +211,9 @@ struct IgemmArgs {
 hipError_t igemm_launch(int kind, int cfg, bool conv, const IgemmArgs& a, hipStream_t s);
 // TILE_256x256_W8 of a bf16 or int8 GEMM whose right-hand side is read as it lies (a.b_kn): given.hip
 hipError_t given_launch(int kind, const IgemmArgs& a, hipStream_t s);
+// bf16 products of many rows and a short K over Bt: stream.hip
+bool stream_takes(int cfg, bool conv, const IgemmArgs& a);
+hipError_t stream_launch(bool conv, const IgemmArgs& a, hipStream_t s);
 // How TILE_64x64_KSPLIT shares the K loop out: slabs of 128 bytes of K in all, and for a device of n_cus compute units
 // the number of splits (1: not worth splitting) with the slabs each takes -- about one workgroup per CU, at least two
 // slabs per split, at most 16 splits.

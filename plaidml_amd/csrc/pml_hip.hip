@@ -584,6 +584,7 @@ void conv_args(const Plan* p, IgemmArgs& g) {
   g.tail = d.tail;
   g.NB = (int)d.n;
   g.n_cus = device_cus();
+  g.stream = PML_HIP_FLAG_TILE_OF(d.flags) < 0;
   g.halo_rows = p->halo_rows;
   g.n_tiles = p->halo_tiles;
   g.halo_variant = p->halo_variant;
@@ -1043,6 +1044,7 @@ static int gemm_run(const pml_hip_gemm_desc& d, int mfma_kind, int tile, const D
   g.init_cs = d.init_col_stride;
   g.c_dtype = d.c_dtype;
   g.n_cus = device_cus();
+  g.stream = PML_HIP_FLAG_TILE_OF(d.flags) < 0;
   classify_tail(d.tail, d.out_dtype, d.c_dtype, &g.tail_mode, &g.tail_relu);
   g.tail_ssr = tail_scale_shift(d.tail, d.out_dtype, g.tail_mode);
   tail_requant(d.tail, d.out_dtype, d.c_dtype, g.tail_mode, &g);

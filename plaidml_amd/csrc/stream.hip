@@ -1,0 +1,225 @@
+// bf16 products of many rows and a short K: the right-hand side lives in registers, the rows stream past it.
+//
+// Such a product (the 1x1 convolutions of a network: 401408 x 256 with K = 64 and a residual, 8 to 30 operations a byte) is
+// bound by memory, and a tile that is loaded, multiplied, finished and stored by one workgroup keeps too little of it in flight:
+// K is one or two slabs, so its life is a load, a wait, a tail with another load and wait, and stores, and only the other
+// workgroup on the CU covers for that.  Here a wavefront keeps the right-hand side of 64 columns (32 past K = 128) in
+// registers for its whole life and walks down the rows, 16 at a time; the left-hand rows and the residual rows of the next
+// tiles are on their way to registers while it multiplies and stores the current one, and nothing is shared between
+// wavefronts -- no LDS, no barrier.  The wavefronts of a workgroup hold neighbouring columns of the same rows, whose
+// left-hand side they find in L1, and the workgroups of one XCD the other columns of these rows, which find it in L2.
+//
+// The MFMAs are the 16 x 16 ones with the right-hand side as the row operand.  Row i of block b of a pair holds column
+// 8 (i / 4) + 4 b + i % 4 of the pair's 32, so that a lane ends with eight neighbouring columns of its row: one 16-byte
+// access, 64 contiguous bytes a row and request, for residual and result alike, without an exchange between lanes.
+#include <hip/hip_runtime.h>
+
+#include "device_common.h"
+#include "igemm_tail.h"
+#include "plans.h"
+
+#include <algorithm>
+
+namespace pml {
+namespace {
+
+constexpr int kThreads = 256;                    // four wavefronts
+constexpr int kRows = 16;                        // rows of a wavefront's step
+constexpr unsigned kRsrcFlags = 0x00020000u;     // raw buffer, 32-bit data format
+constexpr unsigned kOutside = 0x80000000u;       // past every buffer (all below 2 GiB), with any offset of a row's step added
+
+struct StreamArgs {
+  const void *A, *A2, *Bt, *Bt2, *res, *init, *init2;
+  void* C;
+  int64_t lda, lda2, ldbt, ldbt2, ldc, ldr;
+  int M, N, K, K2;               // K2 > 0: a second product over the K-values behind the first one's (K in whole steps)
+  int relu, col_waves;           // wavefronts of a workgroup side by side in N
+  int col_blocks, row_blocks;    // workgroups side by side in N; in M
+};
+
+// KS steps of 32 K-values, NP pairs of 16-column blocks, D steps of rows in flight.
+template <int KS, int NP, int D, int OCC, bool RES, bool SECOND>
+__global__ __launch_bounds__(kThreads, OCC) void stream_kernel(StreamArgs p) {
+  warm_arguments<sizeof(StreamArgs)>();
+  const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  // workgroup ids are dealt to the XCDs one after the other: the column blocks of a row block follow each other on one XCD
+  const int x = blockIdx.x & 7, slot = blockIdx.x >> 3;
+  const int cb = slot % p.col_blocks, rb = slot / p.col_blocks * 8 + x;
+  const int cw = wave % p.col_waves, rw = wave / p.col_waves, row_waves = 4 / p.col_waves;
+  const int n0 = (cb * p.col_waves + cw) * (32 * NP);
+  if (n0 >= p.N) return;
+  const int steps = (p.M + kRows - 1) / kRows, stride = p.row_blocks * row_waves;
+
+  auto matrix = [](const void* at, int rows, int64_t pitch, int cols) {
+    return __builtin_amdgcn_make_buffer_rsrc((void*)at, 0, at ? (int)(((int64_t)(rows - 1) * pitch + cols) * 2) : 0, kRsrcFlags);
+  };
+  const __amdgpu_buffer_rsrc_t ra = matrix(p.A, p.M, p.lda, p.K), rbt = matrix(p.Bt, p.N, p.ldbt, p.K), rc = matrix(p.C, p.M, p.ldc, p.N);
+  const __amdgpu_buffer_rsrc_t rr = matrix(p.res, p.M, p.ldr, p.N), ra2 = matrix(p.A2, p.M, p.lda2, p.K2), rbt2 = matrix(p.Bt2, p.N, p.ldbt2, p.K2);
+  auto fetch = [](__amdgpu_buffer_rsrc_t from, bool ok, unsigned at) {
+    return __builtin_bit_cast(i32x4_t, __builtin_amdgcn_raw_buffer_load_b128(from, (int)(ok ? at : kOutside), 0, 0));
+  };
+  const int k1 = SECOND ? p.K : 32 * KS;  // the K-value the second product begins at
+
+  i32x4_t fb[NP][2][KS];
+  f32x4_t bias[NP][2];
+#pragma unroll
+  for (int q = 0; q < NP; ++q)
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      const int n = n0 + 32 * q + 8 * (r >> 2) + 4 * b + (r & 3);
+#pragma unroll
+      for (int k = 0; k < KS; ++k) {
+        const int kk = 32 * k + 8 * g;
+        if (SECOND && 32 * k >= k1) fb[q][b][k] = fetch(rbt2, n < p.N && kk - k1 < p.K2, (unsigned)(n * (int)p.ldbt2 + kk - k1) * 2);
+        else fb[q][b][k] = fetch(rbt, n < p.N && kk < p.K, (unsigned)(n * (int)p.ldbt + kk) * 2);
+      }
+    }
+
+  // (sums start from the initial values of their columns)
+  auto column_vector = [&](const void* src, int q, float (&out)[8]) {
+    const int col = n0 + 32 * q + 8 * g;
+    unpack_bf16x8(src != nullptr && col < p.N ? *(const i32x4_t*)((const uint16_t*)src + col) : i32x4_t{0, 0, 0, 0}, out);
+  };
+#pragma unroll
+  for (int q = 0; q < NP; ++q) {
+    float one[8], two[8];
+    column_vector(p.init, q, one);
+    column_vector(p.init2, q, two);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) bias[q][e >> 2][e & 3] = one[e] + two[e];
+  }
+
+  const unsigned a_lane = (unsigned)(r * (int)p.lda + 8 * g) * 2, a2_lane = (unsigned)(r * (int)p.lda2 + 8 * g - k1) * 2;
+  const unsigned r_lane = (unsigned)(r * (int)p.ldr + n0 + 8 * g) * 2, c_lane = (unsigned)(r * (int)p.ldc + n0 + 8 * g) * 2;
+  const int k_left = p.K - 8 * g, k2_left = k1 + p.K2 - 8 * g, n_left = p.N - n0 - 8 * g;
+  auto rows_at = [](unsigned lane_at, int step, int64_t pitch) { return lane_at + (unsigned)step * (unsigned)(kRows * 2 * (int)pitch); };
+  i32x4_t fa[D][KS], res[D][RES ? NP : 1];
+  auto request = [&](int d, int step) {
+    const bool live = step < steps;
+    const unsigned a_at = rows_at(a_lane, step, p.lda), a2_at = rows_at(a2_lane, step, p.lda2), r_at = rows_at(r_lane, step, p.ldr);
+#pragma unroll
+    for (int k = 0; k < KS; ++k) {
+      if (SECOND && 32 * k >= k1) fa[d][k] = fetch(ra2, live & (32 * k < k2_left), a2_at + 64 * k);
+      else fa[d][k] = fetch(ra, live & (32 * k < k_left), a_at + 64 * k);
+    }
+    if constexpr (RES) {
+#pragma unroll
+      for (int q = 0; q < NP; ++q) res[d][q] = fetch(rr, live & (32 * q < n_left), r_at + 64 * q);
+    }
+  };
+
+  const int first = rb * row_waves + rw;
+#pragma unroll
+  for (int d = 0; d < D; ++d) request(d, first + d * stride);
+  const float lo = p.relu ? 0.f : -__builtin_inff();  // relu as a lower clamp (the IEEE maximum keeps a NaN)
+  for (int step0 = first; step0 < steps; step0 += D * stride) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      const int step = step0 + d * stride;
+      f32x4_t acc[NP][2];
+#pragma unroll
+      for (int q = 0; q < NP; ++q)
+#pragma unroll
+        for (int b = 0; b < 2; ++b) acc[q][b] = bias[q][b];
+#pragma unroll
+      for (int k = 0; k < KS; ++k)
+#pragma unroll
+        for (int q = 0; q < NP; ++q)
+#pragma unroll
+          for (int b = 0; b < 2; ++b) {
+            bf16x8_t av, bv;
+            __builtin_memcpy(&av, &fa[d][k], 16);
+            __builtin_memcpy(&bv, &fb[q][b][k], 16);
+            acc[q][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bv, av, acc[q][b], 0, 0, 0);
+          }
+      const bool live = step < steps;
+      const unsigned c_at = rows_at(c_lane, step, p.ldc);
+#pragma unroll
+      for (int q = 0; q < NP; ++q) {
+        float v[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = acc[q][e >> 2][e & 3];
+        if constexpr (RES) {
+          // the contraction result is rounded first, then the bf16 addition rounds again
+          float f[8];
+          unpack_bf16x8(res[d][q], f);
+#pragma unroll
+          for (int e = 0; e < 8; e += 2) round_pair_to_bf16(v[e], v[e + 1]);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) v[e] += f[e];
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = __builtin_elementwise_maximum(v[e], lo);
+        const i32x4_t out = pack_bf16x8(v);
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_tail_t, out), rc, (int)(live & (32 * q < n_left) ? c_at + 64 * q : kOutside), 0, 0);
+      }
+      request(d, step + D * stride);
+    }
+  }
+}
+
+template <int KS, int NP, int D, int OCC, bool SECOND = false>
+hipError_t launch(StreamArgs& a, int n_cus, hipStream_t s) {
+  const int groups = (a.N + 32 * NP - 1) / (32 * NP);
+  a.col_waves = groups >= 3 ? 4 : groups;
+  a.col_blocks = (groups + a.col_waves - 1) / a.col_waves;
+  const int steps = (a.M + kRows - 1) / kRows, row_waves = 4 / a.col_waves;
+  // as many workgroups as stay on the device together, no more than there are steps, rows in whole rounds of XCDs
+  const int rows = std::min(n_cus * OCC / a.col_blocks, (steps + row_waves - 1) / row_waves);
+  a.row_blocks = std::max(8, (rows + 7) / 8 * 8);
+  const dim3 grid((unsigned)(a.row_blocks * a.col_blocks));
+  if (a.res) hipLaunchKernelGGL((stream_kernel<KS, NP, D, OCC, true, SECOND>), grid, dim3(kThreads), 0, s, a);
+  else hipLaunchKernelGGL((stream_kernel<KS, NP, D, OCC, false, SECOND>), grid, dim3(kThreads), 0, s, a);
+  return hipGetLastError();
+}
+
+}  // namespace
+
+// Whether a bf16 product with the LDS tile `cfg` (a 1x1 convolution with every pixel in its place is one, too) streams its
+// rows instead.  It pays once a wavefront has several steps to spread its start over (its columns of the right-hand side, one
+// load and one MFMA chain that nothing covers): from 130 products with and without a residual, microseconds, tile -> stream,
+//   K = 32     25088 x 256  9.2 ->  8.4     25088 x 1024  24.3 -> 15.9     401408 x 64  30.5 -> 17.7     401408 x 256  71 ->  40
+//   K = 64     25088 x 256  9.2 (12.0)      25088 x 1024  25.0 -> 20.6     401408 x 64  31.0 -> 22.1     401408 x 256  75 ->  47 (residual 127 -> 97)
+//   K = 128    25088 x 512 15.9 (16.8)      25088 x 1024  27.6 -> 23.4     100352 x 64  11.8 (12.2)      100352 x 512  45 ->  32 (residual  65 -> 46)
+//   K = 200    25088 x 256 11.6 (12.4)      25088 x 1024  35.1 -> 28.4     100352 x 64  16.7 -> 13.7     401408 x 256 153 ->  99 (residual 195 -> 135)
+//   K = 256    100352 x 64 16.2 (18.5)      25088 x 1024  33.0 (37.7)      401408 x 64  54.6 -> 46.0     100352 x 512  56 (60)
+// Rows that are a multiple of 512 bytes apart come in slower (the 16 rows of a request fall into the same banks of L1): such a
+// product takes the tile unless nearly all of its bytes are the left-hand side.
+bool stream_takes(int cfg, bool conv, const IgemmArgs& g) {
+  if (!g.stream || g.b_kn || cfg == TILE_16x16_W8 || cfg == TILE_32x32_W8 || (cfg == TILE_64x64_KSPLIT && g.ws)) return false;
+  if (conv && (g.KH != 1 || g.KW != 1 || g.SH != 1 || g.SW != 1 || g.PH != 0 || g.PW != 0 || g.OH != g.H || g.OW != g.W || g.pix_pitch != 0 ||
+               g.b_raw != 0 || g.pool != 0 || g.K2 != 0))
+    return false;
+  const int64_t K = conv ? g.CI : g.K, lda = conv ? g.CI : g.lda;
+  if (K > 256 || K % 8 != 0 || lda % 8 != 0 || g.ldbt % 8 != 0 || g.N % 8 != 0 || (((uintptr_t)g.A | (uintptr_t)g.Bt) & 15) != 0) return false;
+  if (g.K2 > 0 && (K % 32 != 0 || K + g.K2 > 128 || g.K2 % 8 != 0 || g.lda2 % 8 != 0 || g.ldbt2 % 8 != 0 || (((uintptr_t)g.A2 | (uintptr_t)g.Bt2) & 15) != 0 ||
+                   (g.g2_stride > 0 && (g.g2_stride != 1 || g.g2_h * g.g2_w != g.g2_ohw))))
+    return false;
+  // the common tails: relu?(sum + column vectors), relu?(bf16(sum + column vectors) + residual)
+  if (g.out_dtype != PML_HIP_BF16 || (g.tail_mode != 1 && g.tail_mode != 2) || g.ldc % 8 != 0 || ((uintptr_t)g.C & 15) != 0) return false;
+  if (g.init && !(g.init_rs == 0 && g.init_cs == 1 && g.init_dtype == PML_HIP_BF16 && ((uintptr_t)g.init & 15) == 0)) return false;
+  if (g.init2 && ((uintptr_t)g.init2 & 15) != 0) return false;
+  const int64_t ldr = g.tail_mode == 2 ? g.tail.operand_row_stride[0] : 0;
+  if (ldr % 8 != 0 || ldr < 0 || (g.tail_mode == 2 && ((uintptr_t)g.operands[0] & 15) != 0)) return false;
+  const int64_t groups = K + g.K2 <= 128 ? (g.N + 127) / 128 : (g.N + 63) / 64, steps = (g.M + kRows - 1) / kRows * groups;
+  if (K + g.K2 > 128 && lda % 256 == 0 ? g.N > 128 || steps < 20000 : steps < (K + g.K2 <= 32 ? 4600 : 8700)) return false;
+  // byte offsets of 31 bits, also for the steps a wavefront looks ahead
+  const int64_t limit = ((int64_t)1 << 30) - 1;
+  return (g.M + 64) * std::max({lda, g.ldc, ldr, g.K2 > 0 ? g.lda2 : 0}) <= limit && g.N * std::max(g.ldbt, g.K2 > 0 ? g.ldbt2 : 0) <= limit;
+}
+
+hipError_t stream_launch(bool conv, const IgemmArgs& g, hipStream_t s) {
+  StreamArgs a;
+  a.A = g.A, a.Bt = g.Bt, a.res = g.tail_mode == 2 ? g.operands[0] : nullptr, a.init = g.init, a.init2 = g.init2, a.C = g.C;
+  a.lda = conv ? g.CI : g.lda, a.ldbt = g.ldbt, a.ldc = g.ldc, a.ldr = a.res ? g.tail.operand_row_stride[0] : 0;
+  a.M = (int)g.M, a.N = (int)g.N, a.K = (int)(conv ? g.CI : g.K), a.K2 = (int)g.K2;
+  a.A2 = g.K2 > 0 ? g.A2 : nullptr, a.Bt2 = g.K2 > 0 ? g.Bt2 : nullptr, a.lda2 = g.lda2, a.ldbt2 = g.ldbt2;
+  a.relu = g.tail_relu;
+  if (a.K2 > 0) return launch<4, 4, 1, 2, true>(a, g.n_cus, s);
+  if (a.K <= 64) return launch<2, 4, 2, 3>(a, g.n_cus, s);
+  if (a.K <= 128) return launch<4, 4, 1, 2>(a, g.n_cus, s);
+  return launch<8, 2, 1, 2>(a, g.n_cus, s);
+}
+
+}  // namespace pml
