@@ -975,6 +975,17 @@ static bool reads_b_as_given(const pml_hip_gemm_desc& d, int mfma_kind, const vo
   return true;
 }
 
+// Whether a launch streams its rows past the [K][N] right-hand side `b` as it lies, with the arguments then changed to that.
+static bool streams_given(int mfma_kind, int tile, bool conv, const void* b, int64_t ldb, IgemmArgs& g) {
+  if (mfma_kind != KIND_BF16) return false;
+  const void* const bt = g.Bt;
+  const int64_t ldbt = g.ldbt;
+  g.Bt = b, g.ldbt = ldb, g.b_kn = 1;
+  if (stream_takes(tile, conv, g)) return true;
+  g.Bt = bt, g.ldbt = ldbt, g.b_kn = 0;
+  return false;
+}
+
 static int gemm_run(const pml_hip_gemm_desc& d, int mfma_kind, int tile, const DirectTiles& direct, void* bt, int64_t bt_ld, bool packed,
                     const void* a, const void* b, void* c, const void* init, const void* const* operands,
                     void* const* outs, pml_hip_stream s, const SecondProduct* second = nullptr, bool bt_is_split = false,
@@ -997,8 +1008,7 @@ static int gemm_run(const pml_hip_gemm_desc& d, int mfma_kind, int tile, const D
   }
   const bool packed_kn = bt_is_kn && !b;
   const bool b_as_given = packed_kn || reads_b_as_given(d, mfma_kind, b, tile);
-  if (b && !d.b_layout && !b_as_given && check(transpose_pack(es, b, bt, d.k, d.n, d.ldb, bt_ld, (hipStream_t)s), "transpose_pack"))
-    return 1;
+  const bool transposed = b && !d.b_layout && !b_as_given;
   if (d.k2 > 0) {
     if (!second || !second->a2) return fail("gemm_invoke: the plan has a second product: use pml_hip_gemm_invoke2");
     if (!second->b2 && (!second->packed2 || d.b_layout)) return fail("gemm_invoke2: b2 is null and no packed right-hand side exists");
@@ -1066,6 +1076,10 @@ static int gemm_run(const pml_hip_gemm_desc& d, int mfma_kind, int tile, const D
     if (d.tail.ops[i].opcode == PML_HIP_EPI_STORE && !g.outs[d.tail.ops[i].operand])
       return fail("gemm_invoke: missing extra output");
   if (split_plan && !b_split) split_args(split_plan, g);  // (the K split over workgroups is not built for a right-hand side packed split)
+  // (rows that stream take a [K][N] right-hand side as it lies, too)
+  if (transposed && !(!packed && streams_given(mfma_kind, tile, false, b, d.ldb, g)) &&
+      check(transpose_pack(es, b, bt, d.k, d.n, d.ldb, bt_ld, (hipStream_t)s), "transpose_pack"))
+    return 1;
   return check(igemm_launch(b_split ? KIND_F32X3P : mfma_kind, tile, false, g, (hipStream_t)s), "igemm_launch");
 }
 
@@ -1304,11 +1318,6 @@ int pml_hip_conv2d_invoke(int64_t plan, const void* input, const void* filter, v
   const int64_t K = d.kh * d.kw * d.ci;
   // the HWCK filter is a row-major [K][CO] matrix; the pipelined resident-filter kernel transposes it itself
   const bool raw_filter = filter && p->halo_lds && p->halo_variant && p->mfma_kind != KIND_I8;
-  if (filter && !raw_filter && check(pack_conv_filter(p, filter, (hipStream_t)s), "pack_conv_filter")) return 1;
-  // (a filter that arrives with the call replaces the packed one; its register-order copy follows it)
-  if (filter && !raw_filter && p->reg_image &&
-      check(regfilter_image_launch(p->bt, p->bt_ld * es, p->reg_image, (hipStream_t)s), "regfilter_image_launch"))
-    return 1;
   IgemmArgs g;
   conv_args(p, g);
   if (raw_filter) {
@@ -1339,6 +1348,14 @@ int pml_hip_conv2d_invoke(int64_t plan, const void* input, const void* filter, v
   for (int i = 0; i < d.tail.n_ops; ++i)
     if (d.tail.ops[i].opcode == PML_HIP_EPI_STORE && !g.outs[d.tail.ops[i].operand])
       return fail("conv2d_invoke: missing extra output");
+  const int tile = p->tile_direct >= 0 ? p->tile_direct : p->tile;
+  // (a 1x1 convolution whose rows stream takes the filter as it lies; a packed one stays what later calls use)
+  const bool given_filter = filter && !p->packed && !p->patches && !p->via_s2d && !p->halo_lds && streams_given(p->mfma_kind, tile, true, filter, d.co, g);
+  if (filter && !raw_filter && !given_filter) {
+    if (check(pack_conv_filter(p, filter, (hipStream_t)s), "pack_conv_filter")) return 1;
+    // (a filter that arrives with the call replaces the packed one; its register-order copy follows it)
+    if (p->reg_image && check(regfilter_image_launch(p->bt, p->bt_ld * es, p->reg_image, (hipStream_t)s), "regfilter_image_launch")) return 1;
+  }
   if (p->patches) {
     Im2colArgs ic;
     ic.in = input;
@@ -1390,7 +1407,6 @@ int pml_hip_conv2d_invoke(int64_t plan, const void* input, const void* filter, v
     g.CI = (int)(d.kw * d.ci);
     g.KW = 1;
   }
-  const int tile = p->tile_direct >= 0 ? p->tile_direct : p->tile;
   return check(igemm_launch(p->b_split ? KIND_F32X3P : p->mfma_kind, tile, true, g, (hipStream_t)s), "igemm_launch");
 }
 

@@ -12,6 +12,12 @@
 // The MFMAs are the 16 x 16 ones with the right-hand side as the row operand.  Row i of block b of a pair holds column
 // 8 (i / 4) + 4 b + i % 4 of the pair's 32, so that a lane ends with eight neighbouring columns of its row: one 16-byte
 // access, 64 contiguous bytes a row and request, for residual and result alike, without an exchange between lanes.
+//
+// KN: a right-hand side that arrives as [K][N] is read as it lies, once: four neighbouring columns of every K-row per lane,
+// turned with v_perm into the fragments of four blocks, block j of 64 columns holding the columns 4 i + j; a lane then ends
+// with 16 neighbouring columns.  RAGGED: rows of results that begin and end anywhere; a lane's eight columns are one store
+// wherever they lie, value by value behind the last whole eight, and residual values are fetched as the aligned words around
+// them and shifted together.
 #include <hip/hip_runtime.h>
 
 #include "device_common.h"
@@ -38,7 +44,7 @@ struct StreamArgs {
 };
 
 // KS steps of 32 K-values, NP pairs of 16-column blocks, D steps of rows in flight.
-template <int KS, int NP, int D, int OCC, bool RES, bool SECOND>
+template <int KS, int NP, int D, int OCC, bool RES, bool SECOND, bool KN, bool RAGGED>
 __global__ __launch_bounds__(kThreads, OCC) void stream_kernel(StreamArgs p) {
   warm_arguments<sizeof(StreamArgs)>();
   const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
@@ -51,35 +57,77 @@ __global__ __launch_bounds__(kThreads, OCC) void stream_kernel(StreamArgs p) {
   if (n0 >= p.N) return;
   const int steps = (p.M + kRows - 1) / kRows, stride = p.row_blocks * row_waves;
 
+  // (from the word the matrix begins in to the end of the word it ends in: a word that is partly outside reads as zero)
   auto matrix = [](const void* at, int rows, int64_t pitch, int cols) {
-    return __builtin_amdgcn_make_buffer_rsrc((void*)at, 0, at ? (int)(((int64_t)(rows - 1) * pitch + cols) * 2) : 0, kRsrcFlags);
+    const int odd = KN || RAGGED ? (int)((uintptr_t)at & 2) : 0;
+    return __builtin_amdgcn_make_buffer_rsrc((void*)((uintptr_t)at - odd), 0, at ? (int)((((int64_t)(rows - 1) * pitch + cols) * 2 + odd + 3) & ~3) : 0, kRsrcFlags);
   };
-  const __amdgpu_buffer_rsrc_t ra = matrix(p.A, p.M, p.lda, p.K), rbt = matrix(p.Bt, p.N, p.ldbt, p.K), rc = matrix(p.C, p.M, p.ldc, p.N);
+  const __amdgpu_buffer_rsrc_t ra = matrix(p.A, p.M, p.lda, p.K), rbt = KN ? matrix(p.Bt, p.K, p.ldbt, p.N) : matrix(p.Bt, p.N, p.ldbt, p.K);
+  const __amdgpu_buffer_rsrc_t rc = matrix(p.C, p.M, p.ldc, p.N);
   const __amdgpu_buffer_rsrc_t rr = matrix(p.res, p.M, p.ldr, p.N), ra2 = matrix(p.A2, p.M, p.lda2, p.K2), rbt2 = matrix(p.Bt2, p.N, p.ldbt2, p.K2);
   auto fetch = [](__amdgpu_buffer_rsrc_t from, bool ok, unsigned at) {
     return __builtin_bit_cast(i32x4_t, __builtin_amdgcn_raw_buffer_load_b128(from, (int)(ok ? at : kOutside), 0, 0));
   };
   const int k1 = SECOND ? p.K : 32 * KS;  // the K-value the second product begins at
 
+  // the first of a lane's columns, how far the eight results of pair q lie behind it, where they are among the accumulators
+  const int col0 = n0 + (KN ? 16 : 8) * g;
+  constexpr auto behind = [](int q) constexpr { return KN ? 64 * (q >> 1) + 8 * (q & 1) : 32 * q; };
+  constexpr auto pair_of = [](int q, int e) constexpr { return KN ? (q & ~1) + ((e & 3) >> 1) : q; };
+  constexpr auto block_of = [](int, int e) constexpr { return KN ? e & 1 : e >> 2; };
+  constexpr auto row_of = [](int q, int e) constexpr { return KN ? 2 * (q & 1) + (e >> 2) : e & 3; };
+
   i32x4_t fb[NP][2][KS];
-  f32x4_t bias[NP][2];
+  if constexpr (KN) {
+    typedef int i32x3_t __attribute__((ext_vector_type(3)));
+    const int odd = (int)((uintptr_t)p.Bt & 2);
 #pragma unroll
-  for (int q = 0; q < NP; ++q)
-#pragma unroll
-    for (int b = 0; b < 2; ++b) {
-      const int n = n0 + 32 * q + 8 * (r >> 2) + 4 * b + (r & 3);
+    for (int h = 0; h < NP / 2; ++h)
 #pragma unroll
       for (int k = 0; k < KS; ++k) {
-        const int kk = 32 * k + 8 * g;
-        if (SECOND && 32 * k >= k1) fb[q][b][k] = fetch(rbt2, n < p.N && kk - k1 < p.K2, (unsigned)(n * (int)p.ldbt2 + kk - k1) * 2);
-        else fb[q][b][k] = fetch(rbt, n < p.N && kk < p.K, (unsigned)(n * (int)p.ldbt + kk) * 2);
+        int chunk = 32 * k + 8 * g;
+        asm volatile("" : "+v"(chunk));  // (opaque: the offsets of all chunks worked out ahead take more registers than there are)
+        uint32_t w[8][2];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          // (row e of the chunk begins at the same half of a word in every lane: chunks are 8 rows, lanes 4 columns apart)
+          const int at = odd + e * (int)p.ldbt * 2;
+          const unsigned off = (unsigned)(chunk * (int)p.ldbt + n0 + 64 * h + 4 * r) * 2 + (unsigned)(at & ~3);
+          const i32x3_t v = __builtin_bit_cast(i32x3_t, __builtin_amdgcn_raw_buffer_load_b96(rbt, (int)(chunk + e < p.K && n0 + 64 * h + 4 * r < p.N ? off : kOutside), 0, 0));
+#pragma unroll
+          for (int d = 0; d < 2; ++d) w[e][d] = __builtin_amdgcn_alignbit((uint32_t)v[d + 1], (uint32_t)v[d], (unsigned)(at & 3) * 8);
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int d = 0; d < 4; ++d)
+            fb[2 * h + (j >> 1)][j & 1][k][d] = (int)__builtin_amdgcn_perm(w[2 * d + 1][j >> 1], w[2 * d][j >> 1], (j & 1) ? 0x07060302u : 0x05040100u);
+        if (KS > 4 || (k & 1)) __builtin_amdgcn_sched_barrier(0);  // (one or two chunks in flight: more do not fit beside the fragments)
       }
-    }
-
+  } else {
+#pragma unroll
+    for (int q = 0; q < NP; ++q)
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+        const int n = n0 + 32 * q + 8 * (r >> 2) + 4 * b + (r & 3);
+#pragma unroll
+        for (int k = 0; k < KS; ++k) {
+          const int kk = 32 * k + 8 * g;
+          if (SECOND && 32 * k >= k1) fb[q][b][k] = fetch(rbt2, n < p.N && kk - k1 < p.K2, (unsigned)(n * (int)p.ldbt2 + kk - k1) * 2);
+          else fb[q][b][k] = fetch(rbt, n < p.N && kk < p.K, (unsigned)(n * (int)p.ldbt + kk) * 2);
+        }
+      }
+  }
   // (sums start from the initial values of their columns)
+  f32x4_t bias[NP][2];
   auto column_vector = [&](const void* src, int q, float (&out)[8]) {
-    const int col = n0 + 32 * q + 8 * g;
-    unpack_bf16x8(src != nullptr && col < p.N ? *(const i32x4_t*)((const uint16_t*)src + col) : i32x4_t{0, 0, 0, 0}, out);
+    const int col = col0 + behind(q);
+    if constexpr (RAGGED) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) out[e] = src != nullptr && col + e < p.N ? bf16_bits_to_f32(((const uint16_t*)src)[col + e]) : 0.f;
+    } else {
+      unpack_bf16x8(src != nullptr && col < p.N ? *(const i32x4_t*)((const uint16_t*)src + col) : i32x4_t{0, 0, 0, 0}, out);
+    }
   };
 #pragma unroll
   for (int q = 0; q < NP; ++q) {
@@ -87,14 +135,15 @@ __global__ __launch_bounds__(kThreads, OCC) void stream_kernel(StreamArgs p) {
     column_vector(p.init, q, one);
     column_vector(p.init2, q, two);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) bias[q][e >> 2][e & 3] = one[e] + two[e];
+    for (int e = 0; e < 8; ++e) bias[pair_of(q, e)][block_of(q, e)][row_of(q, e)] = one[e] + two[e];
   }
 
   const unsigned a_lane = (unsigned)(r * (int)p.lda + 8 * g) * 2, a2_lane = (unsigned)(r * (int)p.lda2 + 8 * g - k1) * 2;
-  const unsigned r_lane = (unsigned)(r * (int)p.ldr + n0 + 8 * g) * 2, c_lane = (unsigned)(r * (int)p.ldc + n0 + 8 * g) * 2;
-  const int k_left = p.K - 8 * g, k2_left = k1 + p.K2 - 8 * g, n_left = p.N - n0 - 8 * g;
+  const unsigned r_lane = (unsigned)(r * (int)p.ldr + col0) * 2 + (RAGGED ? (unsigned)((uintptr_t)p.res & 2) : 0u), c_lane = (unsigned)(r * (int)p.ldc + col0) * 2;
+  const int k_left = p.K - 8 * g, k2_left = k1 + p.K2 - 8 * g, n_left = p.N - col0;
   auto rows_at = [](unsigned lane_at, int step, int64_t pitch) { return lane_at + (unsigned)step * (unsigned)(kRows * 2 * (int)pitch); };
   i32x4_t fa[D][KS], res[D][RES ? NP : 1];
+  uint32_t res_end[D][RES && RAGGED ? NP : 1];
   auto request = [&](int d, int step) {
     const bool live = step < steps;
     const unsigned a_at = rows_at(a_lane, step, p.lda), a2_at = rows_at(a2_lane, step, p.lda2), r_at = rows_at(r_lane, step, p.ldr);
@@ -105,7 +154,12 @@ __global__ __launch_bounds__(kThreads, OCC) void stream_kernel(StreamArgs p) {
     }
     if constexpr (RES) {
 #pragma unroll
-      for (int q = 0; q < NP; ++q) res[d][q] = fetch(rr, live & (32 * q < n_left), r_at + 64 * q);
+      for (int q = 0; q < NP; ++q) {
+        const bool in = live & (behind(q) < n_left);
+        const unsigned at = (r_at & (RAGGED ? ~3u : ~0u)) + 2 * behind(q);
+        res[d][q] = fetch(rr, in, at);
+        if constexpr (RAGGED) res_end[d][q] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rr, (int)(in ? at + 16 : kOutside), 0, 0);
+      }
     }
   };
 
@@ -139,11 +193,18 @@ __global__ __launch_bounds__(kThreads, OCC) void stream_kernel(StreamArgs p) {
       for (int q = 0; q < NP; ++q) {
         float v[8];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] = acc[q][e >> 2][e & 3];
+        for (int e = 0; e < 8; ++e) v[e] = acc[pair_of(q, e)][block_of(q, e)][row_of(q, e)];
         if constexpr (RES) {
           // the contraction result is rounded first, then the bf16 addition rounds again
           float f[8];
-          unpack_bf16x8(res[d][q], f);
+          i32x4_t bits = res[d][q];
+          if constexpr (RAGGED) {
+            const unsigned shift = (rows_at(r_lane, step, p.ldr) & 3) * 8;
+#pragma unroll
+            for (int w = 0; w < 4; ++w)
+              bits[w] = (int)__builtin_amdgcn_alignbit(w < 3 ? (uint32_t)res[d][q][w < 3 ? w + 1 : 3] : res_end[d][q], (uint32_t)res[d][q][w], shift);
+          }
+          unpack_bf16x8(bits, f);
 #pragma unroll
           for (int e = 0; e < 8; e += 2) round_pair_to_bf16(v[e], v[e + 1]);
 #pragma unroll
@@ -152,14 +213,28 @@ __global__ __launch_bounds__(kThreads, OCC) void stream_kernel(StreamArgs p) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[e] = __builtin_elementwise_maximum(v[e], lo);
         const i32x4_t out = pack_bf16x8(v);
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_tail_t, out), rc, (int)(live & (32 * q < n_left) ? c_at + 64 * q : kOutside), 0, 0);
+        if constexpr (RAGGED) {
+          const int left = n_left - behind(q);
+          if (step * kRows + r < p.M && live && left > 0) {
+            unsigned char* const to = (unsigned char*)p.C + (c_at + 2 * behind(q));
+            if (left >= 8) {
+              __builtin_memcpy(to, &out, 16);
+            } else {
+#pragma unroll
+              for (int e = 0; e < 7; ++e)
+                if (e < left) *(uint16_t*)(to + 2 * e) = (uint16_t)((uint32_t)out[e >> 1] >> (16 * (e & 1)));
+            }
+          }
+        } else {
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_tail_t, out), rc, (int)(live & (behind(q) < n_left) ? c_at + 2 * behind(q) : kOutside), 0, 0);
+        }
       }
       request(d, step + D * stride);
     }
   }
 }
 
-template <int KS, int NP, int D, int OCC, bool SECOND = false>
+template <int KS, int NP, int D, int OCC, bool SECOND, bool KN, bool RAGGED>
 hipError_t launch(StreamArgs& a, int n_cus, hipStream_t s) {
   const int groups = (a.N + 32 * NP - 1) / (32 * NP);
   a.col_waves = groups >= 3 ? 4 : groups;
@@ -169,9 +244,26 @@ hipError_t launch(StreamArgs& a, int n_cus, hipStream_t s) {
   const int rows = std::min(n_cus * OCC / a.col_blocks, (steps + row_waves - 1) / row_waves);
   a.row_blocks = std::max(8, (rows + 7) / 8 * 8);
   const dim3 grid((unsigned)(a.row_blocks * a.col_blocks));
-  if (a.res) hipLaunchKernelGGL((stream_kernel<KS, NP, D, OCC, true, SECOND>), grid, dim3(kThreads), 0, s, a);
-  else hipLaunchKernelGGL((stream_kernel<KS, NP, D, OCC, false, SECOND>), grid, dim3(kThreads), 0, s, a);
+  if (a.res) hipLaunchKernelGGL((stream_kernel<KS, NP, D, OCC, true, SECOND, KN, RAGGED>), grid, dim3(kThreads), 0, s, a);
+  else hipLaunchKernelGGL((stream_kernel<KS, NP, D, OCC, false, SECOND, KN, RAGGED>), grid, dim3(kThreads), 0, s, a);
   return hipGetLastError();
+}
+
+template <bool KN, bool RAGGED>
+hipError_t launch_k(StreamArgs& a, int n_cus, hipStream_t s) {
+  if constexpr (!KN && !RAGGED)
+    if (a.K2 > 0) return launch<4, 4, 1, 2, true, KN, RAGGED>(a, n_cus, s);
+  if (a.K <= 64) return launch<2, 4, 2, 2, false, KN, RAGGED>(a, n_cus, s);
+  if (a.K <= 128) return launch<4, KN ? 2 : 4, KN ? 2 : 1, 2, false, KN, RAGGED>(a, n_cus, s);
+  if constexpr (KN) return hipErrorInvalidValue;  // (not built: its fragments and the rows they are turned from do not fit together)
+  else return launch<8, 2, 1, 2, false, KN, RAGGED>(a, n_cus, s);
+}
+
+// Whether result or residual rows do not begin and end on 16 bytes, or the column vectors do not.
+bool ragged(const IgemmArgs& g) {
+  const int64_t ldr = g.tail_mode == 2 ? g.tail.operand_row_stride[0] : 0;
+  return ((g.N | g.ldc | ldr) & 7) != 0 ||
+         (((uintptr_t)g.C | (uintptr_t)g.init | (uintptr_t)g.init2 | (g.tail_mode == 2 ? (uintptr_t)g.operands[0] : 0)) & 15) != 0;
 }
 
 }  // namespace
@@ -185,28 +277,34 @@ hipError_t launch(StreamArgs& a, int n_cus, hipStream_t s) {
 //   K = 200    25088 x 256 11.6 (12.4)      25088 x 1024  35.1 -> 28.4     100352 x 64  16.7 -> 13.7     401408 x 256 153 ->  99 (residual 195 -> 135)
 //   K = 256    100352 x 64 16.2 (18.5)      25088 x 1024  33.0 (37.7)      401408 x 64  54.6 -> 46.0     100352 x 512  56 (60)
 // Rows that are a multiple of 512 bytes apart come in slower (the 16 rows of a request fall into the same banks of L1): such a
-// product takes the tile unless nearly all of its bytes are the left-hand side.
+// product takes the tile unless nearly all of its bytes are the left-hand side.  A [K][N] right-hand side that is read as it
+// lies saves the launch that transposes it, and odd rows of results cost a tile its straight tail (with that launch):
+//   K = 64     25088 x 128  8.2 ->  6.8     25088 x 256  11.1 ->  8.3    25088 x 251  15.7 -> 12.9     401408 x 123  63 -> 40
+//   K = 128    25088 x 128  9.0 ->  7.5     25088 x 256  12.1 -> 10.3    25088 x 251  16.3 -> 12.9     100352 x 510  61 -> 46
 bool stream_takes(int cfg, bool conv, const IgemmArgs& g) {
-  if (!g.stream || g.b_kn || cfg == TILE_16x16_W8 || cfg == TILE_32x32_W8 || (cfg == TILE_64x64_KSPLIT && g.ws)) return false;
+  if (!g.stream || cfg == TILE_16x16_W8 || cfg == TILE_32x32_W8 || (cfg == TILE_64x64_KSPLIT && g.ws)) return false;
   if (conv && (g.KH != 1 || g.KW != 1 || g.SH != 1 || g.SW != 1 || g.PH != 0 || g.PW != 0 || g.OH != g.H || g.OW != g.W || g.pix_pitch != 0 ||
                g.b_raw != 0 || g.pool != 0 || g.K2 != 0))
     return false;
   const int64_t K = conv ? g.CI : g.K, lda = conv ? g.CI : g.lda;
-  if (K > 256 || K % 8 != 0 || lda % 8 != 0 || g.ldbt % 8 != 0 || g.N % 8 != 0 || (((uintptr_t)g.A | (uintptr_t)g.Bt) & 15) != 0) return false;
-  if (g.K2 > 0 && (K % 32 != 0 || K + g.K2 > 128 || g.K2 % 8 != 0 || g.lda2 % 8 != 0 || g.ldbt2 % 8 != 0 || (((uintptr_t)g.A2 | (uintptr_t)g.Bt2) & 15) != 0 ||
+  if (K > 256 || K % 8 != 0 || lda % 8 != 0 || ((uintptr_t)g.A & 15) != 0) return false;
+  if (g.b_kn ? K > 128 || ((uintptr_t)g.Bt & 1) != 0 : g.ldbt % 8 != 0 || ((uintptr_t)g.Bt & 15) != 0) return false;
+  const bool odd_rows = ragged(g);
+  if (g.K2 > 0 && (g.b_kn || odd_rows || K % 32 != 0 || K + g.K2 > 128 || g.K2 % 8 != 0 || g.lda2 % 8 != 0 || g.ldbt2 % 8 != 0 || (((uintptr_t)g.A2 | (uintptr_t)g.Bt2) & 15) != 0 ||
                    (g.g2_stride > 0 && (g.g2_stride != 1 || g.g2_h * g.g2_w != g.g2_ohw))))
     return false;
   // the common tails: relu?(sum + column vectors), relu?(bf16(sum + column vectors) + residual)
-  if (g.out_dtype != PML_HIP_BF16 || (g.tail_mode != 1 && g.tail_mode != 2) || g.ldc % 8 != 0 || ((uintptr_t)g.C & 15) != 0) return false;
-  if (g.init && !(g.init_rs == 0 && g.init_cs == 1 && g.init_dtype == PML_HIP_BF16 && ((uintptr_t)g.init & 15) == 0)) return false;
-  if (g.init2 && ((uintptr_t)g.init2 & 15) != 0) return false;
+  if (g.out_dtype != PML_HIP_BF16 || (g.tail_mode != 1 && g.tail_mode != 2) || ((uintptr_t)g.C & 1) != 0) return false;
+  if (g.init && !(g.init_rs == 0 && g.init_cs == 1 && g.init_dtype == PML_HIP_BF16 && ((uintptr_t)g.init & 1) == 0)) return false;
+  if (g.init2 && ((uintptr_t)g.init2 & 1) != 0) return false;
   const int64_t ldr = g.tail_mode == 2 ? g.tail.operand_row_stride[0] : 0;
-  if (ldr % 8 != 0 || ldr < 0 || (g.tail_mode == 2 && ((uintptr_t)g.operands[0] & 15) != 0)) return false;
-  const int64_t groups = K + g.K2 <= 128 ? (g.N + 127) / 128 : (g.N + 63) / 64, steps = (g.M + kRows - 1) / kRows * groups;
-  if (K + g.K2 > 128 && lda % 256 == 0 ? g.N > 128 || steps < 20000 : steps < (K + g.K2 <= 32 ? 4600 : 8700)) return false;
+  if (ldr < 0 || (g.tail_mode == 2 && (((uintptr_t)g.operands[0] & 1) != 0 || g.tail.operand_col_stride[0] != 1))) return false;
+  const int64_t kk = K + g.K2, groups = kk <= (g.b_kn ? 64 : 128) ? (g.N + 127) / 128 : (g.N + 63) / 64, steps = (g.M + kRows - 1) / kRows * groups;
+  if (!g.b_kn && kk > 128 && lda % 256 == 0 && g.N > (odd_rows ? 64 : 128)) return false;
+  if (steps < (g.b_kn ? 1600 : kk <= 32 ? 3000 : kk <= 128 ? 8700 : lda % 256 == 0 ? 20000 : 6200)) return false;
   // byte offsets of 31 bits, also for the steps a wavefront looks ahead
   const int64_t limit = ((int64_t)1 << 30) - 1;
-  return (g.M + 64) * std::max({lda, g.ldc, ldr, g.K2 > 0 ? g.lda2 : 0}) <= limit && g.N * std::max(g.ldbt, g.K2 > 0 ? g.ldbt2 : 0) <= limit;
+  return (g.M + 64) * std::max({lda, g.ldc, ldr, g.K2 > 0 ? g.lda2 : 0}) <= limit && (g.b_kn ? K + 8 : g.N) * std::max(g.ldbt, g.K2 > 0 ? g.ldbt2 : 0) <= limit;
 }
 
 hipError_t stream_launch(bool conv, const IgemmArgs& g, hipStream_t s) {
@@ -216,10 +314,8 @@ hipError_t stream_launch(bool conv, const IgemmArgs& g, hipStream_t s) {
   a.M = (int)g.M, a.N = (int)g.N, a.K = (int)(conv ? g.CI : g.K), a.K2 = (int)g.K2;
   a.A2 = g.K2 > 0 ? g.A2 : nullptr, a.Bt2 = g.K2 > 0 ? g.Bt2 : nullptr, a.lda2 = g.lda2, a.ldbt2 = g.ldbt2;
   a.relu = g.tail_relu;
-  if (a.K2 > 0) return launch<4, 4, 1, 2, true>(a, g.n_cus, s);
-  if (a.K <= 64) return launch<2, 4, 2, 3>(a, g.n_cus, s);
-  if (a.K <= 128) return launch<4, 4, 1, 2>(a, g.n_cus, s);
-  return launch<8, 2, 1, 2>(a, g.n_cus, s);
+  if (g.b_kn) return ragged(g) ? launch_k<true, true>(a, g.n_cus, s) : launch_k<true, false>(a, g.n_cus, s);
+  return ragged(g) ? launch_k<false, true>(a, g.n_cus, s) : launch_k<false, false>(a, g.n_cus, s);
 }
 
 }  // namespace pml

@@ -21,30 +21,57 @@ def whole(rng, shape):
     return rng.integers(-4, 5, shape).astype(np.float32)
 
 
+def run(A, B, packed, at=0, pitch=None, bias=None, res=None, relu=False):
+    """Result rows `pitch` values apart that begin `at` values behind a 16-byte boundary, and whether all else was left alone."""
+    (M, K), N = A.shape, B.shape[1]
+    pitch = pitch or N
+    d = hk.GemmDesc()
+    d.in_dtype = d.out_dtype = d.c_dtype = d.init_dtype = hk.BF16
+    d.m, d.n, d.k, d.lda, d.ldb, d.ldc, d.init_kind, d.init_col_stride = M, N, K, K, N, pitch, int(bias is not None), 1
+    ops = [(hk.EPI_ADD, hk.BF16, hk.OPND_TENSOR, 0, 0.0)] * (res is not None) + [(hk.EPI_RELU, hk.BF16, 0, 0, 0.0)] * relu
+    d.tail = hk.make_tail(ops=ops, operands=[(hk.BF16, N, 1)] * (res is not None))
+    L = hk.lib()
+    plan = L.pml_hip_gemm_dispatch(ctypes.byref(d))
+    assert plan
+    dA, dB = (hk.DeviceBuffer.from_numpy(T.bf16(x)) for x in (A, B))
+    d1, dR = (hk.DeviceBuffer.from_numpy(T.bf16(x)) if x is not None else None for x in (bias, res))
+    n = (at + M * pitch + 9) // 2 * 2
+    dC = hk.DeviceBuffer(n * 2)
+    hk.check(L.pml_hip_fill_u32(dC.ptr, 0xbeefbeef, n // 2, None))
+    if packed:
+        hk.check(L.pml_hip_gemm_pack_b(plan, dB.ptr, None))
+    for _ in range(2):
+        hk.check(L.pml_hip_gemm_invoke(plan, dA.ptr, None if packed else dB.ptr, dC.ptr + 2 * at, d1.ptr if d1 else None, hk.ptr_array([dR.ptr] if dR else []),
+                                       hk.ptr_array([]), None))
+    hk.check(L.pml_hip_stream_sync(None))
+    L.pml_hip_plan_free(plan)
+    flat = dC.to_numpy(np.uint16, (n,))
+    rows = flat[at:at + M * pitch].reshape(M, pitch)
+    assert (flat[:at] == 0xbeef).all() and (flat[at + M * pitch:] == 0xbeef).all() and (rows[:, N:] == 0xbeef).all()
+    return E.bf16_from_bits(np.ascontiguousarray(rows[:, :N]))
+
+
 # rows: one past and one short of a step, more than one round of the device; columns: fewer than a wavefront holds, that end
-# within a quarter, a pair, a wavefront, a workgroup; K: one chunk, just below, at and above each kernel's range
-@pytest.mark.parametrize('M,N,K', [(80000, 72, 8), (73000, 256, 64), (70001, 200, 72), (34832, 512, 128), (36399, 264, 136), (320001, 40, 256), (140000, 8, 248), (17000, 1160, 56)])
-def test_tails(M, N, K):
+# within eight, a quarter, a pair, a wavefront, a workgroup; K: one chunk, just below, at and above each kernel's range; result
+# rows with and without room behind them that begin on 16 bytes, a word, half a word
+@pytest.mark.parametrize('packed', [0, 1])
+@pytest.mark.parametrize('M,N,K,at,pitch', [
+    (80000, 72, 8, 0, 72), (73000, 256, 64, 0, 256), (70001, 200, 72, 0, 208), (34832, 512, 128, 0, 512), (36399, 264, 136, 0, 264), (320001, 40, 256, 0, 40),
+    (17000, 1160, 56, 0, 1160), (80000, 76, 24, 0, 76), (140000, 1, 64, 1, 1), (73000, 260, 40, 2, 263), (140001, 7, 96, 0, 9), (69999, 132, 128, 1, 132),
+    (36399, 250, 248, 3, 250), (320001, 60, 256, 0, 60)])
+def test_tails(M, N, K, at, pitch, packed):
     rng = np.random.default_rng(M + N + K)
     A, B = whole(rng, (M, K)), whole(rng, (K, N))
     S = A @ B  # at most 16 K: exact
     bias, res = whole(rng, N), whole(rng, (M, N))
     A[M - 1, K - 1] = A[0, 0] = np.inf  # (in its own row only)
+    r = E.round_bf16
     with np.errstate(invalid='ignore'):
         S[[0, M - 1]] = A[[0, M - 1]] @ B
-    r = E.round_bf16
-    relu = (hk.EPI_RELU, hk.BF16, 0, 0, 0.0)
-    bits = (T.bf16(A), T.bf16(B), hk.BF16, hk.BF16)
-    kw = dict(init=T.bf16(bias), init_strides=(0, 1), init_dt=hk.BF16, invokes=2)
-
-    def check(got, want):
-        np.testing.assert_array_equal(E.bf16_from_bits(got), want)
-    check(T.run_gemm(*bits), r(S))
-    with np.errstate(invalid='ignore'):
         keep = lambda v: np.where(v < 0, np.float32(0), v)  # (relu keeps a NaN)
-        check(T.run_gemm(*bits, tail=hk.make_tail(ops=[relu]), **kw), r(keep(S + bias)))
-        add = hk.make_tail(ops=[(hk.EPI_ADD, hk.BF16, hk.OPND_TENSOR, 0, 0.0), relu], operands=[(hk.BF16, N, 1)])
-        check(T.run_gemm(*bits, tail=add, operands=[T.bf16(res)], **kw), r(keep(r(S + bias) + res)))
+        np.testing.assert_array_equal(run(A, B, packed, at, pitch), r(S))
+        np.testing.assert_array_equal(run(A, B, packed, at, pitch, bias, relu=True), r(keep(S + bias)))
+        np.testing.assert_array_equal(run(A, B, packed, at, pitch, bias, res, True), r(keep(r(S + bias) + res)))
 
 
 @pytest.mark.parametrize('stride', [0, 1])
