@@ -150,6 +150,7 @@ __global__ __launch_bounds__(kThreads, OCC) void stream_kernel(StreamArgs p) {
 #pragma unroll
     for (int k = 0; k < KS; ++k) {
       if (SECOND && 32 * k >= k1) fa[d][k] = fetch(ra2, live & (32 * k < k2_left), a2_at + 64 * k);
+      else if constexpr (KS > 4) fa[d][k] = fetch(ra, live & (32 * (k ^ (r & 1)) < k_left), a_at + 64 * (k ^ (r & 1)));  // (put in order below)
       else fa[d][k] = fetch(ra, live & (32 * k < k_left), a_at + 64 * k);
     }
     if constexpr (RES) {
@@ -171,6 +172,20 @@ __global__ __launch_bounds__(kThreads, OCC) void stream_kernel(StreamArgs p) {
 #pragma unroll
     for (int d = 0; d < D; ++d) {
       const int step = step0 + d * stride;
+      if constexpr (KS > 4) {
+        // Rows a multiple of 512 bytes apart fall into the same banks of L1, all 16 of a request: odd rows ask for the two
+        // 64-byte halves of a line in the opposite order (25088 x 1024, K = 256 with a residual 43.9 -> 34.5 us; turning
+        // four or eight such pieces costs more in moves than it saves: 36.1, 37.4).
+#pragma unroll
+        for (int k = 0; k < KS; k += 2) {
+          const i32x4_t even = fa[d][k], odd = fa[d][k + 1];
+#pragma unroll
+          for (int w = 0; w < 4; ++w) {
+            fa[d][k][w] = (r & 1) ? odd[w] : even[w];
+            fa[d][k + 1][w] = (r & 1) ? even[w] : odd[w];
+          }
+        }
+      }
       f32x4_t acc[NP][2];
 #pragma unroll
       for (int q = 0; q < NP; ++q)
@@ -270,15 +285,14 @@ bool ragged(const IgemmArgs& g) {
 
 // Whether a bf16 product with the LDS tile `cfg` (a 1x1 convolution with every pixel in its place is one, too) streams its
 // rows instead.  It pays once a wavefront has several steps to spread its start over (its columns of the right-hand side, one
-// load and one MFMA chain that nothing covers): from 130 products with and without a residual, microseconds, tile -> stream,
+// load and one MFMA chain that nothing covers): from 130 to 485 products, microseconds, tile -> stream,
 //   K = 32     25088 x 256  9.2 ->  8.4     25088 x 1024  24.3 -> 15.9     401408 x 64  30.5 -> 17.7     401408 x 256  71 ->  40
 //   K = 64     25088 x 256  9.2 (12.0)      25088 x 1024  25.0 -> 20.6     401408 x 64  31.0 -> 22.1     401408 x 256  75 ->  47 (residual 127 -> 97)
 //   K = 128    25088 x 512 15.9 (16.8)      25088 x 1024  27.6 -> 23.4     100352 x 64  11.8 (12.2)      100352 x 512  45 ->  32 (residual  65 -> 46)
 //   K = 200    25088 x 256 11.6 (12.4)      25088 x 1024  35.1 -> 28.4     100352 x 64  16.7 -> 13.7     401408 x 256 153 ->  99 (residual 195 -> 135)
-//   K = 256    100352 x 64 16.2 (18.5)      25088 x 1024  33.0 (37.7)      401408 x 64  54.6 -> 46.0     100352 x 512  56 (60)
-// Rows that are a multiple of 512 bytes apart come in slower (the 16 rows of a request fall into the same banks of L1): such a
-// product takes the tile unless nearly all of its bytes are the left-hand side.  A [K][N] right-hand side that is read as it
-// lies saves the launch that transposes it, and odd rows of results cost a tile its straight tail (with that launch):
+//   K = 256    12544 x 1024 19.5 (20.0)     25088 x 1024  33.0 -> 29.8     401408 x 64  54.6 -> 45.2     100352 x 512  57 -> 44 (residual  82 -> 64)
+// Past K = 128, rows that are whole lines apart come in slower than others (banks of L1, above).  A [K][N] right-hand side
+// that is read as it lies saves the launch that transposes it, and odd rows of results cost a tile its straight tail:
 //   K = 64     25088 x 128  8.2 ->  6.8     25088 x 256  11.1 ->  8.3    25088 x 251  15.7 -> 12.9     401408 x 123  63 -> 40
 //   K = 128    25088 x 128  9.0 ->  7.5     25088 x 256  12.1 -> 10.3    25088 x 251  16.3 -> 12.9     100352 x 510  61 -> 46
 bool stream_takes(int cfg, bool conv, const IgemmArgs& g) {
@@ -300,8 +314,8 @@ bool stream_takes(int cfg, bool conv, const IgemmArgs& g) {
   const int64_t ldr = g.tail_mode == 2 ? g.tail.operand_row_stride[0] : 0;
   if (ldr < 0 || (g.tail_mode == 2 && (((uintptr_t)g.operands[0] & 1) != 0 || g.tail.operand_col_stride[0] != 1))) return false;
   const int64_t kk = K + g.K2, groups = kk <= (g.b_kn ? 64 : 128) ? (g.N + 127) / 128 : (g.N + 63) / 64, steps = (g.M + kRows - 1) / kRows * groups;
-  if (!g.b_kn && kk > 128 && lda % 256 == 0 && g.N > (odd_rows ? 64 : 128)) return false;
-  if (steps < (g.b_kn ? 1600 : kk <= 32 ? 3000 : kk <= 128 ? 8700 : lda % 256 == 0 ? 20000 : 6200)) return false;
+  const int64_t least = g.b_kn ? 1600 : kk <= 32 ? 3000 : kk <= 128 ? 8700 : lda % 64 != 0 ? 6200 : odd_rows || g.tail_mode == 2 ? 8700 : 20000;
+  if (steps < least) return false;
   // byte offsets of 31 bits, also for the steps a wavefront looks ahead
   const int64_t limit = ((int64_t)1 << 30) - 1;
   return (g.M + 64) * std::max({lda, g.ldc, ldr, g.K2 > 0 ? g.lda2 : 0}) <= limit && (g.b_kn ? K + 8 : g.N) * std::max(g.ldbt, g.K2 > 0 ? g.ldbt2 : 0) <= limit;
