@@ -188,9 +188,10 @@ __device__ __forceinline__ void given_tail_bf16(const IgemmArgs& p, const f32x4_
 
 // int8's requantisation chain (the straight code of tile_tail, tail_mode 4 with tail_rq, and its arithmetic) straight from the
 // accumulators: a lane's sixteen neighbouring columns are one 16-byte store, where the trip through LDS makes 4-byte ones
-// (4096^3: 66.2 us with it).
+// (4096^3: 66.2 us with it).  Not where the sums are stored as well: their rows leave in 16-byte pieces 64 bytes apart here
+// (81.7 us), and whole behind the trip through LDS.
 __device__ __forceinline__ bool requant_direct_ok(const IgemmArgs& p) {
-  if (p.tail_mode != 4 || !p.tail_rq || (p.N & 15) != 0 || (p.ldc & 15) != 0 || ((uintptr_t)p.C & 15) != 0) return false;
+  if (p.tail_mode != 4 || !p.tail_rq || p.rq_store >= 0 || (p.N & 15) != 0 || (p.ldc & 15) != 0 || ((uintptr_t)p.C & 15) != 0) return false;
   return p.init == nullptr || (p.init_rs == 0 && p.init_cs == 1 && p.init_dtype == PML_HIP_I32 && ((uintptr_t)p.init & 15) == 0);
 }
 
@@ -201,7 +202,6 @@ __device__ __forceinline__ void given_tail_requant(const IgemmArgs& p, const i32
   if (n >= p.N) return;
   const float* const scale = (const float*)p.operands[p.rq_scale];
   const bool one_scale = p.tail.operand_col_stride[p.rq_scale] == 0;
-  int* const sums = p.rq_store >= 0 ? (int*)p.outs[p.rq_store] : nullptr;
   const float lo = p.rq_lo, hi = p.rq_hi;
   f32x4_t sc[4];
   i32x4_t start[4];
@@ -220,7 +220,6 @@ __device__ __forceinline__ void given_tail_requant(const IgemmArgs& p, const i32
       i32x4_t a;
 #pragma unroll
       for (int q = 0; q < 4; ++q) a[q] = (int)((unsigned)acc[i][q][e] + (unsigned)start[e][q]);
-      if (sums) *(i32x4_t*)(sums + m * p.ldc + n + 4 * e) = a;
       uint32_t w = 0;
 #pragma unroll
       for (int q = 0; q < 4; ++q) {

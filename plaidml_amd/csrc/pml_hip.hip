@@ -878,8 +878,8 @@ static DirectTiles direct_tiles(const pml_hip_gemm_desc& d, int kind) {
 }
 
 // Whether a product's 256 x 256 tile reads B[K][N] with rows of `ldb` elements as it lies: four neighbouring columns per lane
-// and K-row, through registers (given.hip).  It is then the better form of a packed right-hand side, too: 4096^3 from the
-// [K][N] copy against the LDS kernel on Bt, bf16 104 us against 122, int8 62 against 66.
+// and K-row, through registers (given.hip).  For bf16 it is then the better form of a packed right-hand side, too: 4096^3 from
+// the [K][N] copy 104 us, from Bt through LDS 122 (int8, back to back until the clock settles: 72 and 68).
 static bool takes_b_as_given(const pml_hip_gemm_desc& d, int mfma_kind, int tile, int64_t ldb) {
   return tile == TILE_256x256_W8 && (mfma_kind == KIND_BF16 || mfma_kind == KIND_I8) && !d.b_layout && d.k2 == 0 && d.n % 4 == 0 &&
          ldb % 4 == 0 && d.k * ldb * dt_size(d.in_dtype) < ((int64_t)1 << 31);
@@ -911,7 +911,7 @@ int64_t pml_hip_gemm_dispatch(const pml_hip_gemm_desc* d) {
   const int lds_tile = p->tile;
   if (p->tile == TILE_64x64_KSPLIT && !p->ws) p->tile = TILE_64x64;  // (not worth splitting, no memory for the workspace, or not run)
   p->b_split = kind == KIND_F32X3 && !d->b_layout && d->k % 32 == 0 && !p->ws;
-  p->b_kn = p->direct.rows < 0 && takes_b_as_given(*d, kind, p->tile, d->n);
+  p->b_kn = kind == KIND_BF16 && p->direct.rows < 0 && takes_b_as_given(*d, kind, p->tile, d->n);
   if (!d->b_layout && !(p->bt = p->hold(p->bt_bytes))) {
     delete p;
     fail("gemm: cannot allocate the packed right-hand side");
@@ -945,9 +945,10 @@ struct SecondProduct {
   bool packed2 = false;
 };
 
-// An fp32 or int8 right-hand side that arrives with the call in its row-major [K][N] form is read as it is (the
-// fp32 kinds gather their K-values from [k][n] slabs, int8 reads them with transposing LDS reads); everything else
-// is transposed into Bt[N][K] first.  Rows must be whole 16-byte vectors.
+// Whether a right-hand side that arrives with the call in its row-major [K][N] form is read as it lies: by direct tiles
+// whatever it is, by 256 x 256 tiles of bf16 and int8 through registers, and by the other tiles of fp32 (K-values gathered
+// from [k][n] slabs) and int8 (transposing LDS reads) where rows are whole 16-byte vectors.  Everything else is transposed
+// into Bt[N][K] first, unless its rows stream (streams_given below).
 static bool reads_b_as_given(const pml_hip_gemm_desc& d, int mfma_kind, const void* b, int tile) {
   if ((tile == TILE_16x16_W8 || tile == TILE_32x32_W8) && mfma_kind != KIND_F32X3) {
     // (four neighbouring columns per lane and K-row, whatever the type and wherever the rows begin: direct.hip)
@@ -964,10 +965,10 @@ static bool reads_b_as_given(const pml_hip_gemm_desc& d, int mfma_kind, const vo
         d.k * d.ldb * es < ((int64_t)1 << 31)))
     return false;
   if (mfma_kind == KIND_I8) {
-    // The transposing reads make the int8 kernel about 15 % slower (4096^3: 86 us against 74 + 10 for the copy), so
-    // they pay while the transposed copy -- a launch of at least 5 us, 3.2 TB/s beyond that -- costs more than
-    // that share of the multiplication (priced at the 1.8 POP/s the kernel reaches): up to about 3500 rows at
-    // K = N = 4096, always for small problems.
+    // The transposing reads make an int8 tile about 15 % slower (measured at 4096^3, which takes the path above now: 86 us
+    // against 74 + 10 for the copy), so they pay while the transposed copy -- a launch of at least 5 us, 3.2 TB/s beyond
+    // that -- costs more than that share of the multiplication (priced at the 1.8 POP/s the kernel reaches): always for
+    // small problems.
     const double t_gemm = 2.0 * (double)d.m * (double)d.n * (double)d.k / 1.8e15;
     const double t_copy = std::max(5e-6, 2.0 * (double)d.k * (double)d.n / 3.2e12);
     return 0.15 * t_gemm < t_copy;
