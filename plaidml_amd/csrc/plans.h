@@ -158,7 +158,7 @@ struct IgemmArgs {
   // convolution geometry (CONV instantiations only)
   int H, W, CI, OH, OW, KH, KW, SH, SW, PH, PW, DH, DW;
   // bytes between consecutive input pixels; 0 = CI * element size.  Smaller than that when the "channel
-  // vector" of a tap spans several pixels (igemm_kernel only)
+  // vector" of a tap spans several pixels (igemm_kernel and direct_kernel)
   int pix_pitch;
   // resident-filter convolution only: image count, LDS rows of the input window, number of 256-pixel tiles
   // halo_variant: 0 = general resident kernel, 1 / 2 = pipelined 3x3 kernel with that many 32-pixel chunks per row

@@ -69,9 +69,9 @@ bool isPinned(const void* p, size_t bytes);
 // statistics of the most recent invoke of any hip executable in this thread (for benchmarks)
 struct InvokeStats {
   // The wall time in three parts.  Uploads, launches and downloads are queued on one stream and waited for once, so where
-  // the link's share ends is not seen from here (two more events a run would cost 2 to 15 us): h2d_ms is the host's time up
-  // to the last upload it queues, rounding and staging included; kernel_ms the device's, first launch -> last launch, by HIP
-  // events; d2h_ms the rest -- what of the uploads is still under way then, the downloads, the passes over the results.
+  // the link's share ends is not seen from here (another mark would cost a launch of its own): h2d_ms is the host's time up
+  // to the last upload it queues, rounding and staging included; kernel_ms the device's, first launch -> last launch, by the
+  // device's clock as the kernels that copy small operands and results read it (by events where steps are timed); d2h_ms the rest -- what of the uploads is still under way then, the downloads, the passes over the results.
   double kernel_ms = 0;
   double h2d_ms = 0;
   double d2h_ms = 0;
