@@ -33,7 +33,7 @@ constexpr int kStage = kTile * kSlab;            // LDS bytes of one slab of A
 constexpr int kStages = 4;
 constexpr unsigned kRsrcFlags = 0x00020000u;     // raw buffer, 32-bit data format
 constexpr unsigned kBufRange = 0x80000000u;      // every real offset is below 2 GiB (checked at launch) ...
-constexpr unsigned kOutside = 0x80000000u;       // ... and this one reads as zeros, with any offset below 2 GiB added
+constexpr unsigned kOutside = 0x80000000u;       // ... and this one reads as zeros, with any row's offset added (given_span)
 
 #define PML_LDS(p) ((__attribute__((address_space(3))) void*)(p))
 
@@ -247,6 +247,7 @@ __global__ __launch_bounds__(kThreads, 2) void given_kernel(IgemmArgs p_by_value
   constexpr int MI = 8, NI = 4;               // 16 x 16 blocks of a wavefront: 128 x 64 results
   constexpr int kParts = kStage / (kThreads * 16);  // requests of a thread per slab of A
   constexpr int kPerBlock = kRows + kParts / 2;     // requests of a thread per 64 bytes of K: B's rows and half of A's
+  static_assert(64 / ES + kRows == 80 / ES, "the rows a request's offset reaches are the ones given_span counts");
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -442,7 +443,7 @@ hipError_t given_launch(int kind, const IgemmArgs& a, hipStream_t s) {
   // (rows of A are whole 16-byte vectors; a lane's four columns exist together and lie on a 4-element boundary)
   const int es = kind == KIND_BF16 ? 2 : 1;
   if (!a.b_kn || a.K2 > 0 || a.N % 4 != 0 || a.ldbt % 4 != 0 || a.K * es % 16 != 0 || ((uintptr_t)a.Bt & (4 * es - 1)) != 0) return hipErrorInvalidValue;
-  if (a.M * a.lda * es >= ((int64_t)1 << 31) || a.K * a.ldbt * es >= ((int64_t)1 << 31)) return hipErrorInvalidValue;
+  if (a.M * a.lda * es >= ((int64_t)1 << 31) || given_span(a.K, a.ldbt, es) >= ((int64_t)1 << 31)) return hipErrorInvalidValue;
   switch (kind) {
     case KIND_BF16: return launch<KIND_BF16>(a, s);
     case KIND_I8: return launch<KIND_I8>(a, s);

@@ -209,7 +209,10 @@ struct IgemmArgs {
 };
 
 hipError_t igemm_launch(int kind, int cfg, bool conv, const IgemmArgs& a, hipStream_t s);
-// TILE_256x256_W8 of a bf16 or int8 GEMM whose right-hand side is read as it lies (a.b_kn): given.hip
+// TILE_256x256_W8 of a bf16 or int8 GEMM whose right-hand side is read as it lies (a.b_kn): given.hip.  The bytes its offsets
+// into B span: B's rows, and at least the 80 bytes of K that the row offsets of a slab reach whatever K is (lanes whose rows
+// lie past K carry these offsets, too, on top of the mark that keeps them outside).  They must stay below 2 GiB.
+inline int64_t given_span(int64_t k, int64_t ldb, int es) { return (k > 80 / es ? k : 80 / es) * ldb * es; }
 hipError_t given_launch(int kind, const IgemmArgs& a, hipStream_t s);
 // bf16 products of many rows and a short K over Bt: stream.hip
 bool stream_takes(int cfg, bool conv, const IgemmArgs& a);

@@ -882,7 +882,7 @@ static DirectTiles direct_tiles(const pml_hip_gemm_desc& d, int kind) {
 // the [K][N] copy 104 us, from Bt through LDS 122 (int8, back to back until the clock settles: 72 and 68).
 static bool takes_b_as_given(const pml_hip_gemm_desc& d, int mfma_kind, int tile, int64_t ldb) {
   return tile == TILE_256x256_W8 && (mfma_kind == KIND_BF16 || mfma_kind == KIND_I8) && !d.b_layout && d.k2 == 0 && d.n % 4 == 0 &&
-         ldb % 4 == 0 && d.k * ldb * dt_size(d.in_dtype) < ((int64_t)1 << 31);
+         ldb % 4 == 0 && given_span(d.k, ldb, dt_size(d.in_dtype)) < ((int64_t)1 << 31);
 }
 
 int64_t pml_hip_gemm_dispatch(const pml_hip_gemm_desc* d) {

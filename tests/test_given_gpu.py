@@ -106,3 +106,30 @@ def test_packed_and_given_in_turn(kind, n, ldb):
     hk.check(hk.lib().pml_hip_gemm_pack_b(plan, dB[1].ptr, None))
     np.testing.assert_array_equal(call(None), want[1])
     hk.lib().pml_hip_plan_free(plan)
+
+
+@pytest.mark.parametrize('kind,K', [('i8', 64), ('i8', 16), ('bf16', 32), ('bf16', 8)])
+@pytest.mark.parametrize('ldb', [26843544, 26843548, 30000000])
+def test_rows_far_apart(kind, K, ldb):
+    """Rows of B so far apart that the 80 bytes of K a slab's row offsets reach, more than K holds here, stay just below 2 GiB
+    and do not: as it lies and through the transposed copy."""
+    M, N = 70, 72
+    rng = np.random.default_rng(K)
+    A, B = whole(rng, (M, K)), whole(rng, (K, N))
+    code, es, dt, out = (T.bf16, 2, hk.BF16, hk.F32) if kind == 'bf16' else (lambda x: x.astype(np.int8), 1, hk.I8, hk.I32)
+    ldb //= es
+    L = hk.lib()
+    d = hk.GemmDesc()
+    d.in_dtype, d.out_dtype, d.c_dtype, d.flags = dt, out, out, T.FORCED['flags']
+    d.m, d.n, d.k, d.lda, d.ldb, d.ldc = M, N, K, K, ldb // 4 * 4, N
+    plan = L.pml_hip_gemm_dispatch(ctypes.byref(d))
+    assert plan, L.pml_hip_last_error()
+    dA, dB, dC = hk.DeviceBuffer.from_numpy(code(A)), hk.DeviceBuffer(K * d.ldb * es), hk.DeviceBuffer(M * N * 4)
+    rows = code(B)
+    for k in range(K):
+        hk.check(L.pml_hip_memcpy_h2d(dB.ptr + k * d.ldb * es, rows[k].ctypes.data, N * es, None))
+    none = hk.ptr_array([])
+    hk.check(L.pml_hip_gemm_invoke(plan, dA.ptr, dB.ptr, dC.ptr, None, none, none, None))
+    hk.check(L.pml_hip_stream_sync(None))
+    L.pml_hip_plan_free(plan)
+    np.testing.assert_array_equal(dC.to_numpy(np.float32 if kind == 'bf16' else np.int32, (M, N)), A @ B)
