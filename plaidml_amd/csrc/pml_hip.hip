@@ -64,7 +64,7 @@ struct Plan {
   size_t bt_bytes = 0;
   bool packed = false;
   bool b_split = false;  // split fp32 kind: a right-hand side packed once is kept as bf16 heads + remainders
-  std::atomic<bool> bt_is_split{false};  // ... and `bt` holds that form now (invokes that bring their own right-hand side clear it)
+  std::atomic<bool> bt_is_split{false};  // ... and `bt` holds that form now (an invoke that turns its own right-hand side into `bt` clears it)
   // large tiles that take B[K][N] as it lies (given.hip) keep a packed right-hand side in that form, rows of n elements
   bool b_kn = false;
   std::atomic<bool> bt_is_kn{false};  // ... and `bt` holds it now (as above)
@@ -989,11 +989,10 @@ static bool streams_given(int mfma_kind, int tile, bool conv, const void* b, int
 
 static int gemm_run(const pml_hip_gemm_desc& d, int mfma_kind, int tile, const DirectTiles& direct, void* bt, int64_t bt_ld, bool packed,
                     const void* a, const void* b, void* c, const void* init, const void* const* operands,
-                    void* const* outs, pml_hip_stream s, const SecondProduct* second = nullptr, bool bt_is_split = false,
-                    const Plan* split_plan = nullptr, bool bt_is_kn = false) {
+                    void* const* outs, pml_hip_stream s, const SecondProduct* second = nullptr, Plan* plan = nullptr) {
   // (a right-hand side that arrives with the call is transposed per run and split in the kernel's registers: a
   // second small launch costs more than it saves; one packed once is kept split)
-  const bool b_split = bt_is_split && !b;
+  const bool b_split = plan && plan->bt_is_split && !b;
   if (!a || !c) return fail("gemm_invoke: null operand");
   if (!b && (!packed || d.b_layout)) return fail("gemm_invoke: b is null and no packed right-hand side exists");
   if (d.b_layout && ((uintptr_t)b & 15) != 0) return fail("gemm_invoke: an [N][K] right-hand side must be 16-byte aligned");
@@ -1007,7 +1006,7 @@ static int gemm_run(const pml_hip_gemm_desc& d, int mfma_kind, int tile, const D
   } else if (direct.rows >= 0 && mfma_kind == KIND_F32) {
     tile = direct.rows;
   }
-  const bool packed_kn = bt_is_kn && !b;
+  const bool packed_kn = plan && plan->bt_is_kn && !b;
   const bool b_as_given = packed_kn || reads_b_as_given(d, mfma_kind, b, tile);
   const bool transposed = b && !d.b_layout && !b_as_given;
   if (d.k2 > 0) {
@@ -1076,11 +1075,14 @@ static int gemm_run(const pml_hip_gemm_desc& d, int mfma_kind, int tile, const D
   for (int i = 0; i < d.tail.n_ops; ++i)
     if (d.tail.ops[i].opcode == PML_HIP_EPI_STORE && !g.outs[d.tail.ops[i].operand])
       return fail("gemm_invoke: missing extra output");
-  if (split_plan && !b_split) split_args(split_plan, g);  // (the K split over workgroups is not built for a right-hand side packed split)
+  // (the K split over workgroups is not built for a right-hand side packed split, nor used for two products)
+  if (plan && !second && !b_split) split_args(plan, g);
   // (rows that stream take a [K][N] right-hand side as it lies, too)
-  if (transposed && !(!packed && streams_given(mfma_kind, tile, false, b, d.ldb, g)) &&
-      check(transpose_pack(es, b, bt, d.k, d.n, d.ldb, bt_ld, (hipStream_t)s), "transpose_pack"))
-    return 1;
+  if (transposed && !(!packed && streams_given(mfma_kind, tile, false, b, d.ldb, g))) {
+    // (from here on `bt` holds the plain transposed form, whatever a packed copy was kept in before)
+    if (plan) plan->bt_is_split = plan->bt_is_kn = false;
+    if (check(transpose_pack(es, b, bt, d.k, d.n, d.ldb, bt_ld, (hipStream_t)s), "transpose_pack")) return 1;
+  }
   return check(igemm_launch(b_split ? KIND_F32X3P : mfma_kind, tile, false, g, (hipStream_t)s), "igemm_launch");
 }
 
@@ -1088,10 +1090,7 @@ int pml_hip_gemm_invoke(int64_t plan, const void* a, const void* b, void* c, con
                         const void* const* operands, void* const* outs, pml_hip_stream s) {
   Plan* p = (Plan*)(intptr_t)plan;
   if (!p || p->kind != PLAN_GEMM) return fail("gemm_invoke: not a gemm plan");
-  const bool split = p->bt_is_split, kn = p->bt_is_kn;
-  // a right-hand side that this run transposes overwrites the packed copy
-  if (b && !p->gemm.b_layout && !reads_b_as_given(p->gemm, p->mfma_kind, b, p->tile)) p->bt_is_split = p->bt_is_kn = false;
-  return gemm_run(p->gemm, p->mfma_kind, p->tile, p->direct, p->bt, p->bt_ld, p->packed, a, b, c, init, operands, outs, s, nullptr, split, p, kn);
+  return gemm_run(p->gemm, p->mfma_kind, p->tile, p->direct, p->bt, p->bt_ld, p->packed, a, b, c, init, operands, outs, s, nullptr, p);
 }
 
 int pml_hip_gemm_invoke2(int64_t plan, const void* a, const void* b, void* c, const void* init, const void* a2, const void* b2,
@@ -1105,7 +1104,7 @@ int pml_hip_gemm_invoke2(int64_t plan, const void* a, const void* b, void* c, co
   sp.init2 = init2;
   sp.bt2 = p->bt2;
   sp.packed2 = p->packed2;
-  return gemm_run(p->gemm, p->mfma_kind, p->tile, p->direct, p->bt, p->bt_ld, p->packed, a, b, c, init, operands, outs, s, &sp);
+  return gemm_run(p->gemm, p->mfma_kind, p->tile, p->direct, p->bt, p->bt_ld, p->packed, a, b, c, init, operands, outs, s, &sp, p);
 }
 
 int pml_hip_gemm_run_static(const pml_hip_gemm_desc* d, const void* a, const void* b, void* c, const void* init,

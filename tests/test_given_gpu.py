@@ -133,3 +133,49 @@ def test_rows_far_apart(kind, K, ldb):
     hk.check(L.pml_hip_stream_sync(None))
     L.pml_hip_plan_free(plan)
     np.testing.assert_array_equal(dC.to_numpy(np.float32 if kind == 'bf16' else np.int32, (M, N)), A @ B)
+
+
+def packed_product(kind, M, n, K, ldb, flags=0):
+    """A plan with a right-hand side packed once, its operands and a call that returns the result's bytes."""
+    rng = np.random.default_rng(M)
+    L, dt = hk.lib(), hk.I8 if kind == 'i8' else hk.F32 if kind == 'f32x3' else hk.BF16
+    d = hk.GemmDesc()
+    d.in_dtype, d.out_dtype, d.c_dtype, d.flags = dt, hk.I32 if kind == 'i8' else hk.F32, hk.I32 if kind == 'i8' else hk.F32, flags
+    d.m, d.n, d.k, d.lda, d.ldb, d.ldc = M, n, K, K, ldb, n
+    plan = L.pml_hip_gemm_dispatch(ctypes.byref(d))
+    assert plan, L.pml_hip_last_error()
+    codes = {hk.I8: np.arange(-4, 5).astype(np.int8), hk.F32: np.arange(-4, 5).astype(np.float32), hk.BF16: T.bf16(np.arange(-4, 5))}[dt]
+    A, B = (hk.DeviceBuffer.from_numpy(codes[rng.integers(0, 9, s, np.uint8)]) for s in ((M, K), (K, ldb)))
+    C, none = hk.DeviceBuffer(M * n * 4), hk.ptr_array([])
+    hk.check(L.pml_hip_gemm_pack_b(plan, B.ptr, None))
+
+    def call(b, c=C.ptr):
+        hk.check(L.pml_hip_fill_u32(C.ptr, 0xdeadbeef, M * n, None))
+        rc = L.pml_hip_gemm_invoke(plan, A.ptr, b, c, None, none, none, None)
+        hk.check(L.pml_hip_stream_sync(None))
+        return C.to_numpy(np.uint32, (M, n)) if rc == 0 else None
+
+    return plan, B, call
+
+
+@pytest.mark.parametrize('kind,K', [('bf16', 272), ('i8', 272), ('f32x3', 288)])
+def test_a_refused_call_leaves_the_packed_copy(kind, K):
+    """A call that brings a right-hand side the plan would have to turn, and is refused for another reason before that."""
+    plan, B, call = packed_product(kind, 270, 260, K, 262, hk.flag_tile('64x64') | hk.FP32_AS_BF16X3 if kind == 'f32x3' else T.FORCED['flags'])
+    want = call(None)
+    assert call(B.ptr, None) is None
+    np.testing.assert_array_equal(call(None), want)
+    np.testing.assert_array_equal(call(B.ptr), want)
+    np.testing.assert_array_equal(call(None), want)
+    hk.lib().pml_hip_plan_free(plan)
+
+
+def test_a_direct_tile_leaves_the_packed_copy():
+    """Few rows, many columns: the right-hand side packed for the 256 x 256 tile, one that arrives with the call in rows this
+    tile cannot read taken by a direct tile as it lies, and then the packed one again."""
+    plan, B, call = packed_product('bf16', 256, 49152, 2560, 49154)
+    assert '256x256' in hk.describe(plan) and 'with B as it lies tile=' in hk.describe(plan), hk.describe(plan)
+    want = call(None)
+    np.testing.assert_array_equal(call(B.ptr), want)
+    np.testing.assert_array_equal(call(None), want)
+    hk.lib().pml_hip_plan_free(plan)
