@@ -519,13 +519,18 @@ __global__ __launch_bounds__(NT, (igemm_waves_per_simd<BM, BN, STAGES, SLAB, NT>
 #pragma unroll
           for (int l = m; l < kLoads; l += kSlots) issue_load(l);
         }
+        // (a pair's second block multiplies both of its packed fragments, heads and remainders: there a fragment of Bt is
+        // replaced behind the last block row that takes it)
+        constexpr int kLastUse = (MI - 1) * NI;
+        const bool both = kSplitB && cur == 1;
 #pragma unroll
         for (int d = m; d < MI + NI; d += kSlots) {
           if (d < MI)
             fa[nxt][d] = *(const i32x4_t*)(ra_ + d * 32 * kSlabBytes + fs);
-          else
+          else if (!both)
             fb[nxt][d - MI] = read_b(rb_, d - MI, fs_b);
         }
+        if (both && m >= kLastUse) fb[nxt][m >= kLastUse ? m - kLastUse : 0] = read_b(rb_, m - kLastUse, fs_b);
         __builtin_amdgcn_sched_barrier(0);
       }
     }
