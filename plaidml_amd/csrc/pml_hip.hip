@@ -201,8 +201,9 @@ bool splits_k(int64_t m, int64_t n, int64_t k_bytes, int kind) {
 // its bytes both ways at 2.2 TB/s:
 // bf16 512 x 512 x 512 9.4 -> 5.0, 1024^3 14.6 -> 10.6, 64 x 2048 x 2048 16.5 -> 8.8; fp32 128 x 4096 x 1024 23.4 -> 12.3.
 // kn_ldb: that right-hand side's row pitch in bytes (0: Bt); always: the better of the two whatever the LDS kernel takes;
-// can_split: the LDS kernel may split K
-int direct_tile_of(int64_t m, int64_t n, int64_t k_bytes, int kind, int64_t kn_ldb = 0, bool always = false, bool can_split = true) {
+// can_split: the LDS kernel may split K; as_given: it reads a [K][N] right-hand side as it lies (256 x 49152, K = 4096 bf16:
+// 409 us direct, 135 with 256 x 256 tiles; charged the copy of 800 MB, they lost)
+int direct_tile_of(int64_t m, int64_t n, int64_t k_bytes, int kind, int64_t kn_ldb = 0, bool always = false, bool can_split = true, bool as_given = false) {
   if (kind != KIND_F32 && kind != KIND_BF16 && kind != KIND_I8) return -1;
   auto tiles = [&](int64_t bm, int64_t bn) { return ((m + bm - 1) / bm) * ((n + bn - 1) / bn); };
   const double kb = (double)k_bytes;
@@ -222,7 +223,7 @@ int direct_tile_of(int64_t m, int64_t n, int64_t k_bytes, int kind, int64_t kn_l
   };
   const int64_t slabs = (k_bytes + 127) / 128;
   double lds_us = 4.2 + (f32 ? 0.58 : kind == KIND_I8 ? 0.28 : 0.23) * (double)slabs;
-  bool needs_bt = kind == KIND_BF16 || n % (16 / es) != 0 || kn_ldb % 16 != 0;
+  bool needs_bt = !as_given && (kind == KIND_BF16 || n % (16 / es) != 0 || kn_ldb % 16 != 0);
   if (can_split && splits_k(m, n, k_bytes, kind)) {
     int splits = 1, per = 0;
     igemm_split_plan(m, n, slabs, n_cus, &splits, &per);
@@ -863,26 +864,27 @@ int pml_hip_gemm_tail_cheaper_apart(const pml_hip_gemm_desc* d) {
   return choose_tile(d->m, d->n, k_bytes, kind, true) == TILE_256x256_W8 && choose_tile(d->m, d->n, k_bytes, kind, false) != TILE_256x256_W8;
 }
 
-// The direct tiles of a product (-1: none): over Bt rows that are at hand (packed earlier, or [N][K] as given), and over a
-// [K][N] right-hand side as it lies.  One that has to be transposed first, and a tile the descriptor names, stay with the
-// plan's tile -- except that fp32 sums are the same bits in either layout: there the layout decides which direct tile, not whether.
-static DirectTiles direct_tiles(const pml_hip_gemm_desc& d, int kind) {
-  DirectTiles t;
-  if (PML_HIP_FLAG_TILE_OF(d.flags) >= 0) return t;
-  const int es = dt_size(d.in_dtype);
-  // (the launch of two products does not split K: one chain of all slabs otherwise)
-  t.rows = direct_tile_of(d.m, d.n, (d.k + d.k2) * es, kind, 0, false, /*can_split=*/d.k2 == 0);
-  if (d.b_layout || d.k2 > 0 || (kind == KIND_F32 && t.rows < 0)) return t;
-  t.given = direct_tile_of(d.m, d.n, d.k * es, kind, d.ldb * es, /*always=*/kind == KIND_F32);
-  return t;
-}
-
 // Whether a product's 256 x 256 tile reads B[K][N] with rows of `ldb` elements as it lies: four neighbouring columns per lane
 // and K-row, through registers (given.hip).  For bf16 it is then the better form of a packed right-hand side, too: 4096^3 from
 // the [K][N] copy 104 us, from Bt through LDS 122 (int8, back to back until the clock settles: 72 and 68).
 static bool takes_b_as_given(const pml_hip_gemm_desc& d, int mfma_kind, int tile, int64_t ldb) {
   return tile == TILE_256x256_W8 && (mfma_kind == KIND_BF16 || mfma_kind == KIND_I8) && !d.b_layout && d.k2 == 0 && d.n % 4 == 0 &&
          ldb % 4 == 0 && given_span(d.k, ldb, dt_size(d.in_dtype)) < ((int64_t)1 << 31);
+}
+
+// The direct tiles of a product (-1: none): over Bt rows that are at hand (packed earlier, or [N][K] as given), and over a
+// [K][N] right-hand side as it lies.  One that has to be transposed first, and a tile the descriptor names, stay with the
+// plan's tile -- except that fp32 sums are the same bits in either layout: there the layout decides which direct tile, not whether.
+// lds_tile: the plan's tile.
+static DirectTiles direct_tiles(const pml_hip_gemm_desc& d, int kind, int lds_tile) {
+  DirectTiles t;
+  if (PML_HIP_FLAG_TILE_OF(d.flags) >= 0) return t;
+  const int es = dt_size(d.in_dtype);
+  // (the launch of two products does not split K: one chain of all slabs otherwise)
+  t.rows = direct_tile_of(d.m, d.n, (d.k + d.k2) * es, kind, 0, false, /*can_split=*/d.k2 == 0);
+  if (d.b_layout || d.k2 > 0 || (kind == KIND_F32 && t.rows < 0)) return t;
+  t.given = direct_tile_of(d.m, d.n, d.k * es, kind, d.ldb * es, /*always=*/kind == KIND_F32, /*can_split=*/true, takes_b_as_given(d, kind, lds_tile, d.ldb));
+  return t;
 }
 
 int64_t pml_hip_gemm_dispatch(const pml_hip_gemm_desc* d) {
@@ -901,7 +903,7 @@ int64_t pml_hip_gemm_dispatch(const pml_hip_gemm_desc* d) {
     // (a second product's slabs follow the first one's on the slab axis the splits share out.)  With a direct tile over rows
     // that are at hand the LDS tile is only left for a [K][N] right-hand side that arrives with the call and cannot be read
     // as it lies; pml_hip_gemm_pack_b ends that.
-    p->direct = direct_tiles(*d, kind);
+    p->direct = direct_tiles(*d, kind, p->tile);
     if (!(p->direct.rows >= 0 && (d->b_layout || kind == KIND_F32)))
       prepare_split(p, d->m, d->n, (d->k * dt_size(d->in_dtype) + 127) / 128 + (d->k2 * dt_size(d->in_dtype) + 127) / 128);
   }
@@ -1127,7 +1129,7 @@ int pml_hip_gemm_run_static(const pml_hip_gemm_desc* d, const void* a, const voi
   const bool plain = mode == 1 || mode == 2 || tail_requant(d->tail, d->out_dtype, d->c_dtype, mode, nullptr);
   // (no workspace may be allocated here: the K loop is never split over workgroups)
   const int tile = choose_tile(d->m, d->n, d->k * dt_size(d->in_dtype), kind, plain, PML_HIP_FLAG_TILE_OF(d->flags), /*allow_split=*/false);
-  return gemm_run(*d, kind, tile, direct_tiles(*d, kind), bt, d->k, false, a, b, c, init, operands, outs, s);
+  return gemm_run(*d, kind, tile, direct_tiles(*d, kind, tile), bt, d->k, false, a, b, c, init, operands, outs, s);
 }
 
 // ---------------------------------------------------------------------------

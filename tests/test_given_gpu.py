@@ -179,3 +179,17 @@ def test_a_direct_tile_leaves_the_packed_copy():
     np.testing.assert_array_equal(call(B.ptr), want)
     np.testing.assert_array_equal(call(None), want)
     hk.lib().pml_hip_plan_free(plan)
+
+
+def test_a_direct_tile_is_not_charged_a_copy_that_is_not_made():
+    """256 rows, many columns: the direct tile of 32 x 64 would win only over a 256 x 256 tile that has its right-hand side
+    transposed first; where that tile reads it as it lies, it runs."""
+    for ldb, direct in ((49152, False), (49153, True)):
+        d = hk.GemmDesc()
+        d.in_dtype, d.out_dtype, d.c_dtype = hk.BF16, hk.F32, hk.F32
+        d.m, d.n, d.k, d.lda, d.ldb, d.ldc = 256, 49152, 4096, 4096, ldb, 49152
+        plan = hk.lib().pml_hip_gemm_dispatch(ctypes.byref(d))
+        assert plan, hk.lib().pml_hip_last_error()
+        text = hk.describe(plan)
+        hk.lib().pml_hip_plan_free(plan)
+        assert '256x256' in text and ('with B as it lies tile=' in text) == direct, text
