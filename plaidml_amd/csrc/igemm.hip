@@ -975,6 +975,11 @@ hipError_t igemm_launch(int kind, int cfg, bool conv, const IgemmArgs& a, hipStr
   const int64_t a_bytes = conv ? (int64_t)a.NB * a.H * a.W * (a.pix_pitch ? a.pix_pitch : a.CI * es) + 256 : a.M * a.lda * es;
   const int64_t b_bytes = (a.b_kn ? a.K : a.N) * a.ldbt * es;
   if (a_bytes >= ((int64_t)1 << 31) || b_bytes >= ((int64_t)1 << 31) || (conv && a.M >= ((int64_t)1 << 31))) return hipErrorInvalidValue;
+  if (a.K2 > 0) {
+    // (the same for the second product, up to the last row it reads)
+    const int64_t last = a.g2_stride > 0 ? ((a.M / a.g2_ohw - 1) * a.g2_h + (int64_t)((a.g2_ohw / a.g2_ow) - 1) * a.g2_stride) * a.g2_w + (int64_t)(a.g2_ow - 1) * a.g2_stride : a.M - 1;
+    if ((last * a.lda2 + a.K2) * es >= ((int64_t)1 << 31) || ((a.N - 1) * a.ldbt2 + a.K2) * es >= ((int64_t)1 << 31)) return hipErrorInvalidValue;
+  }
   if (cfg == TILE_256x256_W8 && a.b_kn && (kind == KIND_BF16 || kind == KIND_I8)) return given_launch(kind, a, s);
   if (kind == KIND_BF16 && stream_takes(cfg, conv, a)) return stream_launch(conv, a, s);
   if (cfg == TILE_16x16_W8 || cfg == TILE_32x32_W8) {

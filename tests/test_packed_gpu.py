@@ -59,3 +59,58 @@ def test_convolution(kind, tile, shape, k, co, stride, monkeypatch):
     pad[:, ph:ph + h, pw:pw + w] = I
     want = sum(pad[:, y:y + (oh - 1) * stride + 1:stride, x:x + (ow - 1) * stride + 1:stride] @ F[y, x] for y in range(k) for x in range(k))
     np.testing.assert_array_equal(got, want)
+
+
+def two_products(m, n, k, k2, lda2=None, ldb2=None, pixels=None, layout=0):
+    d = hk.GemmDesc()
+    d.in_dtype = d.out_dtype = d.c_dtype = hk.BF16
+    d.m, d.n, d.k, d.lda, d.ldb, d.ldc, d.b_layout = m, n, k, k, k if layout else n, n, layout
+    d.k2, d.lda2, d.ldb2 = k2, lda2 or k2, ldb2 or (k2 if layout else n)
+    if pixels:
+        d.a2_stride, d.a2_h, d.a2_w, d.a2_oh, d.a2_ow = pixels
+    return d
+
+
+@pytest.mark.parametrize('tile', [None, '64x64', '32x32w8'])
+@pytest.mark.parametrize('desc', [dict(lda2=1 << 30), dict(pixels=(1, 1, 2, 1, 2), lda2=1 << 30), dict(ldb2=1 << 30, layout=1), dict(pixels=(2, 3, 1, 2, 1), lda2=1 << 29)])
+def test_second_product_of_two_gib_is_refused(desc, tile):
+    """Offsets into its operands are 32 bits below 2 GiB, as the first product's are (the rows that would be read lie at 2 GiB
+    exactly: nothing is read where they are not refused either)."""
+    d = two_products(2, 16, 16, 16, **desc)
+    if tile:
+        d.flags = hk.flag_tile(tile)
+    if desc.get('layout'):
+        d.n = 2
+        d.ldc = 16
+    L = hk.lib()
+    plan = L.pml_hip_gemm_dispatch(ctypes.byref(d))
+    assert plan, L.pml_hip_last_error()
+    buf, none = hk.DeviceBuffer(4096), hk.ptr_array([])
+    hk.check(L.pml_hip_fill_u32(buf.ptr, 0, 1024, None))
+    assert L.pml_hip_gemm_invoke2(plan, buf.ptr, buf.ptr, buf.ptr, None, buf.ptr, buf.ptr, None, none, none, None) != 0
+    L.pml_hip_plan_free(plan)
+
+
+@pytest.mark.parametrize('stride', [0, 2])
+def test_second_product_up_to_two_gib(stride):
+    """The last row read ends just below 2 GiB."""
+    rng = np.random.default_rng(stride)
+    K, K2, N = 16, 24, 20
+    A, B, B2 = (rng.integers(-4, 5, s).astype(np.float32) for s in ((2, K), (K, N), (K2, N)))
+    A2 = rng.integers(-4, 5, (2, K2)).astype(np.float32)
+    rows = 2 if stride else 1  # between the two rows read
+    lda2 = ((1 << 30) - 32) // rows // 8 * 8
+    d = two_products(2, N, K, K2, lda2=lda2, pixels=(2, 1, 3, 1, 2) if stride else None)
+    L = hk.lib()
+    plan = L.pml_hip_gemm_dispatch(ctypes.byref(d))
+    assert plan, L.pml_hip_last_error()
+    dA, dB, dB2, dC, none = (hk.DeviceBuffer.from_numpy(T.bf16(A)), hk.DeviceBuffer.from_numpy(T.bf16(B)), hk.DeviceBuffer.from_numpy(T.bf16(B2)),
+                             hk.DeviceBuffer(2 * N * 2), hk.ptr_array([]))
+    dA2 = hk.DeviceBuffer(2 << 30)
+    bits = T.bf16(A2)
+    for i in range(2):
+        hk.check(L.pml_hip_memcpy_h2d(dA2.ptr + i * rows * lda2 * 2, bits[i].ctypes.data, K2 * 2, None))
+    hk.check(L.pml_hip_gemm_invoke2(plan, dA.ptr, dB.ptr, dC.ptr, None, dA2.ptr, dB2.ptr, None, none, none, None))
+    hk.check(L.pml_hip_stream_sync(None))
+    L.pml_hip_plan_free(plan)
+    np.testing.assert_array_equal(E.bf16_from_bits(dC.to_numpy(np.uint16, (2, N))), E.round_bf16(A @ B + A2 @ B2))
