@@ -880,7 +880,8 @@ static DirectTiles direct_tiles(const pml_hip_gemm_desc& d, int kind, int lds_ti
   DirectTiles t;
   if (PML_HIP_FLAG_TILE_OF(d.flags) >= 0) return t;
   const int es = dt_size(d.in_dtype);
-  // (the launch of two products does not split K: one chain of all slabs otherwise)
+  // (Two products are priced against one chain of all slabs: of 49 x 2048, K = 512 + 1024 the split takes 9.2 us and the direct
+  // tile 8.8, of 196 x 256, K = 1024 + 512 9.0 and 5.8; only a K of 4096 turns that round, 10.7 and 17.0.)
   t.rows = direct_tile_of(d.m, d.n, (d.k + d.k2) * es, kind, 0, false, /*can_split=*/d.k2 == 0);
   if (d.b_layout || d.k2 > 0 || (kind == KIND_F32 && t.rows < 0)) return t;
   t.given = direct_tile_of(d.m, d.n, d.k * es, kind, d.ldb * es, /*always=*/kind == KIND_F32, /*can_split=*/true, takes_b_as_given(d, kind, lds_tile, d.ldb));
@@ -1077,8 +1078,8 @@ static int gemm_run(const pml_hip_gemm_desc& d, int mfma_kind, int tile, const D
   for (int i = 0; i < d.tail.n_ops; ++i)
     if (d.tail.ops[i].opcode == PML_HIP_EPI_STORE && !g.outs[d.tail.ops[i].operand])
       return fail("gemm_invoke: missing extra output");
-  // (the K split over workgroups is not built for a right-hand side packed split, nor used for two products)
-  if (plan && !second && !b_split) split_args(plan, g);
+  // (the K split over workgroups is not built for a right-hand side packed split)
+  if (plan && !b_split) split_args(plan, g);
   // (rows that stream take a [K][N] right-hand side as it lies, too)
   if (transposed && !(!packed && streams_given(mfma_kind, tile, false, b, d.ldb, g))) {
     // (from here on `bt` holds the plain transposed form, whatever a packed copy was kept in before)
@@ -1428,9 +1429,8 @@ int pml_hip_gemm_pack_b(int64_t plan, const void* b, pml_hip_stream s) {
   if (p->b_split && check(split_rows_launch(p->bt, d.n, p->bt_ld, d.k, (hipStream_t)s), "split_rows_launch")) return 1;
   p->bt_is_split = p->b_split;
   p->packed = true;
-  if ((p->direct.rows >= 0 || d.k2 > 0) && p->ws) {
-    // (its invokes take the direct tile from now on; one that brings a right-hand side all the same does not split K, nor do
-    // those of two products)
+  if (p->direct.rows >= 0 && p->ws) {
+    // (its invokes take the direct tile from now on; one that brings a right-hand side all the same does not split K)
     p->drop(&p->ws, (size_t)p->sk_splits * d.m * p->sk_pitch * 4);
     p->tile = TILE_64x64;
   }

@@ -114,3 +114,39 @@ def test_second_product_up_to_two_gib(stride):
     hk.check(L.pml_hip_stream_sync(None))
     L.pml_hip_plan_free(plan)
     np.testing.assert_array_equal(E.bf16_from_bits(dC.to_numpy(np.uint16, (2, N))), E.round_bf16(A @ B + A2 @ B2))
+
+
+@pytest.mark.parametrize('form', ['packed', 'given', 'rows'])
+@pytest.mark.parametrize('stride', [0, 2])
+@pytest.mark.parametrize('tile', T.TILE_NAMES + ['16x16w8', '32x32w8', None])
+def test_two_products(tile, stride, form):
+    """Both right-hand sides packed once, as [K][N] with the call, and as [N][K]: slabs of both products behind one another, shared
+    out among workgroups where K is split, from the middle of either on."""
+    rng = np.random.default_rng(stride)
+    K, K2, N, side = 1096, 648, 72, 6
+    M = side * side
+    A, A2, B, B2 = (rng.integers(-4, 5, s).astype(np.float32) for s in ((M, K), (M, K2), (K, N), (K2, N)))
+    b1, b2 = (rng.integers(-9, 10, N).astype(np.float32) for _ in range(2))
+    wide = (side - 1) * 2 + 1
+    image = np.zeros((wide, wide, K2), np.float32)
+    image[::2, ::2] = A2.reshape(side, side, K2)
+    d = two_products(M, N, K, K2, pixels=(stride, wide, wide, side, side) if stride else None, layout=int(form == 'rows'))
+    d.out_dtype = d.c_dtype = d.init_dtype = hk.F32
+    d.init_kind = d.init_col_stride = d.init2_kind = 1
+    d.flags = hk.flag_tile(tile) if tile else 0
+    L = hk.lib()
+    plan = L.pml_hip_gemm_dispatch(ctypes.byref(d))
+    assert plan, L.pml_hip_last_error()
+    turned = (lambda x: np.ascontiguousarray(x.T)) if form == 'rows' else lambda x: x
+    dA, dB, dA2, dB2 = (hk.DeviceBuffer.from_numpy(T.bf16(x)) for x in (A, turned(B), image if stride else A2, turned(B2)))
+    d1, d2, dC, none = hk.DeviceBuffer.from_numpy(b1), hk.DeviceBuffer.from_numpy(b2), hk.DeviceBuffer(M * N * 4), hk.ptr_array([])
+    if form == 'packed':
+        hk.check(L.pml_hip_gemm_pack_b(plan, dB.ptr, None))
+        hk.check(L.pml_hip_gemm_pack_b2(plan, dB2.ptr, None))
+    given = (None, None) if form == 'packed' else (dB.ptr, dB2.ptr)
+    for _ in range(2):
+        hk.check(L.pml_hip_fill_u32(dC.ptr, 0xdeadbeef, M * N, None))
+        hk.check(L.pml_hip_gemm_invoke2(plan, dA.ptr, given[0], dC.ptr, d1.ptr, dA2.ptr, given[1], d2.ptr, none, none, None))
+        hk.check(L.pml_hip_stream_sync(None))
+        np.testing.assert_array_equal(dC.to_numpy(np.float32, (M, N)), A @ B + A2 @ B2 + b1 + b2)
+    L.pml_hip_plan_free(plan)
