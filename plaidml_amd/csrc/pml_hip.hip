@@ -547,7 +547,40 @@ int64_t conv_slabs(const pml_hip_conv2d_desc& d) {
   return d.kh * (conv_tap_runs(d) ? (d.kw * pixel + 127) / 128 : d.kw * ((pixel + 127) / 128));
 }
 
-// Everything of the kernel arguments that the descriptor fixes (no operand pointers).
+// Everything of the kernel arguments that the descriptor fixes (no operand pointers, no right-hand side).
+void gemm_args(const pml_hip_gemm_desc& d, IgemmArgs& g) {
+  std::memset(&g, 0, sizeof g);
+  if (d.k2 > 0) {
+    g.K2 = d.k2;
+    g.lda2 = d.lda2;
+    g.ldbt2 = d.b_layout ? d.ldb2 : d.k2;
+    g.g2_stride = d.a2_stride;
+    if (d.a2_stride > 0) {
+      g.g2_h = (int)d.a2_h;
+      g.g2_w = (int)d.a2_w;
+      g.g2_ohw = (int)(d.a2_oh * d.a2_ow);
+      g.g2_ow = (int)d.a2_ow;
+      fast_div_magic((unsigned)g.g2_ohw, &g.g2_ohw_magic, &g.g2_ohw_shift);
+      fast_div_magic((unsigned)g.g2_ow, &g.g2_ow_magic, &g.g2_ow_shift);
+    }
+  }
+  g.M = d.m;
+  g.N = d.n;
+  g.K = d.k;
+  g.lda = d.lda;
+  g.ldc = d.ldc;
+  g.out_dtype = d.out_dtype;
+  g.init_dtype = d.init_dtype;
+  g.init_rs = d.init_row_stride;
+  g.init_cs = d.init_col_stride;
+  g.c_dtype = d.c_dtype;
+  g.n_cus = device_cus();
+  g.stream = PML_HIP_FLAG_TILE_OF(d.flags) < 0;
+  classify_tail(d.tail, d.out_dtype, d.c_dtype, &g.tail_mode, &g.tail_relu);
+  g.tail_ssr = tail_scale_shift(d.tail, d.out_dtype, g.tail_mode);
+  tail_requant(d.tail, d.out_dtype, d.c_dtype, g.tail_mode, &g);
+  g.tail = d.tail;
+}
 void conv_args(const Plan* p, IgemmArgs& g) {
   const pml_hip_conv2d_desc& d = p->conv;
   const int64_t K = d.kh * d.kw * d.ci;
@@ -888,6 +921,32 @@ static DirectTiles direct_tiles(const pml_hip_gemm_desc& d, int kind, int lds_ti
   return t;
 }
 
+// Whether a launch streams its rows past the [K][N] right-hand side `b` as it lies, with the arguments then changed to that.
+static bool streams_given(int mfma_kind, int tile, bool conv, const void* b, int64_t ldb, IgemmArgs& g) {
+  if (mfma_kind != KIND_BF16) return false;
+  const void* const bt = g.Bt;
+  const int64_t ldbt = g.ldbt;
+  g.Bt = b, g.ldbt = ldb, g.b_kn = 1;
+  if (stream_takes(tile, conv, g)) return true;
+  g.Bt = bt, g.ldbt = ldbt, g.b_kn = 0;
+  return false;
+}
+
+static const char* mfma16_name(int kind) { return kind == KIND_F32 ? "f32_16x16x4" : kind == KIND_BF16 ? "f32_16x16x32_bf16" : "i32_16x16x64_i8"; }
+
+// The part of a plan's text that says which right-hand sides its rows stream past (stream.hip), given operands that are aligned
+// to 16 bytes: rows of K (`rows_tile`: the tile taken otherwise), and a [K][N] one as it lies (kn_ldb > 0).
+static std::string stream_text(int mfma_kind, bool conv, IgemmArgs g, bool init, const pml_hip_epilogue& tail, int rows_tile, bool rows_packed, int kn_tile, int64_t kn_ldb) {
+  if (mfma_kind != KIND_BF16) return "";
+  const void* const aligned = (const void*)256;  // (stands for an operand that is there; nothing is read)
+  if (init) g.init = aligned;
+  for (int i = 0; i < tail.n_operands; ++i) g.operands[i] = aligned;
+  const bool rows = stream_takes(rows_tile, conv, g), kn = kn_ldb > 0 && streams_given(mfma_kind, kn_tile, conv, aligned, kn_ldb, g);
+  if (!rows && !kn) return "";
+  const std::string packed = rows_packed ? "B packed" : "B";
+  return ", streamed rows past " + (rows && kn ? packed + " or as it lies" : rows ? packed : std::string("B as it lies")) + " mfma=" + mfma16_name(mfma_kind);
+}
+
 int64_t pml_hip_gemm_dispatch(const pml_hip_gemm_desc* d) {
   const int kind = gemm_desc_kind(d);
   if (kind < 0) return 0;
@@ -930,9 +989,21 @@ int64_t pml_hip_gemm_dispatch(const pml_hip_gemm_desc* d) {
                 (long long)d->m, (long long)d->n, (long long)d->k, tile_name(p->direct.rows >= 0 ? lds_tile : p->tile),
                 kind == KIND_F32 ? "f32_32x32x2" : kind == KIND_BF16 ? "f32_32x32x16_bf16" : kind == KIND_I8 ? "i32_32x32x32_i8" : "3 x f32_32x32x16_bf16 (fp32 split into bf16 head + remainder)");
   p->text = buf;
-  if (p->direct.rows >= 0) p->text += std::string(", with rows of K at hand tile=") + tile_name(p->direct.rows);
+  if (p->direct.rows >= 0) p->text += std::string(", with rows of K at hand tile=") + tile_name(p->direct.rows) + " mfma=" + mfma16_name(kind);
   if (p->direct.given >= 0)
-    p->text += std::string(", with B as it lies tile=") + (p->direct.given == TILE_16x16_W8 ? "16x64" : "32x64") + " (8 wavefronts sharing K)";
+    p->text += std::string(", with B as it lies tile=") + (p->direct.given == TILE_16x16_W8 ? "16x64" : "32x64") + " (8 wavefronts sharing K) mfma=" + mfma16_name(kind);
+  if (p->direct.given < 0 && takes_b_as_given(*d, kind, p->tile, d->ldb))
+    p->text += std::string(", with B as it lies") + (p->b_kn ? " or packed" : "") + " through registers mfma=" + mfma16_name(kind);
+  else if (p->b_kn)
+    p->text += std::string(", with B packed through registers mfma=") + mfma16_name(kind);
+  {
+    IgemmArgs g;
+    gemm_args(*d, g);
+    g.ldbt = d->b_layout ? d->ldb : p->bt_ld;
+    g.ws = p->ws;
+    p->text += stream_text(kind, false, g, d->init_kind != 0, d->tail, p->direct.rows >= 0 ? p->direct.rows : p->tile, !d->b_layout,
+                           p->direct.given >= 0 ? p->direct.given : p->tile, d->b_layout || d->k2 > 0 ? 0 : d->ldb);
+  }
   if (d->k2 > 0) p->text += " + second product k2=" + std::to_string(d->k2) + (d->a2_stride > 0 ? " over pixel rows of stride " + std::to_string(d->a2_stride) : "");
   return (int64_t)(intptr_t)p;
 }
@@ -951,7 +1022,7 @@ struct SecondProduct {
 // Whether a right-hand side that arrives with the call in its row-major [K][N] form is read as it lies: by direct tiles
 // whatever it is, by 256 x 256 tiles of bf16 and int8 through registers, and by the other tiles of fp32 (K-values gathered
 // from [k][n] slabs) and int8 (transposing LDS reads) where rows are whole 16-byte vectors.  Everything else is transposed
-// into Bt[N][K] first, unless its rows stream (streams_given below).
+// into Bt[N][K] first, unless its rows stream (streams_given).
 static bool reads_b_as_given(const pml_hip_gemm_desc& d, int mfma_kind, const void* b, int tile) {
   if ((tile == TILE_16x16_W8 || tile == TILE_32x32_W8) && mfma_kind != KIND_F32X3) {
     // (four neighbouring columns per lane and K-row, whatever the type and wherever the rows begin: direct.hip)
@@ -977,17 +1048,6 @@ static bool reads_b_as_given(const pml_hip_gemm_desc& d, int mfma_kind, const vo
     return 0.15 * t_gemm < t_copy;
   }
   return true;
-}
-
-// Whether a launch streams its rows past the [K][N] right-hand side `b` as it lies, with the arguments then changed to that.
-static bool streams_given(int mfma_kind, int tile, bool conv, const void* b, int64_t ldb, IgemmArgs& g) {
-  if (mfma_kind != KIND_BF16) return false;
-  const void* const bt = g.Bt;
-  const int64_t ldbt = g.ldbt;
-  g.Bt = b, g.ldbt = ldb, g.b_kn = 1;
-  if (stream_takes(tile, conv, g)) return true;
-  g.Bt = bt, g.ldbt = ldbt, g.b_kn = 0;
-  return false;
 }
 
 static int gemm_run(const pml_hip_gemm_desc& d, int mfma_kind, int tile, const DirectTiles& direct, void* bt, int64_t bt_ld, bool packed,
@@ -1022,46 +1082,18 @@ static int gemm_run(const pml_hip_gemm_desc& d, int mfma_kind, int tile, const D
       return 1;
   }
   IgemmArgs g;
-  std::memset(&g, 0, sizeof g);
+  gemm_args(d, g);
   if (d.k2 > 0) {
-    g.K2 = d.k2;
     g.A2 = second->a2;
-    g.lda2 = d.lda2;
     g.Bt2 = d.b_layout ? second->b2 : second->bt2;
-    g.ldbt2 = d.b_layout ? d.ldb2 : d.k2;
     g.init2 = d.init2_kind ? second->init2 : nullptr;
-    g.g2_stride = d.a2_stride;
-    if (d.a2_stride > 0) {
-      g.g2_h = (int)d.a2_h;
-      g.g2_w = (int)d.a2_w;
-      g.g2_ohw = (int)(d.a2_oh * d.a2_ow);
-      g.g2_ow = (int)d.a2_ow;
-      fast_div_magic((unsigned)g.g2_ohw, &g.g2_ohw_magic, &g.g2_ohw_shift);
-      fast_div_magic((unsigned)g.g2_ow, &g.g2_ow_magic, &g.g2_ow_shift);
-    }
   }
-  g.M = d.m;
-  g.N = d.n;
-  g.K = d.k;
   g.A = a;
-  g.lda = d.lda;
   g.Bt = (d.b_layout || b_as_given) && !packed_kn ? b : bt;
   g.ldbt = packed_kn ? d.n : (d.b_layout || b_as_given) ? d.ldb : bt_ld;
   g.b_kn = b_as_given ? 1 : 0;
   g.C = c;
-  g.ldc = d.ldc;
-  g.out_dtype = d.out_dtype;
   g.init = d.init_kind ? init : nullptr;
-  g.init_dtype = d.init_dtype;
-  g.init_rs = d.init_row_stride;
-  g.init_cs = d.init_col_stride;
-  g.c_dtype = d.c_dtype;
-  g.n_cus = device_cus();
-  g.stream = PML_HIP_FLAG_TILE_OF(d.flags) < 0;
-  classify_tail(d.tail, d.out_dtype, d.c_dtype, &g.tail_mode, &g.tail_relu);
-  g.tail_ssr = tail_scale_shift(d.tail, d.out_dtype, g.tail_mode);
-  tail_requant(d.tail, d.out_dtype, d.c_dtype, g.tail_mode, &g);
-  g.tail = d.tail;
   for (int i = 0; i < d.tail.n_operands; ++i) {
     if (!operands || !operands[i]) return fail("gemm_invoke: missing tail operand");
     g.operands[i] = operands[i];
@@ -1263,6 +1295,14 @@ int64_t pml_hip_conv2d_dispatch(const pml_hip_conv2d_desc* d) {
   if (kind == KIND_F32X3) p->text += " mfma=3 x f32_32x32x16_bf16 (fp32 split into bf16 head + remainder)";
   if (p->tile_direct >= 0 && !p->halo_lds) p->text += std::string(", direct tile=") + tile_name(p->tile_direct);
   if (via_patches) p->text += " via patch matrix (k padded to " + std::to_string(p->kpad) + ")";
+  if (!p->halo_lds && !via_s2d) {
+    IgemmArgs g;
+    conv_args(p, g);
+    if (via_patches) g.K = g.lda = p->kpad;
+    g.ws = p->ws;
+    const int tile = p->tile_direct >= 0 ? p->tile_direct : p->tile;
+    p->text += stream_text(kind, !via_patches, g, d->init_kind != 0, d->tail, tile, true, tile, via_patches ? 0 : d->co);
+  }
   if (via_s2d) {
     p->text += " over 2x2 pixel blocks (" + std::to_string(p->s2d_ka) + "x" + std::to_string(p->s2d_kaw) + " block taps of " +
                std::to_string(p->s2d_ch) + " channels, k=" + std::to_string(p->bt_ld) + ")";

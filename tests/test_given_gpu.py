@@ -108,6 +108,34 @@ def test_packed_and_given_in_turn(kind, n, ldb):
     hk.lib().pml_hip_plan_free(plan)
 
 
+@pytest.mark.parametrize('kind', ['bf16', 'i8'])
+@pytest.mark.parametrize('M,N,K,lda,ldb,at', [(257, 260, 144, 160, 268, 4), (300, 64, 512, 528, 1000, 8), (129, 516, 640, 656, 520, 12)])
+def test_strides(kind, M, N, K, lda, ldb, at):
+    """Rows of A and B further apart than they are long, B on any four elements' boundary; the plan's text names the kernel."""
+    rng = np.random.default_rng(M + N)
+    A, B = whole(rng, (M, K)), whole(rng, (K, N))
+    code, es, dt, out, onp = (T.bf16, 2, hk.BF16, hk.F32, np.float32) if kind == 'bf16' else (lambda x: x.astype(np.int8), 1, hk.I8, hk.I32, np.int32)
+    L = hk.lib()
+    d = hk.GemmDesc()
+    d.in_dtype, d.out_dtype, d.c_dtype, d.flags = dt, out, out, T.FORCED['flags']
+    d.m, d.n, d.k, d.lda, d.ldb, d.ldc = M, N, K, lda, ldb, N
+    plan = L.pml_hip_gemm_dispatch(ctypes.byref(d))
+    want = 'with B as it lies or packed through registers mfma=f32_16x16x32_bf16' if kind == 'bf16' else 'with B as it lies through registers mfma=i32_16x16x64_i8'
+    assert plan and want in hk.describe(plan), hk.describe(plan)
+    wide_a, flat_b = np.full((M, lda), 99, np.float32), np.full(at + K * ldb, 99, np.float32)
+    wide_a[:, :K] = A
+    flat_b[at:].reshape(K, ldb)[:, :N] = B
+    dA, dB, dC, none = hk.DeviceBuffer.from_numpy(code(wide_a)), hk.DeviceBuffer.from_numpy(code(flat_b)), hk.DeviceBuffer(M * N * 4), hk.ptr_array([])
+    for b in (dB.ptr + at * es, None):
+        if b is None:
+            hk.check(L.pml_hip_gemm_pack_b(plan, dB.ptr + at * es, None))
+        hk.check(L.pml_hip_fill_u32(dC.ptr, 0xdeadbeef, M * N, None))
+        hk.check(L.pml_hip_gemm_invoke(plan, dA.ptr, b, dC.ptr, None, none, none, None))
+        hk.check(L.pml_hip_stream_sync(None))
+        np.testing.assert_array_equal(dC.to_numpy(onp, (M, N)), A @ B)
+    L.pml_hip_plan_free(plan)
+
+
 @pytest.mark.parametrize('kind,K', [('i8', 64), ('i8', 16), ('bf16', 32), ('bf16', 8)])
 @pytest.mark.parametrize('ldb', [26843544, 26843548, 30000000])
 def test_rows_far_apart(kind, K, ldb):
@@ -124,6 +152,7 @@ def test_rows_far_apart(kind, K, ldb):
     d.m, d.n, d.k, d.lda, d.ldb, d.ldc = M, N, K, K, ldb // 4 * 4, N
     plan = L.pml_hip_gemm_dispatch(ctypes.byref(d))
     assert plan, L.pml_hip_last_error()
+    assert ('with B as it lies' in hk.describe(plan)) == (80 * d.ldb < 2 ** 31 if kind == 'i8' else 40 * d.ldb * 2 < 2 ** 31), hk.describe(plan)
     dA, dB, dC = hk.DeviceBuffer.from_numpy(code(A)), hk.DeviceBuffer(K * d.ldb * es), hk.DeviceBuffer(M * N * 4)
     rows = code(B)
     for k in range(K):

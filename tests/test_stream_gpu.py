@@ -21,27 +21,39 @@ def whole(rng, shape):
     return rng.integers(-4, 5, shape).astype(np.float32)
 
 
-def run(A, B, packed, at=0, pitch=None, bias=None, res=None, relu=False):
-    """Result rows `pitch` values apart that begin `at` values behind a 16-byte boundary, and whether all else was left alone."""
+def spread(x, pitch, at=0):
+    """Rows `pitch` values apart from the `at`-th value on, NaNs between them."""
+    flat = np.full(at + x.shape[0] * pitch, np.nan, np.float32)
+    flat[at:].reshape(-1, pitch)[:, :x.shape[1]] = x
+    return flat
+
+
+def run(A, B, packed, at=0, pitch=None, bias=None, res=None, relu=False, lda=0, ldb=0, ldr=0, b_at=0):
+    """Result rows `pitch` values apart that begin `at` values behind a 16-byte boundary, and whether all else was left alone.
+    Rows of the operands lie whole behind one another, or `lda`, `ldb`, `ldr` values apart; those of the residual tensor on
+    8-byte boundaries (any others take a tile and the interpreted tail).  B begins `b_at` values behind a boundary.  The plan's
+    text has to name the kernel."""
     (M, K), N = A.shape, B.shape[1]
-    pitch = pitch or N
+    pitch, lda, ldb, ldr = pitch or N, lda or K, ldb or N, ldr or (N + 3) // 4 * 4
     d = hk.GemmDesc()
     d.in_dtype = d.out_dtype = d.c_dtype = d.init_dtype = hk.BF16
-    d.m, d.n, d.k, d.lda, d.ldb, d.ldc, d.init_kind, d.init_col_stride = M, N, K, K, N, pitch, int(bias is not None), 1
+    d.m, d.n, d.k, d.lda, d.ldb, d.ldc, d.init_kind, d.init_col_stride = M, N, K, lda, ldb, pitch, int(bias is not None), 1
     ops = [(hk.EPI_ADD, hk.BF16, hk.OPND_TENSOR, 0, 0.0)] * (res is not None) + [(hk.EPI_RELU, hk.BF16, 0, 0, 0.0)] * relu
-    d.tail = hk.make_tail(ops=ops, operands=[(hk.BF16, N, 1)] * (res is not None))
+    d.tail = hk.make_tail(ops=ops, operands=[(hk.BF16, ldr, 1)] * (res is not None))
     L = hk.lib()
     plan = L.pml_hip_gemm_dispatch(ctypes.byref(d))
     assert plan
-    dA, dB = (hk.DeviceBuffer.from_numpy(T.bf16(x)) for x in (A, B))
-    d1, dR = (hk.DeviceBuffer.from_numpy(T.bf16(x)) if x is not None else None for x in (bias, res))
+    text = hk.describe(plan)
+    assert 'streamed rows past B packed' in text and (packed or K > 128 or 'or as it lies' in text), text
+    dA, dB = (hk.DeviceBuffer.from_numpy(T.bf16(x)) for x in (spread(A, lda), spread(B, ldb, b_at)))
+    d1, dR = (hk.DeviceBuffer.from_numpy(T.bf16(x)) if x is not None else None for x in (bias, None if res is None else spread(res, ldr)))
     n = (at + M * pitch + 9) // 2 * 2
     dC = hk.DeviceBuffer(n * 2)
     hk.check(L.pml_hip_fill_u32(dC.ptr, 0xbeefbeef, n // 2, None))
     if packed:
-        hk.check(L.pml_hip_gemm_pack_b(plan, dB.ptr, None))
+        hk.check(L.pml_hip_gemm_pack_b(plan, dB.ptr + 2 * b_at, None))
     for _ in range(2):
-        hk.check(L.pml_hip_gemm_invoke(plan, dA.ptr, None if packed else dB.ptr, dC.ptr + 2 * at, d1.ptr if d1 else None, hk.ptr_array([dR.ptr] if dR else []),
+        hk.check(L.pml_hip_gemm_invoke(plan, dA.ptr, None if packed else dB.ptr + 2 * b_at, dC.ptr + 2 * at, d1.ptr if d1 else None, hk.ptr_array([dR.ptr] if dR else []),
                                        hk.ptr_array([]), None))
     hk.check(L.pml_hip_stream_sync(None))
     L.pml_hip_plan_free(plan)
@@ -74,6 +86,22 @@ def test_tails(M, N, K, at, pitch, packed):
         np.testing.assert_array_equal(run(A, B, packed, at, pitch, bias, res, True), r(keep(r(S + bias) + res)))
 
 
+# rows of every operand further apart than they are long (A by a part of a line, B by an odd number of values and from an odd
+# value on, the residual by half a vector), in each kernel's range of K
+@pytest.mark.parametrize('packed', [0, 1])
+@pytest.mark.parametrize('M,N,K,lda,ldb,b_at,ldr,pitch', [
+    (70001, 200, 56, 72, 203, 1, 204, 200), (70001, 201, 64, 128, 204, 2, 212, 203), (60001, 264, 128, 136, 265, 3, 268, 264), (140001, 7, 96, 104, 9, 1, 8, 7),
+    (36399, 250, 200, 208, 251, 1, 252, 250), (20003, 1024, 256, 320, 1025, 5, 1028, 1024), (20003, 1000, 256, 264, 1000, 0, 1004, 1001)])
+def test_strides(M, N, K, lda, ldb, b_at, ldr, pitch, packed):
+    rng = np.random.default_rng(M + N + K)
+    A, B = whole(rng, (M, K)), whole(rng, (K, N))
+    S = A @ B
+    bias, res = whole(rng, N), whole(rng, (M, N))
+    r, kw = E.round_bf16, dict(lda=lda, ldb=ldb, b_at=b_at, ldr=ldr)
+    np.testing.assert_array_equal(run(A, B, packed, 0, pitch, bias, relu=True, **kw), r(np.maximum(S + bias, 0)))
+    np.testing.assert_array_equal(run(A, B, packed, 0, pitch, bias, res, True, **kw), r(np.maximum(r(S + bias) + res, 0)))
+
+
 @pytest.mark.parametrize('stride', [0, 1])
 @pytest.mark.parametrize('M,N,K,K2', [(81920, 256, 64, 64), (143360, 72, 32, 96), (73728, 136, 96, 24)])
 def test_second_product(M, N, K, K2, stride):
@@ -89,7 +117,7 @@ def test_second_product(M, N, K, K2, stride):
     d.tail = hk.make_tail(ops=[(hk.EPI_RELU, hk.BF16, 0, 0, 0.0)])
     L = hk.lib()
     plan = L.pml_hip_gemm_dispatch(ctypes.byref(d))
-    assert plan
+    assert plan and 'streamed rows past B packed' in hk.describe(plan), hk.describe(plan)
     dA, dB, dA2, dB2, d1, d2 = (hk.DeviceBuffer.from_numpy(T.bf16(x)) for x in (A, B, A2, B2, b1, b2))
     dC, none = hk.DeviceBuffer(M * N * 2), hk.ptr_array([])
     hk.check(L.pml_hip_gemm_pack_b(plan, dB.ptr, None))
@@ -110,7 +138,7 @@ def test_one_by_one_convolution(n, hw, ci, co):
     d.stride_h = d.stride_w = d.dil_h = d.dil_w = d.init_kind = d.init_col_stride = 1
     L = hk.lib()
     plan = L.pml_hip_conv2d_dispatch(ctypes.byref(d))
-    assert plan
+    assert plan and 'streamed rows past B packed' in hk.describe(plan), hk.describe(plan)
     dX, dF, d1 = (hk.DeviceBuffer.from_numpy(T.bf16(x)) for x in (X, F, bias))
     dC, none = hk.DeviceBuffer(n * hw * hw * co * 2), hk.ptr_array([])
     hk.check(L.pml_hip_conv2d_invoke(plan, dX.ptr, dF.ptr, dC.ptr, d1.ptr, none, none, None))
