@@ -285,16 +285,22 @@ bool ragged(const IgemmArgs& g) {
 
 // Whether a bf16 product with the LDS tile `cfg` (a 1x1 convolution with every pixel in its place is one, too) streams its
 // rows instead.  It pays once a wavefront has several steps to spread its start over (its columns of the right-hand side, one
-// load and one MFMA chain that nothing covers): from 130 to 485 products, microseconds, tile -> stream,
-//   K = 32     25088 x 256  9.2 ->  8.4     25088 x 1024  24.3 -> 15.9     401408 x 64  30.5 -> 17.7     401408 x 256  71 ->  40
-//   K = 64     25088 x 256  9.2 (12.0)      25088 x 1024  25.0 -> 20.6     401408 x 64  31.0 -> 22.1     401408 x 256  75 ->  47 (residual 127 -> 97)
-//   K = 128    25088 x 512 15.9 (16.8)      25088 x 1024  27.6 -> 23.4     100352 x 64  11.8 (12.2)      100352 x 512  45 ->  32 (residual  65 -> 46)
-//   K = 200    25088 x 256 11.6 (12.4)      25088 x 1024  35.1 -> 28.4     100352 x 64  16.7 -> 13.7     401408 x 256 153 ->  99 (residual 195 -> 135)
-//   K = 256    12544 x 1024 19.5 (20.0)     25088 x 1024  33.0 -> 29.8     401408 x 64  54.6 -> 45.2     100352 x 512  57 -> 44 (residual  82 -> 64)
-// Past K = 128, rows that are whole lines apart come in slower than others (banks of L1, above).  A [K][N] right-hand side
-// that is read as it lies saves the launch that transposes it, and odd rows of results cost a tile its straight tail:
-//   K = 64     25088 x 128  8.2 ->  6.8     25088 x 256  11.1 ->  8.3    25088 x 251  15.7 -> 12.9     401408 x 123  63 -> 40
-//   K = 128    25088 x 128  9.0 ->  7.5     25088 x 256  12.1 -> 10.3    25088 x 251  16.3 -> 12.9     100352 x 510  61 -> 46
+// load and one MFMA chain that nothing covers), so the rule counts the steps of each wavefront that the device holds, eight on
+// a CU.  How many it takes shrinks with what a row costs a tile: a residual to fetch, odd rows of results that take its
+// row-by-row tail.  Past K = 128 rows that are whole lines apart come in slower than others (banks of L1, above).  A [K][N]
+// right-hand side costs a tile a transposed copy: wherever no direct tile is taken (the caller's choice, before this one), its
+// rows stream.  Microseconds tile -> stream, in brackets what keeps its tile, back to back in a recorded graph over buffers in
+// turn; the lines lie where 820 products of 48 to 2000 columns and 300 to 25000 steps cross over:
+//   steps a wavefront (256 CUs: 2048)
+//   3/2    K = 32     25088 x 256   8.9 ->  7.1    25088 x 1024  24.3 -> 18.7    401408 x 64  34.3 -> 22.1    401408 x 256   80 ->  66
+//   17/4   K = 64     25088 x 256   9.0 ( 9.8)     25088 x 1024  24.4 -> 23.6    401408 x 64  33.8 -> 26.0    401408 x 256   84 ->  75 (residual 126 ->  94)
+//          K = 128    25088 x 512  15.5 (16.6)     25088 x 1024  30.0 -> 29.3    100352 x 64  12.1 (12.5)     100352 x 512   52 ->  46 (residual  75 ->  57)
+//   13/4   K = 200    25088 x 256  12.3 (12.5)     25088 x 1024  36.3 -> 29.0                                 401408 x 256  152 ->  96 (residual 193 -> 133)
+//   3        up to 64 columns, odd rows, residual                                100352 x 64  21.6 -> 16.8    25088 x 256                (residual 15.8 -> 13.4)
+//   39/4   K = 256    12544 x 1024 17.9 (19.5)     25088 x 1024  36.6 -> 32.8    401408 x 64  66.5 -> 53.7    100352 x 512   67 ->  60 (residual  88 ->  75)
+//   17/4     odd rows, residual                    35000 x 250   20.1 -> 18.5                                 25088 x 512                (residual 26.7 -> 26.5)
+//   any    [K][N] as it lies, K = 64: 19200 x 128 8.1 -> 6.3, 25088 x 128 8.2 -> 6.6, 25088 x 256 11.1 -> 8.4, 25088 x 251 15.7 -> 13.3, 401408 x 123 70 -> 62
+//                             K = 128: 8000 x 200 7.5 -> 6.2, 25088 x 128 9.5 -> 8.0, 25088 x 256 12.1 -> 10.4, 25088 x 251 16.7 -> 13.3, 100352 x 510 68.3 -> 68.6
 bool stream_takes(int cfg, bool conv, const IgemmArgs& g) {
   if (!g.stream || cfg == TILE_16x16_W8 || cfg == TILE_32x32_W8 || (cfg == TILE_64x64_KSPLIT && g.ws)) return false;
   if (conv && (g.KH != 1 || g.KW != 1 || g.SH != 1 || g.SW != 1 || g.PH != 0 || g.PW != 0 || g.OH != g.H || g.OW != g.W || g.pix_pitch != 0 ||
@@ -313,9 +319,12 @@ bool stream_takes(int cfg, bool conv, const IgemmArgs& g) {
   if (g.init2 && ((uintptr_t)g.init2 & 1) != 0) return false;
   const int64_t ldr = g.tail_mode == 2 ? g.tail.operand_row_stride[0] : 0;
   if (ldr < 0 || (g.tail_mode == 2 && (((uintptr_t)g.operands[0] & 1) != 0 || g.tail.operand_col_stride[0] != 1))) return false;
-  const int64_t kk = K + g.K2, groups = kk <= (g.b_kn ? 64 : 128) ? (g.N + 127) / 128 : (g.N + 63) / 64, steps = (g.M + kRows - 1) / kRows * groups;
-  const int64_t least = g.b_kn ? 1600 : kk <= 32 ? 3000 : kk <= 128 ? 8700 : lda % 64 != 0 ? 6200 : odd_rows || g.tail_mode == 2 ? 8700 : 20000;
-  if (steps < least) return false;
+  if (!g.b_kn) {
+    const int64_t kk = K + g.K2, groups = kk <= 128 ? (g.N + 127) / 128 : (g.N + 63) / 64, steps = (g.M + kRows - 1) / kRows * groups;
+    const bool costly = odd_rows || g.tail_mode == 2;
+    const int quarters = kk <= 32 ? 6 : kk <= 128 ? 17 : lda % 64 != 0 ? (costly || g.N <= 64 ? 12 : 13) : costly ? 17 : 39;
+    if (4 * steps < quarters * 8 * (int64_t)g.n_cus) return false;
+  }
   // byte offsets of 31 bits, also for the steps a wavefront looks ahead
   const int64_t limit = ((int64_t)1 << 30) - 1;
   return (g.M + 64) * std::max({lda, g.ldc, ldr, g.K2 > 0 ? g.lda2 : 0}) <= limit && (g.b_kn ? K + 8 : g.N) * std::max(g.ldbt, g.K2 > 0 ? g.ldbt2 : 0) <= limit;

@@ -32,3 +32,16 @@ def test_streamed_rows_are_named():
 @pytest.mark.parametrize('dt,mfma', [(hk.F32, 'f32_16x16x4'), (hk.BF16, 'f32_16x16x32_bf16'), (hk.I8, 'i32_16x16x64_i8')])
 def test_direct_tiles_name_their_instruction(dt, mfma):
     assert text(49, 512, 512, dt=dt).endswith('(8 wavefronts sharing K) mfma=' + mfma)
+
+
+# (both sides of each line of the rule, products that were timed on both sides of it; a device of 256 compute units, which is
+# also what is assumed where there is none)
+@pytest.mark.parametrize('m,n,k,lda,ldr,takes', [
+    (24576, 256, 32, 32, None, True), (24560, 256, 32, 32, None, False), (25088, 256, 64, 64, None, False), (69632, 256, 64, 64, None, True), (69616, 256, 64, 64, None, False),
+    (25088, 512, 128, 128, None, False), (100352, 64, 128, 128, None, False), (100352, 512, 128, 128, None, True), (25088, 256, 200, 200, None, False),
+    (25088, 256, 200, 200, 256, True), (100352, 64, 200, 200, None, True), (100352, 64, 200, 256, None, False), (26624, 256, 200, 200, None, True),
+    (26608, 256, 200, 200, None, False), (25088, 251, 200, 200, None, True), (12544, 1024, 256, 256, None, False), (25088, 1024, 256, 256, None, True),
+    (25088, 512, 256, 256, 512, True), (25088, 512, 256, 256, None, False), (35000, 250, 256, 256, None, True), (25088, 512, 256, 264, None, True)])
+def test_which_rows_stream(m, n, k, lda, ldr, takes):
+    got = text(m, n, k, lda=lda, ldr=ldr)
+    assert ('streamed' in got) == takes, got

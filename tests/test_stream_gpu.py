@@ -44,7 +44,7 @@ def run(A, B, packed, at=0, pitch=None, bias=None, res=None, relu=False, lda=0, 
     plan = L.pml_hip_gemm_dispatch(ctypes.byref(d))
     assert plan
     text = hk.describe(plan)
-    assert 'streamed rows past B packed' in text and (packed or K > 128 or 'or as it lies' in text), text
+    assert ('streamed rows past B packed' if packed or K > 128 else 'as it lies mfma') in text and 'streamed' in text, text
     dA, dB = (hk.DeviceBuffer.from_numpy(T.bf16(x)) for x in (spread(A, lda), spread(B, ldb, b_at)))
     d1, dR = (hk.DeviceBuffer.from_numpy(T.bf16(x)) if x is not None else None for x in (bias, None if res is None else spread(res, ldr)))
     n = (at + M * pitch + 9) // 2 * 2
@@ -146,3 +146,25 @@ def test_one_by_one_convolution(n, hw, ci, co):
     want = E.round_bf16(X.reshape(-1, ci) @ F.reshape(ci, co) + bias)
     np.testing.assert_array_equal(E.bf16_from_bits(dC.to_numpy(np.uint16, (n * hw * hw, co))), want)
     L.pml_hip_plan_free(plan)
+
+
+@pytest.mark.parametrize('M,N,K,takes', [(25088, 128, 64, True), (19200, 128, 64, True), (17600, 128, 64, False), (8000, 200, 128, True), (12288, 128, 128, False), (25088, 128, 136, False)])
+def test_which_rows_stream_past_a_right_hand_side_as_it_lies(M, N, K, takes):
+    """Those that no direct tile takes, up to K = 128."""
+    d = hk.GemmDesc()
+    d.in_dtype = d.out_dtype = d.c_dtype = hk.BF16
+    d.m, d.n, d.k, d.lda, d.ldb, d.ldc = M, N, K, K, N, N
+    plan = hk.lib().pml_hip_gemm_dispatch(ctypes.byref(d))
+    assert plan
+    text = hk.describe(plan)
+    hk.lib().pml_hip_plan_free(plan)
+    assert ('streamed rows past B as it lies' in text or 'or as it lies' in text) == takes, text
+    assert takes or K > 128 or 'with B as it lies tile=' in text, text
+
+
+# few rows and steps fewer than the device has wavefronts
+@pytest.mark.parametrize('M,N,K', [(1374, 2000, 32), (4795, 511, 64), (8001, 200, 128), (9600, 251, 64)])
+def test_few_steps(M, N, K):
+    rng = np.random.default_rng(M)
+    A, B, bias = whole(rng, (M, K)), whole(rng, (K, N)), whole(rng, N)
+    np.testing.assert_array_equal(run(A, B, 0, bias=bias, relu=True), E.round_bf16(np.maximum(A @ B + bias, 0)))
