@@ -864,7 +864,8 @@ __device__ __forceinline__ void tile_tail(const IgemmArgs& p, const typename Acc
     return;
   }
 
-  // The same tails where the last quad of columns is not whole, or rows of C begin anywhere: row by row, and not unrolled -- the
+  // The same tails where the last quad of columns is not whole, or rows of C begin anywhere (of a residual tensor's rows only
+  // those on quads' boundaries get here: classify_tail): row by row, and not unrolled -- the
   // unrolled code above, with the checks this takes in it, spilled 90 registers of the 128 some tiles may have.  (Before
   // this the interpreter below ran every result of such a problem: bf16 1402 x 162, K = 2528 29.9 -> 27.7 us, int8 129 x 35,
   // K = 912 with requantisation 53.9 -> 12.6, 1636 x 749, K = 400 58.1 -> 12.8, a float convolution to 7 x 47 x 47 x 19

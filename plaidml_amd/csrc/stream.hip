@@ -16,8 +16,8 @@
 // KN: a right-hand side that arrives as [K][N] is read as it lies, once: four neighbouring columns of every K-row per lane,
 // turned with v_perm into the fragments of four blocks, block j of 64 columns holding the columns 4 i + j; a lane then ends
 // with 16 neighbouring columns.  RAGGED: rows of results that begin and end anywhere; a lane's eight columns are one store
-// wherever they lie, value by value behind the last whole eight, and residual values are fetched as the aligned words around
-// them and shifted together.
+// wherever they lie, value by value behind the last whole eight.  Rows of the residual tensor begin on 8 bytes in either form:
+// products with any other run the interpreted tail of a tile (classify_tail).
 #include <hip/hip_runtime.h>
 
 #include "device_common.h"
@@ -139,11 +139,10 @@ __global__ __launch_bounds__(kThreads, OCC) void stream_kernel(StreamArgs p) {
   }
 
   const unsigned a_lane = (unsigned)(r * (int)p.lda + 8 * g) * 2, a2_lane = (unsigned)(r * (int)p.lda2 + 8 * g - k1) * 2;
-  const unsigned r_lane = (unsigned)(r * (int)p.ldr + col0) * 2 + (RAGGED ? (unsigned)((uintptr_t)p.res & 2) : 0u), c_lane = (unsigned)(r * (int)p.ldc + col0) * 2;
+  const unsigned r_lane = (unsigned)(r * (int)p.ldr + col0) * 2, c_lane = (unsigned)(r * (int)p.ldc + col0) * 2;
   const int k_left = p.K - 8 * g, k2_left = k1 + p.K2 - 8 * g, n_left = p.N - col0;
   auto rows_at = [](unsigned lane_at, int step, int64_t pitch) { return lane_at + (unsigned)step * (unsigned)(kRows * 2 * (int)pitch); };
   i32x4_t fa[D][KS], res[D][RES ? NP : 1];
-  uint32_t res_end[D][RES && RAGGED ? NP : 1];
   auto request = [&](int d, int step) {
     const bool live = step < steps;
     const unsigned a_at = rows_at(a_lane, step, p.lda), a2_at = rows_at(a2_lane, step, p.lda2), r_at = rows_at(r_lane, step, p.ldr);
@@ -155,12 +154,7 @@ __global__ __launch_bounds__(kThreads, OCC) void stream_kernel(StreamArgs p) {
     }
     if constexpr (RES) {
 #pragma unroll
-      for (int q = 0; q < NP; ++q) {
-        const bool in = live & (behind(q) < n_left);
-        const unsigned at = (r_at & (RAGGED ? ~3u : ~0u)) + 2 * behind(q);
-        res[d][q] = fetch(rr, in, at);
-        if constexpr (RAGGED) res_end[d][q] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rr, (int)(in ? at + 16 : kOutside), 0, 0);
-      }
+      for (int q = 0; q < NP; ++q) res[d][q] = fetch(rr, live & (behind(q) < n_left), r_at + 2 * behind(q));
     }
   };
 
@@ -212,14 +206,7 @@ __global__ __launch_bounds__(kThreads, OCC) void stream_kernel(StreamArgs p) {
         if constexpr (RES) {
           // the contraction result is rounded first, then the bf16 addition rounds again
           float f[8];
-          i32x4_t bits = res[d][q];
-          if constexpr (RAGGED) {
-            const unsigned shift = (rows_at(r_lane, step, p.ldr) & 3) * 8;
-#pragma unroll
-            for (int w = 0; w < 4; ++w)
-              bits[w] = (int)__builtin_amdgcn_alignbit(w < 3 ? (uint32_t)res[d][q][w < 3 ? w + 1 : 3] : res_end[d][q], (uint32_t)res[d][q][w], shift);
-          }
-          unpack_bf16x8(bits, f);
+          unpack_bf16x8(res[d][q], f);
 #pragma unroll
           for (int e = 0; e < 8; e += 2) round_pair_to_bf16(v[e], v[e + 1]);
 #pragma unroll
@@ -318,7 +305,7 @@ bool stream_takes(int cfg, bool conv, const IgemmArgs& g) {
   if (g.init && !(g.init_rs == 0 && g.init_cs == 1 && g.init_dtype == PML_HIP_BF16 && ((uintptr_t)g.init & 1) == 0)) return false;
   if (g.init2 && ((uintptr_t)g.init2 & 1) != 0) return false;
   const int64_t ldr = g.tail_mode == 2 ? g.tail.operand_row_stride[0] : 0;
-  if (ldr < 0 || (g.tail_mode == 2 && (((uintptr_t)g.operands[0] & 1) != 0 || g.tail.operand_col_stride[0] != 1))) return false;
+  if (ldr < 0 || (g.tail_mode == 2 && ((ldr & 3) != 0 || ((uintptr_t)g.operands[0] & 7) != 0 || g.tail.operand_col_stride[0] != 1))) return false;
   if (!g.b_kn) {
     const int64_t kk = K + g.K2, groups = kk <= 128 ? (g.N + 127) / 128 : (g.N + 63) / 64, steps = (g.M + kRows - 1) / kRows * groups;
     const bool costly = odd_rows || g.tail_mode == 2;
