@@ -1,5 +1,7 @@
 """Tails of products and convolutions whose last columns are no whole quad and whose rows begin anywhere (csrc/igemm_tail.h):
 whole numbers, so that every tail is compared value for value with numpy, through tiles whose sums pass through LDS."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -94,3 +96,38 @@ def test_filter_rows_as_one_tap(kind, tile, shape, kh, kw, co, stride, monkeypat
     pad[:, ph:ph + h, pw:pw + w] = I
     want = sum(pad[:, y:y + (oh - 1) * stride + 1:stride, x:x + (ow - 1) * stride + 1:stride] @ F[y, x].astype(np.float64) for y in range(kh) for x in range(kw))
     np.testing.assert_array_equal(E.bf16_from_bits(got) if kind == 'bf16' else got, E.round_bf16(want.astype(np.float32)) if kind == 'bf16' else want)
+
+
+@pytest.mark.parametrize('kind', ['f32', 'f32x3', 'bf16', 'i8'])
+@pytest.mark.parametrize('packed', [False, True])
+@pytest.mark.parametrize('tile', [None, '64x64', '128x128w8', '64x64ks', '32x32w8'])
+@pytest.mark.parametrize('shape,kh,kw,co,stride,dil', [((2, 9, 5, 16), 5, 3, 20, 1, 2), ((1, 13, 9, 48), 3, 5, 70, 2, 3), ((1, 8, 11, 112), 2, 3, 33, 1, 4)])
+def test_filter_rows_as_one_tap_dilated(kind, packed, tile, shape, kh, kw, co, stride, dil):
+    """The same with filter rows further apart (the taps of a row stay neighbours), fp32 as three bf16 products among the kinds,
+    where every value counts as whole numbers do; filters that arrive with the call and packed ones."""
+    rng = np.random.default_rng(co + dil)
+    n, h, w, ci = shape
+    I, F = whole(rng, shape), whole(rng, (kh, kw, ci, co))
+    dt, out, cast, onp = {'f32': (hk.F32, hk.F32, lambda a: a, np.float32), 'f32x3': (hk.F32, hk.F32, lambda a: a, np.float32), 'bf16': (hk.BF16, hk.F32, T.bf16, np.float32),
+                          'i8': (hk.I8, hk.I32, lambda a: a.astype(np.int8), np.int32)}[kind]
+    d = hk.Conv2dDesc()
+    d.in_dtype, d.out_dtype, d.c_dtype = dt, out, out
+    d.flags = hk.flag_conv(hk.CONV_IGEMM) | (hk.flag_tile(tile) if tile else 0) | (hk.FP32_AS_BF16X3 if kind == 'f32x3' else 0)
+    ph, pw = (kh - 1) * dil // 2, (kw - 1) // 2
+    oh, ow = (h + 2 * ph - (kh - 1) * dil - 1) // stride + 1, (w + 2 * pw - kw) // stride + 1
+    d.n, d.h, d.w, d.ci, d.kh, d.kw, d.co, d.oh, d.ow = n, h, w, ci, kh, kw, co, oh, ow
+    d.stride_h = d.stride_w = stride
+    d.dil_h, d.dil_w, d.pad_h, d.pad_w = dil, 1, ph, pw
+    L = hk.lib()
+    plan = L.pml_hip_conv2d_dispatch(ctypes.byref(d))
+    assert plan, L.pml_hip_last_error()
+    dI, dF, dO, none = hk.DeviceBuffer.from_numpy(cast(I)), hk.DeviceBuffer.from_numpy(cast(F)), hk.DeviceBuffer(n * oh * ow * co * 4), hk.ptr_array([])
+    if packed:
+        hk.check(L.pml_hip_conv2d_pack_filter(plan, dF.ptr, None))
+    hk.check(L.pml_hip_conv2d_invoke(plan, dI.ptr, None if packed else dF.ptr, dO.ptr, None, none, none, None))
+    hk.check(L.pml_hip_stream_sync(None))
+    L.pml_hip_plan_free(plan)
+    pad = np.zeros((n, h + 2 * ph, w + 2 * pw, ci))
+    pad[:, ph:ph + h, pw:pw + w] = I
+    want = sum(pad[:, y * dil:y * dil + (oh - 1) * stride + 1:stride, x:x + (ow - 1) * stride + 1:stride] @ F[y, x].astype(np.float64) for y in range(kh) for x in range(kw))
+    np.testing.assert_array_equal(dO.to_numpy(onp, (n, oh, ow, co)), want)
