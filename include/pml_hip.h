@@ -346,11 +346,15 @@ int pml_hip_tile_of_workgroup(int tiles_m, int tiles_n, int workgroup, int* tile
  * own, lives in a fixed array in the library's device image instead: n * k * element size must not exceed
  * PML_HIP_STATIC_SCRATCH_BYTES, larger right-hand sides are rejected with an error text that says so
  * (b_layout 1 needs no copy and has no such limit; a right-hand side that the kernels read where it lies leaves the
- * array untouched -- fp32 with n and ldb multiples of four and 16-byte aligned, int8 with rows of whole 16-byte
- * vectors on problems where transposing reads cost less than the copy -- and the limit applies all the same).
+ * array untouched -- with few result tiles in any type, in large bf16 and int8 products whose n and ldb are multiples of
+ * four, in bf16 products of many rows and k <= 128, fp32 with n and ldb multiples of four and 16-byte aligned, int8 with
+ * rows of whole 16-byte vectors on problems where transposing reads cost less than the copy -- and the limit applies all
+ * the same).
  * Each GPU holds one such array for the life of the process and
  * every call on that GPU uses it: calls that overlap on one GPU (two streams, two threads) race on it.  The
- * result equals pml_hip_gemm_dispatch + pml_hip_gemm_invoke bit for bit (same tile choice, same kernels). */
+ * result equals pml_hip_gemm_dispatch + pml_hip_gemm_invoke bit for bit (same tile choice, same kernels) except where a
+ * plan shares the K loop out among workgroups, which takes memory of its own: sums of floats are then added in another
+ * order. */
 #define PML_HIP_STATIC_SCRATCH_BYTES (32 * 1024 * 1024)
 int pml_hip_gemm_run_static(const pml_hip_gemm_desc* desc, const void* a, const void* b, void* c, const void* init,
                             const void* const* operands, void* const* outs, pml_hip_stream s);

@@ -1,7 +1,7 @@
 // Large products of bf16 or int8 over a right-hand side B[K][N] as it lies: 256 x 256 tiles, A through LDS, B through
 // registers.
 //
-// What bounds a 256 x 256 tile that stages both operands in LDS (igemm.hip) is LDS itself: eight wavefronts of 128 x 64 read
+// A 256 x 256 tile that stages both operands in LDS (igemm.hip) uses LDS up: eight wavefronts of 128 x 64 read
 // 192 bytes of fragments per byte of K where the ring's refill writes another 64, together the 128 bytes per clock and
 // CU that LDS moves -- and a [K][N] right-hand side has to be transposed by a launch of its own before that.  Here only
 // A goes through LDS (160 bytes instead of 256 per byte of K, and room for a ring of four slabs instead of two).  B goes
@@ -12,11 +12,14 @@
 // of B and the ones its A fragment holds.  (32 x 32 MFMAs leave two columns per lane, twice the requests of half the
 // width: bf16 4096^3 115 us.)  There is no transposed copy, no wait for memory at the one barrier of a slab, and the
 // requests are spread evenly between the MFMAs.
-// Measured on N(0,1) / uniform int8 data, B arriving with the call:
-//   bf16 4096^3  133 us (transposed copy 13, igemm 120) -> 104 (1.32 PFLOP/s).  Parts of it compiled out: MFMAs alone 85
-//                (with launch and tail), with A's fragment reads 91, with A's requests 97.
-//   int8 4096^3  73 us (9 + 64) -> 62 (2.2 POP/s); bound by instruction issue: per slab and wavefront 64 MFMAs, 32 requests
-//                and 64 permutations for B (a byte matrix is turned four rows at a time), 16 fragment reads.
+// Measured on N(0,1) / uniform int8 data, B arriving with the call, ranges over boxes:
+//   bf16 4096^3  133 us (transposed copy 13, igemm 120) -> 104-114 with bias and relu (1.21-1.32 PFLOP/s).  It spends as many
+//                cycles as the tile over Bt, the matrix pipe busy for 68 % of them, at a higher clock (1.71 GHz for 1.63 on
+//                one box, 107.6 us for 113.6): less passes through LDS.  Parts of it compiled out: MFMAs alone 85 (with
+//                launch and tail), with A's fragment reads 91, with A's requests 97.
+//   int8 4096^3  73 us (9 + 64) -> 62-68 requantised (2.0-2.2 POP/s), 72 as int32 sums, where the tile over Bt takes 69: matrix
+//                pipe busy 40 %, the other vector instructions (64 permutations for B per slab and wavefront; a byte matrix
+//                is turned four rows at a time) another 22, and 256 tiles on 256 CUs that write their 67 MB at once 17.
 #include <hip/hip_runtime.h>
 
 #include "device_common.h"

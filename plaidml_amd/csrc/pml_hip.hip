@@ -899,7 +899,7 @@ int pml_hip_gemm_tail_cheaper_apart(const pml_hip_gemm_desc* d) {
 
 // Whether a product's 256 x 256 tile reads B[K][N] with rows of `ldb` elements as it lies: four neighbouring columns per lane
 // and K-row, through registers (given.hip).  For bf16 it is then the better form of a packed right-hand side, too: 4096^3 from
-// the [K][N] copy 104 us, from Bt through LDS 122 (int8, back to back until the clock settles: 72 and 68).
+// the [K][N] copy 107.6 us, from Bt through LDS 113.6 (int8: 72.8 and 69.0; all back to back until the clock settles).
 static bool takes_b_as_given(const pml_hip_gemm_desc& d, int mfma_kind, int tile, int64_t ldb) {
   return tile == TILE_256x256_W8 && (mfma_kind == KIND_BF16 || mfma_kind == KIND_I8) && !d.b_layout && d.k2 == 0 && d.n % 4 == 0 &&
          ldb % 4 == 0 && given_span(d.k, ldb, dt_size(d.in_dtype)) < ((int64_t)1 << 31);
