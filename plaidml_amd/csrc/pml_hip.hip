@@ -276,7 +276,7 @@ int choose_tile(int64_t m, int64_t n, int64_t k_bytes, int kind = KIND_BF16, boo
   if (kind == KIND_F32X3) {
     // A fragment that is split in registers costs 24 vector instructions whatever it is multiplied with, so the
     // tile a wavefront holds decides how many MFMAs share that cost -- but the problems this kind meets here are
-    // short of tiles first.  Measured: configs[1] fp32 (n = 64) 137 us with 64x64, 146 with 128x64 as 32x64 per
+    // short of tiles first.  Measured: 128 x 56 x 56 x 64 (*) 3 x 3 x 64 137 us with 64x64, 146 with 128x64 as 32x64 per
     // wavefront, 155 with 128x64 as 64x32; 1024^3 25-27 us with 64x64 (either form), 34-47 with larger tiles.
     if (n > 64 && tiles(128, 128) >= 512) return TILE_128x128;
     if (tiles(64, 64) <= 512 && k_bytes >= 2048) return TILE_64x64_W8_K2;
