@@ -228,7 +228,8 @@ enum {
   PML_HIP_CONV_IGEMM = 1,     /* implicit GEMM, never a resident-filter or row-walking kernel */
   PML_HIP_CONV_PATCHES = 2,   /* few-channel inputs through a patch matrix even where 2x2 pixel blocks would do */
   PML_HIP_CONV_LDSFILTER = 3, /* resident filter kept in LDS rather than in registers */
-  PML_HIP_CONV_BLOCKS = 4     /* the row-walking stem kernel behind a separate re-blocking launch */
+  PML_HIP_CONV_BLOCKS = 4,    /* the row-walking stem kernel behind a separate re-blocking launch */
+  PML_HIP_CONV_WINDOW = 5     /* every tile's input window in LDS, read there once per tap, where the shape allows it */
 };
 #define PML_HIP_FLAG_TILE(t) ((((t) + 1) & 0xff) << 8)
 #define PML_HIP_FLAG_CONV(c) (((c) & 0xf) << 16)

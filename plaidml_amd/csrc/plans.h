@@ -249,6 +249,22 @@ bool regfilter_takes_image(int ow);  // rows of `ow` output pixels leave the ima
 // row-walking kernel, or 0 when `a` (already pointing at the re-blocked input) does not qualify.
 size_t conv_blocks4x4_prepare(int kind, const IgemmArgs& a);
 hipError_t conv_blocks4x4_launch(const IgemmArgs& a, size_t lds_bytes, int n_cus, hipStream_t s);
+// Convolutions with their input window in LDS (winconv.hip).  A shape: one of the kernel's configurations, results a tile's
+// rows hold, 64-byte blocks of channels that a window holds, windows.  config -1: the convolution is not one for this kernel.
+struct WinShape {
+  int config = -1, rows = 0, blocks = 0, windows = 0;
+};
+// The cheapest shape for a convolution whose descriptor's part of `a` is filled in, and the microseconds it is expected to take.
+WinShape winconv_shape(int kind, const IgemmArgs& a, double* us);
+std::string winconv_text(const WinShape& shape);
+// Its filter: value k of column n of a tap at first + tap * tap_stride + k * k_stride + n * n_stride.
+struct WinFilter {
+  int taps, k, n;
+  int64_t first, tap_stride, k_stride, n_stride;
+};
+size_t winconv_pack_bytes(int es, int taps, int64_t k, int64_t n);
+hipError_t winconv_pack_launch(int es, const void* filter, const WinFilter& w, void* out, hipStream_t s);
+hipError_t winconv_launch(int kind, const IgemmArgs& a, const WinShape& shape, hipStream_t s);  // a.Bt: the packed filter
 hipError_t mfma_probe_launch(int blocks, int iters, int random, float* sink, unsigned long long* clk, hipStream_t s);
 // splits a packed fp32 Bt[rows][ld] in place (k values per row, a multiple of 32) into the heads / remainders form
 hipError_t split_rows_launch(void* bt, int64_t rows, int64_t ld, int64_t k, hipStream_t s);

@@ -91,6 +91,8 @@ struct Plan {
   // the direct tiles a product takes instead of `tile`, and the one a convolution takes (-1: none)
   DirectTiles direct;
   int tile_direct = -1;
+  // a convolution that runs over its window in LDS (`bt` holds the filter as that kernel multiplies it)
+  WinShape win;
   // register-filter convolution: a filter packed once, in the order the kernel holds it in registers
   void* reg_image = nullptr;
   // product over free strides, and a convolution's gradients built on it: the prepared arguments (workspace in `ws`),
@@ -166,7 +168,7 @@ const char* tile_name(int t) {
 constexpr int kScheduleBits = 0xff << 8 | 0xf << 16;
 constexpr int kMaxpoolBits = 0x1f << 20;
 bool schedule_bits_ok(int flags) {
-  return PML_HIP_FLAG_TILE_OF(flags) < PML_HIP_TILE_COUNT_ && PML_HIP_FLAG_CONV_OF(flags) <= PML_HIP_CONV_BLOCKS;
+  return PML_HIP_FLAG_TILE_OF(flags) < PML_HIP_TILE_COUNT_ && PML_HIP_FLAG_CONV_OF(flags) <= PML_HIP_CONV_WINDOW;
 }
 const char* const kTileShort[PML_HIP_TILE_COUNT_] = {"64x64", "128x64", "128x128", "128x64w8", "128x128w8", "256x128w16", "128x128w8s2", "64x64w8k2", "256x256w8", "128x64n2", "192x384w8", "64x64ks", "16x16w8", "32x32w8"};
 
@@ -203,7 +205,7 @@ bool splits_k(int64_t m, int64_t n, int64_t k_bytes, int kind) {
 // kn_ldb: that right-hand side's row pitch in bytes (0: Bt); always: the better of the two whatever the LDS kernel takes;
 // can_split: the LDS kernel may split K; as_given: it reads a [K][N] right-hand side as it lies (256 x 49152, K = 4096 bf16:
 // 409 us direct, 135 with 256 x 256 tiles; charged the copy of 800 MB, they lost)
-int direct_tile_of(int64_t m, int64_t n, int64_t k_bytes, int kind, int64_t kn_ldb = 0, bool always = false, bool can_split = true, bool as_given = false) {
+int direct_tile_of(int64_t m, int64_t n, int64_t k_bytes, int kind, int64_t kn_ldb = 0, bool always = false, bool can_split = true, bool as_given = false, double* us = nullptr) {
   if (kind != KIND_F32 && kind != KIND_BF16 && kind != KIND_I8) return -1;
   auto tiles = [&](int64_t bm, int64_t bn) { return ((m + bm - 1) / bm) * ((n + bn - 1) / bn); };
   const double kb = (double)k_bytes;
@@ -234,7 +236,9 @@ int direct_tile_of(int64_t m, int64_t n, int64_t k_bytes, int kind, int64_t kn_l
   }
   if (kn && needs_bt) lds_us += 3.0 + 2.0 * kb * (double)n / 2.2e6;
   const double small = direct_us(16), large = direct_us(32);
-  if (!always && std::min(small, large) > 0.95 * lds_us) return -1;
+  const bool direct = always || std::min(small, large) <= 0.95 * lds_us;
+  if (us) *us = direct ? std::min(small, large) : lds_us;
+  if (!direct) return -1;
   return small <= large ? TILE_16x16_W8 : TILE_32x32_W8;
 }
 
@@ -658,10 +662,45 @@ void s2d_args(const Plan* p, S2dArgs& a) {
   a.EH = (int)d.pad_h & 1, a.EW = (int)d.pad_w & 1;
 }
 
+// Whether and how a convolution runs over its window in LDS (winconv.hip) in the place of an implicit GEMM.
+//   * an implicit GEMM fetches every pixel once per tap: bf16 and int8 always run over windows, 1.2 to 2.6 x as fast (bf16 128 x
+//     28 x 28 x 128 (*) 3 x 3 x 128 44 -> 31 us, 103 x 11 x 11 x 256 (*) 7 x 7 x 29 74.8 -> 28.3).  fp32 is bound by its MFMAs: where
+//     they are not mostly work done for edges, which a tile of 448 x 64 has more of than one of 64 x 64.
+//   * a direct tile, or a K loop split over workgroups, is left where the window is cheaper by these kernels' prices, which are
+//     a microsecond below what launches back to back take (bf16 22 x 11 x 11 x 128 (*) 5 x 5 x 86 15.3 -> 10.4 from a split;
+//     11 x 11 x 11 x 64 (*) 3 x 3 x 20 stays, 5.5 both ways; 3 x 30 x 30 x 256 (*) 7 x 7 x 18 stride 2 stays, 14.6, over windows 34.6).
+//   * 3 x 3 filters that the kernels of conv_halo.hip keep on the chip stay there (128 x 56 x 56 x 64 (*) 3 x 3 x 64 36); their general
+//     form for any other filter that fits LDS does not (40 x 30 x 30 x 64 (*) 3 x 3 x 48 23.9 -> 9.1).
+WinShape window_shape(Plan* p, bool named) {
+  const pml_hip_conv2d_desc& d = p->conv;
+  const int out = p->mfma_kind == KIND_BF16 ? PML_HIP_BF16 : p->mfma_kind == KIND_I8 ? PML_HIP_I32 : PML_HIP_F32;
+  if (d.init_kind && !(d.init_row_stride == 0 && d.init_col_stride == 1 && d.init_dtype == out)) return {};
+  IgemmArgs g;
+  conv_args(p, g);
+  double us = 0;
+  const WinShape shape = winconv_shape(p->mfma_kind, g, &us);
+  if (shape.config < 0 || named) return shape;
+  // (a last block of channels that is mostly empty, int8 of 96 channels: 62 x 45 x 45 x 96 (*) 5 x 5 x 23 stride 2 15.4, over windows 17.0)
+  const int64_t ci_bytes = d.ci * dt_size(d.in_dtype);
+  if ((ci_bytes + 63) / 64 * 64 * 5 > ci_bytes * 6) return {};
+  const int64_t k_bytes = g.K * dt_size(d.in_dtype);
+  if (p->tile_direct >= 0 || splits_k(g.M, g.N, k_bytes, p->mfma_kind)) {
+    double other = 0;
+    (void)direct_tile_of(g.M, g.N, k_bytes, p->mfma_kind, 0, false, true, false, &other);
+    return us < 0.95 * other + 0.6 ? shape : WinShape{};
+  }
+  if (p->mfma_kind == KIND_F32) {
+    const double mma_us = (double)((g.M + 63) / 64 * 64) * (double)((g.N + 63) / 64 * 64) * (double)g.K * 2 / 154e6;
+    return us < 4 + 1.45 * mma_us ? shape : WinShape{};
+  }
+  return shape;
+}
+
 // Packs the caller's HWCK filter into the plan's Bt.
 hipError_t pack_conv_filter(Plan* p, const void* filter, hipStream_t s) {
   const pml_hip_conv2d_desc& d = p->conv;
   const int es = dt_size(d.in_dtype);
+  if (p->win.config >= 0) return winconv_pack_launch(es, filter, {(int)(d.kh * d.kw), (int)d.ci, (int)d.co, 0, d.ci * d.co, d.co, 1}, p->bt, s);
   if (p->via_s2d) {
     S2dArgs a;
     s2d_args(p, a);
@@ -1257,12 +1296,6 @@ int64_t pml_hip_conv2d_dispatch(const pml_hip_conv2d_desc* d) {
     }
   }
   if (!via_s2d && !via_patches && PML_HIP_FLAG_TILE_OF(d->flags) < 0) p->tile_direct = direct_tile_of(M, d->co, K * es, kind);
-  p->bt_bytes = (size_t)d->co * p->bt_ld * es;
-  if (!(p->bt = p->hold(p->bt_bytes)) || hipMemset(p->bt, 0, p->bt_bytes) != hipSuccess) {
-    delete p;
-    fail("conv2d: cannot allocate the packed filter");
-    return 0;
-  }
   {
     // Filter small enough to stay in LDS: persistent resident-filter kernel (PML_HIP_CONV_IGEMM keeps the generic one).
     int dev = 0;
@@ -1281,21 +1314,38 @@ int64_t pml_hip_conv2d_dispatch(const pml_hip_conv2d_desc* d) {
       }
     }
   }
-  if (!via_s2d && !via_patches && !p->halo_lds && p->tile_direct < 0) prepare_split(p, M, d->co, conv_slabs(*d));
+  const bool named = path == PML_HIP_CONV_WINDOW;
+  if (!odd_channels && PML_HIP_FLAG_TILE_OF(d->flags) < 0 && (named || (path == PML_HIP_CONV_AUTO && (!p->halo_lds || p->halo_variant == 0)))) {
+    p->win = window_shape(p, named);
+    if (p->win.config >= 0) {
+      p->halo_lds = 0;
+      p->tile_direct = -1;
+    }
+  }
+  p->bt_bytes = p->win.config >= 0 ? winconv_pack_bytes(es, (int)(d->kh * d->kw), d->ci, d->co) : (size_t)d->co * p->bt_ld * es;
+  if (!(p->bt = p->hold(p->bt_bytes)) || hipMemset(p->bt, 0, p->bt_bytes) != hipSuccess) {
+    delete p;
+    fail("conv2d: cannot allocate the packed filter");
+    return 0;
+  }
+  if (!via_s2d && !via_patches && !p->halo_lds && p->win.config < 0 && p->tile_direct < 0) prepare_split(p, M, d->co, conv_slabs(*d));
   const int lds_tile = p->tile;  // (named in the text beside the direct tile that takes its place)
   if (p->tile == TILE_64x64_KSPLIT && !p->ws) p->tile = TILE_64x64;
   // (whole 128-byte chunks per filter tap, so that no chunk of heads + remainders straddles two taps)
   p->b_split = kind == KIND_F32X3 && !via_s2d && !via_patches && d->ci % 32 == 0 && !p->ws;
+  const std::string kernel = p->win.config >= 0 ? winconv_text(p->win)
+                             : std::string("tile=") + (p->halo_lds ? (p->halo_variant == 3 ? "256x64 resident filter, in registers" : p->halo_variant ? "256x64 resident filter, pipelined 3x3" : "256x64 resident filter")
+                                                                   : tile_name(p->tile_direct >= 0 ? lds_tile : p->tile));
   char buf[256];
-  std::snprintf(buf, sizeof buf, "conv2d %s n=%lld %lldx%lldx%lld k=%lldx%lld co=%lld -> %lldx%lld (implicit gemm m=%lld n=%lld k=%lld) tile=%s",
+  std::snprintf(buf, sizeof buf, "conv2d %s n=%lld %lldx%lldx%lld k=%lldx%lld co=%lld -> %lldx%lld (implicit gemm m=%lld n=%lld k=%lld) %s",
                 d->in_dtype == PML_HIP_F32 ? "f32" : d->in_dtype == PML_HIP_BF16 ? "bf16" : "i8", (long long)d->n,
                 (long long)d->h, (long long)d->w, (long long)d->ci, (long long)d->kh, (long long)d->kw, (long long)d->co,
-                (long long)d->oh, (long long)d->ow, (long long)M, (long long)d->co, (long long)K, p->halo_lds ? (p->halo_variant == 3 ? "256x64 resident filter, in registers" : p->halo_variant ? "256x64 resident filter, pipelined 3x3" : "256x64 resident filter") : tile_name(p->tile_direct >= 0 ? lds_tile : p->tile));
+                (long long)d->oh, (long long)d->ow, (long long)M, (long long)d->co, (long long)K, kernel.c_str());
   p->text = buf;
   if (kind == KIND_F32X3) p->text += " mfma=3 x f32_32x32x16_bf16 (fp32 split into bf16 head + remainder)";
   if (p->tile_direct >= 0 && !p->halo_lds) p->text += std::string(", direct tile=") + tile_name(p->tile_direct);
   if (via_patches) p->text += " via patch matrix (k padded to " + std::to_string(p->kpad) + ")";
-  if (!p->halo_lds && !via_s2d) {
+  if (!p->halo_lds && p->win.config < 0 && !via_s2d) {
     IgemmArgs g;
     conv_args(p, g);
     if (via_patches) g.K = g.lda = p->kpad;
@@ -1393,7 +1443,7 @@ int pml_hip_conv2d_invoke(int64_t plan, const void* input, const void* filter, v
       return fail("conv2d_invoke: missing extra output");
   const int tile = p->tile_direct >= 0 ? p->tile_direct : p->tile;
   // (a 1x1 convolution whose rows stream takes the filter as it lies; a packed one stays what later calls use)
-  const bool given_filter = filter && !p->packed && !p->patches && !p->via_s2d && !p->halo_lds && streams_given(p->mfma_kind, tile, true, filter, d.co, g);
+  const bool given_filter = filter && !p->packed && !p->patches && !p->via_s2d && !p->halo_lds && p->win.config < 0 && streams_given(p->mfma_kind, tile, true, filter, d.co, g);
   if (filter && !raw_filter && !given_filter) {
     if (check(pack_conv_filter(p, filter, (hipStream_t)s), "pack_conv_filter")) return 1;
     // (a filter that arrives with the call replaces the packed one; its register-order copy follows it)
@@ -1442,6 +1492,7 @@ int pml_hip_conv2d_invoke(int64_t plan, const void* input, const void* filter, v
     if (lds) return check(conv_blocks4x4_launch(g, lds, device_cus(), (hipStream_t)s), "conv_blocks4x4_launch");
     return check(igemm_launch(p->mfma_kind, p->tile, true, g, (hipStream_t)s), "igemm_launch");
   }
+  if (p->win.config >= 0) return check(winconv_launch(p->mfma_kind, g, p->win, (hipStream_t)s), "winconv_launch");
   if (p->halo_lds)
     return check(conv_halo_launch(p->mfma_kind, g, p->halo_lds, p->n_cus, (hipStream_t)s), "conv_halo_launch");
   split_args(p, g);
@@ -1902,7 +1953,12 @@ int pml_hip_conv2d_grad_invoke(int64_t plan, const void* g, const void* other, v
       if (check(pad_rows_launch(es, g, p->padded, d.n * d.oh * d.ow, d.co, p->co_pad, st), "pad_rows_launch")) return 1;
       in = p->padded;
     }
-    if (check(flip_filter_launch(es, other, p->sub->bt, d.kh * d.kw, d.ci, d.co, p->co_pad, st), "flip_filter_launch")) return 1;
+    if (p->sub->win.config >= 0) {  // (the taps in reverse, the channels' roles exchanged)
+      const WinFilter w{(int)(d.kh * d.kw), (int)d.co, (int)d.ci, (d.kh * d.kw - 1) * d.ci * d.co, -d.ci * d.co, 1, d.co};
+      if (check(winconv_pack_launch(es, other, w, p->sub->bt, st), "winconv_pack_launch")) return 1;
+    } else if (check(flip_filter_launch(es, other, p->sub->bt, d.kh * d.kw, d.ci, d.co, p->co_pad, st), "flip_filter_launch")) {
+      return 1;
+    }
     if (pml_hip_conv2d_invoke((int64_t)(intptr_t)p->sub, in, nullptr, result, nullptr, nullptr, nullptr, s)) return 1;
     ConvBorderArgs b;
     b.g = g, b.f = other, b.out = result;

@@ -17,7 +17,7 @@ BOOL, I8, U8, I16, U16, I32, U32, I64, U64, F16, F32, F64, BF16 = 4, 5, 6, 7, 8,
 FP32_AS_BF16X3 = 1  # descriptor flag of gemm / conv2d: fp32 operands multiplied as three bf16 products
 # schedule overrides in the same `flags` field (PML_HIP_FLAG_TILE / PML_HIP_FLAG_CONV of include/pml_hip.h)
 TILE_NAMES = ('64x64', '128x64', '128x128', '128x64w8', '128x128w8', '256x128w16', '128x128w8s2', '64x64w8k2', '256x256w8', '128x64n2', '192x384w8', '64x64ks', '16x16w8', '32x32w8')
-CONV_AUTO, CONV_IGEMM, CONV_PATCHES, CONV_LDSFILTER, CONV_BLOCKS = 0, 1, 2, 3, 4
+CONV_AUTO, CONV_IGEMM, CONV_PATCHES, CONV_LDSFILTER, CONV_BLOCKS, CONV_WINDOW = 0, 1, 2, 3, 4, 5
 
 
 def flag_tile(name):

@@ -58,10 +58,10 @@ std::shared_ptr<Plan> Planner::run() {
 // Tiling overrides, per program (target options) and per step (schedule file): they travel to the kernel library in
 // the descriptors' schedule bits.  Runs last, so that a step is keyed by the text the plan dump shows for it.
 int Planner::convPathByName(const std::string& name) {
-  static const char* const names[] = {"auto", "igemm", "patches", "ldsfilter", "blocks"};
-  for (int i = 0; i < 5; ++i)
+  static const char* const names[] = {"auto", "igemm", "patches", "ldsfilter", "blocks", "window"};
+  for (int i = 0; i < 6; ++i)
     if (name == names[i]) return i;
-  throw std::runtime_error("Invalid convolution path '" + name + "' (igemm, patches, ldsfilter or blocks)");
+  throw std::runtime_error("Invalid convolution path '" + name + "' (igemm, patches, ldsfilter, blocks or window)");
 }
 
 int Planner::tileByName(const std::string& name) {
@@ -122,7 +122,7 @@ void Planner::applySchedule() {
       text += std::string("tile=") + pml_hip_tile_name(r.tile);
     }
     if (r.conv > 0) {
-      static const char* const names[] = {"auto", "igemm", "patches", "ldsfilter", "blocks"};
+      static const char* const names[] = {"auto", "igemm", "patches", "ldsfilter", "blocks", "window"};
       flags |= PML_HIP_FLAG_CONV(r.conv);
       text += std::string(text.empty() ? "" : ",") + "conv=" + names[r.conv];
     }
