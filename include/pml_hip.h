@@ -320,6 +320,14 @@ int pml_hip_gemm_pack_b(int64_t plan, const void* b, pml_hip_stream s);
  * constant B2 once (invoke2 may then be given b2 == NULL). */
 int pml_hip_gemm_invoke2(int64_t plan, const void* a, const void* b, void* c, const void* init, const void* a2, const void* b2,
                          const void* init2, const void* const* operands, void* const* outs, pml_hip_stream s);
+
+/* Two products in a row, C = tail(A . B (+ A2 . B2)) and D = tail(C . B'): one launch that multiplies the rows of C onward while
+ * they are on the chip (C is stored as well).  _takes: whether the two descriptors are such a pair and of widths that are built
+ * (bf16 throughout, right-hand sides packed, 256 or 512 columns of C).  The plans are ordinary ones with pml_hip_gemm_pack_b
+ * (and _pack_b2) behind them; operands as in pml_hip_gemm_invoke2. */
+int pml_hip_gemm_chain_takes(const pml_hip_gemm_desc* first, const pml_hip_gemm_desc* next);
+int pml_hip_gemm_chain_invoke(int64_t first, int64_t next, const void* a, void* c, const void* init, const void* a2, const void* init2,
+                              const void* const* operands, void* next_c, const void* next_init, pml_hip_stream s);
 int pml_hip_gemm_pack_b2(int64_t plan, const void* b2, pml_hip_stream s);
 
 /* Measurement aid (no counterpart in the reference): the bf16 rate the matrix cores of the current device sustain on

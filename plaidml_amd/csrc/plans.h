@@ -217,6 +217,9 @@ hipError_t given_launch(int kind, const IgemmArgs& a, hipStream_t s);
 // bf16 products of many rows and a short K over Bt: stream.hip
 bool stream_takes(int cfg, bool conv, const IgemmArgs& a);
 hipError_t stream_launch(bool conv, const IgemmArgs& a, hipStream_t s);
+// Two bf16 products in a row, the second one's left-hand side the first one's result: chain.hip.  Both sides' packed Bt[N][K].
+bool chain_takes(const IgemmArgs& a, const IgemmArgs& next);  // by descriptors
+hipError_t chain_launch(const IgemmArgs& a, const IgemmArgs& next, hipStream_t s);
 // How TILE_64x64_KSPLIT shares the K loop out: slabs of 128 bytes of K in all, and for a device of n_cus compute units
 // the number of splits (1: not worth splitting) with the slabs each takes -- about one workgroup per CU, at least two
 // slabs per split, at most 16 splits.

@@ -1181,6 +1181,49 @@ int pml_hip_gemm_invoke2(int64_t plan, const void* a, const void* b, void* c, co
   return gemm_run(p->gemm, p->mfma_kind, p->tile, p->direct, p->bt, p->bt_ld, p->packed, a, b, c, init, operands, outs, s, &sp, p);
 }
 
+static bool chain_descs(const pml_hip_gemm_desc& first, const pml_hip_gemm_desc& next) {
+  auto columns = [](int kind, int dtype, int64_t rs, int64_t cs) { return kind == 0 || (dtype == PML_HIP_BF16 && rs == 0 && cs == 1); };
+  for (const pml_hip_gemm_desc* d : {&first, &next})
+    if (d->in_dtype != PML_HIP_BF16 || d->b_layout != 0 || d->flags != 0 || d->m <= 0 || !valid_tail(d->tail) ||
+        !columns(d->init_kind, d->init_dtype, d->init_row_stride, d->init_col_stride))
+      return false;
+  IgemmArgs g, n;
+  gemm_args(first, g);
+  gemm_args(next, n);
+  return chain_takes(g, n);
+}
+
+int pml_hip_gemm_chain_takes(const pml_hip_gemm_desc* first, const pml_hip_gemm_desc* next) {
+  return first && next && chain_descs(*first, *next) ? 1 : 0;
+}
+
+int pml_hip_gemm_chain_invoke(int64_t first, int64_t next, const void* a, void* c, const void* init, const void* a2, const void* init2,
+                              const void* const* operands, void* next_c, const void* next_init, pml_hip_stream s) {
+  Plan *p = (Plan*)(intptr_t)first, *q = (Plan*)(intptr_t)next;
+  if (!p || p->kind != PLAN_GEMM || !q || q->kind != PLAN_GEMM) return fail("gemm_chain_invoke: not two gemm plans");
+  if (!chain_descs(p->gemm, q->gemm)) return fail("gemm_chain_invoke: the second plan does not multiply the first one's result onward");
+  IgemmArgs g, n;
+  gemm_args(p->gemm, g);
+  gemm_args(q->gemm, n);
+  const bool second = p->gemm.k2 > 0, residual = g.tail_mode == 2;
+  if (!a || !c || !next_c || !p->packed || !q->packed || (second && (!a2 || !p->packed2))) return fail("gemm_chain_invoke: null operand or unpacked right-hand side");
+  if ((p->gemm.init_kind && !init) || (second && p->gemm.init2_kind && !init2) || (q->gemm.init_kind && !next_init)) return fail("gemm_chain_invoke: the plans expect initial values");
+  if (residual && (!operands || !operands[0])) return fail("gemm_chain_invoke: missing tail operand");
+  const uintptr_t places = (uintptr_t)a | (uintptr_t)c | (uintptr_t)next_c | (second ? (uintptr_t)a2 : 0) | (residual ? (uintptr_t)operands[0] : 0);
+  if ((places & 15) != 0 || p->bt_is_kn || q->bt_is_kn) {  // one after the other
+    void* none[PML_HIP_MAX_EPI_OPERANDS] = {};
+    const int rc = second ? pml_hip_gemm_invoke2(first, a, nullptr, c, init, a2, nullptr, init2, operands, none, s)
+                          : pml_hip_gemm_invoke(first, a, nullptr, c, init, operands, none, s);
+    return rc ? rc : pml_hip_gemm_invoke(next, c, nullptr, next_c, next_init, nullptr, none, s);
+  }
+  g.A = a, g.Bt = p->bt, g.ldbt = p->bt_ld, g.C = c;
+  g.init = p->gemm.init_kind ? init : nullptr;
+  if (second) g.A2 = a2, g.Bt2 = p->bt2, g.init2 = p->gemm.init2_kind ? init2 : nullptr;
+  if (residual) g.operands[0] = operands[0];
+  n.Bt = q->bt, n.ldbt = q->bt_ld, n.C = next_c, n.init = q->gemm.init_kind ? next_init : nullptr;
+  return check(chain_launch(g, n, (hipStream_t)s), "chain_launch");
+}
+
 int pml_hip_gemm_run_static(const pml_hip_gemm_desc* d, const void* a, const void* b, void* c, const void* init,
                             const void* const* operands, void* const* outs, pml_hip_stream s) {
   const int kind = gemm_desc_kind(d);

@@ -50,7 +50,7 @@ EXPORTS = [
     'pml_hip_stream_sync', 'pml_hip_event_create', 'pml_hip_event_destroy', 'pml_hip_event_record',
     'pml_hip_event_sync', 'pml_hip_event_elapsed_ms', 'pml_hip_capture_begin', 'pml_hip_capture_end',
     'pml_hip_graph_launch', 'pml_hip_graph_destroy', 'pml_hip_gemm_dispatch', 'pml_hip_gemm_invoke',
-    'pml_hip_gemm_run_static', 'pml_hip_gemm_invoke2', 'pml_hip_gemm_pack_b2', 'pml_hip_probe_mfma', 'pml_hip_dwconv2d_pack_filter', 'pml_hip_tile_of_workgroup', 'pml_hip_tile_name', 'pml_hip_tile_by_name', 'pml_hip_gemm_tail_cheaper_apart',
+    'pml_hip_gemm_run_static', 'pml_hip_gemm_invoke2', 'pml_hip_gemm_chain_takes', 'pml_hip_gemm_chain_invoke', 'pml_hip_gemm_pack_b2', 'pml_hip_probe_mfma', 'pml_hip_dwconv2d_pack_filter', 'pml_hip_tile_of_workgroup', 'pml_hip_tile_name', 'pml_hip_tile_by_name', 'pml_hip_gemm_tail_cheaper_apart',
     'pml_hip_conv2d_dispatch', 'pml_hip_conv2d_invoke', 'pml_hip_dwconv2d_dispatch', 'pml_hip_dwconv2d_invoke',
     'pml_hip_pool2d_dispatch', 'pml_hip_pool2d_invoke', 'pml_hip_eltwise_dispatch', 'pml_hip_eltwise_invoke',
     'pml_hip_select', 'pml_hip_softmax', 'pml_hip_index', 'pml_hip_contract_dispatch', 'pml_hip_contract_invoke', 'pml_hip_plan_free',
@@ -190,6 +190,8 @@ def lib():
         L.pml_hip_gemm_invoke.argtypes = [ctypes.c_int64, vp, vp, vp, vp, pp, pp, vp]
         L.pml_hip_gemm_run_static.argtypes = [ctypes.POINTER(GemmDesc), vp, vp, vp, vp, pp, pp, vp]
         L.pml_hip_gemm_invoke2.argtypes = [ctypes.c_int64, vp, vp, vp, vp, vp, vp, vp, pp, pp, vp]
+        L.pml_hip_gemm_chain_takes.argtypes = [ctypes.POINTER(GemmDesc), ctypes.POINTER(GemmDesc)]
+        L.pml_hip_gemm_chain_invoke.argtypes = [ctypes.c_int64, ctypes.c_int64, vp, vp, vp, vp, vp, pp, vp, vp, vp]
         L.pml_hip_gemm_pack_b2.argtypes = [ctypes.c_int64, vp, vp]
         L.pml_hip_probe_mfma.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.POINTER(ctypes.c_double), ctypes.POINTER(ctypes.c_double)]
         L.pml_hip_tile_name.restype = ctypes.c_char_p

@@ -51,6 +51,8 @@ std::shared_ptr<Plan> Planner::run() {
   if (opt_.specialise) padDepthwiseResults();
   if (opt_.fuse && opt_.specialise) fusePoolIntoConv();
   pruneDeadSteps();
+  // (a schedule names the tiles of single products, by the text of their steps)
+  if (opt_.fuse && opt_.specialise && opt_.tile.empty() && opt_.schedule_path.empty()) chainProducts();
   applySchedule();
   return plan_;
 }

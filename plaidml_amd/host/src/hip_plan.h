@@ -57,6 +57,12 @@ struct Step {
   int a2 = -1, b2 = -1, init2 = -1;
   int64_t a2_off = 0, b2_off = 0;
   bool b2_constant = false;
+  // Gemm whose result's rows are multiplied onward in the same launch (Planner::chainProducts): the second product's
+  // descriptor, constant right-hand side and per-column initial value; its result is out2
+  bool chained = false;
+  pml_hip_gemm_desc next_gemm{};
+  int next_b = -1, next_init = -1;
+  int64_t next_b_off = 0;
   std::vector<int> operands;       // tail operands / contraction sources / select inputs
   std::vector<int64_t> operand_off;
   std::vector<int> outs;           // extra outputs of STORE steps (index = STORE's operand field)

@@ -226,6 +226,47 @@ void Planner::fusePoolIntoConv() {
   }
 }
 
+// A matrix product whose left-hand side is the result of an earlier one -- the last 1x1 convolution of a residual block and the
+// first one of the next -- becomes part of that one's launch, where the kernel library multiplies the rows of such a result
+// onward while they are on the chip (pml_hip_gemm_chain_takes: bf16, constant right-hand sides, the widths it is built for).
+// The first result is stored as before: whoever else reads it finds it there.
+void Planner::chainProducts() {
+  auto product = [&](const Step& s) {
+    return s.kind == Step::Gemm && !s.chained && s.b_constant && !s.b_is_nk && s.gemm.flags == 0 && s.outs.empty() && s.out2 < 0 && s.c >= 0 &&
+           (s.gemm.k2 == 0 || s.b2_constant);
+  };
+  auto writers = [&](int buf) {
+    int n = 0;
+    for (const Step& s : plan_->steps) {
+      n += (s.c == buf) + (s.out2 == buf);
+      for (int w : s.outs) n += w == buf;
+    }
+    return n;
+  };
+  for (size_t x = 0; x < plan_->steps.size(); ++x) {
+    Step& X = plan_->steps[x];
+    if (!product(X) || X.a_off != 0 || X.a2_off != 0 || X.c_off != 0 || writers(X.c) != 1) continue;
+    for (size_t y = x + 1; y < plan_->steps.size(); ++y) {
+      const Step& Y = plan_->steps[y];
+      if (!product(Y) || Y.a != X.c || Y.a_off != 0 || Y.c_off != 0 || Y.gemm.k2 != 0 || !Y.operands.empty() || Y.c == X.c || writers(Y.c) != 1) continue;
+      // (its initial value has to be there when the first product runs, and nobody may have use for the place of its result till then)
+      if (Y.init >= 0 && plan_->buffers[Y.init].kind != BufferInfo::Constant && plan_->buffers[Y.init].kind != BufferInfo::Input) continue;
+      if (!pml_hip_gemm_chain_takes(&X.gemm, &Y.gemm)) continue;
+      X.chained = true;
+      X.next_gemm = Y.gemm;
+      X.next_b = Y.b;
+      X.next_b_off = Y.b_off;
+      X.next_init = Y.init;
+      X.out2 = Y.c;
+      X.text += ", rows multiplied onward: " + Y.text;
+      X.flops += Y.flops;
+      X.bytes += Y.bytes - 2.0 * static_cast<double>(Y.gemm.m * Y.gemm.k);
+      plan_->steps.erase(plan_->steps.begin() + static_cast<long>(y));
+      break;
+    }
+  }
+}
+
 // A kernel that took over the work of earlier operations (the int8 GEMM reads the un-cast operands, a pool
 // kernel also writes the window argmax) can leave launches whose results nobody reads: drop them.
 void Planner::pruneDeadSteps() {

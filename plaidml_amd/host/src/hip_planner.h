@@ -162,6 +162,7 @@ class Planner {
   void fuseSecondProducts();
   void padDepthwiseResults();
   void fusePoolIntoConv();
+  void chainProducts();
   void pruneDeadSteps();
 
  private:

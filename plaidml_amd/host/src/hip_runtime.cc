@@ -67,6 +67,7 @@ class HipExecutable final : public Executable {
           hipCheck(pml_hip_memcpy_h2d(device_[i], b.constant->data(), b.constant->size(), nullptr), "upload constant");
       }
       handles_.assign(plan_->steps.size(), 0);
+      next_handles_.assign(plan_->steps.size(), 0);
       for (size_t i = 0; i < plan_->steps.size(); ++i) dispatch(i);
       // Where a run begins and ends on the device is read off its clock by the kernels that copy, or by one of their kind
       // (two events around the launches cost a run 8 us); with events where that cannot be had, and under PLAIDML_PROFILE.
@@ -216,6 +217,7 @@ class HipExecutable final : public Executable {
   void* arena_ = nullptr;
   size_t arena_bytes_ = 0, fixed_bytes_ = 0, unshared_temp_bytes_ = 0;
   std::vector<int64_t> handles_;
+  std::vector<int64_t> next_handles_;  // the second product of a step that has one behind its first (Step::chained)
   pml_hip_event ev0_ = nullptr, ev1_ = nullptr;
   uint64_t* stamps_ = nullptr;  // page-locked: the device's clock ahead of and behind a run's launches
   int clock_khz_ = 0;
@@ -422,8 +424,9 @@ class HipExecutable final : public Executable {
     st->arena_bytes = arena_bytes_;
     st->unshared_temp_bytes = unshared_temp_bytes_;
     st->device_bytes = arena_bytes_ + fixed_bytes_;
-    for (int64_t h : handles_)
-      if (h) st->device_bytes += pml_hip_plan_bytes(h);
+    for (const auto* handles : {&handles_, &next_handles_})
+      for (int64_t h : *handles)
+        if (h) st->device_bytes += pml_hip_plan_bytes(h);
     if (!profile) return;
     // One row per launch, in the reference's format (pmlc/rt/instrument.cc:22-43: id, loc, tag, seconds since
     // the previous point, seconds since the start); loc is the plan's line for the step, tag its kind.
@@ -537,9 +540,11 @@ class HipExecutable final : public Executable {
   }
 
   void release() {
-    for (int64_t h : handles_)
-      if (h) pml_hip_plan_free(h);
-    handles_.clear();
+    for (auto* handles : {&handles_, &next_handles_}) {
+      for (int64_t h : *handles)
+        if (h) pml_hip_plan_free(h);
+      handles->clear();
+    }
     for (size_t i = 0; i < device_.size(); ++i)
       if (device_[i] && owned_[i]) pml_hip_free(device_[i]);
     device_.clear();
@@ -605,6 +610,11 @@ class HipExecutable final : public Executable {
       hipCheck(pml_hip_gemm_pack_b(h, ptr(s.b, s.b_off, elemSize(s.gemm.in_dtype)), nullptr), "pack_b");
     if (s.kind == Step::Gemm && s.gemm.k2 > 0 && s.b2_constant && !s.b_is_nk)
       hipCheck(pml_hip_gemm_pack_b2(h, ptr(s.b2, s.b2_off, elemSize(s.gemm.in_dtype)), nullptr), "pack_b2");
+    if (s.chained) {
+      next_handles_[i] = pml_hip_gemm_dispatch(&s.next_gemm);
+      if (!next_handles_[i]) throw std::runtime_error("hip dispatch failed for '" + s.text + "': " + pml_hip_last_error());
+      hipCheck(pml_hip_gemm_pack_b(next_handles_[i], ptr(s.next_b, s.next_b_off, elemSize(s.next_gemm.in_dtype)), nullptr), "pack_b");
+    }
     if (s.kind == Step::Conv2d && s.b_constant) hipCheck(pml_hip_conv2d_pack_filter(h, ptr(s.b), nullptr), "pack_filter");
     if (s.kind == Step::Dwconv2d && s.b_constant) hipCheck(pml_hip_dwconv2d_pack_filter(h, ptr(s.b), nullptr), "pack_filter");
   }
@@ -618,6 +628,12 @@ class HipExecutable final : public Executable {
     switch (s.kind) {
       case Step::Gemm: {
         const size_t es = elemSize(s.gemm.in_dtype);
+        if (s.chained) {
+          hipCheck(pml_hip_gemm_chain_invoke(handles_[i], next_handles_[i], ptr(s.a), ptr(s.c), ptr(s.init), ptr(s.a2), ptr(s.init2), operands, ptr(s.out2),
+                                             ptr(s.next_init), stream_),
+                   s.text.c_str());
+          break;
+        }
         const void* b = ptr(s.b, s.b_off, es);
         if (s.b_constant && !s.b_is_nk) b = nullptr;  // packed when the executable was built
         if (s.gemm.k2 > 0) {
