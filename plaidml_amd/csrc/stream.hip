@@ -6,12 +6,18 @@
 // workgroup on the CU covers for that.  Here a wavefront keeps the right-hand side of 64 columns (32 past K = 128) in
 // registers for its whole life and walks down the rows, 16 at a time; the left-hand rows and the residual rows of the next
 // tiles are on their way to registers while it multiplies and stores the current one, and nothing is shared between
-// wavefronts -- no LDS, no barrier.  The wavefronts of a workgroup hold neighbouring columns of the same rows, whose
+// wavefronts: there is no barrier.  The wavefronts of a workgroup hold neighbouring columns of the same rows, whose
 // left-hand side they find in L1, and the workgroups of one XCD the other columns of these rows, which find it in L2.
 //
 // The MFMAs are the 16 x 16 ones with the right-hand side as the row operand.  Row i of block b of a pair holds column
-// 8 (i / 4) + 4 b + i % 4 of the pair's 32, so that a lane ends with eight neighbouring columns of its row: one 16-byte
-// access, 64 contiguous bytes a row and request, for residual and result alike, without an exchange between lanes.
+// 8 (i / 4) + 4 b + i % 4 of the pair's 32, so that a lane ends with eight neighbouring columns of its row, 16 bytes,
+// without an exchange between lanes.
+//
+// Residual rows and results touch memory in whole 128-byte lines, 8 rows of a wavefront's 64 columns (4 of 128) an instruction,
+// and pass through 16 rows of LDS that are the wavefront's own on their way to and from the arrangement of the accumulators,
+// whose accesses would be 16 rows of 64 bytes (us, over buffers in turn, 64-byte pieces -> lines: 401408 x 256, K = 64 74 -> 53, with
+// a residual 93.6 -> 90.7, K = 32 65 -> 47; 100352 x 512, K = 128 46 -> 36, with a residual 56 -> 51; 25088 x 1024, K = 256 with a
+// residual 43.5 -> 37.8; 401408 x 123, K = 64, rows off any alignment 62 -> 45).
 //
 // KN: a right-hand side that arrives as [K][N] is read as it lies, once: four neighbouring columns of every K-row per lane,
 // turned with v_perm into the fragments of four blocks, block j of 64 columns holding the columns 4 i + j; a lane then ends
@@ -139,10 +145,17 @@ __global__ __launch_bounds__(kThreads, OCC) void stream_kernel(StreamArgs p) {
   }
 
   const unsigned a_lane = (unsigned)(r * (int)p.lda + 8 * g) * 2, a2_lane = (unsigned)(r * (int)p.lda2 + 8 * g - k1) * 2;
-  const unsigned r_lane = (unsigned)(r * (int)p.ldr + col0) * 2, c_lane = (unsigned)(r * (int)p.ldc + col0) * 2;
-  const int k_left = p.K - 8 * g, k2_left = k1 + p.K2 - 8 * g, n_left = p.N - col0;
+  const int k_left = p.K - 8 * g, k2_left = k1 + p.K2 - 8 * g;
+  // the wavefront's rows in LDS (sixteen of them begin in sixteen different banks), and a lane's piece of the rows of an access
+  constexpr int kPieces = 4 * NP, kLineRows = 64 / kPieces, kAccesses = kRows / kLineRows, kPitch = 16 * kPieces + 16;
+  __shared__ __attribute__((aligned(16))) unsigned char staged[kThreads / 64][kRows * kPitch];
+  const int line_row = lane / kPieces, piece = lane % kPieces, left = p.N - (n0 + 8 * piece);
+  unsigned char* const mine = staged[wave];
+  unsigned char* const line_at = mine + line_row * kPitch + 16 * piece;
+  auto lane_at = [&](int q) { return (i32x4_t*)(mine + r * kPitch + (col0 - n0 + behind(q)) * 2); };
+  const unsigned r_lane = (unsigned)(line_row * (int)p.ldr + n0 + 8 * piece) * 2, c_lane = (unsigned)(line_row * (int)p.ldc + n0 + 8 * piece) * 2;
   auto rows_at = [](unsigned lane_at, int step, int64_t pitch) { return lane_at + (unsigned)step * (unsigned)(kRows * 2 * (int)pitch); };
-  i32x4_t fa[D][KS], res[D][RES ? NP : 1];
+  i32x4_t fa[D][KS], res[D][RES ? kAccesses : 1];
   auto request = [&](int d, int step) {
     const bool live = step < steps;
     const unsigned a_at = rows_at(a_lane, step, p.lda), a2_at = rows_at(a2_lane, step, p.lda2), r_at = rows_at(r_lane, step, p.ldr);
@@ -154,7 +167,7 @@ __global__ __launch_bounds__(kThreads, OCC) void stream_kernel(StreamArgs p) {
     }
     if constexpr (RES) {
 #pragma unroll
-      for (int q = 0; q < NP; ++q) res[d][q] = fetch(rr, live & (behind(q) < n_left), r_at + 2 * behind(q));
+      for (int i = 0; i < kAccesses; ++i) res[d][i] = fetch(rr, live & (left > 0), r_at + (unsigned)(i * kLineRows * 2 * (int)p.ldr));
     }
   };
 
@@ -196,8 +209,10 @@ __global__ __launch_bounds__(kThreads, OCC) void stream_kernel(StreamArgs p) {
             __builtin_memcpy(&bv, &fb[q][b][k], 16);
             acc[q][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bv, av, acc[q][b], 0, 0, 0);
           }
-      const bool live = step < steps;
-      const unsigned c_at = rows_at(c_lane, step, p.ldc);
+      if constexpr (RES) {
+#pragma unroll
+        for (int i = 0; i < kAccesses; ++i) *(i32x4_t*)(line_at + i * kLineRows * kPitch) = res[d][i];
+      }
 #pragma unroll
       for (int q = 0; q < NP; ++q) {
         float v[8];
@@ -206,7 +221,7 @@ __global__ __launch_bounds__(kThreads, OCC) void stream_kernel(StreamArgs p) {
         if constexpr (RES) {
           // the contraction result is rounded first, then the bf16 addition rounds again
           float f[8];
-          unpack_bf16x8(res[d][q], f);
+          unpack_bf16x8(*lane_at(q), f);
 #pragma unroll
           for (int e = 0; e < 8; e += 2) round_pair_to_bf16(v[e], v[e + 1]);
 #pragma unroll
@@ -214,11 +229,17 @@ __global__ __launch_bounds__(kThreads, OCC) void stream_kernel(StreamArgs p) {
         }
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[e] = __builtin_elementwise_maximum(v[e], lo);
-        const i32x4_t out = pack_bf16x8(v);
+        *lane_at(q) = pack_bf16x8(v);
+      }
+      const bool live = step < steps;
+      const unsigned c_at = rows_at(c_lane, step, p.ldc);
+#pragma unroll
+      for (int i = 0; i < kAccesses; ++i) {
+        const i32x4_t out = *(const i32x4_t*)(line_at + i * kLineRows * kPitch);
+        const unsigned at = c_at + (unsigned)(i * kLineRows * 2 * (int)p.ldc);
         if constexpr (RAGGED) {
-          const int left = n_left - behind(q);
-          if (step * kRows + r < p.M && live && left > 0) {
-            unsigned char* const to = (unsigned char*)p.C + (c_at + 2 * behind(q));
+          if (step * kRows + i * kLineRows + line_row < p.M && live && left > 0) {
+            unsigned char* const to = (unsigned char*)p.C + at;
             if (left >= 8) {
               __builtin_memcpy(to, &out, 16);
             } else {
@@ -228,7 +249,7 @@ __global__ __launch_bounds__(kThreads, OCC) void stream_kernel(StreamArgs p) {
             }
           }
         } else {
-          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_tail_t, out), rc, (int)(live & (behind(q) < n_left) ? c_at + 2 * behind(q) : kOutside), 0, 0);
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_tail_t, out), rc, (int)(live & (left > 0) ? at : kOutside), 0, 0);
         }
       }
       request(d, step + D * stride);
