@@ -858,6 +858,10 @@ int pml_hip_event_record(pml_hip_event e, pml_hip_stream s) {
   return check(hipEventRecord((hipEvent_t)e, (hipStream_t)s), "hipEventRecord");
 }
 int pml_hip_event_sync(pml_hip_event e) { return check(hipEventSynchronize((hipEvent_t)e), "hipEventSynchronize"); }
+int pml_hip_stream_wait_event(pml_hip_stream s, pml_hip_event e) {
+  return check(hipStreamWaitEvent((hipStream_t)s, (hipEvent_t)e, 0), "hipStreamWaitEvent");
+}
+
 int pml_hip_event_elapsed_ms(pml_hip_event start, pml_hip_event stop, float* ms) {
   return check(hipEventElapsedTime(ms, (hipEvent_t)start, (hipEvent_t)stop), "hipEventElapsedTime");
 }

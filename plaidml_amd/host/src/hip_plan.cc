@@ -54,6 +54,8 @@ std::shared_ptr<Plan> Planner::run() {
   // (a schedule names the tiles of single products, by the text of their steps)
   if (opt_.fuse && opt_.specialise && opt_.tile.empty() && opt_.schedule_path.empty()) chainProducts();
   applySchedule();
+  // (a tile or path that was asked for was asked for the whole step)
+  if (opt_.fuse && opt_.specialise && opt_.tile.empty() && opt_.conv.empty() && opt_.schedule_path.empty()) sliceSteps();
   return plan_;
 }
 
@@ -253,6 +255,7 @@ std::string Plan::dump() const {
   std::stringstream ss;
   ss << "hip plan: " << steps.size() << " launches, " << buffers.size() << " buffers\n";
   for (size_t i = 0; i < steps.size(); ++i) ss << "  [" << i << "] " << steps[i].text << steps[i].schedule << "\n";
+  if (slices > 1) ss << "  steps 0 to " << sliced.size() - 1 << " in " << slices << " parts of the leading dimension\n";
   return ss.str();
 }
 

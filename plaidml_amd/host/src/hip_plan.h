@@ -80,6 +80,13 @@ struct Plan {
   std::vector<int> input_buffers;   // buffer id per program input
   std::vector<int> output_buffers;  // buffer id per program output
   bool graph = true;                // the runtime may replay the launches of a run as one recorded graph
+  // The first sliced.size() steps run `slices` times over, on equal parts of the leading dimension (the last one shorter,
+  // sliced_last): `steps` says what they are on all of it.  part_bytes: of a part of each buffer that lies part behind part, 0
+  // for the others (Planner::sliceSteps).
+  int slices = 1;
+  bool uneven = false;              // the last part is shorter
+  std::vector<Step> sliced, sliced_last;
+  std::vector<size_t> part_bytes;
   std::string dump() const;
 };
 

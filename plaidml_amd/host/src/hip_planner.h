@@ -163,6 +163,7 @@ class Planner {
   void padDepthwiseResults();
   void fusePoolIntoConv();
   void chainProducts();
+  void sliceSteps();
   void pruneDeadSteps();
 
  private:

@@ -66,9 +66,12 @@ class HipExecutable final : public Executable {
         if (b.kind == BufferInfo::Constant)
           hipCheck(pml_hip_memcpy_h2d(device_[i], b.constant->data(), b.constant->size(), nullptr), "upload constant");
       }
-      handles_.assign(plan_->steps.size(), 0);
-      next_handles_.assign(plan_->steps.size(), 0);
-      for (size_t i = 0; i < plan_->steps.size(); ++i) dispatch(i);
+      handles_.resize(plan_->steps.size());
+      for (size_t i = 0; i < plan_->steps.size(); ++i) dispatch(i < plan_->sliced.size() ? plan_->sliced[i] : plan_->steps[i], &handles_[i]);
+      if (plan_->uneven) {
+        last_handles_.resize(plan_->sliced.size());
+        for (size_t i = 0; i < plan_->sliced.size(); ++i) dispatch(plan_->sliced_last[i], &last_handles_[i]);
+      }
       // Where a run begins and ends on the device is read off its clock by the kernels that copy, or by one of their kind
       // (two events around the launches cost a run 8 us); with events where that cannot be had, and under PLAIDML_PROFILE.
       clock_khz_ = pml_hip_clock_khz();
@@ -80,13 +83,19 @@ class HipExecutable final : public Executable {
       hipCheck(pml_hip_stream_sync(nullptr), "sync");
       // Recording is for runs of plain kernel launches and device-to-device copies: the sort, scatter, gather, index and random-number steps keep
       // state or sizes on the host side of their entry points and stay with one-by-one launches.
-      graphable_ = plan_->graph && plan_->steps.size() > 1;
+      graphable_ = plan_->graph && (plan_->steps.size() > 1 || plan_->slices > 1);
       for (const Step& s : plan_->steps)
         if (s.kind != Step::Gemm && s.kind != Step::Conv2d && s.kind != Step::Dwconv2d && s.kind != Step::Pool2d &&
             s.kind != Step::Eltwise && s.kind != Step::Contract && s.kind != Step::Select && s.kind != Step::Copy &&
             s.kind != Step::Softmax && s.kind != Step::Product && s.kind != Step::ConvGrad && s.kind != Step::Rows &&
             s.kind != Step::Argmax && s.kind != Step::TopK)
           graphable_ = false;
+      findSegments();
+      if (segments_.size() > 1) {
+        for (pml_hip_stream* q : {&up_stream_, &down_stream_}) hipCheck(pml_hip_stream_create(q), "stream");
+        for (Segment& seg : segments_)
+          for (pml_hip_event* e : {&seg.up, &seg.done, &seg.down}) hipCheck(pml_hip_event_create(e), "event");
+      }
     } catch (...) {
       release();
       throw;
@@ -119,6 +128,10 @@ class HipExecutable final : public Executable {
       if (outputs[i].bytes < spanBytes(plan_->output_buffers[i], outputs[i])) throw std::runtime_error("output buffer #" + std::to_string(i) + " is too small");
     for (size_t i = 0; i < inputs.size(); ++i)
       if (inputs[i].bytes < spanBytes(plan_->input_buffers[i], inputs[i])) throw std::runtime_error("input buffer #" + std::to_string(i) + " is too small");
+    if (segments_.size() > 1 && !profile && overlapped(inputs, outputs, start, &st)) {
+      g_stats = st;
+      return st.wall_ms;
+    }
     Spans up, down;
     std::vector<Piece> arriving;  // what waits in the staging to be passed on, in the order it is sent
     std::vector<size_t> unstaged;  // outputs that go without it
@@ -216,8 +229,14 @@ class HipExecutable final : public Executable {
   std::vector<bool> owned_;
   void* arena_ = nullptr;
   size_t arena_bytes_ = 0, fixed_bytes_ = 0, unshared_temp_bytes_ = 0;
-  std::vector<int64_t> handles_;
-  std::vector<int64_t> next_handles_;  // the second product of a step that has one behind its first (Step::chained)
+  struct Launch {
+    size_t step;
+    int slice;  // its part of the leading dimension, -1: the whole step
+  };
+  struct Handles {
+    int64_t own = 0, next = 0;  // next: the second product of a step that has one behind its first (Step::chained)
+  };
+  std::vector<Handles> handles_, last_handles_;  // per step; of the sliced ones' last, shorter part
   pml_hip_event ev0_ = nullptr, ev1_ = nullptr;
   uint64_t* stamps_ = nullptr;  // page-locked: the device's clock ahead of and behind a run's launches
   int clock_khz_ = 0;
@@ -289,14 +308,16 @@ class HipExecutable final : public Executable {
       if (!staging_) return s;  // (none now: the next run asks again)
       staging_bytes_ = need;
     }
-    if (in_turn)
-      while (half_events_.size() < 2) {
-        half_events_.push_back(nullptr);
-        hipCheck(pml_hip_event_create(&half_events_.back()), "event");
-      }
+    if (in_turn) needHalfEvents();
     s.base = s.next = static_cast<char*>(staging_);
     if (in_turn) s.slots = s.base + by_kernel;
     return s;
+  }
+  void needHalfEvents() {
+    while (half_events_.size() < 2) {
+      half_events_.push_back(nullptr);
+      hipCheck(pml_hip_event_create(&half_events_.back()), "event");
+    }
   }
   // the place of a value that has its own
   static char* place(Staging* s, size_t bytes) {
@@ -386,14 +407,15 @@ class HipExecutable final : public Executable {
   }
 
   void launchAll(bool profile, InvokeStats* st) {
-    if (profile && step_events_.size() != plan_->steps.size() + 1) {
-      step_events_.assign(plan_->steps.size() + 1, nullptr);
+    const std::vector<Launch>& launches = order_;
+    if (profile && step_events_.size() != launches.size() + 1) {
+      step_events_.assign(launches.size() + 1, nullptr);
       for (auto& e : step_events_) hipCheck(pml_hip_event_create(&e), "event");
     }
     // The launches of a run never change (same plans, same device buffers), so from the third run on they are
     // replayed as one graph recorded during that run; the first two run one by one (first runs of a kernel plan may
     // allocate, which cannot be recorded).  A recording that fails leaves the executable with one-by-one launches.
-    if (graphable_ && !profile && !graph_ && runs_ >= 2) record();
+    if (graphable_ && !profile && !graph_ && runs_ >= 2) graph_ = record(launches);
     ++runs_;
     const bool events = profile || !stamps_;
     if (events) hipCheck(pml_hip_event_record(ev0_, stream_), "event record");
@@ -401,9 +423,9 @@ class HipExecutable final : public Executable {
       hipCheck(pml_hip_graph_launch(graph_, stream_), "graph launch");
       st->replayed = true;
     } else {
-      for (size_t i = 0; i < plan_->steps.size(); ++i) {
-        if (profile) hipCheck(pml_hip_event_record(step_events_[i], stream_), "event record");
-        launch(i);
+      for (size_t k = 0; k < launches.size(); ++k) {
+        if (profile) hipCheck(pml_hip_event_record(step_events_[k], stream_), "event record");
+        launch(launches[k].step, launches[k].slice);
       }
     }
     if (profile) hipCheck(pml_hip_event_record(step_events_.back(), stream_), "event record");
@@ -420,23 +442,35 @@ class HipExecutable final : public Executable {
       st->kernel_ms = ms;
     }
     st->launches = plan_->steps.size();
+    describe(st);
+    if (!profile) return;
+    report(st);
+  }
+
+  // what does not depend on the run
+  void describe(InvokeStats* st) const {
     st->graph_note = graph_note_;
     st->arena_bytes = arena_bytes_;
     st->unshared_temp_bytes = unshared_temp_bytes_;
     st->device_bytes = arena_bytes_ + fixed_bytes_;
-    for (const auto* handles : {&handles_, &next_handles_})
-      for (int64_t h : *handles)
-        if (h) st->device_bytes += pml_hip_plan_bytes(h);
-    if (!profile) return;
+    for (const auto* handles : {&handles_, &last_handles_})
+      for (const Handles& h : *handles)
+        for (int64_t plan : {h.own, h.next})
+          if (plan) st->device_bytes += pml_hip_plan_bytes(plan);
+  }
+
+  void report(InvokeStats* st) {
     // One row per launch, in the reference's format (pmlc/rt/instrument.cc:22-43: id, loc, tag, seconds since
     // the previous point, seconds since the start); loc is the plan's line for the step, tag its kind.
     std::printf("\"id\",\"loc\",\"tag\",\"elapsed\",\"accumulated\"\n");
     double total = 0;
-    st->step_ms.resize(plan_->steps.size());
-    for (size_t i = 0; i < plan_->steps.size(); ++i) {
+    st->step_ms.assign(plan_->steps.size(), 0);
+    const std::vector<Launch>& launches = order_;
+    for (size_t k = 0; k < launches.size(); ++k) {
+      const size_t i = launches[k].step;
       float step = 0;
-      hipCheck(pml_hip_event_elapsed_ms(step_events_[i], step_events_[i + 1], &step), "event elapsed");
-      st->step_ms[i] = step;
+      hipCheck(pml_hip_event_elapsed_ms(step_events_[k], step_events_[k + 1], &step), "event elapsed");
+      st->step_ms[i] += step;
       total += step;
       std::printf("%03d,\"%s\",%d,%7.6f,%7.6f\n", static_cast<int>(i), plan_->steps[i].text.c_str(), static_cast<int>(plan_->steps[i].kind),
                   step * 1e-3, total * 1e-3);
@@ -445,15 +479,16 @@ class HipExecutable final : public Executable {
     std::fflush(stdout);
   }
 
-  void record() {
+  // The launches as one graph, or nullptr (and one-by-one launches from then on).
+  pml_hip_graph record(const std::vector<Launch>& launches) {
     if (pml_hip_capture_begin(stream_) != 0) {
       graph_note_ = pml_hip_last_error();
       graphable_ = false;
-      return;
+      return nullptr;
     }
     bool ok = true;
     try {
-      for (size_t i = 0; i < plan_->steps.size(); ++i) launch(i);
+      for (const Launch& l : launches) launch(l.step, l.slice);
     } catch (const std::exception& e) {
       graph_note_ = e.what();
       ok = false;
@@ -463,9 +498,259 @@ class HipExecutable final : public Executable {
       if (ok) graph_note_ = pml_hip_last_error();
       if (g) pml_hip_graph_destroy(g);
       graphable_ = false;
-      return;
+      return nullptr;
     }
-    graph_ = g;
+    return g;
+  }
+
+  // ---- overlapped runs: copies up, launches and copies down in three queues ------------------------------------------
+
+  // A run of launches, what of the inputs has to be up before them, and what of the outputs may go down behind them.
+  struct Range {
+    size_t index, offset, bytes;
+  };
+  struct Segment {
+    std::vector<Launch> launches;
+    std::vector<Range> needs, yields;
+    pml_hip_graph graph = nullptr;
+    pml_hip_event up = nullptr, done = nullptr, down = nullptr;
+  };
+  std::vector<Segment> segments_;
+  std::vector<Launch> order_;  // of all the segments
+  pml_hip_stream up_stream_ = nullptr, down_stream_ = nullptr;
+  int overlapped_runs_ = 0;
+  // A wait between the queues and a graph of its own cost 20 to 25 us, the link takes 75 us for this many bytes: two 1.6 MB
+  // operands of a product of their own segments took 301 us, in one 275; two of 12.8 MB around a gradient 1070, 1170 in one.
+  static constexpr size_t kWorthASegment = 4 << 20;
+
+  void findSegments() {
+    const Plan& p = *plan_;
+    std::vector<int> input_of(p.buffers.size(), -1);
+    for (size_t i = 0; i < p.input_buffers.size(); ++i) input_of[p.input_buffers[i]] = static_cast<int>(i);
+    std::vector<char> up(p.input_buffers.size(), 0);
+    std::vector<int> writer(p.buffers.size(), -1);  // the last step that writes a buffer
+    for (size_t i = 0; i < p.steps.size(); ++i) {
+      for (int b : {p.steps[i].c, p.steps[i].out2})
+        if (b >= 0) writer[b] = static_cast<int>(i);
+      for (int b : p.steps[i].outs) writer[b] = static_cast<int>(i);
+    }
+    auto reads = [&](const Step& s) {
+      std::vector<size_t> in;
+      auto note = [&](int b) {
+        if (b >= 0 && input_of[b] >= 0) in.push_back(static_cast<size_t>(input_of[b]));
+      };
+      for (int b : {s.a, s.b, s.init, s.a2, s.b2, s.init2, s.next_b, s.next_init, s.out2, s.c}) note(b);
+      for (int b : s.operands) note(b);
+      return in;
+    };
+    const size_t n = p.sliced.size();
+    for (int slice = 0; slice < (n ? p.slices : 0); ++slice) {
+      Segment seg;
+      for (size_t i = 0; i < n; ++i) {
+        seg.launches.push_back({i, slice});
+        for (size_t in : reads(p.steps[i])) {
+          const int buf = p.input_buffers[in];
+          const size_t part = p.part_bytes[buf], bytes = p.buffers[buf].bytes;
+          if (part == 0 && !up[in]) seg.needs.push_back({in, 0, bytes});
+          if (part > 0 && up[in] <= slice) seg.needs.push_back({in, slice * part, std::min(part, bytes - slice * part)});
+          up[in] = static_cast<char>(part > 0 ? slice + 1 : p.slices);
+        }
+      }
+      for (size_t o = 0; o < p.output_buffers.size(); ++o) {
+        const int buf = p.output_buffers[o];
+        if (writer[buf] < 0 || static_cast<size_t>(writer[buf]) >= n) continue;
+        const size_t part = p.part_bytes[buf], bytes = p.buffers[buf].bytes;
+        seg.yields.push_back({o, slice * part, std::min(part, bytes - slice * part)});
+      }
+      segments_.push_back(std::move(seg));
+    }
+    bool fresh = true;
+    for (size_t i = n; i < p.steps.size(); ++i) {
+      std::vector<Range> needs;
+      size_t coming = 0, going = 0;
+      for (size_t in : reads(p.steps[i]))
+        if (!up[in]) {
+          up[in] = 1;
+          needs.push_back({in, 0, p.buffers[p.input_buffers[in]].bytes});
+          coming += needs.back().bytes;
+        }
+      if (fresh || coming >= kWorthASegment) segments_.emplace_back();
+      Segment& seg = segments_.back();
+      seg.launches.push_back({i, -1});
+      seg.needs.insert(seg.needs.end(), needs.begin(), needs.end());
+      for (size_t o = 0; o < p.output_buffers.size(); ++o)
+        if (writer[p.output_buffers[o]] == static_cast<int>(i)) {
+          seg.yields.push_back({o, 0, p.buffers[p.output_buffers[o]].bytes});
+          going += seg.yields.back().bytes;
+        }
+      fresh = going >= kWorthASegment;
+    }
+    for (const Segment& seg : segments_) order_.insert(order_.end(), seg.launches.begin(), seg.launches.end());
+    if (segments_.empty()) return;
+    for (size_t in = 0; in < up.size(); ++in)
+      if (!up[in]) segments_.front().needs.push_back({in, 0, p.buffers[p.input_buffers[in]].bytes});
+    for (size_t o = 0; o < p.output_buffers.size(); ++o)
+      if (writer[p.output_buffers[o]] < 0) segments_.back().yields.push_back({o, 0, p.buffers[p.output_buffers[o]].bytes});
+  }
+
+  // One run, segment by segment: what a segment needs is staged and sent up, its launches wait for that, and what is final behind
+  // it goes down while the link carries the next one's needs up.  Inputs that take more than the slots go through them in turn.
+  // False (and nothing done) where the staging has no place for every other value, or there is none.  An output's place is that of an input which is up before the output exists, where there is one.
+  bool overlapped(const std::vector<HostSpan>& inputs, const std::vector<HostSpan>& outputs, double start, InvokeStats* st) {
+    constexpr size_t kNowhere = ~size_t{0}, kInTurn = kNowhere - 1, kAll = kStageSlots * kStageRun;
+    std::vector<size_t> in_at(inputs.size(), kNowhere), out_at(outputs.size(), kNowhere), up_by(inputs.size(), 0), from(outputs.size(), 0);
+    std::vector<char> lent(inputs.size(), 0);
+    size_t need = 0;
+    auto bytes_of = [&](int buf) { return plan_->buffers[buf].bytes; };
+    for (size_t k = 0; k < segments_.size(); ++k) {
+      for (const Range& r : segments_[k].needs) up_by[r.index] = k;
+      for (size_t q = segments_[k].yields.size(); q-- > 0;)
+        if (segments_[k].yields[q].offset == 0) from[segments_[k].yields[q].index] = k;
+    }
+    size_t staged = 0;
+    for (size_t i = 0; i < inputs.size(); ++i)
+      if (!direct(plan_->input_buffers[i], inputs[i])) staged += padded(bytes_of(plan_->input_buffers[i]));
+    const bool in_turn = staged > kAll;
+    for (size_t i = 0; i < inputs.size(); ++i) {
+      const size_t bytes = bytes_of(plan_->input_buffers[i]);
+      if (direct(plan_->input_buffers[i], inputs[i])) continue;
+      in_at[i] = in_turn && bytes > kKernelCopy ? kInTurn : need;
+      if (in_at[i] != kInTurn) need += padded(bytes);
+    }
+    for (size_t o = 0; o < outputs.size(); ++o) {
+      const int buf = plan_->output_buffers[o];
+      if (direct(buf, outputs[o])) continue;
+      for (size_t i = 0; i < inputs.size() && out_at[o] == kNowhere; ++i) {
+        const int in = plan_->input_buffers[i];
+        if (in_at[i] >= kInTurn || lent[i] || bytes_of(in) < bytes_of(buf)) continue;
+        const bool parts = plan_->slices > 1 && plan_->part_bytes[in] > 0 && plan_->part_bytes[buf] > 0;
+        if (parts ? plan_->part_bytes[in] >= plan_->part_bytes[buf] : up_by[i] <= from[o]) {
+          out_at[o] = in_at[i];
+          lent[i] = 1;
+        }
+      }
+      if (out_at[o] == kNowhere) {
+        out_at[o] = need;
+        need += padded(bytes_of(buf));
+      }
+    }
+    if (need > (in_turn ? kAll / 2 : kAll)) return false;
+    const size_t slots = need;
+    if (in_turn) need += kAll;
+    if (need > staging_bytes_) {
+      if (staging_) pinnedFree(staging_);
+      staging_bytes_ = 0;
+      staging_ = pinnedAllocRaw(need);
+      if (!staging_) return false;
+      staging_bytes_ = need;
+    }
+    if (in_turn) needHalfEvents();
+    char* const base = static_cast<char*>(staging_);
+    // (an output lies in its lender's place part behind part, as far apart as the lender's are)
+    auto out_place = [&](const Range& r) {
+      const size_t part = plan_->slices > 1 ? plan_->part_bytes[plan_->output_buffers[r.index]] : 0;
+      size_t at = out_at[r.index] + r.offset;
+      if (part > 0)
+        for (size_t i = 0; i < inputs.size(); ++i)
+          if (in_at[i] == out_at[r.index] && plan_->part_bytes[plan_->input_buffers[i]] > 0)
+            at = out_at[r.index] + r.offset / part * plan_->part_bytes[plan_->input_buffers[i]];
+      return base + at;
+    };
+    auto sync = [&] {
+      for (pml_hip_stream s : {up_stream_, stream_, down_stream_}) (void)pml_hip_stream_sync(s);
+    };
+    try {
+      const bool record_now = graphable_ && overlapped_runs_++ >= 2;
+      size_t turn = 0;
+      for (Segment& seg : segments_) {
+        Spans up, down;
+        for (const Range& r : seg.needs) {
+          const int buf = plan_->input_buffers[r.index];
+          const HostSpan& in = inputs[r.index];
+          char* const dev = static_cast<char*>(device_[buf]) + r.offset;
+          const bool slotted = in_at[r.index] == kInTurn, by_kernel = r.bytes <= kKernelCopy && !slotted;
+          for (size_t at = 0; at < r.bytes;) {
+            const size_t n = in_at[r.index] == kNowhere ? r.bytes : std::min(kStageRun, r.bytes - at);
+            const char* src = static_cast<const char*>(in.data) + (r.offset + at) * (in.f32 ? 2 : 1);
+            if (in_at[r.index] != kNowhere) {
+              char* const to = base + (slotted ? slots + turn % kStageSlots * kStageRun : in_at[r.index] + r.offset + at);
+              if (slotted && turn >= kStageSlots && turn % kStageHalf == 0) hipCheck(pml_hip_event_sync(half_events_[turn / kStageHalf % 2]), "event sync");
+              if (in.f32)
+                hostToBf16(reinterpret_cast<uint16_t*>(to), reinterpret_cast<const float*>(src), n / 2);
+              else
+                hostCopy(to, src, n);
+              src = to;
+            }
+            if (by_kernel)
+              up.add(dev + at, src, n);
+            else
+              hipCheck(pml_hip_memcpy_h2d_async(dev + at, src, n, up_stream_), "h2d");
+            if (slotted && ++turn % kStageHalf == 0) hipCheck(pml_hip_event_record(half_events_[(turn / kStageHalf - 1) % 2], up_stream_), "event record");
+            at += n;
+          }
+        }
+        up.issue(up_stream_, nullptr, false);
+        if (!seg.needs.empty()) {
+          hipCheck(pml_hip_event_record(seg.up, up_stream_), "event record");
+          hipCheck(pml_hip_stream_wait_event(stream_, seg.up), "wait");
+          st->h2d_ms = nowMs() - start;
+        }
+        if (record_now && !seg.graph && graphable_ && seg.launches.size() > 1) seg.graph = record(seg.launches);
+        if (seg.graph) {
+          hipCheck(pml_hip_graph_launch(seg.graph, stream_), "graph launch");
+          st->replayed = true;
+        } else {
+          for (const Launch& l : seg.launches) launch(l.step, l.slice);
+        }
+        hipCheck(pml_hip_event_record(seg.done, stream_), "event record");
+        if (seg.yields.empty()) continue;
+        hipCheck(pml_hip_stream_wait_event(down_stream_, seg.done), "wait");
+        for (const Range& r : seg.yields) {
+          const HostSpan& out = outputs[r.index];
+          const char* const dev = static_cast<const char*>(device_[plan_->output_buffers[r.index]]) + r.offset;
+          char* const to = out_at[r.index] == kNowhere ? static_cast<char*>(out.data) + r.offset : out_place(r);
+          if (r.bytes <= kKernelCopy)
+            down.add(to, dev, r.bytes);
+          else
+            hipCheck(pml_hip_memcpy_d2h_async(to, dev, r.bytes, down_stream_), "d2h");
+        }
+        down.issue(down_stream_, nullptr, false);
+        hipCheck(pml_hip_event_record(seg.down, down_stream_), "event record");
+      }
+      for (Segment& seg : segments_) {
+        bool waited = false;
+        for (const Range& r : seg.yields) {
+          if (out_at[r.index] == kNowhere) continue;
+          if (!waited) hipCheck(pml_hip_event_sync(seg.down), "event sync");
+          waited = true;
+          const HostSpan& out = outputs[r.index];
+          char* const to = static_cast<char*>(out.data) + r.offset * (out.f32 ? 2 : 1);
+          if (out.f32)
+            hostFromBf16(reinterpret_cast<float*>(to), reinterpret_cast<const uint16_t*>(out_place(r)), r.bytes / 2);
+          else
+            hostCopy(to, out_place(r), r.bytes);
+        }
+      }
+      for (pml_hip_stream s : {up_stream_, stream_, down_stream_}) hipCheck(pml_hip_stream_sync(s), "stream sync");
+    } catch (...) {
+      sync();  // queued copies may still use the caller's memory
+      throw;
+    }
+    st->wall_ms = nowMs() - start;
+    // A segment's time is from where it could begin -- its needs up, the one before it done -- to its end.
+    for (size_t k = 0; k < segments_.size(); ++k) {
+      float ms = 0, behind = 0;
+      const Segment& seg = segments_[k];
+      if (!seg.needs.empty()) hipCheck(pml_hip_event_elapsed_ms(seg.up, seg.done, &ms), "event elapsed");
+      if (k > 0) hipCheck(pml_hip_event_elapsed_ms(segments_[k - 1].done, seg.done, &behind), "event elapsed");
+      st->kernel_ms += k == 0 ? ms : seg.needs.empty() ? behind : std::min(ms, behind);
+    }
+    st->launches = plan_->steps.size();
+    describe(st);
+    st->kernel_ms = std::min(st->kernel_ms, st->wall_ms);
+    st->h2d_ms = std::min(st->h2d_ms, st->wall_ms - st->kernel_ms);
+    st->d2h_ms = st->wall_ms - st->h2d_ms - st->kernel_ms;
+    return true;
   }
 
   // Offsets of the temporaries in the arena.  A temporary is live from the first to the last step that names
@@ -485,6 +770,10 @@ class HipExecutable final : public Executable {
       for (int b : s.operands) touch(b, i);
       for (int b : s.outs) touch(b, i);
     }
+    // (what outlives the sliced steps is written from their first part on)
+    if (plan_->slices > 1)
+      for (size_t b = 0; b < nb; ++b)
+        if (plan_->part_bytes[b] > 0 && first[b] >= 0) first[b] = 0;
     std::vector<size_t> offsets(nb, 0);
     struct Block { size_t off, size; };
     std::vector<Block> free_blocks;
@@ -540,11 +829,21 @@ class HipExecutable final : public Executable {
   }
 
   void release() {
-    for (auto* handles : {&handles_, &next_handles_}) {
-      for (int64_t h : *handles)
-        if (h) pml_hip_plan_free(h);
+    for (auto* handles : {&handles_, &last_handles_}) {
+      for (const Handles& h : *handles)
+        for (int64_t plan : {h.own, h.next})
+          if (plan) pml_hip_plan_free(plan);
       handles->clear();
     }
+    for (Segment& s : segments_) {
+      if (s.graph) pml_hip_graph_destroy(s.graph);
+      for (pml_hip_event e : {s.up, s.done, s.down})
+        if (e) pml_hip_event_destroy(e);
+    }
+    segments_.clear();
+    if (up_stream_) pml_hip_stream_destroy(up_stream_);
+    if (down_stream_) pml_hip_stream_destroy(down_stream_);
+    up_stream_ = down_stream_ = nullptr;
     for (size_t i = 0; i < device_.size(); ++i)
       if (device_[i] && owned_[i]) pml_hip_free(device_[i]);
     device_.clear();
@@ -576,8 +875,7 @@ class HipExecutable final : public Executable {
 
   static size_t elemSize(int dt) { return util::byteSize(static_cast<util::DataType>(dt)); }
 
-  void dispatch(size_t i) {
-    const Step& s = plan_->steps[i];
+  void dispatch(const Step& s, Handles* handles) {
     int64_t h = 0;
     switch (s.kind) {
       case Step::Gemm: {
@@ -604,23 +902,30 @@ class HipExecutable final : public Executable {
       case Step::Copy: return;
     }
     if (!h) throw std::runtime_error("hip dispatch failed for '" + s.text + "': " + pml_hip_last_error());
-    handles_[i] = h;
+    handles->own = h;
     // constant right-hand sides are re-laid-out once, here
     if (s.kind == Step::Gemm && s.b_constant && !s.b_is_nk)
       hipCheck(pml_hip_gemm_pack_b(h, ptr(s.b, s.b_off, elemSize(s.gemm.in_dtype)), nullptr), "pack_b");
     if (s.kind == Step::Gemm && s.gemm.k2 > 0 && s.b2_constant && !s.b_is_nk)
       hipCheck(pml_hip_gemm_pack_b2(h, ptr(s.b2, s.b2_off, elemSize(s.gemm.in_dtype)), nullptr), "pack_b2");
     if (s.chained) {
-      next_handles_[i] = pml_hip_gemm_dispatch(&s.next_gemm);
-      if (!next_handles_[i]) throw std::runtime_error("hip dispatch failed for '" + s.text + "': " + pml_hip_last_error());
-      hipCheck(pml_hip_gemm_pack_b(next_handles_[i], ptr(s.next_b, s.next_b_off, elemSize(s.next_gemm.in_dtype)), nullptr), "pack_b");
+      handles->next = pml_hip_gemm_dispatch(&s.next_gemm);
+      if (!handles->next) throw std::runtime_error("hip dispatch failed for '" + s.text + "': " + pml_hip_last_error());
+      hipCheck(pml_hip_gemm_pack_b(handles->next, ptr(s.next_b, s.next_b_off, elemSize(s.next_gemm.in_dtype)), nullptr), "pack_b");
     }
     if (s.kind == Step::Conv2d && s.b_constant) hipCheck(pml_hip_conv2d_pack_filter(h, ptr(s.b), nullptr), "pack_filter");
     if (s.kind == Step::Dwconv2d && s.b_constant) hipCheck(pml_hip_dwconv2d_pack_filter(h, ptr(s.b), nullptr), "pack_filter");
   }
 
-  void launch(size_t i) {
-    const Step& s = plan_->steps[i];
+  // Step i, or its part `slice` of the leading dimension.
+  void launch(size_t i, int slice = -1) {
+    const bool last = slice >= 0 && slice == plan_->slices - 1;
+    const Step& s = slice < 0 ? plan_->steps[i] : last ? plan_->sliced_last[i] : plan_->sliced[i];
+    const Handles& h = last && plan_->uneven ? last_handles_[i] : handles_[i];
+    auto ptr = [&](int buf, int64_t elem_off = 0, size_t elem_size = 1) -> char* {
+      if (buf < 0) return nullptr;
+      return static_cast<char*>(device_[buf]) + (slice > 0 ? static_cast<size_t>(slice) * plan_->part_bytes[buf] : 0) + elem_off * static_cast<int64_t>(elem_size);
+    };
     const void* operands[PML_HIP_MAX_EPI_OPERANDS] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
     void* outs[PML_HIP_MAX_EPI_OPERANDS] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
     for (size_t k = 0; k < s.operands.size() && k < PML_HIP_MAX_EPI_OPERANDS; ++k) operands[k] = ptr(s.operands[k]);
@@ -629,7 +934,7 @@ class HipExecutable final : public Executable {
       case Step::Gemm: {
         const size_t es = elemSize(s.gemm.in_dtype);
         if (s.chained) {
-          hipCheck(pml_hip_gemm_chain_invoke(handles_[i], next_handles_[i], ptr(s.a), ptr(s.c), ptr(s.init), ptr(s.a2), ptr(s.init2), operands, ptr(s.out2),
+          hipCheck(pml_hip_gemm_chain_invoke(h.own, h.next, ptr(s.a), ptr(s.c), ptr(s.init), ptr(s.a2), ptr(s.init2), operands, ptr(s.out2),
                                              ptr(s.next_init), stream_),
                    s.text.c_str());
           break;
@@ -639,30 +944,30 @@ class HipExecutable final : public Executable {
         if (s.gemm.k2 > 0) {
           const void* b2 = ptr(s.b2, s.b2_off, es);
           if (s.b2_constant && !s.b_is_nk) b2 = nullptr;
-          hipCheck(pml_hip_gemm_invoke2(handles_[i], ptr(s.a, s.a_off, es), b, ptr(s.c, s.c_off, elemSize(s.gemm.c_dtype)), ptr(s.init),
+          hipCheck(pml_hip_gemm_invoke2(h.own, ptr(s.a, s.a_off, es), b, ptr(s.c, s.c_off, elemSize(s.gemm.c_dtype)), ptr(s.init),
                                         ptr(s.a2, s.a2_off, es), b2, ptr(s.init2), operands, outs, stream_),
                    s.text.c_str());
           break;
         }
-        hipCheck(pml_hip_gemm_invoke(handles_[i], ptr(s.a, s.a_off, es), b, ptr(s.c, s.c_off, elemSize(s.gemm.c_dtype)),
+        hipCheck(pml_hip_gemm_invoke(h.own, ptr(s.a, s.a_off, es), b, ptr(s.c, s.c_off, elemSize(s.gemm.c_dtype)),
                                      ptr(s.init), operands, outs, stream_),
                  s.text.c_str());
         break;
       }
       case Step::Conv2d:
-        hipCheck(pml_hip_conv2d_invoke(handles_[i], ptr(s.a), s.b_constant ? nullptr : ptr(s.b), ptr(s.c), ptr(s.init), operands,
+        hipCheck(pml_hip_conv2d_invoke(h.own, ptr(s.a), s.b_constant ? nullptr : ptr(s.b), ptr(s.c), ptr(s.init), operands,
                                        outs, stream_),
                  s.text.c_str());
         break;
       case Step::Dwconv2d:
-        hipCheck(pml_hip_dwconv2d_invoke(handles_[i], ptr(s.a), s.b_constant ? nullptr : ptr(s.b), ptr(s.c), operands, outs, stream_),
+        hipCheck(pml_hip_dwconv2d_invoke(h.own, ptr(s.a), s.b_constant ? nullptr : ptr(s.b), ptr(s.c), operands, outs, stream_),
                  s.text.c_str());
         break;
       case Step::Pool2d:
-        hipCheck(pml_hip_pool2d_invoke(handles_[i], ptr(s.a), ptr(s.c), ptr(s.out2), stream_), s.text.c_str());
+        hipCheck(pml_hip_pool2d_invoke(h.own, ptr(s.a), ptr(s.c), ptr(s.out2), stream_), s.text.c_str());
         break;
       case Step::Eltwise:
-        hipCheck(pml_hip_eltwise_invoke(handles_[i], ptr(s.a), ptr(s.c), operands, outs, stream_), s.text.c_str());
+        hipCheck(pml_hip_eltwise_invoke(h.own, ptr(s.a), ptr(s.c), operands, outs, stream_), s.text.c_str());
         break;
       case Step::Select:
         hipCheck(pml_hip_select(&s.sel, operands[0], operands[1], operands[2], ptr(s.c), stream_), s.text.c_str());
@@ -686,15 +991,15 @@ class HipExecutable final : public Executable {
                  s.text.c_str());
         break;
       case Step::Contract:
-        hipCheck(pml_hip_contract_invoke(handles_[i], operands, ptr(s.c), stream_), s.text.c_str());
+        hipCheck(pml_hip_contract_invoke(h.own, operands, ptr(s.c), stream_), s.text.c_str());
         break;
       case Step::Product:
-        hipCheck(pml_hip_product_invoke(handles_[i], ptr(s.a, s.a_off, elemSize(s.prod.in_dtype)), ptr(s.b, s.b_off, elemSize(s.prod.in_dtype)),
+        hipCheck(pml_hip_product_invoke(h.own, ptr(s.a, s.a_off, elemSize(s.prod.in_dtype)), ptr(s.b, s.b_off, elemSize(s.prod.in_dtype)),
                                         ptr(s.c), ptr(s.init), operands, stream_),
                  s.text.c_str());
         break;
       case Step::ConvGrad:
-        hipCheck(pml_hip_conv2d_grad_invoke(handles_[i], ptr(s.a), ptr(s.b), ptr(s.c), stream_), s.text.c_str());
+        hipCheck(pml_hip_conv2d_grad_invoke(h.own, ptr(s.a), ptr(s.b), ptr(s.c), stream_), s.text.c_str());
         break;
       case Step::Copy:
         hipCheck(pml_hip_memcpy_d2d(ptr(s.c), ptr(s.a), s.copy_bytes, stream_), s.text.c_str());

@@ -1,0 +1,134 @@
+"""Programs that run in parts of the leading dimension, and runs whose copies and launches overlap (host/src/hip_plan_slice.cc,
+hip_runtime.cc): whole numbers, so that every run is compared value for value with numpy."""
+import re
+
+import numpy as np
+import pytest
+
+from plaidml_amd import edsl as P
+from plaidml_amd import op as Pop
+
+DT = {'f32': P.DType.FLOAT32, 'bf16': P.DType.BFLOAT16}
+
+
+def whole(rng, *shape, top=2):
+    return rng.integers(-top, top + 1, shape).astype(np.float32)
+
+
+def dense(dt, m, k=640):
+    """Operands in parts and as a whole, a product on top of the one in parts."""
+    X, R, W, V, b = (P.Placeholder(DT[dt], s) for s in ([m, k], [m, 256], [k, 256], [256, 64], [256]))
+    y = Pop.relu(Pop.dot(X, W) + b + R)
+    draw = lambda rng: [whole(rng, m, k), whole(rng, m, 256), whole(rng, k, 256, top=1), whole(rng, 256, 64, top=1) * (rng.random((256, 64)) < 0.05), whole(rng, 256)]
+
+    def want(x, r, w, v, c):
+        y = np.maximum(x @ w + c + r, 0)
+        return [y, y @ v]
+    return P.Program('dense', [X, R, W, V, b], [y, Pop.dot(y, V)]), draw, want
+
+
+def images(dt, n, hw=64):
+    """A convolution and a maximum over windows in parts, their sum over images not."""
+    X, F = P.Placeholder(DT[dt], [n, hw, hw, 64]), P.Placeholder(DT[dt], [1, 1, 64, 512])
+    y = Pop.relu(Pop.convolution(X, F, strides=[1, 1]))
+    top = Pop.pool(y, 'max', [2, 2], [2, 2], autopad='valid')
+    draw = lambda rng: [whole(rng, n, hw, hw, 64), whole(rng, 1, 1, 64, 512, top=1)]
+
+    def want(x, f):
+        t = np.maximum(x.reshape(-1, 64) @ f.reshape(64, 512), 0).reshape(n, hw // 2, 2, hw // 2, 2, 512).max((2, 4))
+        return [t, t.max(0)]
+    return P.Program('images', [X, F], [top, Pop.max(top, axes=[0])]), draw, want
+
+
+def rows(dt, m, c=520):
+    X, g = P.Placeholder(DT[dt], [m, c]), P.Placeholder(DT[dt], [c])
+    d = X - Pop.max(X, axes=[-1], keepdims=True)
+    draw = lambda rng: [whole(rng, m, c, top=60), whole(rng, c)]
+    return P.Program('rows', [X, g], [d * g]), draw, lambda x, h: [(x - x.max(-1, keepdims=True)) * h]
+
+
+def batches(dt, n, r=96):
+    A, B = P.Placeholder(DT[dt], [n, r, 64]), P.Placeholder(DT[dt], [n, 64, 80])
+    x, i, j, k = P.TensorIndexes(4)
+    C = P.Contraction().outShape(n, r, 80).outAccess(x, i, j).sum(A[x, i, k] * B[x, k, j]).build()
+    draw = lambda rng: [whole(rng, n, r, 64), whole(rng, n, 64, 80, top=1)]
+    return P.Program('batches', [A, B], [C]), draw, lambda a, b: [np.matmul(a, b)]
+
+
+CASES = {'dense': (dense, 3571), 'dense even': (dense, 4096), 'images': (images, 21), 'rows': (rows, 5003), 'batches': (batches, 401)}
+
+
+def build(name, dt, scale=1):
+    fn, size = CASES[name]
+    return fn(dt, size * scale)
+
+
+def parts(program):
+    program.compile('')
+    m = re.search(r'steps 0 to (\d+) in (\d+) parts', dict(program.passes)['hip-plan'])
+    return (int(m.group(1)) + 1, int(m.group(2))) if m else (0, 1)
+
+
+def test_what_runs_in_parts():
+    for name in CASES:
+        steps, n = parts(build(name, 'f32')[0])
+        assert steps >= 1 and 2 <= n <= 4, name
+    assert parts(dense('f32', 64)[0]) == (0, 1)  # (nothing to carry meanwhile)
+    X, W = P.Placeholder(DT['f32'], [4096, 1024]), P.Placeholder(DT['f32'], [4096, 64])
+    i, j, k = P.TensorIndexes(3)
+    # rows of the result are columns of what comes in
+    assert parts(P.Program('across', [X, W], [P.Contraction().outShape(1024, 64).outAccess(i, j).sum(X[k, i] * W[k, j]).build()])) == (0, 1)
+    # the same value in parts and as a whole
+    S = P.Placeholder(DT['f32'], [2048, 2048])
+    assert parts(P.Program('square', [S], [Pop.dot(S, S)])) == (0, 1)
+    # sums over the leading dimension
+    assert parts(P.Program('sum', [X], [Pop.sum(X, axes=[0])])) == (0, 1)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('dt', ['f32', 'bf16'])
+@pytest.mark.parametrize('pinned_results', [True, False])
+@pytest.mark.parametrize('name', sorted(CASES))
+def test_every_run(monkeypatch, dt, pinned_results, name):
+    """Launched one by one, recorded and replayed; whole runs with other values each time; a profile and no page-locked memory between."""
+    print(name, dt, flush=True)
+    if not pinned_results:
+        monkeypatch.setattr(P, '_result_array', lambda d, sizes, nbytes: np.empty(sizes, d))
+    program, draw, want = build(name, dt, 1 if dt == 'f32' else 2)
+    if name == 'dense':
+        assert parts(program)[1] > 1
+    runner = P.Runner(program, target='hip')
+    rounded = (lambda a: a) if dt == 'f32' else P.round_bf16
+    for run in range(7):
+        arrays = draw(np.random.default_rng(run))
+        with monkeypatch.context() as patch:
+            if run == 4:
+                patch.setenv('PLAIDML_PROFILE', '1')
+            if run == 5:
+                patch.setenv('PLAIDML_PINNED', '0')
+            got = runner.run(arrays)
+        s = P.last_run_stats()
+        assert s['kernel_ms'] > 0 and s['h2d_ms'] + s['kernel_ms'] + s['d2h_ms'] == pytest.approx(runner.ms, rel=1e-6, abs=1e-9)
+        exact = want(*arrays)
+        if name.startswith('dense') and dt == 'bf16':  # (the second product takes the rounded first one)
+            exact = [exact[0], rounded(exact[0]) @ arrays[3]]
+        for k, (g, w) in enumerate(zip(got, exact)):
+            np.testing.assert_array_equal(g, rounded(w.astype(np.float32)), err_msg='%s run %d result %d' % (name, run, k))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('dt', ['f32', 'bf16'])
+def test_more_than_the_staging_holds(dt):
+    """Operands past the staging's slots, of which every part takes several."""
+    m = {'f32': 18001, 'bf16': 36001}[dt]  # 46 MB
+    program, draw, want = dense(dt, m)
+    assert parts(program)[1] > 1
+    runner = P.Runner(program, target='hip')
+    for run in range(4):
+        arrays = draw(np.random.default_rng(run))
+        got = runner.run(arrays)
+        exact = want(*arrays)
+        if dt == 'bf16':
+            exact = [P.round_bf16(exact[0]), P.round_bf16(P.round_bf16(exact[0]) @ arrays[3])]
+        for g, w in zip(got, exact):
+            np.testing.assert_array_equal(g, w)
