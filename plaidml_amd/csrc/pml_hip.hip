@@ -93,6 +93,10 @@ struct Plan {
   int tile_direct = -1;
   // a convolution that runs over its window in LDS (`bt` holds the filter as that kernel multiplies it)
   WinShape win;
+  // a product that runs in panels once its right-hand sides are packed: the configuration (-1: it does not) and their fragments
+  int panel = -1;
+  void* panel_bt = nullptr;
+  bool panel_fresh[2] = {false, false};  // they hold what `bt` holds; what `bt2` holds
   // register-filter convolution: a filter packed once, in the order the kernel holds it in registers
   void* reg_image = nullptr;
   // product over free strides, and a convolution's gradients built on it: the prepared arguments (workspace in `ws`),
@@ -124,6 +128,7 @@ struct Plan {
   ~Plan() {
     if (bt) (void)hipFree(bt);
     if (bt2) (void)hipFree(bt2);
+    if (panel_bt) (void)hipFree(panel_bt);
     if (patches) (void)hipFree(patches);
     if (s2d) (void)hipFree(s2d);
     if (reg_image) (void)hipFree(reg_image);
@@ -990,6 +995,26 @@ static std::string stream_text(int mfma_kind, bool conv, IgemmArgs g, bool init,
   return ", streamed rows past " + (rows && kn ? packed + " or as it lies" : rows ? packed : std::string("B as it lies")) + " mfma=" + mfma16_name(mfma_kind);
 }
 
+// Whether, and as what, a product whose right-hand sides are packed runs in panels (panel.hip).  bf16, where no tile is named, no
+// direct tile is cheaper, K is not split over workgroups and the rows do not stream (K up to 256).  Of 800 products (ranges at
+// panel_us) those of 256 x 256, 256 x 128 and 192 x 384 tiles gain 1.21 to 1.25 x on average, of 128 x 128 tiles 1.13 (three
+// stages) and 1.30 (two), of 64 x 64 tiles that share K 1.08; plain 64 x 64 tiles, which several share a CU, lose as often
+// as they gain (0.98), and 128 x 128 tiles over up to 160 columns, most of a 256 columns wide panel, lose (0.86 to 0.97).
+static int panel_of(const pml_hip_gemm_desc& d, int kind, int tile, const DirectTiles& direct, const void* ws) {
+  if (kind != KIND_BF16 || d.b_layout || PML_HIP_FLAG_TILE_OF(d.flags) >= 0 || direct.rows >= 0 || ws || d.k + d.k2 <= 256) return -1;
+  const bool wide = tile == TILE_128x128_W8 || tile == TILE_128x128_W8_S2 || tile == TILE_256x128_W16 || tile == TILE_256x256_W8 || tile == TILE_192x384_W8;
+  if (!(wide && d.n > 160) && tile != TILE_64x64_W8_K2) return -1;
+  IgemmArgs g;
+  gemm_args(d, g);
+  g.Bt = g.A = g.C = (void*)256;  // (stand for operands that are there; nothing is read)
+  for (int i = 0; i < d.tail.n_operands; ++i) g.operands[i] = g.A;
+  if (d.init_kind) g.init = g.A;
+  g.ldbt = d.k;
+  if (stream_takes(tile, false, g)) return -1;
+  double us;
+  return panel_config(g, d.init_kind != 0, &us);
+}
+
 int64_t pml_hip_gemm_dispatch(const pml_hip_gemm_desc* d) {
   const int kind = gemm_desc_kind(d);
   if (kind < 0) return 0;
@@ -1017,6 +1042,7 @@ int64_t pml_hip_gemm_dispatch(const pml_hip_gemm_desc* d) {
   if (p->tile == TILE_64x64_KSPLIT && !p->ws) p->tile = TILE_64x64;  // (not worth splitting, no memory for the workspace, or not run)
   p->b_split = kind == KIND_F32X3 && !d->b_layout && d->k % 32 == 0 && !p->ws;
   p->b_kn = kind == KIND_BF16 && p->direct.rows < 0 && takes_b_as_given(*d, kind, p->tile, d->n);
+  p->panel = panel_of(*d, kind, p->tile, p->direct, p->ws);
   if (!d->b_layout && !(p->bt = p->hold(p->bt_bytes))) {
     delete p;
     fail("gemm: cannot allocate the packed right-hand side");
@@ -1039,6 +1065,7 @@ int64_t pml_hip_gemm_dispatch(const pml_hip_gemm_desc* d) {
     p->text += std::string(", with B as it lies") + (p->b_kn ? " or packed" : "") + " through registers mfma=" + mfma16_name(kind);
   else if (p->b_kn)
     p->text += std::string(", with B packed through registers mfma=") + mfma16_name(kind);
+  if (p->panel >= 0) p->text += ", with B packed " + panel_text(p->panel) + " mfma=" + mfma16_name(kind);
   {
     IgemmArgs g;
     gemm_args(*d, g);
@@ -1120,6 +1147,7 @@ static int gemm_run(const pml_hip_gemm_desc& d, int mfma_kind, int tile, const D
     if (!second->b2 && (!second->packed2 || d.b_layout)) return fail("gemm_invoke2: b2 is null and no packed right-hand side exists");
     if (((uintptr_t)second->a2 & 15) != 0 || (d.b_layout && ((uintptr_t)second->b2 & 15) != 0)) return fail("gemm_invoke2: the second product's operands must be 16-byte aligned");
     if (d.init2_kind && !second->init2) return fail("gemm_invoke2: the plan expects a second initial value");
+    if (plan && second->b2) plan->panel_fresh[1] = false;
     if (second->b2 && !d.b_layout &&
         check(transpose_pack(es, second->b2, second->bt2, d.k2, d.n, d.ldb2, d.k2, (hipStream_t)s), "transpose_pack"))
       return 1;
@@ -1158,9 +1186,10 @@ static int gemm_run(const pml_hip_gemm_desc& d, int mfma_kind, int tile, const D
   // (rows that stream take a [K][N] right-hand side as it lies, too)
   if (transposed && !(!packed && streams_given(mfma_kind, tile, false, b, d.ldb, g))) {
     // (from here on `bt` holds the plain transposed form, whatever a packed copy was kept in before)
-    if (plan) plan->bt_is_split = plan->bt_is_kn = false;
+    if (plan) plan->bt_is_split = plan->bt_is_kn = plan->panel_fresh[0] = false;
     if (check(transpose_pack(es, b, bt, d.k, d.n, d.ldb, bt_ld, (hipStream_t)s), "transpose_pack")) return 1;
   }
+  if (plan && plan->panel_fresh[0] && (d.k2 == 0 || plan->panel_fresh[1]) && !b && (!second || !second->b2) && panel_runs(g)) return check(panel_launch(plan->panel, g, plan->panel_bt, (hipStream_t)s), "panel_launch");
   return check(igemm_launch(b_split ? KIND_F32X3P : mfma_kind, tile, false, g, (hipStream_t)s), "igemm_launch");
 }
 
@@ -1551,6 +1580,20 @@ int pml_hip_conv2d_invoke(int64_t plan, const void* input, const void* filter, v
   return check(igemm_launch(p->b_split ? KIND_F32X3P : p->mfma_kind, tile, true, g, (hipStream_t)s), "igemm_launch");
 }
 
+// The right-hand side (second: of the second product) in the order a panel multiplies it, besides the form that tiles read.
+// (No memory for it: the product runs in tiles.)
+static int pack_panel(Plan* p, const void* b, bool second, hipStream_t s) {
+  if (p->panel < 0) return 0;
+  const pml_hip_gemm_desc& d = p->gemm;
+  p->panel_fresh[second] = false;
+  const size_t first = winconv_pack_bytes(2, 1, d.k, d.n);
+  if (!p->panel_bt && !(p->panel_bt = p->hold(first + winconv_pack_bytes(2, 1, d.k2, d.n)))) return 0;
+  const WinFilter w = {1, (int)(second ? d.k2 : d.k), (int)d.n, 0, 0, second ? d.ldb2 : d.ldb, 1};
+  if (check(winconv_pack_launch(2, b, w, (char*)p->panel_bt + (second ? first : 0), s), "winconv_pack_launch")) return 1;
+  p->panel_fresh[second] = true;
+  return 0;
+}
+
 int pml_hip_gemm_pack_b(int64_t plan, const void* b, pml_hip_stream s) {
   Plan* p = (Plan*)(intptr_t)plan;
   if (!p || p->kind != PLAN_GEMM || !b) return fail("gemm_pack_b: bad argument");
@@ -1566,6 +1609,7 @@ int pml_hip_gemm_pack_b(int64_t plan, const void* b, pml_hip_stream s) {
   p->bt_is_kn = p->b_kn;
   if (p->b_split && check(split_rows_launch(p->bt, d.n, p->bt_ld, d.k, (hipStream_t)s), "split_rows_launch")) return 1;
   p->bt_is_split = p->b_split;
+  if (pack_panel(p, b, false, (hipStream_t)s)) return 1;
   p->packed = true;
   if (p->direct.rows >= 0 && p->ws) {
     // (its invokes take the direct tile from now on; one that brings a right-hand side all the same does not split K)
@@ -1628,6 +1672,7 @@ int pml_hip_gemm_pack_b2(int64_t plan, const void* b2, pml_hip_stream s) {
   const pml_hip_gemm_desc& d = p->gemm;
   if (d.b_layout) return fail("gemm_pack_b2: an [N][K] right-hand side needs no packing");
   if (check(transpose_pack(dt_size(d.in_dtype), b2, p->bt2, d.k2, d.n, d.ldb2, d.k2, (hipStream_t)s), "transpose_pack")) return 1;
+  if (pack_panel(p, b2, true, (hipStream_t)s)) return 1;
   p->packed2 = true;
   return 0;
 }
