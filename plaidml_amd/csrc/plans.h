@@ -264,16 +264,18 @@ std::string winconv_text(const WinShape& shape);
 struct WinFilter {
   int taps, k, n;
   int64_t first, tap_stride, k_stride, n_stride;
+  int frags = 2;  // that hold neighbouring columns
 };
-size_t winconv_pack_bytes(int es, int taps, int64_t k, int64_t n);
+size_t winconv_pack_bytes(int es, int taps, int64_t k, int64_t n, int frags = 2);
 hipError_t winconv_pack_launch(int es, const void* filter, const WinFilter& w, void* out, hipStream_t s);
-// bf16 products over a right-hand side packed as a 1 x 1 filter is (winconv_pack_launch; the second product's behind the first's),
-// A through a ring in LDS: panel.hip.  panel_config: the configuration for a product's sizes, -1 for forms it does not take;
-// panel_runs: whether it takes the operands of a call.
-int panel_config(const IgemmArgs& a, bool init, double* us);
-bool panel_runs(const IgemmArgs& a);
+// bf16 and int8 products over a right-hand side packed as a 1 x 1 filter is (winconv_pack_launch with panel_frags; the second
+// product's behind the first's), A through a ring in LDS: panel.hip.  panel_config: the configuration for a product's sizes, -1 for
+// forms it does not take; panel_runs: whether it takes the operands of a call.
+int panel_config(int kind, const IgemmArgs& a, bool init, double* us);
+int panel_frags(int kind, const IgemmArgs& a);
+bool panel_runs(int kind, const IgemmArgs& a);
 std::string panel_text(int config);
-hipError_t panel_launch(int config, const IgemmArgs& a, const void* packed, hipStream_t s);
+hipError_t panel_launch(int kind, int config, const IgemmArgs& a, const void* packed, hipStream_t s);
 hipError_t winconv_launch(int kind, const IgemmArgs& a, const WinShape& shape, hipStream_t s);  // a.Bt: the packed filter
 hipError_t mfma_probe_launch(int blocks, int iters, int random, float* sink, unsigned long long* clk, hipStream_t s);
 // splits a packed fp32 Bt[rows][ld] in place (k values per row, a multiple of 32) into the heads / remainders form

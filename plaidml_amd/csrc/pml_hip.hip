@@ -995,15 +995,41 @@ static std::string stream_text(int mfma_kind, bool conv, IgemmArgs g, bool init,
   return ", streamed rows past " + (rows && kn ? packed + " or as it lies" : rows ? packed : std::string("B as it lies")) + " mfma=" + mfma16_name(mfma_kind);
 }
 
+// Microseconds of a product in the tiles that a panel may stand in for, from the same timings as panel_us (990 products, 10 to 13 %
+// rms): so many tiles run together on a CU, a tile takes a slab's time for every 128 bytes of K and its results' time; `value_bytes`
+// go to and from memory per result.  Tiles of other kinds: infinity.
+static double tiled_us(int kind, int tile, int64_t m, int64_t n, int64_t k_bytes, int value_bytes, int cus) {
+  struct Times { double launch, tile, slab, value, ceil; int held, edge; };
+  const Times bf16_w8 = {1.64, 1.79, 0.539, 0.898, 0.77, 1, 128}, bf16_s2 = {0, 2.96, 0.616, 0.845, 0.57, 2, 128}, bf16_k2 = {4.91, 2.82, 0.24, 0, 0.77, 2, 64};
+  const Times i8_w8 = {3.0, 3.65, 0.554, 0.194, 0.77, 1, 128}, i8_s2 = {0.41, 4.89, 0.634, 0.471, 0.57, 2, 128};
+  const bool i8 = kind == KIND_I8;
+  const Times* const t = tile == TILE_128x128_W8 ? (i8 ? &i8_w8 : &bf16_w8) : tile == TILE_128x128_W8_S2 ? (i8 ? &i8_s2 : &bf16_s2) :
+                         tile == TILE_64x64_W8_K2 && !i8 ? &bf16_k2 : nullptr;
+  if (!t) return std::numeric_limits<double>::infinity();
+  const double per_cu = (double)((m + t->edge - 1) / t->edge) * (double)((n + t->edge - 1) / t->edge) / cus, turns = per_cu / t->held;
+  const double together = std::min((double)t->held, std::max(1.0, std::ceil(per_cu)));
+  const double rounds = turns <= 1 ? 1 : t->ceil * std::ceil(turns) + (1 - t->ceil) * turns;
+  return t->launch + rounds * (t->tile + (double)((k_bytes + 127) / 128) * t->slab * std::pow(together, 0.9) + t->value * value_bytes * together);
+}
+
 // Whether, and as what, a product whose right-hand sides are packed runs in panels (panel.hip).  bf16, where no tile is named, no
-// direct tile is cheaper, K is not split over workgroups and the rows do not stream (K up to 256).  Of 800 products (ranges at
-// panel_us) those of 256 x 256, 256 x 128 and 192 x 384 tiles gain 1.21 to 1.25 x on average, of 128 x 128 tiles 1.13 (three
-// stages) and 1.30 (two), of 64 x 64 tiles that share K 1.08; plain 64 x 64 tiles, which several share a CU, lose as often
-// as they gain (0.98), and 128 x 128 tiles over up to 160 columns, most of a 256 columns wide panel, lose (0.86 to 0.97).
+// direct tile is cheaper, K is not split over workgroups and the rows do not stream (512 bytes of K).  Of 1000 products (ranges at
+// panel_us) those of 256 x 256, 256 x 128 and 192 x 384 tiles gain 1.21 to 1.25 x on average and none loses; of 128 x 128 tiles
+// those priced 5 % below the tile gain 1.16 (three stages) and 1.32 (two), 1 in 200 loses more than 3 %; of 64 x 64 tiles that share
+// K those priced 10 % below gain 1.12, the others 1.03.  Plain 64 x 64 tiles, several of which share a CU, lose as often as they
+// gain (0.98), and 128 x 128 tiles over up to 160 columns, most of a 256 columns wide panel, lose (0.86 to 0.97).
+// int8, of 650 products: requantised from wide tiles 1.18 to 1.38 x, also over few columns (1.19), from 64 x 64 tiles 0.90 to 1.02;
+// with int32 results, four bytes of which leave for one of A, 1.23 x from 128 x 128 tiles of two stages with 1 KB of K and up to 1024
+// columns, and about as often less as more elsewhere (0.71 to 1.29).
 static int panel_of(const pml_hip_gemm_desc& d, int kind, int tile, const DirectTiles& direct, const void* ws) {
-  if (kind != KIND_BF16 || d.b_layout || PML_HIP_FLAG_TILE_OF(d.flags) >= 0 || direct.rows >= 0 || ws || d.k + d.k2 <= 256) return -1;
+  const int64_t k_bytes = (d.k + d.k2) * dt_size(d.in_dtype);
+  if ((kind != KIND_BF16 && kind != KIND_I8) || d.b_layout || PML_HIP_FLAG_TILE_OF(d.flags) >= 0 || direct.rows >= 0 || ws || k_bytes <= 512) return -1;
   const bool wide = tile == TILE_128x128_W8 || tile == TILE_128x128_W8_S2 || tile == TILE_256x128_W16 || tile == TILE_256x256_W8 || tile == TILE_192x384_W8;
-  if (!(wide && d.n > 160) && tile != TILE_64x64_W8_K2) return -1;
+  if (kind == KIND_I8) {
+    if (!wide || (d.c_dtype == PML_HIP_I32 && !(tile == TILE_128x128_W8_S2 && k_bytes >= 1024 && d.n <= 1024))) return -1;
+  } else if (!(wide && d.n > 160) && tile != TILE_64x64_W8_K2) {
+    return -1;
+  }
   IgemmArgs g;
   gemm_args(d, g);
   g.Bt = g.A = g.C = (void*)256;  // (stand for operands that are there; nothing is read)
@@ -1012,7 +1038,10 @@ static int panel_of(const pml_hip_gemm_desc& d, int kind, int tile, const Direct
   g.ldbt = d.k;
   if (stream_takes(tile, false, g)) return -1;
   double us;
-  return panel_config(g, d.init_kind != 0, &us);
+  const int config = panel_config(kind, g, d.init_kind != 0, &us);
+  const int value_bytes = dt_size(d.c_dtype) * (g.tail_mode == 2 ? 2 : 1);
+  const double share = kind == KIND_BF16 && tile != TILE_64x64_W8_K2 ? 0.95 : 0.9;
+  return us < share * tiled_us(kind, tile, d.m, d.n, k_bytes, value_bytes, g.n_cus) ? config : -1;
 }
 
 int64_t pml_hip_gemm_dispatch(const pml_hip_gemm_desc* d) {
@@ -1043,6 +1072,13 @@ int64_t pml_hip_gemm_dispatch(const pml_hip_gemm_desc* d) {
   p->b_split = kind == KIND_F32X3 && !d->b_layout && d->k % 32 == 0 && !p->ws;
   p->b_kn = kind == KIND_BF16 && p->direct.rows < 0 && takes_b_as_given(*d, kind, p->tile, d->n);
   p->panel = panel_of(*d, kind, p->tile, p->direct, p->ws);
+  if (p->panel >= 0) {
+    IgemmArgs g;
+    gemm_args(*d, g);
+    const int frags = panel_frags(kind, g);
+    // (no memory for it: the product runs in tiles)
+    if (!(p->panel_bt = p->hold(winconv_pack_bytes(es, 1, d->k, d->n, frags) + winconv_pack_bytes(es, 1, d->k2, d->n, frags)))) p->panel = -1;
+  }
   if (!d->b_layout && !(p->bt = p->hold(p->bt_bytes))) {
     delete p;
     fail("gemm: cannot allocate the packed right-hand side");
@@ -1120,6 +1156,20 @@ static bool reads_b_as_given(const pml_hip_gemm_desc& d, int mfma_kind, const vo
   return true;
 }
 
+// The right-hand side (second: of the second product) in the order a panel multiplies it, besides the form that tiles read.
+static int pack_panel(Plan* p, const void* b, bool second, hipStream_t s) {
+  if (p->panel < 0) return 0;
+  const pml_hip_gemm_desc& d = p->gemm;
+  IgemmArgs g;
+  gemm_args(d, g);
+  const int es = dt_size(d.in_dtype), frags = panel_frags(p->mfma_kind, g);
+  const size_t first = winconv_pack_bytes(es, 1, d.k, d.n, frags);
+  const WinFilter w = {1, (int)(second ? d.k2 : d.k), (int)d.n, 0, 0, second ? d.ldb2 : d.ldb, 1, frags};
+  if (check(winconv_pack_launch(es, b, w, (char*)p->panel_bt + (second ? first : 0), s), "winconv_pack_launch")) return 1;
+  p->panel_fresh[second] = true;
+  return 0;
+}
+
 static int gemm_run(const pml_hip_gemm_desc& d, int mfma_kind, int tile, const DirectTiles& direct, void* bt, int64_t bt_ld, bool packed,
                     const void* a, const void* b, void* c, const void* init, const void* const* operands,
                     void* const* outs, pml_hip_stream s, const SecondProduct* second = nullptr, Plan* plan = nullptr) {
@@ -1183,13 +1233,23 @@ static int gemm_run(const pml_hip_gemm_desc& d, int mfma_kind, int tile, const D
       return fail("gemm_invoke: missing extra output");
   // (the K split over workgroups is not built for a right-hand side packed split)
   if (plan && !b_split) split_args(plan, g);
+  // (a right-hand side that comes with the call is packed for a panel by a launch of its own as it would be transposed by one.
+  // Not where one was packed ahead: calls without any would multiply by that from then on, and tiles read `bt`.  An int8 one that
+  // a 256 x 256 tile reads as it lies pays for that launch from 50 G products on: requantised 4096 x 4096, K = 4096 71 us as it lies,
+  // 67.5 packed, 6000 x 3200, K = 3072 90 and 75, 4096 x 4096, K = 2048 38.6 and 40.6.)
+  const bool large_i8 = mfma_kind == KIND_I8 && b && b_as_given && (double)d.m * (double)d.n * (double)d.k >= 5e10;
+  if ((transposed || large_i8) && plan && plan->panel >= 0 && !packed && d.k2 == 0 && panel_runs(mfma_kind, g)) {
+    if (pack_panel(plan, b, false, (hipStream_t)s)) return 1;
+    plan->panel_fresh[0] = false;
+    return check(panel_launch(mfma_kind, plan->panel, g, plan->panel_bt, (hipStream_t)s), "panel_launch");
+  }
   // (rows that stream take a [K][N] right-hand side as it lies, too)
   if (transposed && !(!packed && streams_given(mfma_kind, tile, false, b, d.ldb, g))) {
     // (from here on `bt` holds the plain transposed form, whatever a packed copy was kept in before)
     if (plan) plan->bt_is_split = plan->bt_is_kn = plan->panel_fresh[0] = false;
     if (check(transpose_pack(es, b, bt, d.k, d.n, d.ldb, bt_ld, (hipStream_t)s), "transpose_pack")) return 1;
   }
-  if (plan && plan->panel_fresh[0] && (d.k2 == 0 || plan->panel_fresh[1]) && !b && (!second || !second->b2) && panel_runs(g)) return check(panel_launch(plan->panel, g, plan->panel_bt, (hipStream_t)s), "panel_launch");
+  if (plan && plan->panel_fresh[0] && (d.k2 == 0 || plan->panel_fresh[1]) && !b && (!second || !second->b2) && panel_runs(mfma_kind, g)) return check(panel_launch(mfma_kind, plan->panel, g, plan->panel_bt, (hipStream_t)s), "panel_launch");
   return check(igemm_launch(b_split ? KIND_F32X3P : mfma_kind, tile, false, g, (hipStream_t)s), "igemm_launch");
 }
 
@@ -1578,20 +1638,6 @@ int pml_hip_conv2d_invoke(int64_t plan, const void* input, const void* filter, v
     g.KW = 1;
   }
   return check(igemm_launch(p->b_split ? KIND_F32X3P : p->mfma_kind, tile, true, g, (hipStream_t)s), "igemm_launch");
-}
-
-// The right-hand side (second: of the second product) in the order a panel multiplies it, besides the form that tiles read.
-// (No memory for it: the product runs in tiles.)
-static int pack_panel(Plan* p, const void* b, bool second, hipStream_t s) {
-  if (p->panel < 0) return 0;
-  const pml_hip_gemm_desc& d = p->gemm;
-  p->panel_fresh[second] = false;
-  const size_t first = winconv_pack_bytes(2, 1, d.k, d.n);
-  if (!p->panel_bt && !(p->panel_bt = p->hold(first + winconv_pack_bytes(2, 1, d.k2, d.n)))) return 0;
-  const WinFilter w = {1, (int)(second ? d.k2 : d.k), (int)d.n, 0, 0, second ? d.ldb2 : d.ldb, 1};
-  if (check(winconv_pack_launch(2, b, w, (char*)p->panel_bt + (second ? first : 0), s), "winconv_pack_launch")) return 1;
-  p->panel_fresh[second] = true;
-  return 0;
 }
 
 int pml_hip_gemm_pack_b(int64_t plan, const void* b, pml_hip_stream s) {

@@ -340,16 +340,16 @@ __global__ __launch_bounds__(64 * WM * WN * KS, NB >= 4 ? 2 : 4) void winconv_ke
 
 // A filter in the order the kernel multiplies it: per 32 columns, tap and 64 bytes of channels two fragments of 64 lanes x 16
 // bytes.  Row r of fragment b holds column 8 (r / 4) + 4 b + r % 4, so that a lane ends with eight neighbouring columns of its
-// pixel; channels and columns past the last one are zeros.  (In the form [N][K] the sixteen rows of a fragment are whole
+// pixel (of one fragment: four, of four fragments to 64 columns: sixteen); channels and columns past the last one are zeros.  (In the form [N][K] the sixteen rows of a fragment are whole
 // lines apart and fall into the same banks of L1: 128 x 14 x 14 x 256 (*) 3 x 3 x 256 42.1 us, 32.0 with whole fragments.)
 template <typename T>
 __global__ __launch_bounds__(256) void winconv_pack_kernel(const T* f, i32x4_t* out, WinFilter w, int blocks, int chunks) {
   constexpr int kValues = 16 / (int)sizeof(T);
   const int c = blockIdx.x * 256 + threadIdx.x;
   if (c >= chunks) return;
-  const int lane = c & 63, b = (c >> 6) & 1, step = c >> 7, r = lane & 15;
+  const int lane = c & 63, b = (c >> 6) % w.frags, step = (c >> 6) / w.frags, r = lane & 15;
   const int blk = step % blocks, tap = step / blocks % w.taps, group = step / (blocks * w.taps);
-  const int n = 32 * group + 8 * (r >> 2) + 4 * b + (r & 3), k = (blk * 4 + (lane >> 4)) * kValues;
+  const int n = w.frags * (16 * group + 4 * (r >> 2)) + 4 * b + (r & 3), k = (blk * 4 + (lane >> 4)) * kValues;
   const T* const from = f + w.first + (int64_t)tap * w.tap_stride + (int64_t)n * w.n_stride;
   T v[kValues];
 #pragma unroll
@@ -357,6 +357,54 @@ __global__ __launch_bounds__(256) void winconv_pack_kernel(const T* f, i32x4_t* 
   i32x4_t bits;
   __builtin_memcpy(&bits, v, 16);
   out[c] = bits;
+}
+
+// The same where columns lie side by side, through LDS: 64 bytes of K by 128 columns a workgroup, read row by row.
+constexpr int kPackCols = 128;
+template <typename T>
+__global__ __launch_bounds__(256) void winconv_pack_rows_kernel(const T* f, i32x4_t* out, WinFilter w, int blocks) {
+  constexpr int kValues = 16 / (int)sizeof(T), kDeep = kBlockBytes / (int)sizeof(T), kPitch = kPackCols + 4 / (int)sizeof(T);
+  __shared__ __attribute__((aligned(16))) T tile[kDeep][kPitch];
+  const int n0 = blockIdx.x * kPackCols, blk = blockIdx.y % blocks, tap = blockIdx.y / blocks, k0 = blk * kDeep;
+  const T* const from = f + w.first + (int64_t)tap * w.tap_stride;
+  constexpr int kRow = kPackCols / kValues, kEach = kDeep * kRow / 256;  // 16-byte pieces of a row; of a thread
+  i32x4_t v[kEach];
+#pragma unroll
+  for (int i = 0; i < kEach; ++i) {  // (wherever the piece begins)
+    const int c = threadIdx.x + 256 * i, k = c / kRow, n = n0 + c % kRow * kValues;
+    const T* const at = from + (int64_t)(k0 + k) * w.k_stride + n;
+    v[i] = i32x4_t{0, 0, 0, 0};
+    if (k0 + k >= w.k || n >= w.n) continue;
+    if (n + kValues <= w.n) {
+      __builtin_memcpy(&v[i], at, 16);
+    } else {
+      T e[kValues] = {};
+#pragma unroll
+      for (int j = 0; j < kValues - 1; ++j)
+        if (n + j < w.n) e[j] = at[j];
+      __builtin_memcpy(&v[i], e, 16);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < kEach; ++i) {
+    const int c = threadIdx.x + 256 * i;
+    int* const to = (int*)&tile[c / kRow][c % kRow * kValues];  // (rows are whole words apart)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) to[j] = v[i][j];
+  }
+  __syncthreads();
+  const int group_cols = 16 * w.frags, groups = (w.n + group_cols - 1) / group_cols;
+  for (int c = threadIdx.x; c < kPackCols / 16 * 64; c += 256) {
+    const int lane = c & 63, r = lane & 15, b = (c >> 6) % w.frags, here = (c >> 6) / w.frags, group = n0 / group_cols + here;
+    if (group >= groups) continue;
+    const int n = group_cols * here + 4 * w.frags * (r >> 2) + 4 * b + (r & 3), k = (lane >> 4) * kValues;
+    T v[kValues];
+#pragma unroll
+    for (int e = 0; e < kValues; ++e) v[e] = tile[k + e][n];
+    i32x4_t bits;
+    __builtin_memcpy(&bits, v, 16);
+    out[((((int64_t)group * w.taps + tap) * blocks + blk) * w.frags + b) * 64 + lane] = bits;
+  }
 }
 
 struct WinConfig {
@@ -512,15 +560,24 @@ std::string winconv_text(const WinShape& shape) {
   return s + ")";
 }
 
-size_t winconv_pack_bytes(int es, int taps, int64_t k, int64_t n) {
-  return (size_t)((n + 31) / 32) * taps * ((k * es + kBlockBytes - 1) / kBlockBytes) * 2048;
+size_t winconv_pack_bytes(int es, int taps, int64_t k, int64_t n, int frags) {
+  return (size_t)((n + 16 * frags - 1) / (16 * frags)) * taps * ((k * es + kBlockBytes - 1) / kBlockBytes) * frags * 1024;
 }
 
 hipError_t winconv_pack_launch(int es, const void* filter, const WinFilter& w, void* out, hipStream_t s) {
   const int blocks = (w.k * es + kBlockBytes - 1) / kBlockBytes;
-  const int64_t chunks = (int64_t)winconv_pack_bytes(es, w.taps, w.k, w.n) / 16;
+  const int64_t chunks = (int64_t)winconv_pack_bytes(es, w.taps, w.k, w.n, w.frags) / 16;
   const dim3 grid((unsigned)((chunks + 255) / 256)), block(256);
   i32x4_t* const to = (i32x4_t*)out;
+  if (w.n_stride == 1 && (int64_t)w.taps * blocks < 65536) {
+    const dim3 tiles((unsigned)((w.n + kPackCols - 1) / kPackCols), (unsigned)(w.taps * blocks));
+    switch (es) {
+      case 1: hipLaunchKernelGGL(winconv_pack_rows_kernel<uint8_t>, tiles, block, 0, s, (const uint8_t*)filter, to, w, blocks); break;
+      case 2: hipLaunchKernelGGL(winconv_pack_rows_kernel<uint16_t>, tiles, block, 0, s, (const uint16_t*)filter, to, w, blocks); break;
+      default: hipLaunchKernelGGL(winconv_pack_rows_kernel<uint32_t>, tiles, block, 0, s, (const uint32_t*)filter, to, w, blocks); break;
+    }
+    return hipGetLastError();
+  }
   switch (es) {
     case 1: hipLaunchKernelGGL(winconv_pack_kernel<uint8_t>, grid, block, 0, s, (const uint8_t*)filter, to, w, blocks, (int)chunks); break;
     case 2: hipLaunchKernelGGL(winconv_pack_kernel<uint16_t>, grid, block, 0, s, (const uint16_t*)filter, to, w, blocks, (int)chunks); break;

@@ -42,7 +42,7 @@ SHAPES = [(21353, 650, 304, '96x768'), (8424, 1805, 312, '192x384'), (7483, 1728
           (21950, 174, 592, '112x256'), (4424, 1050, 544, '64x512'), (3001, 705, 520, '64x256'), (4095, 1023, 1032, '64x256')]
 
 
-def run(m, n, k, tile, k2=0, mode='plain', gap=0, lda_gap=0, relu=True, stride=0, image=None, offset=0):
+def run(m, n, k, tile, k2=0, mode='plain', gap=0, lda_gap=0, relu=True, stride=0, image=None, offset=0, packed=True):
     hk.init(0)
     L, none = hk.lib(), hk.ptr_array([])
     rng = np.random.default_rng(m + n + k + k2)
@@ -65,7 +65,8 @@ def run(m, n, k, tile, k2=0, mode='plain', gap=0, lda_gap=0, relu=True, stride=0
     db, db2 = (hk.DeviceBuffer.from_numpy(np.concatenate([pad, T.bf16(x)])) for x in (b, b2))
     dC = hk.DeviceBuffer.from_numpy(np.full(offset // 2 + (m + 1) * (n + gap), 77, np.uint16))
     at = lambda buf: ctypes.c_void_p(int(getattr(buf.ptr, 'value', buf.ptr)) + offset)
-    hk.check(L.pml_hip_gemm_pack_b(p, dB.ptr, None))
+    if packed:
+        hk.check(L.pml_hip_gemm_pack_b(p, dB.ptr, None))
     if k2:
         hk.check(L.pml_hip_gemm_pack_b2(p, dB2.ptr, None))
     ops = {'plain': none, 'residual': hk.ptr_array([dR.ptr]), 'scale': hk.ptr_array([dS.ptr, dZ.ptr])}[mode]
@@ -74,7 +75,7 @@ def run(m, n, k, tile, k2=0, mode='plain', gap=0, lda_gap=0, relu=True, stride=0
         if k2:
             hk.check(L.pml_hip_gemm_invoke2(p, dA.ptr, None, at(dC), init, dA2.ptr, None, at(db2), ops, none, None))
         else:
-            hk.check(L.pml_hip_gemm_invoke(p, dA.ptr, None, at(dC), init, ops, none, None))
+            hk.check(L.pml_hip_gemm_invoke(p, dA.ptr, None if packed else dB.ptr, at(dC), init, ops, none, None))
     hk.check(L.pml_hip_stream_sync(None))
     L.pml_hip_plan_free(p)
     C = dC.to_numpy(np.uint16, (offset // 2 + (m + 1) * (n + gap),))[offset // 2:].reshape(m + 1, n + gap)
@@ -109,9 +110,65 @@ def test_a_second_product(m, n, k, tile):
     run(m // 56 * 56, n // 8 * 8, k1, '', k2=k - k1, mode='plain', stride=2, image=(13, 15, 7, 8))
 
 
+@pytest.mark.parametrize('m,n,k,tile', SHAPES)
+def test_right_hand_sides_that_come_with_the_call(m, n, k, tile):
+    run(m, n, k, tile, lda_gap=8, packed=False)
+    run(m, n // 8 * 8, k, '', mode='residual', packed=False)
+
+
 @pytest.mark.parametrize('n,gap,offset', [(1000, 0, 0), (1000, 0, 2), (1001, 0, 0), (1001, 7, 6), (993, 0, 16), (999, 1, 4)])
 def test_results_anywhere(n, gap, offset):
     run(4100, n, 776, '', gap=gap, offset=offset)
+
+
+@pytest.mark.parametrize('m,n,k,requantised', [(25089, 512, 1040, False), (9001, 1002, 1040, False), (8424, 1805, 656, True), (16280, 650, 1136, True), (20001, 142, 576, True),
+                                               (4093, 3000, 528, True), (11841, 704, 672, True), (19906, 767, 832, True)])
+@pytest.mark.parametrize('init,one_scale,offset,packed', [(False, False, 0, True), (True, True, 4, True), (True, False, 16, False)])
+def test_int8(m, n, k, requantised, init, one_scale, offset, packed):
+    """Sums that wrap past 32 bits among them; value for value."""
+    hk.init(0)
+    L, none = hk.lib(), hk.ptr_array([])
+    rng = np.random.default_rng(m + n + k)
+    A, B = (rng.integers(-128, 128, s).astype(np.int8) for s in ((m, k), (k, n)))
+    b = rng.integers(-2 ** 31, 2 ** 31, n).astype(np.int32) if not requantised else rng.integers(-9000, 9000, n).astype(np.int32)
+    S = rng.uniform(0.0001, 0.0006, 1 if one_scale else n).astype(np.float32)
+    g = hk.GemmDesc()
+    g.in_dtype, g.out_dtype, g.c_dtype = hk.I8, hk.I32, hk.I8 if requantised else hk.I32
+    g.m, g.n, g.k, g.lda, g.ldb, g.ldc = m, n, k, k + 16, n, n
+    if init:
+        g.init_kind, g.init_dtype, g.init_row_stride, g.init_col_stride = 1, hk.I32, 0, 1
+    if requantised:
+        g.tail = hk.make_tail(ops=[(hk.EPI_CAST, hk.F32, 0, 0, 0.0), (hk.EPI_MUL, hk.F32, hk.OPND_TENSOR, 0, 0.0), (hk.EPI_MAX_GT, hk.F32, hk.OPND_IMM, 0, -120.0),
+                                   (hk.EPI_MIN, hk.F32, hk.OPND_IMM, 0, 127.0), (hk.EPI_ROUND, hk.F32, 0, 0, 0.0), (hk.EPI_CAST, hk.I8, 0, 0, 0.0)],
+                              operands=[(hk.F32, 0, 0 if one_scale else 1)])
+    else:
+        g.tail = hk.make_tail(ops=[(hk.EPI_RELU, hk.I32, 0, 0, 0.0)])
+    p = L.pml_hip_gemm_dispatch(ctypes.byref(g))
+    assert p, L.pml_hip_last_error()
+    assert 'in panels' in hk.describe(p), hk.describe(p)
+    dA = hk.DeviceBuffer.from_numpy(np.concatenate([A, np.full((m, 16), 55, np.int8)], 1))
+    dB, dS = hk.DeviceBuffer.from_numpy(B), hk.DeviceBuffer.from_numpy(S)
+    db = hk.DeviceBuffer.from_numpy(np.concatenate([np.zeros(offset // 4, np.int32), b]))
+    out = np.int8 if requantised else np.int32
+    skip = offset // np.dtype(out).itemsize
+    dC = hk.DeviceBuffer.from_numpy(np.full(skip + (m + 1) * n, 77, out))
+    if packed:
+        hk.check(L.pml_hip_gemm_pack_b(p, dB.ptr, None))
+    at = lambda buf: ctypes.c_void_p(int(getattr(buf.ptr, 'value', buf.ptr)) + offset)
+    for _ in range(2):
+        hk.check(L.pml_hip_gemm_invoke(p, dA.ptr, None if packed else dB.ptr, at(dC), at(db) if init else None, hk.ptr_array([dS.ptr]) if requantised else none, none, None))
+    hk.check(L.pml_hip_stream_sync(None))
+    L.pml_hip_plan_free(p)
+    C = dC.to_numpy(out, (skip + (m + 1) * n,))[skip:].reshape(m + 1, n)
+    assert (C[m] == 77).all()
+    sums = (A.astype(np.float64) @ B.astype(np.float64)).astype(np.int64) + (b.astype(np.int64) if init else 0)
+    sums = sums.astype(np.uint64).astype(np.uint32).view(np.int32)
+    if requantised:
+        v = np.clip(sums.astype(np.float32) * S, np.float32(-120), np.float32(127))
+        want = np.trunc(v + np.copysign(np.float32(0.5), v)).astype(np.int8)
+    else:
+        want = np.maximum(sums, 0)
+    np.testing.assert_array_equal(C[:m], want)
 
 
 def test_operands_that_a_panel_does_not_read():
