@@ -187,15 +187,16 @@ double stepUs(const Step& s, int64_t count) { return std::max(6.0, 2.0 + std::ma
 constexpr double kLinkBytesPerUs = 56e3;
 // What a part costs besides: its copies', waits' and launches' places in three queues (18 to 25 us between two parts' kernels)
 constexpr double kPartUs = 20;
-// A part has at least so many bytes to carry (27 us on the link)
-constexpr int64_t kPartBytes = 3 << 19;
+// A part has at least so many bytes to carry, up or down (75 us on the link): every operand and result of every part is a copy of its
+// own.  (6 MB up and down around three launches in four parts: 465 us, 394 in one.)
+constexpr int64_t kPartBytes = 4 << 20;
 constexpr int kMostParts = 4;
 
 }  // namespace
 
 // What is bound by the link is cut where its kernels would wait for it: ResNet-50 on 128 images, 38 MB up ahead of the first launch,
 // 2713 us a run with the kernels behind the copies and 2593 with nine steps in four parts;
-// mean-variance normalisation of 4096x1000 fp32, 16 MB either way, 866 and 639.
+// mean-variance normalisation of 4096x1000 fp32, 16 MB either way, 866 and 639 to 686; of 2048x1024, 8 MB, 428 and 391.
 void Planner::sliceSteps() {
   Plan& p = *plan_;
   int64_t link_in = 0, link_out = 0, units = 0, largest = 0;
@@ -209,7 +210,7 @@ void Planner::sliceSteps() {
     }
   }
   for (int b : p.output_buffers) link_out += static_cast<int64_t>(p.buffers[b].bytes);
-  const int64_t slices = std::min<int64_t>({kMostParts, (link_in + link_out) / kPartBytes, units});
+  const int64_t slices = std::min<int64_t>({kMostParts, std::max(link_in, link_out) / kPartBytes, units});
   if (slices < 2) return;
   const int64_t part = (units + slices - 1) / slices, count = (units + part - 1) / part, last = units - (count - 1) * part;
   if (count < 2) return;

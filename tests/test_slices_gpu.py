@@ -74,6 +74,7 @@ def test_what_runs_in_parts():
         steps, n = parts(build(name, 'f32')[0])
         assert steps >= 1 and 2 <= n <= 4, name
     assert parts(dense('f32', 64)[0]) == (0, 1)  # (nothing to carry meanwhile)
+    assert parts(batches('f32', 150)[0]) == (0, 1) and parts(batches('f32', 220)[0])[1] == 2  # (parts of 4 MB and more)
     X, W = P.Placeholder(DT['f32'], [4096, 1024]), P.Placeholder(DT['f32'], [4096, 64])
     i, j, k = P.TensorIndexes(3)
     # rows of the result are columns of what comes in
