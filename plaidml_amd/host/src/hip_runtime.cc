@@ -594,12 +594,11 @@ class HipExecutable final : public Executable {
   }
 
   // One run, segment by segment: what a segment needs is staged and sent up, its launches wait for that, and what is final behind
-  // it goes down while the link carries the next one's needs up.  Inputs that take more than the slots go through them in turn.
-  // False (and nothing done) where the staging has no place for every other value, or there is none.  An output's place is that of an input which is up before the output exists, where there is one.
+  // it goes down while the link carries the next one's needs up.  Inputs that take more than the slots go through them in turn,
+  // and so do outputs behind the last launch.  False (and nothing done) where the staging has no place for the other values, or there is none.  An output's place is that of an input which is up before the output exists, where there is one.
   bool overlapped(const std::vector<HostSpan>& inputs, const std::vector<HostSpan>& outputs, double start, InvokeStats* st) {
     constexpr size_t kNowhere = ~size_t{0}, kInTurn = kNowhere - 1, kAll = kStageSlots * kStageRun;
-    std::vector<size_t> in_at(inputs.size(), kNowhere), out_at(outputs.size(), kNowhere), up_by(inputs.size(), 0), from(outputs.size(), 0);
-    std::vector<char> lent(inputs.size(), 0);
+    std::vector<size_t> in_at, out_at, up_by(inputs.size(), 0), from(outputs.size(), 0);
     size_t need = 0;
     auto bytes_of = [&](int buf) { return plan_->buffers[buf].bytes; };
     for (size_t k = 0; k < segments_.size(); ++k) {
@@ -610,31 +609,39 @@ class HipExecutable final : public Executable {
     size_t staged = 0;
     for (size_t i = 0; i < inputs.size(); ++i)
       if (!direct(plan_->input_buffers[i], inputs[i])) staged += padded(bytes_of(plan_->input_buffers[i]));
-    const bool in_turn = staged > kAll;
-    for (size_t i = 0; i < inputs.size(); ++i) {
-      const size_t bytes = bytes_of(plan_->input_buffers[i]);
-      if (direct(plan_->input_buffers[i], inputs[i])) continue;
-      in_at[i] = in_turn && bytes > kKernelCopy ? kInTurn : need;
-      if (in_at[i] != kInTurn) need += padded(bytes);
-    }
-    for (size_t o = 0; o < outputs.size(); ++o) {
-      const int buf = plan_->output_buffers[o];
-      if (direct(buf, outputs[o])) continue;
-      for (size_t i = 0; i < inputs.size() && out_at[o] == kNowhere; ++i) {
-        const int in = plan_->input_buffers[i];
-        if (in_at[i] >= kInTurn || lent[i] || bytes_of(in) < bytes_of(buf)) continue;
-        const bool parts = plan_->slices > 1 && plan_->part_bytes[in] > 0 && plan_->part_bytes[buf] > 0;
-        if (parts ? plan_->part_bytes[in] >= plan_->part_bytes[buf] : up_by[i] <= from[o]) {
-          out_at[o] = in_at[i];
-          lent[i] = 1;
+    // a place for every value, or the slots for the long ones: inputs in turn, and outputs that half as much has no place for, at the end
+    auto place_all = [&](bool in_turn) {
+      in_at.assign(inputs.size(), kNowhere);
+      out_at.assign(outputs.size(), kNowhere);
+      std::vector<char> lent(inputs.size(), 0);
+      need = 0;
+      for (size_t i = 0; i < inputs.size(); ++i) {
+        const size_t bytes = bytes_of(plan_->input_buffers[i]);
+        if (direct(plan_->input_buffers[i], inputs[i])) continue;
+        in_at[i] = in_turn && bytes > kKernelCopy ? kInTurn : need;
+        if (in_at[i] != kInTurn) need += padded(bytes);
+      }
+      for (size_t o = 0; o < outputs.size(); ++o) {
+        const int buf = plan_->output_buffers[o];
+        if (direct(buf, outputs[o])) continue;
+        for (size_t i = 0; i < inputs.size() && out_at[o] == kNowhere; ++i) {
+          const int in = plan_->input_buffers[i];
+          if (in_at[i] >= kInTurn || lent[i] || bytes_of(in) < bytes_of(buf)) continue;
+          const bool parts = plan_->slices > 1 && plan_->part_bytes[in] > 0 && plan_->part_bytes[buf] > 0;
+          if (parts ? plan_->part_bytes[in] >= plan_->part_bytes[buf] : up_by[i] <= from[o]) {
+            out_at[o] = in_at[i];
+            lent[i] = 1;
+          }
         }
+        if (out_at[o] != kNowhere) continue;
+        const size_t bytes = padded(bytes_of(buf));
+        out_at[o] = in_turn && bytes > kKernelCopy && need + bytes > kAll / 2 ? kInTurn : need;
+        if (out_at[o] != kInTurn) need += bytes;
       }
-      if (out_at[o] == kNowhere) {
-        out_at[o] = need;
-        need += padded(bytes_of(buf));
-      }
-    }
-    if (need > (in_turn ? kAll / 2 : kAll)) return false;
+      return need <= (in_turn ? kAll / 2 : kAll);
+    };
+    bool in_turn = staged > kAll;
+    if (!place_all(in_turn) && (in_turn || !place_all(in_turn = true))) return false;
     const size_t slots = need;
     if (in_turn) need += kAll;
     if (need > staging_bytes_) {
@@ -708,6 +715,7 @@ class HipExecutable final : public Executable {
         for (const Range& r : seg.yields) {
           const HostSpan& out = outputs[r.index];
           const char* const dev = static_cast<const char*>(device_[plan_->output_buffers[r.index]]) + r.offset;
+          if (out_at[r.index] == kInTurn) continue;
           char* const to = out_at[r.index] == kNowhere ? static_cast<char*>(out.data) + r.offset : out_place(r);
           if (r.bytes <= kKernelCopy)
             down.add(to, dev, r.bytes);
@@ -720,7 +728,7 @@ class HipExecutable final : public Executable {
       for (Segment& seg : segments_) {
         bool waited = false;
         for (const Range& r : seg.yields) {
-          if (out_at[r.index] == kNowhere) continue;
+          if (out_at[r.index] >= kInTurn) continue;
           if (!waited) hipCheck(pml_hip_event_sync(seg.down), "event sync");
           waited = true;
           const HostSpan& out = outputs[r.index];
@@ -731,6 +739,14 @@ class HipExecutable final : public Executable {
             hostCopy(to, out_place(r), r.bytes);
         }
       }
+      // (behind the launches, and so behind every copy out of the slots)
+      Staging late;
+      late.slots = base + slots;
+      std::vector<Piece> arriving;
+      Spans none;
+      for (size_t o = 0; o < outputs.size(); ++o)
+        if (out_at[o] == kInTurn) stageOut(&late, outputs[o], bytes_of(plan_->output_buffers[o]), static_cast<const char*>(device_[plan_->output_buffers[o]]), &arriving, &none);
+      if (!arriving.empty()) collect(&late, arriving);
       for (pml_hip_stream s : {up_stream_, stream_, down_stream_}) hipCheck(pml_hip_stream_sync(s), "stream sync");
     } catch (...) {
       sync();  // queued copies may still use the caller's memory

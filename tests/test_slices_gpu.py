@@ -119,13 +119,16 @@ def test_every_run(monkeypatch, dt, pinned_results, name):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize('dt', ['f32', 'bf16'])
-def test_more_than_the_staging_holds(dt):
-    """Operands past the staging's slots, of which every part takes several."""
+@pytest.mark.parametrize('pinned_results', [True, False])
+def test_more_than_the_staging_holds(monkeypatch, dt, pinned_results):
+    """Operands past the staging's slots, of which every part takes several, and results that come back through them."""
+    if not pinned_results:
+        monkeypatch.setattr(P, '_result_array', lambda d, sizes, nbytes: np.empty(sizes, d))
     m = {'f32': 18001, 'bf16': 36001}[dt]  # 46 MB
     program, draw, want = dense(dt, m)
     assert parts(program)[1] > 1
     runner = P.Runner(program, target='hip')
-    for run in range(4):
+    for run in range(5):
         arrays = draw(np.random.default_rng(run))
         got = runner.run(arrays)
         exact = want(*arrays)
