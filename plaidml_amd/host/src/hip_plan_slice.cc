@@ -180,9 +180,7 @@ class Slicer {
 };
 
 // Microseconds that a `count`-th of a step is taken to take: memory at 3.5 TB/s, matrix products at 500 TFLOP/s, and no less than a
-// launch with a few memory latencies in it.  (Kernels fill the chip less well with a part of their work: nine steps of ResNet-50
-// that take 610 us on 128 images take 764 in four parts.  The number of parts matters little for that: a run ends about as late
-// with two, 1030 us up to the same step, as with four, 1044: what the kernels lose to small parts the link loses to large ones.)
+// launch with a few memory latencies in it.
 double stepUs(const Step& s, int64_t count) { return std::max(6.0, 2.0 + std::max(s.bytes / 3.5e6, s.flops / 500e6) / static_cast<double>(count)); }
 constexpr double kLinkBytesPerUs = 56e3;
 // What a part costs besides: its copies', waits' and launches' places in three queues (18 to 25 us between two parts' kernels)
@@ -190,13 +188,16 @@ constexpr double kPartUs = 20;
 // A part has at least so many bytes to carry, up or down (75 us on the link): every operand and result of every part is a copy of its
 // own.  (6 MB up and down around three launches in four parts: 465 us, 394 in one.)
 constexpr int64_t kPartBytes = 4 << 20;
-constexpr int kMostParts = 4;
+// Kernels fill the chip less well with a part of their work: nine steps of ResNet-50 that take 610 us on 128 images take 764 in four
+// parts.  us a run with four, three and two parts: 128 images 2440, 2437, 2411, 96 images 2093, 2082, 2055, 64 images 1645, 1596,
+// 1582; mean-variance normalisation of 4096x1000 fp32 597, 601, 608.
+constexpr int kMostParts = 2;
 
 }  // namespace
 
 // What is bound by the link is cut where its kernels would wait for it: ResNet-50 on 128 images, 38 MB up ahead of the first launch,
-// 2713 us a run with the kernels behind the copies and 2593 with nine steps in four parts;
-// mean-variance normalisation of 4096x1000 fp32, 16 MB either way, 866 and 639 to 686; of 2048x1024, 8 MB, 428 and 391.
+// 2630 us a run with the kernels behind the copies, 2411 with its first steps in two parts; mean-variance normalisation of 4096x1000
+// fp32, 16 MB either way, 866 and 608 to 680; of 2048x1024, 8 MB, 428 and 391.
 void Planner::sliceSteps() {
   Plan& p = *plan_;
   int64_t link_in = 0, link_out = 0, units = 0, largest = 0;

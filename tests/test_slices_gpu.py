@@ -35,9 +35,8 @@ def images(dt, n, hw=64):
     draw = lambda rng: [whole(rng, n, hw, hw, 64), whole(rng, 1, 1, 64, 512, top=1)]
 
     def want(x, f):
-        t = np.maximum(x.reshape(-1, 64) @ f.reshape(64, 512), 0).reshape(n, hw // 2, 2, hw // 2, 2, 512).max((2, 4))
-        return [t, t.max(0)]
-    return P.Program('images', [X, F], [top, Pop.max(top, axes=[0])]), draw, want
+        return [np.maximum(x.reshape(-1, 64) @ f.reshape(64, 512), 0).reshape(n, hw // 2, 2, hw // 2, 2, 512).max((0, 2, 4))]
+    return P.Program('images', [X, F], [Pop.max(top, axes=[0])]), draw, want
 
 
 def rows(dt, m, c=520):
