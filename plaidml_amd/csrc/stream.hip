@@ -297,18 +297,19 @@ bool ragged(const IgemmArgs& g) {
 // a CU.  How many it takes shrinks with what a row costs a tile: a residual to fetch, odd rows of results that take its
 // row-by-row tail.  Past K = 128 rows that are whole lines apart come in slower than others (banks of L1, above).  A [K][N]
 // right-hand side costs a tile a transposed copy: wherever no direct tile is taken (the caller's choice, before this one), its
-// rows stream.  Microseconds tile -> stream, in brackets what keeps its tile, back to back in a recorded graph over buffers in
-// turn; the lines lie where 820 products of 48 to 2000 columns and 300 to 25000 steps cross over:
+// rows stream.  Microseconds tile -> stream, back to back in a recorded graph over buffers in turn; in brackets what keeps its tile,
+// as it streamed when the lines were drawn where 820 products of 48 to 2000 columns and 300 to 25000 steps crossed over, results
+// and residual then in 64-byte pieces:
 //   steps a wavefront (256 CUs: 2048)
-//   3/2    K = 32     25088 x 256   8.9 ->  7.1    25088 x 1024  24.3 -> 18.7    401408 x 64  34.3 -> 22.1    401408 x 256   80 ->  66
-//   17/4   K = 64     25088 x 256   9.0 ( 9.8)     25088 x 1024  24.4 -> 23.6    401408 x 64  33.8 -> 26.0    401408 x 256   84 ->  75 (residual 126 ->  94)
-//          K = 128    25088 x 512  15.5 (16.6)     25088 x 1024  30.0 -> 29.3    100352 x 64  12.1 (12.5)     100352 x 512   52 ->  46 (residual  75 ->  57)
-//   13/4   K = 200    25088 x 256  12.3 (12.5)     25088 x 1024  36.3 -> 29.0                                 401408 x 256  152 ->  96 (residual 193 -> 133)
-//   3        up to 64 columns, odd rows, residual                                100352 x 64  21.6 -> 16.8    25088 x 256                (residual 15.8 -> 13.4)
-//   39/4   K = 256    12544 x 1024 17.9 (19.5)     25088 x 1024  36.6 -> 32.8    401408 x 64  66.5 -> 53.7    100352 x 512   67 ->  60 (residual  88 ->  75)
-//   17/4     odd rows, residual                    35000 x 250   20.1 -> 18.5                                 25088 x 512                (residual 26.7 -> 26.5)
-//   any    [K][N] as it lies, K = 64: 19200 x 128 8.1 -> 6.3, 25088 x 128 8.2 -> 6.6, 25088 x 256 11.1 -> 8.4, 25088 x 251 15.7 -> 13.3, 401408 x 123 70 -> 62
-//                             K = 128: 8000 x 200 7.5 -> 6.2, 25088 x 128 9.5 -> 8.0, 25088 x 256 12.1 -> 10.4, 25088 x 251 16.7 -> 13.3, 100352 x 510 68.3 -> 68.6
+//   3/2    K = 32     25088 x 256   8.9 ->  6.6    25088 x 1024  24.3 -> 13.9    401408 x 64  34.3 -> 16.1    401408 x 256   80 ->  47
+//   17/4   K = 64     25088 x 256   9.0 ( 9.8)     25088 x 1024  24.4 -> 17.5    401408 x 64  33.8 -> 22.7    401408 x 256   84 ->  54 (residual 126 ->  91)
+//          K = 128    25088 x 512  15.5 (16.6)     25088 x 1024  30.0 -> 24.6    100352 x 64  12.1 (12.5)     100352 x 512   52 ->  36 (residual  75 ->  51)
+//   13/4   K = 200    25088 x 256  12.3 (12.5)     25088 x 1024  36.3 -> 29.3                                 401408 x 256  152 ->  82 (residual 193 -> 121)
+//   3        up to 64 columns, odd rows, residual                                100352 x 64  21.6 -> 14.0    25088 x 256                (residual 15.8 -> 12.8)
+//   39/4   K = 256    12544 x 1024 17.9 (19.5)     25088 x 1024  36.6 -> 32.0    401408 x 64  66.5 -> 54.3    100352 x 512   67 ->  50 (residual  88 ->  64)
+//   17/4     odd rows, residual                    35000 x 250   20.1 -> 18.0                                 25088 x 512                (residual 26.7 -> 23.8)
+//   any    [K][N] as it lies, K = 64: 19200 x 128 8.1 -> 6.3, 25088 x 128 8.2 -> 6.5, 25088 x 256 11.1 -> 7.9, 25088 x 251 15.7 -> 11.6, 401408 x 123 70 -> 45
+//                             K = 128: 8000 x 200 7.5 -> 6.2, 25088 x 128 9.5 -> 7.9, 25088 x 256 12.1 -> 9.9, 25088 x 251 16.7 -> 12.0, 100352 x 510 68.3 -> 62.2
 bool stream_takes(int cfg, bool conv, const IgemmArgs& g) {
   if (!g.stream || cfg == TILE_16x16_W8 || cfg == TILE_32x32_W8 || (cfg == TILE_64x64_KSPLIT && g.ws)) return false;
   if (conv && (g.KH != 1 || g.KW != 1 || g.SH != 1 || g.SW != 1 || g.PH != 0 || g.PW != 0 || g.OH != g.H || g.OW != g.W || g.pix_pitch != 0 ||

@@ -340,8 +340,9 @@ __global__ __launch_bounds__(64 * WM * WN * KS, NB >= 4 ? 2 : 4) void winconv_ke
 
 // A filter in the order the kernel multiplies it: per 32 columns, tap and 64 bytes of channels two fragments of 64 lanes x 16
 // bytes.  Row r of fragment b holds column 8 (r / 4) + 4 b + r % 4, so that a lane ends with eight neighbouring columns of its
-// pixel (of one fragment: four, of four fragments to 64 columns: sixteen); channels and columns past the last one are zeros.  (In the form [N][K] the sixteen rows of a fragment are whole
-// lines apart and fall into the same banks of L1: 128 x 14 x 14 x 256 (*) 3 x 3 x 256 42.1 us, 32.0 with whole fragments.)
+// pixel (one fragment to 16 columns: four; four to 64: sixteen); channels and columns past the last one are zeros.  (In the form
+// [N][K] the sixteen rows of a fragment are whole lines apart and fall into the same banks of L1: 128 x 14 x 14 x 256 (*) 3 x 3 x
+// 256 42.1 us, 32.0 with whole fragments.)  This form for columns that are not side by side (the channels of a data gradient).
 template <typename T>
 __global__ __launch_bounds__(256) void winconv_pack_kernel(const T* f, i32x4_t* out, WinFilter w, int blocks, int chunks) {
   constexpr int kValues = 16 / (int)sizeof(T);
