@@ -1044,6 +1044,14 @@ static int panel_of(const pml_hip_gemm_desc& d, int kind, int tile, const Direct
   return us < share * tiled_us(kind, tile, d.m, d.n, k_bytes, value_bytes, g.n_cus) ? config : -1;
 }
 
+static size_t panel_bytes(const Plan* p) {
+  const pml_hip_gemm_desc& d = p->gemm;
+  IgemmArgs g;
+  gemm_args(d, g);
+  const int es = dt_size(d.in_dtype), frags = panel_frags(p->mfma_kind, g);
+  return winconv_pack_bytes(es, 1, d.k, d.n, frags) + winconv_pack_bytes(es, 1, d.k2, d.n, frags);
+}
+
 int64_t pml_hip_gemm_dispatch(const pml_hip_gemm_desc* d) {
   const int kind = gemm_desc_kind(d);
   if (kind < 0) return 0;
@@ -1071,14 +1079,6 @@ int64_t pml_hip_gemm_dispatch(const pml_hip_gemm_desc* d) {
   if (p->tile == TILE_64x64_KSPLIT && !p->ws) p->tile = TILE_64x64;  // (not worth splitting, no memory for the workspace, or not run)
   p->b_split = kind == KIND_F32X3 && !d->b_layout && d->k % 32 == 0 && !p->ws;
   p->b_kn = kind == KIND_BF16 && p->direct.rows < 0 && takes_b_as_given(*d, kind, p->tile, d->n);
-  p->panel = panel_of(*d, kind, p->tile, p->direct, p->ws);
-  if (p->panel >= 0) {
-    IgemmArgs g;
-    gemm_args(*d, g);
-    const int frags = panel_frags(kind, g);
-    // (no memory for it: the product runs in tiles)
-    if (!(p->panel_bt = p->hold(winconv_pack_bytes(es, 1, d->k, d->n, frags) + winconv_pack_bytes(es, 1, d->k2, d->n, frags)))) p->panel = -1;
-  }
   if (!d->b_layout && !(p->bt = p->hold(p->bt_bytes))) {
     delete p;
     fail("gemm: cannot allocate the packed right-hand side");
@@ -1089,6 +1089,9 @@ int64_t pml_hip_gemm_dispatch(const pml_hip_gemm_desc* d) {
     fail("gemm: cannot allocate the second packed right-hand side");
     return 0;
   }
+  p->panel = panel_of(*d, kind, p->tile, p->direct, p->ws);
+  // (a right-hand side that comes with the call and is read as it lies needs no room; no memory for it: the product runs in tiles)
+  if (p->panel >= 0 && (kind == KIND_I8 || !takes_b_as_given(*d, kind, p->tile, d->ldb)) && !(p->panel_bt = p->hold(panel_bytes(p)))) p->panel = -1;
   char buf[256];
   std::snprintf(buf, sizeof buf, "gemm %s m=%lld n=%lld k=%lld tile=%s mfma=%s", d->in_dtype == PML_HIP_F32 ? "f32" : d->in_dtype == PML_HIP_BF16 ? "bf16" : "i8",
                 (long long)d->m, (long long)d->n, (long long)d->k, tile_name(p->direct.rows >= 0 ? lds_tile : p->tile),
@@ -1160,6 +1163,7 @@ static bool reads_b_as_given(const pml_hip_gemm_desc& d, int mfma_kind, const vo
 static int pack_panel(Plan* p, const void* b, bool second, hipStream_t s) {
   if (p->panel < 0) return 0;
   const pml_hip_gemm_desc& d = p->gemm;
+  if (!p->panel_bt && !(p->panel_bt = p->hold(panel_bytes(p)))) return 0;
   IgemmArgs g;
   gemm_args(d, g);
   const int es = dt_size(d.in_dtype), frags = panel_frags(p->mfma_kind, g);
@@ -1238,7 +1242,7 @@ static int gemm_run(const pml_hip_gemm_desc& d, int mfma_kind, int tile, const D
   // a 256 x 256 tile reads as it lies pays for that launch from 50 G products on: requantised 4096 x 4096, K = 4096 71 us as it lies,
   // 67.5 packed, 6000 x 3200, K = 3072 90 and 75, 4096 x 4096, K = 2048 38.6 and 40.6.)
   const bool large_i8 = mfma_kind == KIND_I8 && b && b_as_given && (double)d.m * (double)d.n * (double)d.k >= 5e10;
-  if ((transposed || large_i8) && plan && plan->panel >= 0 && !packed && d.k2 == 0 && panel_runs(mfma_kind, g)) {
+  if ((transposed || large_i8) && plan && plan->panel_bt && !packed && d.k2 == 0 && panel_runs(mfma_kind, g)) {
     if (pack_panel(plan, b, false, (hipStream_t)s)) return 1;
     plan->panel_fresh[0] = false;
     return check(panel_launch(mfma_kind, plan->panel, g, plan->panel_bt, (hipStream_t)s), "panel_launch");
