@@ -128,7 +128,7 @@ class HipExecutable final : public Executable {
       if (outputs[i].bytes < spanBytes(plan_->output_buffers[i], outputs[i])) throw std::runtime_error("output buffer #" + std::to_string(i) + " is too small");
     for (size_t i = 0; i < inputs.size(); ++i)
       if (inputs[i].bytes < spanBytes(plan_->input_buffers[i], inputs[i])) throw std::runtime_error("input buffer #" + std::to_string(i) + " is too small");
-    if (segments_.size() > 1 && !profile && overlapped(inputs, outputs, start, &st)) {
+    if (segments_.size() > 1 && !profile && !shared(inputs, outputs) && overlapped(inputs, outputs, start, &st)) {
       g_stats = st;
       return st.wall_ms;
     }
@@ -271,6 +271,23 @@ class HipExecutable final : public Executable {
         hipCheck(pml_hip_copy_spans_stamped(static_cast<int>(dst.size()), dst.data(), src.data(), bytes.data(), stamp, after ? 1 : 0, stream), "copy");
     }
   };
+
+  // Whether a result lies in the memory of an operand, or of another result.  On one stream everything is up before anything goes
+  // down, and results arrive in their order; between queues of their own a result would reach an operand that is still to go up.
+  bool shared(const std::vector<HostSpan>& inputs, const std::vector<HostSpan>& outputs) const {
+    auto meet = [](const HostSpan& a, size_t a_bytes, const HostSpan& b, size_t b_bytes) {
+      const uintptr_t p = reinterpret_cast<uintptr_t>(a.data), q = reinterpret_cast<uintptr_t>(b.data);
+      return p < q + b_bytes && q < p + a_bytes;
+    };
+    for (size_t o = 0; o < outputs.size(); ++o) {
+      const size_t bytes = spanBytes(plan_->output_buffers[o], outputs[o]);
+      for (size_t i = 0; i < inputs.size(); ++i)
+        if (meet(outputs[o], bytes, inputs[i], spanBytes(plan_->input_buffers[i], inputs[i]))) return true;
+      for (size_t q = 0; q < o; ++q)
+        if (meet(outputs[o], bytes, outputs[q], spanBytes(plan_->output_buffers[q], outputs[q]))) return true;
+    }
+    return false;
+  }
 
   // bytes the caller's side of a value takes
   size_t spanBytes(int buf, const HostSpan& h) const { return plan_->buffers[buf].bytes * (h.f32 ? 2 : 1); }

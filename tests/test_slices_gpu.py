@@ -135,3 +135,34 @@ def test_more_than_the_staging_holds(monkeypatch, dt, pinned_results):
             exact = [P.round_bf16(exact[0]), P.round_bf16(P.round_bf16(exact[0]) @ arrays[3])]
         for g, w in zip(got, exact):
             np.testing.assert_array_equal(g, w)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('dt', ['f32', 'bf16'])
+def test_results_over_operands(dt):
+    """A result in the memory of an operand that a later launch, or a later part of the same one, is the first to need."""
+    m = 2048 if dt == 'f32' else 4096
+    bits = (lambda a: a) if dt == 'f32' else P.to_bf16_bits
+    value = (lambda a: a) if dt == 'f32' else P.from_bf16_bits
+    rounded = (lambda a: a) if dt == 'f32' else P.round_bf16
+    i, j, k = P.TensorIndexes(3)
+    A, W, B, V = (P.Placeholder(DT[dt], s) for s in ([m, 1024], [1024, 1024], [m, 1024], [m, 64]))
+    second = P.Contraction().outShape(1024, 64).outAccess(i, j).sum(B[k, i] * V[k, j]).build()
+    two = P.Runner(P.Program('two', [A, W, B, V], [Pop.dot(A, W), second]), target='hip')
+    X, U = P.Placeholder(DT[dt], [m, 512]), P.Placeholder(DT[dt], [512, 1024])
+    program = P.Program('longer', [X, U], [Pop.relu(Pop.dot(X, U))])
+    assert parts(program)[1] == 2  # (rows of the result reach further than those of the operand)
+    longer = P.Runner(program, target='hip')
+    for run in range(6):
+        rng = np.random.default_rng(run)
+        a, w, b, v = whole(rng, m, 1024), whole(rng, 1024, 1024, top=1), whole(rng, m, 1024), whole(rng, m, 64, top=1)
+        staged = two.stage([a, w, b, v])
+        two.exe.run(staged, [staged[2], two.outputs[1]])
+        np.testing.assert_array_equal(value(staged[2].as_ndarray()), rounded(a @ w), err_msg='run %d' % run)
+        np.testing.assert_array_equal(value(two.outputs[1].as_ndarray()), rounded(b.T @ v), err_msg='run %d' % run)
+        x, u = whole(rng, m, 512), whole(rng, 512, 1024, top=1)
+        memory = P._result_array(np.dtype(np.float32 if dt == 'f32' else np.uint16), (m, 1024), m * 1024 * (4 if dt == 'f32' else 2))
+        operand, result = P.Buffer(longer.in_shapes[0], data=memory[:m // 2].reshape(m, 512)), P.Buffer(longer.out_shapes[0], data=memory)
+        operand.copy_from_ndarray(bits(x))
+        longer.exe.run([operand, longer.stage([x, u])[1]], [result])
+        np.testing.assert_array_equal(value(memory), rounded(np.maximum(x @ u, 0)), err_msg='run %d' % run)
