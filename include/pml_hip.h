@@ -355,7 +355,8 @@ int pml_hip_tile_of_workgroup(int tiles_m, int tiles_n, int workgroup, int* tile
  * hipMalloc).  The transposed copy of a [K][N] right-hand side (b_layout 0), which a plan keeps in memory of its
  * own, lives in a fixed array in the library's device image instead: n * k * element size must not exceed
  * PML_HIP_STATIC_SCRATCH_BYTES, larger right-hand sides are rejected with an error text that says so
- * (b_layout 1 needs no copy and has no such limit; a right-hand side that the kernels read where it lies leaves the
+ * (b_layout 1 needs no copy and has no such limit; a product that runs in panels has its fragments there in the place of the copy;
+ * a right-hand side that the kernels read where it lies leaves the
  * array untouched -- with few result tiles in any type, in large bf16 and int8 products whose n and ldb are multiples of
  * four, in bf16 products of many rows and k <= 128, fp32 with n and ldb multiples of four and 16-byte aligned, int8 with
  * rows of whole 16-byte vectors on problems where transposing reads cost less than the copy -- and the limit applies all

@@ -1044,12 +1044,25 @@ static int panel_of(const pml_hip_gemm_desc& d, int kind, int tile, const Direct
   return us < share * tiled_us(kind, tile, d.m, d.n, k_bytes, value_bytes, g.n_cus) ? config : -1;
 }
 
-static size_t panel_bytes(const Plan* p) {
-  const pml_hip_gemm_desc& d = p->gemm;
+static size_t panel_bytes(const pml_hip_gemm_desc& d, int kind) {
   IgemmArgs g;
   gemm_args(d, g);
-  const int es = dt_size(d.in_dtype), frags = panel_frags(p->mfma_kind, g);
+  const int es = dt_size(d.in_dtype), frags = panel_frags(kind, g);
   return winconv_pack_bytes(es, 1, d.k, d.n, frags) + winconv_pack_bytes(es, 1, d.k2, d.n, frags);
+}
+
+// The fragments of a product that runs in panels: its configuration (-1: it does not), where they lie.
+struct PanelRoom {
+  int config = -1;
+  void* image = nullptr;
+};
+
+// Whether a product in panels has room for the fragments of a right-hand side that comes with the call: not where that is read as
+// it lies (int8 by size: gemm_run).  And pml_hip_gemm_run_static gives the same bits, so floats are packed where its array holds
+// the fragments, too, which whole blocks make larger than the transposed form, or where it refuses the call.
+static bool packs_given(const pml_hip_gemm_desc& d, int kind, int tile) {
+  if (kind == KIND_I8) return true;
+  return !takes_b_as_given(d, kind, tile, d.ldb) && (panel_bytes(d, kind) <= PML_HIP_STATIC_SCRATCH_BYTES || d.n * d.k * dt_size(d.in_dtype) > PML_HIP_STATIC_SCRATCH_BYTES);
 }
 
 int64_t pml_hip_gemm_dispatch(const pml_hip_gemm_desc* d) {
@@ -1090,8 +1103,8 @@ int64_t pml_hip_gemm_dispatch(const pml_hip_gemm_desc* d) {
     return 0;
   }
   p->panel = panel_of(*d, kind, p->tile, p->direct, p->ws);
-  // (a right-hand side that comes with the call and is read as it lies needs no room; no memory for it: the product runs in tiles)
-  if (p->panel >= 0 && (kind == KIND_I8 || !takes_b_as_given(*d, kind, p->tile, d->ldb)) && !(p->panel_bt = p->hold(panel_bytes(p)))) p->panel = -1;
+  // (no memory for the fragments: the product runs in tiles)
+  if (p->panel >= 0 && packs_given(*d, kind, p->tile) && !(p->panel_bt = p->hold(panel_bytes(*d, kind)))) p->panel = -1;
   char buf[256];
   std::snprintf(buf, sizeof buf, "gemm %s m=%lld n=%lld k=%lld tile=%s mfma=%s", d->in_dtype == PML_HIP_F32 ? "f32" : d->in_dtype == PML_HIP_BF16 ? "bf16" : "i8",
                 (long long)d->m, (long long)d->n, (long long)d->k, tile_name(p->direct.rows >= 0 ? lds_tile : p->tile),
@@ -1159,24 +1172,26 @@ static bool reads_b_as_given(const pml_hip_gemm_desc& d, int mfma_kind, const vo
   return true;
 }
 
-// The right-hand side (second: of the second product) in the order a panel multiplies it, besides the form that tiles read.
-static int pack_panel(Plan* p, const void* b, bool second, hipStream_t s) {
-  if (p->panel < 0) return 0;
-  const pml_hip_gemm_desc& d = p->gemm;
-  if (!p->panel_bt && !(p->panel_bt = p->hold(panel_bytes(p)))) return 0;
+// A right-hand side (second: of the second product) in the order a panel multiplies it.
+static int pack_fragments(const pml_hip_gemm_desc& d, int kind, void* image, const void* b, bool second, hipStream_t s) {
   IgemmArgs g;
   gemm_args(d, g);
-  const int es = dt_size(d.in_dtype), frags = panel_frags(p->mfma_kind, g);
+  const int es = dt_size(d.in_dtype), frags = panel_frags(kind, g);
   const size_t first = winconv_pack_bytes(es, 1, d.k, d.n, frags);
   const WinFilter w = {1, (int)(second ? d.k2 : d.k), (int)d.n, 0, 0, second ? d.ldb2 : d.ldb, 1, frags};
-  if (check(winconv_pack_launch(es, b, w, (char*)p->panel_bt + (second ? first : 0), s), "winconv_pack_launch")) return 1;
+  return check(winconv_pack_launch(es, b, w, (char*)image + (second ? first : 0), s), "winconv_pack_launch");
+}
+// ... kept by a plan, besides the form that tiles read.
+static int pack_panel(Plan* p, const void* b, bool second, hipStream_t s) {
+  if (p->panel < 0) return 0;
+  if (!p->panel_bt && !(p->panel_bt = p->hold(panel_bytes(p->gemm, p->mfma_kind)))) return 0;
+  if (pack_fragments(p->gemm, p->mfma_kind, p->panel_bt, b, second, s)) return 1;
   p->panel_fresh[second] = true;
   return 0;
 }
-
 static int gemm_run(const pml_hip_gemm_desc& d, int mfma_kind, int tile, const DirectTiles& direct, void* bt, int64_t bt_ld, bool packed,
                     const void* a, const void* b, void* c, const void* init, const void* const* operands,
-                    void* const* outs, pml_hip_stream s, const SecondProduct* second = nullptr, Plan* plan = nullptr) {
+                    void* const* outs, pml_hip_stream s, const SecondProduct* second, Plan* plan, PanelRoom panel) {
   // (a right-hand side that arrives with the call is transposed per run and split in the kernel's registers: a
   // second small launch costs more than it saves; one packed once is kept split)
   const bool b_split = plan && plan->bt_is_split && !b;
@@ -1242,10 +1257,9 @@ static int gemm_run(const pml_hip_gemm_desc& d, int mfma_kind, int tile, const D
   // a 256 x 256 tile reads as it lies pays for that launch from 50 G products on: requantised 4096 x 4096, K = 4096 71 us as it lies,
   // 67.5 packed, 6000 x 3200, K = 3072 90 and 75, 4096 x 4096, K = 2048 38.6 and 40.6.)
   const bool large_i8 = mfma_kind == KIND_I8 && b && b_as_given && (double)d.m * (double)d.n * (double)d.k >= 5e10;
-  if ((transposed || large_i8) && plan && plan->panel_bt && !packed && d.k2 == 0 && panel_runs(mfma_kind, g)) {
-    if (pack_panel(plan, b, false, (hipStream_t)s)) return 1;
-    plan->panel_fresh[0] = false;
-    return check(panel_launch(mfma_kind, plan->panel, g, plan->panel_bt, (hipStream_t)s), "panel_launch");
+  if ((transposed || large_i8) && panel.image && !packed && d.k2 == 0 && panel_runs(mfma_kind, g)) {
+    if (pack_fragments(d, mfma_kind, panel.image, b, false, (hipStream_t)s)) return 1;
+    return check(panel_launch(mfma_kind, panel.config, g, panel.image, (hipStream_t)s), "panel_launch");
   }
   // (rows that stream take a [K][N] right-hand side as it lies, too)
   if (transposed && !(!packed && streams_given(mfma_kind, tile, false, b, d.ldb, g))) {
@@ -1253,7 +1267,8 @@ static int gemm_run(const pml_hip_gemm_desc& d, int mfma_kind, int tile, const D
     if (plan) plan->bt_is_split = plan->bt_is_kn = plan->panel_fresh[0] = false;
     if (check(transpose_pack(es, b, bt, d.k, d.n, d.ldb, bt_ld, (hipStream_t)s), "transpose_pack")) return 1;
   }
-  if (plan && plan->panel_fresh[0] && (d.k2 == 0 || plan->panel_fresh[1]) && !b && (!second || !second->b2) && panel_runs(mfma_kind, g)) return check(panel_launch(mfma_kind, plan->panel, g, plan->panel_bt, (hipStream_t)s), "panel_launch");
+  if (plan && plan->panel_fresh[0] && (d.k2 == 0 || plan->panel_fresh[1]) && !b && (!second || !second->b2) && panel_runs(mfma_kind, g))
+    return check(panel_launch(mfma_kind, panel.config, g, panel.image, (hipStream_t)s), "panel_launch");
   return check(igemm_launch(b_split ? KIND_F32X3P : mfma_kind, tile, false, g, (hipStream_t)s), "igemm_launch");
 }
 
@@ -1261,7 +1276,7 @@ int pml_hip_gemm_invoke(int64_t plan, const void* a, const void* b, void* c, con
                         const void* const* operands, void* const* outs, pml_hip_stream s) {
   Plan* p = (Plan*)(intptr_t)plan;
   if (!p || p->kind != PLAN_GEMM) return fail("gemm_invoke: not a gemm plan");
-  return gemm_run(p->gemm, p->mfma_kind, p->tile, p->direct, p->bt, p->bt_ld, p->packed, a, b, c, init, operands, outs, s, nullptr, p);
+  return gemm_run(p->gemm, p->mfma_kind, p->tile, p->direct, p->bt, p->bt_ld, p->packed, a, b, c, init, operands, outs, s, nullptr, p, {p->panel, p->panel_bt});
 }
 
 int pml_hip_gemm_invoke2(int64_t plan, const void* a, const void* b, void* c, const void* init, const void* a2, const void* b2,
@@ -1275,7 +1290,7 @@ int pml_hip_gemm_invoke2(int64_t plan, const void* a, const void* b, void* c, co
   sp.init2 = init2;
   sp.bt2 = p->bt2;
   sp.packed2 = p->packed2;
-  return gemm_run(p->gemm, p->mfma_kind, p->tile, p->direct, p->bt, p->bt_ld, p->packed, a, b, c, init, operands, outs, s, &sp, p);
+  return gemm_run(p->gemm, p->mfma_kind, p->tile, p->direct, p->bt, p->bt_ld, p->packed, a, b, c, init, operands, outs, s, &sp, p, {p->panel, p->panel_bt});
 }
 
 static bool chain_descs(const pml_hip_gemm_desc& first, const pml_hip_gemm_desc& next) {
@@ -1341,7 +1356,11 @@ int pml_hip_gemm_run_static(const pml_hip_gemm_desc* d, const void* a, const voi
   const bool plain = mode == 1 || mode == 2 || tail_requant(d->tail, d->out_dtype, d->c_dtype, mode, nullptr);
   // (no workspace may be allocated here: the K loop is never split over workgroups)
   const int tile = choose_tile(d->m, d->n, d->k * dt_size(d->in_dtype), kind, plain, PML_HIP_FLAG_TILE_OF(d->flags), /*allow_split=*/false);
-  return gemm_run(*d, kind, tile, direct_tiles(*d, kind, tile), bt, d->k, false, a, b, c, init, operands, outs, s);
+  const DirectTiles direct = direct_tiles(*d, kind, tile);
+  PanelRoom panel;
+  if (bt && (panel.config = panel_of(*d, kind, tile, direct, nullptr)) >= 0 && packs_given(*d, kind, tile) && panel_bytes(*d, kind) <= PML_HIP_STATIC_SCRATCH_BYTES)
+    panel.image = bt;
+  return gemm_run(*d, kind, tile, direct, bt, d->k, false, a, b, c, init, operands, outs, s, nullptr, nullptr, panel);
 }
 
 // ---------------------------------------------------------------------------

@@ -225,3 +225,22 @@ def test_which_products():
         g.flags = hk.flag_tile('128x128')
     for change in (layout, floats, rows, tile):
         assert not panels(25088, 512, 1024, change=change), change
+
+
+# (the last ones: a right-hand side that fits the array of the entry without a plan to the last bytes, as fragments too, and not as fragments)
+@pytest.mark.parametrize('m,n,k,tile', SHAPES + [(2000, 3000, 5568, ''), (2000, 3489, 4808, '')])
+def test_the_entry_without_a_plan_gives_the_same_bits(m, n, k, tile):
+    """Sums of floats, which another order would round otherwise."""
+    hk.init(0)
+    L, none = hk.lib(), hk.ptr_array([])
+    rng = np.random.default_rng(m + n + k)
+    g = desc(m, n, k, lda_gap=8)
+    p = L.pml_hip_gemm_dispatch(ctypes.byref(g))
+    assert 'in panels tile=' + tile in hk.describe(p), hk.describe(p)
+    dA, dB, db = (hk.DeviceBuffer.from_numpy(T.bf16(rng.standard_normal(s).astype(np.float32))) for s in ((m, k + 8), (k, n), (n,)))
+    dC, dD = (hk.DeviceBuffer.from_numpy(np.full((m, n), 77, np.uint16)) for _ in range(2))
+    hk.check(L.pml_hip_gemm_invoke(p, dA.ptr, dB.ptr, dC.ptr, db.ptr, none, none, None))
+    hk.check(L.pml_hip_gemm_run_static(ctypes.byref(g), dA.ptr, dB.ptr, dD.ptr, db.ptr, none, none, None))
+    hk.check(L.pml_hip_stream_sync(None))
+    L.pml_hip_plan_free(p)
+    np.testing.assert_array_equal(dC.to_numpy(np.uint16, (m, n)), dD.to_numpy(np.uint16, (m, n)))
