@@ -1255,8 +1255,9 @@ static int gemm_run(const pml_hip_gemm_desc& d, int mfma_kind, int tile, const D
   // (a right-hand side that comes with the call is packed for a panel by a launch of its own as it would be transposed by one.
   // Not where one was packed ahead: calls without any would multiply by that from then on, and tiles read `bt`.  An int8 one that
   // a 256 x 256 tile reads as it lies pays for that launch from 50 G products on: requantised 4096 x 4096, K = 4096 71 us as it lies,
-  // 67.5 packed, 6000 x 3200, K = 3072 90 and 75, 4096 x 4096, K = 2048 38.6 and 40.6.)
-  const bool large_i8 = mfma_kind == KIND_I8 && b && b_as_given && (double)d.m * (double)d.n * (double)d.k >= 5e10;
+  // 67.5 packed, 6000 x 3200, K = 3072 90 and 75, 4096 x 4096, K = 2048 38.6 and 40.6.  The entry without a plan leaves its array
+  // untouched by what can be read as it lies: calls that share the array count on that.)
+  const bool large_i8 = plan && mfma_kind == KIND_I8 && b && b_as_given && (double)d.m * (double)d.n * (double)d.k >= 5e10;
   if ((transposed || large_i8) && panel.image && !packed && d.k2 == 0 && panel_runs(mfma_kind, g)) {
     if (pack_fragments(d, mfma_kind, panel.image, b, false, (hipStream_t)s)) return 1;
     return check(panel_launch(mfma_kind, panel.config, g, panel.image, (hipStream_t)s), "panel_launch");
