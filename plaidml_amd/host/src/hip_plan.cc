@@ -51,16 +51,15 @@ std::shared_ptr<Plan> Planner::run() {
   if (opt_.specialise) padDepthwiseResults();
   if (opt_.fuse && opt_.specialise) fusePoolIntoConv();
   pruneDeadSteps();
-  // (a schedule names the tiles of single products, by the text of their steps)
-  if (opt_.fuse && opt_.specialise && opt_.tile.empty() && opt_.schedule_path.empty()) chainProducts();
   applySchedule();
-  // (a tile or path that was asked for was asked for the whole step)
-  if (opt_.fuse && opt_.specialise && opt_.tile.empty() && opt_.conv.empty() && opt_.schedule_path.empty()) sliceSteps();
+  // (a tile or path that was asked for, by option or for one step, was asked for a product of its own and for the whole step)
+  if (opt_.fuse && opt_.specialise) chainProducts();
+  if (opt_.fuse && opt_.specialise && opt_.tile.empty() && opt_.conv.empty()) sliceSteps();
   return plan_;
 }
 
 // Tiling overrides, per program (target options) and per step (schedule file): they travel to the kernel library in
-// the descriptors' schedule bits.  Runs last, so that a step is keyed by the text the plan dump shows for it.
+// the descriptors' schedule bits.  Runs when the steps have the text the plan dump shows for them.
 int Planner::convPathByName(const std::string& name) {
   static const char* const names[] = {"auto", "igemm", "patches", "ldsfilter", "blocks", "window"};
   for (int i = 0; i < 6; ++i)
@@ -101,7 +100,12 @@ void Planner::applySchedule() {
     for (std::string line; std::getline(f, line);) {
       const auto open = line.rfind(" {"), lead = line.find("] ");
       if (line.empty() || line.back() != '}' || open == std::string::npos || lead == std::string::npos || lead > open) continue;
-      rules[line.substr(lead + 2, open - lead - 2)] = parseRule(line.substr(open + 2, line.size() - open - 3));
+      const Rule rule = parseRule(line.substr(open + 2, line.size() - open - 3));
+      // (two products that a plan runs in one launch stand on one line of its dump: what is asked for there, for either)
+      const std::string text = line.substr(lead + 2, open - lead - 2);
+      const auto onward = text.find(kOnward);
+      rules[text.substr(0, onward)] = rule;
+      if (onward != std::string::npos) rules[text.substr(onward + std::strlen(kOnward))] = rule;
     }
   }
   for (Step& s : plan_->steps) {

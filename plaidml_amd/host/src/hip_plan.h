@@ -99,7 +99,7 @@ struct Options {
   // Schedule overrides (the reference: PLAIDML_SCHEDULE_PATH, pmlc/target/x86/pipeline.cc:267-272).  `tile` / `conv`
   // (`hip{tile=128x128w8,conv=igemm}`) apply to every matrix product / convolution of the program; `schedule_path` names
   // a file of plan-dump lines, "[n] <step text> {tile=...,conv=...}", that apply to the steps whose text they repeat --
-  // a plan dump edited by hand is such a file.  Names: pml_hip_tile_name, and igemm / patches / ldsfilter / blocks / window.
+  // a plan dump edited by hand is such a file (a line that names two products in one launch is for either).  Names: pml_hip_tile_name, and igemm / patches / ldsfilter / blocks / window.
   std::string tile, conv, schedule_path;
   // `hip{graph=0}`: every run launches its kernels one by one (the default records the launches of the third run of an
   // executable into a HIP graph and replays that from then on: at batch 1 the launches cost more than the kernels)

@@ -258,7 +258,7 @@ void Planner::chainProducts() {
       X.next_b_off = Y.b_off;
       X.next_init = Y.init;
       X.out2 = Y.c;
-      X.text += ", rows multiplied onward: " + Y.text;
+      X.text += kOnward + Y.text;
       X.flops += Y.flops;
       X.bytes += Y.bytes - 2.0 * static_cast<double>(Y.gemm.m * Y.gemm.k);
       plan_->steps.erase(plan_->steps.begin() + static_cast<long>(y));

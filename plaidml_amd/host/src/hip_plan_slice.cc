@@ -24,7 +24,7 @@ class Slicer {
   bool slice(const Step& s, int64_t part, Step* out, Uses* uses) const {
     *out = s;
     *uses = {};
-    if (!s.outs.empty() || s.a_off != 0 || s.c_off != 0 || s.a2_off != 0) return false;
+    if (!s.schedule.empty() || !s.outs.empty() || s.a_off != 0 || s.c_off != 0 || s.a2_off != 0) return false;
     for (int64_t off : s.operand_off)
       if (off != 0) return false;
     switch (s.kind) {

@@ -30,6 +30,8 @@ using tile::ValuePtr;
 using util::DataType;
 using util::TensorShape;
 
+constexpr char kOnward[] = ", rows multiplied onward: ";  // between the texts of two products in one launch
+
 inline int hipType(DataType dt) { return static_cast<int>(dt); }  // the kernel library uses plaidml_datatype values
 
 inline int hipAgg(AggKind a) {

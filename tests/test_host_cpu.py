@@ -303,6 +303,51 @@ def test_schedule_overrides_by_option_and_by_file(tmp_path, monkeypatch):
         programs.residual_block(E, op)[0].compile('')
 
 
+def test_a_schedule_file_over_products_in_one_launch_and_steps_in_parts(tmp_path, monkeypatch):
+    """A line of a dump that names two products is a rule for either, and what the file does not name stays in one launch, and in parts."""
+    BF = E.DType.BFLOAT16
+
+    def chains():
+        w, v = (E.Constant(np.zeros(s, np.float32), BF) for s in ((64, 256), (256, 64)))
+        X, Y = E.Placeholder(BF, [16384, 64]), E.Placeholder(BF, [8192, 64])
+        return E.Program('chains', [X, Y], [op.relu(op.dot(op.relu(op.dot(x, w)), v)) for x in (X, Y)])
+
+    def products():
+        w, v = (E.Constant(np.zeros(s, np.float32), BF) for s in ((2048, 2048), (2048, 80)))
+        X = E.Placeholder(BF, [16384, 2048])
+        return E.Program('products', [X], [op.dot(op.relu(op.dot(X, w)), v)])
+
+    def steps(text):
+        return [l.split('] ', 1)[1] for l in text.splitlines() if l.startswith('  [')]
+
+    def named(text, k, rule=' {tile=128x128}'):
+        lines = text.splitlines()
+        lines[1 + k] += rule
+        return '\n'.join(lines) + '\n'
+    onward = ', rows multiplied onward: '
+    plain, whole = plan_of(chains()), plan_of(products())
+    assert [onward in s for s in steps(plain)] == [True, True], plain
+    assert 'steps 0 to 1 in 2 parts' in whole, whole
+    sched = tmp_path / 'schedule.txt'
+    monkeypatch.setenv('PLAIDML_SCHEDULE_PATH', str(sched))
+    sched.write_text(plain + whole)  # (names nothing)
+    assert plan_of(chains()) == plain and plan_of(products()) == whole
+    first, second = (s.split(onward) for s in steps(plain))
+    for k, apart, together in ((0, first, second), (1, second, first)):
+        sched.write_text(named(plain, k))
+        t = plan_of(chains())
+        assert sorted(steps(t)) == sorted([s + ' {tile=128x128}' for s in apart] + [onward.join(together)]), t
+        sched.write_text(t)  # the dump of that is a file for the same plan, too
+        assert plan_of(chains()) == t
+    sched.write_text('[0] %s {tile=64x64}\n' % first[1])  # one of the two products
+    assert sorted(steps(plan_of(chains()))) == sorted([first[0], first[1] + ' {tile=64x64}', onward.join(second)])
+    # steps ahead of one that was named run in parts, those behind it do not
+    for k, parts in ((0, ''), (1, 'steps 0 to 0 in 2 parts')):
+        sched.write_text(named(whole, k))
+        t = plan_of(products())
+        assert steps(t)[k].endswith('{tile=128x128}') and (parts in t if parts else 'parts' not in t), t
+
+
 def test_target_options_switch_specialisation_off():
     prog = programs.config1_conv(E, op, 'BFLOAT16')[0]
     t = plan_of(prog, 'hip{specialise=0,fuse=0}')
