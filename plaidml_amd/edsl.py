@@ -963,14 +963,16 @@ class Executable(_Handle):
 
 
 def last_run_stats():
-    """Of this thread's last run: its wall time as kernel_ms (device, first to last launch), h2d_ms (host, up to the last upload it
-    queues) and d2h_ms (the rest); its launches and whether they ran as a recorded graph; the executable's device memory."""
+    """Of this thread's last run: its wall time as kernel_ms (device, first to last launch; where copies go beside launches the sum
+    over the runs of launches, each from where it could begin to its end), h2d_ms (host, up to the last upload it queues) and d2h_ms
+    (the rest); its launches, a step that runs on parts once a part, and whether they ran as recorded graphs; the executable's
+    device memory."""
     k, h, d, n = f64(), f64(), f64(), sz()
     lib().plaidml_hip_last_run_stats(ctypes.byref(k), ctypes.byref(h), ctypes.byref(d), ctypes.byref(n))
     a, u, t = sz(), sz(), sz()
     lib().plaidml_hip_last_run_memory(ctypes.byref(a), ctypes.byref(u), ctypes.byref(t))
     steps = (f64 * (n.value or 1))()
-    got = lib().plaidml_hip_last_run_step_ms(n.value, steps)  # per launch; empty unless PLAIDML_PROFILE=1 was set
+    got = lib().plaidml_hip_last_run_step_ms(n.value, steps)  # per step of the plan; empty unless PLAIDML_PROFILE=1 was set
     return {'kernel_ms': k.value, 'h2d_ms': h.value, 'd2h_ms': d.value, 'launches': n.value, 'arena_bytes': a.value,
             'unshared_temp_bytes': u.value, 'device_bytes': t.value, 'graph': bool(lib().plaidml_hip_last_run_replayed()),
             'graph_note': lib().plaidml_hip_last_run_graph_note().decode(), 'step_ms': [steps[i] for i in range(got if got < n.value else n.value)]}

@@ -881,7 +881,8 @@ void* plaidml_hip_host_alloc(size_t bytes) {
 void plaidml_hip_host_free(void* p) { rt::pinnedFree(p); }
 
 // Not part of the reference ABI: the wall time of the calling thread's most recent run in three parts, for benchmarks -- the
-// device's from first to last launch, the host's up to the last upload it queues, and the rest (rt::InvokeStats).
+// device's from first to last launch (summed over its runs of launches where copies go beside them), the host's up to the last
+// upload it queues, and the rest (rt::InvokeStats); its launches, a step that runs on parts once a part.
 void plaidml_hip_last_run_stats(double* kernel_ms, double* h2d_ms, double* d2h_ms, size_t* launches) {
   rt::InvokeStats s = rt::lastInvokeStats();
   if (kernel_ms) *kernel_ms = s.kernel_ms;
@@ -908,8 +909,8 @@ const char* plaidml_hip_last_run_graph_note(void) {
   return note.c_str();
 }
 
-// Per-launch device milliseconds of that run (filled only when PLAIDML_PROFILE=1 was set during it): copies up
-// to `capacity` values to `ms` and returns how many launches the run had timed.
+// Device milliseconds of that run per step of its plan, over the parts a step ran on (filled only when PLAIDML_PROFILE=1 was set
+// during it): copies up to `capacity` values to `ms` and returns how many steps were timed.
 size_t plaidml_hip_last_run_step_ms(size_t capacity, double* ms) {
   rt::InvokeStats s = rt::lastInvokeStats();
   for (size_t i = 0; i < s.step_ms.size() && i < capacity && ms; ++i) ms[i] = s.step_ms[i];

@@ -111,7 +111,8 @@ class HipExecutable final : public Executable {
     return invokeHost(in, out);
   }
 
-  // One run.  Everything is queued on the executable's stream -- uploads, launches, downloads -- and waited for once.
+  // One run.  Everything is queued on the executable's stream -- uploads, launches, downloads -- and waited for once, or, where
+  // long copies can go beside launches, on three (overlapped).
   //   inputs   in page-locked memory already: straight from there.  Elsewhere (or fp32 values of a bf16 tensor): through
   //            the executable's page-locked staging, a few megabytes at a time, so that the link carries one piece
   //            while the host passes over the next.
@@ -458,7 +459,6 @@ class HipExecutable final : public Executable {
       hipCheck(pml_hip_event_elapsed_ms(ev0_, ev1_, &ms), "event elapsed");
       st->kernel_ms = ms;
     }
-    st->launches = plan_->steps.size();
     describe(st);
     if (!profile) return;
     report(st);
@@ -466,6 +466,7 @@ class HipExecutable final : public Executable {
 
   // what does not depend on the run
   void describe(InvokeStats* st) const {
+    st->launches = order_.size();
     st->graph_note = graph_note_;
     st->arena_bytes = arena_bytes_;
     st->unshared_temp_bytes = unshared_temp_bytes_;
@@ -718,6 +719,8 @@ class HipExecutable final : public Executable {
           hipCheck(pml_hip_event_record(seg.up, up_stream_), "event record");
           hipCheck(pml_hip_stream_wait_event(stream_, seg.up), "wait");
           st->h2d_ms = nowMs() - start;
+        } else if (&seg == &segments_.front()) {
+          hipCheck(pml_hip_event_record(seg.up, stream_), "event record");  // (where it could begin)
         }
         if (record_now && !seg.graph && graphable_ && seg.launches.size() > 1) seg.graph = record(seg.launches);
         if (seg.graph) {
@@ -774,11 +777,10 @@ class HipExecutable final : public Executable {
     for (size_t k = 0; k < segments_.size(); ++k) {
       float ms = 0, behind = 0;
       const Segment& seg = segments_[k];
-      if (!seg.needs.empty()) hipCheck(pml_hip_event_elapsed_ms(seg.up, seg.done, &ms), "event elapsed");
+      if (k == 0 || !seg.needs.empty()) hipCheck(pml_hip_event_elapsed_ms(seg.up, seg.done, &ms), "event elapsed");
       if (k > 0) hipCheck(pml_hip_event_elapsed_ms(segments_[k - 1].done, seg.done, &behind), "event elapsed");
       st->kernel_ms += k == 0 ? ms : seg.needs.empty() ? behind : std::min(ms, behind);
     }
-    st->launches = plan_->steps.size();
     describe(st);
     st->kernel_ms = std::min(st->kernel_ms, st->wall_ms);
     st->h2d_ms = std::min(st->h2d_ms, st->wall_ms - st->kernel_ms);

@@ -6,7 +6,7 @@
 // constants and re-lays-out constant weights once when it is built (the
 // reference runs its `init` closure once, pmlc/rt/jit_executable.cc:404-418),
 // and on every invoke copies inputs in, launches the plan on one stream and
-// copies outputs back.
+// copies outputs back, long copies on streams of their own beside the launches.
 #pragma once
 
 #include <memory>
@@ -68,19 +68,22 @@ bool isPinned(const void* p, size_t bytes);
 
 // statistics of the most recent invoke of any hip executable in this thread (for benchmarks)
 struct InvokeStats {
-  // The wall time in three parts.  Uploads, launches and downloads are queued on one stream and waited for once, so where
-  // the link's share ends is not seen from here (another mark would cost a launch of its own): h2d_ms is the host's time up
-  // to the last upload it queues, rounding and staging included; kernel_ms the device's, first launch -> last launch, by the
-  // device's clock as the kernels that copy small operands and results read it (by events where steps are timed); d2h_ms the rest -- what of the uploads is still under way then, the downloads, the passes over the results.
+  // The wall time in three parts.  Where the link's share ends is not seen from here (another mark would cost a launch of its
+  // own): h2d_ms is the host's time up to the last upload it queues, rounding and staging included; kernel_ms the device's, first
+  // launch -> last launch, by the device's clock as the kernels that copy small operands and results read it (by events where
+  // steps are timed); d2h_ms the rest -- what of the uploads is still under way then, the downloads, the passes over the results.
+  // A run whose copies and launches go on streams of their own: kernel_ms is the sum, by events, over its runs of launches, each
+  // from where it could begin (what it needs up, the run before it done) to its end -- the time between two streams is in it, time
+  // in which launches wait for the link is not.
   double kernel_ms = 0;
   double h2d_ms = 0;
   double d2h_ms = 0;
-  size_t launches = 0;
+  size_t launches = 0;             // steps of the plan; one that runs on parts counts once a part
   double wall_ms = 0;              // the whole run, transfers included (what invoke returns)
   size_t arena_bytes = 0;          // device memory shared by the temporaries
   size_t unshared_temp_bytes = 0;  // what the temporaries would take with memory of their own
   size_t device_bytes = 0;         // arena + inputs + outputs + constants + what the kernel plans hold
-  std::vector<double> step_ms;     // per launch, only with PLAIDML_PROFILE=1
+  std::vector<double> step_ms;     // per step of the plan, over its parts; only with PLAIDML_PROFILE=1
   bool replayed = false;           // the launches ran as one recorded graph
   std::string graph_note;          // why they did not, when recording was tried and failed
 };

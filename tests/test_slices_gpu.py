@@ -97,6 +97,8 @@ def test_every_run(monkeypatch, dt, pinned_results, name):
     program, draw, want = build(name, dt, 1 if dt == 'f32' else 2)
     if name == 'dense':
         assert parts(program)[1] > 1
+    steps, n = parts(program)
+    launches = int(re.search(r'(\d+) launches', dict(program.passes)['hip-plan']).group(1)) + steps * (n - 1)
     runner = P.Runner(program, target='hip')
     rounded = (lambda a: a) if dt == 'f32' else P.round_bf16
     for run in range(7):
@@ -109,6 +111,7 @@ def test_every_run(monkeypatch, dt, pinned_results, name):
             got = runner.run(arrays)
         s = P.last_run_stats()
         assert s['kernel_ms'] > 0 and s['h2d_ms'] + s['kernel_ms'] + s['d2h_ms'] == pytest.approx(runner.ms, rel=1e-6, abs=1e-9)
+        assert s['launches'] == launches
         exact = want(*arrays)
         if name.startswith('dense') and dt == 'bf16':  # (the second product takes the rounded first one)
             exact = [exact[0], rounded(exact[0]) @ arrays[3]]
@@ -166,3 +169,25 @@ def test_results_over_operands(dt):
         operand.copy_from_ndarray(bits(x))
         longer.exe.run([operand, longer.stage([x, u])[1]], [result])
         np.testing.assert_array_equal(value(memory), rounded(np.maximum(x @ u, 0)), err_msg='run %d' % run)
+
+
+@pytest.mark.gpu
+def test_launches_ahead_of_every_operand():
+    """Launches that need no operand run while operands travel, and their time counts."""
+    one = lambda *shape: np.full(shape, 0.5, np.float32)
+    bf = P.DType.BFLOAT16
+    c, d = P.Constant(one(4096, 4096), bf), P.Constant(one(4096, 4096), bf)
+    X, V = P.Placeholder(bf, [4096, 4096]), P.Placeholder(bf, [4096, 64])
+    program = P.Program('ahead', [X, V], [Pop.dot(c, d), Pop.dot(X, V)])
+    runner = P.Runner(program, target='hip')
+    plan = dict(program.passes)['hip-plan']
+    assert '2 launches' in plan and plan.index('k=4096 B=[k][n]') < plan.index('n=64'), plan
+    for run in range(4):
+        rng = np.random.default_rng(run)
+        x, v = whole(rng, 4096, 4096), whole(rng, 4096, 64, top=1)
+        got = runner.run([x, v])
+        s = P.last_run_stats()
+        # 137 GFLOP at the 2.5 PFLOP/s the device has at most
+        assert s['launches'] == 2 and s['kernel_ms'] > 0.055, s
+        assert (got[0] == 1024).all()
+        np.testing.assert_array_equal(got[1], P.round_bf16(x @ v))
