@@ -181,6 +181,7 @@ void compileProgram(tile::Program* program, const std::string& requested, bool /
   if (opts.count("tile")) options.tile = opts["tile"];
   if (opts.count("conv")) options.conv = opts["conv"];
   if (opts.count("graph")) options.graph = truthy(opts["graph"]);
+  if (opts.count("overlap")) options.overlap = truthy(opts["overlap"]);
   options.schedule_path = util::Settings::Instance()->get("PLAIDML_SCHEDULE_PATH");
   program->passes.resize(1);  // keep only the "tile" text when compiling again
   tile::foldAddIntoInit(program);

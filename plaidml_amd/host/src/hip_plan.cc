@@ -54,7 +54,7 @@ std::shared_ptr<Plan> Planner::run() {
   applySchedule();
   // (a tile or path that was asked for, by option or for one step, was asked for a product of its own and for the whole step)
   if (opt_.fuse && opt_.specialise) chainProducts();
-  if (opt_.fuse && opt_.specialise && opt_.tile.empty() && opt_.conv.empty()) sliceSteps();
+  if (opt_.fuse && opt_.specialise && opt_.overlap && opt_.tile.empty() && opt_.conv.empty()) sliceSteps();
   return plan_;
 }
 

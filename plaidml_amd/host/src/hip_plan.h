@@ -80,6 +80,7 @@ struct Plan {
   std::vector<int> input_buffers;   // buffer id per program input
   std::vector<int> output_buffers;  // buffer id per program output
   bool graph = true;                // the runtime may replay the launches of a run as one recorded graph
+  bool overlap = true;              // copies may go beside launches
   // The first sliced.size() steps run `slices` times over, on equal parts of the leading dimension (the last one shorter,
   // sliced_last): `steps` says what they are on all of it.  part_bytes: of a part of each buffer that lies part behind part, 0
   // for the others (Planner::sliceSteps).
@@ -104,6 +105,9 @@ struct Options {
   // `hip{graph=0}`: every run launches its kernels one by one (the default records the launches of the third run of an
   // executable into a HIP graph and replays that from then on: at batch 1 the launches cost more than the kernels)
   bool graph = true;
+  // `hip{overlap=0}`: whole steps, and copies up, launches and copies down one after the other on one stream (the default cuts
+  // steps and sends long copies beside launches where that makes a call shorter; it takes more of the device's time)
+  bool overlap = true;
 };
 
 // Runs the pipeline on a copy of the program's op list and returns the plan.

@@ -151,6 +151,7 @@ class Planner {
  public:
   Planner(Program* program, const Options& options) : prog_(program), opt_(options), plan_(std::make_shared<Plan>()) {
     plan_->graph = options.graph;
+    plan_->overlap = options.overlap;
   }
 
   std::shared_ptr<Plan> run();

@@ -582,7 +582,7 @@ class HipExecutable final : public Executable {
       }
       segments_.push_back(std::move(seg));
     }
-    bool fresh = true;
+    bool fresh = true;  // (also behind parts)
     for (size_t i = n; i < p.steps.size(); ++i) {
       std::vector<Range> needs;
       size_t coming = 0, going = 0;
@@ -592,7 +592,7 @@ class HipExecutable final : public Executable {
           needs.push_back({in, 0, p.buffers[p.input_buffers[in]].bytes});
           coming += needs.back().bytes;
         }
-      if (fresh || coming >= kWorthASegment) segments_.emplace_back();
+      if (segments_.empty() || (p.overlap && (fresh || coming >= kWorthASegment))) segments_.emplace_back();
       Segment& seg = segments_.back();
       seg.launches.push_back({i, -1});
       seg.needs.insert(seg.needs.end(), needs.begin(), needs.end());

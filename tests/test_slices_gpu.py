@@ -191,3 +191,19 @@ def test_launches_ahead_of_every_operand():
         assert s['launches'] == 2 and s['kernel_ms'] > 0.055, s
         assert (got[0] == 1024).all()
         np.testing.assert_array_equal(got[1], P.round_bf16(x @ v))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('name', ['dense', 'images', 'batches'])
+def test_the_option_that_keeps_steps_whole(name):
+    program, draw, want = build(name, 'f32')
+    assert parts(program)[1] == 2
+    program.compile('hip{overlap=0}')
+    assert 'parts' not in dict(program.passes)['hip-plan']
+    runner = P.Runner(program, target='hip{overlap=0}')
+    launches = int(re.search(r'(\d+) launches', dict(program.passes)['hip-plan']).group(1))
+    for run in range(4):
+        arrays = draw(np.random.default_rng(run))
+        for g, w in zip(runner.run(arrays), want(*arrays)):
+            np.testing.assert_array_equal(g, w.astype(np.float32))
+        assert P.last_run_stats()['launches'] == launches
