@@ -1065,6 +1065,15 @@ static bool packs_given(const pml_hip_gemm_desc& d, int kind, int tile) {
   return !takes_b_as_given(d, kind, tile, d.ldb) && (panel_bytes(d, kind) <= PML_HIP_STATIC_SCRATCH_BYTES || d.n * d.k * dt_size(d.in_dtype) > PML_HIP_STATIC_SCRATCH_BYTES);
 }
 
+// Whether a right-hand side that comes with the call is packed for a panel by a launch of its own, as it would be transposed by
+// one.  An int8 one that a 256 x 256 tile reads as it lies pays for that launch from 50 G products on: requantised 4096 x 4096,
+// K = 4096 71 us as it lies, 67.5 packed, 6000 x 3200, K = 3072 90 and 75, 4096 x 4096, K = 2048 38.6 and 40.6.
+static bool packs_in_call(const pml_hip_gemm_desc& d, int kind, bool as_given) {
+  return d.k2 == 0 && (!as_given || (kind == KIND_I8 && (double)d.m * (double)d.n * (double)d.k >= 5e10));
+}
+
+static bool reads_b_as_given(const pml_hip_gemm_desc& d, int mfma_kind, const void* b, int tile);
+
 int64_t pml_hip_gemm_dispatch(const pml_hip_gemm_desc* d) {
   const int kind = gemm_desc_kind(d);
   if (kind < 0) return 0;
@@ -1113,11 +1122,13 @@ int64_t pml_hip_gemm_dispatch(const pml_hip_gemm_desc* d) {
   if (p->direct.rows >= 0) p->text += std::string(", with rows of K at hand tile=") + tile_name(p->direct.rows) + " mfma=" + mfma16_name(kind);
   if (p->direct.given >= 0)
     p->text += std::string(", with B as it lies tile=") + (p->direct.given == TILE_16x16_W8 ? "16x64" : "32x64") + " (8 wavefronts sharing K) mfma=" + mfma16_name(kind);
-  if (p->direct.given < 0 && takes_b_as_given(*d, kind, p->tile, d->ldb))
-    p->text += std::string(", with B as it lies") + (p->b_kn ? " or packed" : "") + " through registers mfma=" + mfma16_name(kind);
-  else if (p->b_kn)
+  // (of a right-hand side on 16 bytes)
+  const bool in_call = p->panel_bt && p->direct.given < 0 && packs_in_call(*d, kind, reads_b_as_given(*d, kind, (const void*)256, p->tile));
+  if (p->direct.given < 0 && takes_b_as_given(*d, kind, p->tile, d->ldb) && !in_call)
+    p->text += std::string(", with B as it lies") + (p->b_kn && p->panel < 0 ? " or packed" : "") + " through registers mfma=" + mfma16_name(kind);
+  else if (p->b_kn && p->panel < 0)
     p->text += std::string(", with B packed through registers mfma=") + mfma16_name(kind);
-  if (p->panel >= 0) p->text += ", with B packed " + panel_text(p->panel) + " mfma=" + mfma16_name(kind);
+  if (p->panel >= 0) p->text += std::string(", with B packed ") + (in_call ? "ahead or in the call " : "") + panel_text(p->panel) + " mfma=" + mfma16_name(kind);
   {
     IgemmArgs g;
     gemm_args(*d, g);
@@ -1252,13 +1263,9 @@ static int gemm_run(const pml_hip_gemm_desc& d, int mfma_kind, int tile, const D
       return fail("gemm_invoke: missing extra output");
   // (the K split over workgroups is not built for a right-hand side packed split)
   if (plan && !b_split) split_args(plan, g);
-  // (a right-hand side that comes with the call is packed for a panel by a launch of its own as it would be transposed by one.
-  // Not where one was packed ahead: calls without any would multiply by that from then on, and tiles read `bt`.  An int8 one that
-  // a 256 x 256 tile reads as it lies pays for that launch from 50 G products on: requantised 4096 x 4096, K = 4096 71 us as it lies,
-  // 67.5 packed, 6000 x 3200, K = 3072 90 and 75, 4096 x 4096, K = 2048 38.6 and 40.6.  The entry without a plan leaves its array
-  // untouched by what can be read as it lies: calls that share the array count on that.)
-  const bool large_i8 = plan && mfma_kind == KIND_I8 && b && b_as_given && (double)d.m * (double)d.n * (double)d.k >= 5e10;
-  if ((transposed || large_i8) && panel.image && !packed && d.k2 == 0 && panel_runs(mfma_kind, g)) {
+  // (Not where one was packed ahead: calls without any would multiply by that from then on, and tiles read `bt`.  The entry without
+  // a plan leaves its array untouched by what can be read as it lies: calls that share the array count on that.)
+  if (b && !d.b_layout && (transposed || plan) && panel.image && !packed && packs_in_call(d, mfma_kind, b_as_given) && panel_runs(mfma_kind, g)) {
     if (pack_fragments(d, mfma_kind, panel.image, b, false, (hipStream_t)s)) return 1;
     return check(panel_launch(mfma_kind, panel.config, g, panel.image, (hipStream_t)s), "panel_launch");
   }

@@ -244,3 +244,20 @@ def test_the_entry_without_a_plan_gives_the_same_bits(m, n, k, tile):
     hk.check(L.pml_hip_stream_sync(None))
     L.pml_hip_plan_free(p)
     np.testing.assert_array_equal(dC.to_numpy(np.uint16, (m, n)), dD.to_numpy(np.uint16, (m, n)))
+
+
+def test_texts_name_what_multiplies_a_right_hand_side_that_comes_with_the_call():
+    def requantised(m, n, k):
+        g = hk.GemmDesc()
+        g.in_dtype, g.out_dtype, g.c_dtype = hk.I8, hk.I32, hk.I8
+        g.m, g.n, g.k, g.lda, g.ldb, g.ldc = m, n, k, k, n, n
+        g.tail = hk.make_tail(ops=[(hk.EPI_CAST, hk.F32, 0, 0, 0.0), (hk.EPI_MUL, hk.F32, hk.OPND_TENSOR, 0, 0.0), (hk.EPI_MAX_GT, hk.F32, hk.OPND_IMM, 0, -120.0),
+                                   (hk.EPI_MIN, hk.F32, hk.OPND_IMM, 0, 127.0), (hk.EPI_ROUND, hk.F32, 0, 0, 0.0), (hk.EPI_CAST, hk.I8, 0, 0, 0.0)],
+                              operands=[(hk.F32, 0, 1)])
+        return text_of(g)
+    for m, n, k, in_call in ((4096, 4096, 4096, True), (6000, 3200, 3072, True), (4096, 4096, 2048, False), (4096, 4094, 2048, True)):
+        text = requantised(m, n, k)
+        assert 'with B packed ' + ('ahead or in the call in panels' if in_call else 'in panels') in text and ('with B as it lies' in text) != in_call, text
+    for m, n, k, tile in SHAPES:
+        text = text_of(desc(m, n, k))
+        assert 'with B packed ' + ('in panels' if 'as it lies' in text else 'ahead or in the call in panels') in text and 'packed through' not in text, text
