@@ -1192,10 +1192,15 @@ static int pack_fragments(const pml_hip_gemm_desc& d, int kind, void* image, con
   const WinFilter w = {1, (int)(second ? d.k2 : d.k), (int)d.n, 0, 0, second ? d.ldb2 : d.ldb, 1, frags};
   return check(winconv_pack_launch(es, b, w, (char*)image + (second ? first : 0), s), "winconv_pack_launch");
 }
-// ... kept by a plan, besides the form that tiles read.
+// ... kept by a plan, besides the form that tiles read.  (Where the plan has no room for it yet and the packing is recorded into a
+// graph, which may not allocate, the product runs in tiles.)
 static int pack_panel(Plan* p, const void* b, bool second, hipStream_t s) {
   if (p->panel < 0) return 0;
-  if (!p->panel_bt && !(p->panel_bt = p->hold(panel_bytes(p->gemm, p->mfma_kind)))) return 0;
+  if (!p->panel_bt) {
+    hipStreamCaptureStatus recorded = hipStreamCaptureStatusActive;
+    if (hipStreamIsCapturing(s, &recorded) != hipSuccess) (void)hipGetLastError();
+    if (recorded != hipStreamCaptureStatusNone || !(p->panel_bt = p->hold(panel_bytes(p->gemm, p->mfma_kind)))) return 0;
+  }
   if (pack_fragments(p->gemm, p->mfma_kind, p->panel_bt, b, second, s)) return 1;
   p->panel_fresh[second] = true;
   return 0;

@@ -261,3 +261,37 @@ def test_texts_name_what_multiplies_a_right_hand_side_that_comes_with_the_call()
     for m, n, k, tile in SHAPES:
         text = text_of(desc(m, n, k))
         assert 'with B packed ' + ('in panels' if 'as it lies' in text else 'ahead or in the call in panels') in text and 'packed through' not in text, text
+
+
+def test_a_packing_that_is_recorded():
+    """Into a graph, where nothing may be allocated: by a plan that has no room for fragments yet, and by one that has."""
+    hk.init(0)
+    L, none = hk.lib(), hk.ptr_array([])
+    m = n = k = 4096
+    rng = np.random.default_rng(3)
+    A, B = rng.integers(-2, 3, (m, k)).astype(np.float32), rng.integers(-1, 2, (k, n)).astype(np.float32)
+    g = desc(m, n, k, mode='scale')
+    g.tail = hk.make_tail()
+    want = E.round_bf16(A @ B)
+    dA, dB = hk.DeviceBuffer.from_numpy(T.bf16(A)), hk.DeviceBuffer.from_numpy(T.bf16(B))
+    for ahead in (False, True):
+        p = L.pml_hip_gemm_dispatch(ctypes.byref(g))
+        assert 'with B as it lies through registers' in hk.describe(p) and 'with B packed in panels' in hk.describe(p), hk.describe(p)
+        if ahead:
+            hk.check(L.pml_hip_gemm_pack_b(p, dA.ptr, None))
+            hk.check(L.pml_hip_stream_sync(None))
+        stream, graph = ctypes.c_void_p(), ctypes.c_void_p()
+        hk.check(L.pml_hip_stream_create(ctypes.byref(stream)))
+        hk.check(L.pml_hip_capture_begin(stream))
+        rc = L.pml_hip_gemm_pack_b(p, dB.ptr, stream)
+        hk.check(L.pml_hip_capture_end(stream, ctypes.byref(graph)))
+        hk.check(rc)
+        for _ in range(3):
+            dC = hk.DeviceBuffer.from_numpy(np.full((m, n), 77, np.uint16))
+            hk.check(L.pml_hip_graph_launch(graph, stream))
+            hk.check(L.pml_hip_gemm_invoke(p, dA.ptr, None, dC.ptr, None, none, none, stream))
+            hk.check(L.pml_hip_stream_sync(stream))
+            np.testing.assert_array_equal(E.bf16_from_bits(dC.to_numpy(np.uint16, (m, n))), want)
+        L.pml_hip_graph_destroy(graph)
+        L.pml_hip_stream_destroy(stream)
+        L.pml_hip_plan_free(p)
