@@ -72,6 +72,7 @@ def test_what_runs_in_parts():
     for name in CASES:
         steps, n = parts(build(name, 'f32')[0])
         assert steps >= 1 and 2 <= n <= 4, name
+        assert n == 2, name
     assert parts(dense('f32', 64)[0]) == (0, 1)  # (nothing to carry meanwhile)
     assert parts(batches('f32', 150)[0]) == (0, 1) and parts(batches('f32', 220)[0])[1] == 2  # (parts of 4 MB and more)
     X, W = P.Placeholder(DT['f32'], [4096, 1024]), P.Placeholder(DT['f32'], [4096, 64])
@@ -207,3 +208,125 @@ def test_the_option_that_keeps_steps_whole(name):
         for g, w in zip(runner.run(arrays), want(*arrays)):
             np.testing.assert_array_equal(g, w.astype(np.float32))
         assert P.last_run_stats()['launches'] == launches
+
+
+# Every kind of step that is cut, with a shorter last part and rows or images that begin anywhere in their part: (program, draws,
+# what its plan says).  Whole numbers or one and the same kernel: a run on whole steps gives the same bits.
+def softmax(dt, m, c=1001):
+    X = P.Placeholder(DT[dt], [m, c])
+    return P.Program('softmax', [X], [Pop.softmax(X, -1), Pop.argmax(X, 1)]), lambda rng: [whole(rng, m, c, top=9)], ['softmax', 'argmax']
+
+
+def topk(dt, m, c=1001):
+    X = P.Placeholder(DT[dt], [m, c])
+    return P.Program('topk', [X], [Pop.softmax(X, -1)] + list(Pop.topk(X, 5))), lambda rng: [whole(rng, m, c, top=9)], ['softmax', 'top 5']
+
+
+def rows_with_scalars(dt, m, c=1001):
+    X, s, g = (P.Placeholder(DT[dt], sizes) for sizes in ([m, c], [m, 1], [c]))
+    top = Pop.max(X, 1, True)
+    return P.Program('scalars', [X, s, g], [(X - top) * s + g, top * s]), lambda rng: [whole(rng, m, c), whole(rng, m, 1, top=9), whole(rng, c)], ['row program']
+
+
+def odd_batches(dt, n, r=97):
+    A, B = P.Placeholder(DT[dt], [n, r, 63]), P.Placeholder(DT[dt], [n, 63, 81])
+    x, i, j, k = P.TensorIndexes(4)
+    C = P.Contraction().outShape(n, r, 81).outAccess(x, i, j).sum(A[x, i, k] * B[x, k, j]).build()
+    return P.Program('batches', [A, B], [C]), lambda rng: [whole(rng, n, r, 63), whole(rng, n, 63, 81, top=1)], ['97']
+
+
+def odd_rows(dt, m, k=1003):
+    """(K off whole vectors: a product over free strides)"""
+    X, W, b = P.Placeholder(DT[dt], [m, k]), P.Placeholder(DT[dt], [k, 1001]), P.Placeholder(DT[dt], [1001])
+    return P.Program('rows', [X, W, b], [Pop.relu(Pop.dot(X, W) + b)]), lambda rng: [whole(rng, m, k), whole(rng, k, 1001, top=1), whole(rng, 1001)], ['product']
+
+
+def few_channels(dt, n, stride=1, h=63, w=61, co=7):
+    X, F, b = P.Placeholder(DT[dt], [n, h, w, 3]), P.Placeholder(DT[dt], [5, 5, 3, co]), P.Placeholder(DT[dt], [co])
+    y = Pop.relu(Pop.convolution(X, F, strides=[stride] * 2) + b)
+    return P.Program('channels', [X, F, b], [y]), lambda rng: [whole(rng, n, h, w, 3), whole(rng, 5, 5, 3, co, top=1), whole(rng, co)], ['conv2d']
+
+
+def stem(dt, n):
+    return few_channels(dt, n, stride=2, co=64)
+
+
+def pooled_stem(dt, n, hw=128):
+    """(in bf16 the convolution pools inside its launch)"""
+    X = P.Placeholder(DT[dt], [n, hw, hw, 3])
+    rng = np.random.default_rng(6)
+    F, b = P.Constant(whole(rng, 7, 7, 3, 64, top=1), DT[dt]), P.Constant(whole(rng, 64), DT[dt])
+    y = Pop.relu(Pop.convolution(X, F, strides=[2, 2], autopad=Pop.SAME_UPPER) + b)
+    text = '+ max-pool 3x3 stride 2' if dt == 'bf16' else 'pool2d max'
+    return P.Program('stem', [X], [Pop.pool(y, 'max', [3, 3], [2, 2], autopad=Pop.SAME_UPPER)]), lambda rng: [whole(rng, n, hw, hw, 3)], [text]
+
+
+def depthwise(dt, n, hw=33, c=72):
+    X, F = P.Placeholder(DT[dt], [n, hw, hw, c]), P.Placeholder(DT[dt], [3, 3, c, 1])
+    y = Pop.relu(Pop.convolution(X, F, depthwise=True))
+    return P.Program('depthwise', [X, F], [y]), lambda rng: [whole(rng, n, hw, hw, c), whole(rng, 3, 3, c, 1)], ['dwconv2d']
+
+
+def separable(dt, n, hw=19, c=104):
+    """Depthwise, pointwise with scale and shift, maximum and its place in the window."""
+    X = P.Placeholder(DT[dt], [n, hw, hw, c])
+    rng = np.random.default_rng(4)
+    F, W, s, z = (P.Constant(v, DT[dt]) for v in (whole(rng, 3, 3, c, 1), whole(rng, 1, 1, c, c, top=1), 2.0 ** whole(rng, c, top=1), whole(rng, c)))
+    R = Pop.relu(Pop.convolution(Pop.convolution(X, F, depthwise=True), W) * s + z)
+    M = Pop.pool(R, 'max', [3, 3], [2, 2], autopad=Pop.SAME_UPPER)
+    b, x0, x1, ch, k0, k1 = P.TensorIndexes(6)
+    IX = P.index([3, 3], 0) * 3 + P.index([3, 3], 1)
+    AM = P.Contraction().outShape(M.shape).outAccess(b, x0, x1, ch).max(P.cond(R[b, 2 * x0 + k0 - 1, 2 * x1 + k1 - 1, ch], M[b, x0, x1, ch], IX[k0, k1])).build()
+    return P.Program('separable', [X], [R, M, AM]), lambda rng: [whole(rng, n, hw, hw, c)], ['dwconv2d', 'pool2d']
+
+
+def blocks(dt, n, hw=47, stride=1):
+    """A residual block behind a projection of its own rows, and the product that the chip multiplies its rows onward to (bf16)."""
+    side = (hw - 1) // stride + 1
+    X, T = P.Placeholder(DT[dt], [n, hw, hw, 64]), P.Placeholder(DT[dt], [n, side, side, 64])
+    rng = np.random.default_rng(5)
+    w, v, u = (P.Constant(whole(rng, 1, 1, *s, top=1) * (rng.random(s) < 0.2), DT[dt]) for s in ((64, 256), (64, 256), (256, 64)))
+    c, d = (P.Constant(whole(rng, k), DT[dt]) for k in (256, 256))
+    y = Pop.relu(Pop.convolution(T, w) + c + (Pop.convolution(X, v, strides=[stride] * 2) + d))
+    draw = lambda rng: [whole(rng, n, hw, hw, 64), whole(rng, n, side, side, 64, top=1)]
+    return P.Program('blocks', [X, T], [y, Pop.relu(Pop.convolution(y, u))]), draw, ['second product'] if dt == 'bf16' else []
+
+
+def strided_blocks(dt, n):
+    return blocks(dt, n, hw=113, stride=2)
+
+
+# (odd numbers of rows or images, of which the first part has an odd number too)
+KINDS = {f.__name__: (f, sizes) for f, *sizes in ((softmax, 4001, 8001), (topk, 4001, 8001), (rows_with_scalars, 4001, 8001), (odd_batches, 401, 801), (odd_rows, 4001, 8001),
+                                                  (few_channels, 201, 405), (stem, 201, 405), (pooled_stem, 81, 161), (depthwise, 61, 121), (separable, 61, 121), (blocks, 29, 29), (strided_blocks, 21, 21))}
+
+
+def kind(name, dt):
+    fn, (f32, bf16) = KINDS[name]
+    return fn(dt, f32 if dt == 'f32' else bf16)
+
+
+@pytest.mark.parametrize('dt', ['f32', 'bf16'])
+@pytest.mark.parametrize('name', sorted(KINDS))
+def test_which_kinds_run_in_parts(dt, name):
+    """All of the program, in two parts, the second one shorter."""
+    program, _, texts = kind(name, dt)
+    steps, n = parts(program)
+    plan = dict(program.passes)['hip-plan']
+    assert n == 2 and '%d launches' % steps in plan and all(t in plan for t in texts), plan
+    assert all(size % 4 == 1 for size in KINDS[name][1])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('dt', ['f32', 'bf16'])
+@pytest.mark.parametrize('name', sorted(KINDS))
+def test_every_kind_of_step(dt, name):
+    print(name, dt, flush=True)
+    program, draw, _ = kind(name, dt)
+    assert parts(program)[1] == 2
+    cut, whole_steps = P.Runner(program, target='hip'), P.Runner(program, target='hip{overlap=0}')
+    for run in range(4):
+        arrays = draw(np.random.default_rng(run))
+        for k, (g, w) in enumerate(zip(cut.run(arrays), whole_steps.run(arrays))):
+            assert np.any(w) and g.dtype == w.dtype
+            np.testing.assert_array_equal(g, w, err_msg='%s run %d result %d' % (name, run, k))
