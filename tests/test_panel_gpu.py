@@ -295,3 +295,31 @@ def test_a_packing_that_is_recorded():
         L.pml_hip_graph_destroy(graph)
         L.pml_hip_stream_destroy(stream)
         L.pml_hip_plan_free(p)
+
+
+# every configuration with a second product (K: of both), and for either result of int8 (the 192x384 one is no int32 product's)
+SECONDS = [(19945, 193, 272, '112x256'), (2172, 3910, 280, '112x512'), (14793, 614, 296, '128x512'), (13657, 1078, 288, '192x384'),
+           (18752, 611, 320, '224x256'), (1281, 202, 1120, '64x256'), (10897, 309, 272, '64x512'), (11923, 1234, 288, '96x768')]
+INT8 = [(18633, 130, 1024, False, '112x256'), (23195, 257, 1024, False, '112x512'), (15284, 518, 1024, False, '128x512'), (16714, 600, 1024, False, '224x256'),
+        (4030, 919, 1024, False, '64x256'), (11008, 269, 1024, False, '64x512'), (19821, 520, 1024, False, '96x768'), (17666, 141, 528, True, '112x256'),
+        (19422, 258, 528, True, '112x512'), (15482, 542, 528, True, '128x512'), (8216, 1778, 528, True, '192x384'), (16714, 600, 528, True, '224x256'),
+        (8653, 140, 528, True, '64x256'), (8702, 275, 528, True, '64x512'), (19642, 541, 528, True, '96x768')]
+
+
+@pytest.mark.parametrize('m,n,k,tile', SECONDS)
+def test_every_configuration_with_a_second_product(m, n, k, tile):
+    k1 = k // 24 * 8
+    run(m, n, k1, tile + ' (', k2=k - k1, lda_gap=16, gap=3)
+
+
+@pytest.mark.parametrize('m,n,k,requantised,tile', INT8)
+def test_every_configuration_int8(m, n, k, requantised, tile):
+    g = hk.GemmDesc()
+    g.in_dtype, g.out_dtype, g.c_dtype = hk.I8, hk.I32, hk.I8 if requantised else hk.I32
+    g.m, g.n, g.k, g.lda, g.ldb, g.ldc = m, n, k, k + 16, n, n
+    if requantised:
+        g.tail = hk.make_tail(ops=[(hk.EPI_CAST, hk.F32, 0, 0, 0.0), (hk.EPI_MUL, hk.F32, hk.OPND_TENSOR, 0, 0.0), (hk.EPI_MAX_GT, hk.F32, hk.OPND_IMM, 0, -120.0),
+                                   (hk.EPI_MIN, hk.F32, hk.OPND_IMM, 0, 127.0), (hk.EPI_ROUND, hk.F32, 0, 0, 0.0), (hk.EPI_CAST, hk.I8, 0, 0, 0.0)],
+                              operands=[(hk.F32, 0, 1)])
+    assert 'in panels tile=%s (' % tile in text_of(g), text_of(g)
+    test_int8(m, n, k, requantised, True, False, 4, True)

@@ -2,6 +2,7 @@
 The sizes end tiles inside a row, between images and behind the last result, windows with one slab of channels, several of them
 in one window or in two, and a last slab or block that is not full, columns anywhere; strides, dilations and paddings of any sign."""
 import ctypes
+import re
 
 import numpy as np
 import pytest
@@ -149,3 +150,45 @@ def test_infinities_stay_with_their_taps(kind):
     assert np.isnan(got[touched]).all()
     compare(kind, got[~touched], want[~touched])
 
+
+
+# every configuration of every type, on a device of 256 compute units: n, height and width, channels, columns, filter, stride; the
+# columns of a tile, its wavefronts, what each of them holds, how many share K
+EVERY = [('bf16', 75, 53, 64, 20, 2, 1, 32, 4, '112x32', 1), ('bf16', 3, 56, 32, 125, 2, 1, 32, 4, '64x32', 1),
+         ('bf16', 10, 53, 32, 17, 2, 1, 32, 4, '64x32', 2), ('bf16', 1, 8, 64, 30, 2, 2, 32, 8, '32x32', 4),
+         ('bf16', 41, 45, 32, 33, 2, 1, 64, 4, '112x64', 1), ('bf16', 49, 21, 32, 189, 3, 2, 64, 4, '64x64', 2),
+         ('bf16', 77, 25, 128, 78, 2, 2, 64, 4, '64x64', 4), ('bf16', 10, 60, 256, 54, 2, 1, 64, 8, '112x64', 4),
+         ('bf16', 68, 47, 32, 56, 2, 2, 128, 4, '112x64', 1), ('bf16', 90, 30, 32, 72, 2, 2, 128, 8, '112x32', 2),
+         ('bf16', 18, 55, 128, 289, 2, 2, 128, 8, '112x64', 2), ('bf16', 66, 17, 128, 74, 5, 1, 128, 8, '112x64', 4),
+         ('bf16', 14, 54, 64, 299, 2, 2, 128, 8, '64x64', 2), ('f32', 33, 57, 16, 20, 2, 1, 32, 4, '112x32', 1),
+         ('f32', 11, 63, 16, 19, 3, 1, 32, 4, '64x32', 1), ('f32', 16, 41, 16, 22, 2, 1, 32, 4, '64x32', 2),
+         ('f32', 3, 19, 16, 51, 2, 1, 32, 8, '32x32', 4), ('f32', 22, 45, 32, 287, 3, 1, 64, 4, '112x64', 1),
+         ('f32', 36, 50, 32, 39, 3, 1, 64, 4, '64x64', 2), ('f32', 98, 17, 64, 54, 5, 1, 64, 4, '64x64', 4),
+         ('f32', 81, 26, 64, 43, 3, 1, 64, 8, '112x64', 4), ('f32', 82, 36, 64, 114, 2, 1, 128, 4, '112x64', 1),
+         ('f32', 4, 56, 32, 196, 3, 1, 128, 8, '112x32', 2), ('f32', 44, 24, 64, 249, 3, 1, 128, 8, '112x64', 2),
+         ('f32', 42, 19, 64, 197, 2, 1, 128, 8, '64x64', 2), ('i8', 45, 63, 64, 17, 3, 1, 32, 4, '112x32', 1),
+         ('i8', 11, 61, 64, 25, 2, 1, 32, 4, '64x32', 1), ('i8', 34, 34, 64, 87, 2, 2, 32, 4, '64x32', 2),
+         ('i8', 1, 6, 64, 18, 2, 1, 32, 8, '32x32', 4), ('i8', 44, 51, 64, 44, 2, 1, 64, 4, '112x64', 1),
+         ('i8', 7, 60, 64, 190, 2, 2, 64, 4, '64x64', 2), ('i8', 98, 19, 512, 34, 2, 2, 64, 4, '64x64', 4),
+         ('i8', 11, 54, 512, 21, 3, 1, 64, 8, '112x64', 4), ('i8', 14, 51, 64, 40, 2, 1, 128, 4, '112x64', 1),
+         ('i8', 65, 16, 64, 49, 2, 1, 128, 8, '112x32', 2), ('i8', 18, 46, 64, 66, 5, 1, 128, 8, '112x64', 2),
+         ('i8', 15, 45, 128, 34, 3, 1, 128, 8, '64x64', 2)]
+
+
+@pytest.mark.parametrize('kind,n,hw,ci,co,k,s,columns,wavefronts,block,sharing', EVERY)
+def test_every_configuration(kind, n, hw, ci, co, k, s, columns, wavefronts, block, sharing):
+    o = -(-hw // s)
+    p = max(0, (o - 1) * s + k - hw) // 2
+    d = hk.Conv2dDesc()
+    d.in_dtype, (d.out_dtype, d.c_dtype) = KINDS[kind][0], [KINDS[kind][1]] * 2
+    d.n, d.h, d.w, d.ci, d.kh, d.kw, d.co, d.oh, d.ow = n, hw, hw, ci, k, k, co, o, o
+    d.stride_h, d.stride_w, d.dil_h, d.dil_w, d.pad_h, d.pad_w = s, s, 1, 1, p, p
+    plan = hk.lib().pml_hip_conv2d_dispatch(ctypes.byref(d))
+    text = hk.describe(plan)
+    hk.lib().pml_hip_plan_free(plan)
+    shared = ', %d sharing K' % sharing if sharing > 1 else ''
+    assert re.search(r'tile=\d+x%d over its window in LDS \(%d wavefronts of %s%s\)' % (columns, wavefronts, block, shared), text), text
+    rng = np.random.default_rng(hw + co)
+    I, F, bias = whole(rng, (n, hw, hw, ci), 2), whole(rng, (k, k, ci, co), 1), whole(rng, co, 50)
+    geometry = ((o, o), (s, s), (1, 1), (p, p))
+    compare(kind, run(kind, I, F, *geometry, bias=bias, relu=True, tile='%d wavefronts of %s%s)' % (wavefronts, block, shared)), reference(I, F, *geometry, bias=bias, relu=True))
