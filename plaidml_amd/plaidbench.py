@@ -94,7 +94,7 @@ def run(network_name, batch_size=1, examples=DEFAULT_EXAMPLES, warmups=DEFAULT_W
     execution_duration = time.perf_counter() - t0
     results['execution_duration'] = execution_duration
     results['duration_per_example'] = execution_duration / examples            # wall time, transfers included
-    results['tile_duration_per_example'] = kernel_ms * 1e-3 / examples         # device time of the kernels alone
+    results['tile_duration_per_example'] = kernel_ms * 1e-3 / examples         # device time of the kernels (with waits where copies go beside them)
     golden = net.golden(batch_size) if net.golden else None
     if golden is not None:
         correct, max_error, max_abs_error, fail_ratio = check_correctness(golden.expected, golden.select(outputs[0]),
