@@ -92,6 +92,7 @@ int pml_hip_event_create(pml_hip_event* e);
 int pml_hip_event_destroy(pml_hip_event e);
 int pml_hip_event_record(pml_hip_event e, pml_hip_stream s);
 int pml_hip_event_sync(pml_hip_event e);
+int pml_hip_event_done(pml_hip_event e); /* 1: what was queued ahead of its last record is done; 0: not yet, or not known */
 int pml_hip_stream_wait_event(pml_hip_stream s, pml_hip_event e); /* what is queued on s from here on waits for e */
 int pml_hip_event_elapsed_ms(pml_hip_event start, pml_hip_event stop, float* ms);
 

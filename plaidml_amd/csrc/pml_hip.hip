@@ -863,6 +863,11 @@ int pml_hip_event_record(pml_hip_event e, pml_hip_stream s) {
   return check(hipEventRecord((hipEvent_t)e, (hipStream_t)s), "hipEventRecord");
 }
 int pml_hip_event_sync(pml_hip_event e) { return check(hipEventSynchronize((hipEvent_t)e), "hipEventSynchronize"); }
+int pml_hip_event_done(pml_hip_event e) {
+  const bool done = hipEventQuery((hipEvent_t)e) == hipSuccess;
+  if (!done) (void)hipGetLastError();
+  return done ? 1 : 0;
+}
 int pml_hip_stream_wait_event(pml_hip_stream s, pml_hip_event e) {
   return check(hipStreamWaitEvent((hipStream_t)s, (hipEvent_t)e, 0), "hipStreamWaitEvent");
 }

@@ -195,6 +195,36 @@ def test_launches_ahead_of_every_operand():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize('n, hw, ci, co', [(10, 49, 117, 26), (3, 106, 52, 19)])
+def test_copies_up_do_not_wait_for_copies_down(n, hw, ci, co):
+    """Both gradients of a 5x5 convolution, X needed by the second launch only and as long as the first one's result: the one goes up
+    beside the other, whichever copy engines the two are given (the process's other streams decide that).
+
+    One stream: all up, both launches, all down, of which X's way up or the result's is a quarter and more; half of that is asked for
+    (measured 0.70 and 0.74 of the one stream's time; 1.02 and 1.03 where X waited behind a result that waited for its launch)."""
+    import torch
+    torch.zeros(1, device='cuda')
+    X, F, G = (P.Placeholder(DT['f32'], s) for s in ([n, hw, hw, ci], [5, 5, ci, co], [n, hw, hw, co]))
+    program = P.Program('gradients', [X, F, G], [Pop.convolution(G, F, strides=[1, 1], deriv_mode=Pop.DERIV_DATA, result_shape=[hw, hw]),
+                                                 Pop.convolution(X, G, strides=[1, 1], deriv_mode=Pop.DERIV_FILTER, result_shape=[5, 5])])
+    runners = P.Runner(program, target='hip'), P.Runner(program, target='hip{overlap=0}')
+    rng = np.random.default_rng(3)
+    arrays = [whole(rng, n, hw, hw, ci, top=1), whole(rng, 5, 5, ci, co, top=1), whole(rng, n, hw, hw, co, top=1)]
+    times, got = ([], []), [None, None]
+    for block in range(9):
+        for which in (0, 1) if block % 2 else (1, 0):
+            for _ in range(6):
+                got[which] = runners[which].run(arrays)
+                if block:
+                    times[which].append(runners[which].ms)
+    for g, w in zip(*got):  # (whole numbers below 2^24, whatever the order of sums)
+        np.testing.assert_array_equal(g, w)
+    beside, behind = (np.median(t) for t in times)
+    print('%d x %d x %d x %d -> %d: beside %.3f ms, behind %.3f ms' % (n, hw, hw, ci, co, beside, behind), flush=True)
+    assert beside < 0.88 * behind
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize('name', ['dense', 'images', 'batches'])
 def test_the_option_that_keeps_steps_whole(name):
     program, draw, want = build(name, 'f32')
