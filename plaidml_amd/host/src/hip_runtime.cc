@@ -686,9 +686,10 @@ class HipExecutable final : public Executable {
     };
     try {
       const bool record_now = graphable_ && overlapped_runs_++ >= 2;
-      size_t turn = 0, last_up = 0, sent = 0;
+      size_t turn = 0, sent = 0, last_up = 0;  // last_up: of the segments, whose operands go up by copy engine
       for (size_t k = 0; k < segments_.size(); ++k)
-        if (!segments_[k].needs.empty()) last_up = k;
+        for (const Range& r : segments_[k].needs)
+          if (r.bytes > kKernelCopy) last_up = k;
       auto send = [&](Segment& seg) {
         if (seg.yields.empty()) return;
         Spans down;
@@ -708,7 +709,7 @@ class HipExecutable final : public Executable {
       };
       // Sends down what the first `launched` segments yield: of those that are done, or (all) of all of them.  A copy down that waits
       // for its launches holds up whatever is queued behind it on its copy engine, and which engine a copy up gets depends on the
-      // process's other streams: a copy down is queued once its launches are done, or behind the last copy up.  (Both gradients of
+      // process's other streams: a copy down is queued once its launches are done, or behind the last copy up that goes by engine.  (Both gradients of
       // 10 x 49 x 49 x 117 (*) 5 x 5 x 26 with torch's streams in the process: 855 us with the second operand up behind the first
       // result, 836 on one stream, 589 now; on engines of their own 612 and 586.)
       auto send_down = [&](size_t launched, bool all) {
@@ -743,6 +744,7 @@ class HipExecutable final : public Executable {
             send_down(k, false);
           }
         }
+        send_down(k, k >= last_up);
         up.issue(up_stream_, nullptr, false);
         if (!seg.needs.empty()) {
           hipCheck(pml_hip_event_record(seg.up, up_stream_), "event record");
