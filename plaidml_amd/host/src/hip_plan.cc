@@ -55,6 +55,7 @@ std::shared_ptr<Plan> Planner::run() {
   // (a tile or path that was asked for, by option or for one step, was asked for a product of its own and for the whole step)
   if (opt_.fuse && opt_.specialise) chainProducts();
   if (opt_.fuse && opt_.specialise && opt_.overlap && opt_.tile.empty() && opt_.conv.empty()) sliceSteps();
+  if (opt_.overlap) separateRuns();
   return plan_;
 }
 
@@ -260,6 +261,7 @@ std::string Plan::dump() const {
   ss << "hip plan: " << steps.size() << " launches, " << buffers.size() << " buffers\n";
   for (size_t i = 0; i < steps.size(); ++i) ss << "  [" << i << "] " << steps[i].text << steps[i].schedule << "\n";
   if (slices > 1) ss << "  steps 0 to " << sliced.size() - 1 << " in " << slices << " parts of the leading dimension\n";
+  for (size_t k = 0; k < runs.size(); ++k) ss << (k > 0 ? ", " : runs.size() > 1 ? "  copies go beside launches ahead of steps " : "  copies go beside launches ahead of step ") << runs[k] << (k + 1 == runs.size() ? "\n" : "");
   return ss.str();
 }
 

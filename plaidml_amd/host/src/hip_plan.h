@@ -80,7 +80,9 @@ struct Plan {
   std::vector<int> input_buffers;   // buffer id per program input
   std::vector<int> output_buffers;  // buffer id per program output
   bool graph = true;                // the runtime may replay the launches of a run as one recorded graph
-  bool overlap = true;              // copies may go beside launches
+  // Steps that begin a run of launches of their own, so that copies up and down go beside the launches before and behind them
+  // (Planner::separateRuns); the parts of the sliced steps are such runs anyhow.
+  std::vector<size_t> runs;
   // The first sliced.size() steps run `slices` times over, on equal parts of the leading dimension (the last one shorter,
   // sliced_last): `steps` says what they are on all of it.  part_bytes: of a part of each buffer that lies part behind part, 0
   // for the others (Planner::sliceSteps).

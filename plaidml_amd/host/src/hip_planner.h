@@ -151,7 +151,6 @@ class Planner {
  public:
   Planner(Program* program, const Options& options) : prog_(program), opt_(options), plan_(std::make_shared<Plan>()) {
     plan_->graph = options.graph;
-    plan_->overlap = options.overlap;
   }
 
   std::shared_ptr<Plan> run();
@@ -167,6 +166,7 @@ class Planner {
   void fusePoolIntoConv();
   void chainProducts();
   void sliceSteps();
+  void separateRuns();
   void pruneDeadSteps();
 
  private:

@@ -537,9 +537,6 @@ class HipExecutable final : public Executable {
   std::vector<Launch> order_;  // of all the segments
   pml_hip_stream up_stream_ = nullptr, down_stream_ = nullptr;
   int overlapped_runs_ = 0;
-  // A wait between the queues and a graph of its own cost 20 to 25 us, the link takes 75 us for this many bytes: two 1.6 MB
-  // operands of a product of their own segments took 301 us, in one 275; two of 12.8 MB around a gradient 1070, 1170 in one.
-  static constexpr size_t kWorthASegment = 4 << 20;
 
   void findSegments() {
     const Plan& p = *plan_;
@@ -582,26 +579,17 @@ class HipExecutable final : public Executable {
       }
       segments_.push_back(std::move(seg));
     }
-    bool fresh = true;  // (also behind parts)
     for (size_t i = n; i < p.steps.size(); ++i) {
-      std::vector<Range> needs;
-      size_t coming = 0, going = 0;
+      if (segments_.empty() || std::count(p.runs.begin(), p.runs.end(), i)) segments_.emplace_back();
+      Segment& seg = segments_.back();
+      seg.launches.push_back({i, -1});
       for (size_t in : reads(p.steps[i]))
         if (!up[in]) {
           up[in] = 1;
-          needs.push_back({in, 0, p.buffers[p.input_buffers[in]].bytes});
-          coming += needs.back().bytes;
+          seg.needs.push_back({in, 0, p.buffers[p.input_buffers[in]].bytes});
         }
-      if (segments_.empty() || (p.overlap && (fresh || coming >= kWorthASegment))) segments_.emplace_back();
-      Segment& seg = segments_.back();
-      seg.launches.push_back({i, -1});
-      seg.needs.insert(seg.needs.end(), needs.begin(), needs.end());
       for (size_t o = 0; o < p.output_buffers.size(); ++o)
-        if (writer[p.output_buffers[o]] == static_cast<int>(i)) {
-          seg.yields.push_back({o, 0, p.buffers[p.output_buffers[o]].bytes});
-          going += seg.yields.back().bytes;
-        }
-      fresh = going >= kWorthASegment;
+        if (writer[p.output_buffers[o]] == static_cast<int>(i)) seg.yields.push_back({o, 0, p.buffers[p.output_buffers[o]].bytes});
     }
     for (const Segment& seg : segments_) order_.insert(order_.end(), seg.launches.begin(), seg.launches.end());
     if (segments_.empty()) return;
@@ -718,8 +706,8 @@ class HipExecutable final : public Executable {
       };
       // Sends down what the first `launched` segments yield: of those that are done, or (all) of all of them.  A copy down that waits
       // for its launches holds up whatever is queued behind it on its copy engine, and which engine a copy up gets depends on the
-      // process's other streams: a copy down is queued once its launches are done, or behind the last copy up that goes by engine.  (Both gradients of
-      // 10 x 49 x 49 x 117 (*) 5 x 5 x 26 with torch's streams in the process: 855 us with the second operand up behind the first
+      // process's other streams: a copy down is queued once its launches are done, or behind the last copy up that goes by
+      // engine.  (Both gradients of 10 x 49 x 49 x 117 (*) 5 x 5 x 26 with torch's streams in the process: 855 us with the second operand up behind the first
       // result, 836 on one stream, 589 now; on engines of their own 612 and 586.)
       auto send_down = [&](size_t launched, bool all) {
         for (; sent < launched && (all || pml_hip_event_done(segments_[sent].done)); ++sent) send(segments_[sent]);

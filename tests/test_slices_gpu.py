@@ -57,6 +57,36 @@ def batches(dt, n, r=96):
 CASES = {'dense': (dense, 3571), 'dense even': (dense, 4096), 'images': (images, 21), 'rows': (rows, 5003), 'batches': (batches, 401)}
 
 
+def runs_from(program, target=''):
+    program.compile(target)
+    m = re.search(r'beside launches ahead of steps? ([0-9, ]+)', dict(program.passes)['hip-plan'])
+    return [int(i) for i in m.group(1).split(',')] if m else []
+
+
+def test_which_launches_copies_go_beside():
+    """Long results are followed by a run of launches of its own, long operands where there is enough ahead of them to hide it."""
+    i, j, k = P.TensorIndexes(3)
+
+    def result(m):  # of m KB
+        A, W, V = (P.Placeholder(DT['f32'], s) for s in ([m, 64], [64, 256], [256, 8]))
+        y = Pop.dot(A, W)
+        return P.Program('result', [A, W, V], [y, Pop.dot(y, V)])
+
+    def operand(m, launches):  # of m KB behind so many products
+        A, B = P.Placeholder(DT['f32'], [128, 128]), P.Placeholder(DT['f32'], [m, 256])
+        x = A
+        for _ in range(launches):
+            x = Pop.relu(Pop.dot(x, A) * (1 / 64))
+        return P.Program('operand', [A, B], [P.Contraction().outShape(256, 128).outAccess(i, j).sum(B[k, i] * Pop.dot(P.Constant(whole(np.random.default_rng(1), m, 128), DT['f32']), x)[k, j]).build()])
+    assert runs_from(result(4095)) == [] and runs_from(result(4096)) == [1] and runs_from(result(4096), 'hip{overlap=0}') == []
+    # (a launch is taken to take 6 us, 60 have to lie ahead)
+    assert runs_from(operand(8192, 2)) == [] and runs_from(operand(8192, 12)) == [13] and runs_from(operand(4095, 12)) == []
+    A, B, V = (P.Placeholder(DT['f32'], s) for s in ([23, 17, 128], [23, 370, 128], [23, 370, 128]))
+    x, i, j, k = P.TensorIndexes(4)
+    S = Pop.softmax(P.Contraction().outShape(23, 17, 370).outAccess(x, i, j).sum(A[x, i, k] * B[x, j, k]).build(), -1)
+    assert runs_from(P.Program('batched', [A, B, V], [P.Contraction().outShape(23, 17, 128).outAccess(x, i, k).sum(S[x, i, j] * V[x, j, k]).build()])) == []
+
+
 def build(name, dt, scale=1):
     fn, size = CASES[name]
     return fn(dt, size * scale)
