@@ -102,12 +102,14 @@ int pml_hip_event_done(pml_hip_event e); /* 1: what was queued ahead of its last
 int pml_hip_stream_wait_event(pml_hip_stream s, pml_hip_event e); /* what is queued on s from here on waits for e */
 int pml_hip_event_elapsed_ms(pml_hip_event start, pml_hip_event stop, float* ms);
 
-/* Replay of a fixed sequence of launches as one HIP graph: what the reference gets from jitting a whole program into
+/* Replay of a fixed sequence of launches, recorded once: what the reference gets from jitting a whole program into
  * one function (pmlc/rt/jit_executable.cc:484-490 calls it once per run) -- here a run is many launches, and at small
  * batch the launches cost more than the kernels.  Between _begin and _end every launch on `s` (a stream made by
  * pml_hip_stream_create, never NULL) is recorded instead of run; every *_invoke of this library may be recorded once
  * it has run at least once on the same plan (first runs may allocate).  _end returns the replayable graph, or fails
- * (and leaves `s` usable) if something could not be recorded.  Pointers are baked in: replay with the same buffers. */
+ * (and leaves `s` usable) if something could not be recorded.  Pointers are baked in: replay with the same buffers.
+ * A recording of up to 64 kernels is replayed by launching them one by one with the recorded arguments, a longer one as
+ * one HIP graph (plaidml_amd/csrc/replay.hip). */
 typedef void* pml_hip_graph;
 int pml_hip_capture_begin(pml_hip_stream s);
 int pml_hip_capture_end(pml_hip_stream s, pml_hip_graph* graph);

@@ -437,4 +437,10 @@ struct PoolArgs {
 };
 hipError_t pool2d_launch(const PoolArgs& a, hipStream_t s);
 
+// a recorded sequence of launches (replay.hip): made from a recording that it owns from then on
+struct Replay;
+hipError_t replay_create(hipGraph_t recorded, Replay** out);
+hipError_t replay_launch(const Replay& r, hipStream_t s);
+void replay_destroy(Replay* r);
+
 }  // namespace pml

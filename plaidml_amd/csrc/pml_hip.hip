@@ -875,19 +875,18 @@ int pml_hip_capture_end(pml_hip_stream s, pml_hip_graph* graph) {
     (void)hipGetLastError();
     return fail(std::string("hipStreamEndCapture: ") + hipGetErrorString(e));
   }
-  hipGraphExec_t exec = nullptr;
-  const hipError_t ei = hipGraphInstantiate(&exec, g, nullptr, nullptr, 0);
-  (void)hipGraphDestroy(g);
-  if (check(ei, "hipGraphInstantiate")) return 1;
-  *graph = (pml_hip_graph)exec;
+  Replay* r = nullptr;
+  if (check(replay_create(g, &r), "hipGraphInstantiate")) return 1;
+  *graph = (pml_hip_graph)r;
   return 0;
 }
 int pml_hip_graph_launch(pml_hip_graph graph, pml_hip_stream s) {
   if (!graph) return fail("pml_hip_graph_launch: null graph");
-  return check(hipGraphLaunch((hipGraphExec_t)graph, (hipStream_t)s), "hipGraphLaunch");
+  return check(replay_launch(*(const Replay*)graph, (hipStream_t)s), "hipGraphLaunch");
 }
 int pml_hip_graph_destroy(pml_hip_graph graph) {
-  return graph ? check(hipGraphExecDestroy((hipGraphExec_t)graph), "hipGraphExecDestroy") : 0;
+  replay_destroy((Replay*)graph);
+  return 0;
 }
 int pml_hip_event_destroy(pml_hip_event e) { return check(hipEventDestroy((hipEvent_t)e), "hipEventDestroy"); }
 int pml_hip_event_record(pml_hip_event e, pml_hip_stream s) {
