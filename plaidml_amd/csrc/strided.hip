@@ -163,7 +163,7 @@ __device__ __forceinline__ void leave_outside_taps_out(const StridedArgs& p, boo
 
 // One operand's share of a workgroup: T rows (of m or n) by one slab of K.
 //   fetch(k0): the slab's values of this thread, into registers;   put(lds): from there into the slab's LDS buffer
-template <bool BF, int MODE, int T>
+template <bool BF, int MODE, int T, bool FLAT>
 struct Side {
   static constexpr int BK = BF ? 64 : 32;
   static constexpr int kPitch = BF ? 0 : (MODE == ROWS_K ? T + 1 : T + 4);  // fp32: words per K-row
@@ -173,123 +173,172 @@ struct Side {
   const char* base;     // the tile's first row, K-index 0 (ROWS_CONV: the image)
   int64_t ms, ks;       // element strides
   int64_t live;         // rows of the tile that exist
+  int64_t extent;       // elements from the base up to and with the operand's last one that this tile may read (contiguous rows)
   bool whole;           // every row exists and is contiguous where the layout says so
+  bool cut;             // the slab in the registers has runs that clear() has to clear
+  int keep[BF && MODE != ROWS_K ? kBlocks * 4 : kPasses];  // their first value that stays, and how many do
   uint32_t regs[BF ? (MODE == ROWS_K ? kPasses * 4 : kBlocks * 8) : kPasses * 4];
 
   __device__ __forceinline__ static int key(int m) { return (m ^ (m >> 2)) & 7; }
 
-  // `n` values from element `at` on, those at or past `live_n` as zeros; st: their element stride
-  template <int N>
-  __device__ __forceinline__ void gather(uint32_t* to, int64_t at, int64_t live_n, int64_t st) {
-    if constexpr (BF) {
-      uint16_t h[N];
-#pragma unroll
-      for (int e = 0; e < N; ++e) h[e] = e < live_n ? ((const uint16_t*)base)[at + e * st] : (uint16_t)0;
-      __builtin_memcpy(to, h, 2 * N);
-    } else {
-#pragma unroll
-      for (int e = 0; e < N; ++e) to[e] = e < live_n ? ((const uint32_t*)base)[at + e * st] : 0u;
-    }
-  }
-  template <int N>
-  __device__ __forceinline__ void straight(uint32_t* to, int64_t at) {
-    constexpr int W = N * (BF ? 2 : 4) / 4;
-    const Words<W> v = load_words<W>(base + at * (BF ? 2 : 4));
-#pragma unroll
-    for (int e = 0; e < W; ++e) to[e] = v.w[e];
-  }
-  template <int N>
-  __device__ __forceinline__ void checked(uint32_t* to, int64_t at, int64_t live_n, int64_t st) {
-    if (live_n >= N && st == 1)
-      straight<N>(to, at);
-    else
-      gather<N>(to, at, live_n, st);
-  }
-
-  // N neighbouring values of pixel k's window row, the first at column j0 of the tile
-  template <int N>
-  __device__ __forceinline__ void conv_row(const StridedArgs& p, uint32_t* to, int64_t k, int64_t k_end, int j0) {
-    constexpr int W = N * (BF ? 2 : 4) / 4;
-#pragma unroll
-    for (int e = 0; e < W; ++e) to[e] = 0;
-    if (k >= k_end) return;
-    const unsigned pix = (unsigned)k;
-    const unsigned img = fast_div(pix, p.div_per_magic, p.div_per_shift);
-    const unsigned rem = pix - img * (unsigned)(p.OH * p.OW);
+  // ROWS_CONV: where a thread's pixels lie, counted on from slab to slab (two divisions a row of every slab before)
+  struct Pixel {
+    int img, oy, ox;
+  };
+  Pixel px, slab_step, run_step;  // this thread's first pixel; from slab to slab; from one of its runs (bf16: of four) to the next
+  __device__ __forceinline__ static Pixel pixel(const StridedArgs& p, unsigned k) {
+    const unsigned img = fast_div(k, p.div_per_magic, p.div_per_shift), rem = k - img * (unsigned)(p.OH * p.OW);
     const unsigned oy = fast_div(rem, p.div_ow_magic, p.div_ow_shift);
-    const int ox = (int)(rem - oy * (unsigned)p.OW);
-    const int iy = (int)oy * p.SH + (int)ms * p.DH - p.PH;
-    if (iy < 0 || iy >= p.H) return;
-    const int first = (ox * p.SW - p.PW) * p.CI + (int)ks + j0;  // (ks: the tile's first column inside the window row)
-    const int row_elems = p.W * p.CI;
-    const int64_t at = ((int64_t)img * p.H + iy) * row_elems + first;
-    if (j0 + N <= live && first >= 0 && first + N <= row_elems) {
-      straight<N>(to, at);
-    } else {
-      if constexpr (BF) {
-        uint16_t h[N];
-#pragma unroll
-        for (int e = 0; e < N; ++e)
-          h[e] = (j0 + e < live && first + e >= 0 && first + e < row_elems) ? ((const uint16_t*)base)[at + e] : (uint16_t)0;
-        __builtin_memcpy(to, h, 2 * N);
-      } else {
-#pragma unroll
-        for (int e = 0; e < N; ++e)
-          to[e] = (j0 + e < live && first + e >= 0 && first + e < row_elems) ? ((const uint32_t*)base)[at + e] : 0u;
-      }
-    }
+    return {(int)img, (int)oy, (int)(rem - oy * (unsigned)p.OW)};
+  }
+  __device__ __forceinline__ static Pixel ahead(const StridedArgs& p, Pixel a, int img, int oy, int ox) {
+    a.ox += ox;
+    const bool row = a.ox >= p.OW;
+    a.ox -= row ? p.OW : 0;
+    a.oy += oy + (row ? 1 : 0);
+    const bool image = a.oy >= p.OH;
+    a.oy -= image ? p.OH : 0;
+    a.img += img + (image ? 1 : 0);
+    return a;
+  }
+  static constexpr int kPer = T / 4;                                             // runs of four columns
+  static constexpr int kRowStep = BF ? 4 * kThreads / kPer : kThreads / kPer;  // between a thread's rows (bf16: of its blocks of four)
+  __device__ __forceinline__ void start(const StridedArgs& p, int64_t k_begin, int tid) {
+    px = pixel(p, (unsigned)k_begin + (unsigned)(tid / kPer) * (BF ? 4 : 1));
+    slab_step = pixel(p, BK);
+    run_step = pixel(p, BF ? kRowStep - 3 : kRowStep);  // (bf16: from the last row of a block of four)
   }
 
-  __device__ __forceinline__ void fetch(const StridedArgs& p, int64_t k0, int64_t k_end, int tid) {
-    const bool full = whole && k0 + BK <= k_end;  // uniform: no lane checks anything
+  // A thread's runs of neighbouring values: where run r of the slab at k0 begins, and which of its values belong to it.
+  static constexpr int kVals = BF && MODE == ROWS_K ? 8 : 4, kWords = kVals * (BF ? 2 : 4) / 4;
+  static constexpr int kRuns = BF && MODE != ROWS_K ? 4 * kBlocks : kPasses;
+  struct Run {
+    int64_t at;
+    int lo, hi;
+  };
+  __device__ __forceinline__ static int row_of(int r, int tid) {  // in the slab (ROWS_K: in the tile)
+    if constexpr (MODE == ROWS_K) return tid / 8 + 32 * r;
+    if constexpr (BF) return (tid / kPer) * 4 + (r / 4) * kRowStep + r % 4;
+    return tid / kPer + r * kRowStep;
+  }
+  __device__ __forceinline__ Run run(const StridedArgs& p, int r, int64_t k0, int64_t k_end, int tid, const Pixel& pix) const {
+    const int row = row_of(r, tid);
+    Run at;
+    at.lo = 0;
+    int64_t last;
     if constexpr (MODE == ROWS_K) {
-      constexpr int N = BF ? 8 : 4;
-#pragma unroll
-      for (int i = 0; i < kPasses; ++i) {
-        const int row = tid / 8 + 32 * i, kq = (tid % 8) * N;
-        const int64_t at = row * ms + (k0 + kq) * ks;
-        if (full)
-          straight<N>(&regs[4 * i], at);
-        else
-          checked<N>(&regs[4 * i], at, row < live ? k_end - k0 - kq : 0, ks);
-      }
-    } else if constexpr (!BF) {
-      constexpr int PER = T / 4;
-#pragma unroll
-      for (int i = 0; i < kPasses; ++i) {
-        const int c = tid + kThreads * i, k = c / PER, m4 = (c % PER) * 4;
-        if constexpr (MODE == ROWS_CONV) {
-          conv_row<4>(p, &regs[4 * i], k0 + k, k_end, m4);
-        } else {
-          const int64_t at = (k0 + k) * ks + m4 * ms;
-          if (full)
-            straight<4>(&regs[4 * i], at);
-          else
-            checked<4>(&regs[4 * i], at, k0 + k < k_end ? live - m4 : 0, ms);
-        }
-      }
+      const int kq = (tid % 8) * kVals;
+      at.at = row * ms + (k0 + kq) * ks;
+      last = row < live ? k_end - k0 - kq : 0;
+    } else if constexpr (MODE == ROWS_M) {
+      const int m4 = (tid % kPer) * 4;
+      at.at = (k0 + row) * ks + m4 * ms;
+      last = k0 + row < k_end ? live - m4 : 0;
     } else {
-      constexpr int PER = T / 4;  // blocks of four columns
+      // the values of the pixel's window row from column j0 of the tile on (ks: the tile's first column inside the window row)
+      const int j0 = (tid % kPer) * 4, iy = pix.oy * p.SH + (int)ms * p.DH - p.PH, row_elems = p.W * p.CI;
+      const int first = (pix.ox * p.SW - p.PW) * p.CI + (int)ks + j0;
+      at.at = ((int64_t)pix.img * p.H + iy) * row_elems + first;
+      at.lo = first < 0 ? -first : 0;
+      const int end = row_elems - first < (int)live - j0 ? row_elems - first : (int)live - j0;
+      last = k0 + row < k_end && iy >= 0 && iy < p.H ? end : 0;
+    }
+    at.hi = (int)(last < 0 ? 0 : last > kVals ? kVals : last);
+    return at;
+  }
+
+  // a run's values `apart` elements from each other
+  __device__ __forceinline__ void gather(uint32_t* to, int64_t at, int lo, int hi, int64_t apart) const {
+    if constexpr (BF) {
+      uint16_t h[kVals];
 #pragma unroll
-      for (int i = 0; i < kBlocks; ++i) {
-        const int c = tid + kThreads * i, k4 = (c / PER) * 4, m4 = (c % PER) * 4;
+      for (int e = 0; e < kVals; ++e) h[e] = e >= lo && e < hi ? ((const uint16_t*)base)[at + e * apart] : (uint16_t)0;
+      __builtin_memcpy(to, h, sizeof h);
+    } else {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          if constexpr (MODE == ROWS_CONV) {
-            conv_row<4>(p, &regs[8 * i + 2 * e], k0 + k4 + e, k_end, m4);
-          } else {
-            const int64_t at = (k0 + k4 + e) * ks + m4 * ms;
-            if (full)
-              straight<4>(&regs[8 * i + 2 * e], at);
-            else
-              checked<4>(&regs[8 * i + 2 * e], at, k0 + k4 + e < k_end ? live - m4 : 0, ms);
-          }
-        }
+      for (int e = 0; e < kVals; ++e) {
+        to[e] = e >= lo && e < hi ? ((const uint32_t*)base)[at + e * apart] : 0u;
+      }
+    }
+  }
+  __device__ __forceinline__ void straight(uint32_t* to, int64_t at) const {
+    const Words<kWords> v = load_words<kWords>(base + at * (BF ? 2 : 4));
+#pragma unroll
+    for (int e = 0; e < kWords; ++e) to[e] = v.w[e];
+  }
+
+  // Where nothing is cut and rows are contiguous the loads go out as they are.  FLAT (filter gradients, where a slab's pixels
+  // always have cut window rows among them): elsewhere as well, and put() clears what does not belong to the operand.  With a
+  // branch per run, and per value where a run is cut, the loads of a slab waited for each other (567 pixels of 3 x 45 window
+  // values x 20, bf16: 19.6 -> 12.4 us, 154154 of 3 x 51 x 38: 58.6 -> 35.6).  Only where a run sticks out of the operand's
+  // `extent` elements is it read value by value then.  Two slabs on their way instead of one take 219 registers and 46.6 us.  (It takes 30 registers more, which products have no
+  // use for.)
+  __device__ __forceinline__ void fetch(const StridedArgs& p, int64_t k0, int64_t k_end, int tid) {
+    Pixel pix{0, 0, 0};
+    if constexpr (MODE == ROWS_CONV) {
+      pix = px;
+      px = ahead(p, px, slab_step.img, slab_step.oy, slab_step.ox);
+    }
+    const bool full = MODE != ROWS_CONV && whole && k0 + BK <= k_end;  // uniform: no lane checks anything
+    const int64_t apart = MODE == ROWS_K ? ks : MODE == ROWS_M ? ms : 1;
+    cut = false;
+    if (full || !FLAT) {
+#pragma unroll
+      for (int r = 0; r < kRuns; ++r) {
+        const Run at = run(p, r, k0, k_end, tid, pix);
+        if (full || (at.hi == kVals && apart == 1))
+          straight(&regs[kWords * r], at.at);
+        else
+          gather(&regs[kWords * r], at.at, at.lo, at.hi, apart);
+      }
+      return;
+    }
+    Run runs[kRuns];
+    bool out = false;
+#pragma unroll
+    for (int r = 0; r < kRuns; ++r) {
+      runs[r] = run(p, r, k0, k_end, tid, pix);
+      if constexpr (MODE == ROWS_CONV) {
+        if (BF && r % 4 != 3)
+          pix = ahead(p, pix, 0, 0, 1);
+        else if (r + 1 < kRuns)
+          pix = ahead(p, pix, run_step.img, run_step.oy, run_step.ox);
+      }
+      const bool any = runs[r].hi > runs[r].lo;
+      keep[r] = any ? runs[r].lo | (runs[r].hi - runs[r].lo) << 8 : 0;
+      out = out || (any && (runs[r].at < 0 || runs[r].at + kVals > extent));
+    }
+    cut = extent >= kVals && apart == 1 && __ballot(out) == 0;
+    // (nothing but the runs' values differs between the two ways: a store that both end with goes through scratch otherwise)
+    if (cut) {
+#pragma unroll
+      for (int r = 0; r < kRuns; ++r) straight(&regs[kWords * r], runs[r].hi > runs[r].lo ? runs[r].at : 0);
+    } else {
+#pragma unroll
+      for (int r = 0; r < kRuns; ++r) gather(&regs[kWords * r], runs[r].at, runs[r].lo, runs[r].hi, apart);
+    }
+  }
+
+  // clears the values of a slab's runs that do not belong to the operand
+  __device__ __forceinline__ void clear() {
+    if (!FLAT || !cut) return;
+#pragma unroll
+    for (int r = 0; r < kRuns; ++r) {
+      const int lo = keep[r] & 255;
+      const unsigned count = (unsigned)keep[r] >> 8;
+#pragma unroll
+      for (int w = 0; w < kWords; ++w) {
+        uint32_t& v = regs[kWords * r + w];
+        if constexpr (BF)
+          v &= ((unsigned)(2 * w - lo) < count ? 0xffffu : 0u) | ((unsigned)(2 * w + 1 - lo) < count ? 0xffff0000u : 0u);
+        else
+          v = (unsigned)(w - lo) < count ? v : 0u;
       }
     }
   }
 
-  __device__ __forceinline__ void put(char* lds, int tid) const {
+  __device__ __forceinline__ void put(char* lds, int tid) {
+    clear();
     if constexpr (BF && MODE == ROWS_K) {
 #pragma unroll
       for (int i = 0; i < kPasses; ++i) {
@@ -336,8 +385,8 @@ __global__ __launch_bounds__(kThreads) void strided_kernel(StridedArgs p_by_valu
   // (read where the dispatcher put it: indexing a by-value copy would move the copy to scratch memory)
   const StridedArgs& p = *(const StridedArgs*)(const __attribute__((address_space(4))) void*)__builtin_amdgcn_kernarg_segment_ptr();
   constexpr int TM = 64 * MI, TN = 64 * NI, ES = BF ? 2 : 4;
-  typedef Side<BF, AMODE, TM> side_a;
-  typedef Side<BF, BMODE, TN> side_b;
+  typedef Side<BF, AMODE, TM, AMODE == ROWS_CONV> side_a;
+  typedef Side<BF, BMODE, TN, AMODE == ROWS_CONV> side_b;
   constexpr int BK = side_a::BK, kStage = side_a::kBytes + side_b::kBytes;
   extern __shared__ __attribute__((aligned(16))) char smem[];
 
@@ -371,6 +420,7 @@ __global__ __launch_bounds__(kThreads) void strided_kernel(StridedArgs p_by_valu
     sa.ms = tap;  // (the filter row)
     sa.live = m_rows;
     sa.whole = false;
+    sa.extent = (int64_t)fast_div((unsigned)p.K, p.div_per_magic, p.div_per_shift) * p.H * p.W * p.CI;
   } else {
     m0 = (int64_t)tm * TM;
     m_rows = p.M - m0 < TM ? p.M - m0 : TM;
@@ -379,6 +429,7 @@ __global__ __launch_bounds__(kThreads) void strided_kernel(StridedArgs p_by_valu
     sa.ks = p.a_ks;
     sa.live = m_rows;
     sa.whole = m_rows == TM && (AMODE == ROWS_K ? p.a_ks : p.a_ms) == 1;
+    sa.extent = (m_rows - 1) * p.a_ms + (p.K - 1) * p.a_ks + 1;
   }
   const int64_t n0 = (int64_t)tn * TN;
   const int64_t n_cols = p.N - n0 < TN ? p.N - n0 : TN;
@@ -387,6 +438,7 @@ __global__ __launch_bounds__(kThreads) void strided_kernel(StridedArgs p_by_valu
   sb.ks = p.b_ks;
   sb.live = n_cols;
   sb.whole = n_cols == TN && (BMODE == ROWS_K ? p.b_ks : p.b_ns) == 1;
+  sb.extent = (n_cols - 1) * p.b_ns + (p.K - 1) * p.b_ks + 1;
 
   const int64_t k_begin = (int64_t)blockIdx.y * p.k_per_split;
   const int64_t k_end = k_begin + p.k_per_split < p.K ? k_begin + p.k_per_split : p.K;
@@ -399,6 +451,7 @@ __global__ __launch_bounds__(kThreads) void strided_kernel(StridedArgs p_by_valu
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
 
+  if constexpr (AMODE == ROWS_CONV) sa.start(p, k_begin, tid);
   sa.fetch(p, k_begin, k_end, tid);
   sb.fetch(p, k_begin, k_end, tid);
   sa.put(smem, tid);
@@ -502,26 +555,43 @@ __global__ __launch_bounds__(kThreads) void strided_kernel(StridedArgs p_by_valu
   }
 }
 
-// Adds the partial results up in split order and runs the tail: a thread per four columns of a row.
+// Adds the partial results up and runs the tail: PARTS threads per four columns of a row, each with a run of the splits in their
+// order, whose sums are added up in that order.  (What bounds it is a thread's chain of loads, eight at a time: 153 x 38 results
+// of 241 splits 20.2 us with one thread each, 5.4 with sixteen.)
+template <int PARTS>
 __global__ __launch_bounds__(256) void strided_reduce_kernel(StridedArgs p_by_value) {
   const StridedArgs& p = *(const StridedArgs*)(const __attribute__((address_space(4))) void*)__builtin_amdgcn_kernarg_segment_ptr();
+  constexpr int G = 256 / PARTS;
+  __shared__ f32x4_t sums[PARTS > 1 ? 256 : 1];
   const int64_t per_row = p.ws_pitch / 4;
-  int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  const bool conv = p.row_cols != 0, mine = g < p.ws_rows * per_row;
+  int64_t g = (int64_t)blockIdx.x * G + threadIdx.x % G;
+  const int part = threadIdx.x / G, per = (p.splits + PARTS - 1) / PARTS, first = part * per;
+  const int behind = first + per < p.splits ? first + per : p.splits;
+  const bool conv = p.row_cols != 0;
+  bool mine = g < p.ws_rows * per_row;
   if (!mine) {
-    if (!conv) return;
+    if (!conv && PARTS == 1) return;
     g = 0;  // (every lane stays: see leave_outside_taps_out)
   }
   const int64_t row = g / per_row, n = (g - row * per_row) * 4;
   const f32x4_t* at = (const f32x4_t*)(p.ws + row * p.ws_pitch + n);
   const int64_t step = p.ws_rows * p.ws_pitch / 4;
   f32x4_t sum = {0.f, 0.f, 0.f, 0.f};
-  for (int s = 0; s < p.splits; s += 8) {
+  for (int s = first; s < behind; s += 8) {
     f32x4_t got[8];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) got[u] = s + u < p.splits ? at[(s + u) * step] : f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int u = 0; u < 8; ++u) got[u] = s + u < behind ? at[(s + u) * step] : f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int u = 0; u < 8; ++u) sum += got[u];
+  }
+  if constexpr (PARTS > 1) {
+    sums[threadIdx.x] = sum;
+    __syncthreads();
+    if (threadIdx.x >= (G + 63) / 64 * 64) return;  // (whole wavefronts)
+    mine = mine && part == 0;
+    if (!mine && !conv) return;
+#pragma unroll
+    for (int q = 1; q < PARTS; ++q) sum += sums[q * G + threadIdx.x % G];
   }
   float v[4] = {sum[0], sum[1], sum[2], sum[3]};
   int64_t b = row / p.M, c_at = (row - b * p.M) * p.c_ms;
@@ -540,7 +610,7 @@ __global__ __launch_bounds__(256) void strided_reduce_kernel(StridedArgs p_by_va
 
 template <bool BF, int AMODE, int BMODE, int MI, int NI>
 hipError_t launch_tile(const StridedArgs& a, hipStream_t s) {
-  const size_t lds = std::max<size_t>(2 * (Side<BF, AMODE, 64 * MI>::kBytes + Side<BF, BMODE, 64 * NI>::kBytes), 64 * MI * (64 * NI + 4) * 4);
+  const size_t lds = std::max<size_t>(2 * (Side<BF, AMODE, 64 * MI, AMODE == ROWS_CONV>::kBytes + Side<BF, BMODE, 64 * NI, AMODE == ROWS_CONV>::kBytes), 64 * MI * (64 * NI + 4) * 4);
   auto kern = strided_kernel<BF, AMODE, BMODE, MI, NI>;
   static DynamicLdsLimit limit;
   if (hipError_t e = limit.ensure((const void*)kern, lds); e != hipSuccess) return e;
@@ -966,7 +1036,9 @@ hipError_t product_direct_launch(const StridedArgs& a, bool bf, int rows, hipStr
 // operand traffic per result) and covers at most a third more results than 64 x 64, which otherwise is the tile (1000 of
 // 64 x 64 with K = 64, fp32: 43.7 us with tiles of 128, three quarters of them empty, 18.7 with tiles of 64; 1000 of 48 x 48,
 // K = 33, bf16: 44.1 and 18.4); K is split when the tiles alone leave CUs idle, into runs of at least
-// four slabs, for about three workgroups per CU (their LDS fits four times into one).
+// four slabs, for about three workgroups per CU (their LDS fits four times into one).  A filter gradient's slab takes as long as
+// its loads: runs of two slabs and more (567 pixels of 3 x 45 x 20 in bf16 12.4 -> 9.5 us, 2116 of 3 x 60 x 18 in fp32 12.4 -> 9.2),
+// and in fp32, whose workgroups fit four times into a CU's registers, four per CU (50176 of 3 x 192 x 64 64.5 -> 61.1).
 void strided_plan(StridedArgs* a, bool bf, bool conv, int n_cus, int* mi) {
   int64_t batches = 1;
   for (int d = 0; d < a->n_batch; ++d) batches *= a->batch[d];
@@ -986,7 +1058,7 @@ void strided_plan(StridedArgs* a, bool bf, bool conv, int n_cus, int* mi) {
   a->ws_pitch = (a->N + 3) / 4 * 4;
   const int64_t have = tiles(t);
   if (have < n_cus && slabs >= 8) {
-    int64_t want = std::min<int64_t>((3 * n_cus + have - 1) / have, slabs / 4);
+    int64_t want = std::min<int64_t>(conv && !bf ? 4 * n_cus / have : (3 * n_cus + have - 1) / have, slabs / (conv ? 2 : 4));
     // the partial results: at most 256 MiB of them
     want = std::min<int64_t>(want, ((int64_t)256 << 20) / std::max<int64_t>(1, a->ws_rows * a->ws_pitch * 4));
     if (want >= 2) {
@@ -1008,9 +1080,15 @@ hipError_t strided_launch(const StridedArgs& a, bool bf, bool conv, int mi, hipS
   else
     e = mi == 2 ? launch_modes<false, 2>(a, amode, bmode, s) : launch_modes<false, 1>(a, amode, bmode, s);
   if (e != hipSuccess || a.splits == 1) return e;
-  const int64_t groups = a.ws_rows * (a.ws_pitch / 4), blocks = (groups + 255) / 256;
+  // threads per four results: so many that a thread's splits are one round of loads, while workgroups are few
+  const int64_t groups = a.ws_rows * (a.ws_pitch / 4);
+  int parts = 1;
+  while (parts < 16 && a.splits > 8 * parts && groups * parts < 256 * 1024) parts *= 2;
+  const int64_t blocks = (groups * parts + 255) / 256;
   if (blocks > kMaxLaunchThreads / 256) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(strided_reduce_kernel, dim3((unsigned)blocks), dim3(256), 0, s, a);
+  auto* const kern = parts == 1 ? strided_reduce_kernel<1> : parts == 2 ? strided_reduce_kernel<2> : parts == 4 ? strided_reduce_kernel<4>
+                     : parts == 8 ? strided_reduce_kernel<8> : strided_reduce_kernel<16>;
+  hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(256), 0, s, a);
   return hipGetLastError();
 }
 
