@@ -380,6 +380,7 @@ struct Col2imArgs {
   const float* cols;  // [N][OH][OW][KH][KW][CI]
   void* out;          // [N][H][W][CI]
   int N, H, W, CI, OH, OW, KH, KW, SH, SW, PH, PW, DH, DW;
+  int period_h, period_w;  // (of the taps that meet a gradient pixel, set by the launch)
 };
 hipError_t col2im_launch(const Col2imArgs& a, bool bf, hipStream_t s);
 struct ConvBorderArgs {
@@ -389,8 +390,9 @@ struct ConvBorderArgs {
   int y0, y1, x0, x1;  // pixels all of whose taps lie inside the gradient: y0 <= y < y1, x0 <= x < x1
 };
 hipError_t conv_border_launch(const ConvBorderArgs& a, bool bf, hipStream_t s);
-hipError_t pad_rows_launch(int es, const void* in, void* out, int64_t rows, int64_t cols, int64_t pitch, hipStream_t s);
-hipError_t flip_filter_launch(int es, const void* f, void* bt, int64_t taps, int64_t ci, int64_t co, int64_t pitch, hipStream_t s);
+// pad_rows = 0: the gradient's rows are read as they are; bt = nullptr: no filter is flipped
+hipError_t gradient_operands_launch(int es, const void* in, void* out, int64_t pad_rows, int64_t cols, int64_t pitch, const void* f, void* bt, int64_t taps,
+                                    int64_t ci, int64_t co, hipStream_t s);
 
 // window kernels (window.hip)
 struct DwconvArgs {

@@ -2157,17 +2157,16 @@ int pml_hip_conv2d_grad_invoke(int64_t plan, const void* g, const void* other, v
     return check(strided_launch(a, p->strided_bf, true, p->strided_mi, st), "strided_launch");
   }
   if (p->sub) {
-    const void* in = g;
-    if (p->padded) {
-      if (check(pad_rows_launch(es, g, p->padded, d.n * d.oh * d.ow, d.co, p->co_pad, st), "pad_rows_launch")) return 1;
-      in = p->padded;
-    }
-    if (p->sub->win.config >= 0) {  // (the taps in reverse, the channels' roles exchanged)
+    const void* const in = p->padded ? p->padded : g;
+    const bool window = p->sub->win.config >= 0;
+    if (window) {  // (the taps in reverse, the channels' roles exchanged)
       const WinFilter w{(int)(d.kh * d.kw), (int)d.co, (int)d.ci, (d.kh * d.kw - 1) * d.ci * d.co, -d.ci * d.co, 1, d.co};
       if (check(winconv_pack_launch(es, other, w, p->sub->bt, st), "winconv_pack_launch")) return 1;
-    } else if (check(flip_filter_launch(es, other, p->sub->bt, d.kh * d.kw, d.ci, d.co, p->co_pad, st), "flip_filter_launch")) {
-      return 1;
     }
+    if (check(gradient_operands_launch(es, g, p->padded, p->padded ? d.n * d.oh * d.ow : 0, d.co, p->co_pad, other, window ? nullptr : p->sub->bt,
+                                       d.kh * d.kw, d.ci, d.co, st),
+              "gradient_operands_launch"))
+      return 1;
     if (pml_hip_conv2d_invoke((int64_t)(intptr_t)p->sub, in, nullptr, result, nullptr, nullptr, nullptr, s)) return 1;
     ConvBorderArgs b;
     b.g = g, b.f = other, b.out = result;

@@ -23,6 +23,7 @@
 #include <algorithm>
 #include <cmath>
 #include <limits>
+#include <numeric>
 
 #include "device_common.h"
 #include "plans.h"
@@ -1096,62 +1097,94 @@ namespace {
 
 // The columns of a strided convolution's data gradient, cols[pixel of the gradient][ky][kx][ci] in fp32, added up into
 // the image: an image value takes the columns of every tap and gradient pixel whose window covers it, taps in order.
-// A thread per V channels of an image pixel; columns are read once, V * 4 bytes at a time.
+// A thread per V channels of an image pixel (the last V of a pixel overlap the ones before them where CI is no multiple of V);
+// columns are read once, V * 4 bytes at a time.  What bounds it is a thread's chain of loads: only the taps that meet a gradient
+// pixel are visited, up to four of a filter row are on their way at once.  5 x 75 x 75 x 121 from 5 x 5 taps of stride 2, bf16:
+// 60 us a value a thread and a tap at a time, now 16.
 template <bool BF, int V>
 __global__ __launch_bounds__(256) void col2im_kernel(Col2imArgs a) {
-  const int64_t per_img = (int64_t)a.H * a.W * a.CI / V;
-  const int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (g >= per_img * a.N) return;
-  const int64_t img = g / per_img;
-  const unsigned rem = (unsigned)(g - img * per_img), cv = (unsigned)(a.CI / V);
-  const int c = (int)(rem % cv) * V, pix = (int)(rem / cv), y = pix / a.W, x = pix % a.W;
+  const unsigned cv = (unsigned)(a.CI + V - 1) / V, per_img = (unsigned)(a.H * a.W);
+  const unsigned g = blockIdx.x * 256 + threadIdx.x;
+  const unsigned at_pixel = g / cv;
+  if (at_pixel >= (unsigned)a.N * per_img) return;
+  const unsigned chunk = g - at_pixel * cv, img = at_pixel / per_img, pix = at_pixel - img * per_img;
+  const int y = (int)(pix / (unsigned)a.W), x = (int)(pix - (unsigned)y * (unsigned)a.W);
+  const int c = (int)chunk * V + V <= a.CI ? (int)chunk * V : a.CI - V;
+  // the first tap of a column or row of them whose window meets a gradient pixel; from there every period-th does
+  auto first = [](int at, int taps, int period, int stride, int dil) {
+    for (int k = 0; k < period && k < taps; ++k)
+      if ((at - k * dil) % stride == 0) return k;
+    return taps;
+  };
+  const int ky0 = first(y + a.PH, a.KH, a.period_h, a.SH, a.DH), kx0 = first(x + a.PW, a.KW, a.period_w, a.SW, a.DW);
+  const int gy0 = (y + a.PH - ky0 * a.DH) / a.SH, gx0 = (x + a.PW - kx0 * a.DW) / a.SW;
+  const int dy = a.period_h * a.DH / a.SH, dx = a.period_w * a.DW / a.SW;
+  const int taps = a.KH * a.KW;
   float sum[V];
 #pragma unroll
   for (int e = 0; e < V; ++e) sum[e] = 0.f;
-  for (int ky = 0; ky < a.KH; ++ky) {
-    const int ty = y + a.PH - ky * a.DH;
-    if (ty < 0 || ty % a.SH != 0 || ty / a.SH >= a.OH) continue;
-    for (int kx = 0; kx < a.KW; ++kx) {
-      const int tx = x + a.PW - kx * a.DW;
-      if (tx < 0 || tx % a.SW != 0 || tx / a.SW >= a.OW) continue;
-      const float* at = a.cols + (((img * a.OH + ty / a.SH) * a.OW + tx / a.SW) * (a.KH * a.KW) + ky * a.KW + kx) * a.CI + c;
-      const Words<V> w = load_words<V>(at);
+  for (int ky = ky0, gy = gy0; ky < a.KH; ky += a.period_h, gy -= dy) {
+    if (gy < 0 || gy >= a.OH) continue;
+    const float* const row = a.cols + ((int64_t)img * a.OH + gy) * a.OW * taps * a.CI + (int64_t)ky * a.KW * a.CI + c;
+    constexpr int U = 4;
+    for (int kx = kx0, gx = gx0; kx < a.KW; kx += U * a.period_w, gx -= U * dx) {
+      Words<V> w[U];
+      bool in[U];
 #pragma unroll
-      for (int e = 0; e < V; ++e) sum[e] += __uint_as_float(w.w[e]);
+      for (int u = 0; u < U; ++u) {
+        const int k = kx + u * a.period_w, g = gx - u * dx;
+        in[u] = k < a.KW && g >= 0 && g < a.OW;
+        if (in[u]) w[u] = load_words<V>(row + ((int64_t)g * taps + k) * a.CI);
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int e = 0; e < V; ++e) sum[e] += in[u] ? __uint_as_float(w[u].w[e]) : 0.f;
     }
   }
+  const int64_t o = (int64_t)at_pixel * a.CI + c;
+  if constexpr (BF) {
+    uint16_t h[V];
 #pragma unroll
-  for (int e = 0; e < V; ++e) {
-    const int64_t o = g * V + e;
-    if constexpr (BF)
-      ((uint16_t*)a.out)[o] = f32_to_bf16_bits(sum[e]);
-    else
-      ((float*)a.out)[o] = sum[e];
+    for (int e = 0; e < V; ++e) h[e] = f32_to_bf16_bits(sum[e]);
+    __builtin_memcpy((uint16_t*)a.out + o, h, sizeof h);
+  } else {
+    __builtin_memcpy((float*)a.out + o, sum, sizeof sum);
   }
 }
 
-// Rows of `cols` elements copied to rows of `pitch` elements, the rest of a row zeros.
+// What the unit-stride data gradient's convolution reads, in one launch: the gradient's rows of `cols` elements copied to rows of
+// whole 16-byte vectors, the rest of a row zeros (pad_rows = 0: they are so already), and its right-hand side
+//   Bt[ci][tap][pitch] = F[taps - 1 - tap][ci][co]
+// -- the filter's taps in reverse and the channels' roles exchanged, contiguous along what that convolution sums over.  The first
+// `flip_blocks` workgroups flip.  A thread copies 16 bytes of a padded row: 154154 rows of 38 bf16 12.8 us an element at a time and
+// 4.7 for the filter in a launch of its own, now 7.5 for both.
 template <typename T>
-__global__ __launch_bounds__(256) void pad_rows_kernel(const T* in, T* out, int64_t rows, int cols, int pitch) {
-  const int64_t stride = (int64_t)gridDim.x * 256, total = rows * pitch;
-  for (int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x; g < total; g += stride) {
-    const int64_t row = g / pitch;
-    const int c = (int)(g - row * pitch);
-    out[g] = c < cols ? in[row * cols + c] : (T)0;
+__global__ __launch_bounds__(256) void gradient_operands_kernel(const T* in, T* out, int64_t pad_rows, int cols, int pitch, const T* f, T* bt, int taps, int ci,
+                                                                 int co, int64_t flip_blocks) {
+  if (blockIdx.x < flip_blocks) {
+    const int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (g >= (int64_t)ci * taps * co) return;
+    const int c = (int)(g % co);
+    const int64_t r = g / co;
+    const int tap = (int)(r % taps), n = (int)(r / taps);
+    bt[((int64_t)n * taps + tap) * pitch + c] = f[((int64_t)(taps - 1 - tap) * ci + n) * co + c];
+    return;
   }
-}
-
-// Bt[ci][tap][pitch] = F[taps - 1 - tap][ci][co]: the filter of a data gradient seen as a convolution of the gradient,
-// taps in reverse and the channels' roles exchanged; already contiguous along what that convolution sums over.
-template <typename T>
-__global__ __launch_bounds__(256) void flip_filter_kernel(const T* f, T* bt, int taps, int ci, int co, int pitch) {
-  const int64_t total = (int64_t)ci * taps * co;
-  const int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (g >= total) return;
-  const int c = (int)(g % co);
-  const int64_t r = g / co;
-  const int tap = (int)(r % taps), n = (int)(r / taps);
-  bt[((int64_t)n * taps + tap) * pitch + c] = f[((int64_t)(taps - 1 - tap) * ci + n) * co + c];
+  constexpr int V = 16 / sizeof(T);
+  const int64_t per_row = pitch / V, total = pad_rows * per_row, stride = (int64_t)(gridDim.x - flip_blocks) * 256;
+  for (int64_t g = (blockIdx.x - flip_blocks) * 256 + threadIdx.x; g < total; g += stride) {
+    const int64_t row = g / per_row;
+    const int c = (int)(g - row * per_row) * V;
+    T v[V];
+    if (c + V <= cols) {
+      __builtin_memcpy(v, in + row * cols + c, 16);
+    } else {
+#pragma unroll
+      for (int e = 0; e < V; ++e) v[e] = c + e < cols ? in[row * cols + c + e] : (T)0;
+    }
+    __builtin_memcpy(out + g * V, v, 16);
+  }
 }
 
 // The unit-stride data gradient runs as a convolution of the gradient, and the convolution kernels read taps outside the
@@ -1222,9 +1255,12 @@ hipError_t conv_border_launch(const ConvBorderArgs& a, bool bf, hipStream_t s) {
   return hipGetLastError();
 }
 
-hipError_t col2im_launch(const Col2imArgs& a, bool bf, hipStream_t s) {
-  const int v = a.CI % 4 == 0 ? 4 : 1;
-  const int64_t blocks = ((int64_t)a.N * a.H * a.W * a.CI / v + 255) / 256;
+hipError_t col2im_launch(const Col2imArgs& args, bool bf, hipStream_t s) {
+  Col2imArgs a = args;
+  a.period_h = a.SH / std::gcd(a.SH, a.DH);
+  a.period_w = a.SW / std::gcd(a.SW, a.DW);
+  const int v = a.CI >= 4 ? 4 : 1;
+  const int64_t blocks = ((int64_t)a.N * a.H * a.W * ((a.CI + v - 1) / v) + 255) / 256;
   if (blocks <= 0 || blocks > kMaxLaunchThreads / 256) return hipErrorInvalidValue;
   const dim3 grid((unsigned)blocks), block(256);
   if (bf) {
@@ -1237,23 +1273,19 @@ hipError_t col2im_launch(const Col2imArgs& a, bool bf, hipStream_t s) {
   return hipGetLastError();
 }
 
-hipError_t pad_rows_launch(int es, const void* in, void* out, int64_t rows, int64_t cols, int64_t pitch, hipStream_t s) {
-  if (rows * pitch == 0) return hipSuccess;
-  const unsigned blocks = (unsigned)std::min<int64_t>((rows * pitch + 255) / 256, 256 * 32);
+hipError_t gradient_operands_launch(int es, const void* in, void* out, int64_t pad_rows, int64_t cols, int64_t pitch, const void* f, void* bt, int64_t taps,
+                                    int64_t ci, int64_t co, hipStream_t s) {
+  const int64_t flip = bt ? (taps * ci * co + 255) / 256 : 0;
+  const int64_t pad = std::min<int64_t>((pad_rows * (pitch * es / 16) + 255) / 256, 256 * 32);
+  if (flip + pad <= 0) return hipSuccess;
+  if (flip + pad > kMaxLaunchThreads / 256) return hipErrorInvalidValue;
+  const dim3 grid((unsigned)(flip + pad)), block(256);
   if (es == 2)
-    hipLaunchKernelGGL(pad_rows_kernel<uint16_t>, dim3(blocks), dim3(256), 0, s, (const uint16_t*)in, (uint16_t*)out, rows, (int)cols, (int)pitch);
+    hipLaunchKernelGGL(gradient_operands_kernel<uint16_t>, grid, block, 0, s, (const uint16_t*)in, (uint16_t*)out, pad_rows, (int)cols, (int)pitch, (const uint16_t*)f,
+                       (uint16_t*)bt, (int)taps, (int)ci, (int)co, flip);
   else
-    hipLaunchKernelGGL(pad_rows_kernel<uint32_t>, dim3(blocks), dim3(256), 0, s, (const uint32_t*)in, (uint32_t*)out, rows, (int)cols, (int)pitch);
-  return hipGetLastError();
-}
-
-hipError_t flip_filter_launch(int es, const void* f, void* bt, int64_t taps, int64_t ci, int64_t co, int64_t pitch, hipStream_t s) {
-  const int64_t blocks = (taps * ci * co + 255) / 256;
-  if (blocks <= 0 || blocks > kMaxLaunchThreads / 256) return hipErrorInvalidValue;
-  if (es == 2)
-    hipLaunchKernelGGL(flip_filter_kernel<uint16_t>, dim3((unsigned)blocks), dim3(256), 0, s, (const uint16_t*)f, (uint16_t*)bt, (int)taps, (int)ci, (int)co, (int)pitch);
-  else
-    hipLaunchKernelGGL(flip_filter_kernel<uint32_t>, dim3((unsigned)blocks), dim3(256), 0, s, (const uint32_t*)f, (uint32_t*)bt, (int)taps, (int)ci, (int)co, (int)pitch);
+    hipLaunchKernelGGL(gradient_operands_kernel<uint32_t>, grid, block, 0, s, (const uint32_t*)in, (uint32_t*)out, pad_rows, (int)cols, (int)pitch, (const uint32_t*)f,
+                       (uint32_t*)bt, (int)taps, (int)ci, (int)co, flip);
   return hipGetLastError();
 }
 
