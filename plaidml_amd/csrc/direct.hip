@@ -18,6 +18,9 @@
 // K further down the rows lie as before.  Columns past N are fetched as what follows in memory, or as zeros behind the last
 // row (the descriptor ends there), and never stored.  Before, such a right-hand side was transposed by a launch of its own: 7 x 327, K = 192 bf16 10.4 -> 4.5 us,
 // 51 x 861, K = 2272 int8 15.7 -> 9.1, 6 x 3382, K = 256 fp32 (which needs no shifting) 11.4 -> 5.4; 36 sizes drawn 1.43x.
+// A convolution's filter [KH][KW][CI][CO] is such a right-hand side, too, and no packing launch goes
+// ahead: 10 x 37 x 37 x 96 (*) 1 x 1 x 63 stride 2 fp32 11.3 -> 7.0 us, 38 x 8 x 8 x 16 (*) 5 x 5 x 21 bf16 10.8 -> 5.7, 3 x 34 x 34
+// x 256 (*) 3 x 3 x 48 int8 10.6 -> 6.4.
 #include <hip/hip_runtime.h>
 
 #include "device_common.h"
@@ -144,14 +147,14 @@ __global__ __launch_bounds__(64 * kWaves, 4) void direct_kernel(IgemmArgs p_by_v
   warm_arguments<sizeof(IgemmArgs)>();
   // (read where the dispatcher put it: indexing a by-value copy would move the copy to scratch memory)
   const IgemmArgs& p = *(const IgemmArgs*)(const __attribute__((address_space(4))) void*)__builtin_amdgcn_kernarg_segment_ptr();
-  static_assert(!KN || (NB == 4 && !CONV), "a [K][N] right-hand side is taken four columns per lane");
+  static_assert(!KN || NB == 4, "a [K][N] right-hand side is taken four columns per lane");
   static_assert(!RAGGED || (KN && KIND != KIND_F32), "four-byte elements are whole words wherever they lie");
   typedef typename Acc<KIND>::scalar accs_t;
   typedef accs_t acc4_t __attribute__((ext_vector_type(4)));
   constexpr int ES = KIND == KIND_BF16 ? 2 : (KIND == KIND_I8 ? 1 : 4);
   constexpr int TM = 16 * MB, TN = 16 * NB;
   // steps in flight: 64 registers of requests, fewer where the accumulators leave less room
-  constexpr int U = KN ? (KIND == KIND_F32 ? (MB == 1 ? 4 : 2) : MB == 1 && !RAGGED ? 3 : 2) : MB + NB > 4 ? 2 : 16 / (MB + NB);
+  constexpr int U = KN ? (KIND == KIND_F32 ? (MB == 1 ? 4 : CONV ? 1 : 2) : MB == 1 && !RAGGED ? 3 : 2) : MB + NB > 4 ? 2 : 16 / (MB + NB);
   constexpr int RW = RAGGED ? (KIND == KIND_BF16 ? 24 : 32) : 16;  // KN: words fetched for a lane's chunk
   constexpr int CS = TN + 4;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -178,7 +181,7 @@ __global__ __launch_bounds__(64 * kWaves, 4) void direct_kernel(IgemmArgs p_by_v
   // (KN: from the word its first element lies in to the end of the word its last one lies in -- the lanes at the right edge
   // fetch past rows; words are inside or outside the range as a whole)
   const int b_rem = KN ? (int)((uintptr_t)Bt & 3) : 0;
-  const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void*)((uintptr_t)Bt - b_rem), 0, KN ? (b_rem + (int)(((K - 1) * ldbt + N) * ES) + 3) & ~3 : (int)kBufRange, kRsrcFlags);
+  const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void*)((uintptr_t)Bt - b_rem), 0, KN ? (b_rem + (int)((((p.b_rows ? p.b_rows : K) - 1) * ldbt + N) * ES) + 3) & ~3 : (int)kBufRange, kRsrcFlags);
   const bool two = !CONV && !KN && K2 > 0;
   const __amdgpu_buffer_rsrc_t ra2 = __builtin_amdgcn_make_buffer_rsrc((void*)(two ? p.A2 : A), 0, (int)kBufRange, kRsrcFlags);
   const __amdgpu_buffer_rsrc_t rb2 = __builtin_amdgcn_make_buffer_rsrc((void*)(two ? p.Bt2 : Bt), 0, (int)kBufRange, kRsrcFlags);
@@ -262,6 +265,37 @@ __global__ __launch_bounds__(64 * kWaves, 4) void direct_kernel(IgemmArgs p_by_v
   const int64_t tail_m = m0 + tid / (TN / 4), tail_n = n0 + tid % (TN / 4) * 4;
   if (quick) tail_ahead<KIND>(p, tid < kQuads, M, N, tail_m, tail_n, ahead);
 
+  // KN: the words of the lane's four columns in the K-rows from `k` on that its 16 bytes of K stand for
+  auto fetch_rows = [&](int (&raw)[RW], int k, bool ok) {
+    constexpr int E = 16 / ES;  // K-rows of the lane's chunk: all of them exist or none (K is whole 16-byte vectors)
+    const unsigned pitch = (unsigned)(ldbt * ES);
+    const unsigned at = b_off[0] + (unsigned)k * pitch;
+    const bool in = ok & (b_off[0] != kOutside);
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      // (RAGGED: the word a row's first byte lies in, counted from the aligned base; the same for all lanes but `at`)
+      const int row = RAGGED ? (b_rem + e * (int)pitch) & ~3 : e * (int)pitch;
+      const int off = in ? (int)(at + (unsigned)row) : (int)kOutside;
+      if constexpr (KIND == KIND_F32) {
+        const i32x4_t v = __builtin_bit_cast(i32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rb, off, 0, 0));
+#pragma unroll
+        for (int q = 0; q < 4; ++q) raw[4 * e + q] = v[q];
+      } else if constexpr (RAGGED && KIND == KIND_BF16) {
+        typedef int i32x3_t __attribute__((ext_vector_type(3)));
+        const i32x3_t v = __builtin_bit_cast(i32x3_t, __builtin_amdgcn_raw_buffer_load_b96(rb, off, 0, 0));
+#pragma unroll
+        for (int q = 0; q < 3; ++q) raw[3 * e + q] = v[q];
+      } else if constexpr (RAGGED || KIND == KIND_BF16) {
+        typedef int i32x2_t __attribute__((ext_vector_type(2)));
+        const i32x2_t v = __builtin_bit_cast(i32x2_t, __builtin_amdgcn_raw_buffer_load_b64(rb, off, 0, 0));
+        raw[2 * e] = v[0];
+        raw[2 * e + 1] = v[1];
+      } else {
+        raw[e] = (int)__builtin_amdgcn_raw_buffer_load_b32(rb, off, 0, 0);
+      }
+    }
+  };
+
   for (int s0 = first; s0 < last; s0 += U) {
     i32x4_t fa[U][MB];
     i32x4_t fb[KN ? 1 : U][KN ? 1 : NB];
@@ -280,9 +314,13 @@ __global__ __launch_bounds__(64 * kWaves, 4) void direct_kernel(IgemmArgs p_by_v
           fa[u][i] = __builtin_bit_cast(i32x4_t, __builtin_amdgcn_raw_buffer_load_b128(ra, in ? (int)(a_off[i] + at) : (int)kOutside, 0, 0));
         }
         const unsigned bk = (unsigned)((kh * KW + kw) * kbytes + cb);
+        if constexpr (KN) {
+          fetch_rows(raw[u], (int)(bk / ES), ok);
+        } else {
 #pragma unroll
-        for (int j = 0; j < NB; ++j)
-          fb[u][j] = __builtin_bit_cast(i32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rb, ok ? (int)(b_off[j] + bk) : (int)kOutside, 0, 0));
+          for (int j = 0; j < NB; ++j)
+            fb[u][j] = __builtin_bit_cast(i32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rb, ok ? (int)(b_off[j] + bk) : (int)kOutside, 0, 0));
+        }
         if (++cs == steps_per_tap) {
           cs = 0;
           if (++kw == KW) {
@@ -299,33 +337,7 @@ __global__ __launch_bounds__(64 * kWaves, 4) void direct_kernel(IgemmArgs p_by_v
           fa[u][i] = __builtin_bit_cast(i32x4_t, __builtin_amdgcn_raw_buffer_load_b128(
                                                      second ? ra2 : ra, ok ? (int)((second ? a2_off[i] : a_off[i]) + (unsigned)cb) : (int)kOutside, 0, 0));
         if constexpr (KN) {
-          constexpr int E = 16 / ES;  // K-rows of the lane's chunk: all of them exist or none (K is whole 16-byte vectors)
-          const unsigned pitch = (unsigned)(ldbt * ES);
-          const unsigned at = b_off[0] + (unsigned)(cb / ES) * pitch;
-          const bool in = ok & (b_off[0] != kOutside);
-#pragma unroll
-          for (int e = 0; e < E; ++e) {
-            // (RAGGED: the word a row's first byte lies in, counted from the aligned base; the same for all lanes but `at`)
-            const int row = RAGGED ? (b_rem + e * (int)pitch) & ~3 : e * (int)pitch;
-            const int off = in ? (int)(at + (unsigned)row) : (int)kOutside;
-            if constexpr (KIND == KIND_F32) {
-              const i32x4_t v = __builtin_bit_cast(i32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rb, off, 0, 0));
-#pragma unroll
-              for (int q = 0; q < 4; ++q) raw[u][4 * e + q] = v[q];
-            } else if constexpr (RAGGED && KIND == KIND_BF16) {
-              typedef int i32x3_t __attribute__((ext_vector_type(3)));
-              const i32x3_t v = __builtin_bit_cast(i32x3_t, __builtin_amdgcn_raw_buffer_load_b96(rb, off, 0, 0));
-#pragma unroll
-              for (int q = 0; q < 3; ++q) raw[u][3 * e + q] = v[q];
-            } else if constexpr (RAGGED || KIND == KIND_BF16) {
-              typedef int i32x2_t __attribute__((ext_vector_type(2)));
-              const i32x2_t v = __builtin_bit_cast(i32x2_t, __builtin_amdgcn_raw_buffer_load_b64(rb, off, 0, 0));
-              raw[u][2 * e] = v[0];
-              raw[u][2 * e + 1] = v[1];
-            } else {
-              raw[u][e] = (int)__builtin_amdgcn_raw_buffer_load_b32(rb, off, 0, 0);
-            }
-          }
+          fetch_rows(raw[u], cb / ES, ok);
         } else {
 #pragma unroll
           for (int j = 0; j < NB; ++j)
@@ -451,21 +463,21 @@ static hipError_t launch_large(const IgemmArgs& a, hipStream_t s) {
   return ((a.M + 31) / 32) * ((a.N + 31) / 32) > a.n_cus ? launch<PML_KIND, CONV, 2, 4, false>(a, s) : launch<PML_KIND, CONV, 2, 2, false>(a, s);
 }
 
-// cfg: TILE_16x16_W8 or TILE_32x32_W8 (with a [K][N] right-hand side: 16 x 64 and 32 x 64 results)
-hipError_t PML_CAT(direct_launch_kind_, PML_KIND)(int cfg, bool conv, const IgemmArgs& a, hipStream_t s) {
-  const bool small = cfg == TILE_16x16_W8;
-  if (conv) {
-    if (a.b_kn) return hipErrorInvalidValue;
-    return small ? launch<PML_KIND, true, 1, 1, false>(a, s) : launch_large<true>(a, s);
-  }
+template <bool CONV>
+static hipError_t launch_form(bool small, const IgemmArgs& a, hipStream_t s) {
   if (a.b_kn) {
     if (a.K2 > 0) return hipErrorInvalidValue;
     if constexpr (PML_KIND != KIND_F32)
       if (((a.N | a.ldbt) & 3) != 0 || ((uintptr_t)a.Bt & (PML_KIND == KIND_BF16 ? 7 : 3)) != 0)
-        return small ? launch<PML_KIND, false, 1, 4, true, true>(a, s) : launch<PML_KIND, false, 2, 4, true, true>(a, s);
-    return small ? launch<PML_KIND, false, 1, 4, true>(a, s) : launch<PML_KIND, false, 2, 4, true>(a, s);
+        return small ? launch<PML_KIND, CONV, 1, 4, true, true>(a, s) : launch<PML_KIND, CONV, 2, 4, true, true>(a, s);
+    return small ? launch<PML_KIND, CONV, 1, 4, true>(a, s) : launch<PML_KIND, CONV, 2, 4, true>(a, s);
   }
-  return small ? launch<PML_KIND, false, 1, 1, false>(a, s) : launch_large<false>(a, s);
+  return small ? launch<PML_KIND, CONV, 1, 1, false>(a, s) : launch_large<CONV>(a, s);
+}
+
+// cfg: TILE_16x16_W8 or TILE_32x32_W8 (with a [K][N] right-hand side: 16 x 64 and 32 x 64 results)
+hipError_t PML_CAT(direct_launch_kind_, PML_KIND)(int cfg, bool conv, const IgemmArgs& a, hipStream_t s) {
+  return conv ? launch_form<true>(cfg == TILE_16x16_W8, a, s) : launch_form<false>(cfg == TILE_16x16_W8, a, s);
 }
 
 }  // namespace pml

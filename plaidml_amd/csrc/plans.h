@@ -142,7 +142,8 @@ inline void tile_of(const TileOrder& o, unsigned bid, int* tm, int* tn) {
 
 struct IgemmArgs {
   TileOrder order;  // filled in by the launcher for the tile grid of the configuration it launches
-  int b_kn;         // 1: Bt / ldbt are the caller's row-major B[K][N] and its row length (GEMMs)
+  int b_kn;         // 1: Bt / ldbt are the caller's row-major B[K][N] and its row length (GEMMs; direct tiles of convolutions)
+  int b_rows;       // direct tiles over such a B whose K is padded: the rows that it has (0: all K)
   int stream;       // 1: the tile was chosen for the problem's sizes, not named by the caller: rows may stream instead (stream.hip)
   // conv_blocks4x4_kernel only: the caller's NHWC image of 3 bf16 channels (raw_h x raw_w pixels, raw_w even), from
   // which the kernel builds the rows of 2x2 pixel blocks itself; null: A already holds the re-blocked image

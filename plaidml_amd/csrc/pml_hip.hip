@@ -92,6 +92,7 @@ struct Plan {
   // the direct tiles a product takes instead of `tile`, and the one a convolution takes (-1: none)
   DirectTiles direct;
   int tile_direct = -1;
+  int tile_given = -1;  // ... and over a filter that comes with the call, as it lies
   // a convolution that runs over its window in LDS (`bt` holds the filter as that kernel multiplies it)
   WinShape win;
   // a product that runs in panels once its right-hand sides are packed: the configuration (-1: it does not) and their fragments
@@ -677,7 +678,7 @@ void s2d_args(const Plan* p, S2dArgs& a) {
 //     11 x 11 x 11 x 64 (*) 3 x 3 x 20 stays, 5.5 both ways; 3 x 30 x 30 x 256 (*) 7 x 7 x 18 stride 2 stays, 14.6, over windows 34.6).
 //   * 3 x 3 filters that the kernels of conv_halo.hip keep on the chip stay there (128 x 56 x 56 x 64 (*) 3 x 3 x 64 36); their general
 //     form for any other filter that fits LDS does not (40 x 30 x 30 x 64 (*) 3 x 3 x 48 23.9 -> 9.1).
-WinShape window_shape(Plan* p, bool named) {
+WinShape window_shape(Plan* p, bool named, double* window_us) {
   const pml_hip_conv2d_desc& d = p->conv;
   const int out = p->mfma_kind == KIND_BF16 ? PML_HIP_BF16 : p->mfma_kind == KIND_I8 ? PML_HIP_I32 : PML_HIP_F32;
   if (d.init_kind && !(d.init_row_stride == 0 && d.init_col_stride == 1 && d.init_dtype == out)) return {};
@@ -685,6 +686,7 @@ WinShape window_shape(Plan* p, bool named) {
   conv_args(p, g);
   double us = 0;
   const WinShape shape = winconv_shape(p->mfma_kind, g, &us);
+  *window_us = us;
   if (shape.config < 0 || named) return shape;
   // (a last block of channels that is mostly empty, int8 of 96 channels: 62 x 45 x 45 x 96 (*) 5 x 5 x 23 stride 2 15.4, over windows 17.0)
   const int64_t ci_bytes = d.ci * dt_size(d.in_dtype);
@@ -700,6 +702,37 @@ WinShape window_shape(Plan* p, bool named) {
     return us < 4 + 1.45 * mma_us ? shape : WinShape{};
   }
   return shape;
+}
+
+// The direct tile of a convolution whose filter comes with the call and is read as it lies (-1: it is packed by a launch of its
+// own first): where that is cheaper than the plan's kernel and the packing.  The price is fitted to 260 timings of 130
+// convolutions (8 to 13 % rms): 2.6 us, and per round (a last one that is not full counts for most of one) of one 16 x 64 or 32 x 64 tile on each CU a start and so much per KB of K --
+// not per byte of a filter's few columns: it is the requests for K-rows that take the time, more of them for int8, whose rows
+// off a word take two words each.  fp32 sums are the same bits either way, so there it is for convolutions that take a direct
+// tile over a packed filter, too.  us a call, packing first -> as it lies:
+//   1 x 1    bf16 28 x 9 x 9 x 256 (*) 62 10.3 -> 5.9     int8 36 x 7 x 7 x 128 (*) 46 8.5 -> 4.7     fp32 3 x 9 x 9 x 96 (*) 23 stride 2 9.7 -> 6.7
+//   3 x 3    bf16 5 x 25 x 25 x 32 (*) 76 8.8 -> 5.2      int8 34 x 14 x 14 x 64 (*) 59 9.5 -> 6.0    fp32 2 x 15 x 15 x 32 (*) 37 10.2 -> 6.8
+//   5 x 5    bf16 11 x 21 x 21 x 64 (*) 102 stride 2 11.7 -> 8.7; but 2 x 69 x 69 x 64 (*) 19, two rounds, 12.2, as it lies 16.9
+// and of 140 drawn convolutions with the filter in the call 59 take it, 1.36 x in the mean.
+int given_filter_tile(const Plan* p, double window_us) {
+  const pml_hip_conv2d_desc& d = p->conv;
+  const int es = dt_size(d.in_dtype);
+  const int64_t M = d.n * d.oh * d.ow, k_bytes = (p->patches ? p->kpad : d.kh * d.kw * d.ci) * es;
+  const bool window = p->win.config >= 0, odd = d.co % 4 != 0;
+  if (p->mfma_kind == KIND_F32X3 || (p->mfma_kind == KIND_F32 && p->tile_direct < 0)) return -1;
+  auto lies_us = [&](int64_t side) {
+    double start, per_kb;
+    if (p->mfma_kind == KIND_BF16) start = side == 16 ? 1.35 : 1.7, per_kb = side == 16 ? 1.17 : 1.52;
+    else if (p->mfma_kind == KIND_I8) start = side == 16 ? 1.3 : 1.6, per_kb = 1.2 + (!odd ? 0 : side == 16 ? 0.85 : 1.25);
+    else start = side == 16 ? 2.2 : 1.7, per_kb = side == 16 ? 1.2 : 2.3;
+    const double rounds = std::max(1.0, (double)((M + side - 1) / side) * (double)((d.co + 63) / 64) / device_cus());
+    return 2.6 + (0.75 * std::ceil(rounds) + 0.25 * rounds) * (start + per_kb * (double)k_bytes / 1024);
+  };
+  double packed_us = window_us;
+  if (!window) (void)direct_tile_of(M, d.co, k_bytes, p->mfma_kind, 0, p->tile_direct >= 0, /*can_split=*/!p->patches, false, &packed_us);
+  const double small = lies_us(16), large = lies_us(32), packing = 3.0 + 2.0 * (double)k_bytes * (double)d.co / 2.2e6;
+  if (std::min(small, large) > (p->tile_direct >= 0 ? 0.95 : 0.85) * (packed_us + packing)) return -1;
+  return small <= large ? TILE_16x16_W8 : TILE_32x32_W8;
 }
 
 // Packs the caller's HWCK filter into the plan's Bt.
@@ -1502,7 +1535,8 @@ int64_t pml_hip_conv2d_dispatch(const pml_hip_conv2d_desc* d) {
       return 0;
     }
   }
-  if (!via_s2d && !via_patches && PML_HIP_FLAG_TILE_OF(d->flags) < 0) p->tile_direct = direct_tile_of(M, d->co, K * es, kind);
+  if (!via_s2d && PML_HIP_FLAG_TILE_OF(d->flags) < 0)
+    p->tile_direct = direct_tile_of(M, d->co, (via_patches ? p->kpad : K) * es, kind, 0, false, /*can_split=*/!via_patches);
   {
     // Filter small enough to stay in LDS: persistent resident-filter kernel (PML_HIP_CONV_IGEMM keeps the generic one).
     int dev = 0;
@@ -1522,13 +1556,15 @@ int64_t pml_hip_conv2d_dispatch(const pml_hip_conv2d_desc* d) {
     }
   }
   const bool named = path == PML_HIP_CONV_WINDOW;
+  double window_us = 0;
   if (!odd_channels && PML_HIP_FLAG_TILE_OF(d->flags) < 0 && (named || (path == PML_HIP_CONV_AUTO && (!p->halo_lds || p->halo_variant == 0)))) {
-    p->win = window_shape(p, named);
+    p->win = window_shape(p, named, &window_us);
     if (p->win.config >= 0) {
       p->halo_lds = 0;
       p->tile_direct = -1;
     }
   }
+  if (!via_s2d && !p->halo_lds && !named && PML_HIP_FLAG_TILE_OF(d->flags) < 0) p->tile_given = given_filter_tile(p, window_us);
   p->bt_bytes = p->win.config >= 0 ? winconv_pack_bytes(es, (int)(d->kh * d->kw), d->ci, d->co) : (size_t)d->co * p->bt_ld * es;
   if (!(p->bt = p->hold(p->bt_bytes)) || hipMemset(p->bt, 0, p->bt_bytes) != hipSuccess) {
     delete p;
@@ -1551,6 +1587,7 @@ int64_t pml_hip_conv2d_dispatch(const pml_hip_conv2d_desc* d) {
   p->text = buf;
   if (kind == KIND_F32X3) p->text += " mfma=3 x f32_32x32x16_bf16 (fp32 split into bf16 head + remainder)";
   if (p->tile_direct >= 0 && !p->halo_lds) p->text += std::string(", direct tile=") + tile_name(p->tile_direct);
+  if (p->tile_given >= 0) p->text += std::string(", with the filter as it lies tile=") + (p->tile_given == TILE_16x16_W8 ? "16x64" : "32x64") + " (8 wavefronts sharing K)";
   if (via_patches) p->text += " via patch matrix (k padded to " + std::to_string(p->kpad) + ")";
   if (!p->halo_lds && p->win.config < 0 && !via_s2d) {
     IgemmArgs g;
@@ -1648,10 +1685,23 @@ int pml_hip_conv2d_invoke(int64_t plan, const void* input, const void* filter, v
   for (int i = 0; i < d.tail.n_ops; ++i)
     if (d.tail.ops[i].opcode == PML_HIP_EPI_STORE && !g.outs[d.tail.ops[i].operand])
       return fail("conv2d_invoke: missing extra output");
-  const int tile = p->tile_direct >= 0 ? p->tile_direct : p->tile;
+  int tile = p->tile_direct >= 0 ? p->tile_direct : p->tile;
   // (a 1x1 convolution whose rows stream takes the filter as it lies; a packed one stays what later calls use)
   const bool given_filter = filter && !p->packed && !p->patches && !p->via_s2d && !p->halo_lds && p->win.config < 0 && streams_given(p->mfma_kind, tile, true, filter, d.co, g);
-  if (filter && !raw_filter && !given_filter) {
+  // A filter that comes with the call and that no packed one is kept beside: direct tiles read it as it lies.  (Behind a patch
+  // matrix whose rows are padded, the filter has to end on a whole word: what the word holds besides would meet the padding.)
+  const int lies_tile = PML_HIP_FLAG_TILE_OF(d.flags) >= 0 ? p->tile : p->tile_given;
+  const bool as_it_lies = filter && !given_filter && !p->packed && !p->via_s2d && !p->halo_lds && p->mfma_kind != KIND_F32X3 &&
+                          (lies_tile == TILE_16x16_W8 || lies_tile == TILE_32x32_W8) && ((uintptr_t)filter & (es - 1)) == 0 &&
+                          (p->patches ? p->kpad : K) * d.co * es < ((int64_t)1 << 31) && (!p->patches || (((uintptr_t)filter + (uintptr_t)(K * d.co * es)) & 3) == 0);
+  if (as_it_lies) {
+    tile = lies_tile;
+    g.Bt = filter;
+    g.ldbt = d.co;
+    g.b_kn = 1;
+    g.b_rows = (int)K;
+  }
+  if (filter && !raw_filter && !given_filter && !as_it_lies) {
     if (check(pack_conv_filter(p, filter, (hipStream_t)s), "pack_conv_filter")) return 1;
     // (a filter that arrives with the call replaces the packed one; its register-order copy follows it)
     if (p->reg_image && check(regfilter_image_launch(p->bt, p->bt_ld * es, p->reg_image, (hipStream_t)s), "regfilter_image_launch")) return 1;
@@ -1669,7 +1719,7 @@ int pml_hip_conv2d_invoke(int64_t plan, const void* input, const void* filter, v
     g.A = p->patches;
     g.lda = p->kpad;
     g.K = p->kpad;
-    return check(igemm_launch(p->mfma_kind, p->tile, false, g, (hipStream_t)s), "igemm_launch");
+    return check(igemm_launch(p->mfma_kind, tile, false, g, (hipStream_t)s), "igemm_launch");
   }
   if (p->via_s2d) {
     // 4x4 block taps onto 64 channels (the 7x7x3 stride-2 head of an image network): the kernel that walks down
@@ -1699,10 +1749,10 @@ int pml_hip_conv2d_invoke(int64_t plan, const void* input, const void* filter, v
     if (lds) return check(conv_blocks4x4_launch(g, lds, device_cus(), (hipStream_t)s), "conv_blocks4x4_launch");
     return check(igemm_launch(p->mfma_kind, p->tile, true, g, (hipStream_t)s), "igemm_launch");
   }
-  if (p->win.config >= 0) return check(winconv_launch(p->mfma_kind, g, p->win, (hipStream_t)s), "winconv_launch");
+  if (p->win.config >= 0 && !as_it_lies) return check(winconv_launch(p->mfma_kind, g, p->win, (hipStream_t)s), "winconv_launch");
   if (p->halo_lds)
     return check(conv_halo_launch(p->mfma_kind, g, p->halo_lds, p->n_cus, (hipStream_t)s), "conv_halo_launch");
-  split_args(p, g);
+  if (!as_it_lies) split_args(p, g);
   if (conv_tap_runs(d)) {
     g.pix_pitch = (int)(d.ci * es);
     g.CI = (int)(d.kw * d.ci);

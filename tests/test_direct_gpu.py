@@ -286,3 +286,49 @@ def test_long_chains_of_some_tiles_are_split(kind, M, N, K, split):
         assert np.abs(got - want).max() < 4 * 2.0 ** -16 * np.sqrt(K) * 0.25 + 1e-5
     else:
         check(E.bf16_from_bits(T.run_gemm(T.bf16(A), T.bf16(B), hk.BF16, hk.BF16, invokes=2)), want, 'bf16', K)
+
+
+# columns on four and off it, K-rows of one 16-byte chunk, runs of taps, more taps than wavefronts; three channels: a patch matrix
+# whose rows are padded, where a filter that does not end on a whole word is packed first
+@pytest.mark.parametrize('kind', ['f32', 'bf16', 'i8'])
+@pytest.mark.parametrize('shift', [0, 1])
+@pytest.mark.parametrize('tile', TILES + [None])
+@pytest.mark.parametrize('shape,k,co,stride', [((1, 9, 7, 32), 3, 48, 1), ((2, 7, 7, 16), 5, 33, 1), ((1, 8, 8, 96), 3, 131, 2), ((5, 6, 6, 64), 1, 66, 2),
+                                               ((1, 9, 9, 3), 3, 33, 1), ((2, 8, 7, 3), 7, 20, 1), ((3, 5, 5, 5), 1, 17, 1)])
+def test_filter_as_it_lies(kind, shift, tile, shape, k, co, stride):
+    """A filter that comes with the call, `shift` elements into a buffer that ends with it and holds NaNs around it: exact sums
+    of whole numbers, the same as over the packed filter; and again behind a filter of NaNs, which nothing may be kept of."""
+    rng = np.random.default_rng(co + shift)
+    n, h, w, ci = shape
+    I, F = (rng.integers(-5, 6, s).astype(np.float32) for s in (shape, (k, k, ci, co)))
+    dt, out, cast, onp = {'f32': (hk.F32, hk.F32, lambda a: a, np.float32), 'bf16': (hk.BF16, hk.F32, T.bf16, np.float32),
+                          'i8': (hk.I8, hk.I32, lambda a: np.nan_to_num(a, nan=77).astype(np.int8), np.int32)}[kind]
+    flat = np.full(shift + F.size + 8, np.nan, np.float32)
+    flat[shift:shift + F.size] = F.ravel()
+    oh, ow = -(-h // stride), -(-w // stride)
+    d = hk.Conv2dDesc()
+    d.in_dtype, d.out_dtype, d.c_dtype = dt, out, out
+    d.flags = hk.flag_conv(hk.CONV_IGEMM) | (hk.flag_tile(tile) if tile else 0)
+    d.n, d.h, d.w, d.ci, d.kh, d.kw, d.co, d.oh, d.ow = n, h, w, ci, k, k, co, oh, ow
+    d.stride_h = d.stride_w = stride
+    d.dil_h = d.dil_w = 1
+    d.pad_h, d.pad_w = max(0, (oh - 1) * stride + k - h) // 2, max(0, (ow - 1) * stride + k - w) // 2
+    plans = [hk.lib().pml_hip_conv2d_dispatch(ctypes.byref(d)) for _ in range(2)]
+    assert tile or 'with the filter as it lies tile=' in hk.describe(plans[0]), hk.describe(plans[0])
+    dI, dF, dN, dO = hk.DeviceBuffer.from_numpy(cast(I)), hk.DeviceBuffer.from_numpy(cast(flat)), hk.DeviceBuffer.from_numpy(cast(np.full_like(flat, np.nan))), hk.DeviceBuffer(n * oh * ow * co * 4)
+    dP = hk.DeviceBuffer.from_numpy(cast(F))
+    none, at = hk.ptr_array([]), dF.ptr + shift * cast(flat).itemsize
+    got = []
+    for f in (at, dN.ptr, at):
+        hk.check(hk.lib().pml_hip_conv2d_invoke(plans[0], dI.ptr, f, dO.ptr, None, none, none, None))
+        got.append(dO.to_numpy(onp, (n, oh, ow, co)))
+    hk.check(hk.lib().pml_hip_conv2d_pack_filter(plans[1], dP.ptr, None))
+    hk.check(hk.lib().pml_hip_conv2d_invoke(plans[1], dI.ptr, None, dO.ptr, None, none, none, None))
+    got.append(dO.to_numpy(onp, (n, oh, ow, co)))
+    for p in plans:
+        hk.lib().pml_hip_plan_free(p)
+    pad = np.zeros((n, h + 2 * k, w + 2 * k, ci))
+    pad[:, d.pad_h:d.pad_h + h, d.pad_w:d.pad_w + w] = I
+    want = sum(pad[:, y:y + (oh - 1) * stride + 1:stride, x:x + (ow - 1) * stride + 1:stride] @ F[y, x].astype(np.float64) for y in range(k) for x in range(k))
+    for g in (got[0], got[2], got[3]):
+        np.testing.assert_array_equal(g, want)
