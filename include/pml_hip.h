@@ -197,7 +197,8 @@ enum {
 #define PML_HIP_MAX_EPI_OPERANDS 6
 #define PML_HIP_MAX_RANK 6
 
-/* descriptor flag of gemm and conv2d (in_dtype F32 only): multiply fp32 operands as three bf16 products */
+/* descriptor flag of gemm and conv2d (in_dtype F32 only): fp32 operands may be multiplied as three bf16 products (products that
+ * plain fp32 MFMAs finish earlier -- few results, where latency counts -- are not) */
 #define PML_HIP_FP32_AS_BF16X3 1
 
 /* Schedule overrides, carried in `flags` of the gemm and conv2d descriptors beside the flag above (all zero: the
@@ -280,7 +281,7 @@ typedef struct {
  * Replaces plaidml_rt_xsmm_gemm_dispatch_f32 / _invoke_f32 and the bias / relu
  * variants (pmlc/rt/xsmm.cc:17-233), and the strided batch-reduce
  * plaidml_rt_xsmm_brgemm_* (:235-287).
- *   in_dtype F32  -> fp32 MFMA, fp32 accumulate; with PML_HIP_FP32_AS_BF16X3 in `flags` every operand value is
+ *   in_dtype F32  -> fp32 MFMA, fp32 accumulate; with PML_HIP_FP32_AS_BF16X3 in `flags`, but for products of few results, every operand value is
  *                    split into a bf16 head and a bf16 remainder in registers and each product is formed as
  *                    head*head + remainder*head + head*remainder on the bf16 matrix cores (fp32 accumulate):
  *                    about 2^-16 relative error per product instead of 2^-24, at several times the fp32 MFMA rate

@@ -249,6 +249,44 @@ int direct_tile_of(int64_t m, int64_t n, int64_t k_bytes, int kind, int64_t kn_l
   return small <= large ? TILE_16x16_W8 : TILE_32x32_W8;
 }
 
+// Microseconds of a 16 or 32 x 64 direct tile over a right-hand side [K][N] as it lies, from 260 timings of 130 convolutions (8 to
+// 13 % rms): 2.6, and per round of one tile on each CU (a last one that is not full counts for most of one) a start and so much per
+// KB of K -- not per byte of few columns: it is the requests for K-rows that take the time, more of them for int8, whose rows off a
+// word take two words each.
+double direct_lies_us(int64_t m, int64_t n, int64_t k_bytes, int kind, int side) {
+  const bool small = side == 16, odd = n % 4 != 0;
+  double start, per_kb;
+  if (kind == KIND_BF16) start = small ? 1.35 : 1.7, per_kb = small ? 1.17 : 1.52;
+  else if (kind == KIND_I8) start = small ? 1.3 : 1.6, per_kb = 1.2 + (!odd ? 0 : small ? 0.85 : 1.25);
+  else start = small ? 2.2 : 1.7, per_kb = small ? 1.2 : 2.3;
+  const double rounds = std::max(1.0, (double)((m + side - 1) / side) * (double)((n + 63) / 64) / device_cus());
+  return 2.6 + (0.75 * std::ceil(rounds) + 0.25 * rounds) * (start + per_kb * (double)k_bytes / 1024);
+}
+
+// Whether a product that may be taken as three bf16 products is better off in a direct tile of plain fp32 MFMAs: the split kind
+// has no direct tiles, and with few results it is latency that bounds both.  Its tiles take 4.2 us and 0.42 per slab, or split as
+// `direct_tile_of` says.  kn_ldb: pitch in bytes of a right-hand side [K][N] (0: rows of K).  us, split -> direct: 1 x 1724, K = 656 packed 9.4 -> 4.9,
+// 7 x 1293, K = 208 [N][K] 6.9 -> 5.3, 16 x 26, K = 416 [K][N] 12.8 -> 6.1, 382 x 253, K = 336 packed 9.7 -> 6.7; but 2 x 22, K = 3104
+// 15.1 (18.7), 672 x 491, K = 800 packed 12.0 (14.2).  Of 100 drawn products 54 take it, 1.51 x in the mean.
+bool fp32_beats_split(int64_t m, int64_t n, int64_t k_bytes, int64_t kn_ldb) {
+  const int64_t slabs = (k_bytes + 127) / 128;
+  double us = 0, split_us = 4.2 + 0.42 * (double)slabs;
+  bool needs_bt = n % 4 != 0 || kn_ldb % 16 != 0;
+  if (splits_k(m, n, k_bytes, KIND_F32X3)) {
+    int splits = 1, per = 0;
+    igemm_split_plan(m, n, slabs, device_cus(), &splits, &per);
+    if (splits >= 2) {
+      split_us = 5.2 + (((m + 63) / 64) * ((n + 63) / 64) <= 64 ? (double)k_bytes / 2500 : 0.5 * (double)per) + 8.0 * splits * (double)m * (double)n / 3e6;
+      needs_bt = true;
+    }
+  }
+  if (direct_tile_of(m, n, k_bytes, KIND_F32) < 0) return false;
+  (void)direct_tile_of(m, n, k_bytes, KIND_F32, 0, /*always=*/true, true, false, &us);
+  if (us > 0.95 * split_us) return false;
+  const double copy = needs_bt ? 3.0 + 2.0 * (double)k_bytes * (double)n / 2.2e6 : 0;
+  return !kn_ldb || std::min(direct_lies_us(m, n, k_bytes, KIND_F32, 16), direct_lies_us(m, n, k_bytes, KIND_F32, 32)) <= 0.95 * (split_us + copy);
+}
+
 // Stated tiling choice per shape class.  Measured on MI355X, bf16 unless said otherwise (us; w8 / w16 =
 // 8 / 16 wavefronts per workgroup; s2 = two ring stages and LDS cut to what the result tile needs, so that two
 // workgroups share a CU; the 4-wavefront 256x128 and 256x256 tiles that were tried as well are slower than
@@ -705,11 +743,8 @@ WinShape window_shape(Plan* p, bool named, double* window_us) {
 }
 
 // The direct tile of a convolution whose filter comes with the call and is read as it lies (-1: it is packed by a launch of its
-// own first): where that is cheaper than the plan's kernel and the packing.  The price is fitted to 260 timings of 130
-// convolutions (8 to 13 % rms): 2.6 us, and per round (a last one that is not full counts for most of one) of one 16 x 64 or 32 x 64 tile on each CU a start and so much per KB of K --
-// not per byte of a filter's few columns: it is the requests for K-rows that take the time, more of them for int8, whose rows
-// off a word take two words each.  fp32 sums are the same bits either way, so there it is for convolutions that take a direct
-// tile over a packed filter, too.  us a call, packing first -> as it lies:
+// own first): where that is cheaper than the plan's kernel and the packing.  fp32 sums are the same bits either way, so there it is for
+// convolutions that take a direct tile over a packed filter, too.  us a call, packing first -> as it lies:
 //   1 x 1    bf16 28 x 9 x 9 x 256 (*) 62 10.3 -> 5.9     int8 36 x 7 x 7 x 128 (*) 46 8.5 -> 4.7     fp32 3 x 9 x 9 x 96 (*) 23 stride 2 9.7 -> 6.7
 //   3 x 3    bf16 5 x 25 x 25 x 32 (*) 76 8.8 -> 5.2      int8 34 x 14 x 14 x 64 (*) 59 9.5 -> 6.0    fp32 2 x 15 x 15 x 32 (*) 37 10.2 -> 6.8
 //   5 x 5    bf16 11 x 21 x 21 x 64 (*) 102 stride 2 11.7 -> 8.7; but 2 x 69 x 69 x 64 (*) 19, two rounds, 12.2, as it lies 16.9
@@ -718,19 +753,11 @@ int given_filter_tile(const Plan* p, double window_us) {
   const pml_hip_conv2d_desc& d = p->conv;
   const int es = dt_size(d.in_dtype);
   const int64_t M = d.n * d.oh * d.ow, k_bytes = (p->patches ? p->kpad : d.kh * d.kw * d.ci) * es;
-  const bool window = p->win.config >= 0, odd = d.co % 4 != 0;
+  const bool window = p->win.config >= 0;
   if (p->mfma_kind == KIND_F32X3 || (p->mfma_kind == KIND_F32 && p->tile_direct < 0)) return -1;
-  auto lies_us = [&](int64_t side) {
-    double start, per_kb;
-    if (p->mfma_kind == KIND_BF16) start = side == 16 ? 1.35 : 1.7, per_kb = side == 16 ? 1.17 : 1.52;
-    else if (p->mfma_kind == KIND_I8) start = side == 16 ? 1.3 : 1.6, per_kb = 1.2 + (!odd ? 0 : side == 16 ? 0.85 : 1.25);
-    else start = side == 16 ? 2.2 : 1.7, per_kb = side == 16 ? 1.2 : 2.3;
-    const double rounds = std::max(1.0, (double)((M + side - 1) / side) * (double)((d.co + 63) / 64) / device_cus());
-    return 2.6 + (0.75 * std::ceil(rounds) + 0.25 * rounds) * (start + per_kb * (double)k_bytes / 1024);
-  };
   double packed_us = window_us;
   if (!window) (void)direct_tile_of(M, d.co, k_bytes, p->mfma_kind, 0, p->tile_direct >= 0, /*can_split=*/!p->patches, false, &packed_us);
-  const double small = lies_us(16), large = lies_us(32), packing = 3.0 + 2.0 * (double)k_bytes * (double)d.co / 2.2e6;
+  const double small = direct_lies_us(M, d.co, k_bytes, p->mfma_kind, 16), large = direct_lies_us(M, d.co, k_bytes, p->mfma_kind, 32), packing = 3.0 + 2.0 * (double)k_bytes * (double)d.co / 2.2e6;
   if (std::min(small, large) > (p->tile_direct >= 0 ? 0.95 : 0.85) * (packed_us + packing)) return -1;
   return small <= large ? TILE_16x16_W8 : TILE_32x32_W8;
 }
@@ -998,6 +1025,7 @@ static int gemm_desc_kind(const pml_hip_gemm_desc* d) {
     fail("gemm: a second initial value needs a second product");
     return -1;
   }
+  if (kind == KIND_F32X3 && PML_HIP_FLAG_TILE_OF(d->flags) < 0 && fp32_beats_split(d->m, d->n, d->k * es, d->b_layout ? 0 : d->ldb * es)) return KIND_F32;
   return kind;
 }
 

@@ -332,3 +332,29 @@ def test_filter_as_it_lies(kind, shift, tile, shape, k, co, stride):
     want = sum(pad[:, y:y + (oh - 1) * stride + 1:stride, x:x + (ow - 1) * stride + 1:stride] @ F[y, x].astype(np.float64) for y in range(k) for x in range(k))
     for g in (got[0], got[2], got[3]):
         np.testing.assert_array_equal(g, want)
+
+
+@pytest.mark.parametrize('layout', [0, 1])
+@pytest.mark.parametrize('M,N,K,plain', [(1, 17, 16, True), (7, 129, 208, True), (16, 26, 416, True), (100, 88, 272, True), (382, 253, 336, True),
+                                         (2, 22, 3104, False), (1300, 700, 400, False)])
+def test_split_fp32_of_few_results_is_plain_fp32(layout, M, N, K, plain):
+    """fp32 that may be taken as three bf16 products: where direct tiles of fp32 MFMAs are faster the same bits as without the flag."""
+    rng = np.random.default_rng(M + K)
+    A, B = rng.standard_normal((M, K)).astype(np.float32), rng.standard_normal((N, K) if layout else (K, N)).astype(np.float32)
+    dA, dB, dC = hk.DeviceBuffer.from_numpy(A), hk.DeviceBuffer.from_numpy(B), hk.DeviceBuffer(M * N * 4)
+    got, none = [], hk.ptr_array([])
+    for flags in (0, hk.FP32_AS_BF16X3):
+        d = hk.GemmDesc()
+        d.in_dtype = d.out_dtype = d.c_dtype = hk.F32
+        d.m, d.n, d.k, d.lda, d.ldb, d.ldc, d.b_layout, d.flags = M, N, K, K, K if layout else N, N, layout, flags
+        plan = hk.lib().pml_hip_gemm_dispatch(ctypes.byref(d))
+        if flags and (plain or not layout):
+            assert ('3 x f32' in hk.describe(plan)) != plain, hk.describe(plan)
+        hk.check(hk.lib().pml_hip_gemm_invoke(plan, dA.ptr, dB.ptr, dC.ptr, None, none, none, None))
+        got.append(dC.to_numpy(np.float32, (M, N)))
+        hk.lib().pml_hip_plan_free(plan)
+    if plain:
+        np.testing.assert_array_equal(got[0], got[1])
+    want = A.astype(np.float64) @ (B.T if layout else B).astype(np.float64)
+    # (2^-16 of every product, at random; the largest of all results within 8 of its standard deviation sqrt(K))
+    assert np.abs(got[1] - want).max() < 8 * 2.0 ** -16 * np.sqrt(K) + 1e-5
