@@ -191,13 +191,27 @@ bool splits_k(int64_t m, int64_t n, int64_t k_bytes, int kind) {
   return t <= 64 || (t <= 160 && ((kind == KIND_BF16 && k_bytes >= 5632) || (kind == KIND_F32X3 && k_bytes >= 8192)));
 }
 
+// Microseconds per 128-byte slab of K of an fp32 product in tiles through LDS: 0.58 per round of 64 x 64 tiles, or as much less per
+// result in 128 x 128 tiles as those fill their rounds better.  fp32 is bound by its MFMAs, and tiles of 128 gain 5 % at best
+// (3881 x 3959, K = 2992 723 us, 760 in tiles of 64; 2381 x 1595, K = 2608 171, 180), while half a round of them more costs as much as
+// two of 64: 3271 x 547, K = 448 36.2 -> 21.6, 2322 x 2041, K = 304 47.7 -> 35.4, 1246 x 4028, K = 208 35.6 -> 27.1, convolutions
+// 38400 x 122, K = 2304 294 -> 209, 13689 x 179, K = 3200 212 -> 168.
+bool f32_tiles_of_128(int64_t m, int64_t n) {
+  const int64_t cus = device_cus(), t128 = ((m + 127) / 128) * ((n + 127) / 128), t64 = ((m + 63) / 64) * ((n + 63) / 64);
+  return t128 >= 128 && 4 * ((t128 + cus - 1) / cus) <= (t64 + cus - 1) / cus;
+}
+double f32_slab_us(int64_t m, int64_t n) {
+  const int64_t cus = device_cus(), t128 = ((m + 127) / 128) * ((n + 127) / 128), t64 = ((m + 63) / 64) * ((n + 63) / 64);
+  return f32_tiles_of_128(m, n) ? 2.2 * (double)((t128 + cus - 1) / cus) : 0.58 * (double)((t64 + cus - 1) / cus);
+}
+
 // One of the direct tiles (direct.hip) where it beats the LDS kernels, or -1.  Both sides are priced in microseconds, from
 // measurements of 27 matrix products and 18 convolutions per element kind (one row to 3136, K of 64 to 4608; back to back
 // in a recorded graph): a direct kernel takes 2.6 plus, per round of one tile on each CU (fp32 and 32 x 64: whole
 // rounds), 0.8 (fp32 32 x 32: 1.9; 32 x 64, which replaces 32 x 32 beyond one round: bf16 1.6, int8 1.0, fp32 2.3) and its
-// operand bytes at 40 KB a microsecond and CU (32 x 64: bf16 50, int8 60, fp32 32).  An LDS kernel takes 4.2 plus its chain
-// of 128-byte slabs (0.23 each, int8 0.28, fp32 0.58), or -- K split over workgroups -- 5.2 (fp32 5.6) plus 0.4 per KB of K
-// (more than 64 tiles: 0.5 per slab of a split) plus writing and reading the partial tiles at 3 TB/s.  The prices meet the measurements to about 15 %; a direct tile has
+// operand bytes at 40 KB a microsecond and CU (32 x 64: bf16 50, int8 60, fp32, all 64 columns of a tile, 35, of several rounds 42).  An LDS kernel takes 4.2 plus its chain
+// of 128-byte slabs (0.23 each, int8 0.28, fp32 `f32_slab_us`), or -- K split over workgroups -- 5.2 plus 0.4 per KB of K
+// (more than 64 tiles: 0.5 per slab of a split; fp32: 8.5 and 0.68 per slab of a split) plus writing and reading the partial tiles at 3 TB/s.  The prices meet the measurements to about 15 %; a direct tile has
 // to be 5 % ahead.
 //   us, before -> direct                       bf16              fp32              int8
 //   1 x 1000, K = 2048                     7.4 ->  5.0       9.3 ->  7.3       6.7 ->  4.3
@@ -205,6 +219,9 @@ bool splits_k(int64_t m, int64_t n, int64_t k_bytes, int kind) {
 //   784 x 512, K = 256: 32 x 64            5.1 ( 5.4)       9.6 ->  8.5       4.8 ->  4.5
 //   28 x 28 x 128 (*) 3 x 3 x 128          9.1 ->  7.7      11.1 (12.8)        7.4 ->  5.2
 //   49 x 512, K = 4608: stays split        8.6 (11.2)       12.9 (18.7)        7.6 ( 7.4)
+// and of fp32 where tiles through LDS are priced by their rounds and a split by its slabs, as 120 products and convolutions with 5e7
+// multiply-adds and more were timed: 251 x 658, K = 848 [K][N] 18.7 -> 8.2, 836 x 2331, K = 592 46.2 -> 32.6, 214 x 271, K = 3632 17.0 -> 12.5,
+// convolutions 38 x 23 x 23 x 256 (*) 3 x 3 x 39 91.6 -> 67.0, 13 x 25 x 25 x 32 (*) 3 x 3 x 139 28.1 -> 17.0.
 // A right-hand side that arrives with the call as [K][N]: tiles are then 16 or 32 x 64 (60 KB a microsecond; fp32 45,
 // int8 36 unless rows are whole 64-byte runs), and an LDS kernel that needs Bt pays for the transposed copy besides, 3 and
 // its bytes both ways at 2.2 TB/s:
@@ -227,17 +244,17 @@ int direct_tile_of(int64_t m, int64_t n, int64_t k_bytes, int kind, int64_t kn_l
     double rounds = std::max(1.0, (double)tiles(side, wide) / n_cus);
     if ((f32 && !kn) || w) rounds = std::ceil(rounds);
     const double start = w ? (f32 ? 2.3 : kind == KIND_I8 ? 1.0 : 1.6) : f32 && !kn && side == 32 ? 1.9 : 0.8;
-    const double r = w ? (f32 ? 32e3 : kind == KIND_I8 ? 60e3 : 50e3) : rate;
-    return 2.6 + rounds * (start + (double)(std::min(m, side) + std::min(n, wide)) * kb / r);
+    const double r = w ? (f32 ? (rounds > 1 ? 42e3 : 35e3) : kind == KIND_I8 ? 60e3 : 50e3) : rate;
+    return 2.6 + rounds * (start + (double)(std::min(m, side) + (f32 && w ? wide : std::min(n, wide))) * kb / r);
   };
   const int64_t slabs = (k_bytes + 127) / 128;
-  double lds_us = 4.2 + (f32 ? 0.58 : kind == KIND_I8 ? 0.28 : 0.23) * (double)slabs;
+  double lds_us = 4.2 + (f32 ? f32_slab_us(m, n) : kind == KIND_I8 ? 0.28 : 0.23) * (double)slabs;
   bool needs_bt = !as_given && (kind == KIND_BF16 || n % (16 / es) != 0 || kn_ldb % 16 != 0);
   if (can_split && splits_k(m, n, k_bytes, kind)) {
     int splits = 1, per = 0;
     igemm_split_plan(m, n, slabs, n_cus, &splits, &per);
     if (splits >= 2) {
-      lds_us = (f32 ? 5.6 : 5.2) + (tiles(64, 64) <= 64 ? kb / 2500 : 0.5 * (double)per) + 8.0 * splits * (double)m * (double)n / 3e6;
+      lds_us = (f32 ? 8.5 + 0.68 * (double)per : 5.2 + (tiles(64, 64) <= 64 ? kb / 2500 : 0.5 * (double)per)) + 8.0 * splits * (double)m * (double)n / 3e6;
       needs_bt = true;
     }
   }
@@ -353,6 +370,7 @@ int choose_tile(int64_t m, int64_t n, int64_t k_bytes, int kind = KIND_BF16, boo
   // batch 128: the 3x3 convolutions 38.9 -> 37.3 us, the 1x1 layers with K = 1024 26.7 -> 25.3, the network 2.59 -> 2.57 ms
   // (measured with a schedule file before the rule was written down).
   if (kind == KIND_BF16 && k_bytes >= 2048 && tiles(256, 128) >= 192 && tiles(256, 128) <= 256) return TILE_256x128_W16;
+  if (kind == KIND_F32 && !f32_tiles_of_128(m, n)) return tiles(64, 64) <= 512 ? TILE_64x64_W8_K2 : TILE_64x64;
   if (tiles(128, 128) >= 256) return TILE_128x128_W8_S2;
   if (tiles(128, 128) >= 128) return TILE_128x128_W8;
   // at most two 64x64 tiles per CU and a long K: a second wavefront grid takes half of every slab

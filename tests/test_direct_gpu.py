@@ -358,3 +358,26 @@ def test_split_fp32_of_few_results_is_plain_fp32(layout, M, N, K, plain):
     want = A.astype(np.float64) @ (B.T if layout else B).astype(np.float64)
     # (2^-16 of every product, at random; the largest of all results within 8 of its standard deviation sqrt(K))
     assert np.abs(got[1] - want).max() < 8 * 2.0 ** -16 * np.sqrt(K) + 1e-5
+
+
+@pytest.mark.parametrize('M,N,K', [(251, 660, 848), (130, 2049, 80), (1250, 516, 64), (2048, 1024, 32), (2048, 2048, 32), (1030, 1990, 48), (60, 132, 1584)])
+def test_fp32_tiles_agree_in_every_layout(M, N, K):
+    """fp32 where direct tiles, tiles of 64 with K in two halves, plain ones and tiles of 128 meet: the same bits from B as it lies,
+    packed and as [N][K]."""
+    A, B = operands('f32', M, N, K, M + K)
+    dA, dB, dBt, dC = hk.DeviceBuffer.from_numpy(A), hk.DeviceBuffer.from_numpy(B), hk.DeviceBuffer.from_numpy(np.ascontiguousarray(B.T)), hk.DeviceBuffer(M * N * 4)
+    got, none = [], hk.ptr_array([])
+    for form in ('kn', 'packed', 'nk'):
+        d = hk.GemmDesc()
+        d.in_dtype = d.out_dtype = d.c_dtype = hk.F32
+        d.m, d.n, d.k, d.lda, d.ldb, d.ldc, d.b_layout = M, N, K, K, K if form == 'nk' else N, N, form == 'nk'
+        plan = hk.lib().pml_hip_gemm_dispatch(ctypes.byref(d))
+        print(hk.describe(plan), flush=True)
+        if form == 'packed':
+            hk.check(hk.lib().pml_hip_gemm_pack_b(plan, dB.ptr, None))
+        hk.check(hk.lib().pml_hip_gemm_invoke(plan, dA.ptr, {'kn': dB.ptr, 'packed': None, 'nk': dBt.ptr}[form], dC.ptr, None, none, none, None))
+        got.append(dC.to_numpy(np.float32, (M, N)))
+        hk.lib().pml_hip_plan_free(plan)
+    check(got[0], A.astype(np.float64) @ B.astype(np.float64), 'f32', K)
+    np.testing.assert_array_equal(got[0], got[1])
+    np.testing.assert_array_equal(got[0], got[2])
