@@ -348,7 +348,7 @@ int choose_tile(int64_t m, int64_t n, int64_t k_bytes, int kind = KIND_BF16, boo
     if (tiles(64, 64) <= 512 && k_bytes >= 2048) return TILE_64x64_W8_K2;
     return TILE_64x64;
   }
-  if (n <= 64) return TILE_64x64;  // (the 7x7 stem of ResNet-50 over 2x2 pixel blocks: 191 us against 207 us with 128x64w8)
+  if (n <= 64) return kind != KIND_F32 && tiles(64, 64) <= 256 ? TILE_64x64_W8_K2 : TILE_64x64;  // (the 7x7 stem of ResNet-50 over 2x2 pixel blocks: 191 us against 207 us with 128x64w8)
   // Long K, at least three quarters of a round of 256x256 tiles and little of them hanging over the edges:
   // eight wavefronts of 128x64 (0.75 KB of LDS fragment reads per MFMA instead of 1.5).  Measured with N(0,1) /
   // uniform int8 data, 4096^3: bf16 121 us against 139 (256x128, 16 wavefronts), int8 73 against 84.
@@ -372,10 +372,13 @@ int choose_tile(int64_t m, int64_t n, int64_t k_bytes, int kind = KIND_BF16, boo
   if (kind == KIND_BF16 && k_bytes >= 2048 && tiles(256, 128) >= 192 && tiles(256, 128) <= 256) return TILE_256x128_W16;
   if (kind == KIND_F32 && !f32_tiles_of_128(m, n)) return tiles(64, 64) <= 512 ? TILE_64x64_W8_K2 : TILE_64x64;
   if (tiles(128, 128) >= 256) return TILE_128x128_W8_S2;
-  if (tiles(128, 128) >= 128) return TILE_128x128_W8;
+  // (two slabs and less are all launch, first loads and tail: bf16 conv 8750 x 138, K = 64 9.4 -> 6.6 us, 23958 x 105, K = 128 9.6 -> 8.1)
+  if (tiles(128, 128) >= 128 && (kind == KIND_F32 || k_bytes > 256)) return TILE_128x128_W8;
   // at most two 64x64 tiles per CU and a long K: a second wavefront grid takes half of every slab
   // (fp32 1024^3: 32.5 -> 28.8 us; bf16 128x1000x2048: 13.4 -> 11.6 us; bf16 2048^3, 1024 tiles: 26.7 -> 40.5 us)
-  if (tiles(64, 64) <= 512 && k_bytes >= 2048) return TILE_64x64_W8_K2;
+  // (one tile a CU: whatever the K, eight wavefronts to its loads and its tail; bf16 650 x 593, K = 720 8.7 -> 7.5 us, 915 x 588,
+  // K = 224 5.9 -> 5.1, int8 2085 x 435, K = 48 5.6 -> 5.1)
+  if (tiles(64, 64) <= (k_bytes >= 2048 ? 512 : 256)) return TILE_64x64_W8_K2;
   const int64_t rounds_small = (tiles(64, 64) + 5 * 256 - 1) / (5 * 256);
   const int64_t rounds_wide = (tiles(128, 64) + 2 * 256 - 1) / (2 * 256);
   return rounds_small < 2 * rounds_wide ? TILE_64x64 : TILE_128x64;
@@ -1141,7 +1144,7 @@ static int panel_of(const pml_hip_gemm_desc& d, int kind, int tile, const Direct
   const bool wide = tile == TILE_128x128_W8 || tile == TILE_128x128_W8_S2 || tile == TILE_256x128_W16 || tile == TILE_256x256_W8 || tile == TILE_192x384_W8;
   if (kind == KIND_I8) {
     if (!wide || (d.c_dtype == PML_HIP_I32 && !(tile == TILE_128x128_W8_S2 && k_bytes >= 1024 && d.n <= 1024))) return -1;
-  } else if (!(wide && d.n > 160) && tile != TILE_64x64_W8_K2) {
+  } else if (!(wide && d.n > 160) && (tile != TILE_64x64_W8_K2 || k_bytes < 2048)) {
     return -1;
   }
   IgemmArgs g;
