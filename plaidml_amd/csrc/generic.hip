@@ -1000,17 +1000,18 @@ __global__ __launch_bounds__(256) void softmax_rows_kernel(const void* x_, void*
 
 // The same for rows of up to 4 U LANES elements: a lane keeps its U runs of four neighbouring elements in registers from
 // the one read to the one write (the walks above read the row three times and take every exponential twice), and short
-// rows have a wavefront each, which meets no barrier.  500 x 8000 fp32: 37 -> 15 us, 4096 x 1000: 20 -> 13 us.
+// rows have a wavefront each, which meets no barrier.  500 x 8000 fp32: 37 -> 15 us, 4096 x 1000: 20 -> 13 us.  Rows of up to
+// 128 elements share a wavefront: 23868 x 24 fp32 9.7 -> 4.9 us, 12288 x 128 bf16 8.9 -> 6.8.
 template <bool BF, int LANES, int U>
 __global__ __launch_bounds__(256) void softmax_regs_kernel(const void* x_, void* y_, int64_t rows, int cols) {
   __shared__ float part[4];
-  const int lane = LANES == 64 ? (int)(threadIdx.x & 63) : (int)threadIdx.x;
-  const int64_t row = (int64_t)blockIdx.x * (256 / LANES) + (LANES == 64 ? (int)(threadIdx.x >> 6) : 0);
-  if (row >= rows) return;  // (a whole wavefront of a kernel without barriers, or nobody)
+  const int lane = (int)threadIdx.x % LANES;
+  const int64_t row = (int64_t)blockIdx.x * (256 / LANES) + (int)threadIdx.x / LANES;
+  if (row >= rows) return;  // (all lanes of a row in a kernel without barriers, or nobody)
   auto rounded = [](float v) { return BF ? round_to_bf16(v) : v; };
   auto across = [&](float v, auto fold) {
 #pragma unroll
-    for (int d = 32; d > 0; d >>= 1) v = fold(v, __shfl_xor(v, d, 64));
+    for (int d = LANES < 64 ? LANES / 2 : 32; d > 0; d >>= 1) v = fold(v, __shfl_xor(v, d, 64));
     if constexpr (LANES == 256) {
       __syncthreads();
       if ((lane & 63) == 0) part[lane >> 6] = v;
@@ -1086,10 +1087,15 @@ bool softmax_in_regs(const pml_hip_softmax_desc& d, const void* x, void* y, hipS
   // a wavefront per row up to 512 columns, and up to 1024 where the rows fill the chip that way
   const bool narrow = d.cols <= 512 || (d.cols <= 1024 && d.rows >= 1024);
   const int64_t chunks = (d.cols + (narrow ? 255 : 1023)) / (narrow ? 256 : 1024);
-  const dim3 grid((unsigned)(narrow ? (d.rows + 3) / 4 : d.rows)), block(256);
-#define PML_GO(LANES, U) hipLaunchKernelGGL((softmax_regs_kernel<BF, LANES, U>), grid, block, 0, s, x, y, d.rows, (int)d.cols)
+  const dim3 block(256);
+#define PML_GO(LANES, U) \
+  hipLaunchKernelGGL((softmax_regs_kernel<BF, LANES, U>), dim3((unsigned)((d.rows + 256 / LANES - 1) / (256 / LANES))), block, 0, s, x, y, d.rows, (int)d.cols)
   if (narrow) {
-    if (chunks <= 1) PML_GO(64, 1);
+    // (rows that fill half a wavefront and less share one; the lanes that are left out added zeros, so the bits are the same)
+    if (d.cols <= 32) PML_GO(8, 1);
+    else if (d.cols <= 64) PML_GO(16, 1);
+    else if (d.cols <= 128) PML_GO(32, 1);
+    else if (chunks <= 1) PML_GO(64, 1);
     else if (chunks <= 2) PML_GO(64, 2);
     else PML_GO(64, 4);
   } else {

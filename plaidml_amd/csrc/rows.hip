@@ -36,9 +36,12 @@ __global__ __launch_bounds__(256) void rows_program_kernel(RowsProgramArgs p_by_
   const bool live = row_of < d.rows;  // (a whole wavefront; a row past the end repeats the last one and stores nothing)
   const int64_t row = live ? row_of : d.rows - 1;
   const int cols = (int)d.cols, pitch = (cols + 3) & ~3;
-  float* const scalars = lds + group * PML_HIP_ROWS_SCALARS;
-  float* const part = lds + GROUPS * PML_HIP_ROWS_SCALARS;                     // one per wavefront (LANES = 256)
-  float* const vec = part + 4 + group * (size_t)d.n_vectors * pitch;
+  // (every wavefront keeps the row's scalars for itself: a step on them meets no barrier, a reduction over a workgroup one,
+  // its partial results written to one of two places in turn)
+  float* const scalars = lds + (threadIdx.x >> 6) * PML_HIP_ROWS_SCALARS;
+  float* const part = lds + 4 * PML_HIP_ROWS_SCALARS;                          // [2][one per wavefront] (LANES = 256)
+  float* const vec = part + 8 + group * (size_t)d.n_vectors * pitch;
+  int turn = 0;
   // the steps come to LDS in one go instead of one after the other out of the argument block
   __shared__ __attribute__((aligned(16))) int steps[PML_HIP_ROWS_STEPS * sizeof(pml_hip_rows_step) / 4];
   static_assert(sizeof(pml_hip_rows_step) == 32 && sizeof steps / 4 <= 256, "one word of the program per thread");
@@ -46,13 +49,9 @@ __global__ __launch_bounds__(256) void rows_program_kernel(RowsProgramArgs p_by_
   __syncthreads();
   auto rnd = [](float x) { return BF ? round_to_bf16(x) : x; };
   auto barrier = [] {
-    if constexpr (LANES == 64) {
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    } else {
-      __syncthreads();
-    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   };
   auto one = [&](const void* base, int64_t at) { return BF ? bf16_bits_to_f32(((const uint16_t*)base)[at]) : ((const float*)base)[at]; };
   // U chunks of four columns from c0 on, LANES * 4 apart (what lies past the end: anything)
@@ -147,7 +146,7 @@ __global__ __launch_bounds__(256) void rows_program_kernel(RowsProgramArgs p_by_
       const float y[1] = {scalar(st.b_kind, st.b, st.imm)};
       apply(st.opcode, x, y);
       barrier();
-      if (lane == 0) scalars[st.dst] = x[0];
+      if ((lane & 63) == 0) scalars[st.dst] = x[0];
       barrier();
     } else if (st.kind == PML_HIP_ROWS_REDUCE) {
       const int agg = st.opcode;
@@ -164,10 +163,11 @@ __global__ __launch_bounds__(256) void rows_program_kernel(RowsProgramArgs p_by_
 #pragma unroll
         for (int w = 32; w > 0; w >>= 1) acc = fold(acc, __shfl_xor(acc, w, 64));
         if constexpr (LANES == 256) {
+          float* const at = part + turn;
+          turn ^= 4;
+          if ((lane & 63) == 0) at[lane >> 6] = acc;
           __syncthreads();
-          if ((lane & 63) == 0) part[lane >> 6] = acc;
-          __syncthreads();
-          acc = fold(fold(part[0], part[1]), fold(part[2], part[3]));
+          acc = fold(fold(at[0], at[1]), fold(at[2], at[3]));
         }
       };
       if (agg == PML_HIP_AGG_ADD) reduce([](float a, float b) { return a + b; });
@@ -175,7 +175,7 @@ __global__ __launch_bounds__(256) void rows_program_kernel(RowsProgramArgs p_by_
       else if (agg == PML_HIP_AGG_MAX) reduce([](float a, float b) { return b > a ? b : a; });
       else reduce([](float a, float b) { return b < a ? b : a; });
       barrier();
-      if (lane == 0) scalars[st.dst] = rnd(acc);
+      if ((lane & 63) == 0) scalars[st.dst] = rnd(acc);
       barrier();
     } else if (st.kind == PML_HIP_ROWS_STORE) {
       if (!live) continue;
@@ -368,11 +368,17 @@ struct SortKey {  // DT: the element type where it is one of the common ones, 0:
 size_t rows_program_lds(const pml_hip_rows_desc& d, int* lanes) {
   // A wavefront per row needs no barrier between steps, which is what a row costs most of (4096 x 1000: 35 us with a
   // workgroup per row): for short rows, and for rows of up to 2048 when there are enough of them to fill the chip that way
-  // and four of them fit the LDS (from five vectors of 2048 columns on they do not).
+  // and four of them fit the LDS (from five vectors of 2048 columns on they do not).  Fewer rows of more than 256 have a workgroup
+  // each (40 x 300 fp32 11.8 -> 9.0 us).
   const size_t pitch = (size_t)(d.cols + 3) / 4 * 4;
   auto bytes = [&](size_t groups) { return (groups * PML_HIP_ROWS_SCALARS + 4 + groups * (size_t)d.n_vectors * pitch) * 4; };
-  *lanes = d.cols <= 512 || (d.cols <= 2048 && d.rows >= 1024 && bytes(4) <= kRowsLds) ? 64 : 256;
+  *lanes = d.cols <= 256 || (d.cols <= 512 && d.rows >= 1024) || (d.cols <= 2048 && d.rows >= 1024 && bytes(4) <= kRowsLds) ? 64 : 256;
   return bytes(256 / *lanes);
+}
+// ... and what a launch takes of it: scalars for four wavefronts and their partial results twice, whatever the groups.  (At most 208
+// bytes more than what a program is accepted by, which the two KB beside `kRowsLds` hold besides the steps.)
+static size_t launch_lds(const pml_hip_rows_desc& d, int lanes) {
+  return (4 * PML_HIP_ROWS_SCALARS + 8 + (256 / lanes) * (size_t)d.n_vectors * ((size_t)(d.cols + 3) / 4 * 4)) * 4;
 }
 
 namespace {
@@ -399,9 +405,10 @@ hipError_t launch_program(const RowsProgramArgs& a, size_t lds, int64_t blocks, 
 hipError_t rows_program_launch(const RowsProgramArgs& a, hipStream_t s) {
   if (a.d.rows == 0 || a.d.cols == 0) return hipSuccess;
   int lanes = 0;
-  const size_t lds = rows_program_lds(a.d, &lanes);
+  size_t lds = rows_program_lds(a.d, &lanes);
   const int64_t blocks = (a.d.rows + 256 / lanes - 1) / (256 / lanes);
   if (blocks > kMaxLaunchThreads / 256 || lds > kRowsLds) return hipErrorInvalidValue;
+  lds = launch_lds(a.d, lanes);
   if (a.d.dtype == PML_HIP_BF16) return lanes == 64 ? launch_program<true, 64>(a, lds, blocks, s) : launch_program<true, 256>(a, lds, blocks, s);
   return lanes == 64 ? launch_program<false, 64>(a, lds, blocks, s) : launch_program<false, 256>(a, lds, blocks, s);
 }

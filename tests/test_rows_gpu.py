@@ -135,3 +135,27 @@ def test_more_rows_than_one_launch_takes(which):
     else:
         e = np.exp(x - x.max(1, keepdims=True))
         np.testing.assert_allclose(got[0], e / e.sum(1, keepdims=True), rtol=2e-6)
+
+
+@pytest.mark.parametrize('dtype', ['f32', 'bf16'])
+@pytest.mark.parametrize('cols', [1, 31, 32, 33, 64, 65, 127, 128, 129])
+@pytest.mark.parametrize('rows', [1, 7, 31, 33, 100])
+def test_softmax_of_rows_that_share_a_wavefront(dtype, rows, cols):
+    """Rows beside each other in one wavefront, the last ones missing: a row's maximum, sum, infinities and NaNs are its own."""
+    rng = np.random.default_rng(rows * 1000 + cols)
+    x = values(rng, (rows, cols), dtype) * 4
+    if dtype == 'bf16':
+        x = P.round_bf16(x)
+    x[::5] += 64                            # (rows of another size; exact in bf16 up to rounding, rounded again below)
+    if dtype == 'bf16':
+        x = P.round_bf16(x)
+    if cols > 1:
+        x[::7, cols // 2] = -np.inf
+    x[1::9, 0] = np.nan
+    got, = run(lambda X: [Pop.softmax(X, -1)], [x], dtype, 'softmax')
+    odd = np.isnan(x).any(1)
+    assert np.isnan(got[odd]).all()
+    e = np.exp(x[~odd].astype(np.float64) - x[~odd].max(-1, keepdims=True))
+    want = e / e.sum(-1, keepdims=True)
+    # (bf16: the difference, the exponential, the sum and the quotient rounded to 2^-9 each, the first of values up to 32)
+    assert np.linalg.norm(got[~odd] - want) < (4e-2 if dtype == 'bf16' else 4e-6) * np.linalg.norm(want)
