@@ -130,13 +130,30 @@ __global__ __launch_bounds__(64 * WM * WN * KS, NB >= 4 ? 2 : 4) void winconv_ke
   const int requests = (p.win_chunks + 64 * kWaves - 1) / (64 * kWaves);
   for (int q = 0; q < requests; ++q) request(q, 0);
 
-  // steps of K: 64 bytes of channels of a tap.  A wavefront takes every KS-th one of each slab.
+  // Steps of K: 64 bytes of channels of a tap.  A wavefront takes every KS-th one of each slab and counts on from one to the next:
+  // its offsets in the window and in the filter by additions alone, since the scalar instructions between two steps are a chain
+  // that blocks of few results do not cover.  With a branch per tap and products for both offsets, before -> now: int8 33 x 29 x 29 x
+  // 256 (*) 7 x 7 x 26 40.0 -> 30.5 us, bf16 14 x 14 x 14 x 32 (*) 7 x 7 x 178 11.7 -> 9.3, 8 x 37 x 37 x 128 (*) 7 x 7 x 115 36.5 -> 32.5,
+  // 8 x 28 x 28 x 128 (*) 3 x 3 x 128 8.4 -> 8.0, 3 x 14 x 14 x 256 (*) 3 x 3 x 256 8.6 -> 8.3; 65 drawn ones 1.03 x.
   struct Step {
     int slab, ky, kx, blk;
+    int off, b;  // bytes from the window's begin; from the begin of the filter's columns
   };
-  auto blocks_of = [&](int slab) { return slab == p.slabs - 1 ? p.last_blocks : p.blocks; };
-  auto settle = [&](Step& s) {  // carries blk into kx and ky; whether the step is in its slab
-    const int nb = blocks_of(s.slab);
+  // of a slab: its blocks; what a tap to the right, and the first tap of the next row, add to what KS blocks do
+  int nb = 0, tap_off = 0, tap_b = 0, far_x = 0, far_blk = 0, far_off = 0, far_b = 0;
+  bool far = false;
+  const int row_off = p.row_step - p.KW * p.tap_step;
+  auto begin = [&](int slab) {
+    nb = slab == p.slabs - 1 ? p.last_blocks : p.blocks;
+    tap_off = p.tap_step - nb * kBlockBytes;
+    tap_b = (p.total_blocks - nb) * 2048;
+    // (KS blocks are several taps, or one of a long row: no branch per tap)
+    far = nb < KS || (nb == KS && p.KW >= 5);
+    far_x = far ? (nb == KS || nb == 3 ? 1 : nb == 2 ? KS / 2 : KS) : 0;
+    far_blk = KS - far_x * nb;
+    far_off = far_x * p.tap_step + far_blk * kBlockBytes;
+    far_b = KS * 2048 + far_x * tap_b;
+    Step s{slab, 0, 0, kg, 0, 0};
     while (s.blk >= nb) {
       s.blk -= nb;
       if (++s.kx == p.KW) {
@@ -144,14 +161,41 @@ __global__ __launch_bounds__(64 * WM * WN * KS, NB >= 4 ? 2 : 4) void winconv_ke
         ++s.ky;
       }
     }
-    return s.ky < p.KH;
-  };
-  auto begin = [&](int slab) {
-    Step s{slab, 0, 0, kg};
-    (void)settle(s);
+    s.off = s.ky * p.row_step + s.kx * p.tap_step + s.blk * kBlockBytes;
+    s.b = ((s.ky * p.KW + s.kx) * p.total_blocks + slab * p.blocks + s.blk) * 2048;
     return s;
   };
-  auto lds_at = [&](const Step& s) { return (s.slab & 1) * p.win_bytes + s.ky * p.row_step + s.kx * p.tap_step + s.blk * kBlockBytes; };
+  auto count_on = [&](Step& s) {  // whether there is another step in the slab
+    if (far) {
+      s.blk += far_blk;
+      const bool over = s.blk >= nb;
+      s.blk -= over ? nb : 0;
+      s.kx += far_x + (over ? 1 : 0);
+      s.off += far_off + (over ? tap_off : 0);
+      s.b += far_b + (over ? tap_b : 0);
+      while (s.kx >= p.KW) {
+        s.kx -= p.KW;
+        ++s.ky;
+        s.off += row_off;
+      }
+    } else {
+      s.blk += KS;
+      s.off += KS * kBlockBytes;
+      s.b += KS * 2048;
+      if (s.blk >= nb) {
+        s.blk -= nb;
+        s.off += tap_off;
+        s.b += tap_b;
+        if (++s.kx == p.KW) {
+          s.kx = 0;
+          ++s.ky;
+          s.off += row_off;
+        }
+      }
+    }
+    return s.ky < p.KH;
+  };
+  auto lds_at = [&](const Step& s) { return (s.slab & 1) * p.win_bytes + s.off; };
 
   // filter fragments as winconv_pack_kernel lays them out: a step's 32 columns are 2 KB
   const int group_bytes = p.KH * p.KW * p.total_blocks * 2048;
@@ -160,10 +204,9 @@ __global__ __launch_bounds__(64 * WM * WN * KS, NB >= 4 ? 2 : 4) void winconv_ke
   for (int j = 0; j < NB / 2; ++j) b_group[j] = min(n0 / 32 + j, (p.N - 1) / 32) * group_bytes;
   i32x4_t fa[MB], fb[2][NB];
   auto request_b = [&](i32x4_t (&f)[NB], const Step& s) {
-    const int at = ((s.ky * p.KW + s.kx) * p.total_blocks + s.slab * p.blocks + s.blk) * 2048;
 #pragma unroll
     for (int j = 0; j < NB; ++j)
-      f[j] = __builtin_bit_cast(i32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rb, lane * 16 + (j & 1) * 1024, b_group[j >> 1] + at, 0));
+      f[j] = __builtin_bit_cast(i32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rb, lane * 16 + (j & 1) * 1024, b_group[j >> 1] + s.b, 0));
   };
 
   unsigned a_lane[MB];
@@ -206,14 +249,13 @@ __global__ __launch_bounds__(64 * WM * WN * KS, NB >= 4 ? 2 : 4) void winconv_ke
   auto body = [&](auto parity) {
     constexpr int P = decltype(parity)::value;
     const int slab = nxt.slab;
-    nxt.blk += KS;
     bool fresh = false;
-    if (!settle(nxt)) {
+    if (!count_on(nxt)) {
       fresh = true;
       if (slab + 1 < p.slabs) nxt = begin(slab + 1);
       else {
         more = false;
-        nxt = Step{slab, 0, 0, 0};
+        nxt = Step{slab, 0, 0, 0, 0, 0};
       }
     }
     const int at = lds_at(nxt);

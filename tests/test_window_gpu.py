@@ -192,3 +192,15 @@ def test_every_configuration(kind, n, hw, ci, co, k, s, columns, wavefronts, blo
     I, F, bias = whole(rng, (n, hw, hw, ci), 2), whole(rng, (k, k, ci, co), 1), whole(rng, co, 50)
     geometry = ((o, o), (s, s), (1, 1), (p, p))
     compare(kind, run(kind, I, F, *geometry, bias=bias, relu=True, tile='%d wavefronts of %s%s)' % (wavefronts, block, shared)), reference(I, F, *geometry, bias=bias, relu=True))
+
+
+# 64-byte blocks of channels fewer than the wavefronts that share K, as many, and more; filter rows of fewer taps than a step counts on
+@pytest.mark.parametrize('kind', ['f32', 'bf16', 'i8'])
+@pytest.mark.parametrize('vectors,kh,kw', [(4, 2, 2), (4, 7, 1), (4, 1, 7), (8, 3, 1), (8, 2, 3), (12, 1, 4), (12, 7, 2), (16, 4, 1), (16, 1, 5), (16, 5, 5), (20, 2, 1), (28, 3, 2), (36, 1, 3)])
+def test_steps_counted_over_blocks_and_taps(kind, vectors, kh, kw):
+    rng = np.random.default_rng(vectors * 100 + kh * 10 + kw)
+    ci, n, h, w, co = vectors * {'f32': 4, 'bf16': 8, 'i8': 16}[kind], 2, 9, 8, 20
+    pad = ((kh - 1) // 2, (kw - 1) // 2)
+    I, F = whole(rng, (n, h, w, ci)), whole(rng, (kh, kw, ci, co), 2)
+    geometry = ((h, w), (1, 1), (1, 1), pad)
+    compare(kind, run(kind, I, F, *geometry), reference(I, F, *geometry))
