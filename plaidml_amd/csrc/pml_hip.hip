@@ -331,7 +331,8 @@ bool fp32_beats_split(int64_t m, int64_t n, int64_t k_bytes, int64_t kn_ldb) {
 // that; and for small problems the smaller of 64x64 and 128x64 by (rounds of resident workgroups) x
 // (tile area), the larger tile on a tie.
 // forced: a tile named by the descriptor's schedule bits (PML_HIP_FLAG_TILE), -1 = none
-int choose_tile(int64_t m, int64_t n, int64_t k_bytes, int kind = KIND_BF16, bool plain_tail = true, int forced = -1, bool allow_split = true) {
+// bare_tail: start values, ReLU and requantisation at most
+int choose_tile(int64_t m, int64_t n, int64_t k_bytes, int kind = KIND_BF16, bool plain_tail = true, int forced = -1, bool allow_split = true, bool bare_tail = false) {
   if (forced >= 0 && forced < PML_HIP_TILE_COUNT_ && (forced != TILE_128x64_N2 || kind == KIND_F32X3) &&
       (forced != TILE_192x384_W8 || kind == KIND_BF16 || kind == KIND_I8))
     return forced;
@@ -348,7 +349,7 @@ int choose_tile(int64_t m, int64_t n, int64_t k_bytes, int kind = KIND_BF16, boo
     if (tiles(64, 64) <= 512 && k_bytes >= 2048) return TILE_64x64_W8_K2;
     return TILE_64x64;
   }
-  if (n <= 64) return kind != KIND_F32 && tiles(64, 64) <= 256 ? TILE_64x64_W8_K2 : TILE_64x64;  // (the 7x7 stem of ResNet-50 over 2x2 pixel blocks: 191 us against 207 us with 128x64w8)
+  if (n <= 64) return kind != KIND_F32 && bare_tail && tiles(64, 64) <= 256 ? TILE_64x64_W8_K2 : TILE_64x64;  // (the 7x7 stem of ResNet-50 over 2x2 pixel blocks: 191 us against 207 us with 128x64w8)
   // Long K, at least three quarters of a round of 256x256 tiles and little of them hanging over the edges:
   // eight wavefronts of 128x64 (0.75 KB of LDS fragment reads per MFMA instead of 1.5).  Measured with N(0,1) /
   // uniform int8 data, 4096^3: bf16 121 us against 139 (256x128, 16 wavefronts), int8 73 against 84.
@@ -377,8 +378,9 @@ int choose_tile(int64_t m, int64_t n, int64_t k_bytes, int kind = KIND_BF16, boo
   // at most two 64x64 tiles per CU and a long K: a second wavefront grid takes half of every slab
   // (fp32 1024^3: 32.5 -> 28.8 us; bf16 128x1000x2048: 13.4 -> 11.6 us; bf16 2048^3, 1024 tiles: 26.7 -> 40.5 us)
   // (one tile a CU: whatever the K, eight wavefronts to its loads and its tail; bf16 650 x 593, K = 720 8.7 -> 7.5 us, 915 x 588,
-  // K = 224 5.9 -> 5.1, int8 2085 x 435, K = 48 5.6 -> 5.1)
-  if (tiles(64, 64) <= (k_bytes >= 2048 ? 512 : 256)) return TILE_64x64_W8_K2;
+  // K = 224 5.9 -> 5.1, int8 2085 x 435, K = 48 5.6 -> 5.1.  Not under a residual or scale and shift, whose operands it waits for with
+  // half the tiles' wavefronts on a CU: 648 x 632, K = 632 with scale, shift, ReLU in its block 16.4 us, 17.1; ResNet-50 on one image 375, 384)
+  if (tiles(64, 64) <= (k_bytes >= 2048 ? 512 : bare_tail ? 256 : 0)) return TILE_64x64_W8_K2;
   const int64_t rounds_small = (tiles(64, 64) + 5 * 256 - 1) / (5 * 256);
   const int64_t rounds_wide = (tiles(128, 64) + 2 * 256 - 1) / (2 * 256);
   return rounds_small < 2 * rounds_wide ? TILE_64x64 : TILE_128x64;
@@ -1203,7 +1205,7 @@ int64_t pml_hip_gemm_dispatch(const pml_hip_gemm_desc* d) {
     int mode = 0, relu = 0;
     classify_tail(d->tail, d->out_dtype, d->c_dtype, &mode, &relu);
     const bool plain = mode == 1 || mode == 2 || tail_requant(d->tail, d->out_dtype, d->c_dtype, mode, nullptr);
-    p->tile = choose_tile(d->m, d->n, (d->k + d->k2) * dt_size(d->in_dtype), kind, plain, PML_HIP_FLAG_TILE_OF(d->flags));
+    p->tile = choose_tile(d->m, d->n, (d->k + d->k2) * dt_size(d->in_dtype), kind, plain, PML_HIP_FLAG_TILE_OF(d->flags), true, plain && mode != 2);
     // (a second product's slabs follow the first one's on the slab axis the splits share out.)  With a direct tile over rows
     // that are at hand the LDS tile is only left for a [K][N] right-hand side that arrives with the call and cannot be read
     // as it lies; pml_hip_gemm_pack_b ends that.
@@ -1485,7 +1487,7 @@ int pml_hip_gemm_run_static(const pml_hip_gemm_desc* d, const void* a, const voi
   classify_tail(d->tail, d->out_dtype, d->c_dtype, &mode, &relu);
   const bool plain = mode == 1 || mode == 2 || tail_requant(d->tail, d->out_dtype, d->c_dtype, mode, nullptr);
   // (no workspace may be allocated here: the K loop is never split over workgroups)
-  const int tile = choose_tile(d->m, d->n, d->k * dt_size(d->in_dtype), kind, plain, PML_HIP_FLAG_TILE_OF(d->flags), /*allow_split=*/false);
+  const int tile = choose_tile(d->m, d->n, d->k * dt_size(d->in_dtype), kind, plain, PML_HIP_FLAG_TILE_OF(d->flags), /*allow_split=*/false, plain && mode != 2);
   const DirectTiles direct = direct_tiles(*d, kind, tile);
   PanelRoom panel;
   if (bt && (panel.config = panel_of(*d, kind, tile, direct, nullptr)) >= 0 && packs_given(*d, kind, tile) && panel_bytes(*d, kind) <= PML_HIP_STATIC_SCRATCH_BYTES)
@@ -1559,7 +1561,9 @@ int64_t pml_hip_conv2d_dispatch(const pml_hip_conv2d_desc* d) {
   p->conv = *d;
   const int64_t M = d->n * d->oh * d->ow;
   const int64_t K = d->kh * d->kw * d->ci;
-  p->tile = choose_tile(M, d->co, K * es, kind, false, PML_HIP_FLAG_TILE_OF(d->flags));
+  int mode = 0, relu = 0;
+  classify_tail(d->tail, d->out_dtype, d->c_dtype, &mode, &relu);
+  p->tile = choose_tile(M, d->co, K * es, kind, false, PML_HIP_FLAG_TILE_OF(d->flags), true, mode == 1);
   p->bt_ld = K;
   if (via_s2d) {
     const int v = 16 / es;
@@ -1569,7 +1573,7 @@ int64_t pml_hip_conv2d_dispatch(const pml_hip_conv2d_desc* d) {
     p->s2d_ka = (int)(d->kh + (d->pad_h & 1) + 1) / 2;
     p->s2d_kaw = (int)(d->kw + (d->pad_w & 1) + 1) / 2;
     const int64_t k2 = (int64_t)p->s2d_ka * p->s2d_kaw * p->s2d_ch;
-    p->tile = choose_tile(M, d->co, k2 * es, kind, false, PML_HIP_FLAG_TILE_OF(d->flags), /*allow_split=*/false);
+    p->tile = choose_tile(M, d->co, k2 * es, kind, false, PML_HIP_FLAG_TILE_OF(d->flags), /*allow_split=*/false, mode == 1);
     p->bt_ld = k2;
     p->via_s2d = true;
   }

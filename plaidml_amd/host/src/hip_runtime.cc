@@ -60,7 +60,10 @@ class HipExecutable final : public Executable {
           device_[i] = static_cast<char*>(arena_) + offsets[i];
           continue;
         }
-        hipCheck(pml_hip_malloc(&device_[i], b.bytes + 16), "pml_hip_malloc");
+        // (the first one holds the counter of the kernel that marks a run's end, too: an allocation of its own took preparing 0.1 ms)
+        const size_t room = arrived_ ? 0 : 64;
+        hipCheck(pml_hip_malloc(&device_[i], b.bytes + 16 + 2 * room), "pml_hip_malloc");
+        if (room) arrived_ = static_cast<char*>(device_[i]) + (b.bytes + 16 + room - 1) / room * room;
         owned_[i] = true;
         fixed_bytes_ += padded(b.bytes);
         if (b.kind == BufferInfo::Constant)
@@ -77,10 +80,9 @@ class HipExecutable final : public Executable {
       clock_khz_ = pml_hip_clock_khz();
       void* stamps = nullptr;
       if (clock_khz_ > 0 && pml_hip_host_alloc(&stamps, 3 * sizeof(uint64_t)) == 0) stamps_ = static_cast<uint64_t*>(stamps);
-      if (stamps_) {
+      if (stamps_ && arrived_) {
         mark_ = reinterpret_cast<uint32_t*>(stamps_ + 2);
         *mark_ = 0;
-        hipCheck(pml_hip_malloc(&arrived_, sizeof(uint32_t)), "pml_hip_malloc");
         hipCheck(pml_hip_fill_u32(arrived_, 0, 1, nullptr), "fill");
       }
       hipCheck(pml_hip_event_create(&ev0_), "event");
@@ -940,7 +942,6 @@ class HipExecutable final : public Executable {
     if (ev0_) pml_hip_event_destroy(ev0_);
     if (ev1_) pml_hip_event_destroy(ev1_);
     ev0_ = ev1_ = nullptr;
-    if (arrived_) pml_hip_free(arrived_);
     arrived_ = nullptr;
     if (stamps_) pml_hip_host_free(stamps_);
     stamps_ = nullptr;
