@@ -733,7 +733,8 @@ void s2d_args(const Plan* p, S2dArgs& a) {
 // Whether and how a convolution runs over its window in LDS (winconv.hip) in the place of an implicit GEMM.
 //   * an implicit GEMM fetches every pixel once per tap: bf16 and int8 always run over windows, 1.2 to 2.6 x as fast (bf16 128 x
 //     28 x 28 x 128 (*) 3 x 3 x 128 44 -> 31 us, 103 x 11 x 11 x 256 (*) 7 x 7 x 29 74.8 -> 28.3).  fp32 is bound by its MFMAs: where
-//     they are not mostly work done for edges, which a tile of 448 x 64 has more of than one of 64 x 64.
+//     they are not mostly work done for edges, which a tile of 448 x 64 has more of than one of 64 x 64, or where the rounds of tiles
+//     that an implicit GEMM takes cost more (16 x 56 x 56 x 64 (*) 3 x 3 x 64, 3.06 rounds, 44.8 -> 39.2 us, 8 x 40 x 40 x 64 (*) 7 x 7 x 45 72.6 -> 66.3).
 //   * a direct tile, or a K loop split over workgroups, is left where the window is cheaper by these kernels' prices, which are
 //     a microsecond below what launches back to back take (bf16 22 x 11 x 11 x 128 (*) 5 x 5 x 86 15.3 -> 10.4 from a split;
 //     11 x 11 x 11 x 64 (*) 3 x 3 x 20 stays, 5.5 both ways; 3 x 30 x 30 x 256 (*) 7 x 7 x 18 stride 2 stays, 14.6, over windows 34.6).
@@ -760,7 +761,8 @@ WinShape window_shape(Plan* p, bool named, double* window_us) {
   }
   if (p->mfma_kind == KIND_F32) {
     const double mma_us = (double)((g.M + 63) / 64 * 64) * (double)((g.N + 63) / 64 * 64) * (double)g.K * 2 / 154e6;
-    return us < 4 + 1.45 * mma_us ? shape : WinShape{};
+    const double tiles_us = 4.2 + f32_slab_us(g.M, g.N) * (double)conv_slabs(d);
+    return us < std::max(4 + 1.45 * mma_us, 0.93 * tiles_us) ? shape : WinShape{};
   }
   return shape;
 }
