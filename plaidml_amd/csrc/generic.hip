@@ -725,15 +725,6 @@ __global__ __launch_bounds__(256) void copy_spans_kernel(SpanArgs a) {
   }
   for (size_t i = n_vec * 16 + first; i < a.bytes[blockIdx.y]; i += stride) dst[i] = src[i];
   if (stamps && a.stamp_after) *a.stamp = wall_clock64();
-  if (!a.mark) return;
-  // The last workgroup through tells the host, which looks for `value` instead of waiting for the stream: 2.7 us less a run of one
-  // to four launches, 13 less where ten commands and more are queued (which take hipStreamSynchronize that much longer).
-  __threadfence_system();
-  __syncthreads();
-  if (threadIdx.x != 0) return;
-  if (__hip_atomic_fetch_add(a.arrived, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) != gridDim.x * gridDim.y - 1) return;
-  __hip_atomic_store(a.arrived, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  __hip_atomic_store(a.mark, a.value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 inline unsigned grid_for(int64_t work_items) {
@@ -1120,7 +1111,7 @@ hipError_t softmax_launch(const pml_hip_softmax_desc& d, const void* x, void* y,
 }
 
 hipError_t copy_spans_launch(const SpanArgs& a, hipStream_t s) {
-  if (a.n <= 0 && !a.stamp && !a.mark) return hipSuccess;
+  if (a.n <= 0 && !a.stamp) return hipSuccess;
   size_t most = 0;
   for (int i = 0; i < a.n; ++i) most = most < a.bytes[i] ? a.bytes[i] : most;
   size_t blocks = (most / 16 + 4 * 256 - 1) / (4 * 256);

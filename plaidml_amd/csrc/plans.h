@@ -314,9 +314,6 @@ struct SpanArgs {
   size_t bytes[kMaxSpans];
   int n, stamp_after;
   uint64_t* stamp;  // the device's clock goes here, before or after the copies; or null
-  uint32_t* mark;   // `value` goes here, in page-locked memory, when the copies are made and the host can see them; or null
-  uint32_t* arrived;  // with `mark`: workgroups that are through, 0 between launches
-  uint32_t value;
 };
 hipError_t copy_spans_launch(const SpanArgs& a, hipStream_t s);
 hipError_t fill_u32_launch(void* p, uint32_t pattern, size_t n_words, hipStream_t s);

@@ -6,7 +6,6 @@
 #include <algorithm>
 #include <cmath>
 #include <atomic>
-#include <chrono>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -804,26 +803,6 @@ hipError_t pack_conv_filter(Plan* p, const void* filter, hipStream_t s) {
   return hipSuccess;
 }
 
-// n copies, kMaxSpans a launch; the clock (of `form`) with the first or the last of them, the mark with the last.
-int copy_spans(int n, void* const* dst, const void* const* src, const size_t* nbytes, const SpanArgs& form, pml_hip_stream s) {
-  if (n < 0 || (n > 0 && (!dst || !src || !nbytes))) return fail("copy_spans: bad argument");
-  for (int i = 0; i == 0 || i < n; i += kMaxSpans) {
-    SpanArgs a = form;
-    for (int j = i; j < n && j < i + kMaxSpans; ++j) {
-      if (nbytes[j] == 0) continue;
-      if (!dst[j] || !src[j]) return fail("copy_spans: null pointer");
-      a.dst[a.n] = dst[j];
-      a.src[a.n] = src[j];
-      a.bytes[a.n++] = nbytes[j];
-    }
-    const bool last = i + kMaxSpans >= n;
-    if (form.stamp_after ? !last : i > 0) a.stamp = nullptr;
-    if (!last) a.mark = nullptr;
-    if (check(copy_spans_launch(a, (hipStream_t)s), "copy_spans_launch")) return 1;
-  }
-  return 0;
-}
-
 }  // namespace
 }  // namespace pml
 
@@ -891,36 +870,26 @@ int pml_hip_memcpy_d2h_async(void* dst, const void* src, size_t nbytes, pml_hip_
   return nbytes ? check(hipMemcpyAsync(dst, src, nbytes, hipMemcpyDeviceToHost, (hipStream_t)s), "hipMemcpyAsync(d2h)") : 0;
 }
 int pml_hip_copy_spans(int n, void* const* dst, const void* const* src, const size_t* nbytes, pml_hip_stream s) {
-  return copy_spans(n, dst, src, nbytes, {}, s);
+  return pml_hip_copy_spans_stamped(n, dst, src, nbytes, nullptr, 0, s);
 }
 int pml_hip_copy_spans_stamped(int n, void* const* dst, const void* const* src, const size_t* nbytes, uint64_t* stamp, int after,
                                pml_hip_stream s) {
-  SpanArgs a = {};
-  a.stamp = stamp;
-  a.stamp_after = after;
-  return copy_spans(n, dst, src, nbytes, a, s);
-}
-int pml_hip_copy_spans_marked(int n, void* const* dst, const void* const* src, const size_t* nbytes, uint64_t* stamp, uint32_t* mark,
-                              uint32_t* arrived, uint32_t value, pml_hip_stream s) {
-  if (!mark || !arrived) return fail("copy_spans: bad argument");
-  SpanArgs a = {};
-  a.stamp = stamp;
-  a.mark = mark;
-  a.arrived = arrived;
-  a.value = value;
-  return copy_spans(n, dst, src, nbytes, a, s);
-}
-int pml_hip_wait_mark(const uint32_t* mark, uint32_t value, pml_hip_stream s) {
-  if (!mark) return fail("wait_mark: null pointer");
-  using clock = std::chrono::steady_clock;
-  const clock::time_point until = clock::now() + std::chrono::milliseconds(1);
-  do {
-    for (int i = 0; i < 64; ++i) {
-      if (__atomic_load_n(mark, __ATOMIC_ACQUIRE) == value) return 0;
-      __builtin_ia32_pause();
+  if (n < 0 || (n > 0 && (!dst || !src || !nbytes))) return fail("copy_spans: bad argument");
+  for (int i = 0; i == 0 || i < n; i += kMaxSpans) {
+    SpanArgs a;
+    std::memset(&a, 0, sizeof a);
+    for (int j = i; j < n && j < i + kMaxSpans; ++j) {
+      if (nbytes[j] == 0) continue;
+      if (!dst[j] || !src[j]) return fail("copy_spans: null pointer");
+      a.dst[a.n] = dst[j];
+      a.src[a.n] = src[j];
+      a.bytes[a.n++] = nbytes[j];
     }
-  } while (clock::now() < until);
-  return pml_hip_stream_sync(s);
+    if (after ? i + kMaxSpans >= n : i == 0) a.stamp = stamp;
+    a.stamp_after = after;
+    if (check(copy_spans_launch(a, (hipStream_t)s), "copy_spans_launch")) return 1;
+  }
+  return 0;
 }
 int pml_hip_clock_khz(void) {
   int dev = 0, khz = 0;

@@ -60,10 +60,7 @@ class HipExecutable final : public Executable {
           device_[i] = static_cast<char*>(arena_) + offsets[i];
           continue;
         }
-        // (the first one holds the counter of the kernel that marks a run's end, too: an allocation of its own took preparing 0.1 ms)
-        const size_t room = arrived_ ? 0 : 64;
-        hipCheck(pml_hip_malloc(&device_[i], b.bytes + 16 + 2 * room), "pml_hip_malloc");
-        if (room) arrived_ = static_cast<char*>(device_[i]) + (b.bytes + 16 + room - 1) / room * room;
+        hipCheck(pml_hip_malloc(&device_[i], b.bytes + 16), "pml_hip_malloc");
         owned_[i] = true;
         fixed_bytes_ += padded(b.bytes);
         if (b.kind == BufferInfo::Constant)
@@ -79,12 +76,7 @@ class HipExecutable final : public Executable {
       // (two events around the launches cost a run 8 us); with events where that cannot be had, and under PLAIDML_PROFILE.
       clock_khz_ = pml_hip_clock_khz();
       void* stamps = nullptr;
-      if (clock_khz_ > 0 && pml_hip_host_alloc(&stamps, 3 * sizeof(uint64_t)) == 0) stamps_ = static_cast<uint64_t*>(stamps);
-      if (stamps_ && arrived_) {
-        mark_ = reinterpret_cast<uint32_t*>(stamps_ + 2);
-        *mark_ = 0;
-        hipCheck(pml_hip_fill_u32(arrived_, 0, 1, nullptr), "fill");
-      }
+      if (clock_khz_ > 0 && pml_hip_host_alloc(&stamps, 2 * sizeof(uint64_t)) == 0) stamps_ = static_cast<uint64_t*>(stamps);
       hipCheck(pml_hip_event_create(&ev0_), "event");
       hipCheck(pml_hip_event_create(&ev1_), "event");
       hipCheck(pml_hip_stream_create(&stream_), "stream");
@@ -125,8 +117,7 @@ class HipExecutable final : public Executable {
   //            the executable's page-locked staging, a few megabytes at a time, so that the link carries one piece
   //            while the host passes over the next.
   //   outputs  the mirror image: pieces are passed on as they arrive, the last ones after the wait.
-  // Short transfers are made by one kernel each way (pml_hip_copy_spans), long ones by the copy engines.  Where all results are
-  // short, the wait is for the mark that kernel leaves in host memory.
+  // Short transfers are made by one kernel each way (pml_hip_copy_spans), long ones by the copy engines.
   double invokeHost(const std::vector<HostSpan>& inputs, const std::vector<HostSpan>& outputs) override {
     hipCheck(pml_hip_init(ordinal_), "pml_hip_init");
     if (inputs.size() != plan_->input_buffers.size() || outputs.size() != plan_->output_buffers.size())
@@ -195,13 +186,8 @@ class HipExecutable final : public Executable {
         else
           unstaged.push_back(i);
       }
-      // where the last copies are that kernel's it marks them as made, and the host looks for that
-      const bool marks = end && mark_ && !down.dst.empty();
-      if (marks)
-        down.mark(stream_, end, mark_, static_cast<uint32_t*>(arrived_), ++marks_);
-      else
-        down.issue(stream_, end, false);
-      collect(&stage, arriving, marks);
+      down.issue(stream_, end, false);
+      collect(&stage, arriving);
     } catch (...) {
       (void)pml_hip_stream_sync(stream_);  // queued copies may still use the caller's memory
       throw;
@@ -253,10 +239,7 @@ class HipExecutable final : public Executable {
   };
   std::vector<Handles> handles_, last_handles_;  // per step; of the sliced ones' last, shorter part
   pml_hip_event ev0_ = nullptr, ev1_ = nullptr;
-  uint64_t* stamps_ = nullptr;  // page-locked: the device's clock ahead of and behind a run's launches, and
-  uint32_t* mark_ = nullptr;    // ... the number of the last run whose results are down
-  void* arrived_ = nullptr;     // (what the kernel that writes it counts with)
-  uint32_t marks_ = 0;
+  uint64_t* stamps_ = nullptr;  // page-locked: the device's clock ahead of and behind a run's launches
   int clock_khz_ = 0;
   std::vector<pml_hip_event> step_events_;
   pml_hip_stream stream_ = nullptr;  // every copy and launch of this executable
@@ -287,9 +270,6 @@ class HipExecutable final : public Executable {
     void issue(pml_hip_stream stream, uint64_t* stamp, bool after) {
       if (!dst.empty() || stamp)
         hipCheck(pml_hip_copy_spans_stamped(static_cast<int>(dst.size()), dst.data(), src.data(), bytes.data(), stamp, after ? 1 : 0, stream), "copy");
-    }
-    void mark(pml_hip_stream stream, uint64_t* stamp, uint32_t* mark, uint32_t* arrived, uint32_t value) {
-      hipCheck(pml_hip_copy_spans_marked(static_cast<int>(dst.size()), dst.data(), src.data(), bytes.data(), stamp, mark, arrived, value, stream), "copy");
     }
   };
 
@@ -415,7 +395,7 @@ class HipExecutable final : public Executable {
   // Waits for everything queued and passes on what comes back through the staging: pieces that go through the slots while
   // the ones behind them are on the link, the others at the end.  (A piece may go into its slot right away: the uploads
   // from there are before it on the stream.)
-  void collect(Staging* stage, const std::vector<Piece>& pieces, bool marked = false) {
+  void collect(Staging* stage, const std::vector<Piece>& pieces) {
     std::vector<const Piece*> in_turn;
     for (const Piece& p : pieces)
       if (!p.at) in_turn.push_back(&p);
@@ -439,7 +419,7 @@ class HipExecutable final : public Executable {
       each(h, [&](const Piece& p, char* slot) { pass(slot, p); });
       if (h + 2 < halves) send(h + 2);
     }
-    hipCheck(marked ? pml_hip_wait_mark(mark_, marks_, stream_) : pml_hip_stream_sync(stream_), "stream sync");
+    hipCheck(pml_hip_stream_sync(stream_), "stream sync");
     for (const Piece& p : pieces)
       if (p.at) pass(p.at, p);
   }
@@ -942,7 +922,6 @@ class HipExecutable final : public Executable {
     if (ev0_) pml_hip_event_destroy(ev0_);
     if (ev1_) pml_hip_event_destroy(ev1_);
     ev0_ = ev1_ = nullptr;
-    arrived_ = nullptr;
     if (stamps_) pml_hip_host_free(stamps_);
     stamps_ = nullptr;
     if (graph_) pml_hip_graph_destroy(graph_);

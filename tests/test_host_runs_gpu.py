@@ -1,9 +1,11 @@
 """Runs on arrays in host memory (host/src/hip_runtime.cc, Runner) around the edges of their staging."""
 import ctypes
 import threading
+import time
 
 import numpy as np
 import pytest
+import torch
 
 from plaidml_amd import edsl as P
 from plaidml_amd import hipkernels as hk
@@ -170,3 +172,28 @@ def test_arrays_that_do_not_fit_are_refused():
     with pytest.raises(Exception):
         runner.run([x])
     _check(runner.run([x, y]), [x, y], 'f32')
+
+
+@pytest.mark.parametrize('layers', [1, 4, 10])
+def test_a_call_leaves_nothing_to_whoever_waits_next(layers):
+    """A call on host arrays returns when its stream is through: waiting for the device behind it takes what it takes again at once."""
+    rng = np.random.default_rng(layers)
+    X = P.Placeholder(P.DType.FLOAT32, [20, 64])
+    x, i, j, k = X, *P.TensorIndexes(3)
+    for _ in range(layers):
+        W = P.Constant(rng.standard_normal((64, 64)).astype(np.float32) / 8, P.DType.FLOAT32)
+        x = P.Contraction().outShape(20, 64).outAccess(i, j).sum(x[i, k] * W[k, j]).build()
+    runner = P.Runner(P.Program('layers', [X], [x]), target='hip')
+    arrays = [rng.standard_normal((20, 64)).astype(np.float32)]
+    behind, again = [], []
+    for _ in range(210):
+        runner.run(arrays)
+        t = [time.perf_counter()]
+        for _ in range(2):
+            torch.cuda.synchronize()
+            t.append(time.perf_counter())
+        behind.append(t[1] - t[0])
+        again.append(t[2] - t[1])
+    first, second = sorted(behind[10:])[100], sorted(again[10:])[100]
+    print('%d layers: %.1f us behind a call, %.1f again' % (layers, first * 1e6, second * 1e6), flush=True)
+    assert first < 2 * second + 2e-6
