@@ -102,7 +102,7 @@ int pml_hip_event_elapsed_ms(pml_hip_event start, pml_hip_event stop, float* ms)
  * pml_hip_stream_create, never NULL) is recorded instead of run; every *_invoke of this library may be recorded once
  * it has run at least once on the same plan (first runs may allocate).  _end returns the replayable graph, or fails
  * (and leaves `s` usable) if something could not be recorded.  Pointers are baked in: replay with the same buffers.
- * A recording of up to 64 kernels is replayed by launching them one by one with the recorded arguments, a longer one as
+ * A recording of up to five kernels is replayed by launching them one by one with the recorded arguments, a longer one as
  * one HIP graph (plaidml_amd/csrc/replay.hip). */
 typedef void* pml_hip_graph;
 int pml_hip_capture_begin(pml_hip_stream s);

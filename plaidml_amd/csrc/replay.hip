@@ -1,12 +1,14 @@
 // Replay of a recorded sequence of launches.
 //
 // hipGraphLaunch takes 16 to 18 us of the host whatever the graph holds, before the device sees the first kernel; a launch of its
-// own takes 2.1, which the kernels ahead of it cover.  So a recording is replayed launch by launch, with the arguments it holds (no
-// plan is asked again), and only a long one as a graph.  us a run, host to host, as a graph -> one by one, one box:
-//   dense layers of 4 x 64 (3.3 us each on the device)   7 of them 48.9 -> 38.4, 14 66.7 -> 59.0, 80 264 -> 257 (another box 270 -> 276)
-//   ResNet-50 on one image, 52 kernels                   389 -> 375
-// (The first 4 or 8 one by one and the rest as a graph: as a graph.  Both sides with the results' mark in host memory; waiting for
-// the stream takes 13 us more from eight queued commands on.)
+// own takes 2.1, which the kernels ahead of it cover.  So a short recording is replayed launch by launch, with the arguments it
+// holds (no plan is asked again), and a longer one as a graph: from eight commands on -- a run's launches, its copies up and down by
+// kernel and hipStreamSynchronize's own -- retiring them takes the run that waits 13 us more, and a graph is one.  us a call, n dense
+// layers of 8 x 64 on arrays in host memory, as a graph -> one by one (medians, roots in turn on one box):
+//   n                                    2             3             4             5             6             7             8            10            30           52
+//   one behind the other        40.2 -> 30.1  52.4 -> 34.0  47.1 -> 38.2  47.8 -> 41.4  51.0 -> 59.6  59.3 -> 64.3  61.2 -> 66.1  63.6 -> 73.6   130 -> 144    202 -> 227
+//   and a wait for the device   45.1 -> 33.3  56.2 -> 37.1  50.8 -> 41.2  51.0 -> 44.4  54.0 -> 61.8  61.3 -> 67.4  64.2 -> 69.1  67.2 -> 76.9   133 -> 147    205 -> 230
+//   new arrays, 10 ms later     72.3 -> 48.7  85.2 -> 52.0  73.4 -> 47.8  77.5 -> 61.9  73.2 -> 80.5  79.9 -> 89.4  76.7 -> 96.8  78.3 -> 94.5   147 -> 156    219 -> 237
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -19,12 +21,12 @@ namespace pml {
 
 namespace {
 
-constexpr size_t kFewLaunches = 64;  // one by one up to here
+constexpr size_t kFewLaunches = 5;  // one by one up to here
 
-// The kernels of a recording that is one chain of nothing else, in their order (the arguments stay the recording's own).
+// The kernels of a short recording that is one chain of nothing else, in their order (the arguments stay the recording's own).
 bool kernel_chain(hipGraph_t g, std::vector<hipKernelNodeParams>* chain) {
   size_t n = 0, edges = 0;
-  if (hipGraphGetNodes(g, nullptr, &n) != hipSuccess || n == 0) return false;
+  if (hipGraphGetNodes(g, nullptr, &n) != hipSuccess || n == 0 || n > kFewLaunches) return false;
   if (hipGraphGetEdges(g, nullptr, nullptr, &edges) != hipSuccess || edges != n - 1) return false;
   std::vector<hipGraphNode_t> nodes(n), from(edges), to(edges);
   if (hipGraphGetNodes(g, nodes.data(), &n) != hipSuccess) return false;
@@ -52,7 +54,7 @@ bool kernel_chain(hipGraph_t g, std::vector<hipKernelNodeParams>* chain) {
 }  // namespace
 
 struct Replay {
-  hipGraph_t recorded = nullptr;
+  hipGraph_t recorded = nullptr;              // of launches that go out one by one
   std::vector<hipKernelNodeParams> launches;  // one by one (their arguments are `recorded`'s); empty: as a graph
   hipGraphExec_t exec = nullptr;
   ~Replay() {
@@ -68,9 +70,11 @@ hipError_t replay_create(hipGraph_t recorded, Replay** out) {
     (void)hipGetLastError();
     r->launches.clear();
   }
-  if (r->launches.size() > kFewLaunches) r->launches.clear();
-  if (r->launches.empty())
+  if (r->launches.empty()) {
     if (hipError_t e = hipGraphInstantiate(&r->exec, recorded, nullptr, nullptr, 0); e != hipSuccess) return e;
+    (void)hipGraphDestroy(recorded);
+    r->recorded = nullptr;
+  }
   *out = r.release();
   return hipSuccess;
 }

@@ -901,7 +901,7 @@ void plaidml_hip_last_run_memory(size_t* arena_bytes, size_t* unshared_temp_byte
   if (device_bytes) *device_bytes = s.device_bytes;
 }
 
-// 1 when that run replayed its launches as one recorded HIP graph, 0 when it launched them one by one.
+// 1 when that run replayed recorded launches, 0 when it asked every plan for its own.
 int plaidml_hip_last_run_replayed(void) { return rt::lastInvokeStats().replayed ? 1 : 0; }
 // Why not, when recording was tried and failed ("" otherwise); valid until the calling thread's next run.
 const char* plaidml_hip_last_run_graph_note(void) {

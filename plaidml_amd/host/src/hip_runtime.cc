@@ -431,7 +431,7 @@ class HipExecutable final : public Executable {
       for (auto& e : step_events_) hipCheck(pml_hip_event_create(&e), "event");
     }
     // The launches of a run never change (same plans, same device buffers), so from the third run on they are
-    // replayed as one graph recorded during that run; the first two run one by one (first runs of a kernel plan may
+    // replayed from a recording made during that run; the first two run one by one (first runs of a kernel plan may
     // allocate, which cannot be recorded).  A recording that fails leaves the executable with one-by-one launches.
     if (graphable_ && !profile && !graph_ && runs_ >= 2) graph_ = record(launches);
     ++runs_;
@@ -497,7 +497,7 @@ class HipExecutable final : public Executable {
     std::fflush(stdout);
   }
 
-  // The launches as one graph, or nullptr (and one-by-one launches from then on).
+  // The launches as a recording, or nullptr (and one-by-one launches from then on).
   pml_hip_graph record(const std::vector<Launch>& launches) {
     if (pml_hip_capture_begin(stream_) != 0) {
       graph_note_ = pml_hip_last_error();

@@ -84,7 +84,7 @@ struct InvokeStats {
   size_t unshared_temp_bytes = 0;  // what the temporaries would take with memory of their own
   size_t device_bytes = 0;         // arena + inputs + outputs + constants + what the kernel plans hold
   std::vector<double> step_ms;     // per step of the plan, over its parts; only with PLAIDML_PROFILE=1
-  bool replayed = false;           // the launches ran as one recorded graph
+  bool replayed = false;           // the launches came from a recording
   std::string graph_note;          // why they did not, when recording was tried and failed
 };
 InvokeStats lastInvokeStats();
