@@ -330,7 +330,7 @@ bool fp32_beats_split(int64_t m, int64_t n, int64_t k_bytes, int64_t kn_ldb) {
 // that; and for small problems the smaller of 64x64 and 128x64 by (rounds of resident workgroups) x
 // (tile area), the larger tile on a tie.
 // forced: a tile named by the descriptor's schedule bits (PML_HIP_FLAG_TILE), -1 = none
-// bare_tail: start values, ReLU and requantisation at most
+// bare_tail: one product, and start values, ReLU and requantisation at most
 int choose_tile(int64_t m, int64_t n, int64_t k_bytes, int kind = KIND_BF16, bool plain_tail = true, int forced = -1, bool allow_split = true, bool bare_tail = false) {
   if (forced >= 0 && forced < PML_HIP_TILE_COUNT_ && (forced != TILE_128x64_N2 || kind == KIND_F32X3) &&
       (forced != TILE_192x384_W8 || kind == KIND_BF16 || kind == KIND_I8))
@@ -378,7 +378,8 @@ int choose_tile(int64_t m, int64_t n, int64_t k_bytes, int kind = KIND_BF16, boo
   // (fp32 1024^3: 32.5 -> 28.8 us; bf16 128x1000x2048: 13.4 -> 11.6 us; bf16 2048^3, 1024 tiles: 26.7 -> 40.5 us)
   // (one tile a CU: whatever the K, eight wavefronts to its loads and its tail; bf16 650 x 593, K = 720 8.7 -> 7.5 us, 915 x 588,
   // K = 224 5.9 -> 5.1, int8 2085 x 435, K = 48 5.6 -> 5.1.  Not under a residual or scale and shift, whose operands it waits for with
-  // half the tiles' wavefronts on a CU: 648 x 632, K = 632 with scale, shift, ReLU in its block 16.4 us, 17.1; ResNet-50 on one image 375, 384)
+  // half the tiles' wavefronts on a CU: 648 x 632, K = 632 with scale, shift, ReLU in its block 16.4 us, 17.1; ResNet-50 on one image 375, 384.
+  // Nor where a second product follows, with start values of its own: 40 of them 0.96 x, 784 x 512, K = 128 + 256 in ResNet-50 1.4 us a call)
   if (tiles(64, 64) <= (k_bytes >= 2048 ? 512 : bare_tail ? 256 : 0)) return TILE_64x64_W8_K2;
   const int64_t rounds_small = (tiles(64, 64) + 5 * 256 - 1) / (5 * 256);
   const int64_t rounds_wide = (tiles(128, 64) + 2 * 256 - 1) / (2 * 256);
@@ -1176,7 +1177,7 @@ int64_t pml_hip_gemm_dispatch(const pml_hip_gemm_desc* d) {
     int mode = 0, relu = 0;
     classify_tail(d->tail, d->out_dtype, d->c_dtype, &mode, &relu);
     const bool plain = mode == 1 || mode == 2 || tail_requant(d->tail, d->out_dtype, d->c_dtype, mode, nullptr);
-    p->tile = choose_tile(d->m, d->n, (d->k + d->k2) * dt_size(d->in_dtype), kind, plain, PML_HIP_FLAG_TILE_OF(d->flags), true, plain && mode != 2);
+    p->tile = choose_tile(d->m, d->n, (d->k + d->k2) * dt_size(d->in_dtype), kind, plain, PML_HIP_FLAG_TILE_OF(d->flags), true, plain && mode != 2 && d->k2 == 0);
     // (a second product's slabs follow the first one's on the slab axis the splits share out.)  With a direct tile over rows
     // that are at hand the LDS tile is only left for a [K][N] right-hand side that arrives with the call and cannot be read
     // as it lies; pml_hip_gemm_pack_b ends that.

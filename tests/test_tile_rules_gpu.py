@@ -1,0 +1,64 @@
+"""Which 64 x 64 tiles share K in two wavefront grids: by the tail and by what else a tile waits for."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from plaidml_amd import edsl as E
+from plaidml_amd import hipkernels as hk
+
+pytestmark = pytest.mark.gpu
+SHARED, PLAIN = 'tile=64x64 (8 wavefronts, K split in two) ', 'tile=64x64 '
+
+
+def run(kind, m, n, k, tail='relu', k2=0, tile=None):
+    """C and the plan's text; operands from the sizes alone."""
+    L, rng, f32 = hk.lib(), np.random.default_rng(m + n + k), kind == 'f32'
+    dt, cast = (hk.F32, lambda a: a) if f32 else (hk.BF16, E.to_bf16_bits)
+    draw = lambda *s: E.round_bf16(rng.standard_normal(s).astype(np.float32))  # noqa: E731
+    A, B, A2, B2, b, b2, R, S = draw(m, k), draw(k, n), draw(m, max(k2, 1)), draw(max(k2, 1), n), draw(n), draw(n), draw(m, n), draw(n)
+    d = hk.GemmDesc()
+    d.in_dtype = d.out_dtype = d.c_dtype = dt
+    d.m, d.n, d.k, d.lda, d.ldb, d.ldc = m, n, k, k, n, n
+    d.init_kind, d.init_dtype, d.init_row_stride, d.init_col_stride = 1, dt, 0, 1
+    relu, operands, values = (hk.EPI_RELU, dt, 0, 0, 0.0), [], []
+    want = A.astype(np.float64) @ B + b
+    if tail == 'relu':
+        ops = [relu]
+    elif tail == 'residual':
+        ops, operands, values, want = [(hk.EPI_ADD, dt, hk.OPND_TENSOR, 0, 0.0), relu], [(dt, n, 1)], [R], want + R
+    else:
+        ops, operands, values = [(hk.EPI_MUL, dt, hk.OPND_TENSOR, 0, 0.0), (hk.EPI_ADD, dt, hk.OPND_TENSOR, 1, 0.0), relu], [(dt, 0, 1), (dt, 0, 1)], [S, b2]
+        want = want * S + b2
+    d.tail = hk.make_tail(ops=ops, operands=operands)
+    if k2:
+        d.k2, d.lda2, d.ldb2, d.init2_kind = k2, k2, n, 1
+        want = want + A2.astype(np.float64) @ B2 + b2
+    d.flags = hk.flag_tile(tile) if tile else 0
+    plan = L.pml_hip_gemm_dispatch(ctypes.byref(d))
+    assert plan, L.pml_hip_last_error()
+    text = hk.describe(plan)
+    dev = [hk.DeviceBuffer.from_numpy(cast(x)) for x in (A, B, b, A2, B2, b2)]
+    held = [hk.DeviceBuffer.from_numpy(cast(x)) for x in values]
+    out, none, at = hk.DeviceBuffer(m * n * (4 if f32 else 2)), hk.ptr_array([]), hk.ptr_array([x.ptr for x in held])
+    if k2:
+        hk.check(L.pml_hip_gemm_pack_b2(plan, dev[4].ptr, None))
+        hk.check(L.pml_hip_gemm_invoke2(plan, dev[0].ptr, dev[1].ptr, out.ptr, dev[2].ptr, dev[3].ptr, None, dev[5].ptr, at, none, None))
+    else:
+        hk.check(L.pml_hip_gemm_invoke(plan, dev[0].ptr, dev[1].ptr, out.ptr, dev[2].ptr, at, none, None))
+    got = out.to_numpy(np.float32 if f32 else np.uint16, (m, n))
+    L.pml_hip_plan_free(plan)
+    return got, np.maximum(want, 0), text
+
+
+# a network's layer at batch 1, few columns, one tile, a K that two grids share whatever the tail
+@pytest.mark.parametrize('m,n,k,k2,shared', [(784, 512, 128, 256, False), (2831, 72, 32, 96, False), (3400, 64, 64, 32, False), (1281, 520, 128, 128, False),
+                                             (2000, 520, 512, 512, True)])
+def test_two_products(m, n, k, k2, shared):
+    """A second product and its start values are waited for: short K's of two products are not shared."""
+    got, want, text = run('bf16', m, n, k, k2=k2)
+    assert (SHARED if shared else PLAIN) in text and ('K split in two' in text) == shared, text
+    named, _, _ = run('bf16', m, n, k, k2=k2, tile='64x64w8k2' if shared else '64x64')
+    np.testing.assert_array_equal(got, named)
+    # (one rounding to bf16, of sums whose own roundings are far below)
+    assert (np.abs(E.from_bf16_bits(got) - want) <= 2.0 ** -8 * np.abs(want) + 1e-3).all()
