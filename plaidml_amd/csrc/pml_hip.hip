@@ -303,6 +303,14 @@ bool fp32_beats_split(int64_t m, int64_t n, int64_t k_bytes, int64_t kn_ldb) {
   return !kn_ldb || std::min(direct_lies_us(m, n, k_bytes, KIND_F32, 16), direct_lies_us(m, n, k_bytes, KIND_F32, 32)) <= 0.95 * (split_us + copy);
 }
 
+// What of a tail decides between tiles.
+struct TailForm {
+  bool plain;             // leaves a 256 x 256 tile in one go
+  bool bare = false;      // one product, and start values, ReLU and requantisation at most
+  bool residual = false;  // + a whole tensor, ReLU
+  bool two = false;       // a second product, with start values of its own
+};
+
 // Stated tiling choice per shape class.  Measured on MI355X, bf16 unless said otherwise (us; w8 / w16 =
 // 8 / 16 wavefronts per workgroup; s2 = two ring stages and LDS cut to what the result tile needs, so that two
 // workgroups share a CU; the 4-wavefront 256x128 and 256x256 tiles that were tried as well are slower than
@@ -330,8 +338,7 @@ bool fp32_beats_split(int64_t m, int64_t n, int64_t k_bytes, int64_t kn_ldb) {
 // that; and for small problems the smaller of 64x64 and 128x64 by (rounds of resident workgroups) x
 // (tile area), the larger tile on a tie.
 // forced: a tile named by the descriptor's schedule bits (PML_HIP_FLAG_TILE), -1 = none
-// bare_tail: one product, and start values, ReLU and requantisation at most
-int choose_tile(int64_t m, int64_t n, int64_t k_bytes, int kind = KIND_BF16, bool plain_tail = true, int forced = -1, bool allow_split = true, bool bare_tail = false) {
+int choose_tile(int64_t m, int64_t n, int64_t k_bytes, int kind, const TailForm& tail, int forced = -1, bool allow_split = true) {
   if (forced >= 0 && forced < PML_HIP_TILE_COUNT_ && (forced != TILE_128x64_N2 || kind == KIND_F32X3) &&
       (forced != TILE_192x384_W8 || kind == KIND_BF16 || kind == KIND_I8))
     return forced;
@@ -348,13 +355,13 @@ int choose_tile(int64_t m, int64_t n, int64_t k_bytes, int kind = KIND_BF16, boo
     if (tiles(64, 64) <= 512 && k_bytes >= 2048) return TILE_64x64_W8_K2;
     return TILE_64x64;
   }
-  if (n <= 64) return kind != KIND_F32 && bare_tail && tiles(64, 64) <= 256 ? TILE_64x64_W8_K2 : TILE_64x64;  // (the 7x7 stem of ResNet-50 over 2x2 pixel blocks: 191 us against 207 us with 128x64w8)
+  if (n <= 64) return kind != KIND_F32 && tail.bare && tiles(64, 64) <= 256 ? TILE_64x64_W8_K2 : TILE_64x64;  // (the 7x7 stem of ResNet-50 over 2x2 pixel blocks: 191 us against 207 us with 128x64w8)
   // Long K, at least three quarters of a round of 256x256 tiles and little of them hanging over the edges:
   // eight wavefronts of 128x64 (0.75 KB of LDS fragment reads per MFMA instead of 1.5).  Measured with N(0,1) /
   // uniform int8 data, 4096^3: bf16 121 us against 139 (256x128, 16 wavefronts), int8 73 against 84.
   // (Not under a tail that runs in steps -- requantisation chains: a wavefront stages its 128x64 part through a
   // 16 KB share of LDS in four rounds, 4096^3 int8 with that tail 132 us against 106 with 256x128.)
-  if (kind != KIND_F32 && plain_tail && k_bytes >= 2048 && tiles(256, 256) >= 192 && tiles(256, 256) * 65536 * 10 <= m * n * 11)
+  if (kind != KIND_F32 && tail.plain && k_bytes >= 2048 && tiles(256, 256) >= 192 && tiles(256, 256) * 65536 * 10 <= m * n * 11)
     return TILE_256x256_W8;
   // Eight wavefronts of 96 x 96 on a 192 x 384 tile: per MFMA half the global -> LDS bytes of a 128 x 128 tile (the vector
   // memory path moves 64 bytes per clock and CU, which 128 x 128 tiles use up entirely) and 0.67 KB of fragment reads.
@@ -372,15 +379,19 @@ int choose_tile(int64_t m, int64_t n, int64_t k_bytes, int kind = KIND_BF16, boo
   if (kind == KIND_BF16 && k_bytes >= 2048 && tiles(256, 128) >= 192 && tiles(256, 128) <= 256) return TILE_256x128_W16;
   if (kind == KIND_F32 && !f32_tiles_of_128(m, n)) return tiles(64, 64) <= 512 ? TILE_64x64_W8_K2 : TILE_64x64;
   if (tiles(128, 128) >= 256) return TILE_128x128_W8_S2;
-  // (two slabs and less are all launch, first loads and tail: bf16 conv 8750 x 138, K = 64 9.4 -> 6.6 us, 23958 x 105, K = 128 9.6 -> 8.1)
-  if (tiles(128, 128) >= 128 && (kind == KIND_F32 || k_bytes > 256)) return TILE_128x128_W8;
+  // (two slabs and less are all launch, first loads and tail: bf16 conv 8750 x 138, K = 64 9.4 -> 6.6 us, 23958 x 105, K = 128 9.6 -> 8.1.
+  // But bf16 tiles of 64 that are more than three a CU take another round for that: of 60 products and convolutions with whole 16-byte
+  // rows those of up to 768 took 1.06 x as long in tiles of 128 (relu 0.96 to 1.13, scale and shift 1.01 to 1.17), those of more 0.94 x
+  // (0.91 to 0.98, 0.93 to 0.99; residuals 1.02), two products 0.99 x and 0.91; int8 and rows off 16 bytes 1.0 to 1.5 x.)
+  const bool short_k = k_bytes <= 256 && !tail.two && (kind == KIND_I8 || n % 8 != 0 || tail.residual || tiles(64, 64) <= 3 * 256);
+  if (tiles(128, 128) >= 128 && (kind == KIND_F32 || !short_k)) return TILE_128x128_W8;
   // at most two 64x64 tiles per CU and a long K: a second wavefront grid takes half of every slab
   // (fp32 1024^3: 32.5 -> 28.8 us; bf16 128x1000x2048: 13.4 -> 11.6 us; bf16 2048^3, 1024 tiles: 26.7 -> 40.5 us)
   // (one tile a CU: whatever the K, eight wavefronts to its loads and its tail; bf16 650 x 593, K = 720 8.7 -> 7.5 us, 915 x 588,
   // K = 224 5.9 -> 5.1, int8 2085 x 435, K = 48 5.6 -> 5.1.  Not under a residual or scale and shift, whose operands it waits for with
   // half the tiles' wavefronts on a CU: 648 x 632, K = 632 with scale, shift, ReLU in its block 16.4 us, 17.1; ResNet-50 on one image 375, 384.
   // Nor where a second product follows, with start values of its own: 40 of them 0.96 x, 784 x 512, K = 128 + 256 in ResNet-50 1.4 us a call)
-  if (tiles(64, 64) <= (k_bytes >= 2048 ? 512 : bare_tail ? 256 : 0)) return TILE_64x64_W8_K2;
+  if (tiles(64, 64) <= (k_bytes >= 2048 ? 512 : tail.bare ? 256 : 0)) return TILE_64x64_W8_K2;
   const int64_t rounds_small = (tiles(64, 64) + 5 * 256 - 1) / (5 * 256);
   const int64_t rounds_wide = (tiles(128, 64) + 2 * 256 - 1) / (2 * 256);
   return rounds_small < 2 * rounds_wide ? TILE_64x64 : TILE_128x64;
@@ -509,6 +520,14 @@ bool tail_requant(const pml_hip_epilogue& t, int out_dtype, int c_dtype, int mod
     g->rq_hi = (float)o[3].imm;
   }
   return true;
+}
+
+// ... and what of a tail decides between tiles.  (A convolution's never counts as leaving a 256 x 256 tile in one go.)
+TailForm tail_form(const pml_hip_epilogue& t, int out_dtype, int c_dtype, bool conv, bool two) {
+  int mode = 0, relu = 0;
+  classify_tail(t, out_dtype, c_dtype, &mode, &relu);
+  const bool requant = tail_requant(t, out_dtype, c_dtype, mode, nullptr);
+  return {!conv && (mode == 1 || mode == 2 || requant), (mode == 1 || (requant && !conv)) && !two, mode == 2, two};
 }
 
 // allow64: the standalone elementwise kernel also runs 64-bit steps; the tails of the contraction kernels do not
@@ -1033,7 +1052,7 @@ int pml_hip_gemm_tail_cheaper_apart(const pml_hip_gemm_desc* d) {
   if (mode == 1 || mode == 2 || tail_requant(d->tail, d->out_dtype, d->c_dtype, mode, nullptr)) return 0;
   const int64_t k_bytes = d->k * dt_size(d->in_dtype);
   if (PML_HIP_FLAG_TILE_OF(d->flags) >= 0) return 0;  // a named tile is taken whatever the tail
-  return choose_tile(d->m, d->n, k_bytes, kind, true) == TILE_256x256_W8 && choose_tile(d->m, d->n, k_bytes, kind, false) != TILE_256x256_W8;
+  return choose_tile(d->m, d->n, k_bytes, kind, {true}) == TILE_256x256_W8 && choose_tile(d->m, d->n, k_bytes, kind, {false}) != TILE_256x256_W8;
 }
 
 // Whether a product's 256 x 256 tile reads B[K][N] with rows of `ldb` elements as it lies: four neighbouring columns per lane
@@ -1174,10 +1193,7 @@ int64_t pml_hip_gemm_dispatch(const pml_hip_gemm_desc* d) {
   p->mfma_kind = kind;
   p->gemm = *d;
   {
-    int mode = 0, relu = 0;
-    classify_tail(d->tail, d->out_dtype, d->c_dtype, &mode, &relu);
-    const bool plain = mode == 1 || mode == 2 || tail_requant(d->tail, d->out_dtype, d->c_dtype, mode, nullptr);
-    p->tile = choose_tile(d->m, d->n, (d->k + d->k2) * dt_size(d->in_dtype), kind, plain, PML_HIP_FLAG_TILE_OF(d->flags), true, plain && mode != 2 && d->k2 == 0);
+    p->tile = choose_tile(d->m, d->n, (d->k + d->k2) * dt_size(d->in_dtype), kind, tail_form(d->tail, d->out_dtype, d->c_dtype, false, d->k2 > 0), PML_HIP_FLAG_TILE_OF(d->flags));
     // (a second product's slabs follow the first one's on the slab axis the splits share out.)  With a direct tile over rows
     // that are at hand the LDS tile is only left for a [K][N] right-hand side that arrives with the call and cannot be read
     // as it lies; pml_hip_gemm_pack_b ends that.
@@ -1455,11 +1471,8 @@ int pml_hip_gemm_run_static(const pml_hip_gemm_desc* d, const void* a, const voi
     bt = scratch_of_current_device();
     if (!bt) return 1;
   }
-  int mode = 0, relu = 0;
-  classify_tail(d->tail, d->out_dtype, d->c_dtype, &mode, &relu);
-  const bool plain = mode == 1 || mode == 2 || tail_requant(d->tail, d->out_dtype, d->c_dtype, mode, nullptr);
   // (no workspace may be allocated here: the K loop is never split over workgroups)
-  const int tile = choose_tile(d->m, d->n, d->k * dt_size(d->in_dtype), kind, plain, PML_HIP_FLAG_TILE_OF(d->flags), /*allow_split=*/false, plain && mode != 2);
+  const int tile = choose_tile(d->m, d->n, d->k * dt_size(d->in_dtype), kind, tail_form(d->tail, d->out_dtype, d->c_dtype, false, false), PML_HIP_FLAG_TILE_OF(d->flags), /*allow_split=*/false);
   const DirectTiles direct = direct_tiles(*d, kind, tile);
   PanelRoom panel;
   if (bt && (panel.config = panel_of(*d, kind, tile, direct, nullptr)) >= 0 && packs_given(*d, kind, tile) && panel_bytes(*d, kind) <= PML_HIP_STATIC_SCRATCH_BYTES)
@@ -1533,9 +1546,8 @@ int64_t pml_hip_conv2d_dispatch(const pml_hip_conv2d_desc* d) {
   p->conv = *d;
   const int64_t M = d->n * d->oh * d->ow;
   const int64_t K = d->kh * d->kw * d->ci;
-  int mode = 0, relu = 0;
-  classify_tail(d->tail, d->out_dtype, d->c_dtype, &mode, &relu);
-  p->tile = choose_tile(M, d->co, K * es, kind, false, PML_HIP_FLAG_TILE_OF(d->flags), true, mode == 1);
+  const TailForm tail = tail_form(d->tail, d->out_dtype, d->c_dtype, true, false);
+  p->tile = choose_tile(M, d->co, K * es, kind, tail, PML_HIP_FLAG_TILE_OF(d->flags));
   p->bt_ld = K;
   if (via_s2d) {
     const int v = 16 / es;
@@ -1545,7 +1557,7 @@ int64_t pml_hip_conv2d_dispatch(const pml_hip_conv2d_desc* d) {
     p->s2d_ka = (int)(d->kh + (d->pad_h & 1) + 1) / 2;
     p->s2d_kaw = (int)(d->kw + (d->pad_w & 1) + 1) / 2;
     const int64_t k2 = (int64_t)p->s2d_ka * p->s2d_kaw * p->s2d_ch;
-    p->tile = choose_tile(M, d->co, k2 * es, kind, false, PML_HIP_FLAG_TILE_OF(d->flags), /*allow_split=*/false, mode == 1);
+    p->tile = choose_tile(M, d->co, k2 * es, kind, tail, PML_HIP_FLAG_TILE_OF(d->flags), /*allow_split=*/false);
     p->bt_ld = k2;
     p->via_s2d = true;
   }
