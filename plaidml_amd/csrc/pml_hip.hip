@@ -309,6 +309,7 @@ struct TailForm {
   bool bare = false;      // one product, and start values, ReLU and requantisation at most
   bool residual = false;  // + a whole tensor, ReLU
   bool two = false;       // a second product, with start values of its own
+  bool steps = false;     // steps on column vectors and single values: scale and shift
 };
 
 // Stated tiling choice per shape class.  Measured on MI355X, bf16 unless said otherwise (us; w8 / w16 =
@@ -377,7 +378,12 @@ int choose_tile(int64_t m, int64_t n, int64_t k_bytes, int kind, const TailForm&
   // batch 128: the 3x3 convolutions 38.9 -> 37.3 us, the 1x1 layers with K = 1024 26.7 -> 25.3, the network 2.59 -> 2.57 ms
   // (measured with a schedule file before the rule was written down).
   if (kind == KIND_BF16 && k_bytes >= 2048 && tiles(256, 128) >= 192 && tiles(256, 128) <= 256) return TILE_256x128_W16;
-  if (kind == KIND_F32 && !f32_tiles_of_128(m, n)) return tiles(64, 64) <= 512 ? TILE_64x64_W8_K2 : TILE_64x64;
+  // fp32: up to two 64 x 64 tiles a CU share K in two wavefront grids (1024^3 32.5 -> 28.8 us), whatever the K: of 118 products and
+  // convolutions with K of less than 2 KB those of up to 256 tiles took 1.05 to 1.16 x as long in plain ones (relu 1.08, residual 1.11,
+  // scale and shift 1.05), those of up to 512 1.00 to 1.07 -- but for scale and shift, 0.96 to 1.03, unless rows off 16 bytes leave
+  // step by step (1.3).
+  if (kind == KIND_F32 && !f32_tiles_of_128(m, n))
+    return tiles(64, 64) <= (k_bytes < 2048 && tail.steps && n % 4 == 0 ? 256 : 512) ? TILE_64x64_W8_K2 : TILE_64x64;
   if (tiles(128, 128) >= 256) return TILE_128x128_W8_S2;
   // (two slabs and less are all launch, first loads and tail: bf16 conv 8750 x 138, K = 64 9.4 -> 6.6 us, 23958 x 105, K = 128 9.6 -> 8.1.
   // But bf16 tiles of 64 that are more than three a CU take another round for that: of 60 products and convolutions with whole 16-byte
@@ -386,10 +392,10 @@ int choose_tile(int64_t m, int64_t n, int64_t k_bytes, int kind, const TailForm&
   const bool short_k = k_bytes <= 256 && !tail.two && (kind == KIND_I8 || n % 8 != 0 || tail.residual || tiles(64, 64) <= 3 * 256);
   if (tiles(128, 128) >= 128 && (kind == KIND_F32 || !short_k)) return TILE_128x128_W8;
   // at most two 64x64 tiles per CU and a long K: a second wavefront grid takes half of every slab
-  // (fp32 1024^3: 32.5 -> 28.8 us; bf16 128x1000x2048: 13.4 -> 11.6 us; bf16 2048^3, 1024 tiles: 26.7 -> 40.5 us)
+  // (bf16 128x1000x2048: 13.4 -> 11.6 us; bf16 2048^3, 1024 tiles: 26.7 -> 40.5 us)
   // (one tile a CU: whatever the K, eight wavefronts to its loads and its tail; bf16 650 x 593, K = 720 8.7 -> 7.5 us, 915 x 588,
   // K = 224 5.9 -> 5.1, int8 2085 x 435, K = 48 5.6 -> 5.1.  Not under a residual or scale and shift, whose operands it waits for with
-  // half the tiles' wavefronts on a CU: 648 x 632, K = 632 with scale, shift, ReLU in its block 16.4 us, 17.1; ResNet-50 on one image 375, 384.
+  // half the tiles' wavefronts on a CU: 648 x 632, K = 632 with scale, shift, ReLU in its block 16.4 us, 17.1; ResNet-50 on one image, three such layers 394.0, 395.2.
   // Nor where a second product follows, with start values of its own: 40 of them 0.96 x, 784 x 512, K = 128 + 256 in ResNet-50 1.4 us a call)
   if (tiles(64, 64) <= (k_bytes >= 2048 ? 512 : tail.bare ? 256 : 0)) return TILE_64x64_W8_K2;
   const int64_t rounds_small = (tiles(64, 64) + 5 * 256 - 1) / (5 * 256);
@@ -527,7 +533,7 @@ TailForm tail_form(const pml_hip_epilogue& t, int out_dtype, int c_dtype, bool c
   int mode = 0, relu = 0;
   classify_tail(t, out_dtype, c_dtype, &mode, &relu);
   const bool requant = tail_requant(t, out_dtype, c_dtype, mode, nullptr);
-  return {!conv && (mode == 1 || mode == 2 || requant), (mode == 1 || (requant && !conv)) && !two, mode == 2, two};
+  return {!conv && (mode == 1 || mode == 2 || requant), (mode == 1 || (requant && !conv)) && !two, mode == 2, two, mode == 3};
 }
 
 // allow64: the standalone elementwise kernel also runs 64-bit steps; the tails of the contraction kernels do not

@@ -80,3 +80,14 @@ def test_two_slabs_and_less(m, n, k, tail, k2, large):
     named = run('bf16', m, n, k, tail, k2, tile='128x128w8' if large else '64x64')[0]
     for c in (got, named):
         assert (np.abs(c - want) <= bound).all()
+
+
+# fp32, K of less than 2 KB: 264 tiles and 256 of them, rows off 16 bytes; a longer K
+@pytest.mark.parametrize('m,n,k,tail,shared', [(1381, 768, 120, 'scale', False), (1381, 768, 120, 'residual', True), (1381, 768, 120, 'relu', True), (1024, 1024, 120, 'scale', True),
+                                               (1381, 766, 120, 'scale', True), (1381, 768, 512, 'scale', True)])
+def test_fp32_under_scale_and_shift(m, n, k, tail, shared):
+    got, want, bound, text = run('f32', m, n, k, tail)
+    assert (SHARED if shared else PLAIN) in text and ('K split in two' in text) == shared, text
+    named = run('f32', m, n, k, tail, tile='64x64w8k2' if shared else '64x64')[0]
+    np.testing.assert_array_equal(got, named)
+    assert (np.abs(got - want) <= bound).all()
