@@ -281,13 +281,14 @@ double direct_lies_us(int64_t m, int64_t n, int64_t k_bytes, int kind, int side)
 
 // Whether a product that may be taken as three bf16 products is better off in a direct tile of plain fp32 MFMAs: the split kind
 // has no direct tiles, and with few results it is latency that bounds both.  Its tiles take 4.2 us and 0.42 per slab, or split as
-// `direct_tile_of` says.  kn_ldb: pitch in bytes of a right-hand side [K][N] (0: rows of K).  us, split -> direct: 1 x 1724, K = 656 packed 9.4 -> 4.9,
+// `direct_tile_of` says.  Decided by the sizes alone, so that a product has the same bits from [K][N] as it lies, packed and from
+// [N][K]: the direct tiles have to be cheaper over rows of K and over [K][N].  us, split -> direct: 1 x 1724, K = 656 packed 9.4 -> 4.9,
 // 7 x 1293, K = 208 [N][K] 6.9 -> 5.3, 16 x 26, K = 416 [K][N] 12.8 -> 6.1, 382 x 253, K = 336 packed 9.7 -> 6.7; but 2 x 22, K = 3104
-// 15.1 (18.7), 672 x 491, K = 800 packed 12.0 (14.2).  Of 100 drawn products 54 take it, 1.51 x in the mean.
-bool fp32_beats_split(int64_t m, int64_t n, int64_t k_bytes, int64_t kn_ldb) {
+// [K][N] 15.1 (18.7), 672 x 491, K = 800 packed 12.0 (14.2).  Of 100 drawn products 54 are cheaper over the layout that they have.
+bool fp32_beats_split(int64_t m, int64_t n, int64_t k_bytes) {
   const int64_t slabs = (k_bytes + 127) / 128;
   double us = 0, split_us = 4.2 + 0.42 * (double)slabs;
-  bool needs_bt = n % 4 != 0 || kn_ldb % 16 != 0;
+  bool needs_bt = n % 4 != 0;  // (from [K][N]: a transposed copy)
   if (splits_k(m, n, k_bytes, KIND_F32X3)) {
     int splits = 1, per = 0;
     igemm_split_plan(m, n, slabs, device_cus(), &splits, &per);
@@ -298,9 +299,8 @@ bool fp32_beats_split(int64_t m, int64_t n, int64_t k_bytes, int64_t kn_ldb) {
   }
   if (direct_tile_of(m, n, k_bytes, KIND_F32) < 0) return false;
   (void)direct_tile_of(m, n, k_bytes, KIND_F32, 0, /*always=*/true, true, false, &us);
-  if (us > 0.95 * split_us) return false;
   const double copy = needs_bt ? 3.0 + 2.0 * (double)k_bytes * (double)n / 2.2e6 : 0;
-  return !kn_ldb || std::min(direct_lies_us(m, n, k_bytes, KIND_F32, 16), direct_lies_us(m, n, k_bytes, KIND_F32, 32)) <= 0.95 * (split_us + copy);
+  return us <= 0.95 * split_us && std::min(direct_lies_us(m, n, k_bytes, KIND_F32, 16), direct_lies_us(m, n, k_bytes, KIND_F32, 32)) <= 0.95 * (split_us + copy);
 }
 
 // What of a tail decides between tiles.
@@ -1045,7 +1045,7 @@ static int gemm_desc_kind(const pml_hip_gemm_desc* d) {
     fail("gemm: a second initial value needs a second product");
     return -1;
   }
-  if (kind == KIND_F32X3 && PML_HIP_FLAG_TILE_OF(d->flags) < 0 && fp32_beats_split(d->m, d->n, d->k * es, d->b_layout ? 0 : d->ldb * es)) return KIND_F32;
+  if (kind == KIND_F32X3 && PML_HIP_FLAG_TILE_OF(d->flags) < 0 && fp32_beats_split(d->m, d->n, d->k * es)) return KIND_F32;
   return kind;
 }
 

@@ -348,7 +348,7 @@ def test_split_fp32_of_few_results_is_plain_fp32(layout, M, N, K, plain):
         d.in_dtype = d.out_dtype = d.c_dtype = hk.F32
         d.m, d.n, d.k, d.lda, d.ldb, d.ldc, d.b_layout, d.flags = M, N, K, K, K if layout else N, N, layout, flags
         plan = hk.lib().pml_hip_gemm_dispatch(ctypes.byref(d))
-        if flags and (plain or not layout):
+        if flags:
             assert ('3 x f32' in hk.describe(plan)) != plain, hk.describe(plan)
         hk.check(hk.lib().pml_hip_gemm_invoke(plan, dA.ptr, dB.ptr, dC.ptr, None, none, none, None))
         got.append(dC.to_numpy(np.float32, (M, N)))
@@ -358,6 +358,28 @@ def test_split_fp32_of_few_results_is_plain_fp32(layout, M, N, K, plain):
     want = A.astype(np.float64) @ (B.T if layout else B).astype(np.float64)
     # (2^-16 of every product, at random; the largest of all results within 8 of its standard deviation sqrt(K))
     assert np.abs(got[1] - want).max() < 8 * 2.0 ** -16 * np.sqrt(K) + 1e-5
+
+
+def test_which_kind_of_fp32_is_asked_of_sizes_alone():
+    """Products that may be split, at every size either plain fp32 or three bf16 products from [K][N] and from [N][K], whatever the
+    pitch: sizes where one layout's price is past the other's among them."""
+    rng, kinds = np.random.default_rng(5), []
+    sizes = [(2, 22, 3104), (556, 38, 1264), (36, 1896, 64)]
+    sizes += [tuple(int(v) for v in np.exp(rng.uniform(np.log(lo), np.log(hi)))) for lo, hi in [((1, 16, 16), (1500, 1500, 4000))] * 250]
+    for M, N, K in sizes:
+        K = K // 4 * 4
+        texts = []
+        for layout, ldb in ((0, N), (0, N + 1), (0, N + 8), (1, K)):
+            d = hk.GemmDesc()
+            d.in_dtype = d.out_dtype = d.c_dtype = hk.F32
+            d.m, d.n, d.k, d.lda, d.ldb, d.ldc, d.b_layout, d.flags = M, N, K, K, ldb, N, layout, hk.FP32_AS_BF16X3
+            plan = hk.lib().pml_hip_gemm_dispatch(ctypes.byref(d))
+            assert plan, hk.lib().pml_hip_last_error()
+            texts.append('3 x f32' in hk.describe(plan))
+            hk.lib().pml_hip_plan_free(plan)
+        assert len(set(texts)) == 1, (M, N, K, texts)
+        kinds.append(texts[0])
+    assert 50 < sum(kinds) < 200  # (both kinds are met)
 
 
 @pytest.mark.parametrize('M,N,K', [(251, 660, 848), (130, 2049, 80), (1250, 516, 64), (2048, 1024, 32), (2048, 2048, 32), (1030, 1990, 48), (60, 132, 1584)])

@@ -1296,7 +1296,7 @@ def _gemm_f32_layouts(A, B_kn, ldb, flags, packed_first=False):
 @pytest.mark.gpu
 @pytest.mark.parametrize('flags', [0, hk.FP32_AS_BF16X3])
 @pytest.mark.parametrize('M,N,K,ldb', [(1024, 1024, 1024, 1024), (100, 68, 72, 72), (64, 64, 36, 64), (200, 260, 132, 300),
-                                       (130, 4, 8, 4), (96, 512, 2048, 516), (77, 66, 40, 66)])
+                                       (130, 4, 8, 4), (96, 512, 2048, 516), (77, 66, 40, 66), (2, 22, 3104, 22), (556, 38, 1264, 40), (36, 1896, 64, 1896)])
 def test_gemm_f32_right_hand_side_as_given(M, N, K, ldb, flags):
     """An fp32 [K][N] right-hand side that arrives with the call is read where it lies (no transposed copy): the
     result has the same bits as the one from the same values in [N][K] layout -- the two differ only in how the
