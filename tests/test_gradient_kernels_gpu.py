@@ -62,10 +62,15 @@ def test_gradients(case, dtype):
     dev = [hk.DeviceBuffer.from_numpy(E.to_bf16_bits(a) if bf else a) for a in (x, f, g)]
     L.pml_hip_conv2d_grad_dispatch.restype = ctypes.c_int64
     for which, other, want in ((0, dev[1], want_x), (1, dev[0], want_f)):
-        if not L.pml_hip_conv2d_grad_takes(ctypes.byref(d), which):
-            continue
+        assert L.pml_hip_conv2d_grad_takes(ctypes.byref(d), which) == 1
         p = L.pml_hip_conv2d_grad_dispatch(ctypes.byref(d), which)
         assert p, L.pml_hip_last_error()
+        text = hk.describe(ctypes.c_int64(p))
+        if which == 0:
+            assert ('as a convolution of the gradient' if stride == 1 else 'by columns') in text, text
+        else:  # (pixels over one workgroup, over splits of two slabs, over more than a thread adds up)
+            splits = int(text.split('splits=')[1].split()[0])
+            assert splits >= (9 if n * oh * ow > 30000 else 2 if n * oh * ow > 1000 else 1), text
         terms = kh * kw * co if which == 0 else n * oh * ow
         out = hk.DeviceBuffer.from_numpy(np.full(want.size, np.nan, np.float32).astype(np.float32))
         for _ in range(2):
