@@ -493,6 +493,19 @@ def run_conv(I, F, in_dt, out_dt, stride=1, pad=None, autopad=op.SAME_UPPER, bia
                                             hk.ptr_array([o.ptr for o in dops]), hk.ptr_array([]), None))
     hk.check(hk.lib().pml_hip_stream_sync(None))
     out = dO.to_numpy(np_c, (N, OH, OW, CO))
+    direct = [hk.flag_tile(t) for t in ('16x16w8', '32x32w8')]
+    if not packed and ('with the filter as it lies' in hk.describe(plan) or d.flags & 0xff00 in direct):
+        # a direct tile has read the filter as it lies, and not the kernel that the plan names: that one runs over a packed filter
+        lies = out
+        hk.check(hk.lib().pml_hip_conv2d_pack_filter(plan, dF.ptr, None))
+        hk.check(hk.lib().pml_hip_conv2d_invoke(plan, dI.ptr, None, dO.ptr, dB.ptr if dB else None, hk.ptr_array([o.ptr for o in dops]), hk.ptr_array([]), None))
+        out = dO.to_numpy(np_c, (N, OH, OW, CO))
+        if out_dt == hk.BF16:
+            np.testing.assert_allclose(E.bf16_from_bits(lies), E.bf16_from_bits(out), rtol=BF16_RTOL, atol=2e-2)
+        elif in_dt == hk.BF16:
+            np.testing.assert_allclose(lies, out, rtol=FP32_RTOL, atol=1e-3)
+        else:  # integers, and fp32, whose sums are the same bits either way
+            np.testing.assert_array_equal(lies, out)
     hk.lib().pml_hip_plan_free(plan)
     return out
 
