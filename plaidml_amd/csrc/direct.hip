@@ -141,8 +141,13 @@ __device__ __forceinline__ void add_start(const i32x4_t& bits, bool bf, typename
   }
 }
 
-// MB x NB blocks of 16 x 16 results per workgroup.
-template <int KIND, bool CONV, int MB, int NB, bool KN, bool RAGGED>
+// Steps in flight: 64 registers of requests, fewer where the accumulators leave less room.
+constexpr int steps_in_flight(int kind, bool conv, int mb, int nb, bool kn, bool ragged) {
+  return kn ? (kind == KIND_F32 ? (mb == 1 ? 4 : conv ? 1 : 2) : mb == 1 && !ragged ? 3 : 2) : mb + nb > 4 ? 2 : 16 / (mb + nb);
+}
+
+// MB x NB blocks of 16 x 16 results per workgroup, U steps in flight.
+template <int KIND, bool CONV, int MB, int NB, bool KN, bool RAGGED, int U>
 __global__ __launch_bounds__(64 * kWaves, 4) void direct_kernel(IgemmArgs p_by_value) {
   warm_arguments<sizeof(IgemmArgs)>();
   // (read where the dispatcher put it: indexing a by-value copy would move the copy to scratch memory)
@@ -153,8 +158,6 @@ __global__ __launch_bounds__(64 * kWaves, 4) void direct_kernel(IgemmArgs p_by_v
   typedef accs_t acc4_t __attribute__((ext_vector_type(4)));
   constexpr int ES = KIND == KIND_BF16 ? 2 : (KIND == KIND_I8 ? 1 : 4);
   constexpr int TM = 16 * MB, TN = 16 * NB;
-  // steps in flight: 64 registers of requests, fewer where the accumulators leave less room
-  constexpr int U = KN ? (KIND == KIND_F32 ? (MB == 1 ? 4 : CONV ? 1 : 2) : MB == 1 && !RAGGED ? 3 : 2) : MB + NB > 4 ? 2 : 16 / (MB + NB);
   constexpr int RW = RAGGED ? (KIND == KIND_BF16 ? 24 : 32) : 16;  // KN: words fetched for a lane's chunk
   constexpr int CS = TN + 4;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -364,8 +367,8 @@ __global__ __launch_bounds__(64 * kWaves, 4) void direct_kernel(IgemmArgs p_by_v
           }
           turn<KIND>(words, frag);
         } else if constexpr (KIND == KIND_F32) {
-          // (word by word: from an array of fragments the compiler made scratch memory in the 16-row form; 4 x 3343, K = 2176 27.3 -> 18.7
-          // us, 13 x 3127, K = 1600 20.5 -> 15.4, 61 x 125, K = 896 9.7 -> 8.4, with four steps in flight for three)
+          // (word by word: from an array of fragments the compiler made scratch memory in the 16-row form; with four steps in flight for
+          // three 4 x 3343, K = 2176 27.3 -> 18.7 us, 13 x 3127, K = 1600 20.5 -> 15.4, 61 x 125, K = 896 9.7 -> 8.4)
           frag[0] = i32x4_t{raw[u][0], raw[u][4], raw[u][8], raw[u][12]};
           frag[1] = i32x4_t{raw[u][1], raw[u][5], raw[u][9], raw[u][13]};
           frag[2] = i32x4_t{raw[u][2], raw[u][6], raw[u][10], raw[u][14]};
@@ -433,13 +436,13 @@ __global__ __launch_bounds__(64 * kWaves, 4) void direct_kernel(IgemmArgs p_by_v
   tile_tail<KIND, TM, TN, kQuads>(p, parts, m0, n0, tid);
 }
 
-template <int KIND, bool CONV, int MB, int NB, bool KN, bool RAGGED = false>
+template <int KIND, bool CONV, int MB, int NB, bool KN, bool RAGGED = false, int U = steps_in_flight(KIND, CONV, MB, NB, KN, RAGGED)>
 hipError_t launch(const IgemmArgs& a, hipStream_t s) {
   const int64_t tiles_m = (a.M + 16 * MB - 1) / (16 * MB), tiles_n = (a.N + 16 * NB - 1) / (16 * NB);
   const int64_t tiles = tiles_m * tiles_n;
   if (tiles <= 0 || tiles >= ((int64_t)1 << 31)) return hipErrorInvalidValue;
   const size_t lds = (size_t)kWaves * 16 * MB * (16 * NB + 4) * 4;
-  auto kern = direct_kernel<KIND, CONV, MB, NB, KN, RAGGED>;
+  auto kern = direct_kernel<KIND, CONV, MB, NB, KN, RAGGED, U>;
   static DynamicLdsLimit limit;
   if (hipError_t e = limit.ensure((const void*)kern, lds); e != hipSuccess) return e;
   IgemmArgs b = a;
@@ -463,6 +466,19 @@ static hipError_t launch_large(const IgemmArgs& a, hipStream_t s) {
   return ((a.M + 31) / 32) * ((a.N + 31) / 32) > a.n_cus ? launch<PML_KIND, CONV, 2, 4, false>(a, s) : launch<PML_KIND, CONV, 2, 2, false>(a, s);
 }
 
+// fp32, 16 x 64 over [K][N]: steps in flight for wavefronts of `per` steps each.  Steps past a wavefront's last are requested and
+// multiplied, too, so few steps are taken by as many as leave the fewest of those (the same bits: sums do not turn on it).  us with 4, 3
+// and 2 in flight:  1 step, K = 128 2 x 192 5.2, 4.8, 4.45;  2, K = 192 65 x 1227 5.5, 5.15, 4.8;  3, K = 304 2 x 519 5.35, 5.1, 5.7;
+// 5, K = 576 36 x 569 7.6, 7.1, 7.0;  7, K = 864 57 x 2408 7.9, 9.2, 8.65;  8, K = 928 5 x 312 7.35, 8.8, 8.3;  9, K = 1136 11 x 807 10.0, 9.6,
+// 10.1;  10, K = 1264 12 x 285 10.0, 11.35, 10.2;  17, K = 2128 8 x 19 14.5, 15.1, 15.1.
+static int fp32_steps(int64_t per) {
+  int best = 4;
+  if (per < 10)
+    for (int u = 3; u >= 2; --u)
+      if ((per + u - 1) / u * u < (per + best - 1) / best * best) best = u;
+  return best;
+}
+
 template <bool CONV>
 static hipError_t launch_form(bool small, const IgemmArgs& a, hipStream_t s) {
   if (a.b_kn) {
@@ -470,6 +486,11 @@ static hipError_t launch_form(bool small, const IgemmArgs& a, hipStream_t s) {
     if constexpr (PML_KIND != KIND_F32)
       if (((a.N | a.ldbt) & 3) != 0 || ((uintptr_t)a.Bt & (PML_KIND == KIND_BF16 ? 7 : 3)) != 0)
         return small ? launch<PML_KIND, CONV, 1, 4, true, true>(a, s) : launch<PML_KIND, CONV, 2, 4, true, true>(a, s);
+    if constexpr (PML_KIND == KIND_F32)
+      if (small) {
+        const int steps = fp32_steps(((CONV ? (int64_t)a.KH * a.KW * ((a.CI * 4 + 63) / 64) : (a.K * 4 + 63) / 64) + kWaves - 1) / kWaves);
+        if (steps < 4) return steps == 3 ? launch<PML_KIND, CONV, 1, 4, true, false, 3>(a, s) : launch<PML_KIND, CONV, 1, 4, true, false, 2>(a, s);
+      }
     return small ? launch<PML_KIND, CONV, 1, 4, true>(a, s) : launch<PML_KIND, CONV, 2, 4, true>(a, s);
   }
   return small ? launch<PML_KIND, CONV, 1, 1, false>(a, s) : launch_large<CONV>(a, s);

@@ -360,6 +360,27 @@ def test_split_fp32_of_few_results_is_plain_fp32(layout, M, N, K, plain):
     assert np.abs(got[1] - want).max() < 8 * 2.0 ** -16 * np.sqrt(K) + 1e-5
 
 
+# 1 to 10 steps of K a wavefront, which two, three or four in flight share out, and 17; the last step whole, one vector and all but one
+@pytest.mark.parametrize('M,N', [(5, 70), (37, 129)])
+@pytest.mark.parametrize('K', [4, 128, 132, 256, 260, 380, 508, 640, 644, 768, 900, 1024, 1150 // 4 * 4, 1280, 2176])
+def test_fp32_steps_in_flight(M, N, K):
+    """The same bits from [K][N] as it lies as from [N][K], whatever the number of steps in flight; NaNs behind the operands."""
+    A, B = operands('f32', M, N, K, M + K)
+    pad = np.full(64, np.nan, np.float32)
+    dA, dB, dBt = (hk.DeviceBuffer.from_numpy(np.concatenate([x.ravel(), pad])) for x in (A, B, np.ascontiguousarray(B.T)))
+    dC, got, none = hk.DeviceBuffer(M * N * 4), [], hk.ptr_array([])
+    for layout, b in ((0, dB), (1, dBt)):
+        d = hk.GemmDesc()
+        d.in_dtype = d.out_dtype = d.c_dtype = hk.F32
+        d.m, d.n, d.k, d.lda, d.ldb, d.ldc, d.b_layout, d.flags = M, N, K, K, K if layout else N, N, layout, hk.flag_tile('16x16w8')
+        plan = hk.lib().pml_hip_gemm_dispatch(ctypes.byref(d))
+        hk.check(hk.lib().pml_hip_gemm_invoke(plan, dA.ptr, b.ptr, dC.ptr, None, none, none, None))
+        got.append(dC.to_numpy(np.float32, (M, N)))
+        hk.lib().pml_hip_plan_free(plan)
+    check(got[0], A.astype(np.float64) @ B.astype(np.float64), 'f32', K)
+    np.testing.assert_array_equal(got[0], got[1])
+
+
 def test_which_kind_of_fp32_is_asked_of_sizes_alone():
     """Products that may be split, at every size either plain fp32 or three bf16 products from [K][N] and from [N][K], whatever the
     pitch: sizes where one layout's price is past the other's among them."""
