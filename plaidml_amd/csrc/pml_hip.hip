@@ -302,7 +302,8 @@ bool fp32_beats_split(int64_t m, int64_t n, int64_t k_bytes) {
     }
   }
   if (direct_tile_of(m, n, k_bytes, KIND_F32) < 0) return false;
-  (void)direct_tile_of(m, n, k_bytes, KIND_F32, 0, /*always=*/true, true, false, &us);
+  // (two rounds of 16 x 16 tiles over few K take longer than that price: 29 x 3872, K = 96 [N][K] 5.2, direct 6.0)
+  if (direct_tile_of(m, n, k_bytes, KIND_F32, 0, /*always=*/true, true, false, &us) == TILE_16x16_W8 && ((m + 15) / 16) * ((n + 15) / 16) > device_cus()) us += 0.7;
   const double copy = needs_bt ? 3.0 + 2.0 * (double)k_bytes * (double)n / 2.2e6 : 0;
   return us <= 0.95 * split_us && std::min(direct_lies_us(m, n, k_bytes, KIND_F32, 16), direct_lies_us(m, n, k_bytes, KIND_F32, 32)) <= 0.95 * (split_us + copy);
 }
@@ -802,6 +803,8 @@ WinShape window_shape(Plan* p, bool named, double* window_us) {
 //   1 x 1    bf16 28 x 9 x 9 x 256 (*) 62 10.3 -> 5.9     int8 36 x 7 x 7 x 128 (*) 46 8.5 -> 4.7     fp32 3 x 9 x 9 x 96 (*) 23 stride 2 9.7 -> 6.7
 //   3 x 3    bf16 5 x 25 x 25 x 32 (*) 76 8.8 -> 5.2      int8 34 x 14 x 14 x 64 (*) 59 9.5 -> 6.0    fp32 2 x 15 x 15 x 32 (*) 37 10.2 -> 6.8
 //   5 x 5    bf16 11 x 21 x 21 x 64 (*) 102 stride 2 11.7 -> 8.7; but 2 x 69 x 69 x 64 (*) 19, two rounds, 12.2, as it lies 16.9
+//   7 x 7    bf16 from 3 KB of K on by 15 %: 74 x 18 x 40 (*) 16 7.5, as it lies 7.9, under tanh 10.6 and 11.9 (a workgroup's tail is of four
+//            times the results); 2 x 61 x 13 x 32 (*) 9 with a residual 13.9, 14.3
 // and of 140 drawn convolutions with the filter in the call 59 take it, 1.36 x in the mean.
 int given_filter_tile(const Plan* p, double window_us) {
   const pml_hip_conv2d_desc& d = p->conv;
@@ -812,7 +815,8 @@ int given_filter_tile(const Plan* p, double window_us) {
   double packed_us = window_us;
   if (!window) (void)direct_tile_of(M, d.co, k_bytes, p->mfma_kind, 0, p->tile_direct >= 0, /*can_split=*/!p->patches, false, &packed_us);
   const double small = direct_lies_us(M, d.co, k_bytes, p->mfma_kind, 16), large = direct_lies_us(M, d.co, k_bytes, p->mfma_kind, 32), packing = 3.0 + 2.0 * (double)k_bytes * (double)d.co / 2.2e6;
-  if (std::min(small, large) > (p->tile_direct >= 0 ? 0.95 : 0.85) * (packed_us + packing)) return -1;
+  const bool close = p->tile_direct >= 0 && !(p->mfma_kind == KIND_BF16 && k_bytes >= 3072);
+  if (std::min(small, large) > (close ? 0.95 : 0.85) * (packed_us + packing)) return -1;
   return small <= large ? TILE_16x16_W8 : TILE_32x32_W8;
 }
 
@@ -1092,6 +1096,10 @@ static DirectTiles direct_tiles(const pml_hip_gemm_desc& d, int kind, int lds_ti
     const double lies_us = std::min(direct_lies_us(d.m, d.n, d.k * es, kind, 16), direct_lies_us(d.m, d.n, d.k * es, kind, 32));
     if (rows_us > 0.8 * lds_us && lies_us > 1.2 * (lds_us + 3.0 + 2.0 * (double)(d.k * es * d.n) / 2.2e6)) t.rows = -1;
   }
+  if (d.b_layout || d.k2 > 0 || (kind == KIND_F32 && t.rows < 0)) return t;
+  t.given = direct_tile_of(d.m, d.n, d.k * es, kind, d.ldb * es, /*always=*/kind == KIND_F32, /*can_split=*/true, takes_b_as_given(d, kind, lds_tile, d.ldb));
+  return t;
+}
 
 // Whether a launch streams its rows past the [K][N] right-hand side `b` as it lies, with the arguments then changed to that.
 static bool streams_given(int mfma_kind, int tile, bool conv, const void* b, int64_t ldb, IgemmArgs& g) {

@@ -1141,19 +1141,6 @@ __global__ __launch_bounds__(256) void col2im_kernel(Col2imArgs a) {
         *grad = (int)fast_div((unsigned)at, magic, shift);
         if (*grad * stride == at) return k;
       }
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-#pragma unroll
-          for (int e = 0; e < V; ++e) sum[e] += in[u] ? __uint_as_float(w[u].w[e]) : 0.f;
-      }
-    }
-  }
-  const int64_t o = (int64_t)at_pixel * a.CI + c;
-  if constexpr (BF) {
-    uint16_t h[V];
-#pragma unroll
-    for (int e = 0; e < V; ++e) h[e] = f32_to_bf16_bits(sum[e]);
-    __builtin_memcpy((uint16_t*)a.out + o, h, sizeof h);
       return taps;
     };
     int gy0 = 0, gx0 = 0;
@@ -1174,6 +1161,19 @@ __global__ __launch_bounds__(256) void col2im_kernel(Col2imArgs a) {
           in[u] = k < a.KW && g >= 0 && g < a.OW;
           if (in[u]) w[u] = load_words<V>(row + ((int64_t)g * taps + k) * a.CI);
         }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+          for (int e = 0; e < V; ++e) sum[e] += in[u] ? __uint_as_float(w[u].w[e]) : 0.f;
+      }
+    }
+  }
+  const int64_t o = (int64_t)at_pixel * a.CI + c;
+  if constexpr (BF) {
+    uint16_t h[V];
+#pragma unroll
+    for (int e = 0; e < V; ++e) h[e] = f32_to_bf16_bits(sum[e]);
+    __builtin_memcpy((uint16_t*)a.out + o, h, sizeof h);
   } else {
     __builtin_memcpy((float*)a.out + o, sum, sizeof sum);
   }
@@ -1285,9 +1285,14 @@ hipError_t col2im_launch(const Col2imArgs& args, bool bf, hipStream_t s) {
   Col2imArgs a = args;
   a.period_h = a.SH / std::gcd(a.SH, a.DH);
   a.period_w = a.SW / std::gcd(a.SW, a.DW);
+  a.step_h = a.period_h * a.DH / a.SH;
+  a.step_w = a.period_w * a.DW / a.SW;
   const int v = a.CI >= 4 ? 4 : 1;
   const int64_t blocks = ((int64_t)a.N * a.H * a.W * ((a.CI + v - 1) / v) + 255) / 256;
   if (blocks <= 0 || blocks > kMaxLaunchThreads / 256) return hipErrorInvalidValue;
+  fast_div_magic((unsigned)a.W, &a.w_magic, &a.w_shift);
+  fast_div_magic((unsigned)a.SH, &a.sh_magic, &a.sh_shift);
+  fast_div_magic((unsigned)a.SW, &a.sw_magic, &a.sw_shift);
   const dim3 grid((unsigned)blocks), block(256);
   const bool one = a.KH * a.KW == 1;
 #define PML_GO(BF, V)                                                                          \
@@ -1302,15 +1307,11 @@ hipError_t col2im_launch(const Col2imArgs& args, bool bf, hipStream_t s) {
   } else {
     PML_GO(false, 1);
   }
+#undef PML_GO
   return hipGetLastError();
-  a.step_h = a.period_h * a.DH / a.SH;
-  a.step_w = a.period_w * a.DW / a.SW;
 }
 
 hipError_t gradient_operands_launch(int es, const void* in, void* out, int64_t pad_rows, int64_t cols, int64_t pitch, const void* f, void* bt, int64_t taps,
-  fast_div_magic((unsigned)a.W, &a.w_magic, &a.w_shift);
-  fast_div_magic((unsigned)a.SH, &a.sh_magic, &a.sh_shift);
-  fast_div_magic((unsigned)a.SW, &a.sw_magic, &a.sw_shift);
                                     int64_t ci, int64_t co, hipStream_t s) {
   const int64_t flip = bt ? (taps * ci * co + 255) / 256 : 0;
   const int64_t pad = std::min<int64_t>((pad_rows * (pitch * es / 16) + 255) / 256, 256 * 32);
@@ -1319,7 +1320,6 @@ hipError_t gradient_operands_launch(int es, const void* in, void* out, int64_t p
   const dim3 grid((unsigned)(flip + pad)), block(256);
   if (es == 2)
     hipLaunchKernelGGL(gradient_operands_kernel<uint16_t>, grid, block, 0, s, (const uint16_t*)in, (uint16_t*)out, pad_rows, (int)cols, (int)pitch, (const uint16_t*)f,
-#undef PML_GO
                        (uint16_t*)bt, (int)taps, (int)ci, (int)co, flip);
   else
     hipLaunchKernelGGL(gradient_operands_kernel<uint32_t>, grid, block, 0, s, (const uint32_t*)in, (uint32_t*)out, pad_rows, (int)cols, (int)pitch, (const uint32_t*)f,
