@@ -195,16 +195,13 @@ bool splits_k(int64_t m, int64_t n, int64_t k_bytes, int kind) {
 // (3881 x 3959, K = 2992 723 us, 760 in tiles of 64; 2381 x 1595, K = 2608 171, 180), while half a round of them more costs as much as
 // two of 64: 3271 x 547, K = 448 36.2 -> 21.6, 2322 x 2041, K = 304 47.7 -> 35.4, 1246 x 4028, K = 208 35.6 -> 27.1, convolutions
 // 38400 x 122, K = 2304 294 -> 209, 13689 x 179, K = 3200 212 -> 168.
-// (One slab is tail more than MFMAs, and two tiles of 128 share a CU: there a last round more than half full is no whole one.
-// 7295 x 944, K = 12 13.1, in tiles of 64 14.1, 4690 x 1308, K = 28 13.1, 13.7; with a smaller share of both grids for edges alike.)
-bool f32_tiles_of_128(int64_t m, int64_t n, int64_t k_bytes) {
+bool f32_tiles_of_128(int64_t m, int64_t n) {
   const int64_t cus = device_cus(), t128 = ((m + 127) / 128) * ((n + 127) / 128), t64 = ((m + 63) / 64) * ((n + 63) / 64);
-  if (k_bytes <= 128 && t128 >= cus && 2 * (t128 % cus) >= cus && 10 * t64 >= 37 * t128) return true;
   return t128 >= 128 && 4 * ((t128 + cus - 1) / cus) <= (t64 + cus - 1) / cus;
 }
-double f32_slab_us(int64_t m, int64_t n, int64_t k_bytes) {
+double f32_slab_us(int64_t m, int64_t n) {
   const int64_t cus = device_cus(), t128 = ((m + 127) / 128) * ((n + 127) / 128), t64 = ((m + 63) / 64) * ((n + 63) / 64);
-  return f32_tiles_of_128(m, n, k_bytes) ? 2.2 * (double)((t128 + cus - 1) / cus) : 0.58 * (double)((t64 + cus - 1) / cus);
+  return f32_tiles_of_128(m, n) ? 2.2 * (double)((t128 + cus - 1) / cus) : 0.58 * (double)((t64 + cus - 1) / cus);
 }
 
 // One of the direct tiles (direct.hip) where it beats the LDS kernels, or -1.  Both sides are priced in microseconds, from
@@ -229,9 +226,9 @@ double f32_slab_us(int64_t m, int64_t n, int64_t k_bytes) {
 // its bytes both ways at 2.2 TB/s:
 // bf16 512 x 512 x 512 9.4 -> 5.0, 1024^3 14.6 -> 10.6, 64 x 2048 x 2048 16.5 -> 8.8; fp32 128 x 4096 x 1024 23.4 -> 12.3.
 // kn_ldb: that right-hand side's row pitch in bytes (0: Bt); always: the better of the two whatever the LDS kernel takes;
-// can_split: the LDS kernel may split K; lds: what an LDS kernel takes; as_given: it reads a [K][N] right-hand side as it lies (256 x 49152, K = 4096 bf16:
+// can_split: the LDS kernel may split K; as_given: it reads a [K][N] right-hand side as it lies (256 x 49152, K = 4096 bf16:
 // 409 us direct, 135 with 256 x 256 tiles; charged the copy of 800 MB, they lost)
-int direct_tile_of(int64_t m, int64_t n, int64_t k_bytes, int kind, int64_t kn_ldb = 0, bool always = false, bool can_split = true, bool as_given = false, double* us = nullptr, double* lds = nullptr) {
+int direct_tile_of(int64_t m, int64_t n, int64_t k_bytes, int kind, int64_t kn_ldb = 0, bool always = false, bool can_split = true, bool as_given = false, double* us = nullptr) {
   if (kind != KIND_F32 && kind != KIND_BF16 && kind != KIND_I8) return -1;
   auto tiles = [&](int64_t bm, int64_t bn) { return ((m + bm - 1) / bm) * ((n + bn - 1) / bn); };
   const double kb = (double)k_bytes;
@@ -250,7 +247,7 @@ int direct_tile_of(int64_t m, int64_t n, int64_t k_bytes, int kind, int64_t kn_l
     return 2.6 + rounds * (start + (double)(std::min(m, side) + (f32 && w ? wide : std::min(n, wide))) * kb / r);
   };
   const int64_t slabs = (k_bytes + 127) / 128;
-  double lds_us = 4.2 + (f32 ? f32_slab_us(m, n, k_bytes) : kind == KIND_I8 ? 0.28 : 0.23) * (double)slabs;
+  double lds_us = 4.2 + (f32 ? f32_slab_us(m, n) : kind == KIND_I8 ? 0.28 : 0.23) * (double)slabs;
   bool needs_bt = !as_given && (kind == KIND_BF16 || n % (16 / es) != 0 || kn_ldb % 16 != 0);
   if (can_split && splits_k(m, n, k_bytes, kind)) {
     int splits = 1, per = 0;
@@ -264,7 +261,6 @@ int direct_tile_of(int64_t m, int64_t n, int64_t k_bytes, int kind, int64_t kn_l
   const double small = direct_us(16), large = direct_us(32);
   const bool direct = always || std::min(small, large) <= 0.95 * lds_us;
   if (us) *us = direct ? std::min(small, large) : lds_us;
-  if (lds) *lds = lds_us;
   if (!direct) return -1;
   return small <= large ? TILE_16x16_W8 : TILE_32x32_W8;
 }
@@ -302,8 +298,7 @@ bool fp32_beats_split(int64_t m, int64_t n, int64_t k_bytes) {
     }
   }
   if (direct_tile_of(m, n, k_bytes, KIND_F32) < 0) return false;
-  // (two rounds of 16 x 16 tiles over few K take longer than that price: 29 x 3872, K = 96 [N][K] 5.2, direct 6.0)
-  if (direct_tile_of(m, n, k_bytes, KIND_F32, 0, /*always=*/true, true, false, &us) == TILE_16x16_W8 && ((m + 15) / 16) * ((n + 15) / 16) > device_cus()) us += 0.7;
+  (void)direct_tile_of(m, n, k_bytes, KIND_F32, 0, /*always=*/true, true, false, &us);
   const double copy = needs_bt ? 3.0 + 2.0 * (double)k_bytes * (double)n / 2.2e6 : 0;
   return us <= 0.95 * split_us && std::min(direct_lies_us(m, n, k_bytes, KIND_F32, 16), direct_lies_us(m, n, k_bytes, KIND_F32, 32)) <= 0.95 * (split_us + copy);
 }
@@ -387,7 +382,7 @@ int choose_tile(int64_t m, int64_t n, int64_t k_bytes, int kind, const TailForm&
   // convolutions with K of less than 2 KB those of up to 256 tiles took 1.05 to 1.16 x as long in plain ones (relu 1.08, residual 1.11,
   // scale and shift 1.05), those of up to 512 1.00 to 1.07 -- but for scale and shift, 0.96 to 1.03, unless rows off 16 bytes leave
   // step by step (1.3).
-  if (kind == KIND_F32 && !f32_tiles_of_128(m, n, k_bytes))
+  if (kind == KIND_F32 && !f32_tiles_of_128(m, n))
     return tiles(64, 64) <= (k_bytes < 2048 && tail.steps && n % 4 == 0 ? 256 : 512) ? TILE_64x64_W8_K2 : TILE_64x64;
   if (tiles(128, 128) >= 256) return TILE_128x128_W8_S2;
   // (two slabs and less are all launch, first loads and tail: bf16 conv 8750 x 138, K = 64 9.4 -> 6.6 us, 23958 x 105, K = 128 9.6 -> 8.1.
@@ -791,7 +786,7 @@ WinShape window_shape(Plan* p, bool named, double* window_us) {
   }
   if (p->mfma_kind == KIND_F32) {
     const double mma_us = (double)((g.M + 63) / 64 * 64) * (double)((g.N + 63) / 64 * 64) * (double)g.K * 2 / 154e6;
-    const double tiles_us = 4.2 + f32_slab_us(g.M, g.N, k_bytes) * (double)conv_slabs(d);
+    const double tiles_us = 4.2 + f32_slab_us(g.M, g.N) * (double)conv_slabs(d);
     return us < std::max(4 + 1.45 * mma_us, 0.93 * tiles_us) ? shape : WinShape{};
   }
   return shape;
@@ -803,8 +798,6 @@ WinShape window_shape(Plan* p, bool named, double* window_us) {
 //   1 x 1    bf16 28 x 9 x 9 x 256 (*) 62 10.3 -> 5.9     int8 36 x 7 x 7 x 128 (*) 46 8.5 -> 4.7     fp32 3 x 9 x 9 x 96 (*) 23 stride 2 9.7 -> 6.7
 //   3 x 3    bf16 5 x 25 x 25 x 32 (*) 76 8.8 -> 5.2      int8 34 x 14 x 14 x 64 (*) 59 9.5 -> 6.0    fp32 2 x 15 x 15 x 32 (*) 37 10.2 -> 6.8
 //   5 x 5    bf16 11 x 21 x 21 x 64 (*) 102 stride 2 11.7 -> 8.7; but 2 x 69 x 69 x 64 (*) 19, two rounds, 12.2, as it lies 16.9
-//   7 x 7    bf16 from 3 KB of K on by 15 %: 74 x 18 x 40 (*) 16 7.5, as it lies 7.9, under tanh 10.6 and 11.9 (a workgroup's tail is of four
-//            times the results); 2 x 61 x 13 x 32 (*) 9 with a residual 13.9, 14.3
 // and of 140 drawn convolutions with the filter in the call 59 take it, 1.36 x in the mean.
 int given_filter_tile(const Plan* p, double window_us) {
   const pml_hip_conv2d_desc& d = p->conv;
@@ -815,8 +808,7 @@ int given_filter_tile(const Plan* p, double window_us) {
   double packed_us = window_us;
   if (!window) (void)direct_tile_of(M, d.co, k_bytes, p->mfma_kind, 0, p->tile_direct >= 0, /*can_split=*/!p->patches, false, &packed_us);
   const double small = direct_lies_us(M, d.co, k_bytes, p->mfma_kind, 16), large = direct_lies_us(M, d.co, k_bytes, p->mfma_kind, 32), packing = 3.0 + 2.0 * (double)k_bytes * (double)d.co / 2.2e6;
-  const bool close = p->tile_direct >= 0 && !(p->mfma_kind == KIND_BF16 && k_bytes >= 3072);
-  if (std::min(small, large) > (close ? 0.95 : 0.85) * (packed_us + packing)) return -1;
+  if (std::min(small, large) > (p->tile_direct >= 0 ? 0.95 : 0.85) * (packed_us + packing)) return -1;
   return small <= large ? TILE_16x16_W8 : TILE_32x32_W8;
 }
 
@@ -1088,14 +1080,6 @@ static DirectTiles direct_tiles(const pml_hip_gemm_desc& d, int kind, int lds_ti
   // (Two products are priced against one chain of all slabs: of 49 x 2048, K = 512 + 1024 the split takes 9.2 us and the direct
   // tile 8.8, of 196 x 256, K = 1024 + 512 9.0 and 5.8; only a K of 4096 turns that round, 10.7 and 17.0.)
   t.rows = direct_tile_of(d.m, d.n, (d.k + d.k2) * es, kind, 0, false, /*can_split=*/d.k2 == 0);
-  // (fp32 of a long K over a few columns, which gains little from rows of K and loses more over [K][N], where K is not split: 6 x 59,
-  // K = 4000 12.9 -> 13.1 and 17.3 -> 21.4; 1030 x 36, K = 2608 12.6 -> 9.7 and 16.0 -> 16.9 stays)
-  if (kind == KIND_F32 && t.rows >= 0 && splits_k(d.m, d.n, d.k * es, kind)) {
-    double rows_us = 0, lds_us = 0;
-    (void)direct_tile_of(d.m, d.n, d.k * es, kind, 0, /*always=*/true, true, false, &rows_us, &lds_us);
-    const double lies_us = std::min(direct_lies_us(d.m, d.n, d.k * es, kind, 16), direct_lies_us(d.m, d.n, d.k * es, kind, 32));
-    if (rows_us > 0.8 * lds_us && lies_us > 1.2 * (lds_us + 3.0 + 2.0 * (double)(d.k * es * d.n) / 2.2e6)) t.rows = -1;
-  }
   if (d.b_layout || d.k2 > 0 || (kind == KIND_F32 && t.rows < 0)) return t;
   t.given = direct_tile_of(d.m, d.n, d.k * es, kind, d.ldb * es, /*always=*/kind == KIND_F32, /*can_split=*/true, takes_b_as_given(d, kind, lds_tile, d.ldb));
   return t;

@@ -316,12 +316,7 @@ struct Side {
       for (int r = 0; r < kRuns; ++r) straight(&regs[kWords * r], runs[r].hi > runs[r].lo ? runs[r].at : 0);
     } else {
 #pragma unroll
-      for (int r = 0; r < kRuns; ++r) {
-        if (runs[r].lo == 0 && runs[r].hi == kVals && apart == 1)
-          straight(&regs[kWords * r], runs[r].at);
-        else
-          gather(&regs[kWords * r], runs[r].at, runs[r].lo, runs[r].hi, apart);
-      }
+      for (int r = 0; r < kRuns; ++r) gather(&regs[kWords * r], runs[r].at, runs[r].lo, runs[r].hi, apart);
     }
   }
 
@@ -1044,9 +1039,7 @@ hipError_t product_direct_launch(const StridedArgs& a, bool bf, int rows, hipStr
 // K = 33, bf16: 44.1 and 18.4); K is split when the tiles alone leave CUs idle, into runs of at least
 // four slabs, for about three workgroups per CU (their LDS fits four times into one).  A filter gradient's slab takes as long as
 // its loads: runs of two slabs and more (567 pixels of 3 x 45 x 20 in bf16 12.4 -> 9.5 us, 2116 of 3 x 60 x 18 in fp32 12.4 -> 9.2),
-// and in fp32, whose workgroups fit four times into a CU's registers, four per CU (50176 of 3 x 192 x 64 64.5 -> 61.1) -- but for
-// partial results of 300 KB a split, which a second launch reads again: those only up to 6 MB, or with eight slabs a run left (1512
-// pixels of 3 x 348 x 112 in fp32, 468 KB: 12 splits 18.2, 24 of two slabs 20.1; 2173 of 3 x 510 x 66, 404 KB: 14 24.1, 17 25.7).
+// and in fp32, whose workgroups fit four times into a CU's registers, four per CU (50176 of 3 x 192 x 64 64.5 -> 61.1).
 void strided_plan(StridedArgs* a, bool bf, bool conv, int n_cus, int* mi) {
   int64_t batches = 1;
   for (int d = 0; d < a->n_batch; ++d) batches *= a->batch[d];
@@ -1066,14 +1059,9 @@ void strided_plan(StridedArgs* a, bool bf, bool conv, int n_cus, int* mi) {
   a->ws_pitch = (a->N + 3) / 4 * 4;
   const int64_t have = tiles(t);
   if (have < n_cus && slabs >= 8) {
-    const int64_t three = (3 * n_cus + have - 1) / have, bytes = std::max<int64_t>(1, a->ws_rows * a->ws_pitch * 4);
-    int64_t want = std::min(three, slabs / 4);
-    if (conv) {
-      const int64_t fits = bytes <= 300 << 10 ? slabs : std::max(((int64_t)6 << 20) / bytes, slabs / 8);
-      want = std::max(want, std::min({bf ? three : 4 * n_cus / have, slabs / 2, fits}));
-    }
+    int64_t want = std::min<int64_t>(conv && !bf ? 4 * n_cus / have : (3 * n_cus + have - 1) / have, slabs / (conv ? 2 : 4));
     // the partial results: at most 256 MiB of them
-    want = std::min<int64_t>(want, ((int64_t)256 << 20) / bytes);
+    want = std::min<int64_t>(want, ((int64_t)256 << 20) / std::max<int64_t>(1, a->ws_rows * a->ws_pitch * 4));
     if (want >= 2) {
       const int64_t per = (slabs + want - 1) / want;
       a->k_per_split = per * bk;
@@ -1112,60 +1100,46 @@ namespace {
 // A thread per V channels of an image pixel (the last V of a pixel overlap the ones before them where CI is no multiple of V);
 // columns are read once, V * 4 bytes at a time.  What bounds it is a thread's chain of loads: only the taps that meet a gradient
 // pixel are visited, up to four of a filter row are on their way at once.  5 x 75 x 75 x 121 from 5 x 5 taps of stride 2, bf16:
-// 60 us a value a thread and a tap at a time, now 16.  Few taps are a chain of divisions: those by W and the strides are multiplies.
-// ONE: filters of one tap, where there is nothing to add up.
-template <bool BF, int V, bool ONE>
+// 60 us a value a thread and a tap at a time, now 16.
+template <bool BF, int V>
 __global__ __launch_bounds__(256) void col2im_kernel(Col2imArgs a) {
   const unsigned cv = (unsigned)(a.CI + V - 1) / V, per_img = (unsigned)(a.H * a.W);
   const unsigned g = blockIdx.x * 256 + threadIdx.x;
-  const unsigned at_pixel = g / cv;  // (up to 2^32 of them: no multiply-and-shift)
+  const unsigned at_pixel = g / cv;
   if (at_pixel >= (unsigned)a.N * per_img) return;
   const unsigned chunk = g - at_pixel * cv, img = at_pixel / per_img, pix = at_pixel - img * per_img;
-  const int y = (int)fast_div(pix, a.w_magic, a.w_shift), x = (int)(pix - (unsigned)y * (unsigned)a.W);
+  const int y = (int)(pix / (unsigned)a.W), x = (int)(pix - (unsigned)y * (unsigned)a.W);
   const int c = (int)chunk * V + V <= a.CI ? (int)chunk * V : a.CI - V;
+  // the first tap of a column or row of them whose window meets a gradient pixel; from there every period-th does
+  auto first = [](int at, int taps, int period, int stride, int dil) {
+    for (int k = 0; k < period && k < taps; ++k)
+      if ((at - k * dil) % stride == 0) return k;
+    return taps;
+  };
+  const int ky0 = first(y + a.PH, a.KH, a.period_h, a.SH, a.DH), kx0 = first(x + a.PW, a.KW, a.period_w, a.SW, a.DW);
+  const int gy0 = (y + a.PH - ky0 * a.DH) / a.SH, gx0 = (x + a.PW - kx0 * a.DW) / a.SW;
+  const int dy = a.period_h * a.DH / a.SH, dx = a.period_w * a.DW / a.SW;
+  const int taps = a.KH * a.KW;
   float sum[V];
 #pragma unroll
   for (int e = 0; e < V; ++e) sum[e] = 0.f;
-  if constexpr (ONE) {
-    const int gy = (int)fast_div((unsigned)(y + a.PH), a.sh_magic, a.sh_shift), gx = (int)fast_div((unsigned)(x + a.PW), a.sw_magic, a.sw_shift);
-    if (gy * a.SH == y + a.PH && gx * a.SW == x + a.PW && gy < a.OH && gx < a.OW) {
-      const Words<V> w = load_words<V>(a.cols + (((int64_t)img * a.OH + gy) * a.OW + gx) * a.CI + c);
+  for (int ky = ky0, gy = gy0; ky < a.KH; ky += a.period_h, gy -= dy) {
+    if (gy < 0 || gy >= a.OH) continue;
+    const float* const row = a.cols + ((int64_t)img * a.OH + gy) * a.OW * taps * a.CI + (int64_t)ky * a.KW * a.CI + c;
+    constexpr int U = 4;
+    for (int kx = kx0, gx = gx0; kx < a.KW; kx += U * a.period_w, gx -= U * dx) {
+      Words<V> w[U];
+      bool in[U];
 #pragma unroll
-      for (int e = 0; e < V; ++e) sum[e] += __uint_as_float(w.w[e]);
-    }
-  } else {
-    // the first tap of a column or row of them whose window meets a row or column of the gradient, and which; from there every
-    // period-th does, further up and left (above and left of the gradient: no further tap meets it)
-    auto first = [](int at, int taps, int period, int stride, unsigned magic, int shift, int dil, int* grad) {
-      for (int k = 0; k < period && k < taps && at >= 0; ++k, at -= dil) {
-        *grad = (int)fast_div((unsigned)at, magic, shift);
-        if (*grad * stride == at) return k;
+      for (int u = 0; u < U; ++u) {
+        const int k = kx + u * a.period_w, g = gx - u * dx;
+        in[u] = k < a.KW && g >= 0 && g < a.OW;
+        if (in[u]) w[u] = load_words<V>(row + ((int64_t)g * taps + k) * a.CI);
       }
-      return taps;
-    };
-    int gy0 = 0, gx0 = 0;
-    const int ky0 = first(y + a.PH, a.KH, a.period_h, a.SH, a.sh_magic, a.sh_shift, a.DH, &gy0);
-    const int kx0 = first(x + a.PW, a.KW, a.period_w, a.SW, a.sw_magic, a.sw_shift, a.DW, &gx0);
-    const int dy = a.step_h, dx = a.step_w;
-    const int taps = a.KH * a.KW;
-    for (int ky = ky0, gy = gy0; ky < a.KH; ky += a.period_h, gy -= dy) {
-      if (gy < 0 || gy >= a.OH) continue;
-      const float* const row = a.cols + ((int64_t)img * a.OH + gy) * a.OW * taps * a.CI + (int64_t)ky * a.KW * a.CI + c;
-      constexpr int U = 4;
-      for (int kx = kx0, gx = gx0; kx < a.KW; kx += U * a.period_w, gx -= U * dx) {
-        Words<V> w[U];
-        bool in[U];
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-          const int k = kx + u * a.period_w, g = gx - u * dx;
-          in[u] = k < a.KW && g >= 0 && g < a.OW;
-          if (in[u]) w[u] = load_words<V>(row + ((int64_t)g * taps + k) * a.CI);
-        }
+      for (int u = 0; u < U; ++u)
 #pragma unroll
-        for (int u = 0; u < U; ++u)
-#pragma unroll
-          for (int e = 0; e < V; ++e) sum[e] += in[u] ? __uint_as_float(w[u].w[e]) : 0.f;
-      }
+        for (int e = 0; e < V; ++e) sum[e] += in[u] ? __uint_as_float(w[u].w[e]) : 0.f;
     }
   }
   const int64_t o = (int64_t)at_pixel * a.CI + c;
@@ -1285,29 +1259,17 @@ hipError_t col2im_launch(const Col2imArgs& args, bool bf, hipStream_t s) {
   Col2imArgs a = args;
   a.period_h = a.SH / std::gcd(a.SH, a.DH);
   a.period_w = a.SW / std::gcd(a.SW, a.DW);
-  a.step_h = a.period_h * a.DH / a.SH;
-  a.step_w = a.period_w * a.DW / a.SW;
   const int v = a.CI >= 4 ? 4 : 1;
   const int64_t blocks = ((int64_t)a.N * a.H * a.W * ((a.CI + v - 1) / v) + 255) / 256;
   if (blocks <= 0 || blocks > kMaxLaunchThreads / 256) return hipErrorInvalidValue;
-  fast_div_magic((unsigned)a.W, &a.w_magic, &a.w_shift);
-  fast_div_magic((unsigned)a.SH, &a.sh_magic, &a.sh_shift);
-  fast_div_magic((unsigned)a.SW, &a.sw_magic, &a.sw_shift);
   const dim3 grid((unsigned)blocks), block(256);
-  const bool one = a.KH * a.KW == 1;
-#define PML_GO(BF, V)                                                                          \
-  if (one) hipLaunchKernelGGL((col2im_kernel<BF, V, true>), grid, block, 0, s, a);            \
-  else hipLaunchKernelGGL((col2im_kernel<BF, V, false>), grid, block, 0, s, a)
-  if (bf && v == 4) {
-    PML_GO(true, 4);
-  } else if (bf) {
-    PML_GO(true, 1);
-  } else if (v == 4) {
-    PML_GO(false, 4);
+  if (bf) {
+    if (v == 4) hipLaunchKernelGGL((col2im_kernel<true, 4>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((col2im_kernel<true, 1>), grid, block, 0, s, a);
   } else {
-    PML_GO(false, 1);
+    if (v == 4) hipLaunchKernelGGL((col2im_kernel<false, 4>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((col2im_kernel<false, 1>), grid, block, 0, s, a);
   }
-#undef PML_GO
   return hipGetLastError();
 }
 

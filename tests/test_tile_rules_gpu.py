@@ -91,46 +91,3 @@ def test_fp32_under_scale_and_shift(m, n, k, tail, shared):
     named = run('f32', m, n, k, tail, tile='64x64w8k2' if shared else '64x64')[0]
     np.testing.assert_array_equal(got, named)
     assert (np.abs(got - want) <= bound).all()
-
-
-def text_of(kind, m, n, k, layout=0, flags=0):
-    d = hk.GemmDesc()
-    d.in_dtype = d.out_dtype = d.c_dtype = kind
-    d.m, d.n, d.k, d.lda, d.ldb, d.ldc, d.b_layout, d.flags = m, n, k, k, k if layout else n, n, layout, flags
-    plan = hk.lib().pml_hip_gemm_dispatch(ctypes.byref(d))
-    text = hk.describe(plan)
-    hk.lib().pml_hip_plan_free(plan)
-    return text
-
-
-# one slab over 1.78 and 1.59 rounds of 128 x 128; a round less than half full; edges that cost the large tiles more; two slabs
-@pytest.mark.parametrize('m,n,k,large', [(7295, 944, 12, True), (4690, 1308, 28, True), (9911, 400, 12, False), (50809, 272, 28, False), (7295, 944, 36, False)])
-def test_fp32_of_one_slab(m, n, k, large):
-    assert ('tile=128x128 (8 wavefronts, 2 stages) ' if large else PLAIN) in text_of(hk.F32, m, n, k)
-
-
-@pytest.mark.parametrize('layout', [0, 1])
-@pytest.mark.parametrize('m,n,k,direct', [(6, 59, 4000, False), (1030, 36, 2608, True), (2, 37, 3500, True), (6, 59, 1200, True)])
-def test_fp32_of_a_long_k_and_few_columns(m, n, k, direct, layout):
-    """Split in both layouts where a direct tile loses more over [K][N] than it gains over rows of K."""
-    text = text_of(hk.F32, m, n, k, layout)
-    assert ('with rows of K at hand' in text) == direct and ('with B as it lies' in text) == (direct and not layout), text
-
-
-@pytest.mark.parametrize('layout', [0, 1])
-@pytest.mark.parametrize('m,n,k,split', [(29, 3872, 96, True), (34, 2320, 96, True), (40, 1800, 200, False), (16, 3872, 96, False)])
-def test_split_fp32_of_two_rounds(m, n, k, split, layout):
-    assert ('3 x f32' in text_of(hk.F32, m, n, k, layout, hk.FP32_AS_BF16X3)) == split
-
-
-# 7 x 7 taps of 40 channels, 4 KB of K; the same in int8 and of fewer channels
-@pytest.mark.parametrize('kind,out,ci,lies', [(hk.BF16, hk.BF16, 40, False), (hk.I8, hk.I32, 32, True), (hk.BF16, hk.BF16, 16, True)])
-def test_filters_of_a_long_k_that_come_with_the_call(kind, out, ci, lies):
-    d = hk.Conv2dDesc()
-    d.in_dtype, d.out_dtype, d.c_dtype = kind, out, out
-    d.n, d.h, d.w, d.ci, d.kh, d.kw, d.co, d.oh, d.ow = 1, 74, 18, ci, 7, 7, 16, 74, 18
-    d.stride_h = d.stride_w = d.dil_h = d.dil_w = 1
-    d.pad_h = d.pad_w = 3
-    plan = hk.lib().pml_hip_conv2d_dispatch(ctypes.byref(d))
-    assert ('with the filter as it lies' in hk.describe(plan)) == lies, hk.describe(plan)
-    hk.lib().pml_hip_plan_free(plan)
