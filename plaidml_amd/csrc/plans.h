@@ -378,7 +378,11 @@ struct Col2imArgs {
   const float* cols;  // [N][OH][OW][KH][KW][CI]
   void* out;          // [N][H][W][CI]
   int N, H, W, CI, OH, OW, KH, KW, SH, SW, PH, PW, DH, DW;
-  int period_h, period_w;  // (of the taps that meet a gradient pixel, set by the launch)
+  // set by the launch: the period of the taps that meet a gradient pixel, how many pixels further up and left the next one meets;
+  // n / W, n / SH and n / SW as multiply-and-shift (fast_div)
+  int period_h, period_w, step_h, step_w;
+  unsigned w_magic, sh_magic, sw_magic;
+  int w_shift, sh_shift, sw_shift;
 };
 hipError_t col2im_launch(const Col2imArgs& a, bool bf, hipStream_t s);
 struct ConvBorderArgs {

@@ -1100,46 +1100,60 @@ namespace {
 // A thread per V channels of an image pixel (the last V of a pixel overlap the ones before them where CI is no multiple of V);
 // columns are read once, V * 4 bytes at a time.  What bounds it is a thread's chain of loads: only the taps that meet a gradient
 // pixel are visited, up to four of a filter row are on their way at once.  5 x 75 x 75 x 121 from 5 x 5 taps of stride 2, bf16:
-// 60 us a value a thread and a tap at a time, now 16.
-template <bool BF, int V>
+// 60 us a value a thread and a tap at a time, now 16.  Few taps are a chain of divisions: those by W and the strides are multiplies.
+// ONE: filters of one tap, where there is nothing to add up.
+template <bool BF, int V, bool ONE>
 __global__ __launch_bounds__(256) void col2im_kernel(Col2imArgs a) {
   const unsigned cv = (unsigned)(a.CI + V - 1) / V, per_img = (unsigned)(a.H * a.W);
   const unsigned g = blockIdx.x * 256 + threadIdx.x;
-  const unsigned at_pixel = g / cv;
+  const unsigned at_pixel = g / cv;  // (up to 2^32 of them: no multiply-and-shift)
   if (at_pixel >= (unsigned)a.N * per_img) return;
   const unsigned chunk = g - at_pixel * cv, img = at_pixel / per_img, pix = at_pixel - img * per_img;
-  const int y = (int)(pix / (unsigned)a.W), x = (int)(pix - (unsigned)y * (unsigned)a.W);
+  const int y = (int)fast_div(pix, a.w_magic, a.w_shift), x = (int)(pix - (unsigned)y * (unsigned)a.W);
   const int c = (int)chunk * V + V <= a.CI ? (int)chunk * V : a.CI - V;
-  // the first tap of a column or row of them whose window meets a gradient pixel; from there every period-th does
-  auto first = [](int at, int taps, int period, int stride, int dil) {
-    for (int k = 0; k < period && k < taps; ++k)
-      if ((at - k * dil) % stride == 0) return k;
-    return taps;
-  };
-  const int ky0 = first(y + a.PH, a.KH, a.period_h, a.SH, a.DH), kx0 = first(x + a.PW, a.KW, a.period_w, a.SW, a.DW);
-  const int gy0 = (y + a.PH - ky0 * a.DH) / a.SH, gx0 = (x + a.PW - kx0 * a.DW) / a.SW;
-  const int dy = a.period_h * a.DH / a.SH, dx = a.period_w * a.DW / a.SW;
-  const int taps = a.KH * a.KW;
   float sum[V];
 #pragma unroll
   for (int e = 0; e < V; ++e) sum[e] = 0.f;
-  for (int ky = ky0, gy = gy0; ky < a.KH; ky += a.period_h, gy -= dy) {
-    if (gy < 0 || gy >= a.OH) continue;
-    const float* const row = a.cols + ((int64_t)img * a.OH + gy) * a.OW * taps * a.CI + (int64_t)ky * a.KW * a.CI + c;
-    constexpr int U = 4;
-    for (int kx = kx0, gx = gx0; kx < a.KW; kx += U * a.period_w, gx -= U * dx) {
-      Words<V> w[U];
-      bool in[U];
+  if constexpr (ONE) {
+    const int gy = (int)fast_div((unsigned)(y + a.PH), a.sh_magic, a.sh_shift), gx = (int)fast_div((unsigned)(x + a.PW), a.sw_magic, a.sw_shift);
+    if (gy * a.SH == y + a.PH && gx * a.SW == x + a.PW && gy < a.OH && gx < a.OW) {
+      const Words<V> w = load_words<V>(a.cols + (((int64_t)img * a.OH + gy) * a.OW + gx) * a.CI + c);
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int k = kx + u * a.period_w, g = gx - u * dx;
-        in[u] = k < a.KW && g >= 0 && g < a.OW;
-        if (in[u]) w[u] = load_words<V>(row + ((int64_t)g * taps + k) * a.CI);
+      for (int e = 0; e < V; ++e) sum[e] += __uint_as_float(w.w[e]);
+    }
+  } else {
+    // the first tap of a column or row of them whose window meets a row or column of the gradient, and which; from there every
+    // period-th does, further up and left (above and left of the gradient: no further tap meets it)
+    auto first = [](int at, int taps, int period, int stride, unsigned magic, int shift, int dil, int* grad) {
+      for (int k = 0; k < period && k < taps && at >= 0; ++k, at -= dil) {
+        *grad = (int)fast_div((unsigned)at, magic, shift);
+        if (*grad * stride == at) return k;
       }
+      return taps;
+    };
+    int gy0 = 0, gx0 = 0;
+    const int ky0 = first(y + a.PH, a.KH, a.period_h, a.SH, a.sh_magic, a.sh_shift, a.DH, &gy0);
+    const int kx0 = first(x + a.PW, a.KW, a.period_w, a.SW, a.sw_magic, a.sw_shift, a.DW, &gx0);
+    const int dy = a.step_h, dx = a.step_w;
+    const int taps = a.KH * a.KW;
+    for (int ky = ky0, gy = gy0; ky < a.KH; ky += a.period_h, gy -= dy) {
+      if (gy < 0 || gy >= a.OH) continue;
+      const float* const row = a.cols + ((int64_t)img * a.OH + gy) * a.OW * taps * a.CI + (int64_t)ky * a.KW * a.CI + c;
+      constexpr int U = 4;
+      for (int kx = kx0, gx = gx0; kx < a.KW; kx += U * a.period_w, gx -= U * dx) {
+        Words<V> w[U];
+        bool in[U];
 #pragma unroll
-      for (int u = 0; u < U; ++u)
+        for (int u = 0; u < U; ++u) {
+          const int k = kx + u * a.period_w, g = gx - u * dx;
+          in[u] = k < a.KW && g >= 0 && g < a.OW;
+          if (in[u]) w[u] = load_words<V>(row + ((int64_t)g * taps + k) * a.CI);
+        }
 #pragma unroll
-        for (int e = 0; e < V; ++e) sum[e] += in[u] ? __uint_as_float(w[u].w[e]) : 0.f;
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+          for (int e = 0; e < V; ++e) sum[e] += in[u] ? __uint_as_float(w[u].w[e]) : 0.f;
+      }
     }
   }
   const int64_t o = (int64_t)at_pixel * a.CI + c;
@@ -1259,17 +1273,29 @@ hipError_t col2im_launch(const Col2imArgs& args, bool bf, hipStream_t s) {
   Col2imArgs a = args;
   a.period_h = a.SH / std::gcd(a.SH, a.DH);
   a.period_w = a.SW / std::gcd(a.SW, a.DW);
+  a.step_h = a.period_h * a.DH / a.SH;
+  a.step_w = a.period_w * a.DW / a.SW;
   const int v = a.CI >= 4 ? 4 : 1;
   const int64_t blocks = ((int64_t)a.N * a.H * a.W * ((a.CI + v - 1) / v) + 255) / 256;
   if (blocks <= 0 || blocks > kMaxLaunchThreads / 256) return hipErrorInvalidValue;
+  fast_div_magic((unsigned)a.W, &a.w_magic, &a.w_shift);
+  fast_div_magic((unsigned)a.SH, &a.sh_magic, &a.sh_shift);
+  fast_div_magic((unsigned)a.SW, &a.sw_magic, &a.sw_shift);
   const dim3 grid((unsigned)blocks), block(256);
-  if (bf) {
-    if (v == 4) hipLaunchKernelGGL((col2im_kernel<true, 4>), grid, block, 0, s, a);
-    else hipLaunchKernelGGL((col2im_kernel<true, 1>), grid, block, 0, s, a);
+  const bool one = a.KH * a.KW == 1;
+#define PML_GO(BF, V)                                                                          \
+  if (one) hipLaunchKernelGGL((col2im_kernel<BF, V, true>), grid, block, 0, s, a);            \
+  else hipLaunchKernelGGL((col2im_kernel<BF, V, false>), grid, block, 0, s, a)
+  if (bf && v == 4) {
+    PML_GO(true, 4);
+  } else if (bf) {
+    PML_GO(true, 1);
+  } else if (v == 4) {
+    PML_GO(false, 4);
   } else {
-    if (v == 4) hipLaunchKernelGGL((col2im_kernel<false, 4>), grid, block, 0, s, a);
-    else hipLaunchKernelGGL((col2im_kernel<false, 1>), grid, block, 0, s, a);
+    PML_GO(false, 1);
   }
+#undef PML_GO
   return hipGetLastError();
 }
 
