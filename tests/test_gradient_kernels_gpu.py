@@ -38,6 +38,7 @@ CASES = [  # n, h, w, ci, kh, kw, co, oh, ow, stride, pad, dil
     (2, 8, 8, 3, 1, 1, 4, 4, 4, 2, 0, 1),         # pixels that no window covers, one tap
     (3, 9, 7, 13, 1, 1, 20, 3, 2, 3, 0, 1),       # ... and pixels behind the last gradient row and column
     (1, 11, 10, 5, 1, 1, 9, 6, 6, 2, 1, 1),       # ... and gradient pixels beside the image
+    (2, 21, 11, 150, 3, 3, 80, 21, 11, 1, 1, 1),  # 300 KB of results a split
     (1, 15, 1, 6, 3, 1, 8, 7, 1, 2, 0, 2),        # rows of taps apart
     (5, 40, 41, 6, 3, 3, 18, 40, 41, 1, 1, 1),    # 128 slabs and a piece: splits of two slabs
     (9, 64, 64, 17, 3, 3, 38, 64, 64, 1, 1, 1),   # splits that several threads add up
