@@ -316,7 +316,12 @@ struct Side {
       for (int r = 0; r < kRuns; ++r) straight(&regs[kWords * r], runs[r].hi > runs[r].lo ? runs[r].at : 0);
     } else {
 #pragma unroll
-      for (int r = 0; r < kRuns; ++r) gather(&regs[kWords * r], runs[r].at, runs[r].lo, runs[r].hi, apart);
+      for (int r = 0; r < kRuns; ++r) {
+        if (runs[r].lo == 0 && runs[r].hi == kVals && apart == 1)
+          straight(&regs[kWords * r], runs[r].at);
+        else
+          gather(&regs[kWords * r], runs[r].at, runs[r].lo, runs[r].hi, apart);
+      }
     }
   }
 
