@@ -195,13 +195,16 @@ bool splits_k(int64_t m, int64_t n, int64_t k_bytes, int kind) {
 // (3881 x 3959, K = 2992 723 us, 760 in tiles of 64; 2381 x 1595, K = 2608 171, 180), while half a round of them more costs as much as
 // two of 64: 3271 x 547, K = 448 36.2 -> 21.6, 2322 x 2041, K = 304 47.7 -> 35.4, 1246 x 4028, K = 208 35.6 -> 27.1, convolutions
 // 38400 x 122, K = 2304 294 -> 209, 13689 x 179, K = 3200 212 -> 168.
-bool f32_tiles_of_128(int64_t m, int64_t n) {
+// (One slab is tail more than MFMAs, and two tiles of 128 share a CU: there a last round more than half full is no whole one.
+// 7295 x 944, K = 12 13.1, in tiles of 64 14.1, 4690 x 1308, K = 28 13.1, 13.7; with a smaller share of both grids for edges alike.)
+bool f32_tiles_of_128(int64_t m, int64_t n, int64_t k_bytes) {
   const int64_t cus = device_cus(), t128 = ((m + 127) / 128) * ((n + 127) / 128), t64 = ((m + 63) / 64) * ((n + 63) / 64);
+  if (k_bytes <= 128 && t128 >= cus && 2 * (t128 % cus) >= cus && 10 * t64 >= 37 * t128) return true;
   return t128 >= 128 && 4 * ((t128 + cus - 1) / cus) <= (t64 + cus - 1) / cus;
 }
-double f32_slab_us(int64_t m, int64_t n) {
+double f32_slab_us(int64_t m, int64_t n, int64_t k_bytes) {
   const int64_t cus = device_cus(), t128 = ((m + 127) / 128) * ((n + 127) / 128), t64 = ((m + 63) / 64) * ((n + 63) / 64);
-  return f32_tiles_of_128(m, n) ? 2.2 * (double)((t128 + cus - 1) / cus) : 0.58 * (double)((t64 + cus - 1) / cus);
+  return f32_tiles_of_128(m, n, k_bytes) ? 2.2 * (double)((t128 + cus - 1) / cus) : 0.58 * (double)((t64 + cus - 1) / cus);
 }
 
 // One of the direct tiles (direct.hip) where it beats the LDS kernels, or -1.  Both sides are priced in microseconds, from
@@ -247,7 +250,7 @@ int direct_tile_of(int64_t m, int64_t n, int64_t k_bytes, int kind, int64_t kn_l
     return 2.6 + rounds * (start + (double)(std::min(m, side) + (f32 && w ? wide : std::min(n, wide))) * kb / r);
   };
   const int64_t slabs = (k_bytes + 127) / 128;
-  double lds_us = 4.2 + (f32 ? f32_slab_us(m, n) : kind == KIND_I8 ? 0.28 : 0.23) * (double)slabs;
+  double lds_us = 4.2 + (f32 ? f32_slab_us(m, n, k_bytes) : kind == KIND_I8 ? 0.28 : 0.23) * (double)slabs;
   bool needs_bt = !as_given && (kind == KIND_BF16 || n % (16 / es) != 0 || kn_ldb % 16 != 0);
   if (can_split && splits_k(m, n, k_bytes, kind)) {
     int splits = 1, per = 0;
@@ -382,7 +385,7 @@ int choose_tile(int64_t m, int64_t n, int64_t k_bytes, int kind, const TailForm&
   // convolutions with K of less than 2 KB those of up to 256 tiles took 1.05 to 1.16 x as long in plain ones (relu 1.08, residual 1.11,
   // scale and shift 1.05), those of up to 512 1.00 to 1.07 -- but for scale and shift, 0.96 to 1.03, unless rows off 16 bytes leave
   // step by step (1.3).
-  if (kind == KIND_F32 && !f32_tiles_of_128(m, n))
+  if (kind == KIND_F32 && !f32_tiles_of_128(m, n, k_bytes))
     return tiles(64, 64) <= (k_bytes < 2048 && tail.steps && n % 4 == 0 ? 256 : 512) ? TILE_64x64_W8_K2 : TILE_64x64;
   if (tiles(128, 128) >= 256) return TILE_128x128_W8_S2;
   // (two slabs and less are all launch, first loads and tail: bf16 conv 8750 x 138, K = 64 9.4 -> 6.6 us, 23958 x 105, K = 128 9.6 -> 8.1.
@@ -786,7 +789,7 @@ WinShape window_shape(Plan* p, bool named, double* window_us) {
   }
   if (p->mfma_kind == KIND_F32) {
     const double mma_us = (double)((g.M + 63) / 64 * 64) * (double)((g.N + 63) / 64 * 64) * (double)g.K * 2 / 154e6;
-    const double tiles_us = 4.2 + f32_slab_us(g.M, g.N) * (double)conv_slabs(d);
+    const double tiles_us = 4.2 + f32_slab_us(g.M, g.N, k_bytes) * (double)conv_slabs(d);
     return us < std::max(4 + 1.45 * mma_us, 0.93 * tiles_us) ? shape : WinShape{};
   }
   return shape;

@@ -91,3 +91,19 @@ def test_fp32_under_scale_and_shift(m, n, k, tail, shared):
     named = run('f32', m, n, k, tail, tile='64x64w8k2' if shared else '64x64')[0]
     np.testing.assert_array_equal(got, named)
     assert (np.abs(got - want) <= bound).all()
+
+
+def text_of(kind, m, n, k, layout=0, flags=0):
+    d = hk.GemmDesc()
+    d.in_dtype = d.out_dtype = d.c_dtype = kind
+    d.m, d.n, d.k, d.lda, d.ldb, d.ldc, d.b_layout, d.flags = m, n, k, k, k if layout else n, n, layout, flags
+    plan = hk.lib().pml_hip_gemm_dispatch(ctypes.byref(d))
+    text = hk.describe(plan)
+    hk.lib().pml_hip_plan_free(plan)
+    return text
+
+
+# one slab over 1.78 and 1.59 rounds of 128 x 128; a round less than half full; edges that cost the large tiles more; two slabs
+@pytest.mark.parametrize('m,n,k,large', [(7295, 944, 12, True), (4690, 1308, 28, True), (9911, 400, 12, False), (50809, 272, 28, False), (7295, 944, 36, False)])
+def test_fp32_of_one_slab(m, n, k, large):
+    assert ('tile=128x128 (8 wavefronts, 2 stages) ' if large else PLAIN) in text_of(hk.F32, m, n, k)
