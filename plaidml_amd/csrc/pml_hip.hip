@@ -229,9 +229,9 @@ double f32_slab_us(int64_t m, int64_t n, int64_t k_bytes) {
 // its bytes both ways at 2.2 TB/s:
 // bf16 512 x 512 x 512 9.4 -> 5.0, 1024^3 14.6 -> 10.6, 64 x 2048 x 2048 16.5 -> 8.8; fp32 128 x 4096 x 1024 23.4 -> 12.3.
 // kn_ldb: that right-hand side's row pitch in bytes (0: Bt); always: the better of the two whatever the LDS kernel takes;
-// can_split: the LDS kernel may split K; as_given: it reads a [K][N] right-hand side as it lies (256 x 49152, K = 4096 bf16:
+// can_split: the LDS kernel may split K; lds: what an LDS kernel takes; as_given: it reads a [K][N] right-hand side as it lies (256 x 49152, K = 4096 bf16:
 // 409 us direct, 135 with 256 x 256 tiles; charged the copy of 800 MB, they lost)
-int direct_tile_of(int64_t m, int64_t n, int64_t k_bytes, int kind, int64_t kn_ldb = 0, bool always = false, bool can_split = true, bool as_given = false, double* us = nullptr) {
+int direct_tile_of(int64_t m, int64_t n, int64_t k_bytes, int kind, int64_t kn_ldb = 0, bool always = false, bool can_split = true, bool as_given = false, double* us = nullptr, double* lds = nullptr) {
   if (kind != KIND_F32 && kind != KIND_BF16 && kind != KIND_I8) return -1;
   auto tiles = [&](int64_t bm, int64_t bn) { return ((m + bm - 1) / bm) * ((n + bn - 1) / bn); };
   const double kb = (double)k_bytes;
@@ -264,6 +264,7 @@ int direct_tile_of(int64_t m, int64_t n, int64_t k_bytes, int kind, int64_t kn_l
   const double small = direct_us(16), large = direct_us(32);
   const bool direct = always || std::min(small, large) <= 0.95 * lds_us;
   if (us) *us = direct ? std::min(small, large) : lds_us;
+  if (lds) *lds = lds_us;
   if (!direct) return -1;
   return small <= large ? TILE_16x16_W8 : TILE_32x32_W8;
 }
@@ -1083,6 +1084,14 @@ static DirectTiles direct_tiles(const pml_hip_gemm_desc& d, int kind, int lds_ti
   // (Two products are priced against one chain of all slabs: of 49 x 2048, K = 512 + 1024 the split takes 9.2 us and the direct
   // tile 8.8, of 196 x 256, K = 1024 + 512 9.0 and 5.8; only a K of 4096 turns that round, 10.7 and 17.0.)
   t.rows = direct_tile_of(d.m, d.n, (d.k + d.k2) * es, kind, 0, false, /*can_split=*/d.k2 == 0);
+  // (fp32 of a long K over a few columns, which gains little from rows of K and loses more over [K][N], where K is not split: 6 x 59,
+  // K = 4000 12.9 -> 13.1 and 17.3 -> 21.4; 1030 x 36, K = 2608 12.6 -> 9.7 and 16.0 -> 16.9 stays)
+  if (kind == KIND_F32 && t.rows >= 0 && splits_k(d.m, d.n, d.k * es, kind)) {
+    double rows_us = 0, lds_us = 0;
+    (void)direct_tile_of(d.m, d.n, d.k * es, kind, 0, /*always=*/true, true, false, &rows_us, &lds_us);
+    const double lies_us = std::min(direct_lies_us(d.m, d.n, d.k * es, kind, 16), direct_lies_us(d.m, d.n, d.k * es, kind, 32));
+    if (rows_us > 0.8 * lds_us && lies_us > 1.2 * (lds_us + 3.0 + 2.0 * (double)(d.k * es * d.n) / 2.2e6)) t.rows = -1;
+  }
   if (d.b_layout || d.k2 > 0 || (kind == KIND_F32 && t.rows < 0)) return t;
   t.given = direct_tile_of(d.m, d.n, d.k * es, kind, d.ldb * es, /*always=*/kind == KIND_F32, /*can_split=*/true, takes_b_as_given(d, kind, lds_tile, d.ldb));
   return t;

@@ -107,3 +107,11 @@ def text_of(kind, m, n, k, layout=0, flags=0):
 @pytest.mark.parametrize('m,n,k,large', [(7295, 944, 12, True), (4690, 1308, 28, True), (9911, 400, 12, False), (50809, 272, 28, False), (7295, 944, 36, False)])
 def test_fp32_of_one_slab(m, n, k, large):
     assert ('tile=128x128 (8 wavefronts, 2 stages) ' if large else PLAIN) in text_of(hk.F32, m, n, k)
+
+
+@pytest.mark.parametrize('layout', [0, 1])
+@pytest.mark.parametrize('m,n,k,direct', [(6, 59, 4000, False), (1030, 36, 2608, True), (2, 37, 3500, True), (6, 59, 1200, True)])
+def test_fp32_of_a_long_k_and_few_columns(m, n, k, direct, layout):
+    """Split in both layouts where a direct tile loses more over [K][N] than it gains over rows of K."""
+    text = text_of(hk.F32, m, n, k, layout)
+    assert ('with rows of K at hand' in text) == direct and ('with B as it lies' in text) == (direct and not layout), text
