@@ -302,7 +302,8 @@ bool fp32_beats_split(int64_t m, int64_t n, int64_t k_bytes) {
     }
   }
   if (direct_tile_of(m, n, k_bytes, KIND_F32) < 0) return false;
-  (void)direct_tile_of(m, n, k_bytes, KIND_F32, 0, /*always=*/true, true, false, &us);
+  // (two rounds of 16 x 16 tiles over few K take longer than that price: 29 x 3872, K = 96 [N][K] 5.2, direct 6.0)
+  if (direct_tile_of(m, n, k_bytes, KIND_F32, 0, /*always=*/true, true, false, &us) == TILE_16x16_W8 && ((m + 15) / 16) * ((n + 15) / 16) > device_cus()) us += 0.7;
   const double copy = needs_bt ? 3.0 + 2.0 * (double)k_bytes * (double)n / 2.2e6 : 0;
   return us <= 0.95 * split_us && std::min(direct_lies_us(m, n, k_bytes, KIND_F32, 16), direct_lies_us(m, n, k_bytes, KIND_F32, 32)) <= 0.95 * (split_us + copy);
 }

@@ -115,3 +115,9 @@ def test_fp32_of_a_long_k_and_few_columns(m, n, k, direct, layout):
     """Split in both layouts where a direct tile loses more over [K][N] than it gains over rows of K."""
     text = text_of(hk.F32, m, n, k, layout)
     assert ('with rows of K at hand' in text) == direct and ('with B as it lies' in text) == (direct and not layout), text
+
+
+@pytest.mark.parametrize('layout', [0, 1])
+@pytest.mark.parametrize('m,n,k,split', [(29, 3872, 96, True), (34, 2320, 96, True), (40, 1800, 200, False), (16, 3872, 96, False)])
+def test_split_fp32_of_two_rounds(m, n, k, split, layout):
+    assert ('3 x f32' in text_of(hk.F32, m, n, k, layout, hk.FP32_AS_BF16X3)) == split
