@@ -121,3 +121,16 @@ def test_fp32_of_a_long_k_and_few_columns(m, n, k, direct, layout):
 @pytest.mark.parametrize('m,n,k,split', [(29, 3872, 96, True), (34, 2320, 96, True), (40, 1800, 200, False), (16, 3872, 96, False)])
 def test_split_fp32_of_two_rounds(m, n, k, split, layout):
     assert ('3 x f32' in text_of(hk.F32, m, n, k, layout, hk.FP32_AS_BF16X3)) == split
+
+
+# 7 x 7 taps of 40 channels, 4 KB of K; the same in int8 and of fewer channels
+@pytest.mark.parametrize('kind,out,ci,lies', [(hk.BF16, hk.BF16, 40, False), (hk.I8, hk.I32, 32, True), (hk.BF16, hk.BF16, 16, True)])
+def test_filters_of_a_long_k_that_come_with_the_call(kind, out, ci, lies):
+    d = hk.Conv2dDesc()
+    d.in_dtype, d.out_dtype, d.c_dtype = kind, out, out
+    d.n, d.h, d.w, d.ci, d.kh, d.kw, d.co, d.oh, d.ow = 1, 74, 18, ci, 7, 7, 16, 74, 18
+    d.stride_h = d.stride_w = d.dil_h = d.dil_w = 1
+    d.pad_h = d.pad_w = 3
+    plan = hk.lib().pml_hip_conv2d_dispatch(ctypes.byref(d))
+    assert ('with the filter as it lies' in hk.describe(plan)) == lies, hk.describe(plan)
+    hk.lib().pml_hip_plan_free(plan)
