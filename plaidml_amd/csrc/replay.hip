@@ -13,7 +13,7 @@
 
 #include <algorithm>
 #include <memory>
-#include <vector>
+#include <new>
 
 #include "plans.h"
 
@@ -23,39 +23,40 @@ namespace {
 
 constexpr size_t kFewLaunches = 5;  // one by one up to here
 
-// The kernels of a short recording that is one chain of nothing else, in their order (the arguments stay the recording's own).
-bool kernel_chain(hipGraph_t g, std::vector<hipKernelNodeParams>* chain) {
+// The kernels of a short recording that is one chain of nothing else, in their order (the arguments stay the recording's own);
+// their number, or 0.
+size_t kernel_chain(hipGraph_t g, hipKernelNodeParams (&chain)[kFewLaunches]) {
   size_t n = 0, edges = 0;
-  if (hipGraphGetNodes(g, nullptr, &n) != hipSuccess || n == 0 || n > kFewLaunches) return false;
-  if (hipGraphGetEdges(g, nullptr, nullptr, &edges) != hipSuccess || edges != n - 1) return false;
-  std::vector<hipGraphNode_t> nodes(n), from(edges), to(edges);
-  if (hipGraphGetNodes(g, nodes.data(), &n) != hipSuccess) return false;
-  if (edges > 0 && hipGraphGetEdges(g, from.data(), to.data(), &edges) != hipSuccess) return false;
-  hipGraphNode_t at = nullptr;
-  for (hipGraphNode_t node : nodes)
-    if (std::count(to.begin(), to.end(), node) == 0) {
-      if (at) return false;
-      at = node;
+  if (hipGraphGetNodes(g, nullptr, &n) != hipSuccess || n == 0 || n > kFewLaunches) return 0;
+  if (hipGraphGetEdges(g, nullptr, nullptr, &edges) != hipSuccess || edges != n - 1) return 0;
+  hipGraphNode_t nodes[kFewLaunches], from[kFewLaunches], to[kFewLaunches], at = nullptr;
+  if (hipGraphGetNodes(g, nodes, &n) != hipSuccess) return 0;
+  if (edges > 0 && hipGraphGetEdges(g, from, to, &edges) != hipSuccess) return 0;
+  for (size_t i = 0; i < n; ++i)
+    if (std::count(to, to + edges, nodes[i]) == 0) {
+      if (at) return 0;
+      at = nodes[i];
     }
+  size_t count = 0;
   while (at) {
     hipGraphNodeType type;
     hipKernelNodeParams p = {};
-    if (hipGraphNodeGetType(at, &type) != hipSuccess || type != hipGraphNodeTypeKernel) return false;
-    if (hipGraphKernelNodeGetParams(at, &p) != hipSuccess || !p.func || !p.kernelParams || p.extra) return false;
-    chain->push_back(p);
-    if (chain->size() > n) return false;
-    const auto edge = std::find(from.begin(), from.end(), at);
-    if (edge != from.end() && std::find(edge + 1, from.end(), at) != from.end()) return false;
-    at = edge == from.end() ? nullptr : to[edge - from.begin()];
+    if (count == n || hipGraphNodeGetType(at, &type) != hipSuccess || type != hipGraphNodeTypeKernel) return 0;
+    if (hipGraphKernelNodeGetParams(at, &p) != hipSuccess || !p.func || !p.kernelParams || p.extra) return 0;
+    chain[count++] = p;
+    if (std::count(from, from + edges, at) > 1) return 0;
+    const size_t edge = (size_t)(std::find(from, from + edges, at) - from);
+    at = edge == edges ? nullptr : to[edge];
   }
-  return chain->size() == n;
+  return count == n ? count : 0;
 }
 
 }  // namespace
 
 struct Replay {
   hipGraph_t recorded = nullptr;              // of launches that go out one by one
-  std::vector<hipKernelNodeParams> launches;  // one by one (their arguments are `recorded`'s); empty: as a graph
+  hipKernelNodeParams launches[kFewLaunches];  // (their arguments are `recorded`'s)
+  size_t n = 0;                               // 0: as a graph
   hipGraphExec_t exec = nullptr;
   ~Replay() {
     if (exec) (void)hipGraphExecDestroy(exec);
@@ -63,14 +64,17 @@ struct Replay {
   }
 };
 
+// (called by entry points of a C library: nothing here throws)
 hipError_t replay_create(hipGraph_t recorded, Replay** out) {
-  std::unique_ptr<Replay> r(new Replay);
-  r->recorded = recorded;
-  if (!kernel_chain(recorded, &r->launches)) {
-    (void)hipGetLastError();
-    r->launches.clear();
+  std::unique_ptr<Replay> r(new (std::nothrow) Replay);
+  if (!r) {
+    (void)hipGraphDestroy(recorded);
+    return hipErrorOutOfMemory;
   }
-  if (r->launches.empty()) {
+  r->recorded = recorded;
+  r->n = kernel_chain(recorded, r->launches);
+  if (r->n == 0) {
+    (void)hipGetLastError();
     if (hipError_t e = hipGraphInstantiate(&r->exec, recorded, nullptr, nullptr, 0); e != hipSuccess) return e;
     (void)hipGraphDestroy(recorded);
     r->recorded = nullptr;
@@ -80,8 +84,10 @@ hipError_t replay_create(hipGraph_t recorded, Replay** out) {
 }
 
 hipError_t replay_launch(const Replay& r, hipStream_t s) {
-  for (const hipKernelNodeParams& p : r.launches)
+  for (size_t i = 0; i < r.n; ++i) {
+    const hipKernelNodeParams& p = r.launches[i];
     if (hipError_t e = hipLaunchKernel(p.func, p.gridDim, p.blockDim, p.kernelParams, p.sharedMemBytes, s); e != hipSuccess) return e;
+  }
   return r.exec ? hipGraphLaunch(r.exec, s) : hipSuccess;
 }
 
