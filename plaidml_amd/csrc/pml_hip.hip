@@ -151,6 +151,7 @@ int mfma_kind_of(int in_dtype, int flags = 0) {
   return -1;
 }
 
+const char* const kFilterLies = ", with the filter as it lies tile=";
 const char* tile_name(int t) {
   switch (t) {
     case TILE_64x64: return "64x64";
@@ -1646,7 +1647,7 @@ int64_t pml_hip_conv2d_dispatch(const pml_hip_conv2d_desc* d) {
   p->text = buf;
   if (kind == KIND_F32X3) p->text += " mfma=3 x f32_32x32x16_bf16 (fp32 split into bf16 head + remainder)";
   if (p->tile_direct >= 0 && !p->halo_lds) p->text += std::string(", direct tile=") + tile_name(p->tile_direct);
-  if (p->tile_given >= 0) p->text += std::string(", with the filter as it lies tile=") + (p->tile_given == TILE_16x16_W8 ? "16x64" : "32x64") + " (8 wavefronts sharing K)";
+  if (p->tile_given >= 0) p->text += std::string(kFilterLies) + (p->tile_given == TILE_16x16_W8 ? "16x64" : "32x64") + " (8 wavefronts sharing K)";
   if (via_patches) p->text += " via patch matrix (k padded to " + std::to_string(p->kpad) + ")";
   if (!p->halo_lds && p->win.config < 0 && !via_s2d) {
     IgemmArgs g;
@@ -2214,11 +2215,13 @@ int64_t pml_hip_conv2d_grad_dispatch(const pml_hip_conv2d_desc* d, int which) {
       return 0;
     }
     p->sub->packed = true;  // (every invoke lays the filter out itself)
+    p->sub->tile_given = -1;
     if (p->co_pad != d->co && !(p->padded = p->hold((size_t)(d->n * d->oh * d->ow * p->co_pad * es)))) {
       delete p;
       fail("conv2d_grad: cannot allocate the padded gradient");
       return 0;
     }
+    if (const size_t at = p->sub->text.find(kFilterLies); at != std::string::npos) p->sub->text.erase(at, p->sub->text.find(')', at) + 1 - at);
     p->text = "conv2d data gradient as a convolution of the gradient: " + p->sub->text;
     return (int64_t)(intptr_t)p;
   }

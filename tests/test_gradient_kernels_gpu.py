@@ -71,6 +71,7 @@ def test_gradients(case, dtype):
         text = hk.describe(ctypes.c_int64(p))
         if which == 0:
             assert ('as a convolution of the gradient' if stride == 1 else 'by columns') in text, text
+            assert 'as it lies' not in text, text  # (the flipped filter is laid out by every call)
         else:  # (pixels over one workgroup, over splits of two slabs, over more than a thread adds up)
             splits = int(text.split('splits=')[1].split()[0])
             assert splits >= (9 if n * oh * ow > 30000 else 2 if n * oh * ow > 1000 else 1), text
