@@ -556,7 +556,7 @@ def main():
             result['resnet50_b128_img_per_s'] = extra['resnet50_v1_5_b128_bf16']['img_per_s']
         if want('resnet50_b1'):
             # the same network on one image: latency (few tiles per layer: the K loops of the long-K layers are split
-            # over workgroups, the launches replayed as one graph)
+            # over workgroups, the launches replayed from a recording)
             extra['resnet50_v1_5_b1_bf16'] = resnet50_leg(batch=1, runs=20)
         result['extra'] = extra
 

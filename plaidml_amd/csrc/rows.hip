@@ -369,7 +369,8 @@ size_t rows_program_lds(const pml_hip_rows_desc& d, int* lanes) {
   // A wavefront per row needs no barrier between steps, which is what a row costs most of (4096 x 1000: 35 us with a
   // workgroup per row): for short rows, and for rows of up to 2048 when there are enough of them to fill the chip that way
   // and four of them fit the LDS (from five vectors of 2048 columns on they do not).  Fewer rows of more than 256 have a workgroup
-  // each (40 x 300 fp32 11.8 -> 9.0 us).
+  // each: 1 to 1023 rows of 257 to 512 columns, 80 sizes in fp32 and 80 in bf16, 1.08 and 1.13 x as fast in the mean (40 x 300 fp32 12.5 -> 10.0 us
+  // of a whole program, 512 x 384 12.1 -> 10.8, 850 x 384 12.3 -> 11.8; bf16 14.0 -> 11.1, 15.0 -> 13.0, 14.1 -> 13.4); towards 1024 rows both meet (1000 x 512 fp32 11.8, 12.2).
   const size_t pitch = (size_t)(d.cols + 3) / 4 * 4;
   auto bytes = [&](size_t groups) { return (groups * PML_HIP_ROWS_SCALARS + 4 + groups * (size_t)d.n_vectors * pitch) * 4; };
   *lanes = d.cols <= 256 || (d.cols <= 512 && d.rows >= 1024) || (d.cols <= 2048 && d.rows >= 1024 && bytes(4) <= kRowsLds) ? 64 : 256;

@@ -268,12 +268,13 @@ struct Side {
     for (int e = 0; e < kWords; ++e) to[e] = v.w[e];
   }
 
-  // Where nothing is cut and rows are contiguous the loads go out as they are.  FLAT (filter gradients, where a slab's pixels
-  // always have cut window rows among them): elsewhere as well, and put() clears what does not belong to the operand.  With a
-  // branch per run, and per value where a run is cut, the loads of a slab waited for each other (567 pixels of 3 x 45 window
-  // values x 20, bf16: 19.6 -> 12.4 us, 154154 of 3 x 51 x 38: 58.6 -> 35.6).  Only where a run sticks out of the operand's
-  // `extent` elements is it read value by value then.  Two slabs on their way instead of one take 219 registers and 46.6 us.  (It takes 30 registers more, which products have no
-  // use for.)
+  // Where nothing is cut and rows are contiguous the loads go out as they are; elsewhere run by run, or value by value where a run is
+  // cut.  FLAT (filter gradients, where a slab's pixels always have cut window rows among them; it takes 30 registers more, which
+  // products have no use for): the loads go out whole there, too, and put() clears what does not belong to the operand -- but for a slab
+  // with a run that sticks out of the operand's `extent` elements.  With a branch per run, and per value, the loads of a slab waited
+  // for each other: 567 pixels of 3 x 45 window values x 20, bf16 19.6 -> 12.4 us, 154154 of 3 x 51 x 38 58.6 -> 35.6.  (Tried: two slabs on their
+  // way instead of one, 219 registers and 46.6 us.  What it costs: 28 pixels and fewer, one slab that ends the tensor, 0.2 to 0.5 us of 5 to
+  // 6; windows of 140 channels and more in bf16, few of whose runs are cut, 4 to 6 %, 2968 pixels of 5 x 870 x 84 35.6, 37.9.)
   __device__ __forceinline__ void fetch(const StridedArgs& p, int64_t k0, int64_t k_end, int tid) {
     Pixel pix{0, 0, 0};
     if constexpr (MODE == ROWS_CONV) {
