@@ -135,14 +135,29 @@ __global__ __launch_bounds__(64 * WM * WN * KS, NB >= 4 ? 2 : 4) void winconv_ke
   // that blocks of few results do not cover.  With a branch per tap and products for both offsets, before -> now: int8 33 x 29 x 29 x
   // 256 (*) 7 x 7 x 26 40.0 -> 30.5 us, bf16 14 x 14 x 14 x 32 (*) 7 x 7 x 178 11.7 -> 9.3, 8 x 37 x 37 x 128 (*) 7 x 7 x 115 36.5 -> 32.5,
   // 8 x 28 x 28 x 128 (*) 3 x 3 x 128 8.4 -> 8.0, 3 x 14 x 14 x 256 (*) 3 x 3 x 256 8.6 -> 8.3; 65 drawn ones 1.03 x.
+  // fp32, whose MFMAs are four times as long a step, is past that chain: it takes both offsets where they are used, the filter's
+  // between two MFMAs.  Counted on: 24 x 41 x 41 x 128 (*) 3 x 3 x 15 46.9 -> 48.0, now 46.5; 11 x 41 x 41 x 32 (*) 5 x 5 x 200 60.5 -> 62.5,
+  // now 60.3; 24 drawn ones 0.98 x, now 1.00.
   struct Step {
     int slab, ky, kx, blk;
     int off, b;  // bytes from the window's begin; from the begin of the filter's columns
   };
+  constexpr bool kCounts = KIND != KIND_F32;
   // of a slab: its blocks; what a tap to the right, and the first tap of the next row, add to what KS blocks do
   int nb = 0, tap_off = 0, tap_b = 0, far_x = 0, far_blk = 0, far_off = 0, far_b = 0;
   bool far = false;
   const int row_off = p.row_step - p.KW * p.tap_step;
+  auto off_of = [&](const Step& s) { return s.ky * p.row_step + s.kx * p.tap_step + s.blk * kBlockBytes; };
+  auto b_of = [&](const Step& s) { return ((s.ky * p.KW + s.kx) * p.total_blocks + s.slab * p.blocks + s.blk) * 2048; };
+  auto settle = [&](Step& s) {  // carries blk into kx and ky
+    while (s.blk >= nb) {
+      s.blk -= nb;
+      if (++s.kx == p.KW) {
+        s.kx = 0;
+        ++s.ky;
+      }
+    }
+  };
   auto begin = [&](int slab) {
     nb = slab == p.slabs - 1 ? p.last_blocks : p.blocks;
     tap_off = p.tap_step - nb * kBlockBytes;
@@ -154,19 +169,15 @@ __global__ __launch_bounds__(64 * WM * WN * KS, NB >= 4 ? 2 : 4) void winconv_ke
     far_off = far_x * p.tap_step + far_blk * kBlockBytes;
     far_b = KS * 2048 + far_x * tap_b;
     Step s{slab, 0, 0, kg, 0, 0};
-    while (s.blk >= nb) {
-      s.blk -= nb;
-      if (++s.kx == p.KW) {
-        s.kx = 0;
-        ++s.ky;
-      }
-    }
-    s.off = s.ky * p.row_step + s.kx * p.tap_step + s.blk * kBlockBytes;
-    s.b = ((s.ky * p.KW + s.kx) * p.total_blocks + slab * p.blocks + s.blk) * 2048;
+    settle(s);
+    if constexpr (kCounts) s.off = off_of(s), s.b = b_of(s);
     return s;
   };
   auto count_on = [&](Step& s) {  // whether there is another step in the slab
-    if (far) {
+    if constexpr (!kCounts) {
+      s.blk += KS;
+      settle(s);
+    } else if (far) {
       s.blk += far_blk;
       const bool over = s.blk >= nb;
       s.blk -= over ? nb : 0;
@@ -195,7 +206,7 @@ __global__ __launch_bounds__(64 * WM * WN * KS, NB >= 4 ? 2 : 4) void winconv_ke
     }
     return s.ky < p.KH;
   };
-  auto lds_at = [&](const Step& s) { return (s.slab & 1) * p.win_bytes + s.off; };
+  auto lds_at = [&](const Step& s) { return (s.slab & 1) * p.win_bytes + (kCounts ? s.off : off_of(s)); };
 
   // filter fragments as winconv_pack_kernel lays them out: a step's 32 columns are 2 KB
   const int group_bytes = p.KH * p.KW * p.total_blocks * 2048;
@@ -204,9 +215,10 @@ __global__ __launch_bounds__(64 * WM * WN * KS, NB >= 4 ? 2 : 4) void winconv_ke
   for (int j = 0; j < NB / 2; ++j) b_group[j] = min(n0 / 32 + j, (p.N - 1) / 32) * group_bytes;
   i32x4_t fa[MB], fb[2][NB];
   auto request_b = [&](i32x4_t (&f)[NB], const Step& s) {
+    const int at = kCounts ? s.b : b_of(s);
 #pragma unroll
     for (int j = 0; j < NB; ++j)
-      f[j] = __builtin_bit_cast(i32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rb, lane * 16 + (j & 1) * 1024, b_group[j >> 1] + s.b, 0));
+      f[j] = __builtin_bit_cast(i32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rb, lane * 16 + (j & 1) * 1024, b_group[j >> 1] + at, 0));
   };
 
   unsigned a_lane[MB];
