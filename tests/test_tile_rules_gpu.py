@@ -134,3 +134,18 @@ def test_filters_of_a_long_k_that_come_with_the_call(kind, out, ci, lies):
     plan = hk.lib().pml_hip_conv2d_dispatch(ctypes.byref(d))
     assert ('with the filter as it lies' in hk.describe(plan)) == lies, hk.describe(plan)
     hk.lib().pml_hip_plan_free(plan)
+
+
+# int8 of 3 KB of K: ten rows of tiles of 32, and fewer channels
+@pytest.mark.parametrize('kind,out,n,h,ci,k,stride,co,text', [(hk.I8, hk.I32, 4, 20, 64, 7, 2, 12, None), (hk.I8, hk.I32, 4, 20, 16, 3, 2, 12, 'with the filter as it lies')])
+def test_convolutions_beside_their_direct_tiles(kind, out, n, h, ci, k, stride, co, text):
+    d = hk.Conv2dDesc()
+    d.in_dtype, d.out_dtype, d.c_dtype = kind, out, out
+    d.n, d.h, d.w, d.ci, d.kh, d.kw, d.co, d.oh, d.ow = n, h, h, ci, k, k, co, -(-h // stride), -(-h // stride)
+    d.stride_h = d.stride_w = stride
+    d.dil_h = d.dil_w = 1
+    d.pad_h = d.pad_w = k // 2
+    plan = hk.lib().pml_hip_conv2d_dispatch(ctypes.byref(d))
+    got = hk.describe(plan)
+    hk.lib().pml_hip_plan_free(plan)
+    assert text in got if text else 'with the filter as it lies' not in got, got
