@@ -246,7 +246,8 @@ int direct_tile_of(int64_t m, int64_t n, int64_t k_bytes, int kind, int64_t kn_l
     const int64_t wide = kn || w ? 64 : side;
     double rounds = std::max(1.0, (double)tiles(side, wide) / n_cus);
     if ((f32 && !kn) || w) rounds = std::ceil(rounds);
-    const double start = w ? (f32 ? 2.3 : kind == KIND_I8 ? 1.0 : 1.6) : f32 && !kn && side == 32 ? 1.9 : 0.8;
+    // (fp32 in many rounds of 16 x 16: convolution 32368 x 11, K = 1152, eight of them, 42.4)
+    const double start = w ? (f32 ? 2.3 : kind == KIND_I8 ? 1.0 : 1.6) : f32 && !kn ? (side == 32 ? 1.9 : rounds > 4 ? 1.7 : 0.8) : 0.8;
     const double r = w ? (f32 ? (rounds > 1 ? 42e3 : 35e3) : kind == KIND_I8 ? 60e3 : 50e3) : rate;
     return 2.6 + rounds * (start + (double)(std::min(m, side) + (f32 && w ? wide : std::min(n, wide))) * kb / r);
   };
