@@ -1091,12 +1091,13 @@ static DirectTiles direct_tiles(const pml_hip_gemm_desc& d, int kind, int lds_ti
   // tile 8.8, of 196 x 256, K = 1024 + 512 9.0 and 5.8; only a K of 4096 turns that round, 10.7 and 17.0.)
   t.rows = direct_tile_of(d.m, d.n, (d.k + d.k2) * es, kind, 0, false, /*can_split=*/d.k2 == 0);
   // (fp32 of a long K over a few columns, which gains little from rows of K and loses more over [K][N], where K is not split: 6 x 59,
-  // K = 4000 12.9 -> 13.1 and 17.3 -> 21.4; 1030 x 36, K = 2608 12.6 -> 9.7 and 16.0 -> 16.9 stays)
+  // K = 4000 12.9 -> 13.1 and 17.3 -> 21.4, 120 x 71, K = 2688 17.5 -> 18.2 from [K][N]; 1030 x 36, K = 2608 12.6 -> 9.7 and 16.0 -> 16.9 stays)
   if (kind == KIND_F32 && t.rows >= 0 && splits_k(d.m, d.n, d.k * es, kind)) {
     double rows_us = 0, lds_us = 0;
     (void)direct_tile_of(d.m, d.n, d.k * es, kind, 0, /*always=*/true, true, false, &rows_us, &lds_us);
     const double lies_us = std::min(direct_lies_us(d.m, d.n, d.k * es, kind, 16), direct_lies_us(d.m, d.n, d.k * es, kind, 32));
-    if (rows_us > 0.8 * lds_us && lies_us > 1.2 * (lds_us + 3.0 + 2.0 * (double)(d.k * es * d.n) / 2.2e6)) t.rows = -1;
+    const double split_us = lds_us + 3.0 + 2.0 * (double)(d.k * es * d.n) / 2.2e6;
+    if ((rows_us > 0.8 * lds_us && lies_us > 1.2 * split_us) || (rows_us > 0.9 * lds_us && lies_us > split_us)) t.rows = -1;
   }
   if (d.b_layout || d.k2 > 0 || (kind == KIND_F32 && t.rows < 0)) return t;
   t.given = direct_tile_of(d.m, d.n, d.k * es, kind, d.ldb * es, /*always=*/kind == KIND_F32, /*can_split=*/true, takes_b_as_given(d, kind, lds_tile, d.ldb));

@@ -110,7 +110,7 @@ def test_fp32_of_one_slab(m, n, k, large):
 
 
 @pytest.mark.parametrize('layout', [0, 1])
-@pytest.mark.parametrize('m,n,k,direct', [(6, 59, 4000, False), (1030, 36, 2608, True), (2, 37, 3500, True), (6, 59, 1200, True)])
+@pytest.mark.parametrize('m,n,k,direct', [(6, 59, 4000, False), (120, 71, 2688, False), (1030, 36, 2608, True), (2, 37, 3500, True), (6, 59, 1200, True)])
 def test_fp32_of_a_long_k_and_few_columns(m, n, k, direct, layout):
     """Split in both layouts where a direct tile loses more over [K][N] than it gains over rows of K."""
     text = text_of(hk.F32, m, n, k, layout)
