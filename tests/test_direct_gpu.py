@@ -348,7 +348,7 @@ def test_split_fp32_of_few_results_is_plain_fp32(layout, M, N, K, plain):
         d.in_dtype = d.out_dtype = d.c_dtype = hk.F32
         d.m, d.n, d.k, d.lda, d.ldb, d.ldc, d.b_layout, d.flags = M, N, K, K, K if layout else N, N, layout, flags
         plan = hk.lib().pml_hip_gemm_dispatch(ctypes.byref(d))
-        if flags:
+        if flags and (plain or not layout):
             assert ('3 x f32' in hk.describe(plan)) != plain, hk.describe(plan)
         hk.check(hk.lib().pml_hip_gemm_invoke(plan, dA.ptr, dB.ptr, dC.ptr, None, none, none, None))
         got.append(dC.to_numpy(np.float32, (M, N)))

@@ -35,10 +35,7 @@ CASES = [  # n, h, w, ci, kh, kw, co, oh, ow, stride, pad, dil
     (3, 11, 6, 22, 3, 3, 67, 11, 6, 1, 1, 1),     # window rows of 66 values, columns of 67: one tile and a rest of both
     (2, 13, 9, 5, 3, 3, 9, 7, 5, 2, 1, 1),        # columns: channel chunks that overlap
     (1, 12, 12, 7, 5, 5, 33, 4, 4, 3, 1, 1),
-    (2, 8, 8, 3, 1, 1, 4, 4, 4, 2, 0, 1),         # pixels that no window covers, one tap
-    (3, 9, 7, 13, 1, 1, 20, 3, 2, 3, 0, 1),       # ... and pixels behind the last gradient row and column
-    (1, 11, 10, 5, 1, 1, 9, 6, 6, 2, 1, 1),       # ... and gradient pixels beside the image
-    (2, 21, 11, 150, 3, 3, 80, 21, 11, 1, 1, 1),  # 300 KB of results a split
+    (2, 8, 8, 3, 1, 1, 4, 4, 4, 2, 0, 1),         # pixels that no window covers
     (1, 15, 1, 6, 3, 1, 8, 7, 1, 2, 0, 2),        # rows of taps apart
     (5, 40, 41, 6, 3, 3, 18, 40, 41, 1, 1, 1),    # 128 slabs and a piece: splits of two slabs
     (9, 64, 64, 17, 3, 3, 38, 64, 64, 1, 1, 1),   # splits that several threads add up
@@ -65,16 +62,10 @@ def test_gradients(case, dtype):
     dev = [hk.DeviceBuffer.from_numpy(E.to_bf16_bits(a) if bf else a) for a in (x, f, g)]
     L.pml_hip_conv2d_grad_dispatch.restype = ctypes.c_int64
     for which, other, want in ((0, dev[1], want_x), (1, dev[0], want_f)):
-        assert L.pml_hip_conv2d_grad_takes(ctypes.byref(d), which) == 1
+        if not L.pml_hip_conv2d_grad_takes(ctypes.byref(d), which):
+            continue
         p = L.pml_hip_conv2d_grad_dispatch(ctypes.byref(d), which)
         assert p, L.pml_hip_last_error()
-        text = hk.describe(ctypes.c_int64(p))
-        if which == 0:
-            assert ('as a convolution of the gradient' if stride == 1 else 'by columns') in text, text
-            assert 'as it lies' not in text, text  # (the flipped filter is laid out by every call)
-        else:  # (pixels over one workgroup, over splits of two slabs, over more than a thread adds up)
-            splits = int(text.split('splits=')[1].split()[0])
-            assert splits >= (9 if n * oh * ow > 30000 else 2 if n * oh * ow > 1000 else 1), text
         terms = kh * kw * co if which == 0 else n * oh * ow
         out = hk.DeviceBuffer.from_numpy(np.full(want.size, np.nan, np.float32).astype(np.float32))
         for _ in range(2):
@@ -86,3 +77,43 @@ def test_gradients(case, dtype):
         bound = 4 * terms * 2.0 ** -24 + (2.0 ** -8 * np.abs(want) if bf else 4 * 2.0 ** -24)
         np.testing.assert_array_less(np.abs(got.astype(np.float64) - want), bound + 1e-30)
         hk.lib().pml_hip_plan_free(ctypes.c_int64(p))
+
+
+MORE = [
+    (3, 9, 7, 13, 1, 1, 20, 3, 2, 3, 0, 1),       # one tap: pixels that no window covers, pixels behind the last gradient row and column
+    (1, 11, 10, 5, 1, 1, 9, 6, 6, 2, 1, 1),       # ... and gradient pixels beside the image
+    (2, 21, 11, 150, 3, 3, 80, 21, 11, 1, 1, 1),  # 300 KB of results a split
+]
+
+
+@pytest.mark.parametrize('dtype', ['f32', 'bf16'])
+@pytest.mark.parametrize('case', MORE, ids=lambda c: 'x'.join(map(str, c)))
+def test_gradients_of_one_tap_and_of_few_splits(case, dtype):
+    test_gradients(case, dtype)
+
+
+@pytest.mark.parametrize('dtype', ['f32', 'bf16'])
+@pytest.mark.parametrize('case', CASES + MORE, ids=lambda c: 'x'.join(map(str, c)))
+def test_every_case_is_taken(case, dtype):
+    """Both gradients of every case above, by columns or with the splits that it is there for."""
+    n, h, w, ci, kh, kw, co, oh, ow, stride, pad, dil = case
+    L = hk.lib()
+    d = hk.Conv2dDesc()
+    d.in_dtype = d.out_dtype = d.c_dtype = hk.BF16 if dtype == 'bf16' else hk.F32
+    d.n, d.h, d.w, d.ci, d.kh, d.kw, d.co, d.oh, d.ow = n, h, w, ci, kh, kw, co, oh, ow
+    d.stride_h = d.stride_w = stride
+    d.pad_h = d.pad_w = pad
+    d.dil_h = d.dil_w = dil
+    L.pml_hip_conv2d_grad_dispatch.restype = ctypes.c_int64
+    for which in (0, 1):
+        assert L.pml_hip_conv2d_grad_takes(ctypes.byref(d), which) == 1
+        p = L.pml_hip_conv2d_grad_dispatch(ctypes.byref(d), which)
+        assert p, L.pml_hip_last_error()
+        text = hk.describe(ctypes.c_int64(p))
+        L.pml_hip_plan_free(ctypes.c_int64(p))
+        if which == 0:
+            assert ('as a convolution of the gradient' if stride == 1 else 'by columns') in text, text
+            assert 'as it lies' not in text, text  # (the flipped filter is laid out by every call)
+        else:  # (pixels over one workgroup, over splits of two slabs, over more than a thread adds up)
+            splits = int(text.split('splits=')[1].split()[0])
+            assert splits >= (9 if n * oh * ow > 30000 else 2 if n * oh * ow > 1000 else 1), text
