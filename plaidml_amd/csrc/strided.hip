@@ -1128,8 +1128,9 @@ __global__ __launch_bounds__(256) void col2im_kernel(Col2imArgs a) {
 #pragma unroll
   for (int e = 0; e < V; ++e) sum[e] = 0.f;
   if constexpr (ONE) {
-    const int gy = (int)fast_div((unsigned)(y + a.PH), a.sh_magic, a.sh_shift), gx = (int)fast_div((unsigned)(x + a.PW), a.sw_magic, a.sw_shift);
-    if (gy * a.SH == y + a.PH && gx * a.SW == x + a.PW && gy < a.OH && gx < a.OW) {
+    const int ty = y + a.PH, tx = x + a.PW;  // (a crop, which is a negative padding, leaves pixels ahead of the first window)
+    const int gy = (int)fast_div((unsigned)ty, a.sh_magic, a.sh_shift), gx = (int)fast_div((unsigned)tx, a.sw_magic, a.sw_shift);
+    if (ty >= 0 && tx >= 0 && gy * a.SH == ty && gx * a.SW == tx && gy < a.OH && gx < a.OW) {
       const Words<V> w = load_words<V>(a.cols + (((int64_t)img * a.OH + gy) * a.OW + gx) * a.CI + c);
 #pragma unroll
       for (int e = 0; e < V; ++e) sum[e] += __uint_as_float(w.w[e]);

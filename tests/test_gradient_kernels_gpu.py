@@ -117,3 +117,40 @@ def test_every_case_is_taken(case, dtype):
         else:  # (pixels over one workgroup, over splits of two slabs, over more than a thread adds up)
             splits = int(text.split('splits=')[1].split()[0])
             assert splits >= (9 if n * oh * ow > 30000 else 2 if n * oh * ow > 1000 else 1), text
+
+
+# one tap, where the stride is one in one direction; several
+@pytest.mark.parametrize('dtype', ['f32', 'bf16'])
+@pytest.mark.parametrize('stride,k', [((1, 2), 1), ((2, 1), 1), ((3, 2), 1), ((1, 2), 2), ((1, 1), 1)])
+def test_gradients_of_a_cropped_image(stride, k, dtype):
+    """A negative padding crops: pixels ahead of the first window take no gradient, and no filter gradient takes them."""
+    n, h, w, ci, co, crop = 2, 9, 12, 6, 5, (2, 1)
+    oh, ow = (h - crop[0] - k) // stride[0], (w - crop[1] - k) // stride[1]
+    print(stride, k, dtype, flush=True)
+    hk.init(0)
+    L, rng, bf = hk.lib(), np.random.default_rng(k), dtype == 'bf16'
+    x, f, g = (E.round_bf16(rng.standard_normal(s).astype(np.float32)) for s in ((n, h, w, ci), (k, k, ci, co), (n, oh, ow, co)))
+    want_x, want_f = np.zeros((n, h, w, ci)), np.zeros((k, k, ci, co))
+    for ky in range(k):
+        for kx in range(k):
+            at = (slice(None), slice(crop[0] + ky, crop[0] + ky + oh * stride[0], stride[0]), slice(crop[1] + kx, crop[1] + kx + ow * stride[1], stride[1]))
+            want_x[at] += g.astype(np.float64) @ f[ky, kx].T
+            want_f[ky, kx] = np.tensordot(x[at].astype(np.float64), g, ((0, 1, 2), (0, 1, 2)))
+    d = hk.Conv2dDesc()
+    d.in_dtype = d.out_dtype = d.c_dtype = hk.BF16 if bf else hk.F32
+    d.n, d.h, d.w, d.ci, d.kh, d.kw, d.co, d.oh, d.ow = n, h, w, ci, k, k, co, oh, ow
+    d.stride_h, d.stride_w = stride
+    d.pad_h, d.pad_w = -crop[0], -crop[1]
+    d.dil_h = d.dil_w = 1
+    dev = [hk.DeviceBuffer.from_numpy(E.to_bf16_bits(a) if bf else a) for a in (x, f, g)]
+    L.pml_hip_conv2d_grad_dispatch.restype = ctypes.c_int64
+    for which, other, want in ((0, dev[1], want_x), (1, dev[0], want_f)):
+        assert L.pml_hip_conv2d_grad_takes(ctypes.byref(d), which) == 1
+        p = L.pml_hip_conv2d_grad_dispatch(ctypes.byref(d), which)
+        assert p, L.pml_hip_last_error()
+        out = hk.DeviceBuffer.from_numpy(np.full(want.size, np.nan, np.float32))
+        hk.check(L.pml_hip_conv2d_grad_invoke(ctypes.c_int64(p), ctypes.c_void_p(dev[2].ptr), ctypes.c_void_p(other.ptr), ctypes.c_void_p(out.ptr), None))
+        got = E.from_bf16_bits(out.to_numpy(np.uint16, want.shape)) if bf else out.to_numpy(np.float32, want.shape)
+        L.pml_hip_plan_free(ctypes.c_int64(p))
+        terms = k * k * co if which == 0 else n * oh * ow
+        np.testing.assert_allclose(got, want, rtol=2.0 ** -8 if bf else 2.0 ** -20, atol=terms * 2.0 ** -22)
