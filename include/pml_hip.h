@@ -81,6 +81,13 @@ int pml_hip_copy_spans(int n, void* const* dst, const void* const* src, const si
  * the copies begin, or, with `after`, when they are made (to the microsecond).  n = 0: the clock alone. */
 int pml_hip_copy_spans_stamped(int n, void* const* dst, const void* const* src, const size_t* nbytes, uint64_t* stamp, int after,
                                pml_hip_stream s);
+/* The same with the clock ahead of the copies, and `value` to *mark (page-locked memory) when they are made and the host can see
+ * them.  `arrived` (device memory, 4 bytes) is left as it is.  _wait_mark returns when the mark is there, or when the stream is
+ * through: it looks for a millisecond, from the first 20 us on with other threads let ahead, and waits for the stream then.  What is
+ * queued is not retired when the mark is there: a wait for the stream behind it takes the longer. */
+int pml_hip_copy_spans_marked(int n, void* const* dst, const void* const* src, const size_t* nbytes, uint64_t* stamp, uint32_t* mark,
+                              uint32_t* arrived, uint32_t value, pml_hip_stream s);
+int pml_hip_wait_mark(const uint32_t* mark, uint32_t value, pml_hip_stream s);
 int pml_hip_clock_khz(void); /* 0 on failure */
 /* Fills with a 32-bit pattern using a kernel (safe to capture into a graph). */
 int pml_hip_fill_u32(void* dptr, uint32_t pattern, size_t n_words, pml_hip_stream s);

@@ -727,6 +727,12 @@ __global__ __launch_bounds__(256) void copy_spans_kernel(SpanArgs a) {
   if (stamps && a.stamp_after) *a.stamp = wall_clock64();
 }
 
+// `value` to page-locked memory, behind everything that its stream holds so far (a launch begins when the ones ahead have written).
+__global__ void mark_kernel(uint32_t* mark, uint32_t value) {
+  __threadfence_system();
+  __hip_atomic_store(mark, value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 inline unsigned grid_for(int64_t work_items) {
   int64_t blocks = (work_items + 255) / 256;
   if (blocks < 1) blocks = 1;
@@ -1117,6 +1123,11 @@ hipError_t copy_spans_launch(const SpanArgs& a, hipStream_t s) {
   size_t blocks = (most / 16 + 4 * 256 - 1) / (4 * 256);
   blocks = blocks < 1 ? 1 : blocks > 64 ? 64 : blocks;
   hipLaunchKernelGGL(copy_spans_kernel, dim3((unsigned)blocks, (unsigned)(a.n > 0 ? a.n : 1)), dim3(256), 0, s, a);
+  return hipGetLastError();
+}
+
+hipError_t mark_launch(uint32_t* mark, uint32_t value, hipStream_t s) {
+  hipLaunchKernelGGL(mark_kernel, dim3(1), dim3(1), 0, s, mark, value);
   return hipGetLastError();
 }
 

@@ -316,6 +316,7 @@ struct SpanArgs {
   uint64_t* stamp;  // the device's clock goes here, before or after the copies; or null
 };
 hipError_t copy_spans_launch(const SpanArgs& a, hipStream_t s);
+hipError_t mark_launch(uint32_t* mark, uint32_t value, hipStream_t s);
 hipError_t fill_u32_launch(void* p, uint32_t pattern, size_t n_words, hipStream_t s);
 hipError_t softmax_launch(const pml_hip_softmax_desc& d, const void* x, void* y, hipStream_t s);
 

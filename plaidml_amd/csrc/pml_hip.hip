@@ -6,11 +6,13 @@
 #include <algorithm>
 #include <cmath>
 #include <atomic>
+#include <chrono>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "device_common.h"
@@ -926,6 +928,25 @@ int pml_hip_copy_spans_stamped(int n, void* const* dst, const void* const* src, 
     if (check(copy_spans_launch(a, (hipStream_t)s), "copy_spans_launch")) return 1;
   }
   return 0;
+}
+int pml_hip_copy_spans_marked(int n, void* const* dst, const void* const* src, const size_t* nbytes, uint64_t* stamp, uint32_t* mark,
+                              uint32_t* arrived, uint32_t value, pml_hip_stream s) {
+  if (!mark || !arrived) return fail("copy_spans: bad argument");
+  if (pml_hip_copy_spans_stamped(n, dst, src, nbytes, stamp, 0, s)) return 1;
+  return check(mark_launch(mark, value, (hipStream_t)s), "mark");
+}
+int pml_hip_wait_mark(const uint32_t* mark, uint32_t value, pml_hip_stream s) {
+  if (!mark) return fail("wait_mark: null pointer");
+  using clock = std::chrono::steady_clock;
+  const clock::time_point begin = clock::now();
+  for (clock::duration waited{}; waited < std::chrono::milliseconds(1); waited = clock::now() - begin) {
+    for (int i = 0; i < 64; ++i) {
+      if (__atomic_load_n(mark, __ATOMIC_ACQUIRE) == value) return 0;
+      __builtin_ia32_pause();
+    }
+    if (waited > std::chrono::microseconds(20)) std::this_thread::yield();
+  }
+  return pml_hip_stream_sync(s);
 }
 int pml_hip_clock_khz(void) {
   int dev = 0, khz = 0;

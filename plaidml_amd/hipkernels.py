@@ -54,7 +54,7 @@ EXPORTS = [
     'pml_hip_conv2d_dispatch', 'pml_hip_conv2d_invoke', 'pml_hip_dwconv2d_dispatch', 'pml_hip_dwconv2d_invoke',
     'pml_hip_pool2d_dispatch', 'pml_hip_pool2d_invoke', 'pml_hip_eltwise_dispatch', 'pml_hip_eltwise_invoke',
     'pml_hip_select', 'pml_hip_softmax', 'pml_hip_index', 'pml_hip_contract_dispatch', 'pml_hip_contract_invoke', 'pml_hip_plan_free',
-    'pml_hip_rows_takes', 'pml_hip_rows', 'pml_hip_argmax_rows', 'pml_hip_topk_rows', 'pml_hip_memcpy_h2d_async', 'pml_hip_memcpy_d2h_async', 'pml_hip_copy_spans', 'pml_hip_copy_spans_stamped', 'pml_hip_clock_khz', 'pml_hip_product_dispatch', 'pml_hip_product_takes_tail', 'pml_hip_plan_bytes', 'pml_hip_product_pays', 'pml_hip_product_invoke', 'pml_hip_conv2d_grad_takes',
+    'pml_hip_rows_takes', 'pml_hip_rows', 'pml_hip_argmax_rows', 'pml_hip_topk_rows', 'pml_hip_memcpy_h2d_async', 'pml_hip_memcpy_d2h_async', 'pml_hip_copy_spans', 'pml_hip_copy_spans_stamped', 'pml_hip_copy_spans_marked', 'pml_hip_wait_mark', 'pml_hip_clock_khz', 'pml_hip_product_dispatch', 'pml_hip_product_takes_tail', 'pml_hip_plan_bytes', 'pml_hip_product_pays', 'pml_hip_product_invoke', 'pml_hip_conv2d_grad_takes',
     'pml_hip_conv2d_grad_dispatch', 'pml_hip_conv2d_grad_invoke',
     'pml_hip_plan_describe', 'pml_hip_struct_size', 'pml_hip_gemm_pack_b', 'pml_hip_conv2d_pack_filter', 'pml_hip_conv2d_takes_maxpool',
     'pml_hip_gather', 'pml_hip_scatter', 'pml_hip_argsort', 'pml_hip_prng',
@@ -170,12 +170,15 @@ def lib():
                      'pml_hip_pool2d_dispatch', 'pml_hip_eltwise_dispatch', 'pml_hip_contract_dispatch'):
             getattr(L, name).restype = ctypes.c_int64
         vp, sz = ctypes.c_void_p, ctypes.c_size_t
+        pp = ctypes.POINTER(vp)
         L.pml_hip_malloc.argtypes = [ctypes.POINTER(vp), sz]
         L.pml_hip_free.argtypes = [vp]
         L.pml_hip_memcpy_h2d.argtypes = [vp, vp, sz, vp]
         L.pml_hip_memcpy_d2h.argtypes = [vp, vp, sz, vp]
         L.pml_hip_memcpy_d2d.argtypes = [vp, vp, sz, vp]
         L.pml_hip_fill_u32.argtypes = [vp, ctypes.c_uint32, sz, vp]
+        L.pml_hip_copy_spans_marked.argtypes = [ctypes.c_int, pp, pp, ctypes.POINTER(sz), vp, ctypes.POINTER(ctypes.c_uint32), vp, ctypes.c_uint32, vp]
+        L.pml_hip_wait_mark.argtypes = [ctypes.POINTER(ctypes.c_uint32), ctypes.c_uint32, vp]
         L.pml_hip_stream_sync.argtypes = [vp]
         L.pml_hip_event_create.argtypes = [ctypes.POINTER(vp)]
         L.pml_hip_event_destroy.argtypes = [vp]
@@ -186,7 +189,6 @@ def lib():
         L.pml_hip_capture_end.argtypes = [vp, ctypes.POINTER(vp)]
         L.pml_hip_graph_launch.argtypes = [vp, vp]
         L.pml_hip_graph_destroy.argtypes = [vp]
-        pp = ctypes.POINTER(vp)
         L.pml_hip_gemm_invoke.argtypes = [ctypes.c_int64, vp, vp, vp, vp, pp, pp, vp]
         L.pml_hip_gemm_run_static.argtypes = [ctypes.POINTER(GemmDesc), vp, vp, vp, vp, pp, pp, vp]
         L.pml_hip_gemm_invoke2.argtypes = [ctypes.c_int64, vp, vp, vp, vp, vp, vp, vp, pp, pp, vp]
