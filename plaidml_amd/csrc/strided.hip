@@ -210,9 +210,14 @@ struct Side {
     run_step = pixel(p, BF ? kRowStep - 3 : kRowStep);  // (bf16: from the last row of a block of four)
   }
 
-  // A thread's runs of neighbouring values: where run r of the slab at k0 begins, and which of its values belong to it.
   static constexpr int kVals = BF && MODE == ROWS_K ? 8 : 4, kWords = kVals * (BF ? 2 : 4) / 4;
   static constexpr int kRuns = BF && MODE != ROWS_K ? 4 * kBlocks : kPasses;
+  __device__ __forceinline__ Pixel next_pixel(const StridedArgs& p, const Pixel& pix, int r) const {
+    if (BF && r % 4 != 3) return ahead(p, pix, 0, 0, 1);
+    return r + 1 < kRuns ? ahead(p, pix, run_step.img, run_step.oy, run_step.ox) : pix;
+  }
+
+  // A thread's runs of neighbouring values: where run r of the slab at k0 begins, and which of its values belong to it.
   struct Run {
     int64_t at;
     int lo, hi;
@@ -269,12 +274,10 @@ struct Side {
   }
 
   // Where nothing is cut and rows are contiguous the loads go out as they are; elsewhere run by run, or value by value where a run is
-  // cut.  FLAT (filter gradients, where a slab's pixels always have cut window rows among them; it takes 30 registers more, which
-  // products have no use for): the loads go out whole there, too, and put() clears what does not belong to the operand -- but for a slab
-  // with a run that sticks out of the operand's `extent` elements.  With a branch per run, and per value, the loads of a slab waited
-  // for each other: 567 pixels of 3 x 45 window values x 20, bf16 19.6 -> 12.4 us, 154154 of 3 x 51 x 38 58.6 -> 35.6.  (Tried: two slabs on their
-  // way instead of one, 219 registers and 46.6 us.  What it costs: 28 pixels and fewer, one slab that ends the tensor, 0.2 to 0.5 us of 5 to
-  // 6; windows of 140 channels and more in bf16, few of whose runs are cut, 4 to 6 %, 2968 pixels of 5 x 870 x 84 35.6, 37.9.)
+  // cut.  FLAT (filter gradients, where a slab's pixels always have cut window rows among them; see `flat_fetch`): the loads go out whole
+  // there, too, and put() clears what does not belong to the operand -- but for a slab with a run that sticks out of the operand's
+  // `extent` elements.  (Tried: two slabs on their way instead of one, 219 registers, 46.6 us for 35.6; loads of what is not there beside
+  // what is instead of from the base, 3 % slower.)
   __device__ __forceinline__ void fetch(const StridedArgs& p, int64_t k0, int64_t k_end, int tid) {
     Pixel pix{0, 0, 0};
     if constexpr (MODE == ROWS_CONV) {
@@ -288,7 +291,8 @@ struct Side {
 #pragma unroll
       for (int r = 0; r < kRuns; ++r) {
         const Run at = run(p, r, k0, k_end, tid, pix);
-        if (full || (at.hi == kVals && apart == 1))
+        if constexpr (MODE == ROWS_CONV) pix = next_pixel(p, pix, r);
+        if (full || (at.lo == 0 && at.hi == kVals && apart == 1))
           straight(&regs[kWords * r], at.at);
         else
           gather(&regs[kWords * r], at.at, at.lo, at.hi, apart);
@@ -300,12 +304,7 @@ struct Side {
 #pragma unroll
     for (int r = 0; r < kRuns; ++r) {
       runs[r] = run(p, r, k0, k_end, tid, pix);
-      if constexpr (MODE == ROWS_CONV) {
-        if (BF && r % 4 != 3)
-          pix = ahead(p, pix, 0, 0, 1);
-        else if (r + 1 < kRuns)
-          pix = ahead(p, pix, run_step.img, run_step.oy, run_step.ox);
-      }
+      if constexpr (MODE == ROWS_CONV) pix = next_pixel(p, pix, r);
       const bool any = runs[r].hi > runs[r].lo;
       keep[r] = any ? runs[r].lo | (runs[r].hi - runs[r].lo) << 8 : 0;
       out = out || (any && (runs[r].at < 0 || runs[r].at + kVals > extent));
@@ -317,12 +316,7 @@ struct Side {
       for (int r = 0; r < kRuns; ++r) straight(&regs[kWords * r], runs[r].hi > runs[r].lo ? runs[r].at : 0);
     } else {
 #pragma unroll
-      for (int r = 0; r < kRuns; ++r) {
-        if (runs[r].lo == 0 && runs[r].hi == kVals && apart == 1)
-          straight(&regs[kWords * r], runs[r].at);
-        else
-          gather(&regs[kWords * r], runs[r].at, runs[r].lo, runs[r].hi, apart);
-      }
+      for (int r = 0; r < kRuns; ++r) gather(&regs[kWords * r], runs[r].at, runs[r].lo, runs[r].hi, apart);
     }
   }
 
@@ -387,13 +381,13 @@ struct Side {
   }
 };
 
-template <bool BF, int AMODE, int BMODE, int MI, int NI>
+template <bool BF, int AMODE, int BMODE, int MI, int NI, bool FLAT = false>
 __global__ __launch_bounds__(kThreads) void strided_kernel(StridedArgs p_by_value) {
   // (read where the dispatcher put it: indexing a by-value copy would move the copy to scratch memory)
   const StridedArgs& p = *(const StridedArgs*)(const __attribute__((address_space(4))) void*)__builtin_amdgcn_kernarg_segment_ptr();
   constexpr int TM = 64 * MI, TN = 64 * NI, ES = BF ? 2 : 4;
-  typedef Side<BF, AMODE, TM, AMODE == ROWS_CONV> side_a;
-  typedef Side<BF, BMODE, TN, AMODE == ROWS_CONV> side_b;
+  typedef Side<BF, AMODE, TM, FLAT> side_a;
+  typedef Side<BF, BMODE, TN, FLAT> side_b;
   constexpr int BK = side_a::BK, kStage = side_a::kBytes + side_b::kBytes;
   extern __shared__ __attribute__((aligned(16))) char smem[];
 
@@ -615,10 +609,10 @@ __global__ __launch_bounds__(256) void strided_reduce_kernel(StridedArgs p_by_va
   store_results(p, p.C, c_at + n, v, live);
 }
 
-template <bool BF, int AMODE, int BMODE, int MI, int NI>
+template <bool BF, int AMODE, int BMODE, int MI, int NI, bool FLAT = false>
 hipError_t launch_tile(const StridedArgs& a, hipStream_t s) {
-  const size_t lds = std::max<size_t>(2 * (Side<BF, AMODE, 64 * MI, AMODE == ROWS_CONV>::kBytes + Side<BF, BMODE, 64 * NI, AMODE == ROWS_CONV>::kBytes), 64 * MI * (64 * NI + 4) * 4);
-  auto kern = strided_kernel<BF, AMODE, BMODE, MI, NI>;
+  const size_t lds = std::max<size_t>(2 * (Side<BF, AMODE, 64 * MI, FLAT>::kBytes + Side<BF, BMODE, 64 * NI, FLAT>::kBytes), 64 * MI * (64 * NI + 4) * 4);
+  auto kern = strided_kernel<BF, AMODE, BMODE, MI, NI, FLAT>;
   static DynamicLdsLimit limit;
   if (hipError_t e = limit.ensure((const void*)kern, lds); e != hipSuccess) return e;
   int64_t nb = (int64_t)a.tiles_m * a.tiles_n;
@@ -627,9 +621,24 @@ hipError_t launch_tile(const StridedArgs& a, hipStream_t s) {
   return hipGetLastError();
 }
 
+// Whether a filter gradient's loads go out whole.  With a branch per run the loads of a slab wait for each other, without one every
+// run's place and what it keeps are counted out ahead: 35 registers more and twice the instructions.  That pays in bf16, with half the values
+// a load's wait: of 105 sizes 1.03 x as fast (10000 pixels of 3 x 177 x 242 34.9 -> 31.5 us, 30276 of 3 x 519 x 62
+// 72.2 -> 55.1).  It does not in fp32 (135 sizes, run by run 1.06 x as fast, none slower; 33800 pixels of 5 x 185 x 95 130.2 -> 122.9, one pixel
+// of 8 x 47 5.0 -> 4.5), nor for two slabs and less (4 pixels of 7 x 106 5.7 -> 5.0), nor for many pixels of long windows, whose tiles keep
+// every CU at its instructions (5000 of 5 x 480 x 96 38.2 -> 30.2, 12150 of 5 x 775 x 68 123.7 -> 101.2, 2028 of 7 x 434 x 200 39.2 -> 31.7; but
+// 17787 of 5 x 430 x 45 0.89 x, 35000 of 5 x 375 x 24 0.93, and where the tiles alone are more than the CUs 2916 of 7 x 1386 x 164 0.92).
+bool flat_fetch(const StridedArgs& a) {
+  return a.K > 128 && !(a.splits > 1 && a.M >= 5 * a.row_cols && a.M >= 2240 && a.K >= 2000);
+}
+
 template <bool BF, int MI>
 hipError_t launch_modes(const StridedArgs& a, int amode, int bmode, hipStream_t s) {
-  if (amode == ROWS_CONV) return launch_tile<BF, ROWS_CONV, ROWS_M, MI, MI>(a, s);
+  if (amode == ROWS_CONV) {
+    if constexpr (BF)
+      if (flat_fetch(a)) return launch_tile<BF, ROWS_CONV, ROWS_M, MI, MI, true>(a, s);
+    return launch_tile<BF, ROWS_CONV, ROWS_M, MI, MI>(a, s);
+  }
   if (amode == ROWS_K) return bmode == ROWS_K ? launch_tile<BF, ROWS_K, ROWS_K, MI, MI>(a, s) : launch_tile<BF, ROWS_K, ROWS_M, MI, MI>(a, s);
   return bmode == ROWS_K ? launch_tile<BF, ROWS_M, ROWS_K, MI, MI>(a, s) : launch_tile<BF, ROWS_M, ROWS_M, MI, MI>(a, s);
 }

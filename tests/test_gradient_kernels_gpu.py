@@ -83,6 +83,9 @@ MORE = [
     (3, 9, 7, 13, 1, 1, 20, 3, 2, 3, 0, 1),       # one tap: pixels that no window covers, pixels behind the last gradient row and column
     (1, 11, 10, 5, 1, 1, 9, 6, 6, 2, 1, 1),       # ... and gradient pixels beside the image
     (2, 21, 11, 150, 3, 3, 80, 21, 11, 1, 1, 1),  # 300 KB of results a split
+    (1, 46, 45, 90, 5, 5, 9, 46, 45, 1, 2, 1),    # many pixels of long windows, bf16: run by run again
+    (2, 8, 8, 10, 3, 3, 6, 8, 8, 1, 1, 1),        # two slabs of bf16 pixels, and more
+    (2, 9, 8, 10, 3, 3, 6, 9, 8, 1, 1, 1),
 ]
 
 
