@@ -1055,8 +1055,9 @@ hipError_t product_direct_launch(const StridedArgs& a, bool bf, int rows, hipStr
 // four slabs, for about three workgroups per CU (their LDS fits four times into one).  A filter gradient's slab takes as long as
 // its loads: runs of two slabs and more (567 pixels of 3 x 45 x 20 in bf16 12.4 -> 9.5 us, 2116 of 3 x 60 x 18 in fp32 12.4 -> 9.2),
 // and in fp32, whose workgroups fit four times into a CU's registers, four per CU (50176 of 3 x 192 x 64 64.5 -> 61.1) -- but for
-// partial results of 300 KB a split, which a second launch reads again: those only up to 6 MB, or with eight slabs a run left (1512
-// pixels of 3 x 348 x 112 in fp32, 468 KB: 12 splits 18.2, 24 of two slabs 20.1; 2173 of 3 x 510 x 66, 404 KB: 14 24.1, 17 25.7).
+// partial results in fp32 of 300 KB a split, which a second launch reads again: those only up to 6 MB, or with six slabs a run left (1512
+// pixels of 3 x 348 x 112 in fp32, 468 KB: 12 splits 18.2, 24 of two slabs 20.1; 2173 of 3 x 510 x 66, 404 KB: 14 24.1, 17 25.7;
+// bf16, whose slabs are twice the pixels, takes them: 900 of 3 x 456 x 240 4 splits 1.07 x as long as 7, 2304 of 3 x 438 x 190 9 1.07 x 13).
 void strided_plan(StridedArgs* a, bool bf, bool conv, int n_cus, int* mi) {
   int64_t batches = 1;
   for (int d = 0; d < a->n_batch; ++d) batches *= a->batch[d];
@@ -1079,7 +1080,7 @@ void strided_plan(StridedArgs* a, bool bf, bool conv, int n_cus, int* mi) {
     const int64_t three = (3 * n_cus + have - 1) / have, bytes = std::max<int64_t>(1, a->ws_rows * a->ws_pitch * 4);
     int64_t want = std::min(three, slabs / 4);
     if (conv) {
-      const int64_t fits = bytes <= 300 << 10 ? slabs : std::max(((int64_t)6 << 20) / bytes, slabs / 8);
+      const int64_t fits = bf || bytes <= 300 << 10 ? slabs : std::max(((int64_t)6 << 20) / bytes, slabs / 6);
       want = std::max(want, std::min({bf ? three : 4 * n_cus / have, slabs / 2, fits}));
     }
     // the partial results: at most 256 MiB of them
