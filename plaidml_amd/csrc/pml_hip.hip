@@ -807,8 +807,10 @@ WinShape window_shape(Plan* p, bool named, double* window_us) {
 //   1 x 1    bf16 28 x 9 x 9 x 256 (*) 62 10.3 -> 5.9     int8 36 x 7 x 7 x 128 (*) 46 8.5 -> 4.7     fp32 3 x 9 x 9 x 96 (*) 23 stride 2 9.7 -> 6.7
 //   3 x 3    bf16 5 x 25 x 25 x 32 (*) 76 8.8 -> 5.2      int8 34 x 14 x 14 x 64 (*) 59 9.5 -> 6.0    fp32 2 x 15 x 15 x 32 (*) 37 10.2 -> 6.8
 //   5 x 5    bf16 11 x 21 x 21 x 64 (*) 102 stride 2 11.7 -> 8.7; but 2 x 69 x 69 x 64 (*) 19, two rounds, 12.2, as it lies 16.9
-//   7 x 7    bf16 from 3 KB of K on by 15 %: 74 x 18 x 40 (*) 16 7.5, as it lies 7.9, under tanh 10.6 and 11.9 (a workgroup's tail is of four
-//            times the results); 2 x 61 x 13 x 32 (*) 9 with a residual 13.9, 14.3
+//   7 x 7    bf16 from 3 KB of K on by 15 % where whole words of columns are packed quickly, 74 x 18 x 40 (*) 16 7.5, as it lies 7.9, 968
+//            pixels of 64 (*) 56 11.3, 12.3, 5 x 5 432 of 96 (*) 60 9.5, 10.4, and under tails with operands and functions (a workgroup's is of
+//            four times the results): with tanh 10.6, 11.9, 2 x 61 x 13 x 32 (*) 9 with a residual 13.9, 14.3.  But odd columns 300 pixels of
+//            40 (*) 37 9.0, as it lies 8.2, 5 x 5 1089 of 128 (*) 50 18.7, 12.7, and 256 channels 3 x 3 882 of 256 (*) 64 10.3, 9.05
 // and of 140 drawn convolutions with the filter in the call 59 take it, 1.36 x in the mean.
 int given_filter_tile(const Plan* p, double window_us) {
   const pml_hip_conv2d_desc& d = p->conv;
@@ -819,7 +821,8 @@ int given_filter_tile(const Plan* p, double window_us) {
   double packed_us = window_us;
   if (!window) (void)direct_tile_of(M, d.co, k_bytes, p->mfma_kind, 0, p->tile_direct >= 0, /*can_split=*/!p->patches, false, &packed_us);
   const double small = direct_lies_us(M, d.co, k_bytes, p->mfma_kind, 16), large = direct_lies_us(M, d.co, k_bytes, p->mfma_kind, 32), packing = 3.0 + 2.0 * (double)k_bytes * (double)d.co / 2.2e6;
-  const bool close = p->tile_direct >= 0 && !(p->mfma_kind == KIND_BF16 && k_bytes >= 3072);
+  const bool bare = tail_form(d.tail, d.out_dtype, d.c_dtype, true, false).bare;
+  const bool close = p->tile_direct >= 0 && !(p->mfma_kind == KIND_BF16 && k_bytes >= 3072 && ((d.co % 4 == 0 && d.ci < 256) || !bare));
   if (std::min(small, large) > (close ? 0.95 : 0.85) * (packed_us + packing)) return -1;
   return small <= large ? TILE_16x16_W8 : TILE_32x32_W8;
 }

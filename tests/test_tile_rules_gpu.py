@@ -123,14 +123,18 @@ def test_split_fp32_of_two_rounds(m, n, k, split, layout):
     assert ('3 x f32' in text_of(hk.F32, m, n, k, layout, hk.FP32_AS_BF16X3)) == split
 
 
-# 7 x 7 taps of 40 channels, 4 KB of K; the same in int8 and of fewer channels
-@pytest.mark.parametrize('kind,out,ci,lies', [(hk.BF16, hk.BF16, 40, False), (hk.I8, hk.I32, 32, True), (hk.BF16, hk.BF16, 16, True)])
-def test_filters_of_a_long_k_that_come_with_the_call(kind, out, ci, lies):
+# 7 x 7 taps of 40 channels, 4 KB of K; odd columns, a residual over them; the same in int8 and of fewer channels
+@pytest.mark.parametrize('kind,out,ci,co,residual,lies', [(hk.BF16, hk.BF16, 40, 16, False, False), (hk.BF16, hk.BF16, 40, 15, False, True),
+                                                          (hk.BF16, hk.BF16, 40, 15, True, False), (hk.I8, hk.I32, 32, 16, False, True),
+                                                          (hk.BF16, hk.BF16, 16, 16, False, True)])
+def test_filters_of_a_long_k_that_come_with_the_call(kind, out, ci, co, residual, lies):
     d = hk.Conv2dDesc()
     d.in_dtype, d.out_dtype, d.c_dtype = kind, out, out
-    d.n, d.h, d.w, d.ci, d.kh, d.kw, d.co, d.oh, d.ow = 1, 74, 18, ci, 7, 7, 16, 74, 18
+    d.n, d.h, d.w, d.ci, d.kh, d.kw, d.co, d.oh, d.ow = 1, 74, 18, ci, 7, 7, co, 74, 18
     d.stride_h = d.stride_w = d.dil_h = d.dil_w = 1
     d.pad_h = d.pad_w = 3
+    if residual:
+        d.tail = hk.make_tail(ops=[(hk.EPI_ADD, out, hk.OPND_TENSOR, 0, 0.0)], operands=[(out, co, 1)])
     plan = hk.lib().pml_hip_conv2d_dispatch(ctypes.byref(d))
     assert ('with the filter as it lies' in hk.describe(plan)) == lies, hk.describe(plan)
     hk.lib().pml_hip_plan_free(plan)
