@@ -276,12 +276,13 @@ int direct_tile_of(int64_t m, int64_t n, int64_t k_bytes, int kind, int64_t kn_l
 // Microseconds of a 16 or 32 x 64 direct tile over a right-hand side [K][N] as it lies, from 260 timings of 130 convolutions (8 to
 // 13 % rms): 2.6, and per round of one tile on each CU (a last one that is not full counts for most of one) a start and so much per
 // KB of K -- not per byte of few columns: it is the requests for K-rows that take the time, more of them for int8, whose rows off a
-// word take two words each.  (int8 of few columns on a word: 400 x 12, K = 3136 10.4, 864 x 24, K = 2000 7.6, 56 x 92, K = 800 5.4.)
+// word take two words each.  (int8 on a word, but not in whole 16 bytes: 400 x 12, K = 3136 10.4, 864 x 24, K = 2000 7.6, 300 x 92, K = 1600 7.2; in whole ones
+// 441 x 16, K = 3200 7.0, 256 x 208, K = 2400 5.9.)
 double direct_lies_us(int64_t m, int64_t n, int64_t k_bytes, int kind, int side) {
   const bool small = side == 16, odd = n % 4 != 0;
   double start, per_kb;
   if (kind == KIND_BF16) start = small ? 1.35 : 1.7, per_kb = small ? 1.17 : 1.52;
-  else if (kind == KIND_I8) start = small ? 1.3 : 1.6, per_kb = !odd ? 2.0 : small ? 2.05 : 2.45;
+  else if (kind == KIND_I8) start = small ? 1.3 : 1.6, per_kb = n % 16 == 0 ? 1.2 : !odd ? 2.3 : small ? 2.05 : 2.45;
   else start = small ? 2.2 : 1.7, per_kb = small ? 1.2 : 2.3;
   const double rounds = std::max(1.0, (double)((m + side - 1) / side) * (double)((n + 63) / 64) / device_cus());
   return 2.6 + (0.75 * std::ceil(rounds) + 0.25 * rounds) * (start + per_kb * (double)k_bytes / 1024);

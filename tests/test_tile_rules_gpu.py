@@ -143,6 +143,7 @@ def test_filters_of_a_long_k_that_come_with_the_call(kind, out, ci, co, residual
 # int8 of 3 KB of K: ten rows of tiles of 32, and fewer channels; fp32 of a long K in eight rounds of 16 x 16 and in less than one
 @pytest.mark.parametrize('kind,out,n,h,ci,k,stride,co,text', [(hk.I8, hk.I32, 4, 20, 64, 7, 2, 12, None), (hk.I8, hk.I32, 4, 20, 16, 3, 2, 12, 'with the filter as it lies'),
                                                              (hk.F32, hk.F32, 7, 68, 128, 3, 1, 11, 'over its window in LDS'),
+                                                             (hk.I8, hk.I32, 4, 20, 96, 5, 2, 48, 'with the filter as it lies'),
                                                              (hk.F32, hk.F32, 1, 14, 128, 3, 1, 11, 'direct tile=16x16')])
 def test_convolutions_beside_their_direct_tiles(kind, out, n, h, ci, k, stride, co, text):
     d = hk.Conv2dDesc()
