@@ -307,10 +307,14 @@ bool fp32_beats_split(int64_t m, int64_t n, int64_t k_bytes) {
     }
   }
   if (direct_tile_of(m, n, k_bytes, KIND_F32) < 0) return false;
-  // (two rounds of 16 x 16 tiles over few K take longer than that price: 29 x 3872, K = 96 [N][K] 5.2, direct 6.0)
-  if (direct_tile_of(m, n, k_bytes, KIND_F32, 0, /*always=*/true, true, false, &us) == TILE_16x16_W8 && ((m + 15) / 16) * ((n + 15) / 16) > device_cus()) us += 0.7;
+  // (two rounds of 16 x 16 tiles over few K take longer than that price: 29 x 3872, K = 96 [N][K] 5.2, direct 6.0; odd columns,
+  // which the split's tail stores one by one, do not: 191 x 381, K = 64 6.0, direct 5.0)
+  if (direct_tile_of(m, n, k_bytes, KIND_F32, 0, /*always=*/true, true, false, &us) == TILE_16x16_W8 && ((m + 15) / 16) * ((n + 15) / 16) > device_cus() && !needs_bt) us += 0.7;
   const double copy = needs_bt ? 3.0 + 2.0 * (double)k_bytes * (double)n / 2.2e6 : 0;
-  return us <= 0.95 * split_us && std::min(direct_lies_us(m, n, k_bytes, KIND_F32, 16), direct_lies_us(m, n, k_bytes, KIND_F32, 32)) <= 0.95 * (split_us + copy);
+  // (16 x 64 tiles of one round take fewer steps in flight where they have few: 2.6 + 1.3 + 1.25 per KB of K, to 10 %)
+  const bool one_round = ((m + 15) / 16) * ((n + 63) / 64) <= device_cus();
+  const double small = one_round ? 3.9 + 1.25 * (double)k_bytes / 1024 : direct_lies_us(m, n, k_bytes, KIND_F32, 16);
+  return us <= 0.95 * split_us && std::min(small, direct_lies_us(m, n, k_bytes, KIND_F32, 32)) <= 0.95 * (split_us + copy);
 }
 
 // What of a tail decides between tiles.

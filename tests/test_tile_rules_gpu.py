@@ -118,7 +118,8 @@ def test_fp32_of_a_long_k_and_few_columns(m, n, k, direct, layout):
 
 
 @pytest.mark.parametrize('layout', [0, 1])
-@pytest.mark.parametrize('m,n,k,split', [(29, 3872, 96, True), (34, 2320, 96, True), (40, 1800, 200, False), (16, 3872, 96, False)])
+@pytest.mark.parametrize('m,n,k,split', [(29, 3872, 96, True), (34, 2320, 96, True), (40, 1800, 200, False), (16, 3872, 96, False),
+                                         (191, 381, 64, False), (177, 300, 64, False), (5, 27, 1040, False), (4, 36, 2192, True)])
 def test_split_fp32_of_two_rounds(m, n, k, split, layout):
     assert ('3 x f32' in text_of(hk.F32, m, n, k, layout, hk.FP32_AS_BF16X3)) == split
 
