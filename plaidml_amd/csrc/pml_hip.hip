@@ -827,7 +827,8 @@ int given_filter_tile(const Plan* p, double window_us) {
   if (!window) (void)direct_tile_of(M, d.co, k_bytes, p->mfma_kind, 0, p->tile_direct >= 0, /*can_split=*/!p->patches, false, &packed_us);
   const double small = direct_lies_us(M, d.co, k_bytes, p->mfma_kind, 16), large = direct_lies_us(M, d.co, k_bytes, p->mfma_kind, 32), packing = 3.0 + 2.0 * (double)k_bytes * (double)d.co / 2.2e6;
   const bool bare = tail_form(d.tail, d.out_dtype, d.c_dtype, true, false).bare;
-  const bool close = p->tile_direct >= 0 && !(p->mfma_kind == KIND_BF16 && k_bytes >= 3072 && ((d.co % 4 == 0 && d.ci < 256) || !bare));
+  const bool one_round = ((M + 15) / 16) * ((d.co + 15) / 16) <= device_cus();  // (612 pixels of 5 x 5 x 96 (*) 100, two over a packed filter: 12.9, as it lies 10.3)
+  const bool close = p->tile_direct >= 0 && !(p->mfma_kind == KIND_BF16 && k_bytes >= 3072 && ((d.co % 4 == 0 && d.ci < 256 && one_round) || !bare));
   if (std::min(small, large) > (close ? 0.95 : 0.85) * (packed_us + packing)) return -1;
   return small <= large ? TILE_16x16_W8 : TILE_32x32_W8;
 }
