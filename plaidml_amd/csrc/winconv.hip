@@ -87,7 +87,7 @@ struct Mma<KIND_I8> {
 // MB x NB blocks of 16 x 16 results a wavefront; WM x WN wavefronts side by side, KS of them share the steps of K.  Windows are
 // filled by requests that no register waits for: whoever multiplies from one has waited for its own requests (vmcnt 0) and met
 // the others at a barrier since, and a window is filled again only behind a barrier that all its readers have passed.
-template <int KIND, int MB, int NB, int WM, int WN, int KS>
+template <int KIND, int MB, int NB, int WM, int WN, int KS, bool COUNTS>
 __global__ __launch_bounds__(64 * WM * WN * KS, NB >= 4 ? 2 : 4) void winconv_kernel(WinArgs p) {
   warm_arguments<sizeof(WinArgs)>();
   typedef Mma<KIND> X;
@@ -142,7 +142,6 @@ __global__ __launch_bounds__(64 * WM * WN * KS, NB >= 4 ? 2 : 4) void winconv_ke
     int slab, ky, kx, blk;
     int off, b;  // bytes from the window's begin; from the begin of the filter's columns
   };
-  constexpr bool kCounts = KIND != KIND_F32;
   // of a slab: its blocks; what a tap to the right, and the first tap of the next row, add to what KS blocks do
   int nb = 0, tap_off = 0, tap_b = 0, far_x = 0, far_blk = 0, far_off = 0, far_b = 0;
   bool far = false;
@@ -170,11 +169,11 @@ __global__ __launch_bounds__(64 * WM * WN * KS, NB >= 4 ? 2 : 4) void winconv_ke
     far_b = KS * 2048 + far_x * tap_b;
     Step s{slab, 0, 0, kg, 0, 0};
     settle(s);
-    if constexpr (kCounts) s.off = off_of(s), s.b = b_of(s);
+    if constexpr (COUNTS) s.off = off_of(s), s.b = b_of(s);
     return s;
   };
   auto count_on = [&](Step& s) {  // whether there is another step in the slab
-    if constexpr (!kCounts) {
+    if constexpr (!COUNTS) {
       s.blk += KS;
       settle(s);
     } else if (far) {
@@ -206,7 +205,7 @@ __global__ __launch_bounds__(64 * WM * WN * KS, NB >= 4 ? 2 : 4) void winconv_ke
     }
     return s.ky < p.KH;
   };
-  auto lds_at = [&](const Step& s) { return (s.slab & 1) * p.win_bytes + (kCounts ? s.off : off_of(s)); };
+  auto lds_at = [&](const Step& s) { return (s.slab & 1) * p.win_bytes + (COUNTS ? s.off : off_of(s)); };
 
   // filter fragments as winconv_pack_kernel lays them out: a step's 32 columns are 2 KB
   const int group_bytes = p.KH * p.KW * p.total_blocks * 2048;
@@ -215,7 +214,7 @@ __global__ __launch_bounds__(64 * WM * WN * KS, NB >= 4 ? 2 : 4) void winconv_ke
   for (int j = 0; j < NB / 2; ++j) b_group[j] = min(n0 / 32 + j, (p.N - 1) / 32) * group_bytes;
   i32x4_t fa[MB], fb[2][NB];
   auto request_b = [&](i32x4_t (&f)[NB], const Step& s) {
-    const int at = kCounts ? s.b : b_of(s);
+    const int at = COUNTS ? s.b : b_of(s);
 #pragma unroll
     for (int j = 0; j < NB; ++j)
       f[j] = __builtin_bit_cast(i32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rb, lane * 16 + (j & 1) * 1024, b_group[j >> 1] + at, 0));
@@ -478,21 +477,25 @@ hipError_t launch(int cfg, size_t lds, int tiles, const WinArgs& a, hipStream_t 
     hipLaunchKernelGGL(kern, dim3((unsigned)tiles), dim3(64 * c.waves()), lds, s, a);
     return hipGetLastError();
   };
-  static DynamicLdsLimit limits[kNConfigs];
+  constexpr bool COUNTS = KIND != KIND_F32;
+  static DynamicLdsLimit limits[kNConfigs], counted;
+  // (fp32 in 32 x 32 results and slabs of one block, four taps of which are a step: 81608 pixels of 7 x 7 x 64 x 31 227.4 us, counted 216.2,
+  // 19600 of 5 x 5 x 16 x 25 14.1, 13.4; of two blocks and more 0.96 to 1.00 x, larger tiles 0.89 to 1.01 x)
+  if (!COUNTS && cfg == 12 && a.blocks == 1) return go(winconv_kernel<KIND, 2, 2, 2, 1, 4, true>, kConfigs[12], counted);
   switch (cfg) {
-    case 0: return go(winconv_kernel<KIND, 7, 4, 2, 2, 2>, kConfigs[0], limits[0]);
-    case 1: return go(winconv_kernel<KIND, 7, 4, 2, 2, 1>, kConfigs[1], limits[1]);
-    case 2: return go(winconv_kernel<KIND, 7, 4, 1, 2, 4>, kConfigs[2], limits[2]);
-    case 3: return go(winconv_kernel<KIND, 7, 2, 1, 4, 2>, kConfigs[3], limits[3]);
-    case 4: return go(winconv_kernel<KIND, 7, 4, 4, 1, 1>, kConfigs[4], limits[4]);
-    case 5: return go(winconv_kernel<KIND, 7, 4, 2, 1, 4>, kConfigs[5], limits[5]);
-    case 6: return go(winconv_kernel<KIND, 7, 2, 4, 1, 1>, kConfigs[6], limits[6]);
-    case 7: return go(winconv_kernel<KIND, 4, 4, 2, 2, 2>, kConfigs[7], limits[7]);
-    case 8: return go(winconv_kernel<KIND, 4, 4, 2, 1, 2>, kConfigs[8], limits[8]);
-    case 9: return go(winconv_kernel<KIND, 4, 4, 1, 1, 4>, kConfigs[9], limits[9]);
-    case 10: return go(winconv_kernel<KIND, 4, 2, 4, 1, 1>, kConfigs[10], limits[10]);
-    case 11: return go(winconv_kernel<KIND, 4, 2, 2, 1, 2>, kConfigs[11], limits[11]);
-    case 12: return go(winconv_kernel<KIND, 2, 2, 2, 1, 4>, kConfigs[12], limits[12]);
+    case 0: return go(winconv_kernel<KIND, 7, 4, 2, 2, 2, COUNTS>, kConfigs[0], limits[0]);
+    case 1: return go(winconv_kernel<KIND, 7, 4, 2, 2, 1, COUNTS>, kConfigs[1], limits[1]);
+    case 2: return go(winconv_kernel<KIND, 7, 4, 1, 2, 4, COUNTS>, kConfigs[2], limits[2]);
+    case 3: return go(winconv_kernel<KIND, 7, 2, 1, 4, 2, COUNTS>, kConfigs[3], limits[3]);
+    case 4: return go(winconv_kernel<KIND, 7, 4, 4, 1, 1, COUNTS>, kConfigs[4], limits[4]);
+    case 5: return go(winconv_kernel<KIND, 7, 4, 2, 1, 4, COUNTS>, kConfigs[5], limits[5]);
+    case 6: return go(winconv_kernel<KIND, 7, 2, 4, 1, 1, COUNTS>, kConfigs[6], limits[6]);
+    case 7: return go(winconv_kernel<KIND, 4, 4, 2, 2, 2, COUNTS>, kConfigs[7], limits[7]);
+    case 8: return go(winconv_kernel<KIND, 4, 4, 2, 1, 2, COUNTS>, kConfigs[8], limits[8]);
+    case 9: return go(winconv_kernel<KIND, 4, 4, 1, 1, 4, COUNTS>, kConfigs[9], limits[9]);
+    case 10: return go(winconv_kernel<KIND, 4, 2, 4, 1, 1, COUNTS>, kConfigs[10], limits[10]);
+    case 11: return go(winconv_kernel<KIND, 4, 2, 2, 1, 2, COUNTS>, kConfigs[11], limits[11]);
+    case 12: return go(winconv_kernel<KIND, 2, 2, 2, 1, 4, COUNTS>, kConfigs[12], limits[12]);
   }
   return hipErrorInvalidValue;
 }
